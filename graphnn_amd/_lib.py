@@ -1,12 +1,15 @@
 """ctypes binding of libgnnhip.so.  Loading fails loudly: there is no CPU fallback."""
 import ctypes
+import importlib.util
 import os
 from ctypes import POINTER, c_char_p, c_float, c_int, c_size_t, c_void_p
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # GNNHIP_LIBRARY overrides the in-tree location (e.g. an instrumented build of the same ABI)
 _LIB_PATH = os.environ.get("GNNHIP_LIBRARY") or os.path.join(_HERE, "lib", "libgnnhip.so")
+_BINDINGS_PATH = os.path.join(_HERE, "lib", "_gnnhip_torch.so")
 _lib = None
+_bindings = None
 
 
 class GnnHipError(RuntimeError):
@@ -111,6 +114,24 @@ def load_library():
         fn.restype = _RESTYPES.get(name, c_int)
     _lib = lib
     return lib
+
+
+def load_bindings():
+    """The compiled bindings for torch tensors (csrc/torch_bind.cpp), bound to the loaded library.  Raises if they are
+    missing: the helpers of ops have no other way to call a kernel."""
+    global _bindings
+    if _bindings is not None:
+        return _bindings
+    load_library()
+    if not os.path.exists(_BINDINGS_PATH):
+        raise RuntimeError("%s is not built. Run `python -m graphnn_amd.build`." % _BINDINGS_PATH)
+    import torch  # noqa: F401  (the module needs torch's libraries in the process)
+    spec = importlib.util.spec_from_file_location("_gnnhip_torch", _BINDINGS_PATH)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    module.bind(_LIB_PATH, GnnHipError)
+    _bindings = module
+    return module
 
 
 def check(rc):

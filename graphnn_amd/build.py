@@ -1,4 +1,4 @@
-"""Builds libgnnhip.so (the gfx950 HIP kernels + C ABI) in-tree with hipcc.
+"""Builds libgnnhip.so (the gfx950 HIP kernels + C ABI) in-tree with hipcc, and the torch bindings with g++.
 
 Usage: python -m graphnn_amd.build [--force]
 The library is written to graphnn_amd/lib/libgnnhip.so.  hipcc cross-compiles
@@ -16,6 +16,8 @@ CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "lib")
 OBJDIR = os.path.join(LIBDIR, "obj")
 LIB = os.path.join(LIBDIR, "libgnnhip.so")
+BINDINGS_SOURCE = os.path.join(CSRC, "torch_bind.cpp")
+BINDINGS = os.path.join(LIBDIR, "_gnnhip_torch.so")
 
 ARCH = "gfx950"
 # packed-fp32 ops are switched off: hipcc would otherwise form v_pk_*_f32 from plain float code.
@@ -47,6 +49,25 @@ def _compile_one(args):
     return r.stderr
 
 
+def build_bindings(force=True):
+    """Compile the torch bindings (host code only) to graphnn_amd/lib/_gnnhip_torch.so."""
+    if not force and os.path.exists(BINDINGS) and os.path.getmtime(BINDINGS) > max(
+            os.path.getmtime(f) for f in (BINDINGS_SOURCE, os.path.join(ROOT, "include", "gnnhip.h"))):
+        return BINDINGS
+    import sysconfig
+    import torch
+    base = os.path.dirname(torch.__file__)
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, "-w",
+           "-I", os.path.join(ROOT, "include"), "-isystem", os.path.join(base, "include"), "-isystem", "/opt/rocm/include",
+           "-isystem", sysconfig.get_paths()["include"], BINDINGS_SOURCE, "-o", BINDINGS,
+           "-L", os.path.join(base, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ldl"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("g++ failed on %s:\n%s\n%s" % (BINDINGS_SOURCE, r.stdout, r.stderr))
+    return BINDINGS
+
+
 def build(force=True, verbose=True, jobs=8):
     """Compile every .hip source and link libgnnhip.so.  Returns the library path."""
     hipcc = _hipcc()
@@ -75,6 +96,7 @@ def build(force=True, verbose=True, jobs=8):
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError("link failed:\n%s\n%s" % (r.stdout, r.stderr))
+    build_bindings(force)
     if verbose:
         print("built %s (%d sources compiled)" % (LIB, len(todo)))
     return LIB

@@ -9,7 +9,7 @@ import numpy as np
 
 import torch
 
-from ._lib import check, load_library
+from ._lib import check, load_bindings, load_library
 
 UNARY = {
     "set": 0, "truncate": 1, "scale": 2, "add": 3, "abs": 4, "inv": 5, "relu": 6, "sigmoid": 7,
@@ -32,6 +32,24 @@ def _lib():
     if not _initialised:
         init(torch.cuda.current_device())
     return load_library()
+
+
+_bindings = None
+
+
+def _bound():
+    """the compiled bindings: each C entry under its name without gnnhip_, taking torch tensors (checked there for type,
+    device and contiguity) and the current stream, raising GnnHipError"""
+    global _bindings
+    if _bindings is None or not _initialised:
+        _lib()
+        _bindings = load_bindings()
+    return _bindings
+
+
+def _empty(where, kind, *sizes):
+    """uninitialised tensor of float32 ('f') or int32 ('i') on the device of a tensor, or on a torch.device"""
+    return _bound().empty(where, kind, *sizes)
 
 
 def _stream():
@@ -68,12 +86,12 @@ def spmm(row_ptr, col_idx, val, B, m, alpha=1.0, beta=0.0, out=None, nnz_hint=No
     k, n = B.shape
     _check_csr(row_ptr, col_idx, val, m, "A")
     if out is None:
-        out = torch.empty((m, n), dtype=torch.float32, device=B.device)
+        out = _empty(B, "f", m, n)
     elif tuple(out.shape) != (m, n):
         raise ValueError("out has the wrong shape")
     nnz = int(col_idx.numel()) if nnz_hint is None else int(nnz_hint)
-    check(_lib().gnnhip_spmm_csr_f32(m, k, n, nnz, alpha, _i32(row_ptr, "row_ptr"), _i32(col_idx, "col_idx"),
-                                     _f32(val, "val"), _f32(B, "B"), n, beta, _f32(out, "out"), n, _stream()))
+    _bound().spmm_csr_f32(m, k, n, nnz, alpha, row_ptr, col_idx,
+                                     val, B, n, beta, out, n)
     return out
 
 
@@ -100,10 +118,10 @@ class CsrPlan:
         if k != self.k:
             raise ValueError("B must have %d rows" % self.k)
         if out is None:
-            out = torch.empty((self.m, n), dtype=torch.float32, device=B.device)
+            out = _empty(B, "f", self.m, n)
         elif tuple(out.shape) != (self.m, n):
             raise ValueError("out has the wrong shape")
-        check(_lib().gnnhip_spmm_csr_planned_f32(self.handle, n, alpha, _f32(B, "B"), n, beta, _f32(out, "out"), n, _stream()))
+        _bound().spmm_csr_planned_f32(self.handle.value, n, alpha, B, n, beta, out, n)
         return out
 
     def level(self, h_in, W, msg=None, bias=None, out=None):
@@ -111,9 +129,9 @@ class CsrPlan:
         if N != self.m or tuple(W.shape) != (C, C):
             raise ValueError("h_in must be [m,C] and W [C,C]")
         if out is None:
-            out = torch.empty_like(h_in)
-        check(_lib().gnnhip_s2v_level_planned_f32(self.handle, C, _f32(h_in, "h_in"), _f32(W, "W"), _f32(msg, "msg"),
-                                                  _f32(bias, "bias"), _f32(out, "out"), _stream()))
+            out = _empty(h_in, "f", N, C)
+        _bound().s2v_level_planned_f32(self.handle.value, C, h_in, W, msg,
+                                                  bias, out)
         return out
 
     def close(self):
@@ -147,11 +165,11 @@ def gemm(A, B, transA=False, transB=False, alpha=1.0, beta=0.0, out=None, cols_a
     if k != kb:
         raise ValueError("mat dim doesn't match")
     if out is None:
-        out = torch.empty((m, n), dtype=torch.float32, device=A.device)
+        out = _empty(A, "f", m, n)
     elif tuple(out.shape) != (m, n):
         raise ValueError("out has the wrong shape")
-    check(_lib().gnnhip_gemm_f32(int(transA), int(transB), m, n, k, alpha, _f32(A, "A"), A.shape[1],
-                                 _f32(B, "B"), B.shape[1], beta, _f32(out, "out"), n, _stream()))
+    _bound().gemm_f32(int(transA), int(transB), m, n, k, alpha, A, A.shape[1],
+                                 B, B.shape[1], beta, out, n)
     return out
 
 
@@ -168,26 +186,15 @@ def read_scalars(tensors):
 def row_softmax_deriv(dst, out, grad):
     """dst += out * (grad - <grad, out> per row), in place on dst"""
     rows, cols = out.shape
-    check(_lib().gnnhip_row_softmax_deriv_f32(_f32(dst, "dst"), _f32(out, "out"), _f32(grad, "grad"), rows, cols, _stream()))
+    _bound().row_softmax_deriv_f32(dst, out, grad, rows, cols)
     return dst
 
 
 def gemm_tn_batch(products, alpha=1.0, beta=0.0):
     """products: list of (A [k,m], B [k,n], out [m,n]); out = alpha * A^T B + beta * out for all of them in two launches"""
-    import ctypes
-    count = len(products)
-    ints = lambda vals: (ctypes.c_int * count)(*vals)
-    ptrs = lambda ts: (ctypes.c_void_p * count)(*[t.data_ptr() for t in ts])
-    for A, B, out in products:
-        if A.shape[0] != B.shape[0] or tuple(out.shape) != (A.shape[1], B.shape[1]):
-            raise ValueError("mat dim doesn't match")
-        _f32(A, "A"), _f32(B, "B"), _f32(out, "out")
-    As, Bs, Cs = zip(*products) if count else ((), (), ())
-    check(_lib().gnnhip_gemm_tn_batch_f32(count, ints([a.shape[1] for a in As]), ints([b.shape[1] for b in Bs]),
-                                          ints([a.shape[0] for a in As]), ptrs(As), ints([a.shape[1] for a in As]),
-                                          ptrs(Bs), ints([b.shape[1] for b in Bs]), alpha, beta, ptrs(Cs),
-                                          ints([c.shape[1] for c in Cs]), _stream()))
-    return [c for c in Cs]
+    products = [tuple(p) for p in products]
+    _bound().gemm_tn_batch(products, alpha, beta)
+    return [out for _, _, out in products]
 
 
 def s2v_input(X, W_n2l):
@@ -195,10 +202,10 @@ def s2v_input(X, W_n2l):
     if W_n2l.shape[0] != K:
         raise ValueError("X and W_n2l disagree on the label width")
     C = W_n2l.shape[1]
-    msg = torch.empty((N, C), dtype=torch.float32, device=X.device)
-    h0 = torch.empty_like(msg)
-    check(_lib().gnnhip_s2v_input_f32(N, K, C, _f32(X, "X"), _f32(W_n2l, "W_n2l"), _f32(msg, "msg"),
-                                      _f32(h0, "h0"), _stream()))
+    msg = _empty(X, "f", N, C)
+    h0 = _empty(msg, "f", N, C)
+    _bound().s2v_input_f32(N, K, C, X, W_n2l, msg,
+                                      h0)
     return msg, h0
 
 
@@ -206,10 +213,10 @@ def s2v_input_labels(label, W_n2l, status=None):
     """msg = W_n2l[label], h0 = ReLU(msg): the input stage from one int label per node."""
     N = label.numel()
     K, C = W_n2l.shape
-    msg = torch.empty((N, C), dtype=torch.float32, device=W_n2l.device)
-    h0 = torch.empty_like(msg)
-    check(_lib().gnnhip_s2v_input_labels_f32(N, K, C, _i32(label, "label"), _f32(W_n2l, "W_n2l"), _f32(msg, "msg"),
-                                             _f32(h0, "h0"), _i32(status, "status"), _stream()))
+    msg = _empty(W_n2l, "f", N, C)
+    h0 = _empty(msg, "f", N, C)
+    _bound().s2v_input_labels_f32(N, K, C, label, W_n2l, msg,
+                                             h0, status)
     return msg, h0
 
 
@@ -225,11 +232,11 @@ def s2v_level(row_ptr, col_idx, val, h_in, W, msg=None, bias=None, out=None, nnz
     if bias is not None and bias.numel() != C:
         raise ValueError("bias must have C entries")
     if out is None:
-        out = torch.empty_like(h_in)
+        out = _empty(h_in, "f", N, C)
     nnz = int(col_idx.numel()) if nnz_hint is None else int(nnz_hint)
-    check(_lib().gnnhip_s2v_level_f32(N, C, nnz, _i32(row_ptr, "row_ptr"), _i32(col_idx, "col_idx"), _f32(val, "val"),
-                                      _f32(h_in, "h_in"), _f32(W, "W"), _f32(msg, "msg"), _f32(bias, "bias"),
-                                      _f32(out, "out"), _stream()))
+    _bound().s2v_level_f32(N, C, nnz, row_ptr, col_idx, val,
+                                      h_in, W, msg, bias,
+                                      out)
     return out
 
 
@@ -240,15 +247,15 @@ def s2v_readout(s_row_ptr, s_col_idx, s_val, h, W_h1, W_h2, B):
     if W_h1.shape[0] != C or W_h2.shape[0] != H:
         raise ValueError("readout weight shapes do not chain")
     dev = h.device
-    pool = torch.empty((B, C), dtype=torch.float32, device=dev)
-    hidden = torch.empty((B, H), dtype=torch.float32, device=dev)
-    logits = torch.empty((B, Q), dtype=torch.float32, device=dev)
-    probs = torch.empty((B, Q), dtype=torch.float32, device=dev)
-    pred = torch.empty((B,), dtype=torch.int32, device=dev)
-    check(_lib().gnnhip_s2v_readout_f32(B, N, C, H, Q, _i32(s_row_ptr, "s_row_ptr"), _i32(s_col_idx, "s_col_idx"),
-                                        _f32(s_val, "s_val"), _f32(h, "h"), _f32(W_h1, "W_h1"), _f32(W_h2, "W_h2"),
-                                        _f32(pool, "pool"), _f32(hidden, "hidden"), _f32(logits, "logits"),
-                                        _f32(probs, "probs"), _i32(pred, "pred"), _stream()))
+    pool = _empty(dev, "f", B, C)
+    hidden = _empty(dev, "f", B, H)
+    logits = _empty(dev, "f", B, Q)
+    probs = _empty(dev, "f", B, Q)
+    pred = _empty(dev, "i", B)
+    _bound().s2v_readout_f32(B, N, C, H, Q, s_row_ptr, s_col_idx,
+                                        s_val, h, W_h1, W_h2,
+                                        pool, hidden, logits,
+                                        probs, pred)
     return pool, hidden, logits, probs, pred
 
 
@@ -283,14 +290,14 @@ def s2v_forward(a_csr, s_csr, X, W_n2l, W_conv, W_h1, W_h2, L, bufs=None):
         raise ValueError("weight shapes do not chain")
     if bufs is None:
         bufs = ForwardBuffers(N, B, C, H, Q, X.device)
-    check(_lib().gnnhip_s2v_forward_f32(
+    _bound().s2v_forward_f32(
         N, B, K, C, H, Q, L, int(a_csr[1].numel()),
-        _i32(a_csr[0], "a_row_ptr"), _i32(a_csr[1], "a_col_idx"), _f32(a_csr[2], "a_val"),
-        _i32(s_csr[0], "s_row_ptr"), _i32(s_csr[1], "s_col_idx"), _f32(s_csr[2], "s_val"),
-        _f32(X, "X"), _f32(W_n2l, "W_n2l"), _f32(W_conv, "W_conv"), _f32(W_h1, "W_h1"), _f32(W_h2, "W_h2"),
-        _f32(bufs.msg, "msg"), _f32(bufs.h_a, "h_a"), _f32(bufs.h_b, "h_b"), _f32(bufs.pool, "pool"),
-        _f32(bufs.hidden, "hidden"), _f32(bufs.logits, "logits"), _f32(bufs.probs, "probs"),
-        _i32(bufs.pred, "pred"), ctypes.byref(bufs.which), _stream()))
+        a_csr[0], a_csr[1], a_csr[2],
+        s_csr[0], s_csr[1], s_csr[2],
+        X, W_n2l, W_conv, W_h1, W_h2,
+        bufs.msg, bufs.h_a, bufs.h_b, bufs.pool,
+        bufs.hidden, bufs.logits, bufs.probs,
+        bufs.pred, ctypes.addressof(bufs.which))
     return bufs
 
 
@@ -306,13 +313,13 @@ def s2v_forward_planned(plan, s_csr, X, W_n2l, W_conv, W_h1, W_h2, L, bufs=None)
         raise ValueError("weight shapes do not chain")
     if bufs is None:
         bufs = ForwardBuffers(N, B, C, H, Q, X.device)
-    check(_lib().gnnhip_s2v_forward_planned_f32(
-        plan.handle, B, K, C, H, Q, L,
-        _i32(s_csr[0], "s_row_ptr"), _i32(s_csr[1], "s_col_idx"), _f32(s_csr[2], "s_val"),
-        _f32(X, "X"), _f32(W_n2l, "W_n2l"), _f32(W_conv, "W_conv"), _f32(W_h1, "W_h1"), _f32(W_h2, "W_h2"),
-        _f32(bufs.msg, "msg"), _f32(bufs.h_a, "h_a"), _f32(bufs.h_b, "h_b"), _f32(bufs.pool, "pool"),
-        _f32(bufs.hidden, "hidden"), _f32(bufs.logits, "logits"), _f32(bufs.probs, "probs"),
-        _i32(bufs.pred, "pred"), ctypes.byref(bufs.which), _stream()))
+    _bound().s2v_forward_planned_f32(
+        plan.handle.value, B, K, C, H, Q, L,
+        s_csr[0], s_csr[1], s_csr[2],
+        X, W_n2l, W_conv, W_h1, W_h2,
+        bufs.msg, bufs.h_a, bufs.h_b, bufs.pool,
+        bufs.hidden, bufs.logits, bufs.probs,
+        bufs.pred, ctypes.addressof(bufs.which))
     return bufs
 
 
@@ -344,14 +351,14 @@ def s2v_forward_batched(a_csr, s_csr, X, W_n2l, W_conv, W_h1, W_h2, L, max_graph
         raise ValueError("weight shapes do not chain")
     if bufs is None:
         bufs = BatchedBuffers(N, B, C, H, Q, X.device)
-    check(_lib().gnnhip_s2v_forward_batched_f32(
+    _bound().s2v_forward_batched_f32(
         N, B, K, C, H, Q, L, int(max_graph_nodes),
-        _i32(a_csr[0], "a_row_ptr"), _i32(a_csr[1], "a_col_idx"), _f32(a_csr[2], "a_val"),
-        _i32(s_csr[0], "s_row_ptr"), _i32(s_csr[1], "s_col_idx"), _f32(s_csr[2], "s_val"),
-        _f32(X, "X"), _f32(W_n2l, "W_n2l"), _f32(W_conv, "W_conv"), _f32(W_h1, "W_h1"), _f32(W_h2, "W_h2"),
-        _f32(bufs.msg, "msg"), _f32(bufs.h_final, "h_final"), _f32(bufs.pool, "pool"),
-        _f32(bufs.hidden, "hidden"), _f32(bufs.logits, "logits"), _f32(bufs.probs, "probs"),
-        _i32(bufs.pred, "pred"), _i32(bufs.status, "status"), _stream()))
+        a_csr[0], a_csr[1], a_csr[2],
+        s_csr[0], s_csr[1], s_csr[2],
+        X, W_n2l, W_conv, W_h1, W_h2,
+        bufs.msg, bufs.h_final, bufs.pool,
+        bufs.hidden, bufs.logits, bufs.probs,
+        bufs.pred, bufs.status)
     return bufs
 
 
@@ -369,15 +376,15 @@ def s2v_forward_batched_train(a_csr, s_csr, X, W_n2l, W_conv, W_h1, W_h2, L, max
         raise ValueError("weight shapes do not chain")
     if bufs is None:
         bufs = BatchedBuffers(N, B, C, H, Q, X.device)
-    h_levels = torch.empty((L + 1, N, C), dtype=torch.float32, device=X.device)
-    check(_lib().gnnhip_s2v_forward_batched_train_f32(
+    h_levels = _empty(X, "f", L + 1, N, C)
+    _bound().s2v_forward_batched_train_f32(
         N, B, K, C, H, Q, L, int(max_graph_nodes),
-        _i32(a_csr[0], "a_row_ptr"), _i32(a_csr[1], "a_col_idx"), _f32(a_csr[2], "a_val"),
-        _i32(s_csr[0], "s_row_ptr"), _i32(s_csr[1], "s_col_idx"), _f32(s_csr[2], "s_val"),
-        _f32(X, "X"), _f32(W_n2l, "W_n2l"), _f32(W_conv, "W_conv"), _f32(W_h1, "W_h1"), _f32(W_h2, "W_h2"),
-        _f32(bufs.msg, "msg"), _f32(h_levels, "h_levels"), _f32(bufs.pool, "pool"),
-        _f32(bufs.hidden, "hidden"), _f32(bufs.logits, "logits"), _f32(bufs.probs, "probs"),
-        _i32(bufs.pred, "pred"), _i32(bufs.status, "status"), _stream()))
+        a_csr[0], a_csr[1], a_csr[2],
+        s_csr[0], s_csr[1], s_csr[2],
+        X, W_n2l, W_conv, W_h1, W_h2,
+        bufs.msg, h_levels, bufs.pool,
+        bufs.hidden, bufs.logits, bufs.probs,
+        bufs.pred, bufs.status)
     return bufs, h_levels
 
 
@@ -425,40 +432,40 @@ def s2v_forward_batched_labels(a_csr, s_csr, label, W_n2l, W_conv, W_h1, W_h2, L
         raise ValueError("weight shapes do not chain")
     if bufs is None:
         bufs = BatchedBuffers(N, B, C, H, Q, W_n2l.device)
-    check(_lib().gnnhip_s2v_forward_batched_labels_f32(
+    _bound().s2v_forward_batched_labels_f32(
         N, B, K, C, H, Q, L, int(max_graph_nodes),
-        _i32(a_csr[0], "a_row_ptr"), _i32(a_csr[1], "a_col_idx"), _f32(a_csr[2], "a_val"),
-        _i32(s_csr[0], "s_row_ptr"), _i32(s_csr[1], "s_col_idx"), _f32(s_csr[2], "s_val"),
-        _i32(label, "label"), _f32(W_n2l, "W_n2l"), _f32(W_conv, "W_conv"), _f32(W_h1, "W_h1"), _f32(W_h2, "W_h2"),
-        _f32(bufs.msg, "msg"), _f32(bufs.h_final, "h_final"), _f32(bufs.pool, "pool"),
-        _f32(bufs.hidden, "hidden"), _f32(bufs.logits, "logits"), _f32(bufs.probs, "probs"),
-        _i32(bufs.pred, "pred"), _i32(bufs.status, "status"), _stream()))
+        a_csr[0], a_csr[1], a_csr[2],
+        s_csr[0], s_csr[1], s_csr[2],
+        label, W_n2l, W_conv, W_h1, W_h2,
+        bufs.msg, bufs.h_final, bufs.pool,
+        bufs.hidden, bufs.logits, bufs.probs,
+        bufs.pred, bufs.status)
     return bufs
 
 
 def unary(op, x, a0=0.0, a1=0.0):
-    check(_lib().gnnhip_unary_f32(UNARY[op], _f32(x, "x"), x.numel(), a0, a1, _stream()))
+    _bound().unary_f32(UNARY[op], x, x.numel(), a0, a1)
     return x
 
 
 def relu(x, out=None):
     if out is None:
         out = torch.empty_like(x)
-    check(_lib().gnnhip_relu_f32(_f32(x, "x"), _f32(out, "out"), x.numel(), _stream()))
+    _bound().relu_f32(x, out, x.numel())
     return out
 
 
 def axpy(a, x, y):
     if x.numel() != y.numel():
         raise ValueError("shape doesn't match in Axpy")
-    check(_lib().gnnhip_axpy_f32(x.numel(), a, _f32(x, "x"), _f32(y, "y"), _stream()))
+    _bound().axpy_f32(x.numel(), a, x, y)
     return y
 
 
 def axpby(a, x, b, y):
     if x.numel() != y.numel():
         raise ValueError("shape doesn't match in Axpby")
-    check(_lib().gnnhip_axpby_f32(x.numel(), a, _f32(x, "x"), b, _f32(y, "y"), _stream()))
+    _bound().axpby_f32(x.numel(), a, x, b, y)
     return y
 
 
@@ -467,62 +474,61 @@ def add(a, b, out=None):
         raise ValueError("no broadcasting is supported")
     if out is None:
         out = torch.empty_like(a)
-    check(_lib().gnnhip_add_f32(a.numel(), _f32(a, "a"), _f32(b, "b"), _f32(out, "out"), _stream()))
+    _bound().add_f32(a.numel(), a, b, out)
     return out
 
 
 def row_softmax(x):
     rows, cols = x.shape
-    check(_lib().gnnhip_row_softmax_f32(_f32(x, "x"), rows, cols, _stream()))
+    _bound().row_softmax_f32(x, rows, cols)
     return x
 
 
 def jagged_softmax(x, lens):
-    check(_lib().gnnhip_jagged_softmax_f32(_f32(x, "x"), _i32(lens, "lens"), lens.numel(), _stream()))
+    _bound().jagged_softmax_f32(x, lens, lens.numel())
     return x
 
 
 def jagged_softmax_deriv(dst, out, grad, lens):
     """dst += (grad - <grad, out> per segment) * out"""
-    check(_lib().gnnhip_jagged_softmax_deriv_f32(_f32(dst, "dst"), _f32(out, "out"), _f32(grad, "grad"), _i32(lens, "lens"),
-                                                 lens.numel(), _stream()))
+    _bound().jagged_softmax_deriv_f32(dst, out, grad, lens,
+                                                 lens.numel())
     return dst
 
 
 def jagged_softmax_static(x, lens):
     """gnnhip_jagged_softmax_static_f32: the same result, segment offsets in the library's static array."""
-    check(_lib().gnnhip_jagged_softmax_static_f32(_f32(x, "x"), _i32(lens, "lens"), lens.numel(), _stream()))
+    _bound().jagged_softmax_static_f32(x, lens, lens.numel())
     return x
 
 
 def reduce(op, x):
-    out = torch.empty((1,), dtype=torch.float32, device=x.device)
-    check(_lib().gnnhip_reduce_f32(REDUCE[op], _f32(x, "x"), x.numel(), _f32(out, "out"), _stream()))
+    out = _empty(x, "f", 1)
+    _bound().reduce_f32(REDUCE[op], x, x.numel(), out)
     return out
 
 
 def row_argmax(x):
     rows, cols = x.shape
-    out = torch.empty((rows,), dtype=torch.int32, device=x.device)
-    check(_lib().gnnhip_row_argmax_f32(_f32(x, "x"), rows, cols, _i32(out, "out"), _stream()))
+    out = _empty(x, "i", rows)
+    _bound().row_argmax_f32(x, rows, cols, out)
     return out
 
 
 def csr_row_argmax(row_ptr, col_idx, val):
     rows = row_ptr.numel() - 1
-    out = torch.empty((rows,), dtype=torch.int32, device=row_ptr.device)
-    check(_lib().gnnhip_csr_row_argmax_f32(_i32(row_ptr, "row_ptr"), _i32(col_idx, "col_idx"), _f32(val, "val"),
-                                           rows, _i32(out, "out"), _stream()))
+    out = _empty(row_ptr, "i", rows)
+    _bound().csr_row_argmax_f32(row_ptr, col_idx, val,
+                                           rows, out)
     return out
 
 
 def cross_entropy(prob, l_row_ptr, l_col_idx, l_val):
     rows, cols = prob.shape
     _check_csr(l_row_ptr, l_col_idx, l_val, rows, "label")
-    out = torch.empty((rows, 1), dtype=torch.float32, device=prob.device)
-    check(_lib().gnnhip_cross_entropy_f32(_f32(prob, "prob"), rows, cols, _i32(l_row_ptr, "l_row_ptr"),
-                                          _i32(l_col_idx, "l_col_idx"), _f32(l_val, "l_val"), _f32(out, "out"),
-                                          _stream()))
+    out = _empty(prob, "f", rows, 1)
+    _bound().cross_entropy_f32(prob, rows, cols, l_row_ptr,
+                                          l_col_idx, l_val, out)
     return out
 
 
@@ -530,15 +536,14 @@ def in_top_k(pred, label, k=1):
     rows, cols = pred.shape
     if label.numel() != rows:
         raise ValueError("# instances doesn't match")
-    out = torch.empty((rows,), dtype=torch.int32, device=pred.device)
-    check(_lib().gnnhip_in_top_k_f32(_f32(pred, "pred"), _i32(label, "label"), rows, cols, k, _i32(out, "out"),
-                                     _stream()))
+    out = _empty(pred, "i", rows)
+    _bound().in_top_k_f32(pred, label, rows, cols, k, out)
     return out
 
 
 def cast_i32_f32(src):
     dst = torch.empty(src.shape, dtype=torch.float32, device=src.device)
-    check(_lib().gnnhip_cast_i32_f32(_i32(src, "src"), _f32(dst, "dst"), src.numel(), _stream()))
+    _bound().cast_i32_f32(src, dst, src.numel())
     return dst
 
 
@@ -565,30 +570,30 @@ def spmm_t(row_ptr, col_idx, val, B, m, k, alpha=1.0, beta=0.0, out=None):
         raise ValueError("mat dim doesn't match")
     if out is None:
         out = torch.zeros((k, n), dtype=torch.float32, device=B.device)
-    check(_lib().gnnhip_spmm_csr_t_f32(m, k, n, alpha, _i32(row_ptr, "row_ptr"), _i32(col_idx, "col_idx"),
-                                       _f32(val, "val"), _f32(B, "B"), n, beta, _f32(out, "out"), n, _stream()))
+    _bound().spmm_csr_t_f32(m, k, n, alpha, row_ptr, col_idx,
+                                       val, B, n, beta, out, n)
     return out
 
 
 def csr_axpy(a, row_ptr, col_idx, val, dense):
     rows, cols = dense.shape
     _check_csr(row_ptr, col_idx, val, rows, "x")
-    check(_lib().gnnhip_csr_axpy_f32(rows, cols, a, _i32(row_ptr, "row_ptr"), _i32(col_idx, "col_idx"), _f32(val, "val"),
-                                     _f32(dense, "dense"), _stream()))
+    _bound().csr_axpy_f32(rows, cols, a, row_ptr, col_idx, val,
+                                     dense)
     return dense
 
 
 def relu_deriv(dst, out, grad):
     if not (dst.numel() == out.numel() == grad.numel()):
         raise ValueError("shape mismatch in ReLUDeriv")
-    check(_lib().gnnhip_relu_deriv_f32(dst.numel(), _f32(out, "out"), _f32(grad, "grad"), _f32(dst, "dst"), _stream()))
+    _bound().relu_deriv_f32(dst.numel(), out, grad, dst)
     return dst
 
 
 def mul(x, y):
     if x.numel() != y.numel():
         raise ValueError("shape mismatch in ElewiseMul")
-    check(_lib().gnnhip_mul_f32(x.numel(), _f32(x, "x"), _f32(y, "y"), _stream()))
+    _bound().mul_f32(x.numel(), x, y)
     return y
 
 
@@ -596,7 +601,7 @@ def row_scale(scale, y):
     rows, cols = y.shape
     if scale.numel() != rows:
         raise ValueError("one factor per row is needed")
-    check(_lib().gnnhip_row_scale_f32(rows, cols, _f32(scale, "scale"), _f32(y, "y"), _stream()))
+    _bound().row_scale_f32(rows, cols, scale, y)
     return y
 
 
@@ -606,11 +611,11 @@ def csr_group(rows, key, payload, average=False, key_stride=1, payload_stride=1,
     if n is None:
         n = key.numel() // key_stride
     dev = key.device
-    row_ptr = torch.empty(rows + 1, dtype=torch.int32, device=dev)
-    col_idx = torch.empty(n, dtype=torch.int32, device=dev)
-    val = torch.empty(n, dtype=torch.float32, device=dev)
-    check(_lib().gnnhip_csr_group_i32(rows, n, _i32(key, "key"), key_stride, _i32(payload, "payload"), payload_stride,
-                                      int(average), _i32(row_ptr, "row_ptr"), _i32(col_idx, "col_idx"), _f32(val, "val"), _stream()))
+    row_ptr = _empty(dev, "i", rows + 1)
+    col_idx = _empty(dev, "i", n)
+    val = _empty(dev, "f", n)
+    _bound().csr_group_i32(rows, n, key, key_stride, payload, payload_stride,
+                                      int(average), row_ptr, col_idx, val)
     return row_ptr, col_idx, val
 
 
@@ -621,11 +626,11 @@ def csr_group_both(rows, x, y, x_stride=1, y_stride=1, n=None):
     dev = x.device
     out = []
     for _ in range(2):
-        out += [torch.empty(rows + 1, dtype=torch.int32, device=dev), torch.empty(n, dtype=torch.int32, device=dev),
-                torch.empty(n, dtype=torch.float32, device=dev)]
-    check(_lib().gnnhip_csr_group_both_i32(rows, n, _i32(x, "x"), x_stride, _i32(y, "y"), y_stride,
-                                           _i32(out[0], "row_ptr"), _i32(out[1], "col_idx"), _f32(out[2], "val"),
-                                           _i32(out[3], "t_row_ptr"), _i32(out[4], "t_col_idx"), _f32(out[5], "t_val"), _stream()))
+        out += [_empty(dev, "i", rows + 1), _empty(dev, "i", n),
+                _empty(dev, "f", n)]
+    _bound().csr_group_both_i32(rows, n, x, x_stride, y, y_stride,
+                                           out[0], out[1], out[2],
+                                           out[3], out[4], out[5])
     return tuple(out[:3]), tuple(out[3:])
 
 
@@ -633,10 +638,10 @@ def csr_consecutive_rows(row_ptr, average=False):
     """col_idx, val of the CSR matrix whose row i lists the columns row_ptr[i] .. row_ptr[i+1]-1 (row_ptr on the device)"""
     rows = row_ptr.numel() - 1
     n = int(row_ptr[-1].item())
-    col_idx = torch.empty(n, dtype=torch.int32, device=row_ptr.device)
-    val = torch.empty(n, dtype=torch.float32, device=row_ptr.device)
-    check(_lib().gnnhip_csr_consecutive_rows_f32(rows, _i32(row_ptr, "row_ptr"), int(average), _i32(col_idx, "col_idx"),
-                                                 _f32(val, "val"), _stream()))
+    col_idx = _empty(row_ptr, "i", n)
+    val = _empty(row_ptr, "f", n)
+    _bound().csr_consecutive_rows_f32(rows, row_ptr, int(average), col_idx,
+                                                 val)
     return col_idx, val
 
 
@@ -644,22 +649,23 @@ def csr_consecutive_rows_host(offsets, device, average=False):
     """(row_ptr, col_idx, val) on the device from the row offsets in a host int32 array"""
     offsets = np.ascontiguousarray(offsets, np.int32)
     rows, n = offsets.size - 1, int(offsets[-1])
-    row_ptr = torch.empty(rows + 1, dtype=torch.int32, device=device)
-    col_idx = torch.empty(n, dtype=torch.int32, device=device)
-    val = torch.empty(n, dtype=torch.float32, device=device)
-    check(_lib().gnnhip_csr_consecutive_rows_host_f32(rows, ctypes.c_void_p(offsets.ctypes.data), int(average), _i32(row_ptr, "row_ptr"),
-                                                      _i32(col_idx, "col_idx") if n else None, _f32(val, "val") if n else None, _stream()))
+    device = torch.device(device)
+    row_ptr = _empty(device, "i", rows + 1)
+    col_idx = _empty(device, "i", n)
+    val = _empty(device, "f", n)
+    _bound().csr_consecutive_rows_host_f32(rows, offsets.__array_interface__["data"][0], int(average), row_ptr,
+                                                      col_idx if n else None, val if n else None)
     return row_ptr, col_idx, val
 
 
 def csr_transpose(row_ptr, col_idx, val, m, k):
     nnz = col_idx.numel()
     dev = row_ptr.device
-    t_rp = torch.empty(k + 1, dtype=torch.int32, device=dev)
-    t_ci = torch.empty(nnz, dtype=torch.int32, device=dev)
-    t_v = torch.empty(nnz, dtype=torch.float32, device=dev)
-    check(_lib().gnnhip_csr_transpose_f32(m, k, nnz, _i32(row_ptr, "row_ptr"), _i32(col_idx, "col_idx"), _f32(val, "val"),
-                                          _i32(t_rp, "t_row_ptr"), _i32(t_ci, "t_col_idx"), _f32(t_v, "t_val"), _stream()))
+    t_rp = _empty(dev, "i", k + 1)
+    t_ci = _empty(dev, "i", nnz)
+    t_v = _empty(dev, "f", nnz)
+    _bound().csr_transpose_f32(m, k, nnz, row_ptr, col_idx, val,
+                                          t_rp, t_ci, t_v)
     return t_rp, t_ci, t_v
 
 
@@ -668,14 +674,14 @@ def loss_acc(logits, lrow_ptr, lcol, lval, want_rows=False):
     """mean cross-entropy (softmax inside) and mean top-1 accuracy of a batch in one pass over the logits"""
     B, Q = logits.shape
     dev = logits.device
-    probs = torch.empty_like(logits)
-    loss = torch.empty((1,), dtype=torch.float32, device=dev)
-    acc = torch.empty((1,), dtype=torch.float32, device=dev)
-    loss_rows = torch.empty((B,), dtype=torch.float32, device=dev) if want_rows else None
-    hit = torch.empty((B,), dtype=torch.int32, device=dev) if want_rows else None
-    check(_lib().gnnhip_s2v_loss_acc_f32(B, Q, _f32(logits, "logits"), _i32(lrow_ptr, "lrow_ptr"), _i32(lcol, "lcol"),
-                                         _f32(lval, "lval"), _f32(probs, "probs"), _f32(loss_rows, "loss_rows"),
-                                         _i32(hit, "hit"), _f32(loss, "loss"), _f32(acc, "acc"), _stream()))
+    probs = _empty(logits, "f", B, Q)
+    loss = _empty(dev, "f", 1)
+    acc = _empty(dev, "f", 1)
+    loss_rows = _empty(dev, "f", B) if want_rows else None
+    hit = _empty(dev, "i", B) if want_rows else None
+    _bound().s2v_loss_acc_f32(B, Q, logits, lrow_ptr, lcol,
+                                         lval, probs, loss_rows,
+                                         hit, loss, acc)
     return loss, acc, probs, loss_rows, hit
 
 
@@ -683,14 +689,14 @@ def readout_backward(s_csr, probs, label_csr, scale, hidden, W_h1, W_h2, N):
     B, Q = probs.shape
     C, H = W_h1.shape
     dev = probs.device
-    dlogits = torch.empty((B, Q), dtype=torch.float32, device=dev)
-    du = torch.empty((B, H), dtype=torch.float32, device=dev)
-    g_h = torch.empty((N, C), dtype=torch.float32, device=dev)
-    check(_lib().gnnhip_s2v_readout_backward_f32(
-        B, N, C, H, Q, _i32(s_csr[0], "s_row_ptr"), _i32(s_csr[1], "s_col_idx"), _f32(s_csr[2], "s_val"),
-        _f32(probs, "probs"), _i32(label_csr[0], "lrow_ptr"), _i32(label_csr[1], "lcol"), _f32(label_csr[2], "lval"),
-        float(scale), _f32(hidden, "hidden"), _f32(W_h1, "W_h1"), _f32(W_h2, "W_h2"),
-        _f32(dlogits, "dlogits"), _f32(du, "du"), _f32(g_h, "g_h"), _stream()))
+    dlogits = _empty(dev, "f", B, Q)
+    du = _empty(dev, "f", B, H)
+    g_h = _empty(dev, "f", N, C)
+    _bound().s2v_readout_backward_f32(
+        B, N, C, H, Q, s_csr[0], s_csr[1], s_csr[2],
+        probs, label_csr[0], label_csr[1], label_csr[2],
+        float(scale), hidden, W_h1, W_h2,
+        dlogits, du, g_h)
     return dlogits, du, g_h
 
 
@@ -700,44 +706,30 @@ def s2v_level_backward(t_row_ptr, t_col_idx, t_val, dz, W, u=None, g_prev=None, 
     N, C = dz.shape
     _check_csr(t_row_ptr, t_col_idx, t_val, N, "A^T")
     if u is None:
-        u = torch.empty_like(dz)
+        u = _empty(dz, "f", N, C)
     if g_prev is None:
-        g_prev = torch.empty_like(dz)
-    check(_lib().gnnhip_s2v_level_backward_f32(N, C, int(t_col_idx.numel()), _i32(t_row_ptr, "t_row_ptr"), _i32(t_col_idx, "t_col_idx"),
-                                               _f32(t_val, "t_val"), _f32(dz, "dz"), _f32(W, "W"), _f32(u, "u"), _f32(g_prev, "g_prev"),
-                                               _f32(gate_h, "gate_h"), _f32(acc, "acc"), _stream()))
+        g_prev = _empty(dz, "f", N, C)
+    _bound().s2v_level_backward_f32(N, C, int(t_col_idx.numel()), t_row_ptr, t_col_idx,
+                                               t_val, dz, W, u, g_prev,
+                                               gate_h, acc)
     return u, g_prev
 
 
 def grad_gate(h, g, dz=None, acc=None, accumulate=False):
-    check(_lib().gnnhip_s2v_grad_gate_f32(h.numel(), _f32(h, "h"), _f32(g, "g"), _f32(dz, "dz"), _f32(acc, "acc"),
-                                          1 if accumulate else 0, _stream()))
+    _bound().s2v_grad_gate_f32(h.numel(), h, g, dz, acc,
+                                          1 if accumulate else 0)
 
 
 def momentum_sgd_batch(ws, gs, vs, lr, momentum, l2):
-    n = len(ws)
-    P = ctypes.c_void_p * n
-    Z = ctypes.c_size_t * n
-    wp, gp = P(*[t.data_ptr() for t in ws]), P(*[t.data_ptr() for t in gs])
-    vp = P(*[t.data_ptr() for t in vs]) if vs is not None else None
-    for t in list(ws) + list(gs) + (list(vs) if vs is not None else []):
-        _f32(t, "tensor")
-    cnt = Z(*[t.numel() for t in ws])
-    check(_lib().gnnhip_momentum_sgd_batch_f32(n, wp, gp, vp, cnt, float(lr), float(momentum), float(l2), _stream()))
+    _bound().momentum_sgd_batch(list(ws), list(gs), list(vs) if vs is not None else None, float(lr), float(momentum), float(l2))
 
 
 def adam_batch(ws, gs, ms, vs, lr, l2, clip_threshold, beta1, beta2, eps, t):
     """one AdamOptimizer::Update over the tensors, t = the iteration count after the increment (1 for the first)"""
-    n = len(ws)
-    P = ctypes.c_void_p * n
-    Z = ctypes.c_size_t * n
-    for x in list(ws) + list(gs) + list(ms) + list(vs):
-        _f32(x, "tensor")
-    ptr = lambda ts: P(*[x.data_ptr() for x in ts])
     s1 = np.float32(1.0 / (1 - float(np.float32(beta1)) ** t))
     s2 = np.float32(1.0 / (1 - float(np.float32(beta2)) ** t))
-    check(_lib().gnnhip_adam_batch_f32(n, ptr(ws), ptr(gs), ptr(ms), ptr(vs), Z(*[x.numel() for x in ws]), float(lr), float(l2),
-                                       float(clip_threshold), float(beta1), float(beta2), float(eps), float(s1), float(s2), _stream()))
+    _bound().adam_batch(list(ws), list(gs), list(ms), list(vs), float(lr), float(l2), float(clip_threshold), float(beta1), float(beta2),
+                        float(eps), float(s1), float(s2))
 
 
 def upload_sparse32(host_array, out=None):
