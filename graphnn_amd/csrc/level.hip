@@ -47,7 +47,11 @@ int level_wide_dispatch(int N, int C, long long nnz, const int* row_ptr, const i
                         const float* h_in, const float* W, const float* msg, const float* bias, float* h_out, bool relu_in,
                         hipStream_t s);
 bool level_wide_covers(int N, int C);
-int level_wide_backward_dispatch(int N, int C, const int* row_ptr, const int* col_idx, const float* val, const float* dz, const float* W,
+// level_wide_split.hip
+int level_split_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val,
+                         const float* h_in, const float* W, const float* msg, const float* bias, float* h_out, bool relu_in,
+                         hipStream_t s);
+int level_split_backward_dispatch(int N, int C, const int* row_ptr, const int* col_idx, const float* val, const float* dz, const float* W,
                                  float* u, float* g_prev, const float* gate, float* acc, hipStream_t s);
 
 namespace {
@@ -607,8 +611,10 @@ __global__ __launch_bounds__(kBlock) void identity_csr_kernel(int n, int* __rest
 
 int level_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* h_in,
                    const float* W, const float* msg, const float* bias, float* h_out, hipStream_t s, bool same_graph,
-                   bool relu_in, CsrPlan* plan)
+                   bool relu_in, CsrPlan* plan, bool inference)
 {
+    // inference: no gradient passes through the result, so its contraction may be rounded differently from the
+    // contraction whose signs a backward pass relies on (level_wide_split.hip)
     // plan: made by gnnhip_csr_plan_create for exactly these CSR arrays (then nnz is the matrix's own count), or null
     // relu_in: h_in is read as ReLU(h_in); only where level_accepts_relu_input says so
     // same_graph: the previous call on this stream had the same A (a later level of one forward), so the
@@ -655,6 +661,7 @@ int level_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* c
         }
     }
     if (!level_wide_covers(N, C)) return GNNHIP_EUNSUPPORTED;
+    const auto wide = inference ? level_split_dispatch : level_wide_dispatch;
     // The wide kernel sums a row of any length inside one wavefront.  Large graphs with many entries per row
     // (in practice the skewed ones, see above) take two steps: the SpMM, which balances long rows, leaves A * h_in
     // in scratch, and the wide kernel reads those rows through the identity matrix (one entry per row: its
@@ -673,9 +680,9 @@ int level_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* c
         hipLaunchKernelGGL(identity_csr_kernel, dim3((unsigned)(((long long)N + kBlock) / kBlock)), dim3(kBlock), 0, s, N, id_row_ptr,
                            id_col, id_val);
         GNNHIP_LAUNCH_CHECK("identity_csr");
-        return level_wide_dispatch(N, C, N, id_row_ptr, id_col, id_val, agg, W, msg, bias, h_out, false, s);
+        return wide(N, C, N, id_row_ptr, id_col, id_val, agg, W, msg, bias, h_out, false, s);
     }
-    return level_wide_dispatch(N, C, nnz, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, relu_in, s);
+    return wide(N, C, nnz, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, relu_in, s);
 }
 
 // u = A' dz and g_prev = u W^T in one pass (A' = the transposed adjacency in CSR form); GNNHIP_EUNSUPPORTED where
@@ -690,7 +697,7 @@ int level_backward_dispatch(int N, int C, long long nnz, const int* row_ptr, con
         if (N >= kHubMinRows && nnz >= two_step_degree() * (long long)N) return GNNHIP_EUNSUPPORTED;
         if (!(aligned16(dz) && aligned16(W) && aligned16(u) && aligned16(g_prev) && (!gate || aligned16(gate)) && (!acc || aligned16(acc))))
             return GNNHIP_EUNSUPPORTED;
-        return level_wide_backward_dispatch(N, C, row_ptr, col_idx, val, dz, W, u, g_prev, gate, acc, s);
+        return level_split_backward_dispatch(N, C, row_ptr, col_idx, val, dz, W, u, g_prev, gate, acc, s);
     }
     if (!(C == 16 || C == 32 || C == 64) || !level_stream_covers(N, C)) return GNNHIP_EUNSUPPORTED;
     if (!(aligned16(dz) && aligned16(W) && aligned16(u) && aligned16(g_prev) && (!gate || aligned16(gate)) && (!acc || aligned16(acc))))

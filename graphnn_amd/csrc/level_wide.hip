@@ -8,6 +8,9 @@
 // contraction takes about twice as long as the HBM traffic, so this kernel is
 // organised around keeping the matrix pipes fed.
 //
+// This kernel forms the levels of a training forward (and the level entries); level_wide_split.hip does inference and
+// the backward pass on the bf16 matrix cores and says why the two are kept apart.
+//
 // One persistent workgroup of 8 wavefronts per compute unit.  W never moves
 // after start-up: wavefront w keeps the W^T operand of its C/8 output columns
 // in registers (C = 256: 128 registers per lane, half of the register file of
@@ -45,8 +48,7 @@
 //     conditions; the compiler then assumes a path on which loads are still in
 //     flight and waits at the top of the next block.  One explicit wait after
 //     the contraction removes that.
-#include "gnnhip_internal.h"
-#include "buffer_addr.h"
+#include "level_wide.h"
 
 // Phase accounting for a timing build of this file; expands to nothing in the library.
 #ifndef GNNHIP_PHASE_ACC
@@ -59,68 +61,6 @@
 namespace gnnhip {
 namespace {
 
-constexpr int kInFlight = 6;                     // row gathers in flight per wavefront
-constexpr int kWaitVmcnt0 = 0x0F70;              // s_waitcnt operand: vmcnt(0), other counters unconstrained
-
-template <int VEC> struct VecT;
-template <> struct VecT<2> { using type = float2; };
-template <> struct VecT<4> { using type = float4; };
-
-// Buffer addressing (buffer_addr.h): the memory instruction takes a 128-bit descriptor (base, size), a
-// per-lane 32-bit offset and a scalar 32-bit offset, so a gathered row costs one scalar shift and no
-// per-lane address arithmetic, and lanes whose offset lies past the size are dropped by the hardware.
-template <int VEC> struct BufLoad;
-template <> struct BufLoad<4> { static __device__ __forceinline__ float4 get(rsrc_t r, int v, int s) { return buf_load4(r, v, s); } };
-template <> struct BufLoad<2> { static __device__ __forceinline__ float2 get(rsrc_t r, int v, int s) { return buf_load2(r, v, s); } };
-template <int VEC> struct BufStore;
-template <> struct BufStore<4> { static __device__ __forceinline__ void put(rsrc_t r, int v, int s, const float4& x) { buf_store4(r, v, s, x); } };
-template <> struct BufStore<2> { static __device__ __forceinline__ void put(rsrc_t r, int v, int s, const float2& x) { buf_store2(r, v, s, x); } };
-
-// A batch of kInFlight consecutive entries of a CSR array (column indices, or edge weights as bit
-// patterns) in scalar registers.  The two scalar loads are written as inline assembly with the batch as a
-// read-write operand: the loaded values land in the registers the batch already occupies, so a batch that
-// is (conditionally) refilled inside the loop needs no copy of the loaded values, and with it no wait for
-// the scalar cache right behind the load.  The compiler does not know that these registers are in flight:
-// batch_wait() must run before a batch is read.
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-typedef int i32x2 __attribute__((ext_vector_type(2)));
-struct Batch { i32x4 lo; i32x2 hi; };
-static_assert(kInFlight == 6, "a batch is one 4-dword and one 2-dword scalar load");
-__device__ __forceinline__ void batch_load(Batch& b, const int* p)
-{
-    asm volatile("s_load_dwordx4 %0, %2, 0x0\n\ts_load_dwordx2 %1, %2, 0x10" : "+s"(b.lo), "+s"(b.hi) : "s"(p));
-}
-// The first n < kInFlight entries of an array that holds no more than n, zeros behind them: one scalar load
-// per entry, each under its own (uniform) condition, and the wait right here.
-__device__ __forceinline__ void batch_load_short(Batch& b, const int* p, int n)
-{
-    int t0 = 0, t1 = 0, t2 = 0, t3 = 0, t4 = 0;
-    if (n > 0) asm volatile("s_load_dword %0, %1, 0x0" : "+s"(t0) : "s"(p));
-    if (n > 1) asm volatile("s_load_dword %0, %1, 0x4" : "+s"(t1) : "s"(p));
-    if (n > 2) asm volatile("s_load_dword %0, %1, 0x8" : "+s"(t2) : "s"(p));
-    if (n > 3) asm volatile("s_load_dword %0, %1, 0xc" : "+s"(t3) : "s"(p));
-    if (n > 4) asm volatile("s_load_dword %0, %1, 0x10" : "+s"(t4) : "s"(p));
-    asm volatile("s_waitcnt lgkmcnt(0)" : "+s"(t0), "+s"(t1), "+s"(t2), "+s"(t3), "+s"(t4));
-    b.lo.x = t0; b.lo.y = t1; b.lo.z = t2; b.lo.w = t3;
-    b.hi.x = t4; b.hi.y = 0;
-}
-__device__ __forceinline__ void batch_wait(Batch& b)
-{
-    asm volatile("s_waitcnt lgkmcnt(0)" : "+s"(b.lo), "+s"(b.hi));
-}
-__device__ __forceinline__ int batch_get(const Batch& b, int u)      // u is a compile-time constant after unrolling
-{
-    return u == 0 ? b.lo.x : u == 1 ? b.lo.y : u == 2 ? b.lo.z : u == 3 ? b.lo.w : u == 4 ? b.hi.x : b.hi.y;
-}
-
-template <int VEC, bool RELU_IN>
-__device__ __forceinline__ void vec_fma(float (&acc)[VEC], float a, const typename VecT<VEC>::type& x)
-{
-    const float* p = reinterpret_cast<const float*>(&x);
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) acc[i] = fmaf(a, RELU_IN ? relu_ref(p[i]) : p[i], acc[i]);
-}
-
 // Everything that steers the gather (row pointers, column indices, edge weights) is uniform
 // across the wavefront and is fetched with scalar loads: the values land in scalar registers, cost
 // no vector instruction to broadcast, and are counted apart from vector memory operations, so
@@ -129,17 +69,11 @@ __device__ __forceinline__ void vec_fma(float (&acc)[VEC], float a, const typena
 // either wavefront of a SIMD takes time away from its matrix pipe.
 // RELU_IN: the gathered rows count as ReLU(row) (the first level reading msg where h0 was not stored)
 // TR: rows per pass (16, 32 or 64)
-// BWD: the backward pass of a level through the same machinery.  The CSR arrays are those of A^T, h_in is dz, the
-//      summed rows u = A^T dz are also stored to u_out as each one is finished (they are the other factor of the
-//      weight gradient), the contraction takes W transposed (g = u W^T), and the epilogue, instead of adding msg and
-//      applying ReLU, lets g through where the rows of `msg` (here: the embedding whose ReLU the gradient passes next,
-//      or null for no gate) are positive and adds what it stores to acc_io (or null).
-template <int C, int WAVES, bool RELU_IN, int TR, bool BWD = false>
+template <int C, int WAVES, bool RELU_IN, int TR>
 __global__ __launch_bounds__(WAVES * kWave) void s2v_level_wide_kernel(
     int N, int tiles_per_block, const int* __restrict__ row_ptr, const int* __restrict__ col_idx,
     const float* __restrict__ val, const float* __restrict__ h_in, const float* __restrict__ W,
-    const float* __restrict__ msg, const float* __restrict__ bias, float* __restrict__ h_out,
-    float* __restrict__ u_out, float* __restrict__ acc_io)
+    const float* __restrict__ msg, const float* __restrict__ bias, float* __restrict__ h_out)
 {
     constexpr int KS = C / 4;                    // contraction steps
     constexpr int kWideBlock = WAVES * kWave;
@@ -162,29 +96,17 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_wide_kernel(
     if (bias)
         for (int i = threadIdx.x; i < C; i += kWideBlock) bias_lds[i] = bias[i];
 
-    // W^T operand: wreg[jb][s] = W[KS q + s][col0 + 16 jb + t]; BWD: W itself, wreg[jb][s] = W[col0 + 16 jb + t][KS q + s]
+    // W^T operand: wreg[jb][s] = W[KS q + s][col0 + 16 jb + t]
     // (buffer loads: one lane offset, the steps as scalar offsets, so no 64-bit address per element is formed)
     float wreg[NB][KS];
     {
         const rsrc_t w_rsrc = make_rsrc(W, (unsigned)(C * C * 4));
-        const int w_lane_off = BWD ? ((col0 + t) * C + KS * q) * 4 : ((KS * q) * C + col0 + t) * 4;
-        if constexpr (BWD) {
-            // a lane's steps are consecutive floats of one row of W: 128-bit loads (with one float per load, lanes
-            // 1 KB apart, the start-up of a launch on 7,450 rows took longer than its passes)
+        const int w_lane_off = ((KS * q) * C + col0 + t) * 4;
 #pragma unroll
-            for (int jb = 0; jb < NB; ++jb)
+        for (int jb = 0; jb < NB; ++jb)
 #pragma unroll
-                for (int s4 = 0; s4 < KS / 4; ++s4) {
-                    const float4 v = buf_load4(w_rsrc, w_lane_off + 16 * C * 4 * jb, s4 * 16);
-                    wreg[jb][4 * s4 + 0] = v.x; wreg[jb][4 * s4 + 1] = v.y; wreg[jb][4 * s4 + 2] = v.z; wreg[jb][4 * s4 + 3] = v.w;
-                }
-        } else {
-#pragma unroll
-            for (int jb = 0; jb < NB; ++jb)
-#pragma unroll
-                for (int s = 0; s < KS; ++s)
-                    wreg[jb][s] = buf_load_f(w_rsrc, w_lane_off + 64 * jb, s * (C * 4));
-        }
+            for (int s = 0; s < KS; ++s)
+                wreg[jb][s] = buf_load_f(w_rsrc, w_lane_off + 64 * jb, s * (C * 4));
     }
 
     const int ntiles = (int)(((long long)N + kTileRows - 1) / kTileRows);
@@ -235,24 +157,16 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_wide_kernel(
     int e = 0, ee = 0, lr = 0, row_end = 0, rpv = 0;
     float* dstp = nullptr;
     float acc[VEC];
-    rsrc_t u_rsrc = make_rsrc(u_out, 0);         // BWD: the rows of u_out that the pass being gathered covers
-    auto begin = [&](int rp_lanes, int eb, int eend, float* dst, int tile_id) {
+    auto begin = [&](int rp_lanes, int eb, int eend, float* dst) {
         rpv = rp_lanes;
         e = eb; ee = eend; lr = 0;
         row_end = __builtin_amdgcn_readlane(rpv, 1);
         dstp = dst;
 #pragma unroll
         for (int i = 0; i < VEC; ++i) acc[i] = 0.f;
-        if constexpr (BWD) {
-            const long long r0 = (long long)tile_id * kTileRows;
-            const long long rows = max(min((long long)N - r0, (long long)kTileRows), 0ll);      // none past the last pass
-            u_rsrc = make_rsrc(u_out + (size_t)min(r0, (long long)N) * C, (unsigned)(rows * (C * 4)));
-        }
     };
     auto flush_row = [&]() {
         *reinterpret_cast<vec_t*>(dstp) = *reinterpret_cast<vec_t*>(acc);
-        if constexpr (BWD)                        // rows past N lie outside the descriptor
-            BufStore<VEC>::put(u_rsrc, lane * (VEC * 4), (wave * RPW + lr) * (C * 4), *reinterpret_cast<vec_t*>(acc));
 #pragma unroll
         for (int i = 0; i < VEC; ++i) acc[i] = 0.f;
         dstp += LDT;
@@ -280,7 +194,7 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_wide_kernel(
 #pragma unroll
     for (int jb = 0; jb < NB; ++jb) outv[jb] = f4_zero();
     const int lane_off = (t * C + col0 + 4 * q) * 4;              // byte offset of this lane inside a 16-row block
-    rsrc_t msg_rsrc = make_rsrc(msg, 0), out_rsrc = make_rsrc(h_out, 0), acc_rsrc = make_rsrc(acc_io, 0);
+    rsrc_t msg_rsrc = make_rsrc(msg, 0), out_rsrc = make_rsrc(h_out, 0);
     auto store_pending = [&]() {
         if (out_rt >= 0) {
 #pragma unroll
@@ -298,7 +212,7 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_wide_kernel(
     // ---- first pass: its gather has nothing to hide behind
     int rp_next = load_rowptrs(tile_begin);      // row pointers of the next pass to gather
     int ebN = __builtin_amdgcn_readlane(rp_next, 0), eeN = __builtin_amdgcn_readlane(rp_next, RPW);
-    begin(rp_next, ebN, eeN, tiles + gather_off, tile_begin);
+    begin(rp_next, ebN, eeN, tiles + gather_off);
     while (e < ee) {
         vec_t x[kInFlight];
         cShift = load_batch(col_idx, e, cC);
@@ -325,13 +239,12 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_wide_kernel(
         const float* cur = tiles + parity * (kTileRows * LDT);
         const bool has_next = tile_id + 1 < tile_end;
         const bool has_next2 = tile_id + 2 < tile_end;
-        begin(rp_next, ebN, eeN, tiles + (parity ^ 1) * (kTileRows * LDT) + gather_off, tile_id + 1);   // empty when !has_next
+        begin(rp_next, ebN, eeN, tiles + (parity ^ 1) * (kTileRows * LDT) + gather_off);   // empty when !has_next
         {
             const long long left = (long long)N - row0;
             const unsigned bytes = (unsigned)(min(left, (long long)kTileRows) * (C * 4));
             out_rsrc = make_rsrc(h_out + (size_t)row0 * C, bytes);
             msg_rsrc = make_rsrc(msg ? msg + (size_t)row0 * C : nullptr, msg ? bytes : 0u);   // no msg: every load reads 0
-            if constexpr (BWD) acc_rsrc = make_rsrc(acc_io ? acc_io + (size_t)row0 * C : nullptr, acc_io ? bytes : 0u);
         }
         if (has_next2) rp_next = load_rowptrs(tile_id + 2);
 
@@ -341,18 +254,12 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_wide_kernel(
         for (int rt = 0; rt < kTileRows / 16; ++rt) {
             // msg is asked for now and added after the contraction (as the accumulators' initial value it
             // would have to arrive before the first matrix instruction)
-            float4 mm[NB], aa[BWD ? NB : 1];
+            float4 mm[NB];
             mfma_f4 acc_m[NB];
 #pragma unroll
             for (int jb = 0; jb < NB; ++jb) {
                 mm[jb] = buf_load4(msg_rsrc, lane_off + rt * (16 * C * 4) + 64 * jb, 0);
                 acc_m[jb] = mfma_f4{0.f, 0.f, 0.f, 0.f};
-            }
-            if constexpr (BWD) {
-                if (acc_io) {
-#pragma unroll
-                    for (int jb = 0; jb < NB; ++jb) aa[jb] = buf_load4(acc_rsrc, lane_off + rt * (16 * C * 4) + 64 * jb, 0);
-                }
             }
             vec_t x[kInFlight];
             const bool batch = e < ee;
@@ -416,34 +323,18 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_wide_kernel(
                 }
             }
             GNNHIP_PHASE_ACC(3);
-            if constexpr (BWD) {
 #pragma unroll
-                for (int jb = 0; jb < NB; ++jb) {
-                    float4 v = make_float4(acc_m[jb][0], acc_m[jb][1], acc_m[jb][2], acc_m[jb][3]);
-                    if (msg) {                   // past the ReLU whose output these rows are
-                        v.x = mm[jb].x > 0.f ? v.x : 0.f; v.y = mm[jb].y > 0.f ? v.y : 0.f;
-                        v.z = mm[jb].z > 0.f ? v.z : 0.f; v.w = mm[jb].w > 0.f ? v.w : 0.f;
-                    }
-                    if (acc_io) {                // every row belongs to one pass: nobody else touches it during the launch
-                        const float4 a = make_float4(aa[jb].x + v.x, aa[jb].y + v.y, aa[jb].z + v.z, aa[jb].w + v.w);
-                        buf_store4(acc_rsrc, lane_off + rt * (16 * C * 4) + 64 * jb, 0, a);
-                    }
-                    outv[jb] = v;
-                }
-            } else {
+            for (int jb = 0; jb < NB; ++jb) {
+                acc_m[jb][0] += mm[jb].x; acc_m[jb][1] += mm[jb].y; acc_m[jb][2] += mm[jb].z; acc_m[jb][3] += mm[jb].w;
+            }
 #pragma unroll
-                for (int jb = 0; jb < NB; ++jb) {
-                    acc_m[jb][0] += mm[jb].x; acc_m[jb][1] += mm[jb].y; acc_m[jb][2] += mm[jb].z; acc_m[jb][3] += mm[jb].w;
+            for (int jb = 0; jb < NB; ++jb) {
+                float4 v = make_float4(acc_m[jb][0], acc_m[jb][1], acc_m[jb][2], acc_m[jb][3]);
+                if (bias) {
+                    const float4 b4 = *reinterpret_cast<const float4*>(bias_lds + col0 + 16 * jb + 4 * q);
+                    v.x += b4.x; v.y += b4.y; v.z += b4.z; v.w += b4.w;
                 }
-#pragma unroll
-                for (int jb = 0; jb < NB; ++jb) {
-                    float4 v = make_float4(acc_m[jb][0], acc_m[jb][1], acc_m[jb][2], acc_m[jb][3]);
-                    if (bias) {
-                        const float4 b4 = *reinterpret_cast<const float4*>(bias_lds + col0 + 16 * jb + 4 * q);
-                        v.x += b4.x; v.y += b4.y; v.z += b4.z; v.w += b4.w;
-                    }
-                    outv[jb] = make_float4(relu_ref(v.x), relu_ref(v.y), relu_ref(v.z), relu_ref(v.w));
-                }
+                outv[jb] = make_float4(relu_ref(v.x), relu_ref(v.y), relu_ref(v.z), relu_ref(v.w));
             }
             out_rt = rt;
             GNNHIP_PHASE_ACC(4);
@@ -469,10 +360,9 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_wide_kernel(
     GNNHIP_PHASE_FINI
 }
 
-template <int C, int WAVES, bool RELU_IN, int TR, bool BWD = false>
+template <int C, int WAVES, bool RELU_IN, int TR>
 int launch_level_wide_t(int N, const int* row_ptr, const int* col_idx, const float* val, const float* h_in,
-                      const float* W, const float* msg, const float* bias, float* h_out, hipStream_t s,
-                      float* u_out = nullptr, float* acc_io = nullptr)
+                      const float* W, const float* msg, const float* bias, float* h_out, hipStream_t s)
 {
     if ((unsigned long long)N * C * 4ull >= (1ull << 32)) return GNNHIP_EUNSUPPORTED;   // 32-bit buffer offsets
     constexpr int kTileRows = TR;
@@ -484,10 +374,10 @@ int launch_level_wide_t(int N, const int* row_ptr, const int* col_idx, const flo
     const long long blocks = (ntiles + per - 1) / per;
     const size_t smem = sizeof(float) * (2 * kTileRows * (C + 4) + C);
     static LdsLimit lds_limit;                                       // one per kernel instantiation
-    GNNHIP_HIP(lds_limit.raise(reinterpret_cast<const void*>(&s2v_level_wide_kernel<C, WAVES, RELU_IN, TR, BWD>), smem));
-    hipLaunchKernelGGL((s2v_level_wide_kernel<C, WAVES, RELU_IN, TR, BWD>), dim3((unsigned)blocks), dim3(WAVES * kWave), smem, s,
-                       N, (int)per, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, u_out, acc_io);
-    GNNHIP_LAUNCH_CHECK(BWD ? "s2v_level_wide backward" : "s2v_level_wide");
+    GNNHIP_HIP(lds_limit.raise(reinterpret_cast<const void*>(&s2v_level_wide_kernel<C, WAVES, RELU_IN, TR>), smem));
+    hipLaunchKernelGGL((s2v_level_wide_kernel<C, WAVES, RELU_IN, TR>), dim3((unsigned)blocks), dim3(WAVES * kWave), smem, s,
+                       N, (int)per, row_ptr, col_idx, val, h_in, W, msg, bias, h_out);
+    GNNHIP_LAUNCH_CHECK("s2v_level_wide");
     return GNNHIP_OK;
 }
 
@@ -501,17 +391,6 @@ int launch_level_wide(int N, const int* row_ptr, const int* col_idx, const float
     if (N >= 2 * kSlots * 64) return launch_level_wide_t<C, WAVES, RELU_IN, 64>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, s);
     if (N >= 2 * kSlots * 32) return launch_level_wide_t<C, WAVES, RELU_IN, 32>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, s);
     return launch_level_wide_t<C, WAVES, RELU_IN, 16>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, s);
-}
-
-// The backward pass: same choice of rows per pass.
-template <int C, int WAVES>
-int launch_level_wide_backward(int N, const int* row_ptr, const int* col_idx, const float* val, const float* dz, const float* W,
-                               float* u, float* g_prev, const float* gate, float* acc, hipStream_t s)
-{
-    constexpr int kSlots = kNumCU * ((C == 128) ? 2 : 1);
-    if (N >= 2 * kSlots * 64) return launch_level_wide_t<C, WAVES, false, 64, true>(N, row_ptr, col_idx, val, dz, W, gate, nullptr, g_prev, s, u, acc);
-    if (N >= 2 * kSlots * 32) return launch_level_wide_t<C, WAVES, false, 32, true>(N, row_ptr, col_idx, val, dz, W, gate, nullptr, g_prev, s, u, acc);
-    return launch_level_wide_t<C, WAVES, false, 16, true>(N, row_ptr, col_idx, val, dz, W, gate, nullptr, g_prev, s, u, acc);
 }
 
 }  // namespace
@@ -534,18 +413,6 @@ int level_wide_dispatch(int N, int C, long long nnz, const int* row_ptr, const i
     case 256:
         return relu_in ? launch_level_wide<256, 8, true>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, s)
                        : launch_level_wide<256, 8, false>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, s);
-    }
-    return GNNHIP_EUNSUPPORTED;
-}
-
-// u = A' dz (stored) and g_prev = u W^T past the gate of `gate` (may be null), added to acc (may be null): the wide
-// kernel's backward variant over the CSR arrays of A' = A^T.
-int level_wide_backward_dispatch(int N, int C, const int* row_ptr, const int* col_idx, const float* val, const float* dz, const float* W,
-                                 float* u, float* g_prev, const float* gate, float* acc, hipStream_t s)
-{
-    switch (C) {
-    case 128: return launch_level_wide_backward<128, 8>(N, row_ptr, col_idx, val, dz, W, u, g_prev, gate, acc, s);
-    case 256: return launch_level_wide_backward<256, 8>(N, row_ptr, col_idx, val, dz, W, u, g_prev, gate, acc, s);
     }
     return GNNHIP_EUNSUPPORTED;
 }

@@ -1,0 +1,490 @@
+// The wide mean-field level (C = 128 or 256) with its contraction on the bf16 matrix cores:
+//     h_out = ReLU((A * h_in) * W + bias + msg)
+// (examples/graph_classification/src/kernel_mean_field.cpp:35-42), every product formed from three bf16 pieces of
+// either operand (bf16_split.h: fp32 sums of exact products), and the backward pass of a level through the same
+// machinery.
+//
+// On FP32 matrix cores the contraction takes 8,192 cycles of a SIMD per 16 rows at C = 256, twice what the level's HBM
+// traffic takes; six bf16 products take 3,072, which leaves the kernel bound by memory.  The structure is that of
+// level_wide.hip: a persistent workgroup of eight wavefronts per compute unit, W in registers for the whole launch,
+// the rows of a pass summed into one LDS tile while the matrix cores read the other, one batch of six row loads per
+// 16-row block.  What is different:
+//   * A row is split into its pieces once, by the wavefront that summed it, and lies in LDS as three bf16 planes.
+//   * W in pieces takes 192 of a lane's 256 registers at C = 256.  The few fragments that do not fit are read from LDS;
+//     spilled to scratch memory they were reloaded behind the gather's loads, in whose order they had to wait (350 us
+//     per level instead of 240).
+//   * A wavefront whose rows hold more entries than the tops of the remaining blocks can take starts a second batch in
+//     the middle of a block; gathering behind the pass would hold up the other seven.
+//
+// 299,536 nodes, 659,010 entries, C = 256: 370 -> 240 us per level (0.92 GB of activations at 3.8 TB/s), backward
+// 474 -> 425 us (1.84 GB at 4.3 TB/s).
+//
+// Used by the inference forward and by the backward pass.  The levels of a training forward stay on level_wide.hip:
+// the sign of its outputs decides which gradients pass, so two roundings of the same sum give gradients that differ
+// by whole terms wherever a pre-activation is within rounding of zero (a few of 400 million per iteration).
+#include "bf16_split.h"
+#include "level_wide.h"
+
+namespace gnnhip {
+namespace {
+
+// C = 256: W in pieces takes 192 of a lane's 256 registers, and what does not fit would be reloaded from scratch memory
+// right behind the gather's loads, in whose order it would have to wait.  The third piece of this many contraction steps
+// of the first column block is read from LDS instead (one 128-bit read per step).
+template <int C, bool BWD> constexpr int wide_lds_fragments() { return C == 256 ? (BWD ? 7 : 6) : 0; }
+
+// Everything that steers the gather (row pointers, column indices, edge weights) is uniform
+// across the wavefront and is fetched with scalar loads: the values land in scalar registers, cost
+// no vector instruction to broadcast, and are counted apart from vector memory operations, so
+// waiting for them never waits for a store.
+// RELU_IN: the gathered rows count as ReLU(row) (the first level reading msg where h0 was not stored)
+// TR: rows per pass (16 or 32)
+// BWD: the backward pass of a level through the same machinery.  The CSR arrays are those of A^T, h_in is dz, the
+//      summed rows u = A^T dz are also stored to u_out as each one is finished (they are the other factor of the
+//      weight gradient), the contraction takes W transposed (g = u W^T), and the epilogue, instead of adding msg and
+//      applying ReLU, lets g through where the rows of `msg` (here: the embedding whose ReLU the gradient passes next,
+//      or null for no gate) are positive and adds what it stores to acc_io (or null).
+template <int C, int WAVES, bool RELU_IN, int TR, bool BWD = false>
+__global__ __launch_bounds__(WAVES * kWave) void s2v_level_split_kernel(
+    int N, int tiles_per_block, const int* __restrict__ row_ptr, const int* __restrict__ col_idx,
+    const float* __restrict__ val, const float* __restrict__ h_in, const float* __restrict__ W,
+    const float* __restrict__ msg, const float* __restrict__ bias, float* __restrict__ h_out,
+    float* __restrict__ u_out, float* __restrict__ acc_io)
+{
+    constexpr int KS = C / 32;                   // contraction steps
+    constexpr int kWideBlock = WAVES * kWave;
+    constexpr int CW = C / WAVES;                // output columns per wavefront
+    constexpr int NB = CW / 16;                  // 16-column blocks per wavefront
+    constexpr int VEC = C / kWave;               // gathered floats per lane
+    // A tile in LDS is [3 pieces][2 halves of the columns][kTileRows][LDT] of bf16.  A 128-bit LDS read serves sixteen lanes per
+    // cycle, lanes 0-3, 12-15 of one sixteen together with lanes 4-11 of its neighbour; rows that start in distinct
+    // 16-byte bank groups and neighbours that read the two halves (a multiple of 256 bytes apart) make that free of conflicts.
+    constexpr int LDT = C / 2 + 8;
+    constexpr int kTileRows = TR;
+    constexpr int RPW = kTileRows / WAVES;       // rows gathered per wavefront per pass
+    constexpr int kHalf = kTileRows * LDT;
+    constexpr int kPiece = 2 * kHalf;            // one piece of every element of a tile
+    static_assert(kHalf * 2 % 256 == 0, "halves start at the same bank");
+    constexpr int NF = wide_lds_fragments<C, BWD>();
+    using vec_t = typename VecT<VEC>::type;
+
+    extern __shared__ unsigned short tiles[];    // two tiles [3 pieces][kTileRows][LDT] of bf16: one read by the matrix
+                                                 // cores, the other being filled for the next pass
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int q = lane >> 4, t = lane & 15;
+    const int col0 = wave * CW;
+    const int gather_off = (lane >> 5) * kHalf + (wave * RPW) * LDT + (lane & 31) * VEC;
+    const int k_lane = (q & 1) * (C / 2) + (q >> 1) * 8;            // contraction step s of this lane: k = k_lane + 16 s .. + 7
+    float* bias_lds = reinterpret_cast<float*>(tiles + 2 * 3 * kPiece);      // [C], read in the epilogue without a trip to memory
+    if (bias)
+        for (int i = threadIdx.x; i < C; i += kWideBlock) bias_lds[i] = bias[i];
+
+    // W^T operand, in pieces: wreg[jb][s] holds W[k_lane + 16 s + 0..7][col0 + 16 jb + t]; BWD: of W itself,
+    // W[col0 + 16 jb + t][k_lane + 16 s + 0..7] (buffer loads: one lane offset, the steps as scalar offsets, so no 64-bit
+    // address per element is formed)
+    bf16_words4 wreg[NB][KS][3];
+    bf16_words4* w_lds = reinterpret_cast<bf16_words4*>(bias_lds + C) + (size_t)wave * NF * kWave + lane;
+    {
+        const rsrc_t w_rsrc = make_rsrc(W, (unsigned)(C * C * 4));
+        const int w_lane_off = BWD ? ((col0 + t) * C + k_lane) * 4 : (k_lane * C + col0 + t) * 4;
+#pragma unroll
+        for (int jb = 0; jb < NB; ++jb)
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+                float w[8];
+                if constexpr (BWD) {             // consecutive floats of one row of W
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const float4 v = buf_load4(w_rsrc, w_lane_off + 16 * C * 4 * jb, s * 64 + 16 * h);
+                        w[4 * h + 0] = v.x; w[4 * h + 1] = v.y; w[4 * h + 2] = v.z; w[4 * h + 3] = v.w;
+                    }
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) w[i] = buf_load_f(w_rsrc, w_lane_off + 64 * jb, (16 * s + i) * (C * 4));
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    unsigned p[3];
+                    bf16_split2(w[2 * i], w[2 * i + 1], p);
+                    wreg[jb][s][0][i] = p[0]; wreg[jb][s][1][i] = p[1]; wreg[jb][s][2][i] = p[2];
+                }
+                if (jb == 0 && s < NF) w_lds[s * kWave] = wreg[jb][s][2];
+            }
+    }
+
+    const int ntiles = (int)(((long long)N + kTileRows - 1) / kTileRows);
+    const int tile_begin = (int)min((long long)blockIdx.x * tiles_per_block, (long long)ntiles);
+    const int tile_end = (int)min((long long)ntiles, (long long)tile_begin + tiles_per_block);
+    if (tile_begin >= tile_end) return;
+
+    // ---- loaders.  The RPW + 1 row pointers of a pass sit in lanes 0..RPW of one vector register; columns
+    //      and weights of a batch are uniform and come through scalar loads (weights as bit patterns
+    //      so that selecting them stays on the scalar unit).
+    auto load_rowptrs = [&](int tile_id) {
+        const long long r0 = (long long)tile_id * kTileRows + wave * RPW;
+        int v = 0;
+        if (lane <= RPW) v = row_ptr[min(r0 + lane, (long long)N)];
+        return v;
+    };
+    const int* val_bits = reinterpret_cast<const int*>(val);
+    // entries [s, s + kInFlight) of the CSR arrays.  What lies past the end of the wavefront's rows is
+    // loaded but never added, so the batch is read as it lies.  Only a batch that would run past the end
+    // of the arrays starts earlier; batch_ready() then shifts it into place.  The entry count that bounds
+    // these reads is the matrix's own (row_ptr[N], read here), never a count passed by the host.  A matrix
+    // with fewer entries than one batch is read entry by entry, with zeros behind the last one.
+    const int nnz = row_ptr[N];
+    auto load_batch = [&](const int* arr, int s, Batch& b) {
+        if (nnz < kInFlight) {
+            batch_load_short(b, arr, nnz);
+            return s;
+        }
+        const int base = max(min(s, nnz - kInFlight), 0);
+        batch_load(b, arr + base);
+        return s - base;                         // by how many entries the batch has to be shifted
+    };
+    auto batch_ready = [&](Batch& b, int shift) {
+        batch_wait(b);
+        for (; shift > 0; --shift) {             // only at the very end of the arrays
+            b.lo.x = b.lo.y; b.lo.y = b.lo.z; b.lo.z = b.lo.w; b.lo.w = b.hi.x; b.hi.x = b.hi.y;
+        }
+    };
+    const rsrc_t h_rsrc = make_rsrc(h_in, (unsigned)((size_t)N * C * 4));
+    auto issue = [&](const Batch& c, vec_t (&x)[kInFlight]) {
+#pragma unroll
+        for (int u = 0; u < kInFlight; ++u)
+            x[u] = BufLoad<VEC>::get(h_rsrc, lane * (VEC * 4), batch_get(c, u) * (C * 4));     // N C 4 < 2^32 (host-checked)
+    };
+
+    // ---- state of the gather of one pass: entries [e, ee) of the wavefront's RPW rows, taken in order;
+    //      a row goes to LDS when its last entry has been added
+    int e = 0, ee = 0, lr = 0, row_end = 0, rpv = 0;
+    unsigned short* dstp = nullptr;
+    float acc[VEC];
+    rsrc_t u_rsrc = make_rsrc(u_out, 0);         // BWD: the rows of u_out that the pass being gathered covers
+    auto begin = [&](int rp_lanes, int eb, int eend, unsigned short* dst, int tile_id) {
+        rpv = rp_lanes;
+        e = eb; ee = eend; lr = 0;
+        row_end = __builtin_amdgcn_readlane(rpv, 1);
+        dstp = dst;
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) acc[i] = 0.f;
+        if constexpr (BWD) {
+            const long long r0 = (long long)tile_id * kTileRows;
+            const long long rows = max(min((long long)N - r0, (long long)kTileRows), 0ll);      // none past the last pass
+            u_rsrc = make_rsrc(u_out + (size_t)min(r0, (long long)N) * C, (unsigned)(rows * (C * 4)));
+        }
+    };
+    auto flush_row = [&]() {
+        unsigned p[VEC / 2][3];
+#pragma unroll
+        for (int i = 0; i < VEC / 2; ++i) bf16_split2(acc[2 * i], acc[2 * i + 1], p[i]);
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            if constexpr (VEC == 4) *reinterpret_cast<uint2*>(dstp + j * kPiece) = make_uint2(p[0][j], p[1][j]);
+            else *reinterpret_cast<unsigned*>(dstp + j * kPiece) = p[0][j];
+        }
+        if constexpr (BWD)                        // rows past N lie outside the descriptor
+            BufStore<VEC>::put(u_rsrc, lane * (VEC * 4), (wave * RPW + lr) * (C * 4), *reinterpret_cast<vec_t*>(acc));
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) acc[i] = 0.f;
+        dstp += LDT;
+        ++lr;
+        row_end = __builtin_amdgcn_readlane(rpv, min(lr + 1, RPW));
+    };
+    auto consume = [&](const Batch& a, const vec_t (&x)[kInFlight]) {
+#pragma unroll
+        for (int u = 0; u < kInFlight; ++u) {
+            if (e + u < ee) {
+                while (e + u >= row_end) flush_row();          // rows ending here (possibly empty ones)
+                vec_fma<VEC, RELU_IN>(acc, __int_as_float(batch_get(a, u)), x[u]);
+            }
+        }
+        e += kInFlight;
+    };
+    auto finish = [&]() { while (lr < RPW) flush_row(); };      // the open row and empty rows after it
+
+    // Output of the last finished 16-row block, stored at the top of the following block (or at the end
+    // of the pass): a store then has a whole contraction between its issue and the next wait on
+    // vector memory.  msg and h_out are addressed through descriptors that cover the rows of the
+    // current pass only, so rows past N fall outside and need no predicate.
+    float4 outv[NB];
+    int out_rt = -1;                             // block of this pass held in outv, -1: none
+#pragma unroll
+    for (int jb = 0; jb < NB; ++jb) outv[jb] = f4_zero();
+    const int lane_off = (t * C + col0 + 4 * q) * 4;              // byte offset of this lane inside a 16-row block
+    rsrc_t msg_rsrc = make_rsrc(msg, 0), out_rsrc = make_rsrc(h_out, 0), acc_rsrc = make_rsrc(acc_io, 0);
+    auto store_pending = [&]() {
+        if (out_rt >= 0) {
+#pragma unroll
+            for (int jb = 0; jb < NB; ++jb) buf_store4(out_rsrc, lane_off + out_rt * (16 * C * 4) + 64 * jb, 0, outv[jb]);
+        }
+        out_rt = -1;
+    };
+
+    Batch cC, aC;                                // columns / weights of the next batch to issue / to sum
+    cC.lo = i32x4{0, 0, 0, 0}; cC.hi = i32x2{0, 0};
+    aC.lo = i32x4{0, 0, 0, 0}; aC.hi = i32x2{0, 0};
+    int cShift = 0, aShift = 0;                  // shifts owed to cC / aC when they are next read
+
+    // ---- first pass: its gather has nothing to hide behind
+    int rp_next = load_rowptrs(tile_begin);      // row pointers of the next pass to gather
+    int ebN = __builtin_amdgcn_readlane(rp_next, 0), eeN = __builtin_amdgcn_readlane(rp_next, RPW);
+    begin(rp_next, ebN, eeN, tiles + gather_off, tile_begin);
+    while (e < ee) {
+        vec_t x[kInFlight];
+        cShift = load_batch(col_idx, e, cC);
+        aShift = load_batch(val_bits, e, aC);
+        batch_ready(cC, cShift);
+        batch_ready(aC, aShift);
+        issue(cC, x);
+        consume(aC, x);
+    }
+    finish();
+    ebN = eeN = 0;
+    if (tile_begin + 1 < tile_end) {
+        rp_next = load_rowptrs(tile_begin + 1);
+        ebN = __builtin_amdgcn_readlane(rp_next, 0);
+        eeN = __builtin_amdgcn_readlane(rp_next, RPW);
+        if (ebN < eeN) { cShift = load_batch(col_idx, ebN, cC); aShift = load_batch(val_bits, ebN, aC); }
+    }
+    __syncthreads();
+
+    for (int tile_id = tile_begin; tile_id < tile_end; ++tile_id) {
+        const long long row0 = (long long)tile_id * kTileRows;
+        const int parity = (tile_id - tile_begin) & 1;
+        const unsigned short* cur = tiles + parity * (3 * kPiece);
+        const bool has_next = tile_id + 1 < tile_end;
+        const bool has_next2 = tile_id + 2 < tile_end;
+        begin(rp_next, ebN, eeN, tiles + (parity ^ 1) * (3 * kPiece) + gather_off, tile_id + 1);   // empty when !has_next
+        {
+            const long long left = (long long)N - row0;
+            const unsigned bytes = (unsigned)(min(left, (long long)kTileRows) * (C * 4));
+            out_rsrc = make_rsrc(h_out + (size_t)row0 * C, bytes);
+            msg_rsrc = make_rsrc(msg ? msg + (size_t)row0 * C : nullptr, msg ? bytes : 0u);   // no msg: every load reads 0
+            if constexpr (BWD) acc_rsrc = make_rsrc(acc_io ? acc_io + (size_t)row0 * C : nullptr, acc_io ? bytes : 0u);
+        }
+        if (has_next2) rp_next = load_rowptrs(tile_id + 2);
+
+        // ---- contraction and epilogue, one 16-row block at a time; each block also carries one batch
+        //      of the next pass's gather, issued before its matrix instructions and summed after them
+#pragma unroll 1
+        for (int rt = 0; rt < kTileRows / 16; ++rt) {
+            // msg is asked for now and added after the contraction (as the accumulators' initial value it
+            // would have to arrive before the first matrix instruction)
+            float4 mm[NB], aa[BWD ? NB : 1];
+            mfma_f4 acc_m[NB];
+#pragma unroll
+            for (int jb = 0; jb < NB; ++jb) {
+                if constexpr (!BWD) mm[jb] = buf_load4(msg_rsrc, lane_off + rt * (16 * C * 4) + 64 * jb, 0);
+                acc_m[jb] = mfma_f4{0.f, 0.f, 0.f, 0.f};
+            }
+            vec_t x[kInFlight];
+            const bool batch = e < ee;
+            if (batch) { batch_ready(cC, cShift); issue(cC, x); }
+            store_pending();
+            // where the follower of this batch starts: inside this pass, or (after the last block) at the
+            // first entry of the next pass; its columns travel while the matrix cores work
+            int ns = 0, nend = 0;
+            if (rt < kTileRows / 16 - 1) {
+                if (e + kInFlight < ee) { ns = e + kInFlight; nend = ee; }
+            } else if (kTileRows > 16 && e + kInFlight >= ee) {
+                ns = ebN; nend = eeN;                     // both zero when there is no next pass
+            }
+            // (a 16-row pass has one block: ebN/eeN still describe the pass being gathered, the row pointers of
+            // the one after it arrive during this block, so its first batch is asked for after the block)
+
+            const unsigned short* src = cur + (q & 1) * kHalf + (rt * 16 + t) * LDT + (q >> 1) * 8;
+            // A piece of the tile operand is read for the next step as soon as this step's products with it are issued:
+            // the pieces are used in the order 3, 2, 1, so that each read has six or more matrix instructions to arrive in.
+            bool again = false;
+            bf16_words4 b[3];
+#pragma unroll
+            for (int j = 2; j >= 0; --j) b[j] = *reinterpret_cast<const bf16_words4*>(src + j * kPiece);
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+                bf16_words4 w3;
+                if (s < NF) w3 = w_lds[s * kWave];
+#pragma unroll
+                for (int j = 2; j >= 0; --j) {
+#pragma unroll
+                    for (int i = 2 - j; i >= 0; --i)
+#pragma unroll
+                        for (int jb = 0; jb < NB; ++jb)
+                            acc_m[jb] = mfma_bf16(i == 2 && jb == 0 && s < NF ? w3 : wreg[jb][s][i], b[j], acc_m[jb]);
+                    if (s + 1 < KS) b[j] = *reinterpret_cast<const bf16_words4*>(src + j * kPiece + 16 * (s + 1));
+                    __builtin_amdgcn_sched_barrier(0);            // keeps the read-ahead where it is written
+                }
+                // the follower's columns are asked for here, behind the first wait for LDS of this block: a
+                // scalar load in flight counts with the LDS reads, and the next wait is 6 NB matrix instructions away
+                if (s == 0 && ns < nend) cShift = load_batch(col_idx, ns, cC);
+                if (s == KS / 2 - 1 && batch && ee - (e + kInFlight) > kInFlight * (kTileRows / 16 - 1 - rt)) {
+                    // more entries than the tops of the blocks that are left can take: this wavefront takes a second batch
+                    // in this block (in the open behind the pass it would keep the other seven waiting)
+                    __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+                    batch_ready(aC, aShift);
+                    consume(aC, x);
+                    aShift = load_batch(val_bits, e, aC);
+                    if (rt == kTileRows / 16 - 1) cShift = load_batch(col_idx, e, cC);
+                    batch_ready(cC, cShift);
+                    batch_ready(aC, aShift);                  // both have to land before the paths join
+                    aShift = 0;
+                    issue(cC, x);
+                    ns = nend = 0;
+                    if (e + kInFlight < ee) {
+                        if (rt < kTileRows / 16 - 1) { ns = e + kInFlight; nend = ee; }
+                    } else if (kTileRows > 16 && rt == kTileRows / 16 - 1) {
+                        ns = ebN; nend = eeN;
+                    }
+                    again = ns < nend;
+                }
+                if (s == KS / 2 && again) cShift = load_batch(col_idx, ns, cC);
+            }
+            // One unconditional wait for everything this block asked for (gathered rows, msg).  The loads
+            // and their uses sit under separate conditions; without this the compiler has to assume a
+            // path on which they are still in flight and waits at the top of the next block instead,
+            // where the wait also covers the stores issued just before it.
+            if constexpr (BWD) {
+                // the gate and the old values of acc_io are asked for here, where the operands of the contraction have left
+                // their registers, and arrive while the gathered rows are summed; where a buffer is null its loads touch
+                // nothing
+#pragma unroll
+                for (int jb = 0; jb < NB; ++jb) mm[jb] = buf_load4(msg_rsrc, lane_off + rt * (16 * C * 4) + 64 * jb, 0);
+#pragma unroll
+                for (int jb = 0; jb < NB; ++jb) aa[jb] = buf_load4(acc_rsrc, lane_off + rt * (16 * C * 4) + 64 * jb, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            __builtin_amdgcn_s_waitcnt(kWaitVmcnt0 + (BWD ? 2 * NB : 0));
+            if (batch) { batch_ready(aC, aShift); consume(aC, x); }
+            if (ns < nend) aShift = load_batch(val_bits, ns, aC);
+            if (rt == 0) {                                // the row pointers asked for at the top have arrived
+                ebN = eeN = 0;
+                if (has_next2) {
+                    ebN = __builtin_amdgcn_readlane(rp_next, 0);
+                    eeN = __builtin_amdgcn_readlane(rp_next, RPW);
+                }
+            }
+            if constexpr (BWD) {
+#pragma unroll
+                for (int jb = 0; jb < NB; ++jb) {
+                    float4 v = make_float4(acc_m[jb][0], acc_m[jb][1], acc_m[jb][2], acc_m[jb][3]);
+                    if (msg) {                   // past the ReLU whose output these rows are
+                        v.x = mm[jb].x > 0.f ? v.x : 0.f; v.y = mm[jb].y > 0.f ? v.y : 0.f;
+                        v.z = mm[jb].z > 0.f ? v.z : 0.f; v.w = mm[jb].w > 0.f ? v.w : 0.f;
+                    }
+                    if (acc_io) {                // every row belongs to one pass: nobody else touches it during the launch
+                        const float4 a = make_float4(aa[jb].x + v.x, aa[jb].y + v.y, aa[jb].z + v.z, aa[jb].w + v.w);
+                        buf_store4(acc_rsrc, lane_off + rt * (16 * C * 4) + 64 * jb, 0, a);
+                    }
+                    outv[jb] = v;
+                }
+            } else {
+#pragma unroll
+                for (int jb = 0; jb < NB; ++jb) {
+                    acc_m[jb][0] += mm[jb].x; acc_m[jb][1] += mm[jb].y; acc_m[jb][2] += mm[jb].z; acc_m[jb][3] += mm[jb].w;
+                }
+#pragma unroll
+                for (int jb = 0; jb < NB; ++jb) {
+                    float4 v = make_float4(acc_m[jb][0], acc_m[jb][1], acc_m[jb][2], acc_m[jb][3]);
+                    if (bias) {
+                        const float4 b4 = *reinterpret_cast<const float4*>(bias_lds + col0 + 16 * jb + 4 * q);
+                        v.x += b4.x; v.y += b4.y; v.z += b4.z; v.w += b4.w;
+                    }
+                    outv[jb] = make_float4(relu_ref(v.x), relu_ref(v.y), relu_ref(v.z), relu_ref(v.w));
+                }
+            }
+            out_rt = rt;
+        }
+        if (kTileRows == 16 || e < ee) {                  // more batches than blocks: finish in the open
+            while (e < ee) {
+                vec_t x[kInFlight];
+                cShift = load_batch(col_idx, e, cC);
+                aShift = load_batch(val_bits, e, aC);
+                batch_ready(cC, cShift);
+                batch_ready(aC, aShift);
+                issue(cC, x);
+                consume(aC, x);
+            }
+            if (ebN < eeN) { cShift = load_batch(col_idx, ebN, cC); aShift = load_batch(val_bits, ebN, aC); }
+        }
+        if (has_next) finish();
+        store_pending();
+        __syncthreads();                                  // the tile just filled is complete, the other one is free
+    }
+}
+
+template <int C, int WAVES, bool RELU_IN, int TR, bool BWD = false>
+int launch_level_split_t(int N, const int* row_ptr, const int* col_idx, const float* val, const float* h_in,
+                      const float* W, const float* msg, const float* bias, float* h_out, hipStream_t s,
+                      float* u_out = nullptr, float* acc_io = nullptr)
+{
+    if ((unsigned long long)N * C * 4ull >= (1ull << 32)) return GNNHIP_EUNSUPPORTED;   // 32-bit buffer offsets
+    constexpr int kTileRows = TR;
+    const long long ntiles = ((long long)N + kTileRows - 1) / kTileRows;
+    // workgroups that fit one compute unit together: two at C = 128 (82 registers per lane, 68 KB of LDS each)
+    constexpr int kPerCU = (C == 128) ? 2 : 1;
+    const long long slots = (long long)kNumCU * kPerCU;
+    const long long per = (ntiles + slots - 1) / slots;              // contiguous run of tiles per workgroup
+    const long long blocks = (ntiles + per - 1) / per;
+    const size_t smem = 2 * 3 * 2 * sizeof(unsigned short) * kTileRows * (C / 2 + 8) + sizeof(float) * C +
+                        sizeof(bf16_words4) * (size_t)wide_lds_fragments<C, BWD>() * WAVES * kWave;
+    static LdsLimit lds_limit;                                       // one per kernel instantiation
+    GNNHIP_HIP(lds_limit.raise(reinterpret_cast<const void*>(&s2v_level_split_kernel<C, WAVES, RELU_IN, TR, BWD>), smem));
+    hipLaunchKernelGGL((s2v_level_split_kernel<C, WAVES, RELU_IN, TR, BWD>), dim3((unsigned)blocks), dim3(WAVES * kWave), smem, s,
+                       N, (int)per, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, u_out, acc_io);
+    GNNHIP_LAUNCH_CHECK(BWD ? "s2v_level_split backward" : "s2v_level_split");
+    return GNNHIP_OK;
+}
+
+// Rows per pass: 32 (two tiles of 64 rows do not fit the LDS at C = 256), 16 on matrices with fewer 32-row passes than
+// twice the workgroups.
+template <int C, int WAVES, bool RELU_IN>
+int launch_level_split(int N, const int* row_ptr, const int* col_idx, const float* val, const float* h_in,
+                      const float* W, const float* msg, const float* bias, float* h_out, hipStream_t s)
+{
+    constexpr int kSlots = kNumCU * ((C == 128) ? 2 : 1);
+    if (N >= 2 * kSlots * 32) return launch_level_split_t<C, WAVES, RELU_IN, 32>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, s);
+    return launch_level_split_t<C, WAVES, RELU_IN, 16>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, s);
+}
+
+// The backward pass: same choice of rows per pass.
+template <int C, int WAVES>
+int launch_level_split_backward(int N, const int* row_ptr, const int* col_idx, const float* val, const float* dz, const float* W,
+                               float* u, float* g_prev, const float* gate, float* acc, hipStream_t s)
+{
+    constexpr int kSlots = kNumCU * ((C == 128) ? 2 : 1);
+    if (N >= 2 * kSlots * 32) return launch_level_split_t<C, WAVES, false, 32, true>(N, row_ptr, col_idx, val, dz, W, gate, nullptr, g_prev, s, u, acc);
+    return launch_level_split_t<C, WAVES, false, 16, true>(N, row_ptr, col_idx, val, dz, W, gate, nullptr, g_prev, s, u, acc);
+}
+
+}  // namespace
+
+int level_split_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val,
+                        const float* h_in, const float* W, const float* msg, const float* bias, float* h_out, bool relu_in,
+                        hipStream_t s)
+{
+    (void)nnz;                                   // the kernel bounds its index reads with row_ptr[N]
+    switch (C) {
+    case 128:
+        return relu_in ? launch_level_split<128, 8, true>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, s)
+                       : launch_level_split<128, 8, false>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, s);
+    case 256:
+        return relu_in ? launch_level_split<256, 8, true>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, s)
+                       : launch_level_split<256, 8, false>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, s);
+    }
+    return GNNHIP_EUNSUPPORTED;
+}
+
+// u = A' dz (stored) and g_prev = u W^T past the gate of `gate` (may be null), added to acc (may be null): the wide
+// kernel's backward variant over the CSR arrays of A' = A^T.
+int level_split_backward_dispatch(int N, int C, const int* row_ptr, const int* col_idx, const float* val, const float* dz, const float* W,
+                                 float* u, float* g_prev, const float* gate, float* acc, hipStream_t s)
+{
+    switch (C) {
+    case 128: return launch_level_split_backward<128, 8>(N, row_ptr, col_idx, val, dz, W, u, g_prev, gate, acc, s);
+    case 256: return launch_level_split_backward<256, 8>(N, row_ptr, col_idx, val, dz, W, u, g_prev, gate, acc, s);
+    }
+    return GNNHIP_EUNSUPPORTED;
+}
+
+}  // namespace gnnhip
