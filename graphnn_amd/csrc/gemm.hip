@@ -345,9 +345,8 @@ void launch_skinny(bool tb, int m, int k, float alpha, const float* A, int lda, 
 
 }  // namespace
 
-// gemm_tn_tall.hip: square outputs of 128 / 256 over a very long k
-bool gemm_tn_tall_applies(int m, int n, int k, const float* A, int lda, const float* B, int ldb);
-int gemm_tn_tall_dispatch(int m, int n, int k, float alpha, const float* A, int lda, const float* B, int ldb, float beta, float* C,
+// gemm_tn_split.hip: outputs of up to 256 x 256 over a very long k
+int gemm_tn_split_dispatch(int m, int n, int k, float alpha, const float* A, int lda, const float* B, int ldb, float beta, float* C,
                           int ldc, hipStream_t s);
 
 void launch_splitk_reduce(int m, int n, int splits, float alpha, const float* partial, float beta, float* C, int ldc, hipStream_t s)
@@ -378,9 +377,10 @@ int gemm_tn_batch_dispatch(int count, const int* m, const int* n, const int* k, 
     int z = 0;
     for (int p = 0; p < count; ++p) {
         if (m[p] == 0 || n[p] == 0) continue;
-        // the rule of the single product here too: a wide square output over a very long k has a kernel of its own
-        if (gemm_tn_tall_applies(m[p], n[p], k[p], A[p], lda[p], B[p], ldb[p])) {
-            if (int rc = gemm_tn_tall_dispatch(m[p], n[p], k[p], alpha, A[p], lda[p], B[p], ldb[p], beta, C[p], ldc[p], s)) return rc;
+        // the rule of the single product here too: an output of up to 256 x 256 over a very long k has a kernel of its own
+        if (int rc = gemm_tn_split_dispatch(m[p], n[p], k[p], alpha, A[p], lda[p], B[p], ldb[p], beta, C[p], ldc[p], s);
+            rc != GNNHIP_EUNSUPPORTED) {
+            if (rc) return rc;
             continue;
         }
         const int q = b.count++;
@@ -427,7 +427,7 @@ int gemm_dispatch(int transA, int transB, int m, int n, int k, float alpha, cons
         return GNNHIP_OK;
     }
     if (transA && !transB) {
-        if (int rc = gemm_tn_tall_dispatch(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, s); rc != GNNHIP_EUNSUPPORTED) return rc;
+        if (int rc = gemm_tn_split_dispatch(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, s); rc != GNNHIP_EUNSUPPORTED) return rc;
     }
     dim3 grid(ceil_div_u((size_t)m, BM), ceil_div_u((size_t)n, BN));
     dim3 block(kBlock);

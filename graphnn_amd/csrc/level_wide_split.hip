@@ -80,6 +80,10 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_split_kernel(
     if (bias)
         for (int i = threadIdx.x; i < C; i += kWideBlock) bias_lds[i] = bias[i];
 
+    // The matrix instruction rounds its sum towards minus infinity.  The middle half of the contraction steps is formed with
+    // -W on the negated sum, so that the drift of one half of the steps cancels that of the other.
+    auto negated = [](int s) { return s >= KS / 4 && s < KS - KS / 4; };
+
     // W^T operand, in pieces: wreg[jb][s] holds W[k_lane + 16 s + 0..7][col0 + 16 jb + t]; BWD: of W itself,
     // W[col0 + 16 jb + t][k_lane + 16 s + 0..7] (buffer loads: one lane offset, the steps as scalar offsets, so no 64-bit
     // address per element is formed)
@@ -108,6 +112,10 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_split_kernel(
                     unsigned p[3];
                     bf16_split2(w[2 * i], w[2 * i + 1], p);
                     wreg[jb][s][0][i] = p[0]; wreg[jb][s][1][i] = p[1]; wreg[jb][s][2][i] = p[2];
+                }
+                if (negated(s)) {
+#pragma unroll
+                    for (int p = 0; p < 3; ++p) wreg[jb][s][p] ^= 0x80008000u;
                 }
                 if (jb == 0 && s < NF) w_lds[s * kWave] = wreg[jb][s][2];
             }
@@ -303,6 +311,10 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_split_kernel(
             for (int j = 2; j >= 0; --j) b[j] = *reinterpret_cast<const bf16_words4*>(src + j * kPiece);
 #pragma unroll
             for (int s = 0; s < KS; ++s) {
+                if (s > 0 && negated(s) != negated(s - 1)) {
+#pragma unroll
+                    for (int jb = 0; jb < NB; ++jb) acc_m[jb] = -acc_m[jb];
+                }
                 bf16_words4 w3;
                 if (s < NF) w3 = w_lds[s * kWave];
 #pragma unroll

@@ -301,3 +301,38 @@ def test_training_iteration_composed_from_the_c_abi(gpu, oracle, config_id, C):
     for t, w0, g0 in zip(ws, (w.W_n2l, w.W_conv, w.W_h1, w.W_h2), (gWn, gWc, gW1, gW2)):
         want_w, _, _ = oracle.momentum_sgd(w0, _n(g0), np.zeros_like(w0), 0.01, 0.9, 1e-4)
         assert np.allclose(_n(t), want_w, rtol=1e-6, atol=1e-8)
+
+
+@pytest.mark.parametrize("m,n,k", [(256, 256, 8192), (256, 256, 20_011), (255, 33, 40_007), (129, 256, 9_001), (64, 256, 16_385),
+                                   (1, 256, 1_048_577), (128, 128, 16_384), (100, 127, 23_456), (65, 64, 65_600), (64, 64, 65_543)])
+def test_weight_gradient_over_a_long_k(gpu, m, n, k):
+    """A^T B with an output of up to 256 x 256 over a long k (operands in bf16 pieces on the matrix cores, the whole output in
+    one workgroup): every tile shape and its transposed form, columns short of a tile, k short of a stage, against float64;
+    the error stays within what an fp32 sum of this length has, and the batch call gives the same bits"""
+    import torch
+    from graphnn_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(m * 1000 + n)
+    A = torch.randn(k, m, generator=gen, device=gpu)
+    B = torch.randn(k, n, generator=gen, device=gpu) + 0.5
+    out0 = torch.randn(m, n, generator=gen, device=gpu)
+    got = ops.gemm(A, B, transA=True, alpha=0.5, beta=2.0, out=out0.clone())
+    want = 0.5 * (A.double().T.contiguous() @ B.double()) + 2.0 * out0.double()
+    terms = 0.5 * (A.double().abs().T.contiguous() @ B.double().abs()) + 2.0 * out0.double().abs()
+    assert float(((got.double() - want).abs() / terms).max()) < 1e-6
+    assert float((got.double() - want).norm() / want.norm()) < 2e-6
+    batched = out0.clone()
+    ops.gemm_tn_batch([(A, B, batched)], alpha=0.5, beta=2.0)
+    assert torch.equal(batched, got)
+
+
+def test_weight_gradient_carries_infinities_and_nan(gpu):
+    """an infinite or NaN term reaches the outputs it is part of and no others, next to values whose bf16 rounding would overflow"""
+    import torch
+    from graphnn_amd import ops
+    k, m, n = 20_000, 64, 256
+    A = torch.zeros(k, m, device=gpu)
+    B = torch.ones(k, n, device=gpu)
+    A[5, 1], A[6, 2], A[7, 3], A[8, 4] = float("inf"), float("-inf"), float("nan"), 3.4028e38
+    got = ops.gemm(A, B, transA=True)
+    assert bool((got[1] == float("inf")).all()) and bool((got[2] == float("-inf")).all()) and bool(torch.isnan(got[3]).all())
+    assert bool(torch.isfinite(got[4]).all()) and bool((got[0] == 0).all()) and bool((got[5:] == 0).all())
