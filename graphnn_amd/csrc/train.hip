@@ -192,6 +192,29 @@ __global__ __launch_bounds__(kBlock) void grad_gate_kernel(size_t n, const float
     }
 }
 
+// The same for 16-byte aligned tensors in 128-bit words, n4 of them: two reads and two writes at the copy rate (299,536 x
+// 256: 319 -> 219 us, 1.23 GB).
+template <bool DZ, bool ACC, bool ACCUMULATE>
+__global__ __launch_bounds__(kBlock) void grad_gate4_kernel(size_t n4, const float4* __restrict__ h, const float4* g, float4* dz, float4* acc)
+{
+    const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n4) return;
+    const float4 x = h[i], y = g[i];
+    float4 a = f4_zero();
+    if (ACC && ACCUMULATE) a = acc[i];
+    const float4 v = make_float4(x.x > 0.f ? y.x : 0.f, x.y > 0.f ? y.y : 0.f, x.z > 0.f ? y.z : 0.f, x.w > 0.f ? y.w : 0.f);
+    if (DZ) dz[i] = v;
+    if (ACC) acc[i] = ACCUMULATE ? make_float4(a.x + v.x, a.y + v.y, a.z + v.z, a.w + v.w) : v;
+}
+
+template <bool DZ, bool ACC, bool ACCUMULATE>
+void launch_gate4(size_t n4, const float* h, const float* g, float* dz, float* acc, hipStream_t s)
+{
+    hipLaunchKernelGGL((grad_gate4_kernel<DZ, ACC, ACCUMULATE>), dim3(ceil_div_u(n4, kBlock)), dim3(kBlock), 0, s, n4,
+                       reinterpret_cast<const float4*>(h), reinterpret_cast<const float4*>(g), reinterpret_cast<float4*>(dz),
+                       reinterpret_cast<float4*>(acc));
+}
+
 // ------------------------------------------------------------------ parameter update
 constexpr int kUpdateBatch = 16;
 struct UpdateBatch {
@@ -324,7 +347,7 @@ int gnnhip_s2v_loss_acc_f32(int B, int Q, const float* logits, const int* lrow_p
     GNNHIP_REQUIRE(logits && lrow_ptr && lcol && lval && (loss_mean || acc_mean), "null tensor in s2v_loss_acc");
     if (int rc = require_ready()) return rc;
     hipStream_t s = as_stream(stream);
-    int nb = (B + 4 * kBlock - 1) / (4 * kBlock);         // about four rows per lane
+    int nb = B <= 4 * kBlock ? 1 : (B + kBlock - 1) / kBlock;           // one launch up to four rows per lane, else a row per lane
     if (nb > 1024) nb = 1024;
     void* partial = nullptr;
     if (int rc = stream_scratch(s, sizeof(float) * 2 * (size_t)nb, &partial)) return rc;
@@ -376,7 +399,18 @@ int gnnhip_s2v_grad_gate_f32(size_t n, const float* h, const float* g, float* dz
     if (n == 0) return GNNHIP_OK;
     GNNHIP_REQUIRE(h && g && (dz || acc), "null tensor in s2v_grad_gate");
     if (int rc = require_ready()) return rc;
-    hipLaunchKernelGGL(grad_gate_kernel, dim3(ew_grid(n)), dim3(kBlock), 0, as_stream(stream), n, h, g, dz, acc, accumulate);
+    hipStream_t s = as_stream(stream);
+    const size_t n4 = aligned16(h) && aligned16(g) && aligned16(dz) && aligned16(acc) ? n / 4 : 0;        // null counts as aligned
+    if (n4 > 0) {
+        if (dz && !acc) launch_gate4<true, false, false>(n4, h, g, dz, acc, s);
+        else if (!dz && accumulate) launch_gate4<false, true, true>(n4, h, g, dz, acc, s);
+        else if (!dz) launch_gate4<false, true, false>(n4, h, g, dz, acc, s);
+        else if (accumulate) launch_gate4<true, true, true>(n4, h, g, dz, acc, s);
+        else launch_gate4<true, true, false>(n4, h, g, dz, acc, s);
+    }
+    if (const size_t done = 4 * n4; done < n)
+        hipLaunchKernelGGL(grad_gate_kernel, dim3(ew_grid(n - done)), dim3(kBlock), 0, s, n - done, h + done, g + done, dz ? dz + done : nullptr,
+                           acc ? acc + done : nullptr, accumulate);
     GNNHIP_LAUNCH_CHECK("grad_gate");
     return GNNHIP_OK;
 }
