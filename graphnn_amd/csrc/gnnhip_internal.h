@@ -189,9 +189,33 @@ constexpr int kHubThreshold = 64;      // rows with more entries are summed by t
 constexpr int kHubChunk = 2048;        // entries per partial sum of the pre-pass
 constexpr int kHubMinRows = 32768;     // smaller matrices skip the pre-pass: its launches would cost more than a long row
 struct HubPlan {
-    const int* row_slot;               // [m], defined for rows longer than the pass's threshold only; -1: not summed
-    const float* agg;                  // [slots][ld]
-    int ld;
+    const int* row_chunk = nullptr;    // [m], defined for rows longer than the pass's threshold only: first chunk, -1: not summed
+    const float* part = nullptr;       // [chunks][ld]
+    int ld = 0;
+    int shift = 0;                     // entries of a row per chunk: 1 << shift
+};
+// A row's sum from the sums of its chunks, added in chunk order; p: the first chunk's sum at this lane's columns.
+// V: load(const float*), add(a, b), zero().
+template <class V>
+__device__ __forceinline__ typename V::T hub_row_sum(const float* p, int ld, int entries, int shift)
+{
+    const int nc = (entries + (1 << shift) - 1) >> shift;
+    typename V::T sum = V::load(p);
+    for (int j0 = 1; j0 < nc; j0 += 4) {         // four in flight: more registers would cost the callers wavefronts
+        typename V::T x[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[u] = j0 + u < nc ? V::load(p + (size_t)(j0 + u) * ld) : V::zero();
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (j0 + u < nc) sum = V::add(sum, x[u]);
+    }
+    return sum;
+}
+struct HubF4 {                         // V for 128-bit columns
+    using T = float4;
+    static __device__ __forceinline__ T zero() { return f4_zero(); }
+    static __device__ __forceinline__ T load(const float* p) { return *reinterpret_cast<const float4*>(p); }
+    static __device__ __forceinline__ T add(T a, T b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
 };
 // A block of pool memory that holds the plan and the sums of one balanced pass for an owner that keeps it across
 // calls (a CSR plan); planned: the planning launches have run in it.
@@ -201,7 +225,7 @@ struct HubStore {
     bool planned = false;
 };
 // threshold / chunk_len: rows with more entries than `threshold` are summed, cut into chunks of `chunk_len`
-// (the consumer must apply the same threshold when it looks a row up in row_slot); max_hubs >= 0: the caller's
+// (the consumer must apply the same threshold when it looks a row up in row_chunk); max_hubs >= 0: the caller's
 // bound on the number of such rows; store: where the pass keeps its arrays (null: the stream's scratch slot 1)
 // reuse_plan: the caller states that the previous call on this stream had the very same matrix: same arrays, same structure
 // AND same values (the column-ordered pieces keep a copy of the values), nothing rewritten in between.

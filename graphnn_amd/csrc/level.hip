@@ -195,7 +195,7 @@ __global__ __launch_bounds__(kBlock) void s2v_level_kernel(
     int N, const int* __restrict__ row_ptr, const int* __restrict__ col_idx, const float* __restrict__ val,
     const float* __restrict__ h_in, const float* __restrict__ W, const float* __restrict__ msg,
     const float* __restrict__ bias, float* __restrict__ h_out,
-    const int* __restrict__ hub_slot, const float* __restrict__ hub_agg, int hub_ld)
+    HubPlan hubs)
 {
     constexpr int G = C / 4;             // lanes per gathered row
     constexpr int RPR = kWave / G;       // rows gathered per round
@@ -284,7 +284,7 @@ __global__ __launch_bounds__(kBlock) void s2v_level_kernel(
                 is_long[rd] = (en[rd] - st[rd] > kWaveLongRow);
                 hub[rd] = -1;
                 if (is_long[rd]) {
-                    if (hub_slot && en[rd] - st[rd] > kHubThreshold) hub[rd] = hub_slot[row0 + lr];   // summed by the pre-pass
+                    if (hubs.row_chunk && en[rd] - st[rd] > kHubThreshold) hub[rd] = hubs.row_chunk[row0 + lr];   // summed by the pre-pass
                     if (hub[rd] >= 0) is_long[rd] = false;
                     en[rd] = st[rd];
                 }
@@ -342,7 +342,7 @@ __global__ __launch_bounds__(kBlock) void s2v_level_kernel(
                             if (j + u < cnt) f4_fma(acc, vj[u], xx[u]);
                     }
                 }
-                if (hub[rd] >= 0) acc = *reinterpret_cast<const float4*>(hub_agg + (size_t)hub[rd] * hub_ld + tx * 4);
+                if (hub[rd] >= 0) acc = hub_row_sum<HubF4>(hubs.part + (size_t)hub[rd] * hubs.ld + tx * 4, hubs.ld, en[rd] - st[rd], hubs.shift);
                 *reinterpret_cast<float4*>(tile + lr * LDT + tx * 4) = acc;
             }
 
@@ -543,7 +543,7 @@ int launch_level(int N, const int* row_ptr, const int* col_idx, const float* val
     long long blocks = (ntiles + kWavesPerBlock - 1) / kWavesPerBlock;
     if (blocks > kNumCU * 8) blocks = kNumCU * 8;          // persistent beyond this
     hipLaunchKernelGGL((s2v_level_kernel<C, DENSE>), dim3((unsigned)blocks), dim3(kBlock), 0, s,
-                       N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs.row_slot, hubs.agg, hubs.ld);
+                       N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs);
     GNNHIP_LAUNCH_CHECK("s2v_level");
     return GNNHIP_OK;
 }
@@ -636,7 +636,7 @@ int level_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* c
             // them, so the product need not write them (on R-MAT more than half of the rows)
             const bool skip_empty = level_stream_covers(N, C);
             if (int rc = spmm_dispatch(N, N, C, nnz, 1.f, row_ptr, col_idx, val, h_in, C, 0.f, h_out, C, s, same_graph, skip_empty, plan)) return rc;
-            const HubPlan none{nullptr, nullptr, 0};
+            const HubPlan none{};
             if (int rc = level_stream_dispatch(N, C, true, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, none, false, s);
                 rc != GNNHIP_EUNSUPPORTED)
                 return rc;
@@ -646,7 +646,7 @@ int level_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* c
             default: return launch_level<64, true>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, none, s);
             }
         }
-        HubPlan hubs{nullptr, nullptr, 0};
+        HubPlan hubs{};
         if (int rc = hub_prepass(N, C, nnz, row_ptr, col_idx, val, h_in, C, s, &hubs, same_graph, relu_in, kHubThreshold, kHubChunk, -1,
                                  plan ? &plan->row_hub : nullptr))
             return rc;
@@ -703,7 +703,7 @@ int level_backward_dispatch(int N, int C, long long nnz, const int* row_ptr, con
     if (!(aligned16(dz) && aligned16(W) && aligned16(u) && aligned16(g_prev) && (!gate || aligned16(gate)) && (!acc || aligned16(acc))))
         return GNNHIP_EUNSUPPORTED;
     if (N >= kHubMinRows && nnz >= two_step_degree() * (long long)N) return GNNHIP_EUNSUPPORTED;     // dense and skewed: balanced SpMM
-    HubPlan hubs{nullptr, nullptr, 0};
+    HubPlan hubs{};
     if (int rc = hub_prepass(N, C, nnz, row_ptr, col_idx, val, dz, C, s, &hubs, false, false)) return rc;
     return level_stream_backward_dispatch(N, C, row_ptr, col_idx, val, dz, W, u, g_prev, gate, acc, hubs, s);
 }

@@ -100,7 +100,7 @@ __global__ __launch_bounds__(kBlock, MINW) void s2v_level_stream_kernel(
     int N, const int* __restrict__ row_ptr, const int* __restrict__ col_idx, const float* __restrict__ val,
     const float* __restrict__ h_in, const float* __restrict__ W, const float* __restrict__ msg,
     const float* __restrict__ bias, float* __restrict__ h_out,
-    const int* __restrict__ hub_slot, const float* __restrict__ hub_agg, int hub_ld, float* __restrict__ agg_out = nullptr,
+    HubPlan hubs, float* __restrict__ agg_out = nullptr,
     float* __restrict__ acc_io = nullptr)
 {
     constexpr int G = C / 4;             // lanes per gathered row
@@ -323,11 +323,11 @@ __global__ __launch_bounds__(kBlock, MINW) void s2v_level_stream_kernel(
                     const int lr = grp * ROUNDS + rd;
                     const int cnt = rp[rd + 1] - rp[rd];
                     bool coop = cnt > kWaveLongRow || (rp[rd + 1] > kBufEntries && cnt > 0);
-                    if (coop && hub_slot && cnt > kHubThreshold) {
-                        const int slot = hub_slot[row0 + lr];          // summed by the pre-pass unless -1
-                        if (slot >= 0) {
+                    if (coop && hubs.row_chunk && cnt > kHubThreshold) {
+                        const int chunk = hubs.row_chunk[row0 + lr];    // summed by the pre-pass unless -1
+                        if (chunk >= 0) {
                             *reinterpret_cast<float4*>(tile + lr * LDT + tx * 4) =
-                                *reinterpret_cast<const float4*>(hub_agg + (size_t)slot * hub_ld + tx * 4);
+                                hub_row_sum<HubF4>(hubs.part + (size_t)chunk * hubs.ld + tx * 4, hubs.ld, cnt, hubs.shift);
                             coop = false;
                         }
                     }
@@ -480,7 +480,7 @@ int launch_level_stream_p(int N, const int* row_ptr, const int* col_idx, const f
     const long long resident = (long long)kNumCU * kMinW;  // a workgroup puts one wavefront on each SIMD
     if (blocks > resident) blocks = resident;              // persistent beyond this
     hipLaunchKernelGGL((s2v_level_stream_kernel<C, DENSE, kWLds, kMinW, RELU_IN, PIPE>), dim3((unsigned)blocks), dim3(kBlock), 0, s,
-                       N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs.row_slot, hubs.agg, hubs.ld);
+                       N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs);
     GNNHIP_LAUNCH_CHECK("s2v_level_stream");
     return GNNHIP_OK;
 }
@@ -522,8 +522,7 @@ int launch_level_stream_backward(int N, const int* row_ptr, const int* col_idx, 
     const long long resident = (long long)kNumCU * kMinW;
     if (blocks > resident) blocks = resident;
     hipLaunchKernelGGL((s2v_level_stream_kernel<C, false, kWLds, kMinW, false, false, true>), dim3((unsigned)blocks), dim3(kBlock), 0, s,
-                       N, row_ptr, col_idx, val, x, W, gate, (const float*)nullptr, out, hubs.row_slot, hubs.agg,
-                       hubs.ld, agg_out, acc);
+                       N, row_ptr, col_idx, val, x, W, gate, (const float*)nullptr, out, hubs, agg_out, acc);
     GNNHIP_LAUNCH_CHECK("s2v_level_stream (backward)");
     return GNNHIP_OK;
 }

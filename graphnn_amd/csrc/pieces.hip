@@ -151,6 +151,7 @@ template <> struct PV<4> {
     static __device__ __forceinline__ void store(float* p, T v) { *reinterpret_cast<float4*>(p) = v; }
     static __device__ __forceinline__ void fma(T& a, float s, T x) { a.x += s * x.x; a.y += s * x.y; a.z += s * x.z; a.w += s * x.w; }
     static __device__ __forceinline__ T axpby(T a, float b, T c) { return make_float4(a.x + b * c.x, a.y + b * c.y, a.z + b * c.z, a.w + b * c.w); }
+    static __device__ __forceinline__ T add(T a, T b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
 };
 template <> struct PV<1> {
     using T = float;
@@ -159,6 +160,7 @@ template <> struct PV<1> {
     static __device__ __forceinline__ void store(float* p, T v) { *p = v; }
     static __device__ __forceinline__ void fma(T& a, float s, T x) { a += s * x; }
     static __device__ __forceinline__ T axpby(T a, float b, T c) { return a + b * c; }
+    static __device__ __forceinline__ T add(T a, T b) { return a + b; }
 };
 
 // One lane group (G lanes) per piece, pieces taken in order; die x (workgroups x, x + 8, ...) walks the
@@ -287,7 +289,7 @@ __global__ __launch_bounds__(kBlock) void piece_tail_kernel(int m, int n, float 
 // so that every step keeps all groups busy and a step of rows without entries waits for nothing (taking the rows in
 // order, a group for each run of eight, every wavefront carried the chain row -> sums of the row eight steps long:
 // 0.29 ms where the bytes take 0.15).  A row's pieces are added in piece order, eight loads in flight.  A row of
-// more than kCombineLong pieces takes its sum from the balanced pass (hub_slot / hub_agg) when that pass has one
+// more than kCombineLong pieces takes its sum from the balanced pass (hubs) when that pass has one
 // for it: on a power-law matrix the rows of many pieces sit next to each other.
 // skip_empty: rows without entries are not written (the consumer knows them from row_ptr and reads zeros instead);
 // otherwise they get beta * C.
@@ -296,7 +298,7 @@ constexpr int kCombineChunk = 256;
 template <int VEC, int ITERS>
 __global__ __launch_bounds__(kBlock) void piece_combine_kernel(
     int m, int n, const int* __restrict__ first, const int* __restrict__ pfirst, const float* __restrict__ part, int ldp, float beta,
-    float* __restrict__ C, int ldc, int logG, const int* __restrict__ hub_slot, const float* __restrict__ hub_agg, int hub_ld,
+    float* __restrict__ C, int ldc, int logG, HubPlan hubs,
     int skip_empty)
 {
     using V = PV<VEC>;
@@ -346,13 +348,13 @@ __global__ __launch_bounds__(kBlock) void piece_combine_kernel(
         typename V::T acc[ITERS];
 #pragma unroll
         for (int it = 0; it < ITERS; ++it) acc[it] = V::zero();
-        int hslot = -1;
-        if (hub_slot && e - b > kCombineLong) hslot = hub_slot[row];
-        if (hslot >= 0) {
+        int chunk = -1;
+        if (hubs.row_chunk && e - b > kCombineLong) chunk = hubs.row_chunk[row];
+        if (chunk >= 0) {
 #pragma unroll
             for (int it = 0; it < ITERS; ++it) {
                 const int col0 = (sub + it * G) * VEC;
-                if (col0 < n) acc[it] = V::load(hub_agg + (size_t)hslot * hub_ld + col0);
+                if (col0 < n) acc[it] = hub_row_sum<V>(hubs.part + (size_t)chunk * hubs.ld + col0, hubs.ld, e - b, hubs.shift);
             }
         } else {
             for (int p = b; p < e; p += kFlight) {
@@ -552,7 +554,7 @@ int run_pieces(const CsrPlan* p, const Width& w, int n, float alpha, const float
     const unsigned grid = (unsigned)(((long long)m + kBlock - 1) / kBlock);        // a wavefront per 64 rows
 #define GNNHIP_PIECES_COMBINE(V, I)                                                                                             \
     hipLaunchKernelGGL((piece_combine_kernel<V, I>), dim3(grid), dim3(kBlock), 0, s, m, n, p->first, p->pfirst, part, ldp, beta, C, ldc, \
-                       logG, hubs.row_slot, hubs.agg, hubs.ld, skip_empty ? 1 : 0)
+                       logG, hubs, skip_empty ? 1 : 0)
     if (w.vec4) {
         if (iters <= 1) GNNHIP_PIECES_COMBINE(4, 1);
         else if (iters == 2) GNNHIP_PIECES_COMBINE(4, 2);

@@ -69,7 +69,7 @@ template <int VEC, int ITERS>
 __global__ __launch_bounds__(kBlock) void spmm_rowgroup_kernel(
     int m, int n, float alpha, const int* __restrict__ row_ptr, const int* __restrict__ col_idx,
     const float* __restrict__ val, const float* __restrict__ B, int ldb, float beta, float* C, int ldc,
-    int logG, int long_row, const int* __restrict__ hub_slot, const float* __restrict__ hub_agg, int hub_ld)
+    int logG, int long_row, HubPlan hubs)
 {
     using V = Vec<VEC>;
     __shared__ int lr_list[kBlock];
@@ -91,9 +91,10 @@ __global__ __launch_bounds__(kBlock) void spmm_rowgroup_kernel(
     int start = 0, end = 0;
     if (row < m && owner) { start = row_ptr[row]; end = row_ptr[row + 1]; }
     // a row summed by the hub pre-pass only scales and stores
-    int hslot = -1;
-    if (hub_slot && end - start > kHubThreshold) hslot = hub_slot[row];
-    if (hslot >= 0) end = start;
+    int hub = -1;
+    const int entries = end - start;
+    if (hubs.row_chunk && entries > kHubThreshold) hub = hubs.row_chunk[row];
+    if (hub >= 0) end = start;
     const bool deferred = one_row ? (end > start) : (end - start > long_row);
     if (deferred) {
         if (sub == 0) lr_list[atomicAdd(&lr_count, 1)] = (int)row;
@@ -139,7 +140,7 @@ __global__ __launch_bounds__(kBlock) void spmm_rowgroup_kernel(
         for (int it = 0; it < ITERS; ++it) {
             const int col0 = (sub + it * G) * VEC;
             if (col0 < n) {
-                if (hslot >= 0) acc[it] = V::axpby(V::zero(), alpha, V::load(hub_agg + (size_t)hslot * hub_ld + col0));
+                if (hub >= 0) acc[it] = V::axpby(V::zero(), alpha, hub_row_sum<V>(hubs.part + (size_t)hub * hubs.ld + col0, hubs.ld, entries, hubs.shift));
                 float* dst = C + (size_t)row * ldc + col0;
                 if (beta == 0.f) V::store(dst, acc[it]);
                 else V::store(dst, V::axpby(acc[it], beta, V::load(dst)));
@@ -219,8 +220,7 @@ int launch_slab(int m, int n, float alpha, const int* row_ptr, const int* col_id
     const int groups_per_block = one_row ? 1 : kBlock >> logG;
     const unsigned blocks = ceil_div_u((size_t)m, (size_t)groups_per_block);
     hipLaunchKernelGGL((spmm_rowgroup_kernel<VEC, ITERS>), dim3(blocks), dim3(kBlock), 0, s,
-                       m, n, alpha, row_ptr, col_idx, val, B, ldb, beta, C, ldc, logG, one_row ? -1 : kLongRow, hubs.row_slot, hubs.agg,
-                       hubs.ld);
+                       m, n, alpha, row_ptr, col_idx, val, B, ldb, beta, C, ldc, logG, one_row ? -1 : kLongRow, hubs);
     GNNHIP_LAUNCH_CHECK("spmm_rowgroup");
     return GNNHIP_OK;
 }
