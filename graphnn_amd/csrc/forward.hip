@@ -13,7 +13,7 @@ int input_dispatch(int N, int K, int C, const float* X, const float* Wn2l, float
 int level_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* h_in,
                    const float* W, const float* msg, const float* bias, float* h_out, hipStream_t s, bool same_graph = false,
                    bool relu_in = false, CsrPlan* plan = nullptr, bool inference = false);
-bool level_accepts_relu_input(int N, int C, long long nnz);
+bool level_accepts_relu_input(int N, int C);
 int level_backward_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* dz,
                             const float* W, float* u, float* g_prev, const float* gate, float* acc, hipStream_t s);
 int readout_dispatch(int B, int C, int H, int Q, const int* s_row_ptr, const int* s_col_idx, const float* s_val,
@@ -145,7 +145,7 @@ int forward_any(int N, int B, int K, int C, int H, int Q, int L, long long a_nnz
 {
     // With at least one level, and a level kernel that can read its input through ReLU, h0 = ReLU(msg) is
     // never stored: the first level gathers from msg.
-    const bool lazy_h0 = L >= 1 && level_accepts_relu_input(N, C, a_nnz);
+    const bool lazy_h0 = L >= 1 && level_accepts_relu_input(N, C) && aligned16(msg) && aligned16(h_a) && aligned16(h_b) && aligned16(W_conv);
     int rc = input_any(N, K, C, X, W_n2l, msg, lazy_h0 ? nullptr : h_a, s);
     if (rc) return rc;
     float* cur = lazy_h0 ? msg : h_a;

@@ -593,10 +593,8 @@ int input_dispatch(int N, int K, int C, const float* X, const float* Wn2l, float
 // Whether level_dispatch can read h_in as ReLU(h_in): then the forward does not store h0 = ReLU(msg) and the
 // first level gathers from msg (one activation less written, and the gathered rows are the ones the level
 // reads anyway).
-bool level_accepts_relu_input(int N, int C, long long nnz)
+bool level_accepts_relu_input(int N, int C)
 {
-    const bool two_step = N >= kHubMinRows && nnz >= two_step_degree() * (long long)N;
-    if (two_step) return false;
     return level_wide_covers(N, C) || level_stream_covers(N, C);
 }
 
@@ -630,12 +628,12 @@ int level_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* c
         // mean degree, and dense graphs in practice are the skewed ones, so large graphs with at least
         // kTwoStepMeanDegree entries per row take the two launches.
         const bool two_step = N >= kHubMinRows && nnz >= two_step_degree() * (long long)N;
-        if (relu_in && (two_step || !level_stream_covers(N, C))) return GNNHIP_EUNSUPPORTED;
+        if (relu_in && !level_stream_covers(N, C)) return GNNHIP_EUNSUPPORTED;
         if (two_step) {
             // the streaming kernel knows the rows without entries from row_ptr and takes them as zero without reading
             // them, so the product need not write them (on R-MAT more than half of the rows)
             const bool skip_empty = level_stream_covers(N, C);
-            if (int rc = spmm_dispatch(N, N, C, nnz, 1.f, row_ptr, col_idx, val, h_in, C, 0.f, h_out, C, s, same_graph, skip_empty, plan)) return rc;
+            if (int rc = spmm_dispatch(N, N, C, nnz, 1.f, row_ptr, col_idx, val, h_in, C, 0.f, h_out, C, s, same_graph, skip_empty, plan, relu_in)) return rc;
             const HubPlan none{};
             if (int rc = level_stream_dispatch(N, C, true, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, none, false, s);
                 rc != GNNHIP_EUNSUPPORTED)
@@ -668,7 +666,6 @@ int level_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* c
     // gather becomes a plain read of the row, 12 bytes of indices against C * 4 of data) for the contraction
     // and the epilogue.
     if (N >= kHubMinRows && nnz >= two_step_degree() * (long long)N) {
-        if (relu_in) return GNNHIP_EUNSUPPORTED;
         void *tmp = nullptr, *idp = nullptr;
         if (int rc = stream_scratch(s, sizeof(float) * (size_t)N * C, &tmp)) return rc;
         if (int rc = stream_scratch_slot(s, 5, sizeof(int) * (3 * (size_t)N + 1), &idp)) return rc;
@@ -676,7 +673,7 @@ int level_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* c
         int* id_row_ptr = static_cast<int*>(idp);
         int* id_col = id_row_ptr + N + 1;
         float* id_val = reinterpret_cast<float*>(id_col + N);
-        if (int rc = spmm_dispatch(N, N, C, nnz, 1.f, row_ptr, col_idx, val, h_in, C, 0.f, agg, C, s, same_graph, false, plan)) return rc;
+        if (int rc = spmm_dispatch(N, N, C, nnz, 1.f, row_ptr, col_idx, val, h_in, C, 0.f, agg, C, s, same_graph, false, plan, relu_in)) return rc;
         hipLaunchKernelGGL(identity_csr_kernel, dim3((unsigned)(((long long)N + kBlock) / kBlock)), dim3(kBlock), 0, s, N, id_row_ptr,
                            id_col, id_val);
         GNNHIP_LAUNCH_CHECK("identity_csr");

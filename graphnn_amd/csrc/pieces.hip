@@ -152,6 +152,7 @@ template <> struct PV<4> {
     static __device__ __forceinline__ void fma(T& a, float s, T x) { a.x += s * x.x; a.y += s * x.y; a.z += s * x.z; a.w += s * x.w; }
     static __device__ __forceinline__ T axpby(T a, float b, T c) { return make_float4(a.x + b * c.x, a.y + b * c.y, a.z + b * c.z, a.w + b * c.w); }
     static __device__ __forceinline__ T add(T a, T b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
+    static __device__ __forceinline__ T relu(T a) { return relu_ref4(a); }
 };
 template <> struct PV<1> {
     using T = float;
@@ -161,6 +162,7 @@ template <> struct PV<1> {
     static __device__ __forceinline__ void fma(T& a, float s, T x) { a += s * x; }
     static __device__ __forceinline__ T axpby(T a, float b, T c) { return a + b * c; }
     static __device__ __forceinline__ T add(T a, T b) { return a + b; }
+    static __device__ __forceinline__ T relu(T a) { return relu_ref(a); }
 };
 
 // One lane group (G lanes) per piece, pieces taken in order; die x (workgroups x, x + 8, ...) walks the
@@ -171,7 +173,8 @@ template <> struct PV<1> {
 // the group reads G column indices and values at once and hands them round by shuffle, four gathers in flight.
 // The sum of a piece that is all of its row goes to C (as sum + beta * C, what the combining pass would make of
 // it), the others to the place of their piece id among the partial sums.
-template <int VEC, int ITERS>
+// RELU_IN: the rows of B count as ReLU(B).
+template <int VEC, int ITERS, bool RELU_IN>
 __global__ __launch_bounds__(kBlock) void piece_sum_kernel(
     const int* __restrict__ count, int n, float alpha, const int* __restrict__ at, const int* __restrict__ col_idx, const float* __restrict__ val,
     const float* __restrict__ B, int ldb, float* __restrict__ part, int ldp, int logG, const int* __restrict__ target, float beta,
@@ -216,7 +219,7 @@ __global__ __launch_bounds__(kBlock) void piece_sum_kernel(
                             x[u] = (j + u < cnt) ? V::load(B + (size_t)cj[u] * ldb + col0) : V::zero();
 #pragma unroll
                         for (int u = 0; u < 4; ++u)
-                            if (j + u < cnt) V::fma(acc[it], vj[u], x[u]);
+                            if (j + u < cnt) V::fma(acc[it], vj[u], RELU_IN ? V::relu(x[u]) : x[u]);
                     }
                 }
             }
@@ -242,7 +245,7 @@ __global__ __launch_bounds__(kBlock) void piece_sum_kernel(
 // stand-in piece without entries, so neither the sums nor the combining pass write it; its result,
 // alpha * A[row] * B + beta * C[row], is formed here.  Rows are taken from the last one down, a lane group each;
 // the first row that ends inside the plan ends the walk.
-template <int VEC, int ITERS>
+template <int VEC, int ITERS, bool RELU_IN>
 __global__ __launch_bounds__(kBlock) void piece_tail_kernel(int m, int n, float alpha, const int* __restrict__ row_ptr, int cap,
                                                             const int* __restrict__ col_idx, const float* __restrict__ val,
                                                             const float* __restrict__ B, int ldb, float beta, float* __restrict__ C,
@@ -267,7 +270,10 @@ __global__ __launch_bounds__(kBlock) void piece_tail_kernel(int m, int n, float 
 #pragma unroll
             for (int it = 0; it < ITERS; ++it) {
                 const int col0 = (sub + it * G) * VEC;
-                if (col0 < n) V::fma(acc[it], v, V::load(B + (size_t)c * ldb + col0));
+                if (col0 < n) {
+                    const typename V::T x = V::load(B + (size_t)c * ldb + col0);
+                    V::fma(acc[it], v, RELU_IN ? V::relu(x) : x);
+                }
             }
         }
         float* dst = C + (size_t)row * ldc;
@@ -505,14 +511,14 @@ void point_plan(CsrPlan* p, const Layout& L, char* head, char* body)
 // The sums over a finished plan: C = alpha * A * B + beta * C.  `part` holds p->pslots rows of w.ldp floats;
 // hub_store: where the balanced pass over P keeps its arrays (null: stream scratch slot 1, which the caller has reserved).
 int run_pieces(const CsrPlan* p, const Width& w, int n, float alpha, const float* B, int ldb, float beta, float* C, int ldc, float* part,
-               bool hub_planned, HubStore* hub_store, bool skip_empty, hipStream_t s)
+               bool hub_planned, HubStore* hub_store, bool skip_empty, bool relu_in, hipStream_t s)
 {
     const int m = p->m, logG = w.logG, iters = w.iters, ldp = w.ldp;
     // workgroups for the bound on the pieces of one die, times the number of dies; those past the real count leave at once
     const int sum_groups = kBlock >> logG;
     const unsigned sgrid = (unsigned)(((p->slots + kNumXCD - 1) / kNumXCD + 1 + sum_groups - 1) / sum_groups) * kNumXCD;
 #define GNNHIP_PIECES_LAUNCH(V, I)                                                                                            \
-    hipLaunchKernelGGL((piece_sum_kernel<V, I>), dim3(sgrid), dim3(kBlock), 0, s, p->first + m, n, alpha, p->at, p->col_ord, p->val_ord, B, \
+    hipLaunchKernelGGL((relu_in ? piece_sum_kernel<V, I, true> : piece_sum_kernel<V, I, false>), dim3(sgrid), dim3(kBlock), 0, s, p->first + m, n, alpha, p->at, p->col_ord, p->val_ord, B, \
                        ldb, part, ldp, logG, p->target, beta, C, ldc)
     if (w.vec4) {
         if (iters <= 1) GNNHIP_PIECES_LAUNCH(4, 1);
@@ -529,7 +535,7 @@ int run_pieces(const CsrPlan* p, const Width& w, int n, float alpha, const float
         // rows past the host's entry count, if any (a plan of its own knows the matrix's count)
         const unsigned tgrid = kNumCU * 4;
 #define GNNHIP_PIECES_TAIL(V, I)                                                                                                   \
-    hipLaunchKernelGGL((piece_tail_kernel<V, I>), dim3(tgrid), dim3(kBlock), 0, s, m, n, alpha, p->row_ptr, (int)p->nnz, p->col_idx, p->val, \
+    hipLaunchKernelGGL((relu_in ? piece_tail_kernel<V, I, true> : piece_tail_kernel<V, I, false>), dim3(tgrid), dim3(kBlock), 0, s, m, n, alpha, p->row_ptr, (int)p->nnz, p->col_idx, p->val, \
                        B, ldb, beta, C, ldc, logG)
         if (w.vec4) {
             if (iters <= 1) GNNHIP_PIECES_TAIL(4, 1);
@@ -598,7 +604,7 @@ CsrPlan* as_csr_plan(void* handle)
 // All scratch is taken before the first launch: GNNHIP_ENOMEM and GNNHIP_EUNSUPPORTED leave C untouched.
 int spmm_pieces_dispatch(int m, int k, int n, long long nnz, float alpha, const int* row_ptr, const int* col_idx, const float* val,
                          const float* B, int ldb, float beta, float* C, int ldc, hipStream_t s, bool reuse_plan, bool skip_empty_rows,
-                         CsrPlan* plan)
+                         CsrPlan* plan, bool relu_in)
 {
     const Width w = width_of(n, B, ldb, C, ldc);
     if (!w.ok) return GNNHIP_EUNSUPPORTED;
@@ -629,7 +635,7 @@ int spmm_pieces_dispatch(int m, int k, int n, long long nnz, float alpha, const 
             if (int rc = pool_acquire_exact(&plan->combine_hub.base, hb)) return rc;
             plan->combine_hub.bytes = hb;
         }
-        return run_pieces(plan, w, n, alpha, B, ldb, beta, C, ldc, plan->part, true, &plan->combine_hub, skip_empty_rows, s);
+        return run_pieces(plan, w, n, alpha, B, ldb, beta, C, ldc, plan->part, true, &plan->combine_hub, skip_empty_rows, relu_in, s);
     }
 
     if (!pieces_route_applies(m, nnz)) return GNNHIP_EUNSUPPORTED;
@@ -663,7 +669,7 @@ int spmm_pieces_dispatch(int m, int k, int n, long long nnz, float alpha, const 
         if (int rc = count_pieces(&p, (int)nnz, reinterpret_cast<int*>(temp + L.o_seg), s)) return rc;
         if (int rc = order_pieces(&p, (int)nnz, L, temp, s)) return rc;
     }
-    return run_pieces(&p, w, n, alpha, B, ldb, beta, C, ldc, static_cast<float*>(pbase), planned, nullptr, skip_empty_rows, s);
+    return run_pieces(&p, w, n, alpha, B, ldb, beta, C, ldc, static_cast<float*>(pbase), planned, nullptr, skip_empty_rows, relu_in, s);
 }
 
 }  // namespace gnnhip

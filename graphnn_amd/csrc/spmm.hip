@@ -47,6 +47,7 @@ template <> struct Vec<4> {
     static __device__ __forceinline__ void fma(T& a, float s, T x) { a.x += s * x.x; a.y += s * x.y; a.z += s * x.z; a.w += s * x.w; }
     static __device__ __forceinline__ T axpby(T a, float b, T c) { return make_float4(a.x + b * c.x, a.y + b * c.y, a.z + b * c.z, a.w + b * c.w); }
     static __device__ __forceinline__ T add(T a, T b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
+    static __device__ __forceinline__ T relu(T a) { return relu_ref4(a); }
 };
 template <> struct Vec<1> {
     using T = float;
@@ -56,6 +57,7 @@ template <> struct Vec<1> {
     static __device__ __forceinline__ void fma(T& a, float s, T x) { a += s * x; }
     static __device__ __forceinline__ T axpby(T a, float b, T c) { return a + b * c; }
     static __device__ __forceinline__ T add(T a, T b) { return a + b; }
+    static __device__ __forceinline__ T relu(T a) { return relu_ref(a); }
 };
 
 // One row per group of G = 1 << logG lanes.  A lane owns column slabs
@@ -65,7 +67,8 @@ template <> struct Vec<1> {
 // and the partial sums are added through LDS in group order.
 // long_row < 0: one row per workgroup, summed that way whatever its length (few, long rows: pooling 1,024 nodes
 // into each of 4,096 subgraphs ran one workgroup per compute unit with a lane group per row: 0.265 ms).
-template <int VEC, int ITERS>
+// RELU_IN: the rows of B count as ReLU(B).
+template <int VEC, int ITERS, bool RELU_IN>
 __global__ __launch_bounds__(kBlock) void spmm_rowgroup_kernel(
     int m, int n, float alpha, const int* __restrict__ row_ptr, const int* __restrict__ col_idx,
     const float* __restrict__ val, const float* __restrict__ B, int ldb, float beta, float* C, int ldc,
@@ -129,7 +132,7 @@ __global__ __launch_bounds__(kBlock) void spmm_rowgroup_kernel(
                         x[u] = (j + u < cnt) ? V::load(B + (size_t)cj[u] * ldb + col0) : V::zero();
 #pragma unroll
                     for (int u = 0; u < 4; ++u)
-                        if (j + u < cnt) V::fma(acc[it], vj[u], x[u]);
+                        if (j + u < cnt) V::fma(acc[it], vj[u], RELU_IN ? V::relu(x[u]) : x[u]);
                 }
             }
         }
@@ -171,7 +174,7 @@ __global__ __launch_bounds__(kBlock) void spmm_rowgroup_kernel(
 #pragma unroll
                     for (int u = 0; u < 4; ++u) x[u] = V::load(B + (size_t)c4[u] * ldb + col0);
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) V::fma(acc[it], v4[u], x[u]);
+                    for (int u = 0; u < 4; ++u) V::fma(acc[it], v4[u], RELU_IN ? V::relu(x[u]) : x[u]);
                 }
             }
         }
@@ -181,7 +184,10 @@ __global__ __launch_bounds__(kBlock) void spmm_rowgroup_kernel(
 #pragma unroll
             for (int it = 0; it < ITERS; ++it) {
                 const int col0 = (sub + it * G) * VEC;
-                if (col0 < n) V::fma(acc[it], v0, V::load(B + (size_t)c0 * ldb + col0));
+                if (col0 < n) {
+                    const typename V::T x = V::load(B + (size_t)c0 * ldb + col0);
+                    V::fma(acc[it], v0, RELU_IN ? V::relu(x) : x);
+                }
             }
         }
 
@@ -215,11 +221,12 @@ inline int ilog2_ceil(int x)
 
 template <int VEC, int ITERS>
 int launch_slab(int m, int n, float alpha, const int* row_ptr, const int* col_idx, const float* val,
-                const float* B, int ldb, float beta, float* C, int ldc, int logG, const HubPlan& hubs, bool one_row, hipStream_t s)
+                const float* B, int ldb, float beta, float* C, int ldc, int logG, const HubPlan& hubs, bool one_row, bool relu_in, hipStream_t s)
 {
     const int groups_per_block = one_row ? 1 : kBlock >> logG;
     const unsigned blocks = ceil_div_u((size_t)m, (size_t)groups_per_block);
-    hipLaunchKernelGGL((spmm_rowgroup_kernel<VEC, ITERS>), dim3(blocks), dim3(kBlock), 0, s,
+    const auto kernel = relu_in ? spmm_rowgroup_kernel<VEC, ITERS, true> : spmm_rowgroup_kernel<VEC, ITERS, false>;
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kBlock), 0, s,
                        m, n, alpha, row_ptr, col_idx, val, B, ldb, beta, C, ldc, logG, one_row ? -1 : kLongRow, hubs);
     GNNHIP_LAUNCH_CHECK("spmm_rowgroup");
     return GNNHIP_OK;
@@ -230,21 +237,21 @@ int launch_slab(int m, int n, float alpha, const int* row_ptr, const int* col_id
 // Shared with the fused forward: C = alpha*A*B + beta*C on stream s.
 int spmm_dispatch(int m, int k, int n, long long nnz, float alpha, const int* row_ptr, const int* col_idx, const float* val,
                   const float* B, int ldb, float beta, float* C, int ldc, hipStream_t s, bool reuse_plan, bool skip_empty_rows,
-                  CsrPlan* plan)
+                  CsrPlan* plan, bool relu_in)
 {
     // large matrices with many entries per row (power-law graphs): rows cut into pieces, summed in column order.  That
     // route takes all its scratch (about 40 bytes per entry of A + 4 n bytes per piece) before its first launch: when
     // the device cannot give it, C is untouched and the row-group route below, which needs far less, does the product.
-    if (int rc = spmm_pieces_dispatch(m, k, n, nnz, alpha, row_ptr, col_idx, val, B, ldb, beta, C, ldc, s, reuse_plan, skip_empty_rows, plan);
+    if (int rc = spmm_pieces_dispatch(m, k, n, nnz, alpha, row_ptr, col_idx, val, B, ldb, beta, C, ldc, s, reuse_plan, skip_empty_rows, plan, relu_in);
         rc != GNNHIP_EUNSUPPORTED && rc != GNNHIP_ENOMEM)
         return rc;
-    return spmm_plain_dispatch(m, k, n, nnz, alpha, row_ptr, col_idx, val, B, ldb, beta, C, ldc, s, reuse_plan, plan ? &plan->row_hub : nullptr);
+    return spmm_plain_dispatch(m, k, n, nnz, alpha, row_ptr, col_idx, val, B, ldb, beta, C, ldc, s, reuse_plan, plan ? &plan->row_hub : nullptr, relu_in);
 }
 
 // The row-group route alone (with its pass over very long rows); nnz may be an upper bound.  row_hub: where a plan's
 // owner keeps the pass's arrays across calls.
 int spmm_plain_dispatch(int m, int k, int n, long long nnz, float alpha, const int* row_ptr, const int* col_idx, const float* val,
-                        const float* B, int ldb, float beta, float* C, int ldc, hipStream_t s, bool reuse_plan, HubStore* row_hub)
+                        const float* B, int ldb, float beta, float* C, int ldc, hipStream_t s, bool reuse_plan, HubStore* row_hub, bool relu_in)
 {
     (void)k;
     // few rows of hundreds of entries each (sum-pooling into subgraphs): a workgroup per row instead of a lane group
@@ -263,15 +270,15 @@ int spmm_plain_dispatch(int m, int k, int n, long long nnz, float alpha, const i
         float* Cs = C + col0;
         int rc;
         HubPlan hubs;
-        if ((rc = hub_prepass(m, w, nnz, row_ptr, col_idx, val, Bs, ldb, s, &hubs, reuse_plan && n <= slab_max, false, kHubThreshold, kHubChunk, -1, row_hub))) return rc;
+        if ((rc = hub_prepass(m, w, nnz, row_ptr, col_idx, val, Bs, ldb, s, &hubs, reuse_plan && n <= slab_max, relu_in, kHubThreshold, kHubChunk, -1, row_hub))) return rc;
         if (vec4) {
-            if (iters <= 1) rc = launch_slab<4, 1>(m, w, alpha, row_ptr, col_idx, val, Bs, ldb, beta, Cs, ldc, logG, hubs, one_row, s);
-            else if (iters == 2) rc = launch_slab<4, 2>(m, w, alpha, row_ptr, col_idx, val, Bs, ldb, beta, Cs, ldc, logG, hubs, one_row, s);
-            else rc = launch_slab<4, 4>(m, w, alpha, row_ptr, col_idx, val, Bs, ldb, beta, Cs, ldc, logG, hubs, one_row, s);
+            if (iters <= 1) rc = launch_slab<4, 1>(m, w, alpha, row_ptr, col_idx, val, Bs, ldb, beta, Cs, ldc, logG, hubs, one_row, relu_in, s);
+            else if (iters == 2) rc = launch_slab<4, 2>(m, w, alpha, row_ptr, col_idx, val, Bs, ldb, beta, Cs, ldc, logG, hubs, one_row, relu_in, s);
+            else rc = launch_slab<4, 4>(m, w, alpha, row_ptr, col_idx, val, Bs, ldb, beta, Cs, ldc, logG, hubs, one_row, relu_in, s);
         } else {
-            if (iters <= 1) rc = launch_slab<1, 1>(m, w, alpha, row_ptr, col_idx, val, Bs, ldb, beta, Cs, ldc, logG, hubs, one_row, s);
-            else if (iters == 2) rc = launch_slab<1, 2>(m, w, alpha, row_ptr, col_idx, val, Bs, ldb, beta, Cs, ldc, logG, hubs, one_row, s);
-            else rc = launch_slab<1, 4>(m, w, alpha, row_ptr, col_idx, val, Bs, ldb, beta, Cs, ldc, logG, hubs, one_row, s);
+            if (iters <= 1) rc = launch_slab<1, 1>(m, w, alpha, row_ptr, col_idx, val, Bs, ldb, beta, Cs, ldc, logG, hubs, one_row, relu_in, s);
+            else if (iters == 2) rc = launch_slab<1, 2>(m, w, alpha, row_ptr, col_idx, val, Bs, ldb, beta, Cs, ldc, logG, hubs, one_row, relu_in, s);
+            else rc = launch_slab<1, 4>(m, w, alpha, row_ptr, col_idx, val, Bs, ldb, beta, Cs, ldc, logG, hubs, one_row, relu_in, s);
         }
         if (rc) return rc;
     }
