@@ -269,12 +269,11 @@ struct CsrPlan {
 constexpr unsigned kCsrPlanMagic = 0x43535250u;
 
 // spmm.hip: C = alpha*A*B + beta*C on stream s (A is [m,k]); reuse_plan as for hub_prepass.
-// skip_empty_rows: rows of A without entries are left as they are in C (the caller treats them as zero; beta must be 0).
 // plan: a plan made for exactly these arrays (then nnz is exact and reuse_plan is ignored), or null.
 // relu_in: the rows of B count as ReLU(B) (a first level that reads msg where h0 = ReLU(msg) was not stored).
 int spmm_dispatch(int m, int k, int n, long long nnz, float alpha, const int* row_ptr, const int* col_idx, const float* val,
                   const float* B, int ldb, float beta, float* C, int ldc, hipStream_t s, bool reuse_plan = false,
-                  bool skip_empty_rows = false, CsrPlan* plan = nullptr, bool relu_in = false);
+                  CsrPlan* plan = nullptr, bool relu_in = false);
 
 // sort.hip
 int exclusive_scan_i32(int* x, long long n, int* seg_scratch, hipStream_t s);
@@ -288,9 +287,19 @@ int spmm_plain_dispatch(int m, int k, int n, long long nnz, float alpha, const i
 // pieces.hip: C = alpha*A*B + beta*C for large matrices with many entries per row, the rows cut into pieces that
 // are summed in the order of their first column; GNNHIP_EUNSUPPORTED (nothing launched, C untouched) where the caller
 // keeps its own route, GNNHIP_ENOMEM likewise when the device cannot give the scratch
+// sums (beta must be 0): the rows of several pieces are not put together in C; the consumer adds up their sums itself
+struct PieceSums {
+    const int* first = nullptr;        // [m + 1] pieces before a row: a row of one piece has its result in C, one of none is zero
+    const int* pfirst = nullptr;       // [m + 1] sums of rows of several pieces before a row
+    const float* part = nullptr;       // those sums, [.., ld]
+    int ld = 0;
+    unsigned bytes = 0;                // of part; less than 4 GiB
+    HubPlan hubs;                      // of the rows of more than kCombineLong pieces (a row's entries are its pieces)
+};
+constexpr int kCombineLong = 8;        // pieces; the balanced pass sums the pieces of such rows
 int spmm_pieces_dispatch(int m, int k, int n, long long nnz, float alpha, const int* row_ptr, const int* col_idx, const float* val,
-                         const float* B, int ldb, float beta, float* C, int ldc, hipStream_t s, bool reuse_plan, bool skip_empty_rows,
-                         CsrPlan* plan, bool relu_in);
+                         const float* B, int ldb, float beta, float* C, int ldc, hipStream_t s, bool reuse_plan,
+                         CsrPlan* plan, bool relu_in, PieceSums* sums = nullptr);
 // whether a matrix of this shape takes the pieces route at all (the width of the dense operand decides the rest)
 bool pieces_route_applies(int m, long long nnz);
 CsrPlan* as_csr_plan(void* handle);      // null unless handle is a live plan

@@ -40,6 +40,8 @@ bool level_stream_covers(int N, int C);
 int level_stream_backward_dispatch(int N, int C, const int* row_ptr, const int* col_idx, const float* val, const float* x,
                                    const float* W, float* agg_out, float* out, const float* gate, float* acc, const HubPlan& hubs,
                                    hipStream_t s);
+int level_stream_pieces_dispatch(int N, int C, const float* W, const float* msg, const float* bias, float* h_out, const PieceSums& sums,
+                                 hipStream_t s);
 // input_wide.hip
 int input_wide_dispatch(int N, int K, int C, const float* X, const float* Wn2l, float* msg, float* h0, hipStream_t s);
 // level_wide.hip
@@ -630,10 +632,13 @@ int level_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* c
         const bool two_step = N >= kHubMinRows && nnz >= two_step_degree() * (long long)N;
         if (relu_in && !level_stream_covers(N, C)) return GNNHIP_EUNSUPPORTED;
         if (two_step) {
-            // the streaming kernel knows the rows without entries from row_ptr and takes them as zero without reading
-            // them, so the product need not write them (on R-MAT more than half of the rows)
-            const bool skip_empty = level_stream_covers(N, C);
-            if (int rc = spmm_dispatch(N, N, C, nnz, 1.f, row_ptr, col_idx, val, h_in, C, 0.f, h_out, C, s, same_graph, skip_empty, plan, relu_in)) return rc;
+            if (level_stream_covers(N, C)) {
+                PieceSums sums;
+                const int rc = spmm_pieces_dispatch(N, N, C, nnz, 1.f, row_ptr, col_idx, val, h_in, C, 0.f, h_out, C, s, same_graph, plan, relu_in, &sums);
+                if (rc == GNNHIP_OK) return level_stream_pieces_dispatch(N, C, W, msg, bias, h_out, sums, s);
+                if (rc != GNNHIP_EUNSUPPORTED && rc != GNNHIP_ENOMEM) return rc;
+            }
+            if (int rc = spmm_dispatch(N, N, C, nnz, 1.f, row_ptr, col_idx, val, h_in, C, 0.f, h_out, C, s, same_graph, plan, relu_in)) return rc;
             const HubPlan none{};
             if (int rc = level_stream_dispatch(N, C, true, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, none, false, s);
                 rc != GNNHIP_EUNSUPPORTED)
@@ -673,7 +678,7 @@ int level_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* c
         int* id_row_ptr = static_cast<int*>(idp);
         int* id_col = id_row_ptr + N + 1;
         float* id_val = reinterpret_cast<float*>(id_col + N);
-        if (int rc = spmm_dispatch(N, N, C, nnz, 1.f, row_ptr, col_idx, val, h_in, C, 0.f, agg, C, s, same_graph, false, plan, relu_in)) return rc;
+        if (int rc = spmm_dispatch(N, N, C, nnz, 1.f, row_ptr, col_idx, val, h_in, C, 0.f, agg, C, s, same_graph, plan, relu_in)) return rc;
         hipLaunchKernelGGL(identity_csr_kernel, dim3((unsigned)(((long long)N + kBlock) / kBlock)), dim3(kBlock), 0, s, N, id_row_ptr,
                            id_col, id_val);
         GNNHIP_LAUNCH_CHECK("identity_csr");

@@ -27,8 +27,11 @@
 // the register count and doubles the wavefronts per SIMD.
 //
 // DENSE: A * h_in has already been written to h_out (by the SpMM); the tile is read from there
-// and overwritten in place.  Rows of A without entries (known from row_ptr) are taken as zero and not read, so the
-// product may leave them unwritten.
+// and overwritten in place.
+// PIECES (with DENSE): the product has written the rows of one piece only (pieces.hip); a row of several pieces is put
+// together here from their sums, four of each of the tile's rows in flight, and a row without entries is zero without a
+// read.  Putting the rows together in a launch of its own cost 155 us per level on R-MAT with
+// 4M rows; here it adds 60 to the 545 us of the level.
 //
 // Algorithmic bytes: 4(N+1) + 8E + 12NC + 4C^2.
 #include "gnnhip_internal.h"
@@ -95,13 +98,13 @@ __device__ __forceinline__ void sum4(float4& acc, float w, const float4 (&x)[4])
 // CSR matrix: W is read transposed, the aggregated rows A' x are also stored (agg_out: they are the other
 // factor of the weight gradient).  No ReLU and no bias; `msg`, when given, is the embedding whose ReLU the
 // gradient passes next: out = out where msg > 0, else 0, and acc_io (when given) += out.
-template <int C, bool DENSE, bool WLDS, int MINW, bool RELU_IN, bool PIPE, bool BWD = false>
+template <int C, bool DENSE, bool WLDS, int MINW, bool RELU_IN, bool PIPE, bool BWD = false, bool PIECES = false>
 __global__ __launch_bounds__(kBlock, MINW) void s2v_level_stream_kernel(
     int N, const int* __restrict__ row_ptr, const int* __restrict__ col_idx, const float* __restrict__ val,
     const float* __restrict__ h_in, const float* __restrict__ W, const float* __restrict__ msg,
     const float* __restrict__ bias, float* __restrict__ h_out,
     HubPlan hubs, float* __restrict__ agg_out = nullptr,
-    float* __restrict__ acc_io = nullptr)
+    float* __restrict__ acc_io = nullptr, PieceSums sums = PieceSums())
 {
     constexpr int G = C / 4;             // lanes per gathered row
     constexpr int RPR = kWave / G;       // lane groups per wavefront
@@ -219,6 +222,20 @@ __global__ __launch_bounds__(kBlock, MINW) void s2v_level_stream_kernel(
     int rpq[PIPE ? RN : 1], offq[PIPE ? ROUNDS : 1];
     float wq[PIPE ? ROUNDS : 1];
     float4 x[ROUNDS][4];                     // gathered rows: four entries of each of the lane group's rows
+    // PIECES: rp counts pieces (sums.first in place of row_ptr), pp the sums of rows of several pieces
+    const rsrc_t pf_rsrc = make_rsrc(PIECES ? sums.pfirst : nullptr, PIECES ? (unsigned)(N + 1) * 4u : 0u);
+    const rsrc_t part_rsrc = make_rsrc(PIECES ? sums.part : nullptr, PIECES ? sums.bytes : 0u);
+    int pp[PIECES ? RN : 1], ppn[PIECES ? RN : 1];
+    auto load_pp = [&](int tile) {
+#pragma unroll
+        for (int i = 0; i < RN; ++i) ppn[i] = buf_load_i(pf_rsrc, (tile * 16 + grp * ROUNDS + i) * 4, 0);
+    };
+    if constexpr (PIECES) {
+        load_pp(tile_id < ntiles ? tile_id : ntiles);
+#pragma unroll
+        for (int i = 0; i < RN; ++i) pp[i] = ppn[i];
+        load_pp(tile_n1 < ntiles ? tile_n1 : ntiles);
+    }
     if constexpr (PIPE && !DENSE) {
         load_rp(rpq, tile_n2 < ntiles ? tile_n2 : ntiles);
         load_first_batch(rpn, offq, wq);
@@ -237,12 +254,73 @@ __global__ __launch_bounds__(kBlock, MINW) void s2v_level_stream_kernel(
         float w0n[ROUNDS];
 
         if constexpr (DENSE) {
-            // a row of A without entries was not written by the product: it counts as zero and is not read (an
-            // offset past the end returns zeros without a memory access)
             float4 xd[ROUNDS];
 #pragma unroll
-            for (int rd = 0; rd < ROUNDS; ++rd)
-                xd[rd] = buf_load4(out_rsrc, rp[rd + 1] > rp[rd] ? row_off(row0 + grp * ROUNDS + rd) : kPastEndRow, 0);
+            for (int rd = 0; rd < ROUNDS; ++rd)      // an offset past the end returns zeros without a memory access
+                xd[rd] = buf_load4(out_rsrc, !PIECES || rp[rd + 1] - rp[rd] == 1 ? row_off(row0 + grp * ROUNDS + rd) : kPastEndRow, 0);
+            if constexpr (PIECES) {
+                // Two trips to memory at most for what rows have in general: the first four sums of every row of several
+                // pieces and the place of the balanced pass's sum for a row of more than kCombineLong, then sums 5 to 8
+                // and that pass's sum.  (Rows past N read pointers of 0: no pieces.)
+                int most = 0;
+#pragma unroll
+                for (int rd = 0; rd < ROUNDS; ++rd) most = max(most, pp[rd + 1] - pp[rd]);
+                if (__any(most > 0)) {
+                    const bool long_rows = __any(most > kCombineLong);
+                    float4 y[ROUNDS][4];
+                    int chunk[ROUNDS];
+                    auto part_off = [&](int id) { return (int)((unsigned)id * (unsigned)kRowBytes + tx_off); };
+                    auto add_y = [&]() {
+#pragma unroll
+                        for (int rd = 0; rd < ROUNDS; ++rd)
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {
+                                xd[rd].x += y[rd][i].x; xd[rd].y += y[rd][i].y; xd[rd].z += y[rd][i].z; xd[rd].w += y[rd][i].w;
+                            }
+                    };
+#pragma unroll
+                    for (int rd = 0; rd < ROUNDS; ++rd) {
+                        const int np = pp[rd + 1] - pp[rd];
+                        chunk[rd] = -1;
+                        if (long_rows && np > kCombineLong && sums.hubs.row_chunk) chunk[rd] = sums.hubs.row_chunk[row0 + grp * ROUNDS + rd];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) y[rd][i] = buf_load4(part_rsrc, i < np && np <= kCombineLong ? part_off(pp[rd] + i) : kBufPastEnd, 0);
+                    }
+                    add_y();
+                    if (__any(most > 4)) {
+                        static_assert(kCombineLong == 8, "two turns of four");
+#pragma unroll
+                        for (int rd = 0; rd < ROUNDS; ++rd) {
+                            const int np = pp[rd + 1] - pp[rd];
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) y[rd][i] = buf_load4(part_rsrc, i < np - 4 && np <= kCombineLong ? part_off(pp[rd] + 4 + i) : kBufPastEnd, 0);
+                            if (chunk[rd] >= 0) y[rd][0] = *reinterpret_cast<const float4*>(sums.hubs.part + (size_t)chunk[rd] * sums.hubs.ld + tx * 4);
+                        }
+                        add_y();
+                    }
+                    if (long_rows) {
+#pragma unroll
+                        for (int rd = 0; rd < ROUNDS; ++rd) {
+                            const int np = pp[rd + 1] - pp[rd];
+                            if (chunk[rd] >= 0) {
+                                const int nc = (np + (1 << sums.hubs.shift) - 1) >> sums.hubs.shift;
+                                for (int u = 1; u < nc; ++u) {
+                                    const float4 z = *reinterpret_cast<const float4*>(sums.hubs.part + (size_t)(chunk[rd] + u) * sums.hubs.ld + tx * 4);
+                                    xd[rd].x += z.x; xd[rd].y += z.y; xd[rd].z += z.z; xd[rd].w += z.w;
+                                }
+                            } else if (np > kCombineLong) {              // no room in the balanced pass
+                                for (int u = 0; u < np; ++u) {
+                                    const float4 z = buf_load4(part_rsrc, part_off(pp[rd] + u), 0);
+                                    xd[rd].x += z.x; xd[rd].y += z.y; xd[rd].z += z.z; xd[rd].w += z.w;
+                                }
+                            }
+                        }
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < RN; ++i) pp[i] = ppn[i];
+                load_pp(tile_n2 < ntiles ? tile_n2 : ntiles);
+            }
             load_rp(rpnn, tile_n2 < ntiles ? tile_n2 : ntiles);      // behind the rows: the pointers of the tile after next
 #pragma unroll
             for (int rd = 0; rd < ROUNDS; ++rd)
@@ -485,6 +563,25 @@ int launch_level_stream_p(int N, const int* row_ptr, const int* col_idx, const f
     return GNNHIP_OK;
 }
 
+// The level over sums of pieces: h_out holds the rows of one piece.
+template <int C>
+int launch_level_stream_pieces(int N, const float* W, const float* msg, const float* bias, float* h_out, const PieceSums& sums, hipStream_t s)
+{
+    const long long ntiles = ((long long)N + 15) / 16;
+    long long blocks = (ntiles + kWavesPerBlock - 1) / kWavesPerBlock;
+    constexpr int kMinW = 4;
+    // 1,009 workgroups, a prime: on R-MAT matrices the rows of many pieces are those whose index has few bits
+    // set, and a power-of-two stride between a wavefront's tiles would give all of them to the
+    // same wavefronts (4M rows, C = 64: 1,024 workgroups 828 us, 1,023 669, 1,009 605).
+    const long long resident = (long long)kNumCU * kMinW - 15;
+    if (blocks > resident) blocks = resident;
+    hipLaunchKernelGGL((s2v_level_stream_kernel<C, true, C == 64, kMinW, false, false, false, true>), dim3((unsigned)blocks), dim3(kBlock), 0, s,
+                       N, sums.first, (const int*)nullptr, (const float*)nullptr, (const float*)nullptr, W, msg, bias, h_out, HubPlan(),
+                       (float*)nullptr, (float*)nullptr, sums);
+    GNNHIP_LAUNCH_CHECK("s2v_level_stream (pieces)");
+    return GNNHIP_OK;
+}
+
 template <int C, bool DENSE, bool RELU_IN>
 int launch_level_stream(int N, const int* row_ptr, const int* col_idx, const float* val, const float* h_in,
                         const float* W, const float* msg, const float* bias, float* h_out, const HubPlan& hubs,
@@ -547,6 +644,17 @@ int level_stream_backward_dispatch(int N, int C, const int* row_ptr, const int* 
     case 16: return launch_level_stream_backward<16>(N, row_ptr, col_idx, val, x, W, agg_out, out, gate, acc, hubs, s);
     case 32: return launch_level_stream_backward<32>(N, row_ptr, col_idx, val, x, W, agg_out, out, gate, acc, hubs, s);
     default: return launch_level_stream_backward<64>(N, row_ptr, col_idx, val, x, W, agg_out, out, gate, acc, hubs, s);
+    }
+}
+
+// The level whose product left sums of pieces (spmm_pieces_dispatch with `sums`, into h_out); sums.ld must be C.
+int level_stream_pieces_dispatch(int N, int C, const float* W, const float* msg, const float* bias, float* h_out, const PieceSums& sums,
+                                 hipStream_t s)
+{
+    switch (C) {
+    case 16: return launch_level_stream_pieces<16>(N, W, msg, bias, h_out, sums, s);
+    case 32: return launch_level_stream_pieces<32>(N, W, msg, bias, h_out, sums, s);
+    default: return launch_level_stream_pieces<64>(N, W, msg, bias, h_out, sums, s);
     }
 }
 

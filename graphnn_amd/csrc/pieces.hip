@@ -297,15 +297,12 @@ __global__ __launch_bounds__(kBlock) void piece_tail_kernel(int m, int n, float 
 // 0.29 ms where the bytes take 0.15).  A row's pieces are added in piece order, eight loads in flight.  A row of
 // more than kCombineLong pieces takes its sum from the balanced pass (hubs) when that pass has one
 // for it: on a power-law matrix the rows of many pieces sit next to each other.
-// skip_empty: rows without entries are not written (the consumer knows them from row_ptr and reads zeros instead);
-// otherwise they get beta * C.
-constexpr int kCombineLong = 8;         // pieces; the balanced pass cuts such rows into chunks of kCombineChunk pieces
-constexpr int kCombineChunk = 256;
+// Rows without entries get beta * C.
+constexpr int kCombineChunk = 256;      // pieces per chunk of the balanced pass over rows of more than kCombineLong
 template <int VEC, int ITERS>
 __global__ __launch_bounds__(kBlock) void piece_combine_kernel(
     int m, int n, const int* __restrict__ first, const int* __restrict__ pfirst, const float* __restrict__ part, int ldp, float beta,
-    float* __restrict__ C, int ldc, int logG, HubPlan hubs,
-    int skip_empty)
+    float* __restrict__ C, int ldc, int logG, HubPlan hubs)
 {
     using V = PV<VEC>;
     constexpr int kFlight = 8;
@@ -321,7 +318,7 @@ __global__ __launch_bounds__(kBlock) void piece_combine_kernel(
     if (r < m) pieces = first[r + 1] - first[r];
     const bool several = r < m && pieces > 1;
     if (several) { pb = pfirst[r]; pe = pfirst[r + 1]; }
-    unsigned long long none_left = __ballot(r < m && pieces == 0 && !skip_empty);
+    unsigned long long none_left = __ballot(r < m && pieces == 0);
     unsigned long long several_left = __ballot(several);
     // the next ngroups rows of a kind, one per lane group (-1: none left for this group)
     auto take = [&](unsigned long long& left) {
@@ -511,7 +508,7 @@ void point_plan(CsrPlan* p, const Layout& L, char* head, char* body)
 // The sums over a finished plan: C = alpha * A * B + beta * C.  `part` holds p->pslots rows of w.ldp floats;
 // hub_store: where the balanced pass over P keeps its arrays (null: stream scratch slot 1, which the caller has reserved).
 int run_pieces(const CsrPlan* p, const Width& w, int n, float alpha, const float* B, int ldb, float beta, float* C, int ldc, float* part,
-               bool hub_planned, HubStore* hub_store, bool skip_empty, bool relu_in, hipStream_t s)
+               bool hub_planned, HubStore* hub_store, bool relu_in, PieceSums* sums, hipStream_t s)
 {
     const int m = p->m, logG = w.logG, iters = w.iters, ldp = w.ldp;
     // workgroups for the bound on the pieces of one die, times the number of dies; those past the real count leave at once
@@ -557,10 +554,14 @@ int run_pieces(const CsrPlan* p, const Width& w, int n, float alpha, const float
     if (int rc = hub_prepass(m, n, p->pslots, p->pfirst, nullptr, nullptr, part, ldp, s, &hubs, hub_planned, false, kCombineLong,
                              kCombineChunk, p->nnz / ((long long)kCombineLong * kPiece + 1) + 1, hub_store))
         return rc;
+    if (sums) {
+        *sums = PieceSums{p->first, p->pfirst, part, ldp, (unsigned)((size_t)p->pslots * ldp * sizeof(float)), hubs};
+        return GNNHIP_OK;
+    }
     const unsigned grid = (unsigned)(((long long)m + kBlock - 1) / kBlock);        // a wavefront per 64 rows
 #define GNNHIP_PIECES_COMBINE(V, I)                                                                                             \
     hipLaunchKernelGGL((piece_combine_kernel<V, I>), dim3(grid), dim3(kBlock), 0, s, m, n, p->first, p->pfirst, part, ldp, beta, C, ldc, \
-                       logG, hubs, skip_empty ? 1 : 0)
+                       logG, hubs)
     if (w.vec4) {
         if (iters <= 1) GNNHIP_PIECES_COMBINE(4, 1);
         else if (iters == 2) GNNHIP_PIECES_COMBINE(4, 2);
@@ -603,14 +604,14 @@ CsrPlan* as_csr_plan(void* handle)
 // reused when reuse_plan says the previous call on the stream had the same matrix (structure and values).
 // All scratch is taken before the first launch: GNNHIP_ENOMEM and GNNHIP_EUNSUPPORTED leave C untouched.
 int spmm_pieces_dispatch(int m, int k, int n, long long nnz, float alpha, const int* row_ptr, const int* col_idx, const float* val,
-                         const float* B, int ldb, float beta, float* C, int ldc, hipStream_t s, bool reuse_plan, bool skip_empty_rows,
-                         CsrPlan* plan, bool relu_in)
+                         const float* B, int ldb, float beta, float* C, int ldc, hipStream_t s, bool reuse_plan, CsrPlan* plan, bool relu_in,
+                         PieceSums* sums)
 {
     const Width w = width_of(n, B, ldb, C, ldc);
     if (!w.ok) return GNNHIP_EUNSUPPORTED;
-    if (skip_empty_rows && beta != 0.f) return set_error(GNNHIP_EINVAL, "rows without entries can only be skipped when beta is 0");
+    auto sums_fit = [&](long long pslots) { return (unsigned long long)pslots * w.ldp * 4ull < (1ull << 32); };
     if (plan) {
-        if (!plan->has_pieces) return GNNHIP_EUNSUPPORTED;
+        if (!plan->has_pieces || (sums && !sums_fit(plan->pslots))) return GNNHIP_EUNSUPPORTED;
         const size_t need = sizeof(float) * (size_t)(plan->pslots > 0 ? plan->pslots : 1) * w.ldp;
         if (plan->part_bytes < need) {
             if (plan->part) {
@@ -635,7 +636,7 @@ int spmm_pieces_dispatch(int m, int k, int n, long long nnz, float alpha, const 
             if (int rc = pool_acquire_exact(&plan->combine_hub.base, hb)) return rc;
             plan->combine_hub.bytes = hb;
         }
-        return run_pieces(plan, w, n, alpha, B, ldb, beta, C, ldc, plan->part, true, &plan->combine_hub, skip_empty_rows, relu_in, s);
+        return run_pieces(plan, w, n, alpha, B, ldb, beta, C, ldc, plan->part, true, &plan->combine_hub, relu_in, sums, s);
     }
 
     if (!pieces_route_applies(m, nnz)) return GNNHIP_EUNSUPPORTED;
@@ -645,6 +646,7 @@ int spmm_pieces_dispatch(int m, int k, int n, long long nnz, float alpha, const 
     p.slots = slots_bound(m, nnz);
     p.pslots = pslots_bound(nnz) < p.slots ? pslots_bound(nnz) : p.slots;
     p.has_pieces = true;
+    if (sums && !sums_fit(p.pslots)) return GNNHIP_EUNSUPPORTED;
     const Layout L = layout_of(m, nnz, p.slots, p.pslots);
     void *base = nullptr, *pbase = nullptr, *hbase = nullptr;
     if (int rc = stream_scratch_slot(s, 3, L.head_bytes + L.body_bytes + L.temp_bytes, &base)) return rc;
@@ -669,7 +671,7 @@ int spmm_pieces_dispatch(int m, int k, int n, long long nnz, float alpha, const 
         if (int rc = count_pieces(&p, (int)nnz, reinterpret_cast<int*>(temp + L.o_seg), s)) return rc;
         if (int rc = order_pieces(&p, (int)nnz, L, temp, s)) return rc;
     }
-    return run_pieces(&p, w, n, alpha, B, ldb, beta, C, ldc, static_cast<float*>(pbase), planned, nullptr, skip_empty_rows, relu_in, s);
+    return run_pieces(&p, w, n, alpha, B, ldb, beta, C, ldc, static_cast<float*>(pbase), planned, nullptr, relu_in, sums, s);
 }
 
 }  // namespace gnnhip

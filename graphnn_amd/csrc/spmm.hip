@@ -236,13 +236,13 @@ int launch_slab(int m, int n, float alpha, const int* row_ptr, const int* col_id
 
 // Shared with the fused forward: C = alpha*A*B + beta*C on stream s.
 int spmm_dispatch(int m, int k, int n, long long nnz, float alpha, const int* row_ptr, const int* col_idx, const float* val,
-                  const float* B, int ldb, float beta, float* C, int ldc, hipStream_t s, bool reuse_plan, bool skip_empty_rows,
+                  const float* B, int ldb, float beta, float* C, int ldc, hipStream_t s, bool reuse_plan,
                   CsrPlan* plan, bool relu_in)
 {
     // large matrices with many entries per row (power-law graphs): rows cut into pieces, summed in column order.  That
     // route takes all its scratch (about 40 bytes per entry of A + 4 n bytes per piece) before its first launch: when
     // the device cannot give it, C is untouched and the row-group route below, which needs far less, does the product.
-    if (int rc = spmm_pieces_dispatch(m, k, n, nnz, alpha, row_ptr, col_idx, val, B, ldb, beta, C, ldc, s, reuse_plan, skip_empty_rows, plan, relu_in);
+    if (int rc = spmm_pieces_dispatch(m, k, n, nnz, alpha, row_ptr, col_idx, val, B, ldb, beta, C, ldc, s, reuse_plan, plan, relu_in);
         rc != GNNHIP_EUNSUPPORTED && rc != GNNHIP_ENOMEM)
         return rc;
     return spmm_plain_dispatch(m, k, n, nnz, alpha, row_ptr, col_idx, val, B, ldb, beta, C, ldc, s, reuse_plan, plan ? &plan->row_hub : nullptr, relu_in);
@@ -313,5 +313,5 @@ extern "C" int gnnhip_spmm_csr_planned_f32(void* plan, int n, float alpha, const
     GNNHIP_REQUIRE(ldb >= n && ldc >= n, "leading dimension smaller than n in spmm_csr_planned (ldb=%d ldc=%d n=%d)", ldb, ldc, n);
     GNNHIP_REQUIRE(p->k == 0 || B, "null dense operand in spmm_csr_planned");
     if (int rc = require_ready()) return rc;
-    return spmm_dispatch(p->m, p->k, n, p->nnz, alpha, p->row_ptr, p->col_idx, p->val, B, ldb, beta, C, ldc, as_stream(stream), false, false, p);
+    return spmm_dispatch(p->m, p->k, n, p->nnz, alpha, p->row_ptr, p->col_idx, p->val, B, ldb, beta, C, ldc, as_stream(stream), false, p);
 }
