@@ -277,6 +277,7 @@ int spmm_dispatch(int m, int k, int n, long long nnz, float alpha, const int* ro
 
 // sort.hip
 int exclusive_scan_i32(int* x, long long n, int* seg_scratch, hipStream_t s);
+int exclusive_scan_pair_i32(int* x, int* y, long long n, int* seg_scratch, hipStream_t s);
 size_t radix_hist_ints(long long n);
 size_t radix_seg_ints(long long n);
 int radix_order_by_digit(const unsigned* keys, long long n, int shift, unsigned* keys_out, unsigned* perm_out, int* hist, int* seg,

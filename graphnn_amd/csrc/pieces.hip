@@ -444,7 +444,7 @@ Layout layout_of(int m, long long nnz, long long slots, long long pslots)
     L.body_bytes = off;
     off = 0;
     const size_t longest = (size_t)(slots + 1 > (long long)m + 1 ? slots + 1 : (long long)m + 1);
-    L.o_seg = carve(sizeof(int) * (longest / 4096 + 2 + radix_seg_ints(slots)));
+    L.o_seg = carve(sizeof(int) * (2 * (longest / 4096 + 2) + radix_seg_ints(slots)));
     L.o_rec = carve(sizeof(PieceRec) * (size_t)slots);
     L.o_ord = carve(sizeof(PieceRec) * (size_t)slots);
     L.o_keys = carve(sizeof(unsigned) * (size_t)slots);
@@ -462,8 +462,7 @@ constexpr unsigned kElemGrid = kNumCU * 16;
 int count_pieces(CsrPlan* p, int cap, int* seg, hipStream_t s)
 {
     hipLaunchKernelGGL(piece_count_kernel, dim3(kElemGrid), dim3(kBlock), 0, s, p->m, p->row_ptr, cap, p->first, p->pfirst);
-    if (int rc = exclusive_scan_i32(p->first, (long long)p->m + 1, seg, s)) return rc;
-    if (int rc = exclusive_scan_i32(p->pfirst, (long long)p->m + 1, seg, s)) return rc;
+    if (int rc = exclusive_scan_pair_i32(p->first, p->pfirst, (long long)p->m + 1, seg, s)) return rc;
     GNNHIP_LAUNCH_CHECK("spmm_pieces count");
     return GNNHIP_OK;
 }

@@ -3,18 +3,23 @@
 // graphnn builds the CSR operands of a batch on the host by walking per-node lists
 // (src/nn/msg_pass.cpp:46-177); row i of such a matrix lists the payloads of the pairs
 // whose key is i, in insertion order.  That is a stable sort of the pair indices by key.
-// Here: a least-significant-digit radix sort (8-bit digits, as many passes as the key range
-// needs) whose every pass is stable, then the row pointers from the sorted keys.
+// Here: a least-significant-digit radix sort (digits of 8, 10 or 11 bits, so that up to 4M rows
+// take two passes) whose every pass is stable, then the row pointers from the sorted keys.
+// A matrix and its transpose are grouped side by side in the same launches.
 //
 // One pass over n pairs, tiles of 2048 pairs per workgroup:
-//   histogram   per tile, 256 LDS counters -> hist[digit][tile]
-//   scan        exclusive scan of hist in digit-major order (three launches, any length)
+//   histogram   per tile, an LDS counter per digit -> hist[digit][tile]
+//   scan        exclusive scan of hist in digit-major order
 //   scatter     a wavefront takes 512 consecutive pairs of the tile, 64 at a time; lanes with
-//               the same digit find each other with eight ballots, their rank is the running
+//               the same digit find each other with a ballot per bit, their rank is the running
 //               count of that digit in the wavefront's segment plus the number of lower lanes;
 //               segment counts are then prefixed over the four wavefronts.  Destination =
 //               scanned hist[digit][tile] + rank.  Order inside a digit = input order: stable.
 // No atomics on global memory; the result is a pure function of the input.
+//
+// At the sizes of training batches (10^5 to 10^6 pairs) a launch costs about what it does: 659,010 pairs on 299,536
+// rows, both ways, took 36 launches and 206 us with 8-bit digits, one grouping after the other; 9 launches and
+// 114 us now.
 #include "gnnhip_internal.h"
 
 namespace gnnhip {
@@ -25,22 +30,47 @@ constexpr int kWavesPerBlock = kBlock / kWave;
 constexpr int kItems = 8;
 constexpr int kTile = kBlock * kItems;          // 2048 pairs per workgroup
 constexpr int kSeg = kTile / kWavesPerBlock;    // 512 consecutive pairs per wavefront
-constexpr int kDigits = 256;
 
-__global__ __launch_bounds__(kBlock) void radix_hist_kernel(const unsigned* __restrict__ keys, long long n, int shift,
-                                                             int ntiles, int* __restrict__ hist)
+// What one grouping reads and writes, and its part of the scratch.
+struct GroupJob {
+    const int* key;                              // as the caller holds them, read by the first pass
+    const int* payload;
+    const float* val_in;                         // null: 1
+    int key_stride, payload_stride;
+    int* row_ptr;
+    int* col_idx;
+    float* val;
+    unsigned *k0, *k1, *v0, *v1;                 // keys and pair indices, before and after a pass
+    int *hist, *seg;
+};
+constexpr int kMaxJobs = 2;                      // blockIdx.y picks one
+struct GroupJobs { GroupJob job[kMaxJobs]; };
+
+// a key outside [0, rows) is a caller error, but it must not send the row-pointer kernels out of bounds
+__device__ __forceinline__ unsigned first_key(const GroupJob& j, long long i, int rows) { return (unsigned)min(max(j.key[i * j.key_stride], 0), rows - 1); }
+
+template <int BITS>
+__device__ __forceinline__ void tile_histogram(int* h, int ntiles, int* __restrict__ hist)
 {
-    __shared__ int h[kDigits];
-    h[threadIdx.x] = 0;
+    for (int d = threadIdx.x; d < (1 << BITS); d += kBlock) hist[(size_t)d * ntiles + blockIdx.x] = h[d];
+}
+
+// FIRST: the keys are the caller's
+template <int BITS, bool FIRST>
+__global__ __launch_bounds__(kBlock) void radix_hist_kernel(GroupJobs jobs, long long n, int rows, int shift, int ntiles)
+{
+    const GroupJob& j = jobs.job[blockIdx.y];
+    __shared__ int h[1 << BITS];
+    for (int d = threadIdx.x; d < (1 << BITS); d += kBlock) h[d] = 0;
     __syncthreads();
     const long long base = (long long)blockIdx.x * kTile;
 #pragma unroll
     for (int i = 0; i < kItems; ++i) {
         const long long idx = base + i * kBlock + threadIdx.x;
-        if (idx < n) atomicAdd(&h[(keys[idx] >> shift) & (kDigits - 1)], 1);
+        if (idx < n) atomicAdd(&h[((FIRST ? first_key(j, idx, rows) : j.k0[idx]) >> shift) & ((1 << BITS) - 1)], 1);
     }
     __syncthreads();
-    hist[(size_t)threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
+    tile_histogram<BITS>(h, ntiles, j.hist);
 }
 
 // ---- exclusive scan of an int array of any length: segment sums, scan of the sums, apply
@@ -67,8 +97,11 @@ __device__ __forceinline__ int block_scan_256(int v, int* sh, int* total)
     return base + incl - v;
 }
 
-__global__ __launch_bounds__(kBlock) void scan_segment_sums_kernel(const int* __restrict__ x, long long n, int* __restrict__ seg_sum)
+struct ScanJobs { int* x[kMaxJobs]; int* seg[kMaxJobs]; };      // blockIdx.y picks one; all of the same length
+
+__global__ __launch_bounds__(kBlock) void scan_segment_sums_kernel(ScanJobs jobs, long long n)
 {
+    const int* __restrict__ x = jobs.x[blockIdx.y];
     __shared__ int sh[kWavesPerBlock];
     const long long base = (long long)blockIdx.x * kScanSeg + threadIdx.x * 16;
     int s = 0;
@@ -76,12 +109,13 @@ __global__ __launch_bounds__(kBlock) void scan_segment_sums_kernel(const int* __
     for (int i = 0; i < 16; ++i) if (base + i < n) s += x[base + i];
     int tot;
     block_scan_256(s, sh, &tot);
-    if (threadIdx.x == 0) seg_sum[blockIdx.x] = tot;
+    if (threadIdx.x == 0) jobs.seg[blockIdx.y][blockIdx.x] = tot;
 }
 
-// one workgroup: exclusive scan of nseg values in place; total to *total_out (may be null)
-__global__ __launch_bounds__(1024) void scan_small_kernel(int* __restrict__ x, int nseg, int* __restrict__ total_out)
+// one workgroup: exclusive scan of the nseg segment sums in place
+__global__ __launch_bounds__(1024) void scan_small_kernel(ScanJobs jobs, int nseg)
 {
+    int* __restrict__ x = jobs.seg[blockIdx.y];
     __shared__ int wave_tot[1024 / kWave];
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
     const int per = (nseg + 1023) / 1024;
@@ -100,24 +134,49 @@ __global__ __launch_bounds__(1024) void scan_small_kernel(int* __restrict__ x, i
     for (int w = 0; w < wave; ++w) base += wave_tot[w];
     int run = base + incl - local;
     for (int i = lo; i < hi; ++i) { const int v = x[i]; x[i] = run; run += v; }
-    if (tid == 1023 && total_out) *total_out = run;
 }
 
-__global__ __launch_bounds__(kBlock) void scan_apply_kernel(int* __restrict__ x, long long n, const int* __restrict__ seg_off)
+// SUMS: seg holds the segments' sums and the workgroup adds up those before its own; else their scan
+template <bool SUMS>
+__global__ __launch_bounds__(kBlock) void scan_apply_kernel(ScanJobs jobs, long long n)
 {
+    int* __restrict__ x = jobs.x[blockIdx.y];
+    const int* __restrict__ seg = jobs.seg[blockIdx.y];
     __shared__ int sh[kWavesPerBlock];
     const long long base = (long long)blockIdx.x * kScanSeg + threadIdx.x * 16;
     int v[16];
-    int s = 0;
+    int s = 0, ahead = 0;
+    if (SUMS) {
+        for (int i = threadIdx.x; i < (int)blockIdx.x; i += kBlock) ahead += seg[i];
+    }
 #pragma unroll
     for (int i = 0; i < 16; ++i) { v[i] = (base + i < n) ? x[base + i] : 0; s += v[i]; }
     int tot;
-    int run = seg_off[blockIdx.x] + block_scan_256(s, sh, &tot);
+    if (SUMS) block_scan_256(ahead, sh, &ahead);
+    else ahead = seg[blockIdx.x];
+    int run = ahead + block_scan_256(s, sh, &tot);
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
         if (base + i < n) x[base + i] = run;
         run += v[i];
     }
+}
+
+constexpr int kSumsMaxSegments = 2048;          // up to here (8M elements) a workgroup adds up the segments itself
+
+int exclusive_scans(int count, const ScanJobs& jobs, long long n, hipStream_t s)
+{
+    if (n <= 0) return GNNHIP_OK;
+    const int nseg = (int)((n + kScanSeg - 1) / kScanSeg);
+    hipLaunchKernelGGL(scan_segment_sums_kernel, dim3(nseg, count), dim3(kBlock), 0, s, jobs, n);
+    if (nseg <= kSumsMaxSegments) {
+        hipLaunchKernelGGL(scan_apply_kernel<true>, dim3(nseg, count), dim3(kBlock), 0, s, jobs, n);
+    } else {
+        hipLaunchKernelGGL(scan_small_kernel, dim3(1, count), dim3(1024), 0, s, jobs, nseg);
+        hipLaunchKernelGGL(scan_apply_kernel<false>, dim3(nseg, count), dim3(kBlock), 0, s, jobs, n);
+    }
+    GNNHIP_LAUNCH_CHECK("exclusive_scan_i32");
+    return GNNHIP_OK;
 }
 
 }  // namespace
@@ -126,21 +185,24 @@ __global__ __launch_bounds__(kBlock) void scan_apply_kernel(int* __restrict__ x,
 // workgroup walks comfortably; far beyond every use here).
 int exclusive_scan_i32(int* x, long long n, int* seg_scratch, hipStream_t s)
 {
-    if (n <= 0) return GNNHIP_OK;
-    const int nseg = (int)((n + kScanSeg - 1) / kScanSeg);
-    hipLaunchKernelGGL(scan_segment_sums_kernel, dim3(nseg), dim3(kBlock), 0, s, x, n, seg_scratch);
-    hipLaunchKernelGGL(scan_small_kernel, dim3(1), dim3(1024), 0, s, seg_scratch, nseg, (int*)nullptr);
-    hipLaunchKernelGGL(scan_apply_kernel, dim3(nseg), dim3(kBlock), 0, s, x, n, seg_scratch);
-    GNNHIP_LAUNCH_CHECK("exclusive_scan_i32");
-    return GNNHIP_OK;
+    return exclusive_scans(1, ScanJobs{{x, nullptr}, {seg_scratch, nullptr}}, n, s);
+}
+
+// two arrays of n elements in the same launches; seg_scratch: twice as many ints
+int exclusive_scan_pair_i32(int* x, int* y, long long n, int* seg_scratch, hipStream_t s)
+{
+    return exclusive_scans(2, ScanJobs{{x, y}, {seg_scratch, seg_scratch + (n + kScanSeg - 1) / kScanSeg}}, n, s);
 }
 
 namespace {
 
-__global__ __launch_bounds__(kBlock) void radix_scatter_kernel(
-    const unsigned* __restrict__ keys, const unsigned* __restrict__ vals, long long n, int shift, int ntiles,
-    const int* __restrict__ hist_scanned, unsigned* __restrict__ keys_out, unsigned* __restrict__ vals_out, int first_pass)
+// FIRST: the keys are the caller's and a pair's value is its index, or carried[index] where that is given
+template <int BITS, bool FIRST>
+__global__ __launch_bounds__(kBlock) void radix_scatter_kernel(GroupJobs jobs, long long n, int rows, int shift, int ntiles)
 {
+    constexpr int kDigits = 1 << BITS;
+    const GroupJob& j = jobs.job[blockIdx.y];
+    const int* __restrict__ hist_scanned = j.hist;
     __shared__ int cnt[kWavesPerBlock][kDigits];      // running, then total, count of each digit per wavefront segment
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     for (int i = threadIdx.x; i < kWavesPerBlock * kDigits; i += kBlock) (&cnt[0][0])[i] = 0;
@@ -154,13 +216,13 @@ __global__ __launch_bounds__(kBlock) void radix_scatter_kernel(
     for (int i = 0; i < kItems; ++i) {
         const long long idx = seg0 + i * kWave + lane;
         const bool live = idx < n;
-        k[i] = live ? keys[idx] : 0u;
-        v[i] = live ? (first_pass ? (unsigned)idx : vals[idx]) : 0u;
+        k[i] = !live ? 0u : FIRST ? first_key(j, idx, rows) : j.k0[idx];
+        v[i] = !live ? 0u : FIRST ? (unsigned)idx : j.v0[idx];
         const unsigned d = (k[i] >> shift) & (kDigits - 1);
         // lanes of this round with the same digit (dead lanes match nobody)
         unsigned long long same = __ballot(live);
 #pragma unroll
-        for (int b = 0; b < 8; ++b) {
+        for (int b = 0; b < BITS; ++b) {
             const unsigned long long bal = __ballot((d >> b) & 1u);
             same &= ((d >> b) & 1u) ? bal : ~bal;
         }
@@ -174,9 +236,8 @@ __global__ __launch_bounds__(kBlock) void radix_scatter_kernel(
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     }
     __syncthreads();
-    // prefix of the segment counts over the wavefronts, per digit (lane t handles digit t)
-    {
-        const int d = threadIdx.x;
+    // prefix of the segment counts over the wavefronts, per digit
+    for (int d = threadIdx.x; d < kDigits; d += kBlock) {
         int run = 0;
 #pragma unroll
         for (int w = 0; w < kWavesPerBlock; ++w) { const int c = cnt[w][d]; cnt[w][d] = run; run += c; }
@@ -188,52 +249,50 @@ __global__ __launch_bounds__(kBlock) void radix_scatter_kernel(
         if (idx < n) {
             const unsigned d = (k[i] >> shift) & (kDigits - 1);
             const long long dst = (long long)hist_scanned[(size_t)d * ntiles + blockIdx.x] + cnt[wave][d] + rank[i];
-            keys_out[dst] = k[i];
-            vals_out[dst] = v[i];
+            j.k1[dst] = k[i];
+            j.v1[dst] = v[i];
         }
     }
 }
 
-// keys as unsigned, forced into [0, rows): a key outside that range is a caller error, but it must not
-// send the row-pointer kernels out of bounds
-__global__ __launch_bounds__(kBlock) void gather_strided_kernel(const int* __restrict__ src, int stride, long long n, int rows,
-                                                                 unsigned* __restrict__ dst)
-{
-    const long long i = (long long)blockIdx.x * kBlock + threadIdx.x;
-    if (i < n) dst[i] = (unsigned)min(max(src[i * stride], 0), rows - 1);
-}
-
 // row_ptr from the sorted keys: position i opens every row in (key[i-1], key[i]]; the last position closes the rest
-__global__ __launch_bounds__(kBlock) void row_ptr_from_sorted_kernel(const unsigned* __restrict__ keys, long long n, int rows, int* __restrict__ row_ptr)
+__device__ __forceinline__ void open_rows(const GroupJob& j, long long i, long long n, int rows)
 {
-    const long long i = (long long)blockIdx.x * kBlock + threadIdx.x;
-    if (n == 0) {
-        for (long long r = i; r <= rows; r += (long long)gridDim.x * kBlock) row_ptr[r] = 0;
-        return;
-    }
-    if (i >= n) return;
-    const long long k = keys[i];
-    const long long kprev = (i == 0) ? -1 : (long long)keys[i - 1];
-    for (long long r = kprev + 1; r <= k; ++r) row_ptr[r] = (int)i;
+    const long long k = j.k0[i];
+    const long long kprev = (i == 0) ? -1 : (long long)j.k0[i - 1];
+    for (long long r = kprev + 1; r <= k; ++r) j.row_ptr[r] = (int)i;
     if (i == n - 1)
-        for (long long r = k + 1; r <= rows; ++r) row_ptr[r] = (int)n;
+        for (long long r = k + 1; r <= rows; ++r) j.row_ptr[r] = (int)n;
 }
 
-__global__ __launch_bounds__(kBlock) void fill_grouped_kernel(const unsigned* __restrict__ keys_sorted, const unsigned* __restrict__ perm,
-                                                               long long n, const int* __restrict__ payload, int stride,
-                                                               const float* __restrict__ val_in, int average,
-                                                               const int* __restrict__ row_ptr, int* __restrict__ col_idx, float* __restrict__ val)
+__global__ __launch_bounds__(kBlock) void empty_rows_kernel(GroupJobs jobs, int rows)
+{
+    const long long r = (long long)blockIdx.x * kBlock + threadIdx.x;
+    if (r <= rows) jobs.job[blockIdx.y].row_ptr[r] = 0;
+}
+
+__global__ __launch_bounds__(kBlock) void row_ptr_from_sorted_kernel(GroupJobs jobs, long long n, int rows)
+{
+    const long long i = (long long)blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) open_rows(jobs.job[blockIdx.y], i, n, rows);
+}
+
+// AVERAGE: values 1 / row length, which wait for the finished row pointers; otherwise the row pointers are formed here too
+template <bool AVERAGE>
+__global__ __launch_bounds__(kBlock) void fill_grouped_kernel(GroupJobs jobs, long long n, int rows)
 {
     const long long i = (long long)blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
-    const unsigned src = perm[i];
-    col_idx[i] = payload[(long long)src * stride];
-    float w = val_in ? val_in[src] : 1.0f;
-    if (average) {
-        const unsigned r = keys_sorted[i];
-        w = (float)(1.0 / (double)(row_ptr[r + 1] - row_ptr[r]));      // as the reference: double divide, then narrowed
+    const GroupJob& j = jobs.job[blockIdx.y];
+    const unsigned src = j.v0[i];
+    j.col_idx[i] = j.payload[(long long)src * j.payload_stride];
+    float w = j.val_in ? j.val_in[src] : 1.0f;
+    if (AVERAGE) {
+        const unsigned r = j.k0[i];
+        w = (float)(1.0 / (double)(j.row_ptr[r + 1] - j.row_ptr[r]));      // as the reference: double divide, then narrowed
     }
-    val[i] = w;
+    j.val[i] = w;
+    if (!AVERAGE) open_rows(j, i, n, rows);
 }
 
 // row index of every entry of a CSR matrix
@@ -593,22 +652,45 @@ inline size_t round_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 }  // namespace
 
 // One stable pass of the radix sort: perm_out[i] = index of the key that comes i-th when the n keys are ordered by
-// the 8-bit digit (key >> shift) & 255 (equal digits keep their input order); keys_out receives the keys in that
+// the 8-bit digit (key >> shift) & 255 of their 16 bits (equal digits keep their input order); keys_out receives the keys in that
 // order.  With `carried`, perm_out[i] = carried[that index] instead (the order of an earlier pass carried along).
 // hist needs radix_hist_ints(n) ints, seg radix_seg_ints(n).
-size_t radix_hist_ints(long long n) { return (size_t)kDigits * (size_t)((n + kTile - 1) / kTile > 0 ? (n + kTile - 1) / kTile : 1); }
+size_t radix_hist_ints(long long n) { return 256 * (size_t)((n + kTile - 1) / kTile > 0 ? (n + kTile - 1) / kTile : 1); }
 size_t radix_seg_ints(long long n) { return (radix_hist_ints(n) + kScanSeg - 1) / kScanSeg + 1; }
+
+namespace {
+
+template <int BITS>
+int radix_pass(int count, const GroupJobs& jobs, bool first, long long n, int rows, int shift, hipStream_t s)
+{
+    const int ntiles = (int)((n + kTile - 1) / kTile);
+    const dim3 grid(ntiles, count);
+    if (first) hipLaunchKernelGGL((radix_hist_kernel<BITS, true>), grid, dim3(kBlock), 0, s, jobs, n, rows, shift, ntiles);
+    else hipLaunchKernelGGL((radix_hist_kernel<BITS, false>), grid, dim3(kBlock), 0, s, jobs, n, rows, shift, ntiles);
+    ScanJobs scans{};
+    for (int i = 0; i < count; ++i) { scans.x[i] = jobs.job[i].hist; scans.seg[i] = jobs.job[i].seg; }
+    if (int rc = exclusive_scans(count, scans, (long long)(1 << BITS) * ntiles, s)) return rc;
+    if (first) hipLaunchKernelGGL((radix_scatter_kernel<BITS, true>), grid, dim3(kBlock), 0, s, jobs, n, rows, shift, ntiles);
+    else hipLaunchKernelGGL((radix_scatter_kernel<BITS, false>), grid, dim3(kBlock), 0, s, jobs, n, rows, shift, ntiles);
+    GNNHIP_LAUNCH_CHECK("radix pass");
+    return GNNHIP_OK;
+}
+
+}  // namespace
+
 int radix_order_by_digit(const unsigned* keys, long long n, int shift, unsigned* keys_out, unsigned* perm_out, int* hist, int* seg,
                          hipStream_t s, const unsigned* carried)
 {
     if (n <= 0) return GNNHIP_OK;
-    const int ntiles = (int)((n + kTile - 1) / kTile);
-    hipLaunchKernelGGL(radix_hist_kernel, dim3(ntiles), dim3(kBlock), 0, s, keys, n, shift, ntiles, hist);
-    if (int rc = exclusive_scan_i32(hist, (long long)kDigits * ntiles, seg, s)) return rc;
-    hipLaunchKernelGGL(radix_scatter_kernel, dim3(ntiles), dim3(kBlock), 0, s, keys, carried, n, shift, ntiles, hist,
-                       keys_out, perm_out, carried ? 0 : 1);
-    GNNHIP_LAUNCH_CHECK("radix_order_by_digit");
-    return GNNHIP_OK;
+    GroupJobs jobs{};
+    GroupJob& j = jobs.job[0];
+    j.key = reinterpret_cast<const int*>(keys);                  // 16-bit values: never clamped
+    j.key_stride = 1;
+    j.k0 = const_cast<unsigned*>(keys);
+    j.v0 = const_cast<unsigned*>(carried);
+    j.k1 = keys_out; j.v1 = perm_out;
+    j.hist = hist; j.seg = seg;
+    return radix_pass<8>(1, jobs, !carried, n, 1 << 16, shift, s);
 }
 
 // The one-launch grouping where it fits; false: it does not (nothing launched).  With t_row_ptr the same launch
@@ -633,55 +715,72 @@ inline int last_launch_status(const char* what)
     return GNNHIP_OK;
 }
 
-// Groups n pairs by key (0 <= key < rows) keeping input order inside a group:
+// Groups n pairs by key (0 <= key < rows) keeping input order inside a group, `count` groupings side by side:
 //   row_ptr[rows + 1], col_idx[i] = payload of the i-th pair in grouped order,
 //   val[i] = val_in of that pair (or 1), or 1 / group size when average is set.
 // key / payload are read with the given strides (in ints).  Uses scratch slot 0 of the stream.
-int csr_group_pairs(int rows, long long n, const int* key, int key_stride, const int* payload, int payload_stride,
-                    const float* val_in, int average, int* row_ptr, int* col_idx, float* val, hipStream_t s)
+int csr_group_pairs(int count, GroupJobs jobs, int rows, long long n, int average, hipStream_t s)
 {
-    if (csr_group_small(rows, n, key, key_stride, payload, payload_stride, val_in, average, row_ptr, col_idx, val, nullptr, nullptr, nullptr, s))
-        return last_launch_status("csr_group_small");
+    if (n == 0) {
+        hipLaunchKernelGGL(empty_rows_kernel, dim3((unsigned)(((long long)rows + kBlock) / kBlock), count), dim3(kBlock), 0, s, jobs, rows);
+        GNNHIP_LAUNCH_CHECK("csr_group_pairs");
+        return GNNHIP_OK;
+    }
+    int bits = 1;
+    while (bits < 31 && (1ll << bits) < (long long)rows) ++bits;
+    // two passes up to 4M rows: the narrowest digits that do it (the counters of a digit per tile are one more array to scan)
+    const int digit = bits <= 16 ? 8 : bits <= 20 ? 10 : bits <= 22 ? 11 : 8;
     const int ntiles = (int)((n + kTile - 1) / kTile);
-    const long long nhist = (long long)kDigits * (ntiles > 0 ? ntiles : 1);
+    const size_t nhist = ((size_t)1 << digit) * ntiles;
     size_t off = 0;
     auto carve = [&](size_t bytes) { const size_t o = off; off = round_up(off + bytes, 256); return o; };
-    const size_t o_k0 = carve(sizeof(unsigned) * (size_t)(n > 0 ? n : 1)), o_k1 = carve(sizeof(unsigned) * (size_t)(n > 0 ? n : 1));
-    const size_t o_v0 = carve(sizeof(unsigned) * (size_t)(n > 0 ? n : 1)), o_v1 = carve(sizeof(unsigned) * (size_t)(n > 0 ? n : 1));
-    const size_t o_hist = carve(sizeof(int) * (size_t)nhist);
-    const size_t o_seg = carve(sizeof(int) * (size_t)((nhist + kScanSeg - 1) / kScanSeg + 1));
+    size_t o[kMaxJobs][6];
+    for (int i = 0; i < count; ++i) {
+        for (int a = 0; a < 4; ++a) o[i][a] = carve(sizeof(unsigned) * (size_t)n);
+        o[i][4] = carve(sizeof(int) * nhist);
+        o[i][5] = carve(sizeof(int) * ((nhist + kScanSeg - 1) / kScanSeg + 1));
+    }
     void* base = nullptr;
     if (int rc = stream_scratch(s, off, &base)) return rc;
     char* b = static_cast<char*>(base);
-    unsigned* k0 = reinterpret_cast<unsigned*>(b + o_k0);
-    unsigned* k1 = reinterpret_cast<unsigned*>(b + o_k1);
-    unsigned* v0 = reinterpret_cast<unsigned*>(b + o_v0);
-    unsigned* v1 = reinterpret_cast<unsigned*>(b + o_v1);
-    int* hist = reinterpret_cast<int*>(b + o_hist);
-    int* seg = reinterpret_cast<int*>(b + o_seg);
-
-    const unsigned egrid = (unsigned)((n + kBlock - 1) / kBlock);
-    if (n > 0) {
-        hipLaunchKernelGGL(gather_strided_kernel, dim3(egrid), dim3(kBlock), 0, s, key, key_stride, n, rows, k0);
-        int bits = 1;
-        while (bits < 31 && (1ll << bits) < (long long)rows) ++bits;
-        bool first = true;
-        for (int shift = 0; shift < bits; shift += 8) {
-            hipLaunchKernelGGL(radix_hist_kernel, dim3(ntiles), dim3(kBlock), 0, s, k0, n, shift, ntiles, hist);
-            if (int rc = exclusive_scan_i32(hist, nhist, seg, s)) return rc;
-            hipLaunchKernelGGL(radix_scatter_kernel, dim3(ntiles), dim3(kBlock), 0, s, k0, v0, n, shift, ntiles, hist, k1, v1, first ? 1 : 0);
-            unsigned* t = k0; k0 = k1; k1 = t;
-            t = v0; v0 = v1; v1 = t;
-            first = false;
+    for (int i = 0; i < count; ++i) {
+        GroupJob& j = jobs.job[i];
+        auto words = [&](int a) { return reinterpret_cast<unsigned*>(b + o[i][a]); };
+        j.k0 = words(0); j.k1 = words(1); j.v0 = words(2); j.v1 = words(3);
+        j.hist = reinterpret_cast<int*>(b + o[i][4]);
+        j.seg = reinterpret_cast<int*>(b + o[i][5]);
+    }
+    for (int shift = 0; shift < bits; shift += digit) {
+        const bool first = shift == 0;
+        const int rc = digit == 8 ? radix_pass<8>(count, jobs, first, n, rows, shift, s)
+                     : digit == 10 ? radix_pass<10>(count, jobs, first, n, rows, shift, s) : radix_pass<11>(count, jobs, first, n, rows, shift, s);
+        if (rc) return rc;
+        for (int i = 0; i < count; ++i) {
+            GroupJob& j = jobs.job[i];
+            unsigned* t = j.k0; j.k0 = j.k1; j.k1 = t;
+            t = j.v0; j.v0 = j.v1; j.v1 = t;
         }
     }
-    const unsigned rgrid = n > 0 ? egrid : (unsigned)(((long long)rows + kBlock) / kBlock);
-    hipLaunchKernelGGL(row_ptr_from_sorted_kernel, dim3(rgrid), dim3(kBlock), 0, s, k0, n, rows, row_ptr);
-    if (n > 0)
-        hipLaunchKernelGGL(fill_grouped_kernel, dim3(egrid), dim3(kBlock), 0, s, k0, v0, n, payload, payload_stride, val_in, average,
-                           row_ptr, col_idx, val);
+    const dim3 grid((unsigned)((n + kBlock - 1) / kBlock), count);
+    if (average) {
+        hipLaunchKernelGGL(row_ptr_from_sorted_kernel, grid, dim3(kBlock), 0, s, jobs, n, rows);
+        hipLaunchKernelGGL(fill_grouped_kernel<true>, grid, dim3(kBlock), 0, s, jobs, n, rows);
+    } else {
+        hipLaunchKernelGGL(fill_grouped_kernel<false>, grid, dim3(kBlock), 0, s, jobs, n, rows);
+    }
     GNNHIP_LAUNCH_CHECK("csr_group_pairs");
     return GNNHIP_OK;
+}
+
+// One grouping, in one launch where that fits.
+int csr_group(int rows, long long n, const int* key, int key_stride, const int* payload, int payload_stride, const float* val_in, int average,
+              int* row_ptr, int* col_idx, float* val, hipStream_t s)
+{
+    if (csr_group_small(rows, n, key, key_stride, payload, payload_stride, val_in, average, row_ptr, col_idx, val, nullptr, nullptr, nullptr, s))
+        return last_launch_status("csr_group_small");
+    GroupJobs jobs{};
+    jobs.job[0] = GroupJob{key, payload, val_in, key_stride, payload_stride, row_ptr, col_idx, val};
+    return csr_group_pairs(1, jobs, rows, n, average, s);
 }
 
 }  // namespace gnnhip
@@ -698,7 +797,7 @@ int gnnhip_csr_group_i32(int rows, int n, const int* key, int key_stride, const 
     GNNHIP_REQUIRE(n == 0 || (key && payload && col_idx && val), "null array in csr_group");
     GNNHIP_REQUIRE(n == 0 || rows >= 1, "pairs but no rows in csr_group");
     if (int rc = require_ready()) return rc;
-    return csr_group_pairs(rows, n, key, key_stride, payload, payload_stride, nullptr, average, row_ptr, col_idx, val, as_stream(stream));
+    return csr_group(rows, n, key, key_stride, payload, payload_stride, nullptr, average, row_ptr, col_idx, val, as_stream(stream));
 }
 
 int gnnhip_csr_consecutive_rows_f32(int rows, const int* row_ptr, int average, int* col_idx, float* val, void* stream)
@@ -746,8 +845,10 @@ int gnnhip_csr_group_both_i32(int rows, int n, const int* x, int x_stride, const
     hipStream_t s = as_stream(stream);
     if (csr_group_small(rows, n, y, y_stride, x, x_stride, nullptr, 0, row_ptr, col_idx, val, t_row_ptr, t_col_idx, t_val, s))
         return last_launch_status("csr_group_small");
-    if (int rc = csr_group_pairs(rows, n, y, y_stride, x, x_stride, nullptr, 0, row_ptr, col_idx, val, s)) return rc;
-    return csr_group_pairs(rows, n, x, x_stride, y, y_stride, nullptr, 0, t_row_ptr, t_col_idx, t_val, s);
+    GroupJobs jobs{};
+    jobs.job[0] = GroupJob{y, x, nullptr, y_stride, x_stride, row_ptr, col_idx, val};
+    jobs.job[1] = GroupJob{x, y, nullptr, x_stride, y_stride, t_row_ptr, t_col_idx, t_val};
+    return csr_group_pairs(2, jobs, rows, n, 0, s);
 }
 
 int gnnhip_csr_transpose_f32(int m, int k, int nnz, const int* row_ptr, const int* col_idx, const float* val,
@@ -768,7 +869,7 @@ int gnnhip_csr_transpose_f32(int m, int k, int nnz, const int* row_ptr, const in
         const unsigned grid = (unsigned)(((long long)m * kWave + kBlock - 1) / kBlock);
         if (m > 0) hipLaunchKernelGGL(expand_rows_kernel, dim3(grid), dim3(kBlock), 0, s, m, row_ptr, row_of);
     }
-    return csr_group_pairs(k, nnz, col_idx, 1, row_of, 1, val, 0, t_row_ptr, t_col_idx, t_val, s);
+    return csr_group(k, nnz, col_idx, 1, row_of, 1, val, 0, t_row_ptr, t_col_idx, t_val, s);
 }
 
 }  // extern "C"
