@@ -19,7 +19,7 @@
 //
 // Most matrices have no hubs, and then the pass is nothing but its launches: with a launch that turned the counts into
 // one list of all chunks and a launch that added up the chunks of a hub it was four per product instead of two.
-#include "gnnhip_internal.h"
+#include "columns.h"
 
 #include <map>
 
@@ -107,43 +107,22 @@ __global__ __launch_bounds__(kBlock) void hub_count_kernel(int m, int rows, cons
     if (threadIdx.x == 0) { run_hubs[blockIdx.x] = hubs; run_chunks[blockIdx.x] = chunks; }
 }
 
-template <int VEC> struct HV;
-template <> struct HV<4> {
-    using T = float4;
-    static __device__ __forceinline__ T zero() { return make_float4(0.f, 0.f, 0.f, 0.f); }
-    static __device__ __forceinline__ T load(const float* p) { return *reinterpret_cast<const float4*>(p); }
-    static __device__ __forceinline__ T load(const float* p, int relu) { const T v = load(p); return relu ? relu_ref4(v) : v; }
-    static __device__ __forceinline__ void store(float* p, T v) { *reinterpret_cast<float4*>(p) = v; }
-    static __device__ __forceinline__ void fma(T& a, float s, T x) { f4_fma(a, s, x); }
-    static __device__ __forceinline__ T add(T a, T b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
-};
-template <> struct HV<1> {
-    using T = float;
-    static __device__ __forceinline__ T zero() { return 0.f; }
-    static __device__ __forceinline__ T load(const float* p) { return *p; }
-    static __device__ __forceinline__ T load(const float* p, int relu) { const T v = *p; return relu ? relu_ref(v) : v; }
-    static __device__ __forceinline__ void store(float* p, T v) { *p = v; }
-    static __device__ __forceinline__ void fma(T& a, float s, T x) { a += s * x; }
-    static __device__ __forceinline__ T add(T a, T b) { return a + b; }
-};
-
 // One wavefront per chunk.  The wavefront is split into 64 / G lane groups; group g takes the
 // chunk's entries g, g + ngroups, ... eight at a time, a lane owns the column slabs
-// (sub + it * G) * VEC.  The groups' sums are added through LDS in group order.
-template <int VEC, int ITERS>
+// (sub + it * G) * V::kVec.  The groups' sums are added through LDS in group order.
+template <class V, int ITERS>
 __global__ __launch_bounds__(kBlock) void hub_partial_kernel(
     int run_rows, int runs, const int* __restrict__ run_hubs, const int* __restrict__ run_chunks, const int* __restrict__ list_row,
     const int* __restrict__ list_chunk, int chunk_cap, int n, const int* __restrict__ row_ptr, const int* __restrict__ col_idx, const float* __restrict__ val, const float* __restrict__ B, int ldb, int logG,
     int* __restrict__ row_chunk, float* __restrict__ part, int ldp, int relu_in, int threshold, int shift)
 {
     // relu_in: the rows of B are used as ReLU(B) (a first level that reads msg in place of h0)
-    using V = HV<VEC>;
-    __shared__ float red[kWavesPerBlock][kWave * VEC * ITERS];
+    __shared__ float red[kWavesPerBlock][kWave * V::kVec * ITERS];
     __shared__ int before[kMaxRuns + 1];         // chunks ahead of a run
     __shared__ int wave_total[kWavesPerBlock];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int G = 1 << logG, sub = lane & (G - 1), grp = lane >> logG, ngroups = kWave >> logG;
-    const int width = G * VEC * ITERS;
+    const int width = G * V::kVec * ITERS;
 
     int nchunks;
     {
@@ -205,30 +184,31 @@ __global__ __launch_bounds__(kBlock) void hub_partial_kernel(
             }
 #pragma unroll
             for (int it = 0; it < ITERS; ++it) {
-                const int col0 = (sub + it * G) * VEC;
-                if (col0 < n) {
+                const int unit = sub + it * G;
+                if (unit * V::kVec < n) {
+                    const int col0 = V::at(unit, n);
                     typename V::T x[8];
 #pragma unroll
                     for (int u = 0; u < 8; ++u)
-                        x[u] = (t + u * ngroups < ce) ? V::load(B + (size_t)c8[u] * ldb + col0, relu_in) : V::zero();
+                        x[u] = (t + u * ngroups < ce) ? V::load(B + (size_t)c8[u] * ldb + col0) : V::zero();
 #pragma unroll
                     for (int u = 0; u < 8; ++u)
-                        if (t + u * ngroups < ce) V::fma(acc[it], v8[u], x[u]);
+                        if (t + u * ngroups < ce) V::fma(acc[it], v8[u], relu_in ? V::relu(x[u]) : x[u]);
                 }
             }
         }
 #pragma unroll
-        for (int it = 0; it < ITERS; ++it) V::store(red[wave] + grp * width + (sub + it * G) * VEC, acc[it]);
+        for (int it = 0; it < ITERS; ++it) V::store(red[wave] + grp * width + (sub + it * G) * V::kVec, acc[it]);
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         float* dst = part + (size_t)c * ldp;
         if (grp == 0) {
 #pragma unroll
             for (int it = 0; it < ITERS; ++it) {
-                const int col0 = (sub + it * G) * VEC;
-                if (col0 < n) {
+                const int unit = sub + it * G;
+                if (unit * V::kVec < n) {
                     typename V::T s = V::zero();
-                    for (int g = 0; g < ngroups; ++g) s = V::add(s, V::load(red[wave] + g * width + col0));
-                    V::store(dst + col0, s);
+                    for (int g = 0; g < ngroups; ++g) s = V::add(s, V::load(red[wave] + g * width + unit * V::kVec));
+                    V::store(dst + V::at(unit, n), s);
                 }
             }
         }
@@ -276,7 +256,7 @@ HubLayout hub_layout(int m, int n, long long nnz, int threshold, int chunk_len, 
     return L;
 }
 
-template <int VEC, int ITERS>
+template <class V, int ITERS>
 void launch_partial(hipStream_t s, const HubLayout& L, char* base, int n, const int* row_ptr, const int* col_idx, const float* val,
                     const float* B, int ldb, int logG, int relu_in, int threshold, int shift)
 {
@@ -284,7 +264,7 @@ void launch_partial(hipStream_t s, const HubLayout& L, char* base, int n, const 
     long long grid = ((long long)L.chunk_cap + kWavesPerBlock - 1) / kWavesPerBlock;
     if (grid > kNumCU * 8) grid = kNumCU * 8;
     auto ints = [base](size_t o) { return reinterpret_cast<int*>(base + o); };
-    hipLaunchKernelGGL((hub_partial_kernel<VEC, ITERS>), dim3((unsigned)grid), dim3(kBlock), 0, s, L.run_rows, L.runs, ints(L.o_hubs),
+    hipLaunchKernelGGL((hub_partial_kernel<V, ITERS>), dim3((unsigned)grid), dim3(kBlock), 0, s, L.run_rows, L.runs, ints(L.o_hubs),
                        ints(L.o_chunks), ints(L.o_lrow), ints(L.o_lchunk), L.chunk_cap, n, row_ptr, col_idx, val, B, ldb, logG,
                        ints(L.o_row), reinterpret_cast<float*>(base + L.o_part), L.ldp, relu_in, threshold, shift);
 }
@@ -315,8 +295,7 @@ int hub_prepass(int m, int n, long long nnz, const int* row_ptr, const int* col_
     *plan = HubPlan{};
     if (!hub_pass_applies(m, n, nnz, threshold)) return GNNHIP_OK;
     const bool vec4 = (n % 4 == 0) && (ldb % 4 == 0) && aligned16(B);
-    const int vec = vec4 ? 4 : 1;
-    const int units = (n + vec - 1) / vec;
+    const int units = n < 4 ? n : (n + 3) / 4;
     const int logG = ilog2_ceil_(units < kWave ? units : kWave);
     const int G = 1 << logG;
     const int iters = (units + G - 1) / G;                   // 1..4
@@ -364,14 +343,16 @@ int hub_prepass(int m, int n, long long nnz, const int* row_ptr, const int* col_
                            reinterpret_cast<int*>(b + L.o_lchunk), threshold, shift);
         if (store) store->planned = true;
     }
-    if (vec4) {
-        if (iters <= 1) launch_partial<4, 1>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift);
-        else if (iters == 2) launch_partial<4, 2>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift);
-        else launch_partial<4, 4>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift);
+    if (n < 4) {
+        launch_partial<ColsOne, 1>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift);
+    } else if (vec4) {
+        if (iters <= 1) launch_partial<ColsWide, 1>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift);
+        else if (iters == 2) launch_partial<ColsWide, 2>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift);
+        else launch_partial<ColsWide, 4>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift);
     } else {
-        if (iters <= 1) launch_partial<1, 1>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift);
-        else if (iters == 2) launch_partial<1, 2>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift);
-        else launch_partial<1, 4>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift);
+        if (iters <= 1) launch_partial<ColsLoose, 1>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift);
+        else if (iters == 2) launch_partial<ColsLoose, 2>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift);
+        else launch_partial<ColsLoose, 4>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift);
     }
     GNNHIP_LAUNCH_CHECK("hub_prepass");
     *plan = HubPlan{reinterpret_cast<int*>(b + L.o_row), reinterpret_cast<float*>(b + L.o_part), L.ldp, shift};

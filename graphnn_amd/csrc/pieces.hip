@@ -22,7 +22,7 @@
 // Every sum is taken in an order fixed by the matrix (no atomics): the result does not depend on scheduling.
 // The plan depends on A only (structure and values) and is reused by the later levels of one forward.
 // Bound: HBM / L2.  Algorithmic bytes as for the plain SpMM, plus 8 bytes of partial sums per column and piece.
-#include "gnnhip_internal.h"
+#include "columns.h"
 
 #include <map>
 #include <set>
@@ -143,28 +143,6 @@ __global__ __launch_bounds__(kBlock) void piece_gather_kernel(const int* __restr
     }
 }
 
-template <int VEC> struct PV;
-template <> struct PV<4> {
-    using T = float4;
-    static __device__ __forceinline__ T zero() { return make_float4(0.f, 0.f, 0.f, 0.f); }
-    static __device__ __forceinline__ T load(const float* p) { return *reinterpret_cast<const float4*>(p); }
-    static __device__ __forceinline__ void store(float* p, T v) { *reinterpret_cast<float4*>(p) = v; }
-    static __device__ __forceinline__ void fma(T& a, float s, T x) { a.x += s * x.x; a.y += s * x.y; a.z += s * x.z; a.w += s * x.w; }
-    static __device__ __forceinline__ T axpby(T a, float b, T c) { return make_float4(a.x + b * c.x, a.y + b * c.y, a.z + b * c.z, a.w + b * c.w); }
-    static __device__ __forceinline__ T add(T a, T b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
-    static __device__ __forceinline__ T relu(T a) { return relu_ref4(a); }
-};
-template <> struct PV<1> {
-    using T = float;
-    static __device__ __forceinline__ T zero() { return 0.f; }
-    static __device__ __forceinline__ T load(const float* p) { return *p; }
-    static __device__ __forceinline__ void store(float* p, T v) { *p = v; }
-    static __device__ __forceinline__ void fma(T& a, float s, T x) { a += s * x; }
-    static __device__ __forceinline__ T axpby(T a, float b, T c) { return a + b * c; }
-    static __device__ __forceinline__ T add(T a, T b) { return a + b; }
-    static __device__ __forceinline__ T relu(T a) { return relu_ref(a); }
-};
-
 // One lane group (G lanes) per piece, pieces taken in order; die x (workgroups x, x + 8, ...) walks the
 // x-th eighth of that order front to back, a workgroup taking the next ngroups pieces of its die when the
 // hardware starts it (so the pieces in flight on a die stay close together in the order; a fixed stride per
@@ -174,13 +152,12 @@ template <> struct PV<1> {
 // The sum of a piece that is all of its row goes to C (as sum + beta * C, what the combining pass would make of
 // it), the others to the place of their piece id among the partial sums.
 // RELU_IN: the rows of B count as ReLU(B).
-template <int VEC, int ITERS, bool RELU_IN>
+template <class V, int ITERS, bool RELU_IN>
 __global__ __launch_bounds__(kBlock) void piece_sum_kernel(
     const int* __restrict__ count, int n, float alpha, const int* __restrict__ at, const int* __restrict__ col_idx, const float* __restrict__ val,
     const float* __restrict__ B, int ldb, float* __restrict__ part, int ldp, int logG, const int* __restrict__ target, float beta,
     float* __restrict__ C, int ldc)
 {
-    using V = PV<VEC>;
     const int G = 1 << logG;
     const int sub = threadIdx.x & (G - 1);
     const int grp = threadIdx.x >> logG;
@@ -211,8 +188,9 @@ __global__ __launch_bounds__(kBlock) void piece_sum_kernel(
                 }
 #pragma unroll
                 for (int it = 0; it < ITERS; ++it) {
-                    const int col0 = (sub + it * G) * VEC;
-                    if (col0 < n) {
+                    const int unit = sub + it * G;
+                    if (unit * V::kVec < n) {
+                        const int col0 = V::at(unit, n);
                         typename V::T x[4];
 #pragma unroll
                         for (int u = 0; u < 4; ++u)
@@ -228,15 +206,10 @@ __global__ __launch_bounds__(kBlock) void piece_sum_kernel(
         if (row == kNoPlace) return;
 #pragma unroll
         for (int it = 0; it < ITERS; ++it) {
-            const int col0 = (sub + it * G) * VEC;
-            if (col0 >= n) continue;
-            if (row < 0) {
-                V::store(part + (size_t)(-1 - row) * ldp + col0, acc[it]);
-            } else {
-                float* dst = C + (size_t)row * ldc + col0;
-                if (beta == 0.f) V::store(dst, acc[it]);
-                else V::store(dst, V::axpby(acc[it], beta, V::load(dst)));
-            }
+            const int unit = sub + it * G;
+            if (unit * V::kVec >= n) continue;
+            if (row < 0) V::store(part + (size_t)(-1 - row) * ldp + V::at(unit, n), acc[it]);
+            else V::update(C + (size_t)row * ldc, unit, n, acc[it], beta);
         }
     }
 }
@@ -245,13 +218,12 @@ __global__ __launch_bounds__(kBlock) void piece_sum_kernel(
 // stand-in piece without entries, so neither the sums nor the combining pass write it; its result,
 // alpha * A[row] * B + beta * C[row], is formed here.  Rows are taken from the last one down, a lane group each;
 // the first row that ends inside the plan ends the walk.
-template <int VEC, int ITERS, bool RELU_IN>
+template <class V, int ITERS, bool RELU_IN>
 __global__ __launch_bounds__(kBlock) void piece_tail_kernel(int m, int n, float alpha, const int* __restrict__ row_ptr, int cap,
                                                             const int* __restrict__ col_idx, const float* __restrict__ val,
                                                             const float* __restrict__ B, int ldb, float beta, float* __restrict__ C,
                                                             int ldc, int logG)
 {
-    using V = PV<VEC>;
     const int G = 1 << logG;
     const int sub = threadIdx.x & (G - 1);
     const int grp = threadIdx.x >> logG;
@@ -269,20 +241,19 @@ __global__ __launch_bounds__(kBlock) void piece_tail_kernel(int m, int n, float 
             const float v = alpha * val[t];
 #pragma unroll
             for (int it = 0; it < ITERS; ++it) {
-                const int col0 = (sub + it * G) * VEC;
-                if (col0 < n) {
+                const int unit = sub + it * G;
+                if (unit * V::kVec < n) {
+                    const int col0 = V::at(unit, n);
                     const typename V::T x = V::load(B + (size_t)c * ldb + col0);
                     V::fma(acc[it], v, RELU_IN ? V::relu(x) : x);
                 }
             }
         }
-        float* dst = C + (size_t)row * ldc;
 #pragma unroll
         for (int it = 0; it < ITERS; ++it) {
-            const int col0 = (sub + it * G) * VEC;
-            if (col0 >= n) continue;
-            if (beta == 0.f) V::store(dst + col0, acc[it]);
-            else V::store(dst + col0, V::axpby(acc[it], beta, V::load(dst + col0)));
+            const int unit = sub + it * G;
+            if (unit * V::kVec >= n) continue;
+            V::update(C + (size_t)row * ldc, unit, n, acc[it], beta);
         }
     }
 }
@@ -299,12 +270,11 @@ __global__ __launch_bounds__(kBlock) void piece_tail_kernel(int m, int n, float 
 // for it: on a power-law matrix the rows of many pieces sit next to each other.
 // Rows without entries get beta * C.
 constexpr int kCombineChunk = 256;      // pieces per chunk of the balanced pass over rows of more than kCombineLong
-template <int VEC, int ITERS>
+template <class V, int ITERS>
 __global__ __launch_bounds__(kBlock) void piece_combine_kernel(
     int m, int n, const int* __restrict__ first, const int* __restrict__ pfirst, const float* __restrict__ part, int ldp, float beta,
     float* __restrict__ C, int ldc, int logG, HubPlan hubs)
 {
-    using V = PV<VEC>;
     constexpr int kFlight = 8;
     const int lane = threadIdx.x & (kWave - 1);
     const int G = 1 << logG;                       // lanes per row: 8 .. 64
@@ -335,11 +305,9 @@ __global__ __launch_bounds__(kBlock) void piece_combine_kernel(
         if (o < 0) continue;
 #pragma unroll
         for (int it = 0; it < ITERS; ++it) {
-            const int col0 = (sub + it * G) * VEC;
-            if (col0 >= n) continue;
-            float* dst = C + (size_t)(row0 + o) * ldc + col0;
-            if (beta == 0.f) V::store(dst, V::zero());
-            else V::store(dst, V::axpby(V::zero(), beta, V::load(dst)));
+            const int unit = sub + it * G;
+            if (unit * V::kVec >= n) continue;
+            V::update(C + (size_t)(row0 + o) * ldc, unit, n, V::zero(), beta);
         }
     }
     while (several_left) {
@@ -356,15 +324,16 @@ __global__ __launch_bounds__(kBlock) void piece_combine_kernel(
         if (chunk >= 0) {
 #pragma unroll
             for (int it = 0; it < ITERS; ++it) {
-                const int col0 = (sub + it * G) * VEC;
-                if (col0 < n) acc[it] = hub_row_sum<V>(hubs.part + (size_t)chunk * hubs.ld + col0, hubs.ld, e - b, hubs.shift);
+                const int unit = sub + it * G;
+                if (unit * V::kVec < n) acc[it] = hub_row_sum<V>(hubs.part + (size_t)chunk * hubs.ld + V::at(unit, n), hubs.ld, e - b, hubs.shift);
             }
         } else {
             for (int p = b; p < e; p += kFlight) {
 #pragma unroll
                 for (int it = 0; it < ITERS; ++it) {
-                    const int col0 = (sub + it * G) * VEC;
-                    if (col0 < n) {
+                    const int unit = sub + it * G;
+                    if (unit * V::kVec < n) {
+                        const int col0 = V::at(unit, n);
                         typename V::T x[kFlight];
 #pragma unroll
                         for (int u = 0; u < kFlight; ++u)
@@ -378,11 +347,9 @@ __global__ __launch_bounds__(kBlock) void piece_combine_kernel(
         }
 #pragma unroll
         for (int it = 0; it < ITERS; ++it) {
-            const int col0 = (sub + it * G) * VEC;
-            if (col0 >= n) continue;
-            float* dst = C + (size_t)row * ldc + col0;
-            if (beta == 0.f) V::store(dst, acc[it]);
-            else V::store(dst, V::axpby(acc[it], beta, V::load(dst)));
+            const int unit = sub + it * G;
+            if (unit * V::kVec >= n) continue;
+            V::update(C + (size_t)row * ldc, unit, n, acc[it], beta);
         }
     }
 }
@@ -399,15 +366,15 @@ inline size_t round_up_p(size_t x, size_t a) { return (x + a - 1) / a * a; }
 constexpr long long kPiecesMeanDegree = 12;
 
 struct Width {            // how a lane group covers the columns of an operand of width n
-    bool ok, vec4;
+    bool ok;
+    int cols;             // packing: 4 ColsWide, 3 ColsLoose, 1 ColsOne
     int logG, iters, ldp;
 };
 Width width_of(int n, const float* B, int ldb, const float* C, int ldc)
 {
     Width w;
-    w.vec4 = (n % 4 == 0) && (ldb % 4 == 0) && (ldc % 4 == 0) && aligned16(B) && aligned16(C);
-    const int vec = w.vec4 ? 4 : 1;
-    const int units = (n + vec - 1) / vec;
+    w.cols = (n % 4 == 0) && (ldb % 4 == 0) && (ldc % 4 == 0) && aligned16(B) && aligned16(C) ? 4 : n > 28 ? 3 : 1;
+    const int units = w.cols == 1 ? n : (n + 3) / 4;
     // A lane group covers at most 64 x 4 column units (wider operands stay with the caller's route, which cuts them into
     // slabs).  Narrow operands stay with the row-group route too: with fewer than eight lanes per piece a wavefront reads
     // the entries of more than eight pieces at once, 128 bytes apart, and fetches whole lines for a few bytes each
@@ -516,14 +483,16 @@ int run_pieces(const CsrPlan* p, const Width& w, int n, float alpha, const float
 #define GNNHIP_PIECES_LAUNCH(V, I)                                                                                            \
     hipLaunchKernelGGL((relu_in ? piece_sum_kernel<V, I, true> : piece_sum_kernel<V, I, false>), dim3(sgrid), dim3(kBlock), 0, s, p->first + m, n, alpha, p->at, p->col_ord, p->val_ord, B, \
                        ldb, part, ldp, logG, p->target, beta, C, ldc)
-    if (w.vec4) {
-        if (iters <= 1) GNNHIP_PIECES_LAUNCH(4, 1);
-        else if (iters == 2) GNNHIP_PIECES_LAUNCH(4, 2);
-        else GNNHIP_PIECES_LAUNCH(4, 4);
+    if (w.cols == 4) {
+        if (iters <= 1) GNNHIP_PIECES_LAUNCH(ColsWide, 1);
+        else if (iters == 2) GNNHIP_PIECES_LAUNCH(ColsWide, 2);
+        else GNNHIP_PIECES_LAUNCH(ColsWide, 4);
+    } else if (w.cols == 3) {
+        if (iters <= 1) GNNHIP_PIECES_LAUNCH(ColsLoose, 1);
+        else if (iters == 2) GNNHIP_PIECES_LAUNCH(ColsLoose, 2);
+        else GNNHIP_PIECES_LAUNCH(ColsLoose, 4);
     } else {
-        if (iters <= 1) GNNHIP_PIECES_LAUNCH(1, 1);
-        else if (iters == 2) GNNHIP_PIECES_LAUNCH(1, 2);
-        else GNNHIP_PIECES_LAUNCH(1, 4);
+        GNNHIP_PIECES_LAUNCH(ColsOne, 1);
     }
 #undef GNNHIP_PIECES_LAUNCH
     GNNHIP_LAUNCH_CHECK("spmm_pieces sums");
@@ -533,14 +502,16 @@ int run_pieces(const CsrPlan* p, const Width& w, int n, float alpha, const float
 #define GNNHIP_PIECES_TAIL(V, I)                                                                                                   \
     hipLaunchKernelGGL((relu_in ? piece_tail_kernel<V, I, true> : piece_tail_kernel<V, I, false>), dim3(tgrid), dim3(kBlock), 0, s, m, n, alpha, p->row_ptr, (int)p->nnz, p->col_idx, p->val, \
                        B, ldb, beta, C, ldc, logG)
-        if (w.vec4) {
-            if (iters <= 1) GNNHIP_PIECES_TAIL(4, 1);
-            else if (iters == 2) GNNHIP_PIECES_TAIL(4, 2);
-            else GNNHIP_PIECES_TAIL(4, 4);
+        if (w.cols == 4) {
+            if (iters <= 1) GNNHIP_PIECES_TAIL(ColsWide, 1);
+            else if (iters == 2) GNNHIP_PIECES_TAIL(ColsWide, 2);
+            else GNNHIP_PIECES_TAIL(ColsWide, 4);
+        } else if (w.cols == 3) {
+            if (iters <= 1) GNNHIP_PIECES_TAIL(ColsLoose, 1);
+            else if (iters == 2) GNNHIP_PIECES_TAIL(ColsLoose, 2);
+            else GNNHIP_PIECES_TAIL(ColsLoose, 4);
         } else {
-            if (iters <= 1) GNNHIP_PIECES_TAIL(1, 1);
-            else if (iters == 2) GNNHIP_PIECES_TAIL(1, 2);
-            else GNNHIP_PIECES_TAIL(1, 4);
+            GNNHIP_PIECES_TAIL(ColsOne, 1);
         }
 #undef GNNHIP_PIECES_TAIL
         GNNHIP_LAUNCH_CHECK("spmm_pieces tail");
@@ -561,14 +532,16 @@ int run_pieces(const CsrPlan* p, const Width& w, int n, float alpha, const float
 #define GNNHIP_PIECES_COMBINE(V, I)                                                                                             \
     hipLaunchKernelGGL((piece_combine_kernel<V, I>), dim3(grid), dim3(kBlock), 0, s, m, n, p->first, p->pfirst, part, ldp, beta, C, ldc, \
                        logG, hubs)
-    if (w.vec4) {
-        if (iters <= 1) GNNHIP_PIECES_COMBINE(4, 1);
-        else if (iters == 2) GNNHIP_PIECES_COMBINE(4, 2);
-        else GNNHIP_PIECES_COMBINE(4, 4);
+    if (w.cols == 4) {
+        if (iters <= 1) GNNHIP_PIECES_COMBINE(ColsWide, 1);
+        else if (iters == 2) GNNHIP_PIECES_COMBINE(ColsWide, 2);
+        else GNNHIP_PIECES_COMBINE(ColsWide, 4);
+    } else if (w.cols == 3) {
+        if (iters <= 1) GNNHIP_PIECES_COMBINE(ColsLoose, 1);
+        else if (iters == 2) GNNHIP_PIECES_COMBINE(ColsLoose, 2);
+        else GNNHIP_PIECES_COMBINE(ColsLoose, 4);
     } else {
-        if (iters <= 1) GNNHIP_PIECES_COMBINE(1, 1);
-        else if (iters == 2) GNNHIP_PIECES_COMBINE(1, 2);
-        else GNNHIP_PIECES_COMBINE(1, 4);
+        GNNHIP_PIECES_COMBINE(ColsOne, 1);
     }
 #undef GNNHIP_PIECES_COMBINE
     GNNHIP_LAUNCH_CHECK("spmm_pieces combine");

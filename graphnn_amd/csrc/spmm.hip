@@ -19,7 +19,7 @@
 // in a fixed order (still deterministic).
 //
 // Bound: HBM.  Algorithmic bytes per launch: 4(m+1) + 8 nnz + 4 k n + 4 m n.
-#include "gnnhip_internal.h"
+#include "columns.h"
 
 namespace gnnhip {
 namespace {
@@ -38,46 +38,30 @@ __device__ __forceinline__ unsigned xcd_remap(unsigned bid, unsigned nblocks)
     return (bid % kNumXCD) * per + bid / kNumXCD;
 }
 
-template <int VEC> struct Vec;
-template <> struct Vec<4> {
-    using T = float4;
-    static __device__ __forceinline__ T zero() { return make_float4(0.f, 0.f, 0.f, 0.f); }
-    static __device__ __forceinline__ T load(const float* p) { return *reinterpret_cast<const float4*>(p); }
-    static __device__ __forceinline__ void store(float* p, T v) { *reinterpret_cast<float4*>(p) = v; }
-    static __device__ __forceinline__ void fma(T& a, float s, T x) { a.x += s * x.x; a.y += s * x.y; a.z += s * x.z; a.w += s * x.w; }
-    static __device__ __forceinline__ T axpby(T a, float b, T c) { return make_float4(a.x + b * c.x, a.y + b * c.y, a.z + b * c.z, a.w + b * c.w); }
-    static __device__ __forceinline__ T add(T a, T b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
-    static __device__ __forceinline__ T relu(T a) { return relu_ref4(a); }
-};
-template <> struct Vec<1> {
-    using T = float;
-    static __device__ __forceinline__ T zero() { return 0.f; }
-    static __device__ __forceinline__ T load(const float* p) { return *p; }
-    static __device__ __forceinline__ void store(float* p, T v) { *p = v; }
-    static __device__ __forceinline__ void fma(T& a, float s, T x) { a += s * x; }
-    static __device__ __forceinline__ T axpby(T a, float b, T c) { return a + b * c; }
-    static __device__ __forceinline__ T add(T a, T b) { return a + b; }
-    static __device__ __forceinline__ T relu(T a) { return relu_ref(a); }
-};
-
 // One row per group of G = 1 << logG lanes.  A lane owns column slabs
-// (sub + it * G) * VEC, it < ITERS; slabs at or beyond n are skipped.
+// (sub + it * G) * V::kVec, it < ITERS; slabs at or beyond n are skipped.
 // Rows longer than long_row entries are parked in an LDS list and processed
 // afterwards by the whole workgroup: group g takes entries g, g + ngroups, ...
 // and the partial sums are added through LDS in group order.
 // long_row < 0: one row per workgroup, summed that way whatever its length (few, long rows: pooling 1,024 nodes
 // into each of 4,096 subgraphs ran one workgroup per compute unit with a lane group per row: 0.265 ms).
 // RELU_IN: the rows of B count as ReLU(B).
-template <int VEC, int ITERS, bool RELU_IN>
+// NARROW (G <= kNarrowGroup): a group that read its entries G at a time would have G gathers in flight, and its wavefront
+// would touch a line per row and read.  The rows of a wavefront are consecutive and so are their entries: the wavefront
+// copies them to LDS, coalesced, when there are at most kStaged (else every lane reads its row's entries itself), and the
+// groups take eight at a time.  Sums are added in the same order.  (300,000 rows of 10 entries: width 4 77 -> 30 us, width 16
+// 66 -> 55; groups of eight lanes gain 4 % there and lose 8 % at two entries per row, so the line is at four.)
+constexpr int kNarrowGroup = 4;
+constexpr int kStaged = 768;
+template <class V, int ITERS, bool RELU_IN, bool NARROW>
 __global__ __launch_bounds__(kBlock) void spmm_rowgroup_kernel(
     int m, int n, float alpha, const int* __restrict__ row_ptr, const int* __restrict__ col_idx,
     const float* __restrict__ val, const float* __restrict__ B, int ldb, float beta, float* C, int ldc,
     int logG, int long_row, HubPlan hubs)
 {
-    using V = Vec<VEC>;
     __shared__ int lr_list[kBlock];
     __shared__ int lr_count;
-    __shared__ float red[kBlock * VEC * ITERS];      // [ngroups][G * VEC * ITERS]
+    __shared__ float red[kBlock * V::kVec * ITERS];      // [ngroups][G * V::kVec * ITERS]
 
     const int G = 1 << logG;
     const int sub = threadIdx.x & (G - 1);
@@ -108,7 +92,43 @@ __global__ __launch_bounds__(kBlock) void spmm_rowgroup_kernel(
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) acc[it] = V::zero();
 
-    for (int base = start; base < end; base += G) {
+    if constexpr (NARROW) {
+        __shared__ int2 staged[kBlock / kWave][kStaged];
+        int2* mine = staged[threadIdx.x / kWave];
+        const int lane = threadIdx.x & (kWave - 1);
+        const int col0 = V::at(sub, n);
+        constexpr int kFlight = 8;
+        auto add_row = [&](auto entry) {
+            for (int base = start; base < end; base += kFlight) {
+                int2 cv[kFlight];
+                typename V::T x[kFlight];
+#pragma unroll
+                for (int u = 0; u < kFlight; ++u) cv[u] = base + u < end ? entry(base + u) : make_int2(0, 0);
+#pragma unroll
+                for (int u = 0; u < kFlight; ++u)
+                    x[u] = base + u < end && sub * V::kVec < n ? V::load(B + (size_t)cv[u].x * ldb + col0) : V::zero();
+#pragma unroll
+                for (int u = 0; u < kFlight; ++u)
+                    if (base + u < end) V::fma(acc[0], alpha * __int_as_float(cv[u].y), RELU_IN ? V::relu(x[u]) : x[u]);
+            }
+        };
+        // rows past the end, hubs and deferred rows are empty here and take no part in the range
+        const unsigned long long busy = __ballot(end > start);
+        int lo = 0, hi = 0;
+        if (busy) {
+            lo = __builtin_amdgcn_readlane(start, (int)__builtin_ctzll(busy));
+            hi = __builtin_amdgcn_readlane(end, 63 - (int)__builtin_clzll(busy));
+        }
+        if (hi - lo <= kStaged) {
+            for (int e = lo + lane; e < hi; e += kWave) mine[e - lo] = make_int2(col_idx[e], __float_as_int(val[e]));
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            add_row([&](int e) { return mine[e - lo]; });
+        } else {
+            add_row([&](int e) { return make_int2(col_idx[e], __float_as_int(val[e])); });
+        }
+        end = start;
+    }
+    for (int base = start; !NARROW && base < end; base += G) {
         const int t = base + sub;
         int c = 0;
         float v = 0.f;
@@ -124,8 +144,9 @@ __global__ __launch_bounds__(kBlock) void spmm_rowgroup_kernel(
             }
 #pragma unroll
             for (int it = 0; it < ITERS; ++it) {
-                const int col0 = (sub + it * G) * VEC;
-                if (col0 < n) {
+                const int unit = sub + it * G;
+                if (unit * V::kVec < n) {
+                    const int col0 = V::at(unit, n);
                     typename V::T x[4];
 #pragma unroll
                     for (int u = 0; u < 4; ++u)
@@ -141,19 +162,18 @@ __global__ __launch_bounds__(kBlock) void spmm_rowgroup_kernel(
     if (row < m && !deferred && owner) {
 #pragma unroll
         for (int it = 0; it < ITERS; ++it) {
-            const int col0 = (sub + it * G) * VEC;
-            if (col0 < n) {
+            const int unit = sub + it * G;
+            if (unit * V::kVec < n) {
+                const int col0 = V::at(unit, n);
                 if (hub >= 0) acc[it] = V::axpby(V::zero(), alpha, hub_row_sum<V>(hubs.part + (size_t)hub * hubs.ld + col0, hubs.ld, entries, hubs.shift));
-                float* dst = C + (size_t)row * ldc + col0;
-                if (beta == 0.f) V::store(dst, acc[it]);
-                else V::store(dst, V::axpby(acc[it], beta, V::load(dst)));
+                V::update(C + (size_t)row * ldc, unit, n, acc[it], beta);
             }
         }
     }
 
     __syncthreads();
     const int nlong = lr_count;           // uniform across the workgroup
-    const int width = G * VEC * ITERS;
+    const int width = G * V::kVec * ITERS;
     for (int li = 0; li < nlong; ++li) {
         const int lrow = lr_list[li];
         const int ls = row_ptr[lrow], le = row_ptr[lrow + 1];
@@ -168,8 +188,9 @@ __global__ __launch_bounds__(kBlock) void spmm_rowgroup_kernel(
             for (int u = 0; u < 4; ++u) { c4[u] = col_idx[t + u * ngroups]; v4[u] = alpha * val[t + u * ngroups]; }
 #pragma unroll
             for (int it = 0; it < ITERS; ++it) {
-                const int col0 = (sub + it * G) * VEC;
-                if (col0 < n) {
+                const int unit = sub + it * G;
+                if (unit * V::kVec < n) {
+                    const int col0 = V::at(unit, n);
                     typename V::T x[4];
 #pragma unroll
                     for (int u = 0; u < 4; ++u) x[u] = V::load(B + (size_t)c4[u] * ldb + col0);
@@ -183,8 +204,9 @@ __global__ __launch_bounds__(kBlock) void spmm_rowgroup_kernel(
             const float v0 = alpha * val[t];
 #pragma unroll
             for (int it = 0; it < ITERS; ++it) {
-                const int col0 = (sub + it * G) * VEC;
-                if (col0 < n) {
+                const int unit = sub + it * G;
+                if (unit * V::kVec < n) {
+                    const int col0 = V::at(unit, n);
                     const typename V::T x = V::load(B + (size_t)c0 * ldb + col0);
                     V::fma(acc[it], v0, RELU_IN ? V::relu(x) : x);
                 }
@@ -193,18 +215,16 @@ __global__ __launch_bounds__(kBlock) void spmm_rowgroup_kernel(
 
 #pragma unroll
         for (int it = 0; it < ITERS; ++it)
-            V::store(red + (size_t)grp * width + (sub + it * G) * VEC, acc[it]);
+            V::store(red + (size_t)grp * width + (sub + it * G) * V::kVec, acc[it]);
         __syncthreads();
         if (grp == 0) {
 #pragma unroll
             for (int it = 0; it < ITERS; ++it) {
-                const int col0 = (sub + it * G) * VEC;
-                if (col0 < n) {
+                const int unit = sub + it * G;
+                if (unit * V::kVec < n) {
                     typename V::T s = V::zero();
-                    for (int g = 0; g < ngroups; ++g) s = V::add(s, V::load(red + (size_t)g * width + col0));
-                    float* dst = C + (size_t)lrow * ldc + col0;
-                    if (beta == 0.f) V::store(dst, s);
-                    else V::store(dst, V::axpby(s, beta, V::load(dst)));
+                    for (int g = 0; g < ngroups; ++g) s = V::add(s, V::load(red + (size_t)g * width + unit * V::kVec));
+                    V::update(C + (size_t)lrow * ldc, unit, n, s, beta);
                 }
             }
         }
@@ -219,13 +239,16 @@ inline int ilog2_ceil(int x)
     return l;
 }
 
-template <int VEC, int ITERS>
+template <class V, int ITERS>
 int launch_slab(int m, int n, float alpha, const int* row_ptr, const int* col_idx, const float* val,
                 const float* B, int ldb, float beta, float* C, int ldc, int logG, const HubPlan& hubs, bool one_row, bool relu_in, hipStream_t s)
 {
     const int groups_per_block = one_row ? 1 : kBlock >> logG;
     const unsigned blocks = ceil_div_u((size_t)m, (size_t)groups_per_block);
-    const auto kernel = relu_in ? spmm_rowgroup_kernel<VEC, ITERS, true> : spmm_rowgroup_kernel<VEC, ITERS, false>;
+    auto kernel = relu_in ? spmm_rowgroup_kernel<V, ITERS, true, false> : spmm_rowgroup_kernel<V, ITERS, false, false>;
+    if constexpr (ITERS == 1) {
+        if ((1 << logG) <= kNarrowGroup) kernel = relu_in ? spmm_rowgroup_kernel<V, 1, true, true> : spmm_rowgroup_kernel<V, 1, false, true>;
+    }
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kBlock), 0, s,
                        m, n, alpha, row_ptr, col_idx, val, B, ldb, beta, C, ldc, logG, one_row ? -1 : kLongRow, hubs);
     GNNHIP_LAUNCH_CHECK("spmm_rowgroup");
@@ -257,12 +280,13 @@ int spmm_plain_dispatch(int m, int k, int n, long long nnz, float alpha, const i
     // few rows of hundreds of entries each (sum-pooling into subgraphs): a workgroup per row instead of a lane group
     const bool one_row = m < kHubMinRows && nnz >= kOneRowMeanEntries * (long long)m;
     const bool vec4 = (n % 4 == 0) && (ldb % 4 == 0) && (ldc % 4 == 0) && aligned16(B) && aligned16(C);
-    const int vec = vec4 ? 4 : 1;
+    const int vec = n >= 4 ? 4 : 1;
     // columns are processed in slabs of at most 64 lanes * vec * 4
     const int slab_max = kWave * vec * 4;
     for (int col0 = 0; col0 < n; col0 += slab_max) {
         const int w = (n - col0 < slab_max) ? (n - col0) : slab_max;
-        const int units = (w + vec - 1) / vec;              // column units of `vec` floats
+        const bool one = w < 4;                             // also what n mod 1024 leaves behind the full slabs
+        const int units = one ? w : (w + 3) / 4;            // column units of a lane
         int logG = ilog2_ceil(units < kWave ? units : kWave);
         const int G = 1 << logG;
         const int iters = (units + G - 1) / G;              // 1..4
@@ -271,14 +295,16 @@ int spmm_plain_dispatch(int m, int k, int n, long long nnz, float alpha, const i
         int rc;
         HubPlan hubs;
         if ((rc = hub_prepass(m, w, nnz, row_ptr, col_idx, val, Bs, ldb, s, &hubs, reuse_plan && n <= slab_max, relu_in, kHubThreshold, kHubChunk, -1, row_hub))) return rc;
-        if (vec4) {
-            if (iters <= 1) rc = launch_slab<4, 1>(m, w, alpha, row_ptr, col_idx, val, Bs, ldb, beta, Cs, ldc, logG, hubs, one_row, relu_in, s);
-            else if (iters == 2) rc = launch_slab<4, 2>(m, w, alpha, row_ptr, col_idx, val, Bs, ldb, beta, Cs, ldc, logG, hubs, one_row, relu_in, s);
-            else rc = launch_slab<4, 4>(m, w, alpha, row_ptr, col_idx, val, Bs, ldb, beta, Cs, ldc, logG, hubs, one_row, relu_in, s);
+        if (one) {
+            rc = launch_slab<ColsOne, 1>(m, w, alpha, row_ptr, col_idx, val, Bs, ldb, beta, Cs, ldc, logG, hubs, one_row, relu_in, s);
+        } else if (vec4) {
+            if (iters <= 1) rc = launch_slab<ColsWide, 1>(m, w, alpha, row_ptr, col_idx, val, Bs, ldb, beta, Cs, ldc, logG, hubs, one_row, relu_in, s);
+            else if (iters == 2) rc = launch_slab<ColsWide, 2>(m, w, alpha, row_ptr, col_idx, val, Bs, ldb, beta, Cs, ldc, logG, hubs, one_row, relu_in, s);
+            else rc = launch_slab<ColsWide, 4>(m, w, alpha, row_ptr, col_idx, val, Bs, ldb, beta, Cs, ldc, logG, hubs, one_row, relu_in, s);
         } else {
-            if (iters <= 1) rc = launch_slab<1, 1>(m, w, alpha, row_ptr, col_idx, val, Bs, ldb, beta, Cs, ldc, logG, hubs, one_row, relu_in, s);
-            else if (iters == 2) rc = launch_slab<1, 2>(m, w, alpha, row_ptr, col_idx, val, Bs, ldb, beta, Cs, ldc, logG, hubs, one_row, relu_in, s);
-            else rc = launch_slab<1, 4>(m, w, alpha, row_ptr, col_idx, val, Bs, ldb, beta, Cs, ldc, logG, hubs, one_row, relu_in, s);
+            if (iters <= 1) rc = launch_slab<ColsLoose, 1>(m, w, alpha, row_ptr, col_idx, val, Bs, ldb, beta, Cs, ldc, logG, hubs, one_row, relu_in, s);
+            else if (iters == 2) rc = launch_slab<ColsLoose, 2>(m, w, alpha, row_ptr, col_idx, val, Bs, ldb, beta, Cs, ldc, logG, hubs, one_row, relu_in, s);
+            else rc = launch_slab<ColsLoose, 4>(m, w, alpha, row_ptr, col_idx, val, Bs, ldb, beta, Cs, ldc, logG, hubs, one_row, relu_in, s);
         }
         if (rc) return rc;
     }

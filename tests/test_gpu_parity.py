@@ -1496,6 +1496,28 @@ def test_spmm_hub_rows_balanced_pass(gpu, oracle, n):
     assert np.array_equal(got, _n(ops.spmm(*_csr_t(csr, gpu), _t(B, gpu), m)))
 
 
+@pytest.mark.parametrize("n", [3, 5, 13, 17, 31, 101, 259, 1026])
+def test_spmm_rows_of_any_alignment(gpu, oracle, n):
+    """widths whose rows end inside a lane's four columns (the last unit is moved back, also across two sets of columns per
+    lane and in a last slab of two), and narrow ones, whose wavefronts copy their rows' entries first: runs of rows just
+    inside and past what is copied at once (768 entries), empty rows, a deferred row and a ragged end; also above
+    32,768 rows, where long rows come from the balanced pass"""
+    from graphnn_amd import ops
+    for m in (1_003, 32_801):
+        if m > 2_000 and n > 300:
+            continue
+        rng = np.random.default_rng(1200 + n + m)
+        k = 701
+        long_rows = [(r, 48) for r in range(64, 80)] + [(r, 49) for r in range(128, 144)] + [(200, 0), (201, 2_500), (m - 2, 0), (m - 1, 70)]
+        csr = _hub_matrix(rng, m, k, long_rows)
+        B = rng.standard_normal((k, n)).astype(np.float32)
+        C0 = rng.standard_normal((m, n)).astype(np.float32)
+        got = _n(ops.spmm(*_csr_t(csr, gpu), _t(B, gpu), m))
+        assert_parity("spmm", got, *_spmm_want(oracle, *csr, B, m))
+        got2 = _n(ops.spmm(*_csr_t(csr, gpu), _t(B, gpu), m, alpha=-0.5, beta=1.5, out=_t(C0, gpu)))
+        assert_parity("spmm", got2, *_spmm_want(oracle, *csr, B, m, alpha=-0.5, beta=1.5, C=C0))
+
+
 @pytest.mark.parametrize("m,n", [(37, 64), (300, 7), (1, 128), (2000, 300), (4096, 4)])
 def test_spmm_few_long_rows_take_a_workgroup_each(gpu, oracle, m, n):
     """rows of several hundred entries on average and fewer than 32,768 of them (sum-pooling into subgraphs): every
