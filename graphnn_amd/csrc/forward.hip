@@ -16,6 +16,14 @@ int level_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* c
 bool level_accepts_relu_input(int N, int C);
 int level_backward_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* dz,
                             const float* W, float* u, float* g_prev, const float* gate, float* acc, hipStream_t s);
+// level_rows.hip
+int level_rows_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* h_in,
+                        const float* W, const float* msg, const float* bias, float* h_out, bool same_graph, bool relu_in, CsrPlan* plan,
+                        hipStream_t s);
+int level_rows_backward_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* dz,
+                                 const float* W, float* u, float* g_prev, const float* gate, float* acc, hipStream_t s);
+int level_rows_dense_dispatch(int N, int K, int n, const float* x, const float* W, const float* bias, const float* msg, float* out,
+                              bool relu, float* relu_out, hipStream_t s);
 int readout_dispatch(int B, int C, int H, int Q, const int* s_row_ptr, const int* s_col_idx, const float* s_val,
                      const float* h, const float* Wh1, const float* Wh2, float* pool, float* hidden,
                      float* logits, float* probs, int* pred, hipStream_t s);
@@ -58,17 +66,27 @@ inline unsigned ew_grid(size_t n)
     return (unsigned)b;
 }
 
+// out = ReLU(x * W + bias + msg) or, with relu_out, out = x * W and relu_out = ReLU(out)
+int product_any(int N, int K, int n, const float* x, const float* W, const float* bias, const float* msg, float* out, float* relu_out,
+                hipStream_t s)
+{
+    int rc = level_rows_dense_dispatch(N, K, n, x, W, bias, msg, out, !relu_out, relu_out, s);
+    if (rc != GNNHIP_EUNSUPPORTED) return rc;
+    if ((rc = gemm_dispatch(0, 0, N, n, K, 1.f, x, K, W, n, 0.f, out, n, s))) return rc;
+    const size_t total = (size_t)N * n;
+    hipLaunchKernelGGL(bias_add_relu_kernel, dim3(ew_grid(total)), dim3(kBlock), 0, s, out, bias, msg, out, relu_out, total, n, 1);
+    GNNHIP_LAUNCH_CHECK("bias_add_relu");
+    return GNNHIP_OK;
+}
+
 int input_any(int N, int K, int C, const float* X, const float* Wn2l, float* msg, float* h0, hipStream_t s)
 {
     int rc = input_dispatch(N, K, C, X, Wn2l, msg, h0, s);
     if (rc != GNNHIP_EUNSUPPORTED) return rc;
-    if ((rc = gemm_dispatch(0, 0, N, C, K, 1.f, X, K, Wn2l, C, 0.f, msg, C, s))) return rc;
-    if (!h0) return GNNHIP_OK;
-    const size_t total = (size_t)N * C;
-    hipLaunchKernelGGL(bias_add_relu_kernel, dim3(ew_grid(total)), dim3(kBlock), 0, s,
-                       msg, (const float*)nullptr, (const float*)nullptr, msg, h0, total, C, 1);
-    GNNHIP_LAUNCH_CHECK("bias_add_relu");
-    return GNNHIP_OK;
+    if (h0) return product_any(N, K, C, X, Wn2l, nullptr, nullptr, msg, h0, s);
+    rc = level_rows_dense_dispatch(N, K, C, X, Wn2l, nullptr, nullptr, msg, false, nullptr, s);
+    if (rc != GNNHIP_EUNSUPPORTED) return rc;
+    return gemm_dispatch(0, 0, N, C, K, 1.f, X, K, Wn2l, C, 0.f, msg, C, s);
 }
 
 int level_any(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* h_in,
@@ -77,17 +95,13 @@ int level_any(int N, int C, long long nnz, const int* row_ptr, const int* col_id
 {
     int rc = level_dispatch(N, C, nnz, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, s, same_graph, relu_in, plan, inference);
     if (rc != GNNHIP_EUNSUPPORTED) return rc;
-    if (relu_in) return set_error(GNNHIP_EUNSUPPORTED, "no level kernel reads its input through ReLU for this shape");
+    rc = level_rows_dispatch(N, C, nnz, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, same_graph, relu_in, plan, s);
+    if (rc != GNNHIP_EUNSUPPORTED) return rc;
     void* tmp = nullptr;
-    const size_t total = (size_t)N * C;
-    if ((rc = stream_scratch(s, sizeof(float) * total, &tmp))) return rc;
+    if ((rc = stream_scratch(s, sizeof(float) * (size_t)N * C, &tmp))) return rc;
     float* agg = static_cast<float*>(tmp);
-    if ((rc = spmm_dispatch(N, N, C, nnz, 1.f, row_ptr, col_idx, val, h_in, C, 0.f, agg, C, s, same_graph, plan))) return rc;
-    if ((rc = gemm_dispatch(0, 0, N, C, C, 1.f, agg, C, W, C, 0.f, h_out, C, s))) return rc;
-    hipLaunchKernelGGL(bias_add_relu_kernel, dim3(ew_grid(total)), dim3(kBlock), 0, s,
-                       h_out, bias, msg, h_out, (float*)nullptr, total, C, 1);
-    GNNHIP_LAUNCH_CHECK("bias_add_relu");
-    return GNNHIP_OK;
+    if ((rc = spmm_dispatch(N, N, C, nnz, 1.f, row_ptr, col_idx, val, h_in, C, 0.f, agg, C, s, same_graph, plan, relu_in))) return rc;
+    return product_any(N, C, C, agg, W, bias, msg, h_out, nullptr, s);
 }
 
 __global__ __launch_bounds__(kBlock) void copy_kernel(const float* __restrict__ src, float* __restrict__ dst, size_t n)
@@ -121,11 +135,7 @@ int readout_any(int B, int N, int C, int H, int Q, const int* s_row_ptr, const i
         rc = readout_dispatch(B, C, H, Q, s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2, pool, hidden, logits, probs, pred, s);
     if (rc != GNNHIP_EUNSUPPORTED) return rc;
     if ((rc = spmm_dispatch(B, N, C, (long long)N, 1.f, s_row_ptr, s_col_idx, s_val, h, C, 0.f, pool, C, s))) return rc;
-    if ((rc = gemm_dispatch(0, 0, B, H, C, 1.f, pool, C, Wh1, H, 0.f, hidden, H, s))) return rc;
-    const size_t bh = (size_t)B * H;
-    hipLaunchKernelGGL(bias_add_relu_kernel, dim3(ew_grid(bh)), dim3(kBlock), 0, s,
-                       hidden, (const float*)nullptr, (const float*)nullptr, hidden, (float*)nullptr, bh, H, 1);
-    GNNHIP_LAUNCH_CHECK("bias_add_relu");
+    if ((rc = product_any(B, C, H, pool, Wh1, nullptr, nullptr, hidden, nullptr, s))) return rc;
     if ((rc = gemm_dispatch(0, 0, B, Q, H, 1.f, hidden, H, Wh2, Q, 0.f, logits, Q, s))) return rc;
     if (pred && (rc = row_argmax_dispatch(logits, B, Q, pred, s))) return rc;
     if (probs) {
@@ -145,7 +155,8 @@ int forward_any(int N, int B, int K, int C, int H, int Q, int L, long long a_nnz
 {
     // With at least one level, and a level kernel that can read its input through ReLU, h0 = ReLU(msg) is
     // never stored: the first level gathers from msg.
-    const bool lazy_h0 = L >= 1 && level_accepts_relu_input(N, C) && aligned16(msg) && aligned16(h_a) && aligned16(h_b) && aligned16(W_conv);
+    // (the routes of the other sizes can too)
+    const bool lazy_h0 = L >= 1 && (level_accepts_relu_input(N, C) || !fused_hidden_supported(C)) && aligned16(msg) && aligned16(h_a) && aligned16(h_b) && aligned16(W_conv);
     int rc = input_any(N, K, C, X, W_n2l, msg, lazy_h0 ? nullptr : h_a, s);
     if (rc) return rc;
     float* cur = lazy_h0 ? msg : h_a;
@@ -217,6 +228,8 @@ int gnnhip_s2v_level_backward_f32(int N, int C, int nnz, const int* t_row_ptr, c
     if (int rc = require_ready()) return rc;
     hipStream_t s = as_stream(stream);
     int rc = level_backward_dispatch(N, C, nnz, t_row_ptr, t_col_idx, t_val, dz, W, u, g_prev, gate_h, acc, s);
+    if (rc != GNNHIP_EUNSUPPORTED) return rc;
+    rc = level_rows_backward_dispatch(N, C, nnz, t_row_ptr, t_col_idx, t_val, dz, W, u, g_prev, gate_h, acc, s);
     if (rc != GNNHIP_EUNSUPPORTED) return rc;
     if ((rc = spmm_dispatch(N, N, C, nnz, 1.f, t_row_ptr, t_col_idx, t_val, dz, C, 0.f, u, C, s))) return rc;
     if ((rc = gemm_dispatch(0, 1, N, C, C, 1.f, u, C, W, C, 0.f, g_prev, C, s))) return rc;

@@ -1,0 +1,378 @@
+// Mean-field level and its input stage for hidden sizes that no tuned kernel covers (4 <= C <= 256):
+//
+//   level      h_out = ReLU((A * h_in) * W + bias + msg)
+//   backward   u = A' * dz ; g_prev = u * W^T, zeroed where gate <= 0 ; acc += g_prev
+//   dense      out = X * W (+ bias + msg, ReLU), and a second output ReLU(out)
+//
+// as one launch each, instead of an SpMM, a GEMM and an element-wise pass over N x C.  Measured at 48,750 nodes, hidden 100,
+// 4.8 entries per row: 41 -> 31 us per level and 28 -> 11 us for the input stage; 130,000 nodes, hidden 199: 400 -> 190 us.
+// The FP32 matrix cores bound the wide sizes (11 of the 31 us, 115 of the 190), memory the narrow ones.
+//
+// A workgroup takes R = 16 RT consecutive rows:
+//   1. the rows of the left operand are put into LDS [R][KP + 4], KP = their width rounded up to 16, zeros behind it.  Gathered
+//      rows: the tile's CSR entries, which lie next to each other, are copied to LDS first when there are at most kStaged,
+//      then a group of G lanes (a power of two, 4 G >= width) sums a row, eight gathers in flight, entries in order;
+//   2. the four wavefronts share the 16-column blocks of the product, up to NB each, all R rows: v_mfma_f32_16x16x4_f32, W
+//      straight from L2 one step of 16 k ahead (40 KB per tile at hidden 100 against 128 KB of gathered rows).  Sharing out
+//      the blocks of the last, uneven round row by row of blocks was tried: the extra loads of W cost more (179 -> 214 us at
+//      390,000 nodes, hidden 85);
+//   3. the product goes back through the same LDS, rows packed at their own width, so that what follows (msg, gate, sums,
+//      ReLU, stores) walks flat 16-byte words of memory whatever the width: the R rows of a tile are contiguous, and R times
+//      any width is a multiple of four.
+// Sums have the order of the row-group SpMM and of the GEMM tile kernel, so every bit is theirs.
+//
+// Rows of more than kHubThreshold entries come from the balanced pass (hub.hip) where it runs, as in the SpMM; elsewhere rows
+// longer than kLongRow are summed by the whole workgroup.
+#include "columns.h"
+#include "buffer_addr.h"
+#include <initializer_list>
+
+namespace gnnhip {
+namespace {
+
+constexpr int kBlock = 256;
+constexpr int kWaves = kBlock / kWave;
+constexpr int kStaged = 1024;             // CSR entries of a tile copied to LDS (8 KB)
+constexpr int kLongRow = 2048;
+constexpr int kMaxWidth = 256;            // of the left operand's rows and of the product's
+constexpr int kFlight = 8;
+
+struct RowsArgs {
+    int N, K, n;                          // rows, width of the left operand, width of the product
+    const int *row_ptr, *col_idx;         // gathered left operand (A * x); null row_ptr: x itself
+    const float *val, *x, *W;
+    const float *bias, *msg, *gate;       // msg: added; gate: product zeroed where gate <= 0
+    float *agg_out, *out, *relu_out, *acc;   // agg_out: the left operand's rows; relu_out: ReLU(out); acc: += out
+    int relu, relu_in;
+    unsigned k_magic;                     // ceil(2^32 / K)
+    HubPlan hubs;
+};
+
+// GATHER: the left operand is A * x.  WT: the product is with W^T.
+template <int RT, int NB, bool GATHER, bool WT>
+__global__ __launch_bounds__(kBlock, 3) void s2v_rows_kernel(RowsArgs a)
+{
+    using V = ColsLoose;
+    constexpr int R = 16 * RT;
+    extern __shared__ float4 smem4[];
+    __shared__ int rp[R + 1];
+    __shared__ float4 shared4[GATHER ? kStaged / 2 : 1];       // the tile's entries, then the sums of its long rows
+    int2* staged = reinterpret_cast<int2*>(shared4);
+    static_assert(kStaged / 2 >= kBlock, "a word per lane");
+    __shared__ int long_row[GATHER ? R : 1];
+    __shared__ int long_count;
+    float* tile = reinterpret_cast<float*>(smem4);
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    const int q = lane >> 4, t = lane & 15;
+    const int K = a.K, n = a.n;
+    const int KP = (K + 15) & ~15, LD = KP + 4;
+    const long long row0 = (long long)blockIdx.x * R;
+    const int rows = (int)min((long long)R, (long long)a.N - row0);
+
+    // ---- W of step k0 for this wavefront's column blocks: wf[b][s] = W[k0 + 4 q + s][16 (wave + 4 b) + t], zero from k = K on
+    const rsrc_t w_rsrc = make_rsrc(a.W, (unsigned)((size_t)K * n * 4));
+    const int nb = wave < (n + 15) / 16 ? ((n + 15) / 16 - wave + kWaves - 1) / kWaves : 0;      // blocks of this wavefront
+    auto load_w = [&](int k0, float (&wf)[NB][4]) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            if (b >= nb) continue;                             // uniform
+            const int col = 16 * (wave + kWaves * b) + t;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const int k = k0 + 4 * q + s;
+                const int off = WT ? (col * K + k) * 4 : (k * n + col) * 4;       // a column past n: a word that is not stored
+                wf[b][s] = buf_load_f(w_rsrc, k < K ? off : kBufPastEnd, 0);
+            }
+        }
+    };
+    float wf[NB][4];
+    load_w(0, wf);
+
+    // ---- 1. the left operand's rows
+    if constexpr (GATHER) {
+        if (tid <= R) rp[tid] = a.row_ptr[min(row0 + tid, (long long)a.N)];
+        if (tid == 0) long_count = 0;
+        for (int i = tid; i < R * 16; i += kBlock) {                    // the columns behind K
+            const int c = KP - 16 + (i & 15);
+            if (c >= K) tile[(i >> 4) * LD + c] = 0.f;
+        }
+        __syncthreads();
+        const int lo = rp[0], hi = rp[R];
+        const bool in_lds = hi - lo <= kStaged;
+        if (in_lds) {
+            for (int e = lo + tid; e < hi; e += kBlock) staged[e - lo] = make_int2(a.col_idx[e], __float_as_int(a.val[e]));
+            __syncthreads();
+        }
+        const int units = (K + 3) / 4;
+        const int logG = units <= 1 ? 0 : 32 - __builtin_clz((unsigned)(units - 1));
+        const int G = 1 << logG, sub = tid & (G - 1), grp = tid >> logG, ngroups = kBlock >> logG;
+        const bool live = sub < units;
+        const int col0 = V::at(sub, K);
+        auto add_row = [&](int start, int end, auto entry) {
+            float4 sum = f4_zero();
+            for (int base = start; base < end; base += kFlight) {
+                int2 cv[kFlight];
+                float4 x[kFlight];
+#pragma unroll
+                for (int u = 0; u < kFlight; ++u) cv[u] = base + u < end ? entry(base + u) : make_int2(0, 0);
+#pragma unroll
+                for (int u = 0; u < kFlight; ++u) x[u] = base + u < end && live ? V::load(a.x + (size_t)cv[u].x * K + col0) : f4_zero();
+#pragma unroll
+                for (int u = 0; u < kFlight; ++u)
+                    if (base + u < end) f4_fma(sum, __int_as_float(cv[u].y), a.relu_in ? relu_ref4(x[u]) : x[u]);
+            }
+            return sum;
+        };
+        auto finish_row = [&](int r, const float4& sum) {
+            if (!live) return;
+            V::store(tile + r * LD + col0, sum);
+            if (a.agg_out && r < rows) V::store(a.agg_out + (size_t)(row0 + r) * K + col0, sum);
+        };
+        for (int r = grp; r < R; r += ngroups) {
+            const int start = rp[r], end = rp[r + 1];
+            const int entries = end - start;
+            int hub = -1;
+            if (a.hubs.row_chunk && entries > kHubThreshold) hub = a.hubs.row_chunk[row0 + r];
+            if (hub >= 0) {
+                float4 sum = f4_zero();
+                if (live) sum = V::axpby(f4_zero(), 1.f, hub_row_sum<V>(a.hubs.part + (size_t)hub * a.hubs.ld + col0, a.hubs.ld, entries, a.hubs.shift));
+                finish_row(r, sum);
+            } else if (entries > kLongRow) {
+                if (sub == 0) long_row[atomicAdd(&long_count, 1)] = r;
+            } else if (in_lds) {
+                finish_row(r, add_row(start, end, [&](int e) { return staged[e - lo]; }));
+            } else {
+                finish_row(r, add_row(start, end, [&](int e) { return make_int2(a.col_idx[e], __float_as_int(a.val[e])); }));
+            }
+        }
+        __syncthreads();
+        const int nlong = long_count;
+        for (int li = 0; li < nlong; ++li) {
+            // the groups take entries grp, grp + ngroups, ...; their sums are added in group order
+            const int r = long_row[li];
+            const int start = rp[r], end = rp[r + 1];
+            float4 sum = f4_zero();
+            for (int e = start + grp; e < end; e += 4 * ngroups) {
+                int c[4];
+                float v[4];
+                float4 x[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const bool ok = e + u * ngroups < end;
+                    c[u] = ok ? a.col_idx[e + u * ngroups] : 0;
+                    v[u] = ok ? a.val[e + u * ngroups] : 0.f;
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) x[u] = e + u * ngroups < end && live ? V::load(a.x + (size_t)c[u] * K + col0) : f4_zero();
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (e + u * ngroups < end) f4_fma(sum, v[u], a.relu_in ? relu_ref4(x[u]) : x[u]);
+            }
+            shared4[tid] = sum;
+            __syncthreads();
+            if (grp == 0 && live) {
+                float4 s = f4_zero();
+                for (int g = 0; g < ngroups; ++g) s = V::add(s, shared4[g * G + sub]);
+                V::store(tile + r * LD + col0, s);
+                if (a.agg_out) V::store(a.agg_out + (size_t)(row0 + r) * K + col0, s);
+            }
+            __syncthreads();
+        }
+    } else {
+        // rows are contiguous: element i of the tile's part of x is row i / K, column i % K
+        for (int i = tid; i < R * 16; i += kBlock) {
+            const int c = KP - 16 + (i & 15);
+            if (c >= K || (i >> 4) >= rows) tile[(i >> 4) * LD + c] = 0.f;
+        }
+        const float* src = a.x + (size_t)row0 * K;
+        const int total = rows * K;
+        for (int base = 0; base < total; base += kFlight * kBlock) {
+            float v[kFlight];
+#pragma unroll
+            for (int u = 0; u < kFlight; ++u) { const int i = base + tid + u * kBlock; v[u] = i < total ? src[i] : 0.f; }
+#pragma unroll
+            for (int u = 0; u < kFlight; ++u) {
+                const int i = base + tid + u * kBlock;
+                const int r = K >= 2 ? (int)__umulhi((unsigned)i, a.k_magic) : i;
+                if (i < total) tile[r * LD + i - r * K] = v[u];
+            }
+        }
+        __syncthreads();
+    }
+
+    // ---- 2. the product: lane (q, t) supplies row t's k = k0 + 4 q + s at instruction s and ends up with columns 4 q .. + 3 of
+    // that row of a block
+    mfma_f4 acc[NB][RT];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int i = 0; i < RT; ++i) acc[b][i] = mfma_f4{0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < KP; k0 += 16) {
+        float wn[NB][4];
+        load_w(k0 + 16, wn);                                   // past the end: zeros, nothing is read
+        float4 x[RT];
+#pragma unroll
+        for (int i = 0; i < RT; ++i) x[i] = *reinterpret_cast<const float4*>(tile + (16 * i + t) * LD + k0 + 4 * q);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            if (b >= nb) continue;                          // uniform
+#pragma unroll
+            for (int i = 0; i < RT; ++i) acc[b][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[b][0], x[i].x, acc[b][i], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < RT; ++i) acc[b][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[b][1], x[i].y, acc[b][i], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < RT; ++i) acc[b][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[b][2], x[i].z, acc[b][i], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < RT; ++i) acc[b][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[b][3], x[i].w, acc[b][i], 0, 0, 0);
+        }
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) wf[b][s] = wn[b][s];
+    }
+    __syncthreads();                                           // the left operand has been read
+    auto put = [&](int row_block, int col_block, const mfma_f4& v) {
+        const int col = col_block + 4 * q;
+        float* dst = tile + (16 * row_block + t) * n + col;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (col + j < n) dst[j] = v[j];
+    };
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+        if (b < nb) {
+#pragma unroll
+            for (int i = 0; i < RT; ++i) put(i, 16 * (wave + kWaves * b), acc[b][i]);
+        }
+
+    // ---- 3. flat words of the tile's rows; everything they wait for from memory is asked for at once
+    constexpr int EX = R * 64 * NB / (4 * kBlock);
+    const size_t flat0 = (size_t)row0 * n;
+    const int total = rows * n;
+    auto load = [&](const float* p, int i) {
+        float4 v = f4_zero();
+        if (i + 4 <= total) return *reinterpret_cast<const float4*>(p + flat0 + i);
+        if (i < total) v.x = p[flat0 + i];
+        if (i + 1 < total) v.y = p[flat0 + i + 1];
+        if (i + 2 < total) v.z = p[flat0 + i + 2];
+        return v;
+    };
+    auto store = [&](float* p, int i, const float4& v) {
+        if (i + 4 <= total) { *reinterpret_cast<float4*>(p + flat0 + i) = v; return; }
+        p[flat0 + i] = v.x;
+        if (i + 1 < total) p[flat0 + i + 1] = v.y;
+        if (i + 2 < total) p[flat0 + i + 2] = v.z;
+    };
+    const float* first = a.msg ? a.msg : a.gate;
+    float4 ex[EX], ac[WT ? EX : 1];
+#pragma unroll
+    for (int u = 0; u < EX; ++u) ex[u] = first ? load(first, 4 * (tid + u * kBlock)) : f4_zero();
+    if constexpr (WT) {
+#pragma unroll
+        for (int u = 0; u < EX; ++u) ac[u] = a.acc ? load(a.acc, 4 * (tid + u * kBlock)) : f4_zero();
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < EX; ++u) {
+        const int i = 4 * (tid + u * kBlock);
+        if (i < total) {
+            float4 v = *reinterpret_cast<const float4*>(tile + i);
+            if (a.bias) { v.x += a.bias[i % n]; v.y += a.bias[(i + 1) % n]; v.z += a.bias[(i + 2) % n]; v.w += a.bias[(i + 3) % n]; }
+            if (a.msg) v = V::add(v, ex[u]);
+            if constexpr (WT) {
+                if (a.gate)
+                    v = make_float4(ex[u].x > 0.f ? v.x : 0.f, ex[u].y > 0.f ? v.y : 0.f, ex[u].z > 0.f ? v.z : 0.f, ex[u].w > 0.f ? v.w : 0.f);
+            }
+            if (a.relu) v = relu_ref4(v);
+            store(a.out, i, v);
+            if (a.relu_out) store(a.relu_out, i, relu_ref4(v));
+            if constexpr (WT) {
+                if (a.acc) store(a.acc, i, V::add(ac[u], v));
+            }
+        }
+    }
+}
+
+template <int RT, int NB, bool GATHER, bool WT>
+int launch_rows(const RowsArgs& a, hipStream_t s)
+{
+    const int KP = (a.K + 15) & ~15;
+    const int width = KP + 4 > a.n ? KP + 4 : a.n;
+    const unsigned grid = (unsigned)(((long long)a.N + 16 * RT - 1) / (16 * RT));
+    hipLaunchKernelGGL((s2v_rows_kernel<RT, NB, GATHER, WT>), dim3(grid), dim3(kBlock), sizeof(float) * 16 * RT * width, s, a);
+    GNNHIP_LAUNCH_CHECK("s2v_rows");
+    return GNNHIP_OK;
+}
+
+template <bool GATHER, bool WT>
+int rows_dispatch(RowsArgs a, hipStream_t s)
+{
+    a.k_magic = a.K >= 2 ? (unsigned)(((1ull << 32) + a.K - 1) / a.K) : 0;
+    // Few rows: the smallest tiles, so that there is a workgroup for every compute unit; else 64 rows, which use every
+    // fetched word of W four times, or 32 where the tile would leave room for two workgroups per compute unit.
+    const bool few = a.N < 64 * kNumCU;
+    if (a.n <= 64) return few ? launch_rows<1, 1, GATHER, WT>(a, s) : launch_rows<4, 1, GATHER, WT>(a, s);
+    if (a.n <= 128) return few ? launch_rows<1, 2, GATHER, WT>(a, s) : launch_rows<4, 2, GATHER, WT>(a, s);
+    return few ? launch_rows<1, 4, GATHER, WT>(a, s) : launch_rows<2, 4, GATHER, WT>(a, s);
+}
+
+inline bool all_aligned(std::initializer_list<const void*> ps)
+{
+    for (const void* p : ps)
+        if (!aligned16(p)) return false;
+    return true;
+}
+
+}  // namespace
+
+namespace {
+// Whether the gathered products below take a matrix of this size.  Denser ones go through the SpMM, which cuts long rows into
+// pieces from kHubMinRows rows and 12 entries per row on and gives a row a workgroup from 256 entries per row on, and
+// level_rows_dense_dispatch.
+bool level_rows_covers(int N, int C, long long nnz)
+{
+    const long long mean = N >= kHubMinRows ? 12 : 256;
+    return C >= 4 && C <= kMaxWidth && nnz < mean * (long long)N;
+}
+}  // namespace
+
+int level_rows_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* h_in,
+                        const float* W, const float* msg, const float* bias, float* h_out, bool same_graph, bool relu_in, CsrPlan* plan,
+                        hipStream_t s)
+{
+    if (!level_rows_covers(N, C, nnz) || !all_aligned({msg, h_out})) return GNNHIP_EUNSUPPORTED;
+    RowsArgs a{};
+    if (int rc = hub_prepass(N, C, nnz, row_ptr, col_idx, val, h_in, C, s, &a.hubs, same_graph, relu_in, kHubThreshold, kHubChunk, -1,
+                             plan ? &plan->row_hub : nullptr))
+        return rc;
+    a.N = N; a.K = C; a.n = C;
+    a.row_ptr = row_ptr; a.col_idx = col_idx; a.val = val; a.x = h_in; a.W = W;
+    a.bias = bias; a.msg = msg; a.out = h_out; a.relu = 1; a.relu_in = relu_in;
+    return rows_dispatch<true, false>(a, s);
+}
+
+int level_rows_backward_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* dz,
+                                 const float* W, float* u, float* g_prev, const float* gate, float* acc, hipStream_t s)
+{
+    if (!level_rows_covers(N, C, nnz) || !all_aligned({g_prev, gate, acc})) return GNNHIP_EUNSUPPORTED;
+    RowsArgs a{};
+    if (int rc = hub_prepass(N, C, nnz, row_ptr, col_idx, val, dz, C, s, &a.hubs)) return rc;
+    a.N = N; a.K = C; a.n = C;
+    a.row_ptr = row_ptr; a.col_idx = col_idx; a.val = val; a.x = dz; a.W = W;
+    a.gate = gate; a.agg_out = u; a.out = g_prev; a.acc = acc;
+    return rows_dispatch<true, true>(a, s);
+}
+
+// out = x * W (+ bias + msg); relu: out = ReLU of that; relu_out (or null) = ReLU(out).  x [N, K], W [K, n].
+int level_rows_dense_dispatch(int N, int K, int n, const float* x, const float* W, const float* bias, const float* msg, float* out,
+                              bool relu, float* relu_out, hipStream_t s)
+{
+    // (64 rows of more than 252 columns would not fit 64 KB of LDS)
+    if (K < 1 || K > (n <= 128 ? 128 : kMaxWidth) || n > kMaxWidth || !all_aligned({msg, out, relu_out})) return GNNHIP_EUNSUPPORTED;
+    RowsArgs a{};
+    a.N = N; a.K = K; a.n = n;
+    a.x = x; a.W = W; a.bias = bias; a.msg = msg; a.out = out; a.relu = relu; a.relu_out = relu_out;
+    return rows_dispatch<false, false>(a, s);
+}
+
+}  // namespace gnnhip

@@ -127,6 +127,47 @@ def test_level_backward(gpu, oracle, C, N):
     assert np.array_equal(_n(g3), _n(g)) and np.array_equal(_n(acc), acc0 + _n(g))
 
 
+@pytest.mark.parametrize("C", [4, 7, 48, 63, 65, 100, 129, 255])
+@pytest.mark.parametrize("N", [1, 17, 1_500, 16_421, 32_770])
+def test_level_of_any_hidden_size_both_directions(gpu, oracle, C, N):
+    """hidden sizes without a kernel of their own, forward and backward in one launch each: column counts around the blocks of
+    16 and the shares of the wavefronts, row counts around the tiles of 16, 32 and 64 rows, tiles whose entries do not fit
+    LDS, rows longer than 64 (the balanced pass from 32,768 rows on) and 2,048 entries, empty rows, the input stage"""
+    from graphnn_amd import ops
+    if N * C > 2_200_000:
+        pytest.skip("the float64 model of the larger sizes adds nothing")
+    rng = np.random.default_rng(C + N)
+    lens = rng.integers(0, 6, N)
+    if N > 100:
+        lens[10:40] = 60; lens[41] = 0; lens[N // 2] = 3000; lens[N - 1] = 70
+    rp = np.zeros(N + 1, np.int32); np.cumsum(lens, out=rp[1:])
+    nnz = int(rp[-1])
+    ci = rng.integers(0, N, nnz).astype(np.int32)
+    v = (rng.random(nnz) * 0.5).astype(np.float32)
+    x = rng.random((N, C)).astype(np.float32)           # sums of 3,000 signed terms would cancel
+    W = (rng.standard_normal((C, C)) * 0.1).astype(np.float32)
+    msg = rng.standard_normal((N, C)).astype(np.float32)
+    bias = rng.standard_normal(C).astype(np.float32)
+    pad = lambda a, dt: _t(np.concatenate([a, np.zeros(1, dt)]), gpu)[:a.size]      # never a null pointer for an empty array
+    A = (_t(rp, gpu), pad(ci, np.int32), pad(v, np.float32))
+    import scipy.sparse as sp
+    u64 = sp.csr_matrix((v.astype(np.float64), ci, rp), shape=(N, N)) @ x.astype(np.float64)
+    got = ops.s2v_level(*A, _t(x, gpu), _t(W, gpu), _t(msg, gpu), _t(bias, gpu))
+    assert_parity("level", _n(got), oracle.level(rp, ci, v, x, W, msg, bias), np.maximum(u64 @ W.astype(np.float64) + bias + msg, 0))
+    h_prev = rng.standard_normal((N, C)).astype(np.float32)
+    acc = _t(msg, gpu)
+    u, g = ops.s2v_level_backward(*A, _t(x, gpu), _t(W, gpu), gate_h=_t(h_prev, gpu), acc=acc)
+    w_u = oracle.spmm(rp, ci, v, x, N)
+    assert_parity("u", _n(u), w_u, u64)
+    assert_parity("g_prev", _n(g), (oracle.gemm(w_u, W, transB=True) * (h_prev > 0)).astype(np.float32), (u64 @ W.astype(np.float64).T) * (h_prev > 0))
+    assert np.array_equal(_n(acc), msg + _n(g))
+    X = rng.standard_normal((N, 19)).astype(np.float32)
+    Wn = rng.standard_normal((19, C)).astype(np.float32)
+    m, h0 = ops.s2v_input(_t(X, gpu), _t(Wn, gpu))
+    assert_parity("msg", _n(m), oracle.gemm(X, Wn), X.astype(np.float64) @ Wn.astype(np.float64))
+    assert np.array_equal(_n(h0), np.maximum(_n(m), 0))
+
+
 @pytest.mark.parametrize("C", [128, 256])
 @pytest.mark.parametrize("nnz", [0, 3, 6])
 def test_level_backward_wide_with_hardly_any_entries(gpu, oracle, C, nnz):
