@@ -24,9 +24,8 @@ int level_rows_backward_dispatch(int N, int C, long long nnz, const int* row_ptr
                                  const float* W, float* u, float* g_prev, const float* gate, float* acc, hipStream_t s);
 int level_rows_dense_dispatch(int N, int K, int n, const float* x, const float* W, const float* bias, const float* msg, float* out,
                               bool relu, float* relu_out, hipStream_t s);
-int readout_dispatch(int B, int C, int H, int Q, const int* s_row_ptr, const int* s_col_idx, const float* s_val,
-                     const float* h, const float* Wh1, const float* Wh2, float* pool, float* hidden,
-                     float* logits, float* probs, int* pred, hipStream_t s);
+int readout_rows_dispatch(int B, int N, int C, int H, int Q, const int* s_row_ptr, const int* s_col_idx, const float* s_val, const float* h,
+                          const float* Wh1, const float* Wh2, float* pool, float* hidden, float* logits, float* probs, int* pred, hipStream_t s);
 int readout_wave_dispatch(int B, int C, int H, int Q, const int* s_row_ptr, const int* s_col_idx, const float* s_val,
                           const float* h, const float* Wh1, const float* Wh2, float* pool, float* hidden,
                           float* logits, float* probs, int* pred, hipStream_t s);
@@ -112,27 +111,24 @@ __global__ __launch_bounds__(kBlock) void copy_kernel(const float* __restrict__ 
 
 constexpr int kWaveReadoutMinGraphs = 1024;        // below this a workgroup per graph
 constexpr int kWaveReadoutMaxMeanNodes = 2048;     // mean nodes per graph
-constexpr int kBlockReadoutMaxGraphsWide = 4096;   // hidden 128/256: above this a workgroup per tile of graphs (or SpMM + GEMM)
-constexpr int kTileReadoutMinGraphs = 4096;
+constexpr int kTileReadoutMinGraphs = 4096;        // hidden 128/256
 
 int readout_any(int B, int N, int C, int H, int Q, const int* s_row_ptr, const int* s_col_idx, const float* s_val,
                 const float* h, const float* Wh1, const float* Wh2, float* pool, float* hidden,
                 float* logits, float* probs, int* pred, hipStream_t s)
 {
     // Many graphs of moderate size: one wavefront per graph (30,000 graphs of 29 nodes, hidden 64: 78 us with
-    // a workgroup per graph).  Few graphs: a workgroup per graph reaches more of the chip.  Graphs of
-    // thousands of nodes are left to the SpMM, which balances long rows.
+    // a workgroup per graph).  Few graphs, and graphs of thousands of nodes: a workgroup per graph reaches more
+    // of the chip.
     int rc = GNNHIP_EUNSUPPORTED;
     if (B >= kWaveReadoutMinGraphs && (long long)N <= (long long)B * kWaveReadoutMaxMeanNodes)
         rc = readout_wave_dispatch(B, C, H, Q, s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2, pool, hidden, logits, probs, pred, s);
     if (rc != GNNHIP_EUNSUPPORTED) return rc;
-    // hidden 128/256: a workgroup per graph up to a few thousand graphs (256 graphs, hidden 256: 20 us against
-    // 67 us for the seven launches below); 10,000 graphs: 116 against 106 us
+    // hidden 128/256: a workgroup per graph up to a few thousand graphs, then a tile of graphs per workgroup
     if (C > 64 && B > kTileReadoutMinGraphs && (long long)N <= (long long)B * kWaveReadoutMaxMeanNodes)
         rc = readout_tile_dispatch(B, C, H, Q, s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2, pool, hidden, logits, probs, pred, s);
     if (rc != GNNHIP_EUNSUPPORTED) return rc;
-    if (C <= 64 || B <= kBlockReadoutMaxGraphsWide)
-        rc = readout_dispatch(B, C, H, Q, s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2, pool, hidden, logits, probs, pred, s);
+    rc = readout_rows_dispatch(B, N, C, H, Q, s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2, pool, hidden, logits, probs, pred, s);
     if (rc != GNNHIP_EUNSUPPORTED) return rc;
     if ((rc = spmm_dispatch(B, N, C, (long long)N, 1.f, s_row_ptr, s_col_idx, s_val, h, C, 0.f, pool, C, s))) return rc;
     if ((rc = product_any(B, C, H, pool, Wh1, nullptr, nullptr, hidden, nullptr, s))) return rc;

@@ -14,7 +14,7 @@
 // so such products are split along k from k = 256:
 // every workgroup takes a range of k, writes its partial tile to scratch, and a second kernel adds the
 // partial tiles in range order (deterministic) and applies alpha and beta.
-#include "gnnhip_internal.h"
+#include "columns.h"
 
 namespace gnnhip {
 namespace {
@@ -265,7 +265,9 @@ __global__ __launch_bounds__(kBlock) void sgemm_skinny_kernel(
 
 // The same product for k <= 256: a lane keeps its four rows of B in registers, the groups stride the rows of A
 // eight at a time (eight 128-bit loads in flight per lane), and groups of up to 16 lanes reduce with DPP.
-template <int NCOL, bool TB>
+// LOOSE: rows of any alignment and length; the row's last lane reads its last four columns (columns.h) and counts only its own
+// (1M rows of 53: 99 us with the tile kernel, 33 here).
+template <int NCOL, bool TB, bool LOOSE>
 __global__ __launch_bounds__(kBlock) void sgemm_skinny_rows_kernel(
     int m, int k, float alpha, const float* __restrict__ A, int lda, const float* __restrict__ B, int ldb,
     float beta, float* C, int ldc, int logG)
@@ -273,8 +275,9 @@ __global__ __launch_bounds__(kBlock) void sgemm_skinny_rows_kernel(
     constexpr int R = 8;
     const int G = 1 << logG;
     const int sub = threadIdx.x & (G - 1);
-    const int kk = sub * 4;
-    const bool live = kk < k;                              // k is a multiple of 4
+    const bool live = sub * 4 < k;
+    const int kk = LOOSE ? ColsLoose::at(sub, k) : sub * 4;
+    const int skip = sub * 4 - kk;                         // columns of the lane before
     float4 b[NCOL];
 #pragma unroll
     for (int j = 0; j < NCOL; ++j) {
@@ -299,7 +302,14 @@ __global__ __launch_bounds__(kBlock) void sgemm_skinny_rows_kernel(
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const long long row = base + r * groups + group;
-            x[r] = (live && row < row1) ? *reinterpret_cast<const float4*>(A + (size_t)row * lda + kk) : f4_zero();
+            if (!LOOSE) {
+                x[r] = (live && row < row1) ? ColsWide::load(A + (size_t)row * lda + kk) : f4_zero();
+            } else {
+                x[r] = (live && row < row1) ? ColsLoose::load(A + (size_t)row * lda + kk) : f4_zero();
+                if (skip > 0) x[r].x = 0.f;
+                if (skip > 1) x[r].y = 0.f;
+                if (skip > 2) x[r].z = 0.f;
+            }
         }
 #pragma unroll
         for (int r = 0; r < R; ++r) {
@@ -323,7 +333,7 @@ __global__ __launch_bounds__(kBlock) void sgemm_skinny_rows_kernel(
 }
 
 template <int NCOL>
-void launch_skinny(bool tb, int m, int k, float alpha, const float* A, int lda, const float* B, int ldb,
+void launch_skinny(bool tb, bool loose, int m, int k, float alpha, const float* A, int lda, const float* B, int ldb,
                    float beta, float* C, int ldc, hipStream_t s)
 {
     int logG = 0;
@@ -334,8 +344,9 @@ void launch_skinny(bool tb, int m, int k, float alpha, const float* A, int lda, 
         if (blocks > (size_t)kNumCU * 32) blocks = (size_t)kNumCU * 32;
         if (blocks < 1) blocks = 1;
         const unsigned grid = (unsigned)blocks;
-        if (tb) hipLaunchKernelGGL((sgemm_skinny_rows_kernel<NCOL, true>), dim3(grid), dim3(kBlock), 0, s, m, k, alpha, A, lda, B, ldb, beta, C, ldc, logG);
-        else hipLaunchKernelGGL((sgemm_skinny_rows_kernel<NCOL, false>), dim3(grid), dim3(kBlock), 0, s, m, k, alpha, A, lda, B, ldb, beta, C, ldc, logG);
+        const auto kernel = loose ? (tb ? sgemm_skinny_rows_kernel<NCOL, true, true> : sgemm_skinny_rows_kernel<NCOL, false, true>)
+                                  : (tb ? sgemm_skinny_rows_kernel<NCOL, true, false> : sgemm_skinny_rows_kernel<NCOL, false, false>);
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBlock), 0, s, m, k, alpha, A, lda, B, ldb, beta, C, ldc, logG);
         return;
     }
     const unsigned grid = ceil_div_u((size_t)m << logG, kBlock);
@@ -416,12 +427,13 @@ int gemm_tn_batch_dispatch(int count, const int* m, const int* n, const int* k, 
 int gemm_dispatch(int transA, int transB, int m, int n, int k, float alpha, const float* A, int lda,
                   const float* B, int ldb, float beta, float* C, int ldc, hipStream_t s)
 {
-    if (!transA && n <= 4 && m >= 4096 && k >= 4 && k % 4 == 0 && lda % 4 == 0 && aligned16(A)) {
+    const bool wide_rows = k % 4 == 0 && lda % 4 == 0 && aligned16(A);
+    if (!transA && n <= 4 && m >= 4096 && k >= 4 && (wide_rows || k <= 4 * kWave)) {
         switch (n) {
-        case 1: launch_skinny<1>(transB, m, k, alpha, A, lda, B, ldb, beta, C, ldc, s); break;
-        case 2: launch_skinny<2>(transB, m, k, alpha, A, lda, B, ldb, beta, C, ldc, s); break;
-        case 3: launch_skinny<3>(transB, m, k, alpha, A, lda, B, ldb, beta, C, ldc, s); break;
-        default: launch_skinny<4>(transB, m, k, alpha, A, lda, B, ldb, beta, C, ldc, s); break;
+        case 1: launch_skinny<1>(transB, !wide_rows, m, k, alpha, A, lda, B, ldb, beta, C, ldc, s); break;
+        case 2: launch_skinny<2>(transB, !wide_rows, m, k, alpha, A, lda, B, ldb, beta, C, ldc, s); break;
+        case 3: launch_skinny<3>(transB, !wide_rows, m, k, alpha, A, lda, B, ldb, beta, C, ldc, s); break;
+        default: launch_skinny<4>(transB, !wide_rows, m, k, alpha, A, lda, B, ldb, beta, C, ldc, s); break;
         }
         GNNHIP_LAUNCH_CHECK("sgemm_skinny");
         return GNNHIP_OK;

@@ -1,13 +1,10 @@
 // Fused structure2vec kernels for gfx950, hidden size C in {16, 32, 64}, and the dispatchers of the
-// three stages (wider hidden sizes: input_wide.hip, level_wide.hip; other sizes: the unfused route in
+// input and level stages (readout: readout.hip; wider hidden sizes: input_wide.hip, level_wide.hip; other sizes: the unfused route in
 // forward.hip):
 //
 //   s2v_input_kernel    msg = X * W_n2l ; h0 = ReLU(msg)
 //   s2v_level_kernel    h_out = ReLU((A * h_in) * W + bias + msg), with 64-bit addressing: the kernel for
 //                       activations of 4 GiB and more (smaller ones take level_stream.hip)
-//   s2v_readout_kernel  pool = S * h ; hidden = ReLU(pool * W_h1) ;
-//                       logits = hidden * W_h2 ; probs = softmax(logits) ; pred = argmax,
-//                       one workgroup per graph (many graphs: readout.hip)
 //
 // A level reads h_in (gathered), msg and the CSR arrays once and writes h_out
 // once: 4(N+1) + 8E + 12NC + 4C^2 algorithmic bytes, against roughly nine
@@ -429,96 +426,6 @@ __global__ __launch_bounds__(kBlock) void s2v_level_kernel(
     }
 }
 
-// ---------------------------------------------------------------- readout, one workgroup per subgraph
-// LDS: part[P][C] | pool[C] | hid[H] | lg[Q]
-template <int C>
-__global__ __launch_bounds__(kBlock) void s2v_readout_kernel(
-    int B, int H, int Q, const int* __restrict__ s_row_ptr, const int* __restrict__ s_col_idx,
-    const float* __restrict__ s_val, const float* __restrict__ h, const float* __restrict__ Wh1,
-    const float* __restrict__ Wh2, float* __restrict__ pool, float* __restrict__ hidden,
-    float* __restrict__ logits, float* __restrict__ probs, int* __restrict__ pred)
-{
-    constexpr int G = C / 4, P = kBlock / G;
-    extern __shared__ float smem[];
-    float* part = smem;
-    float* pl = part + P * C;
-    float* hid = pl + C;
-    float* lg = hid + H;
-    const int tid = threadIdx.x, tx = tid % G, ty = tid / G;
-
-    for (int g = blockIdx.x; g < B; g += gridDim.x) {
-        const int start = s_row_ptr[g], end = s_row_ptr[g + 1];
-        // sum-pool: group ty takes entries start+ty, start+ty+P, ...
-        float4 acc = f4_zero();
-        int t = start + ty;
-        for (; t + P < end; t += 2 * P) {
-            const int c0 = s_col_idx[t], c1 = s_col_idx[t + P];
-            const float v0 = s_val[t], v1 = s_val[t + P];
-            const float4 x0 = *reinterpret_cast<const float4*>(h + (size_t)c0 * C + tx * 4);
-            const float4 x1 = *reinterpret_cast<const float4*>(h + (size_t)c1 * C + tx * 4);
-            f4_fma(acc, v0, x0);
-            f4_fma(acc, v1, x1);
-        }
-        if (t < end) f4_fma(acc, s_val[t], *reinterpret_cast<const float4*>(h + (size_t)s_col_idx[t] * C + tx * 4));
-        *reinterpret_cast<float4*>(part + (size_t)ty * C + tx * 4) = acc;
-        __syncthreads();
-        if (tid < C) {
-            float s = 0.f;
-            for (int p = 0; p < P; ++p) s += part[(size_t)p * C + tid];
-            pl[tid] = s;
-            pool[(size_t)g * C + tid] = s;
-        }
-        __syncthreads();
-        // hidden = ReLU(pool * W_h1)
-        for (int j = tid; j < H; j += kBlock) {
-            float s = 0.f;
-#pragma unroll 16
-            for (int c = 0; c < C; ++c) s += pl[c] * Wh1[(size_t)c * H + j];
-            s = relu_ref(s);
-            hid[j] = s;
-            hidden[(size_t)g * H + j] = s;
-        }
-        __syncthreads();
-        // logits = hidden * W_h2
-        for (int q = tid; q < Q; q += kBlock) {
-            float s = 0.f;
-#pragma unroll 8
-            for (int j = 0; j < H; ++j) s += hid[j] * Wh2[(size_t)j * Q + q];
-            lg[q] = s;
-            logits[(size_t)g * Q + q] = s;
-        }
-        __syncthreads();
-        // softmax + argmax over Q by the first wavefront
-        if (tid < kWave) {
-            const float first = lg[0];
-            float mx = first;                       // reference scan starts at element 0
-            float bv = -INFINITY;
-            int bi = 0x7fffffff;
-            for (int q = tid; q < Q; q += kWave) {
-                const float v = lg[q];
-                mx = max_keep(mx, v);
-                const float vv = (v != v) ? -INFINITY : v;     // a NaN that is not first never wins
-                argmax_combine(bv, bi, vv, q);
-            }
-            mx = wave_max(mx);
-            wave_argmax(bv, bi);
-            if (first != first) bi = 0;            // NaN in column 0 is never displaced
-            if (pred && tid == 0) pred[g] = bi;
-            if (probs) {
-                float s = 0.f;
-                for (int q = tid; q < Q; q += kWave) {
-                    const float e = expf(lg[q] - mx);
-                    lg[q] = e;
-                    s += e;
-                }
-                s = wave_sum(s);
-                for (int q = tid; q < Q; q += kWave) probs[(size_t)g * Q + q] = lg[q] / s;
-            }
-        }
-        __syncthreads();
-    }
-}
-
 // Mean entries per row from which the two-launch route is taken.
 inline long long two_step_degree() { return (long long)kTwoStepMeanDegree; }
 
@@ -547,21 +454,6 @@ int launch_level(int N, const int* row_ptr, const int* col_idx, const float* val
     hipLaunchKernelGGL((s2v_level_kernel<C, DENSE>), dim3((unsigned)blocks), dim3(kBlock), 0, s,
                        N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs);
     GNNHIP_LAUNCH_CHECK("s2v_level");
-    return GNNHIP_OK;
-}
-
-template <int C>
-int launch_readout(int B, int H, int Q, const int* s_row_ptr, const int* s_col_idx, const float* s_val,
-                   const float* h, const float* Wh1, const float* Wh2, float* pool, float* hidden,
-                   float* logits, float* probs, int* pred, hipStream_t s)
-{
-    constexpr int P = kBlock / (C / 4);
-    const size_t smem = sizeof(float) * ((size_t)P * C + C + (size_t)H + (size_t)Q);
-    if (smem > 64 * 1024) return GNNHIP_EUNSUPPORTED;
-    const int grid = B < kNumCU * 8 ? B : kNumCU * 8;
-    hipLaunchKernelGGL((s2v_readout_kernel<C>), dim3(grid), dim3(kBlock), smem, s,
-                       B, H, Q, s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2, pool, hidden, logits, probs, pred);
-    GNNHIP_LAUNCH_CHECK("s2v_readout");
     return GNNHIP_OK;
 }
 
@@ -708,21 +600,6 @@ int level_backward_dispatch(int N, int C, long long nnz, const int* row_ptr, con
     HubPlan hubs{};
     if (int rc = hub_prepass(N, C, nnz, row_ptr, col_idx, val, dz, C, s, &hubs, false, false)) return rc;
     return level_stream_backward_dispatch(N, C, row_ptr, col_idx, val, dz, W, u, g_prev, gate, acc, hubs, s);
-}
-
-int readout_dispatch(int B, int C, int H, int Q, const int* s_row_ptr, const int* s_col_idx, const float* s_val,
-                     const float* h, const float* Wh1, const float* Wh2, float* pool, float* hidden,
-                     float* logits, float* probs, int* pred, hipStream_t s)
-{
-    if (!aligned16(h)) return GNNHIP_EUNSUPPORTED;
-    switch (C) {
-    case 16: return launch_readout<16>(B, H, Q, s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2, pool, hidden, logits, probs, pred, s);
-    case 32: return launch_readout<32>(B, H, Q, s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2, pool, hidden, logits, probs, pred, s);
-    case 64: return launch_readout<64>(B, H, Q, s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2, pool, hidden, logits, probs, pred, s);
-    case 128: return launch_readout<128>(B, H, Q, s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2, pool, hidden, logits, probs, pred, s);
-    case 256: return launch_readout<256>(B, H, Q, s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2, pool, hidden, logits, probs, pred, s);
-    }
-    return GNNHIP_EUNSUPPORTED;
 }
 
 }  // namespace gnnhip

@@ -17,15 +17,13 @@
 //      the blocks of the last, uneven round row by row of blocks was tried: the extra loads of W cost more (179 -> 214 us at
 //      390,000 nodes, hidden 85);
 //   3. the product goes back through the same LDS, rows packed at their own width, so that what follows (msg, gate, sums,
-//      ReLU, stores) walks flat 16-byte words of memory whatever the width: the R rows of a tile are contiguous, and R times
-//      any width is a multiple of four.
+//      ReLU, stores) walks flat words of four floats whatever the width: the R rows of a tile are contiguous.
 // Sums have the order of the row-group SpMM and of the GEMM tile kernel, so every bit is theirs.
 //
 // Rows of more than kHubThreshold entries come from the balanced pass (hub.hip) where it runs, as in the SpMM; elsewhere rows
 // longer than kLongRow are summed by the whole workgroup.
 #include "columns.h"
 #include "buffer_addr.h"
-#include <initializer_list>
 
 namespace gnnhip {
 namespace {
@@ -251,14 +249,14 @@ __global__ __launch_bounds__(kBlock, 3) void s2v_rows_kernel(RowsArgs a)
     const int total = rows * n;
     auto load = [&](const float* p, int i) {
         float4 v = f4_zero();
-        if (i + 4 <= total) return *reinterpret_cast<const float4*>(p + flat0 + i);
+        if (i + 4 <= total) return V::load(p + flat0 + i);
         if (i < total) v.x = p[flat0 + i];
         if (i + 1 < total) v.y = p[flat0 + i + 1];
         if (i + 2 < total) v.z = p[flat0 + i + 2];
         return v;
     };
     auto store = [&](float* p, int i, const float4& v) {
-        if (i + 4 <= total) { *reinterpret_cast<float4*>(p + flat0 + i) = v; return; }
+        if (i + 4 <= total) { V::store(p + flat0 + i, v); return; }
         p[flat0 + i] = v.x;
         if (i + 1 < total) p[flat0 + i + 1] = v.y;
         if (i + 2 < total) p[flat0 + i + 2] = v.z;
@@ -316,13 +314,6 @@ int rows_dispatch(RowsArgs a, hipStream_t s)
     return few ? launch_rows<1, 4, GATHER, WT>(a, s) : launch_rows<2, 4, GATHER, WT>(a, s);
 }
 
-inline bool all_aligned(std::initializer_list<const void*> ps)
-{
-    for (const void* p : ps)
-        if (!aligned16(p)) return false;
-    return true;
-}
-
 }  // namespace
 
 namespace {
@@ -340,7 +331,7 @@ int level_rows_dispatch(int N, int C, long long nnz, const int* row_ptr, const i
                         const float* W, const float* msg, const float* bias, float* h_out, bool same_graph, bool relu_in, CsrPlan* plan,
                         hipStream_t s)
 {
-    if (!level_rows_covers(N, C, nnz) || !all_aligned({msg, h_out})) return GNNHIP_EUNSUPPORTED;
+    if (!level_rows_covers(N, C, nnz)) return GNNHIP_EUNSUPPORTED;
     RowsArgs a{};
     if (int rc = hub_prepass(N, C, nnz, row_ptr, col_idx, val, h_in, C, s, &a.hubs, same_graph, relu_in, kHubThreshold, kHubChunk, -1,
                              plan ? &plan->row_hub : nullptr))
@@ -354,7 +345,7 @@ int level_rows_dispatch(int N, int C, long long nnz, const int* row_ptr, const i
 int level_rows_backward_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* dz,
                                  const float* W, float* u, float* g_prev, const float* gate, float* acc, hipStream_t s)
 {
-    if (!level_rows_covers(N, C, nnz) || !all_aligned({g_prev, gate, acc})) return GNNHIP_EUNSUPPORTED;
+    if (!level_rows_covers(N, C, nnz)) return GNNHIP_EUNSUPPORTED;
     RowsArgs a{};
     if (int rc = hub_prepass(N, C, nnz, row_ptr, col_idx, val, dz, C, s, &a.hubs)) return rc;
     a.N = N; a.K = C; a.n = C;
@@ -368,7 +359,7 @@ int level_rows_dense_dispatch(int N, int K, int n, const float* x, const float* 
                               bool relu, float* relu_out, hipStream_t s)
 {
     // (64 rows of more than 252 columns would not fit 64 KB of LDS)
-    if (K < 1 || K > (n <= 128 ? 128 : kMaxWidth) || n > kMaxWidth || !all_aligned({msg, out, relu_out})) return GNNHIP_EUNSUPPORTED;
+    if (K < 1 || K > (n <= 128 ? 128 : kMaxWidth) || n > kMaxWidth) return GNNHIP_EUNSUPPORTED;
     RowsArgs a{};
     a.N = N; a.K = K; a.n = n;
     a.x = x; a.W = W; a.bias = bias; a.msg = msg; a.out = out; a.relu = relu; a.relu_out = relu_out;

@@ -14,7 +14,7 @@
 //   3. logits the same way over the hidden units, then softmax and arg-max inside the wavefront.
 // Hidden sizes 16, 32 and 64 (at 256 the weights fill LDS, one workgroup per CU remains, and SpMM + GEMM
 // are faster: 140 against 204 us for 10,000 graphs).  Algorithmic bytes: 4NC (h) + 8N (S) + 4B(C + H + 2Q) + 4(CH + HQ).
-#include "gnnhip_internal.h"
+#include "columns.h"
 #include <math.h>
 #include <type_traits>
 
@@ -307,6 +307,147 @@ int launch_readout_tile(int B, int H, int Q, const int* s_row_ptr, const int* s_
     return GNNHIP_OK;
 }
 
+// Readout for any hidden size up to 256 and any number of graphs: TG graphs per workgroup of BLOCK lanes, a quarter of it (one
+// wavefront) or all of it per graph.
+//   1. sum-pool   groups of G lanes (a power of two, 4 G >= C) take the graph's rows in turn, eight in flight each; the sums of a
+//                 wavefront's groups are added by shuffles, those of the graph's wavefronts in order through LDS;
+//   2. hidden     each wavefront of the graph adds up its share of the columns of W_h1, a lane per unit;
+//   3. logits     a wavefront per class, lanes over the hidden units;
+//   4. softmax and arg-max by the graph's first wavefront.
+// Bound by memory where graphs are large (what is in flight decides: 301 graphs of 1,000 nodes, hidden 32: 17 us with two rows
+// in flight per group of a 256-lane workgroup, 12 with eight of a 512-lane one, 18 with
+// 1,024 lanes, which leave 45 of the workgroups to a second turn), by the chain of its four steps where they are
+// small.  Hidden sizes without another readout took six launches (1,500 graphs of 32 nodes, hidden 100: 35 us).
+template <int TG, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void s2v_readout_rows_kernel(
+    int B, int C, int H, int Q, const int* __restrict__ s_row_ptr, const int* __restrict__ s_col_idx, const float* __restrict__ s_val,
+    const float* __restrict__ h, const float* __restrict__ Wh1, const float* __restrict__ Wh2, float* __restrict__ pool,
+    float* __restrict__ hidden, float* __restrict__ logits, float* __restrict__ probs, int* __restrict__ pred)
+{
+    using V = ColsLoose;
+    constexpr int LG = BLOCK / TG, WG = LG / kWave;      // lanes and wavefronts per graph
+    constexpr int kFlight = 8;
+    const int units = (C + 3) / 4, C4 = 4 * units;
+    const int logG = units <= 1 ? 0 : 32 - __builtin_clz((unsigned)(units - 1));
+    const int G = 1 << logG;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int k = tid / LG, w = (tid % LG) / kWave;      // graph of the tile, wavefront of the graph
+    const int sub = lane & (G - 1), grp = (tid % LG) >> logG, ngroups = LG >> logG;
+    const bool live = sub < units;
+    const int col0 = V::at(sub, C);
+    extern __shared__ float4 smem4[];
+    float* part = reinterpret_cast<float*>(smem4) + (size_t)k * WG * C4;                     // [WG][C4], a unit's columns at 4 unit
+    float* pl = reinterpret_cast<float*>(smem4) + (size_t)TG * WG * C4 + (size_t)k * C4;     // [C]
+    float* ph = reinterpret_cast<float*>(smem4) + (size_t)TG * (WG + 1) * C4 + (size_t)k * (WG * H + H + Q);
+    float* hid = ph + WG * H;                            // ph: [WG][H]
+    float* lg = hid + H;
+
+    for (long long tile = blockIdx.x; tile * TG < B; tile += gridDim.x) {
+        const long long g = tile * TG + k;
+        const bool own = g < B;
+        const int start = own ? s_row_ptr[g] : 0, end = own ? s_row_ptr[g + 1] : 0;
+        float4 acc = f4_zero();
+        for (int t = start + grp; t < end; t += kFlight * ngroups) {
+            int c[kFlight];
+            float v[kFlight];
+            float4 x[kFlight];
+#pragma unroll
+            for (int u = 0; u < kFlight; ++u) {
+                const bool ok = t + u * ngroups < end;
+                c[u] = ok ? s_col_idx[t + u * ngroups] : 0;
+                v[u] = ok ? s_val[t + u * ngroups] : 0.f;
+            }
+#pragma unroll
+            for (int u = 0; u < kFlight; ++u) x[u] = live && t + u * ngroups < end ? V::load(h + (size_t)c[u] * C + col0) : f4_zero();
+#pragma unroll
+            for (int u = 0; u < kFlight; ++u)
+                if (t + u * ngroups < end) f4_fma(acc, v[u], x[u]);
+        }
+        for (int d = G; d < kWave; d <<= 1)
+            acc = V::add(acc, make_float4(__shfl_xor(acc.x, d, kWave), __shfl_xor(acc.y, d, kWave), __shfl_xor(acc.z, d, kWave), __shfl_xor(acc.w, d, kWave)));
+        if (lane < units) *reinterpret_cast<float4*>(part + w * C4 + 4 * lane) = acc;
+        __syncthreads();
+        if (w == 0 && lane < units) {
+            float4 s = *reinterpret_cast<const float4*>(part + 4 * lane);
+#pragma unroll
+            for (int i = 1; i < WG; ++i) s = V::add(s, *reinterpret_cast<const float4*>(part + i * C4 + 4 * lane));
+            V::store(pl + V::at(lane, C), s);
+            if (own) V::store(pool + (size_t)g * C + V::at(lane, C), s);
+        }
+        __syncthreads();
+        // ---- hidden = ReLU(pool * W_h1)
+        const int share = (C + WG - 1) / WG, c_lo = min(w * share, C), c_hi = min(c_lo + share, C);
+        for (int j = lane; j < H; j += kWave) {
+            float s = 0.f;
+#pragma unroll 16
+            for (int c = c_lo; c < c_hi; ++c) s = fmaf(pl[c], Wh1[(size_t)c * H + j], s);
+            ph[w * H + j] = s;
+        }
+        __syncthreads();
+        for (int j = tid % LG; j < H; j += LG) {
+            float s = ph[j];
+#pragma unroll
+            for (int i = 1; i < WG; ++i) s += ph[i * H + j];
+            s = relu_ref(s);
+            hid[j] = s;
+            if (own) hidden[(size_t)g * H + j] = s;
+        }
+        __syncthreads();
+        // ---- logits = hidden * W_h2
+        for (int q = w; q < Q; q += WG) {
+            float s = 0.f;
+            for (int j = lane; j < H; j += kWave) s = fmaf(hid[j], Wh2[(size_t)j * Q + q], s);
+            s = wave_sum(s);
+            if (lane == 0) {
+                lg[q] = s;
+                if (own) logits[(size_t)g * Q + q] = s;
+            }
+        }
+        __syncthreads();
+        // ---- softmax + argmax over Q
+        if (w == 0 && own && (probs || pred)) {
+            const float first = lg[0];
+            float mx = first;                       // the reference scan starts at element 0
+            float bv = -INFINITY;
+            int bi = 0x7fffffff;
+            for (int q = lane; q < Q; q += kWave) {
+                const float v = lg[q];
+                mx = max_keep(mx, v);
+                argmax_combine(bv, bi, (v != v) ? -INFINITY : v, q);     // a NaN that is not first never wins
+            }
+            mx = wave_max(mx);
+            wave_argmax(bv, bi);
+            if (first != first) bi = 0;             // a NaN in column 0 is never displaced
+            if (pred && lane == 0) pred[g] = bi;
+            if (probs) {
+                float s = 0.f;
+                for (int q = lane; q < Q; q += kWave) {
+                    const float e = expf(lg[q] - mx);
+                    lg[q] = e;
+                    s += e;
+                }
+                s = wave_sum(s);
+                for (int q = lane; q < Q; q += kWave) probs[(size_t)g * Q + q] = lg[q] / s;
+            }
+        }
+        __syncthreads();                            // LDS is reused by the next tile
+    }
+}
+
+template <int TG, int BLOCK>
+int launch_readout_rows(int B, int C, int H, int Q, const int* s_row_ptr, const int* s_col_idx, const float* s_val, const float* h,
+                        const float* Wh1, const float* Wh2, float* pool, float* hidden, float* logits, float* probs, int* pred, hipStream_t s)
+{
+    constexpr int WG = BLOCK / TG / kWave;
+    const size_t smem = sizeof(float) * TG * ((size_t)(WG + 1) * ((C + 3) / 4 * 4) + (size_t)(WG + 1) * H + Q);
+    if (smem > 64 * 1024) return GNNHIP_EUNSUPPORTED;
+    const int tiles = (B + TG - 1) / TG, most = kNumCU * (2048 / BLOCK);
+    hipLaunchKernelGGL((s2v_readout_rows_kernel<TG, BLOCK>), dim3((unsigned)(tiles < most ? tiles : most)), dim3(BLOCK), smem, s, B, C, H, Q,
+                       s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2, pool, hidden, logits, probs, pred);
+    GNNHIP_LAUNCH_CHECK("s2v_readout_rows");
+    return GNNHIP_OK;
+}
+
 }  // namespace
 
 // A workgroup per tile of graphs, hidden sizes 128 and 256; for batches of thousands of small graphs (the caller decides).
@@ -339,6 +480,23 @@ int readout_wave_dispatch(int B, int C, int H, int Q, const int* s_row_ptr, cons
     }
 #undef GNNHIP_RO_ARGS
     return GNNHIP_EUNSUPPORTED;
+}
+
+// Any hidden size of 4 .. 256.
+int readout_rows_dispatch(int B, int N, int C, int H, int Q, const int* s_row_ptr, const int* s_col_idx, const float* s_val, const float* h,
+                          const float* Wh1, const float* Wh2, float* pool, float* hidden, float* logits, float* probs, int* pred, hipStream_t s)
+{
+    if (C < 4 || C > 256) return GNNHIP_EUNSUPPORTED;
+#define GNNHIP_RO_ARGS B, C, H, Q, s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2, pool, hidden, logits, probs, pred, s
+    // Many small graphs: a wavefront each (4,000 graphs of 32 nodes, hidden 100: 22 us, with a workgroup each 29; 1,500 of them:
+    // 16.6 against 15.6).  Graphs of hundreds of rows: 512 lanes each.
+    const long long mean = (long long)N / B;
+    int rc = GNNHIP_EUNSUPPORTED;
+    if (B >= 8 * kNumCU && mean <= 256) rc = launch_readout_rows<4, kBlock>(GNNHIP_RO_ARGS);
+    else if (mean > 256) rc = launch_readout_rows<1, 512>(GNNHIP_RO_ARGS);
+    if (rc == GNNHIP_EUNSUPPORTED) rc = launch_readout_rows<1, kBlock>(GNNHIP_RO_ARGS);
+    return rc;
+#undef GNNHIP_RO_ARGS
 }
 
 }  // namespace gnnhip

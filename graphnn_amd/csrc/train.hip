@@ -9,7 +9,7 @@
 //   parameter update         momentum SGD over every tensor of a parameter set in one launch
 //
 // All of them are launch- or HBM-bound; the dense products of the backward pass stay with gemm.hip / spmm.hip.
-#include "gnnhip_internal.h"
+#include "columns.h"
 
 namespace gnnhip {
 // gemm.hip
@@ -192,27 +192,26 @@ __global__ __launch_bounds__(kBlock) void grad_gate_kernel(size_t n, const float
     }
 }
 
-// The same for 16-byte aligned tensors in 128-bit words, n4 of them: two reads and two writes at the copy rate (299,536 x
-// 256: 319 -> 219 us, 1.23 GB).
+// The same in 128-bit words, n4 of them: two reads and two writes at the copy rate (299,536 x 256: 319 -> 219 us, 1.23 GB).
+// The tensors need not be 16-byte aligned (a level of an odd width inside one tensor of all levels).
 template <bool DZ, bool ACC, bool ACCUMULATE>
-__global__ __launch_bounds__(kBlock) void grad_gate4_kernel(size_t n4, const float4* __restrict__ h, const float4* g, float4* dz, float4* acc)
+__global__ __launch_bounds__(kBlock) void grad_gate4_kernel(size_t n4, const float* __restrict__ h, const float* g, float* dz, float* acc)
 {
+    using V = ColsLoose;
     const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
     if (i >= n4) return;
-    const float4 x = h[i], y = g[i];
+    const float4 x = V::load(h + 4 * i), y = V::load(g + 4 * i);
     float4 a = f4_zero();
-    if (ACC && ACCUMULATE) a = acc[i];
+    if (ACC && ACCUMULATE) a = V::load(acc + 4 * i);
     const float4 v = make_float4(x.x > 0.f ? y.x : 0.f, x.y > 0.f ? y.y : 0.f, x.z > 0.f ? y.z : 0.f, x.w > 0.f ? y.w : 0.f);
-    if (DZ) dz[i] = v;
-    if (ACC) acc[i] = ACCUMULATE ? make_float4(a.x + v.x, a.y + v.y, a.z + v.z, a.w + v.w) : v;
+    if (DZ) V::store(dz + 4 * i, v);
+    if (ACC) V::store(acc + 4 * i, ACCUMULATE ? V::add(a, v) : v);
 }
 
 template <bool DZ, bool ACC, bool ACCUMULATE>
 void launch_gate4(size_t n4, const float* h, const float* g, float* dz, float* acc, hipStream_t s)
 {
-    hipLaunchKernelGGL((grad_gate4_kernel<DZ, ACC, ACCUMULATE>), dim3(ceil_div_u(n4, kBlock)), dim3(kBlock), 0, s, n4,
-                       reinterpret_cast<const float4*>(h), reinterpret_cast<const float4*>(g), reinterpret_cast<float4*>(dz),
-                       reinterpret_cast<float4*>(acc));
+    hipLaunchKernelGGL((grad_gate4_kernel<DZ, ACC, ACCUMULATE>), dim3(ceil_div_u(n4, kBlock)), dim3(kBlock), 0, s, n4, h, g, dz, acc);
 }
 
 // ------------------------------------------------------------------ parameter update
@@ -400,7 +399,7 @@ int gnnhip_s2v_grad_gate_f32(size_t n, const float* h, const float* g, float* dz
     GNNHIP_REQUIRE(h && g && (dz || acc), "null tensor in s2v_grad_gate");
     if (int rc = require_ready()) return rc;
     hipStream_t s = as_stream(stream);
-    const size_t n4 = aligned16(h) && aligned16(g) && aligned16(dz) && aligned16(acc) ? n / 4 : 0;        // null counts as aligned
+    const size_t n4 = n / 4;
     if (n4 > 0) {
         if (dz && !acc) launch_gate4<true, false, false>(n4, h, g, dz, acc, s);
         else if (!dz && accumulate) launch_gate4<false, true, true>(n4, h, g, dz, acc, s);

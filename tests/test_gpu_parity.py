@@ -786,6 +786,30 @@ def test_readout_stage_many_graphs(gpu, oracle, C, H, Q, B):
     assert np.array_equal(pred, oracle.row_argmax(logits))      # arg-max of the logits the device produced: exact
 
 
+@pytest.mark.parametrize("C,H,Q,B,hi", [(4, 8, 2, 5, 40), (7, 130, 70, 41, 90), (100, 50, 6, 2051, 9), (255, 20, 3, 2049, 5), (33, 64, 2, 7, 1500), (129, 32, 2, 3, 900)])
+def test_readout_of_any_hidden_size(gpu, oracle, C, H, Q, B, hi):
+    """a wavefront per graph (from 2,048 small ones on, the last tile of four not full), a workgroup of 256 lanes, one of 512
+    for graphs of hundreds of rows; an empty graph, one node, weights other than 1; then the scores of the rows as a product
+    with one column, from 4,096 rows on a kernel of its own at any width"""
+    from graphnn_amd import ops
+    rng = np.random.default_rng(C + B)
+    lens = rng.integers(hi // 2, hi + 1, B); lens[1] = 0; lens[2] = 1
+    rp = np.zeros(B + 1, np.int32); np.cumsum(lens, out=rp[1:])
+    N = int(rp[-1])
+    S = (rp, np.arange(N, dtype=np.int32), (0.5 + rng.random(N)).astype(np.float32))
+    h = np.maximum(rng.standard_normal((N, C)), 0).astype(np.float32)
+    W1 = (rng.standard_normal((C, H)) * 0.2).astype(np.float32); W2 = (rng.standard_normal((H, Q)) * 0.2).astype(np.float32)
+    pool, hidden, logits, probs, pred = (_n(t) for t in ops.s2v_readout(*_csr_t(S, gpu), _t(h, gpu), _t(W1, gpu), _t(W2, gpu), B))
+    w_pool = oracle.spmm(*S, h, B)
+    w_hidden = np.maximum(oracle.gemm(w_pool, W1), 0)
+    w_logits = oracle.gemm(w_hidden, W2)
+    for got, want in ((pool, w_pool), (hidden, w_hidden), (logits, w_logits), (probs, oracle.row_softmax(w_logits))):
+        assert max_rel(got, want) < PARITY_TOL
+    assert np.all(pool[1] == 0) and np.array_equal(pred, oracle.row_argmax(logits))
+    w = rng.standard_normal((C, 1)).astype(np.float32)
+    assert_parity("score", _n(ops.gemm(_t(h, gpu), _t(w, gpu))), *_gemm_want(oracle, h, w))
+
+
 # ------------------------------------------------------------------ whole forward, configurations 1 and 2
 def _forward_case(gpu, oracle, config_id, B=None):
     from graphnn_amd import ops
