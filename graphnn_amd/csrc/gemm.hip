@@ -23,7 +23,8 @@ constexpr int BM = 64, BN = 64, BK = 16, kBlock = 256;
 
 // One 64 x 64 output tile (tile_x, tile_y) over k in [k_lo, k_hi).  part != nullptr: the raw sums go to
 // part[m][n]; otherwise the tile finishes C itself.
-template <bool TA, bool TB>
+// AHEAD: steps whose elements are under way (8 registers each).
+template <bool TA, bool TB, int AHEAD>
 __device__ __forceinline__ void sgemm_tile_body(
     int m, int n, float alpha, const float* __restrict__ A, int lda,
     const float* __restrict__ B, int ldb, float beta, float* C, int ldc, int k_lo, int k_hi, float* __restrict__ part,
@@ -47,10 +48,10 @@ __device__ __forceinline__ void sgemm_tile_body(
 #pragma unroll
     for (int jb = 0; jb < BN / 16; ++jb) acc[jb] = mfma_f4{0.f, 0.f, 0.f, 0.f};
 
-    // each lane moves 4 elements of each tile; the elements of step k0 + BK are requested before the
-    // products of step k0 are formed, so a step costs the longer of the two instead of their sum
-    float ra[4], rb[4];
-    auto fetch = [&](int k0) {
+    // each lane moves 4 elements of each tile; the elements of AHEAD steps on are requested before the
+    // products of a step are formed, so a step costs the longer of the two instead of their sum
+    float ra[AHEAD][4], rb[AHEAD][4];
+    auto fetch = [&](int k0, float (&ra)[4], float (&rb)[4]) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int idx = tid + e * kBlock;        // 0 .. 1023
@@ -77,27 +78,33 @@ __device__ __forceinline__ void sgemm_tile_body(
             }
         }
     };
-    if (k_lo < k_hi) fetch(k_lo);
-    for (int k0 = k_lo; k0 < k_hi; k0 += BK) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int idx = tid + e * kBlock;
-            if (TA) As[idx & (BM - 1)][idx >> 6] = ra[e]; else As[idx >> 4][idx & (BK - 1)] = ra[e];
-            if (TB) Bs[idx >> 4][idx & (BK - 1)] = rb[e]; else Bs[idx & (BN - 1)][idx >> 6] = rb[e];
-        }
-        __syncthreads();
-        if (k0 + BK < k_hi) fetch(k0 + BK);
-        // lane (q, t): k = 4 q + s at instruction s of the step
-        const float4 a = *reinterpret_cast<const float4*>(&As[wave * 16 + t][4 * q]);
+    for (int d = 0; d < AHEAD; ++d) if (d == 0 || k_lo + d * BK < k_hi) fetch(k_lo + d * BK, ra[d], rb[d]);
+    for (int kb = k_lo; kb < k_hi; kb += AHEAD * BK) {
 #pragma unroll
-        for (int jb = 0; jb < BN / 16; ++jb) {
-            const float4 b = *reinterpret_cast<const float4*>(&Bs[jb * 16 + t][4 * q]);
-            acc[jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.x, a.x, acc[jb], 0, 0, 0);
-            acc[jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.y, a.y, acc[jb], 0, 0, 0);
-            acc[jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.z, a.z, acc[jb], 0, 0, 0);
-            acc[jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.w, a.w, acc[jb], 0, 0, 0);
+        for (int d = 0; d < AHEAD; ++d) {
+            const int k0 = kb + d * BK;
+            if (AHEAD > 1 && k0 >= k_hi) break;                // uniform
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int idx = tid + e * kBlock;
+                if (TA) As[idx & (BM - 1)][idx >> 6] = ra[d][e]; else As[idx >> 4][idx & (BK - 1)] = ra[d][e];
+                if (TB) Bs[idx >> 4][idx & (BK - 1)] = rb[d][e]; else Bs[idx & (BN - 1)][idx >> 6] = rb[d][e];
+            }
+            __syncthreads();
+            if (k0 + AHEAD * BK < k_hi) fetch(k0 + AHEAD * BK, ra[d], rb[d]);
+            // lane (q, t): k = 4 q + s at instruction s of the step
+            const float4 a = *reinterpret_cast<const float4*>(&As[wave * 16 + t][4 * q]);
+#pragma unroll
+            for (int jb = 0; jb < BN / 16; ++jb) {
+                const float4 b = *reinterpret_cast<const float4*>(&Bs[jb * 16 + t][4 * q]);
+                acc[jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.x, a.x, acc[jb], 0, 0, 0);
+                acc[jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.y, a.y, acc[jb], 0, 0, 0);
+                acc[jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.z, a.z, acc[jb], 0, 0, 0);
+                acc[jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.w, a.w, acc[jb], 0, 0, 0);
+            }
+            __syncthreads();
         }
-        __syncthreads();
     }
 
     // lane (q, t) holds out[row0 + 16 wave + t][col0 + 16 jb + 4 q + i], i = 0..3
@@ -130,7 +137,7 @@ __global__ __launch_bounds__(kBlock) void sgemm_tile_kernel(
 {
     const int k_lo = partial ? (int)blockIdx.z * k_chunk : 0;
     const int k_hi = partial ? min(k, k_lo + k_chunk) : k;
-    sgemm_tile_body<TA, TB>(m, n, alpha, A, lda, B, ldb, beta, C, ldc, k_lo, k_hi,
+    sgemm_tile_body<TA, TB, 1>(m, n, alpha, A, lda, B, ldb, beta, C, ldc, k_lo, k_hi,
                             partial ? partial + (size_t)blockIdx.z * m * n : nullptr, (int)blockIdx.x, (int)blockIdx.y);
 }
 
@@ -156,7 +163,7 @@ __global__ __launch_bounds__(kBlock) void sgemm_tn_batch_kernel(GemmBatch b)
     if ((long long)blockIdx.x * BM >= m || (int)blockIdx.y * BN >= n) return;
     const int z = (int)blockIdx.z - b.z0[p];
     const int k_lo = z * b.k_chunk[p], k_hi = min(b.k[p], k_lo + b.k_chunk[p]);
-    sgemm_tile_body<true, false>(m, n, 1.0f, b.A[p], b.lda[p], b.B[p], b.ldb[p], 0.0f, b.C[p], b.ldc[p], k_lo, k_hi,
+    sgemm_tile_body<true, false, 4>(m, n, 1.0f, b.A[p], b.lda[p], b.B[p], b.ldb[p], 0.0f, b.C[p], b.ldc[p], k_lo, k_hi,
                                  b.partial[p] + (size_t)z * m * n, (int)blockIdx.x, (int)blockIdx.y);
 }
 
