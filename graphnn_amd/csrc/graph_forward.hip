@@ -324,8 +324,12 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_graph_forward_kernel(
     float* l_sv = reinterpret_cast<float*>(l_rp + n16max + 4);  // [n16max] pooling weights of the graph's rows
     float* hid = l_sv + n16max;                          // [H]
     float* lg = hid + H;                                 // [Q]
-    float* w1s = lg + Q;                                 // W_h1 transposed, [H][C], when staged
-    float* w2s = w1s + (size_t)C * H;                    // W_h2 transposed, [Q][H], when staged
+    // When staged: W_h1 transposed, [H][C], the columns of row j exchanged by j (lanes that write one column of consecutive
+    // rows, as the copy does, would all meet in one bank), and W_h2 as in memory, from 17 classes on transposed, [Q][H].
+    float* w1s = lg + Q;
+    float* w2s = w1s + (size_t)C * H;
+    auto w1_at = [&](int j, int c) { return j * C + (c ^ (j & (C - 1))); };
+    auto w2_at = [&](int j, int q) { return Q <= 16 ? j * Q + q : q * H + j; };
     float* tail = ro_staged ? (w2s + (size_t)H * Q) : w1s;
     tail = smem + ((size_t)(tail - smem) + 3) / 4 * 4;
     int* e_col = reinterpret_cast<int*>(tail);           // [ecap] neighbour index local to the graph
@@ -382,10 +386,10 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_graph_forward_kernel(
         for (int u = 0; u < 4; ++u) { const int i = tid0 + u * kBlock; v1[u] = i < n1 ? Wh1[i] : 0.f; }
         const float v2 = tid0 < n2 ? Wh2[tid0] : 0.f;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) { const int i = tid0 + u * kBlock; if (i < n1) w1s[(i % H) * C + i / H] = v1[u]; }
-        if (tid0 < n2) w2s[(tid0 % Q) * H + tid0 / Q] = v2;
-        for (int i = tid0 + 4 * kBlock; i < n1; i += kBlock) w1s[(i % H) * C + i / H] = Wh1[i];
-        for (int i = tid0 + kBlock; i < n2; i += kBlock) w2s[(i % Q) * H + i / Q] = Wh2[i];
+        for (int u = 0; u < 4; ++u) { const int i = tid0 + u * kBlock; if (i < n1) w1s[w1_at(i % H, i / H)] = v1[u]; }
+        if (tid0 < n2) w2s[w2_at(tid0 / Q, tid0 % Q)] = v2;
+        for (int i = tid0 + 4 * kBlock; i < n1; i += kBlock) w1s[w1_at(i % H, i / H)] = Wh1[i];
+        for (int i = tid0 + kBlock; i < n2; i += kBlock) w2s[w2_at(i / Q, i % Q)] = Wh2[i];
     }
     if (LABELS && wn_in_lds)
         for (int i = tid0; i < K * C; i += kBlock) wn_s[i] = Wn2l[i];
@@ -764,8 +768,8 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_graph_forward_kernel(
                 const int c = lane + u * kWave;
                 if (c < C) {
                     if (ro_staged) {
-                        s0 = fmaf(plv[u], w1s[j * C + c], s0);
-                        if (two) s1 = fmaf(plv[u], w1s[j1 * C + c], s1);
+                        s0 = fmaf(plv[u], w1s[w1_at(j, c)], s0);
+                        if (two) s1 = fmaf(plv[u], w1s[w1_at(j1, c)], s1);
                     } else {
                         s0 = fmaf(plv[u], Wh1[(size_t)c * H + j], s0);
                         if (two) s1 = fmaf(plv[u], Wh1[(size_t)c * H + j1], s1);
@@ -789,7 +793,7 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_graph_forward_kernel(
                 if (lane < Q) {
                     if (ro_staged) {
 #pragma unroll 8
-                        for (int j = 0; j < H; ++j) s = fmaf(hid[j], w2s[lane * H + j], s);
+                        for (int j = 0; j < H; ++j) s = fmaf(hid[j], w2s[j * Q + lane], s);
                     } else {
 #pragma unroll 8
                         for (int j = 0; j < H; ++j) s = fmaf(hid[j], Wh2[(size_t)j * Q + lane], s);
@@ -817,7 +821,7 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_graph_forward_kernel(
             for (int qq = wave; qq < Q; qq += kWavesPerBlock) {
                 float s = 0.f;
                 if (ro_staged) {
-                    for (int j = lane; j < H; j += kWave) s += hid[j] * w2s[qq * H + j];
+                    for (int j = lane; j < H; j += kWave) s += hid[j] * w2s[w2_at(j, qq)];
                 } else {
                     for (int j = lane; j < H; j += kWave) s += hid[j] * Wh2[(size_t)j * Q + qq];
                 }
