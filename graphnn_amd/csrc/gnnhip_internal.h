@@ -280,8 +280,7 @@ int exclusive_scan_i32(int* x, long long n, int* seg_scratch, hipStream_t s);
 int exclusive_scan_pair_i32(int* x, int* y, long long n, int* seg_scratch, hipStream_t s);
 size_t radix_hist_ints(long long n);
 size_t radix_seg_ints(long long n);
-int radix_order_by_digit(const unsigned* keys, long long n, int shift, unsigned* keys_out, unsigned* perm_out, int* hist, int* seg,
-                         hipStream_t s, const unsigned* carried = nullptr);
+int radix_order(unsigned* keys, int bits, long long n, unsigned* keys_out, unsigned* spare, unsigned* order, int* hist, int* seg, hipStream_t s);
 int spmm_plain_dispatch(int m, int k, int n, long long nnz, float alpha, const int* row_ptr, const int* col_idx, const float* val,
                         const float* B, int ldb, float beta, float* C, int ldc, hipStream_t s, bool reuse_plan = false,
                         HubStore* row_hub = nullptr, bool relu_in = false);

@@ -4,14 +4,13 @@
 // workgroup walks touch unrelated rows of B, and a popular row of B is fetched again and again (counted: ten
 // times the size of B).  CSR columns are sorted inside a row, so a run of consecutive entries of a long row
 // covers a narrow range of columns.  This pass cuts every row into pieces of at most kPiece consecutive
-// entries, orders the pieces by the column they start at (two stable radix passes on the top sixteen bits of
+// entries, orders the pieces by the column they start at (radix passes on the top bits of
 // that column), copies the entries into that order, and sums the pieces in that order, each die taking one
 // contiguous eighth of it.  What runs together then starts in the same narrow band of B; measured on R-MAT
 // with 4M rows and 16 entries per row this brings the fetched bytes from 14 GB (pieces in row order) to 8 GB.
 //
-//   plan     pieces per row -> offsets (scan) -> piece records + keys -> order by first column (the second radix
-//            pass carries the first one's order along, the records themselves stay where they are) ->
-//            entries copied in piece order (a CSR matrix whose rows are the pieces)
+//   plan     pieces per row -> offsets (scan) -> piece records + keys -> order by first column (the records themselves
+//            stay where they are) -> entries copied in piece order (a CSR matrix whose rows are the pieces)
 //   sums     one lane group per piece, entries read front to back; a row of one piece (most rows) gets its
 //            result, beta * C included, straight from here
 //   combine  the other rows: the sums are stored by piece id, so the pieces of a row, and of the rows after it, lie
@@ -43,7 +42,7 @@ __device__ __forceinline__ int pieces_of(int deg) { return (deg + kPiece - 1) / 
 // counts[r] = pieces of row r, pcounts[r] = the same for rows of several pieces and 0 for the others (entry m of both
 // is 0, so that the scans leave the totals there).  The host's entry count `cap` sizes every array of the plan; should
 // the matrix hold more entries than that, a row that reaches past entry `cap` (the last rows) is one piece whatever
-// its length: no entries are copied for it, and piece_tail_kernel forms the row's result from the CSR arrays.
+// its length: no entries are copied for it, and piece_tail forms the row's result from the CSR arrays.
 __global__ __launch_bounds__(kBlock) void piece_count_kernel(int m, const int* __restrict__ row_ptr, int cap, int* __restrict__ counts,
                                                              int* __restrict__ pcounts)
 {
@@ -59,19 +58,19 @@ __global__ __launch_bounds__(kBlock) void piece_count_kernel(int m, const int* _
 }
 
 // One lane per piece slot: the row that owns piece id is found by bisection in the scanned counts.
-// Slots at or past the number of pieces get an empty record and the largest key (they sort to the end).
+// Slots at or past the number of pieces get an empty record and the largest key, top (they sort to the end).
 // rec.id: the place of the piece's sum among the partial sums (pfirst[row] + index of the piece in its row) when its row
 // has several pieces, else -1.
 __global__ __launch_bounds__(kBlock) void piece_fill_kernel(int m, long long slots, const int* __restrict__ row_ptr, int cap,
                                                             const int* __restrict__ col_idx, const int* __restrict__ first,
-                                                            const int* __restrict__ pfirst, int shift, PieceRec* __restrict__ rec,
+                                                            const int* __restrict__ pfirst, int shift, unsigned top, PieceRec* __restrict__ rec,
                                                             unsigned* __restrict__ keys)
 {
     const int total = first[m];
     for (long long id = (long long)blockIdx.x * kBlock + threadIdx.x; id < slots; id += (long long)gridDim.x * kBlock) {
         if (id >= total) {
             rec[id] = PieceRec{0, 0, -1, -1};
-            keys[id] = 0xFFFFu;
+            keys[id] = top;
             continue;
         }
         int lo = 0, hi = m;                          // largest row with first[row] <= id
@@ -86,7 +85,7 @@ __global__ __launch_bounds__(kBlock) void piece_fill_kernel(int m, long long slo
         const int end = re <= cap ? min(start + kPiece, re) : start;     // a row past the host's count: an empty stand-in
         const bool alone = first[row + 1] - first[row] == 1;
         rec[id] = PieceRec{start, end, alone ? -1 : pfirst[row] + k, (end > start && alone) ? row : -1};
-        keys[id] = ((unsigned)col_idx[start] >> shift) & 0xFFFFu;
+        keys[id] = ((unsigned)col_idx[start] >> shift) & top;
     }
 }
 
@@ -143,6 +142,60 @@ __global__ __launch_bounds__(kBlock) void piece_gather_kernel(const int* __restr
     }
 }
 
+// The rows that reach past entry `cap` (none when the host's entry count is the matrix's own): such a row has one
+// stand-in piece without entries, so neither the sums nor the combining pass write it; its result,
+// alpha * A[row] * B + beta * C[row], is formed here.  Rows are taken from the last one down, a lane group each;
+// the first row that ends inside the plan ends the walk.
+// The last workgroups of the sums' launch do it (a launch of its own was 4.5 us per product).
+constexpr unsigned kTailGroups = kNumCU;
+struct PieceTail {
+    unsigned first;               // workgroups of the sums ahead of the tail's; all of them when there is no tail
+    int m, cap;
+    const int *row_ptr, *col_idx;
+    const float* val;
+};
+template <class V, int ITERS, bool RELU_IN>
+__device__ __forceinline__ void piece_tail(const PieceTail& tail, int n, float alpha, const float* __restrict__ B, int ldb, float beta,
+                                           float* __restrict__ C, int ldc, int logG)
+{
+    const int m = tail.m, cap = tail.cap;
+    const int* __restrict__ row_ptr = tail.row_ptr;
+    const int* __restrict__ col_idx = tail.col_idx;
+    const float* __restrict__ val = tail.val;
+    const int G = 1 << logG;
+    const int sub = threadIdx.x & (G - 1);
+    const int grp = threadIdx.x >> logG;
+    const int ngroups = kBlock >> logG;
+    for (long long back = (long long)(blockIdx.x - tail.first) * ngroups + grp; back < m; back += (long long)kTailGroups * ngroups) {
+        const int row = m - 1 - (int)back;
+        const int start = row_ptr[row], end = row_ptr[row + 1];
+        if (end <= cap) break;
+        if (start == end) continue;
+        typename V::T acc[ITERS];
+#pragma unroll
+        for (int it = 0; it < ITERS; ++it) acc[it] = V::zero();
+        for (int t = start; t < end; ++t) {
+            const int c = col_idx[t];
+            const float v = alpha * val[t];
+#pragma unroll
+            for (int it = 0; it < ITERS; ++it) {
+                const int unit = sub + it * G;
+                if (unit * V::kVec < n) {
+                    const int col0 = V::at(unit, n);
+                    const typename V::T x = V::load(B + (size_t)c * ldb + col0);
+                    V::fma(acc[it], v, RELU_IN ? V::relu(x) : x);
+                }
+            }
+        }
+#pragma unroll
+        for (int it = 0; it < ITERS; ++it) {
+            const int unit = sub + it * G;
+            if (unit * V::kVec >= n) continue;
+            V::update(C + (size_t)row * ldc, unit, n, acc[it], beta);
+        }
+    }
+}
+
 // One lane group (G lanes) per piece, pieces taken in order; die x (workgroups x, x + 8, ...) walks the
 // x-th eighth of that order front to back, a workgroup taking the next ngroups pieces of its die when the
 // hardware starts it (so the pieces in flight on a die stay close together in the order; a fixed stride per
@@ -156,8 +209,12 @@ template <class V, int ITERS, bool RELU_IN>
 __global__ __launch_bounds__(kBlock) void piece_sum_kernel(
     const int* __restrict__ count, int n, float alpha, const int* __restrict__ at, const int* __restrict__ col_idx, const float* __restrict__ val,
     const float* __restrict__ B, int ldb, float* __restrict__ part, int ldp, int logG, const int* __restrict__ target, float beta,
-    float* __restrict__ C, int ldc)
+    float* __restrict__ C, int ldc, PieceTail tail)
 {
+    if (blockIdx.x >= tail.first) {
+        piece_tail<V, ITERS, RELU_IN>(tail, n, alpha, B, ldb, beta, C, ldc, logG);
+        return;
+    }
     const int G = 1 << logG;
     const int sub = threadIdx.x & (G - 1);
     const int grp = threadIdx.x >> logG;
@@ -210,50 +267,6 @@ __global__ __launch_bounds__(kBlock) void piece_sum_kernel(
             if (unit * V::kVec >= n) continue;
             if (row < 0) V::store(part + (size_t)(-1 - row) * ldp + V::at(unit, n), acc[it]);
             else V::update(C + (size_t)row * ldc, unit, n, acc[it], beta);
-        }
-    }
-}
-
-// The rows that reach past entry `cap` (none when the host's entry count is the matrix's own): such a row has one
-// stand-in piece without entries, so neither the sums nor the combining pass write it; its result,
-// alpha * A[row] * B + beta * C[row], is formed here.  Rows are taken from the last one down, a lane group each;
-// the first row that ends inside the plan ends the walk.
-template <class V, int ITERS, bool RELU_IN>
-__global__ __launch_bounds__(kBlock) void piece_tail_kernel(int m, int n, float alpha, const int* __restrict__ row_ptr, int cap,
-                                                            const int* __restrict__ col_idx, const float* __restrict__ val,
-                                                            const float* __restrict__ B, int ldb, float beta, float* __restrict__ C,
-                                                            int ldc, int logG)
-{
-    const int G = 1 << logG;
-    const int sub = threadIdx.x & (G - 1);
-    const int grp = threadIdx.x >> logG;
-    const int ngroups = kBlock >> logG;
-    for (long long back = (long long)blockIdx.x * ngroups + grp; back < m; back += (long long)gridDim.x * ngroups) {
-        const int row = m - 1 - (int)back;
-        const int start = row_ptr[row], end = row_ptr[row + 1];
-        if (end <= cap) break;
-        if (start == end) continue;
-        typename V::T acc[ITERS];
-#pragma unroll
-        for (int it = 0; it < ITERS; ++it) acc[it] = V::zero();
-        for (int t = start; t < end; ++t) {
-            const int c = col_idx[t];
-            const float v = alpha * val[t];
-#pragma unroll
-            for (int it = 0; it < ITERS; ++it) {
-                const int unit = sub + it * G;
-                if (unit * V::kVec < n) {
-                    const int col0 = V::at(unit, n);
-                    const typename V::T x = V::load(B + (size_t)c * ldb + col0);
-                    V::fma(acc[it], v, RELU_IN ? V::relu(x) : x);
-                }
-            }
-        }
-#pragma unroll
-        for (int it = 0; it < ITERS; ++it) {
-            const int unit = sub + it * G;
-            if (unit * V::kVec >= n) continue;
-            V::update(C + (size_t)row * ldc, unit, n, acc[it], beta);
         }
     }
 }
@@ -447,12 +460,15 @@ int order_pieces(CsrPlan* p, int cap, const Layout& L, char* temp, hipStream_t s
     int* hist = reinterpret_cast<int*>(temp + L.o_hist);
     int bits = 1;
     while (bits < 31 && (1ll << bits) < (long long)p->k) ++bits;
-    const int shift = bits > 16 ? bits - 16 : 0;
+    // Up to 2^20 columns the top eleven bits put pieces within 512 columns of each other, which is as good as sixteen (the sums of
+    // 300,001 columns take the same 44 us) for one pass instead of two (22 us less there); at 4M columns the sums lose 1 %
+    // by it and the passes gain nothing.
+    const int order_bits = bits <= 20 ? 11 : 16;
+    const int shift = bits > order_bits ? bits - order_bits : 0;
     hipLaunchKernelGGL(piece_fill_kernel, dim3(kElemGrid), dim3(kBlock), 0, s, p->m, p->slots, p->row_ptr, cap, p->col_idx, p->first,
-                       p->pfirst, shift, rec, keys);
-    // two stable passes, low digit first: order[i] = id of the piece that comes i-th by the top 16 bits of its first column
-    if (int rc = radix_order_by_digit(keys, p->slots, 0, keys2, perm, hist, seg, s)) return rc;
-    if (int rc = radix_order_by_digit(keys2, p->slots, 8, keys, order, hist, seg, s, perm)) return rc;
+                       p->pfirst, shift, (1u << order_bits) - 1, rec, keys);
+    // order[i] = id of the piece that comes i-th by the top order_bits bits of its first column, equal ones by id
+    if (int rc = radix_order(keys, order_bits, p->slots, keys2, perm, order, hist, seg, s)) return rc;
     hipLaunchKernelGGL(piece_place_kernel, dim3(kElemGrid), dim3(kBlock), 0, s, p->slots, p->pslots, order, rec, ordered, p->at, p->target);
     if (int rc = exclusive_scan_i32(p->at, p->slots + 1, seg, s)) return rc;
     hipLaunchKernelGGL(piece_gather_kernel, dim3(kElemGrid), dim3(kBlock), 0, s, p->first + p->m, ordered, p->at, p->col_idx, p->val,
@@ -480,9 +496,12 @@ int run_pieces(const CsrPlan* p, const Width& w, int n, float alpha, const float
     // workgroups for the bound on the pieces of one die, times the number of dies; those past the real count leave at once
     const int sum_groups = kBlock >> logG;
     const unsigned sgrid = (unsigned)(((p->slots + kNumXCD - 1) / kNumXCD + 1 + sum_groups - 1) / sum_groups) * kNumXCD;
+    // (a plan of its own knows the matrix's count: no tail)
+    const PieceTail tail{sgrid, m, (int)p->nnz, p->row_ptr, p->col_idx, p->val};
+    const unsigned grid_all = sgrid + (p->owned ? 0u : kTailGroups);
 #define GNNHIP_PIECES_LAUNCH(V, I)                                                                                            \
-    hipLaunchKernelGGL((relu_in ? piece_sum_kernel<V, I, true> : piece_sum_kernel<V, I, false>), dim3(sgrid), dim3(kBlock), 0, s, p->first + m, n, alpha, p->at, p->col_ord, p->val_ord, B, \
-                       ldb, part, ldp, logG, p->target, beta, C, ldc)
+    hipLaunchKernelGGL((relu_in ? piece_sum_kernel<V, I, true> : piece_sum_kernel<V, I, false>), dim3(grid_all), dim3(kBlock), 0, s, p->first + m, n, alpha, p->at, p->col_ord, p->val_ord, B, \
+                       ldb, part, ldp, logG, p->target, beta, C, ldc, tail)
     if (w.cols == 4) {
         if (iters <= 1) GNNHIP_PIECES_LAUNCH(ColsWide, 1);
         else if (iters == 2) GNNHIP_PIECES_LAUNCH(ColsWide, 2);
@@ -496,26 +515,6 @@ int run_pieces(const CsrPlan* p, const Width& w, int n, float alpha, const float
     }
 #undef GNNHIP_PIECES_LAUNCH
     GNNHIP_LAUNCH_CHECK("spmm_pieces sums");
-    if (!p->owned) {
-        // rows past the host's entry count, if any (a plan of its own knows the matrix's count)
-        const unsigned tgrid = kNumCU * 4;
-#define GNNHIP_PIECES_TAIL(V, I)                                                                                                   \
-    hipLaunchKernelGGL((relu_in ? piece_tail_kernel<V, I, true> : piece_tail_kernel<V, I, false>), dim3(tgrid), dim3(kBlock), 0, s, m, n, alpha, p->row_ptr, (int)p->nnz, p->col_idx, p->val, \
-                       B, ldb, beta, C, ldc, logG)
-        if (w.cols == 4) {
-            if (iters <= 1) GNNHIP_PIECES_TAIL(ColsWide, 1);
-            else if (iters == 2) GNNHIP_PIECES_TAIL(ColsWide, 2);
-            else GNNHIP_PIECES_TAIL(ColsWide, 4);
-        } else if (w.cols == 3) {
-            if (iters <= 1) GNNHIP_PIECES_TAIL(ColsLoose, 1);
-            else if (iters == 2) GNNHIP_PIECES_TAIL(ColsLoose, 2);
-            else GNNHIP_PIECES_TAIL(ColsLoose, 4);
-        } else {
-            GNNHIP_PIECES_TAIL(ColsOne, 1);
-        }
-#undef GNNHIP_PIECES_TAIL
-        GNNHIP_LAUNCH_CHECK("spmm_pieces tail");
-    }
     // the rows of very many pieces: the balanced pass over long rows, on P times part (P: row pointers pfirst, entry j
     // = column j with weight 1, which that pass takes when it is handed no index and value arrays)
     // (`pslots` stands in for the number of entries of P: an upper bound is all that pass needs; a row of more than

@@ -651,11 +651,10 @@ inline size_t round_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 }  // namespace
 
-// One stable pass of the radix sort: perm_out[i] = index of the key that comes i-th when the n keys are ordered by
-// the 8-bit digit (key >> shift) & 255 of their 16 bits (equal digits keep their input order); keys_out receives the keys in that
-// order.  With `carried`, perm_out[i] = carried[that index] instead (the order of an earlier pass carried along).
-// hist needs radix_hist_ints(n) ints, seg radix_seg_ints(n).
-size_t radix_hist_ints(long long n) { return 256 * (size_t)((n + kTile - 1) / kTile > 0 ? (n + kTile - 1) / kTile : 1); }
+// order[i] = index of the key that comes i-th when n keys of `bits` bits (11: one pass of the radix sort, 16: two) are put in
+// order, equal keys in input order.  keys, keys_out and spare are overwritten.  hist needs radix_hist_ints(n) ints, seg
+// radix_seg_ints(n).
+size_t radix_hist_ints(long long n) { return ((size_t)1 << 11) * (size_t)((n + kTile - 1) / kTile > 0 ? (n + kTile - 1) / kTile : 1); }
 size_t radix_seg_ints(long long n) { return (radix_hist_ints(n) + kScanSeg - 1) / kScanSeg + 1; }
 
 namespace {
@@ -678,19 +677,24 @@ int radix_pass(int count, const GroupJobs& jobs, bool first, long long n, int ro
 
 }  // namespace
 
-int radix_order_by_digit(const unsigned* keys, long long n, int shift, unsigned* keys_out, unsigned* perm_out, int* hist, int* seg,
-                         hipStream_t s, const unsigned* carried)
+int radix_order(unsigned* keys, int bits, long long n, unsigned* keys_out, unsigned* spare, unsigned* order, int* hist, int* seg, hipStream_t s)
 {
     if (n <= 0) return GNNHIP_OK;
     GroupJobs jobs{};
     GroupJob& j = jobs.job[0];
-    j.key = reinterpret_cast<const int*>(keys);                  // 16-bit values: never clamped
+    j.key = reinterpret_cast<const int*>(keys);                  // `bits` bits: never clamped
     j.key_stride = 1;
-    j.k0 = const_cast<unsigned*>(keys);
-    j.v0 = const_cast<unsigned*>(carried);
-    j.k1 = keys_out; j.v1 = perm_out;
+    j.k1 = keys_out;
     j.hist = hist; j.seg = seg;
-    return radix_pass<8>(1, jobs, !carried, n, 1 << 16, shift, s);
+    if (bits <= 11) {
+        j.v1 = order;
+        return radix_pass<11>(1, jobs, true, n, 1 << 11, 0, s);
+    }
+    j.v1 = spare;
+    if (int rc = radix_pass<8>(1, jobs, true, n, 1 << 16, 0, s)) return rc;
+    j.k0 = keys_out; j.v0 = spare;
+    j.k1 = keys; j.v1 = order;
+    return radix_pass<8>(1, jobs, false, n, 1 << 16, 8, s);
 }
 
 // The one-launch grouping where it fits; false: it does not (nothing launched).  With t_row_ptr the same launch
