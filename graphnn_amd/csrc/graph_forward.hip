@@ -72,6 +72,13 @@ struct GraphLds {
         if (labels) f += (label_floats(n16, C, K) + 3) / 4 * 4;
         return f;
     }
+    // Entries of the edge cache with which two workgroups fit a compute unit, where that leaves five per node; else -1.  (Eight
+    // wavefronts of up to 128 registers: the latency chain of one workgroup then runs under the other's.)
+    static int half_edge_cap(int n16, int C, int K, int H, int Q, int block, bool labels)
+    {
+        const long long left = (long long)(kLdsLimit / 2 / sizeof(float)) - (long long)fixed_floats(n16, C, K, H, Q, block, labels);
+        return left >= 10 * n16 ? (int)(left / 2 / 4 * 4) : -1;
+    }
     // entries of the edge cache that still fit under the LDS limit
     static int edge_cap(int n16, int C, int K, int H, int Q, int block, bool labels = false)
     {
@@ -866,16 +873,20 @@ int launch_graph_forward(int B, int K, int H, int Q, int L, int n16max,
                          const int* s_row_ptr, const int* s_col_idx, const float* s_val,
                          const float* X, const float* Wn2l, const float* Wc, const float* Wh1, const float* Wh2,
                          float* msg, float* h_final, float* pool, float* hidden, float* logits, float* probs,
-                         int* pred, int* status, float* h_levels, long long level_stride, bool pack, hipStream_t s)
+                         int* pred, int* status, float* h_levels, long long level_stride, int pack, hipStream_t s)
 {
     constexpr int kBlock = WAVES * kWave;
     constexpr bool LABELS = (KSX == 0);
-    const int ecap = GraphLds::edge_cap(n16max, C, K, H, Q, kBlock, LABELS);
+    int ecap = GraphLds::edge_cap(n16max, C, K, H, Q, kBlock, LABELS);
     if (ecap < 0) return GNNHIP_EUNSUPPORTED;
+    if (WAVES <= 8) {
+        const int half = GraphLds::half_edge_cap(n16max, C, K, H, Q, kBlock, LABELS);
+        if (half >= 0 && half < ecap) ecap = half;
+    }
     const size_t smem = sizeof(float) * (GraphLds::fixed_floats(n16max, C, K, H, Q, kBlock, LABELS) + 2 * (size_t)ecap);
     constexpr bool kKeepBuilt = !LABELS;    // the variant that keeps all levels exists for the dense input only
     // the variant that packs graphs into bins exists for the workgroup shapes bins of 128 nodes and more select
-    constexpr bool kPackBuilt = C <= 64 && ((WAVES == 16) || (C == 16 && WAVES == 8));
+    constexpr bool kPackBuilt = (C == 64 && WAVES == 16) || (C == 32 && WAVES >= 8) || (C == 16 && WAVES == 8);
     const bool keep = h_levels != nullptr;
     if (keep && !kKeepBuilt) return GNNHIP_EUNSUPPORTED;
     if (pack && (!kPackBuilt || keep)) return GNNHIP_EUNSUPPORTED;
@@ -927,7 +938,7 @@ int dispatch_ksx(bool labels, int B, int K, int H, int Q, int L, int n16max,
                  const int* s_row_ptr, const int* s_col_idx, const float* s_val,
                  const float* X, const float* Wn2l, const float* Wc, const float* Wh1, const float* Wh2,
                  float* msg, float* h_final, float* pool, float* hidden, float* logits, float* probs,
-                 int* pred, int* status, float* h_levels, long long level_stride, bool pack, hipStream_t s)
+                 int* pred, int* status, float* h_levels, long long level_stride, int pack, hipStream_t s)
 {
 #define GNNHIP_GF_ARGS B, K, H, Q, L, n16max, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx, s_val, \
                        X, Wn2l, Wc, Wh1, Wh2, msg, h_final, pool, hidden, logits, probs, pred, status, h_levels, level_stride, pack, s
@@ -946,7 +957,7 @@ int dispatch_waves(bool labels, int B, int K, int H, int Q, int L, int n16max,
                    const int* s_row_ptr, const int* s_col_idx, const float* s_val,
                    const float* X, const float* Wn2l, const float* Wc, const float* Wh1, const float* Wh2,
                    float* msg, float* h_final, float* pool, float* hidden, float* logits, float* probs,
-                   int* pred, int* status, float* h_levels, long long level_stride, bool pack, hipStream_t s)
+                   int* pred, int* status, float* h_levels, long long level_stride, int pack, hipStream_t s)
 {
 #define GNNHIP_GF_ARGS B, K, H, Q, L, n16max, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx, s_val, \
                        X, Wn2l, Wc, Wh1, Wh2, msg, h_final, pool, hidden, logits, probs, pred, status, h_levels, level_stride, pack, s
@@ -957,7 +968,7 @@ int dispatch_waves(bool labels, int B, int K, int H, int Q, int L, int n16max,
     } else {
         const int tasks = (C / 16) * (n16max / 16);         // (column block x row tile) tasks of the largest graph
         if (tasks <= 4) return dispatch_ksx<C, 4>(labels, GNNHIP_GF_ARGS);
-        if (tasks <= 8) return dispatch_ksx<C, 8>(labels, GNNHIP_GF_ARGS);
+        if (tasks <= 8 || pack == 2) return dispatch_ksx<C, 8>(labels, GNNHIP_GF_ARGS);
         return dispatch_ksx<C, 16>(labels, GNNHIP_GF_ARGS);
     }
 #undef GNNHIP_GF_ARGS
@@ -998,7 +1009,7 @@ int forward_batched_entry(bool labels, int N, int B, int K, int C, int H, int Q,
     const float* Xf = static_cast<const float*>(X);
     if (h_levels && !aligned16(h_levels)) return set_error(GNNHIP_EUNSUPPORTED, "h_levels must be 16-byte aligned");
     const long long level_stride = (long long)N * C;
-    auto run = [&](int n16v, bool pack) {
+    auto run = [&](int n16v, int pack) {      // pack: 0 graph by graph, 1 bins, 2 bins for workgroups of eight wavefronts
 #define GNNHIP_GF_ARGS labels, B, K, H, Q, L, n16v, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx, s_val, \
                        Xf, W_n2l, W_conv, W_h1, W_h2, msg, h_final, pool, hidden, logits, probs, pred, status, h_levels, level_stride, pack, s
         switch (C) {
@@ -1012,22 +1023,32 @@ int forward_batched_entry(bool labels, int N, int B, int K, int C, int H, int Q,
     int rc = GNNHIP_EUNSUPPORTED;
     // more graphs than compute units: runs of consecutive graphs share a workgroup (bins of at least kPackNodes nodes)
     if (B >= kPackMinGraphs && B <= kBinMaxGraphs && H <= kWave && Q <= kWave && !h_levels) {
-        // Bin size: a workgroup's time grows with its bin (about 6 us + 20 us per 128 nodes), and the bins run in
-        // rounds of one per compute unit, so the size that just avoids another round wins.  The host knows the
-        // totals only: a bin wastes about half a mean graph, and every 64 graphs about half a bin.
-        int best = 0;
+        // Bin size: a workgroup's time grows with its bin and the bins run in rounds of one per compute unit, so the size that
+        // just avoids another round wins.  Hidden 16 and 32 also have workgroups of eight wavefronts, two to a compute unit:
+        // slower alone (1,000 graphs, hidden 32: 28 against 27 us), but a round of theirs takes twice the bins (3,001 graphs:
+        // 53 -> 43 us in one round of bins of 208 nodes).  Times of a round in us, from sweeps of the bin size at 17,000 to
+        // 120,000 nodes.  The host knows the totals only: a bin wastes about half a mean graph, and every 64 graphs about half
+        // a bin.
+        int best = 0, best_pack = 1;
         double best_cost = 0.0;
-        for (int cand = n16 > kPackNodes ? n16 : kPackNodes; cand <= kPackMaxNodes; cand += 16) {
-            if (GraphLds::edge_cap(cand, C, K, H, Q, 1024, labels) < 256) break;
-            const double fill = (double)cand - 0.5 * (double)N / (double)B;
-            const double nbins = (double)N / (fill > 16.0 ? fill : 16.0) + (double)B / 128.0;
-            const double rounds = (double)(long long)((nbins + kNumCU - 1) / kNumCU);
-            const double cost = rounds * (6.0 + 20.0 * cand / 128.0);
-            if (!best || cost < best_cost) { best = cand; best_cost = cost; }
+        for (int pack = C == 16 ? 2 : 1; pack <= (C <= 32 ? 2 : 1); ++pack) {
+            for (int cand = n16 > kPackNodes ? n16 : kPackNodes; cand <= kPackMaxNodes; cand += 16) {
+                const int block = pack == 2 ? 512 : 1024;
+                if (GraphLds::edge_cap(cand, C, K, H, Q, block, labels) < 256) break;
+                const bool two = pack == 2 && GraphLds::half_edge_cap(cand, C, K, H, Q, block, labels) >= 0;
+                if (pack == 2 && C == 32 && !two) break;
+                const int slots = two ? 2 * kNumCU : kNumCU;
+                const double fill = (double)cand - 0.5 * (double)N / (double)B;
+                const double nbins = (double)N / (fill > 16.0 ? fill : 16.0) + (double)B / 128.0;
+                const double rounds = (double)(long long)((nbins + slots - 1) / slots);
+                const double per = cand / 128.0;
+                const double cost = rounds * (C == 64 ? 6.0 + 20.0 * per : pack == 2 ? 11.0 + 14.0 * per : 12.0 + 8.0 * per);
+                if (!best || cost < best_cost) { best = cand; best_cost = cost; best_pack = pack; }
+            }
         }
-        if (best) rc = run(best, true);
+        if (best) rc = run(best, best_pack);
     }
-    if (rc == GNNHIP_EUNSUPPORTED) rc = run(n16, false);
+    if (rc == GNNHIP_EUNSUPPORTED) rc = run(n16, 0);
     if (rc == GNNHIP_EUNSUPPORTED) return set_error(rc, "graph-resident forward could not be configured for this shape");
     return rc;
 }
