@@ -295,6 +295,11 @@ __global__ __launch_bounds__(kBlock) void sgemm_skinny_rows_kernel(
             b[j].z = TB ? B[(size_t)j * ldb + kk + 2] : B[(size_t)(kk + 2) * ldb + j];
             b[j].w = TB ? B[(size_t)j * ldb + kk + 3] : B[(size_t)(kk + 3) * ldb + j];
         }
+        if (LOOSE) {                                       // both factors of a repeated column are zeros: either may be infinite
+            if (skip > 0) b[j].x = 0.f;
+            if (skip > 1) b[j].y = 0.f;
+            if (skip > 2) b[j].z = 0.f;
+        }
     }
     // A workgroup walks one contiguous run of rows (its groups side by side, R turns ahead), so that what is in flight
     // from one workgroup is one stretch of memory.  All lanes of a wavefront run the same number of iterations (the

@@ -278,6 +278,30 @@ def test_gemm_reference_test_shape(gpu, oracle):
         ops.gemm(_t(A, gpu), _t(B, gpu), False, False)
 
 
+@pytest.mark.parametrize("k", [5, 6, 7, 8, 53, 255, 260])
+@pytest.mark.parametrize("n", [1, 4])
+@pytest.mark.parametrize("side", ["A", "B"])
+def test_gemm_of_few_columns_carries_infinities(gpu, n, k, side):
+    """an infinity in any of the last columns of A, or rows of B, reaches the sums it is a term of, with its sign, and no
+    others: where k is no multiple of four a lane group's last lane reads columns of the lane before it a second time"""
+    from graphnn_amd import ops
+    rng = np.random.default_rng(7 * k + n)
+    m = 4133
+    for tb in (False, True):
+        for at in range(max(0, k - 6), k):
+            A = (0.5 + rng.random((m, k))).astype(np.float32)
+            B = (0.5 + rng.random((k, n))).astype(np.float32)
+            want = A.astype(np.float64) @ B
+            if side == "A":
+                A[17, at], want[17] = -np.inf, -np.inf
+            else:
+                B[at, n - 1], want[:, n - 1] = np.inf, np.inf
+            got = _n(ops.gemm(_t(A, gpu), _t(np.ascontiguousarray(B.T) if tb else B, gpu), False, tb))
+            finite = np.isfinite(want)
+            assert np.array_equal(got[~finite], want[~finite]), (tb, at)
+            assert np.allclose(got[finite], want[finite], rtol=1e-5, atol=0), (tb, at)     # k <= 260 positive terms: 2^-24 k
+
+
 # ------------------------------------------------------------------ element-wise engine
 EXACT_UNARY = [("set", 0, 3.5, 0.0), ("truncate", 1, -0.5, 0.75), ("scale", 2, -1.75, 0.0), ("add", 3, 0.125, 0.0),
                ("abs", 4, 0, 0), ("relu", 6, 0, 0), ("square", 12, 0, 0)]
