@@ -4,8 +4,9 @@
 // feeding them from Python through ctypes (argument objects, tensor checks and the stream looked up in Python)
 // took longer than running them: 172 us per iteration against 96 us of kernels (50 graphs, hidden 64).  Here an
 // argument is checked and unpacked in C++: a float* or int* parameter takes a contiguous float32 / int32 device
-// tensor, None, or an address as a plain integer; the last parameter, the stream, is the current one.  The
-// functions carry the names of the C entries without `gnnhip_` and raise GnnHipError on a non-zero status.
+// tensor or None and nothing else, except for the few host pointers of the table below, which take an address as a
+// plain integer; the last parameter, the stream, is the current one.  The functions carry the names of the C entries
+// without `gnnhip_` and raise GnnHipError on a non-zero status.
 //
 // The entries are looked up in the library whose path bind() is given, so the module has no link to it.
 #include <Python.h>
@@ -15,6 +16,7 @@
 
 #include <string>
 #include <tuple>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -44,12 +46,15 @@ bool tensor_pointer(PyObject* o, at::ScalarType type, const char* type_name, con
     } else if (o == Py_None) {
         *p = nullptr;
         return true;
-    } else if (PyLong_Check(o)) {
-        *p = PyLong_AsVoidPtr(o);
-        return !PyErr_Occurred();
     }
     PyErr_Format(PyExc_ValueError, "%s must be a contiguous %s CUDA tensor", name, type_name);
     return false;
+}
+
+bool host_pointer(PyObject* o, void** p)
+{
+    *p = o == Py_None ? nullptr : PyLong_AsVoidPtr(o);
+    return !PyErr_Occurred();
 }
 
 template <class T> struct Arg;
@@ -117,18 +122,30 @@ bool current_stream(void** s)
 }
 
 // ---------------------------------------------------------------- one function per entry
-// An entry's parameter names as the C header spells them ("N, C, row_ptr, ..."), for error texts.
+// An entry's parameter names as the C header spells them ("N, C, row_ptr, ..."), for error texts; '@' marks a pointer to
+// host memory.
 std::string nth_name(const char* names, size_t i)
 {
     for (; i > 0 && *names; ++names) i -= *names == ',';
-    while (*names == ' ') ++names;
+    while (*names == ' ' || *names == '@') ++names;
     std::string s;
     for (; *names && *names != ','; ++names) s += *names;
     return s;
 }
 
-template <class Fn> struct Entry;
-template <class... P> struct Entry<int (*)(P...)> {
+// index of the parameter marked '@', or past the last one
+constexpr size_t host_argument(const char* names)
+{
+    size_t i = 0;
+    for (; *names; ++names) {
+        if (*names == '@') return i;
+        i += *names == ',';
+    }
+    return i + 1;
+}
+
+template <class Fn, size_t HOST> struct Entry;
+template <size_t HOST, class... P> struct Entry<int (*)(P...), HOST> {
     typedef int (*Fn)(P...);
     static constexpr size_t kArgs = sizeof...(P) - 1;       // the stream comes last and is not passed
 
@@ -137,15 +154,20 @@ template <class... P> struct Entry<int (*)(P...)> {
     {
         std::tuple<Arg<P>...> a;
         size_t failed = kArgs;
+        auto one = [&](auto& arg, size_t i, const char* name) {
+            if constexpr (std::is_pointer_v<decltype(arg.v)>)
+                if (i == HOST) return host_pointer(args[i], (void**)&arg.v);
+            return arg.take(args[i], name);
+        };
         auto take = [&](auto& arg, size_t i) {
             // the name is only worked out where an argument is refused
-            if (arg.take(args[i], "argument")) return true;
+            if (one(arg, i, "argument")) return true;
             failed = i;
             return false;
         };
         if (!(take(std::get<I>(a), I) && ...)) {
             PyErr_Clear();
-            auto again = [&](auto& arg, size_t i) { return i != failed || arg.take(args[i], nth_name(names, i).c_str()); };
+            auto again = [&](auto& arg, size_t i) { return i != failed || one(arg, i, nth_name(names, i).c_str()); };
             (void)(again(std::get<I>(a), I) && ...);
             return nullptr;
         }
@@ -172,7 +194,7 @@ template <class... P> struct Entry<int (*)(P...)> {
     X(csr_group_i32, "rows, n, key, key_stride, payload, payload_stride, average, row_ptr, col_idx, val")                               \
     X(csr_group_both_i32, "rows, n, x, x_stride, y, y_stride, row_ptr, col_idx, val, t_row_ptr, t_col_idx, t_val")                      \
     X(csr_consecutive_rows_f32, "rows, row_ptr, average, col_idx, val")                                                                 \
-    X(csr_consecutive_rows_host_f32, "rows, offsets, average, row_ptr, col_idx, val")                                                   \
+    X(csr_consecutive_rows_host_f32, "rows, @offsets, average, row_ptr, col_idx, val")                                                   \
     X(csr_transpose_f32, "m, k, nnz, row_ptr, col_idx, val, t_row_ptr, t_col_idx, t_val")                                               \
     X(gemm_f32, "transA, transB, m, n, k, alpha, A, lda, B, ldb, beta, out, ldc")                                                       \
     X(s2v_level_f32, "N, C, nnz, row_ptr, col_idx, val, h_in, W, msg, bias, out")                                                       \
@@ -180,9 +202,9 @@ template <class... P> struct Entry<int (*)(P...)> {
     X(s2v_input_labels_f32, "N, K, C, label, W_n2l, msg, h0, status")                                                                   \
     X(s2v_readout_f32, "B, N, C, H, Q, s_row_ptr, s_col_idx, s_val, h, W_h1, W_h2, pool, hidden, logits, probs, pred")                  \
     X(s2v_forward_f32, "N, B, K, C, H, Q, L, nnz, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx, s_val, X, W_n2l, W_conv, W_h1, "   \
-                       "W_h2, msg, h_a, h_b, pool, hidden, logits, probs, pred, which")                                                 \
+                       "W_h2, msg, h_a, h_b, pool, hidden, logits, probs, pred, @which")                                                 \
     X(s2v_forward_planned_f32, "plan, B, K, C, H, Q, L, s_row_ptr, s_col_idx, s_val, X, W_n2l, W_conv, W_h1, W_h2, msg, h_a, h_b, "     \
-                               "pool, hidden, logits, probs, pred, which")                                                              \
+                               "pool, hidden, logits, probs, pred, @which")                                                              \
     X(s2v_forward_batched_f32, "N, B, K, C, H, Q, L, max_graph_nodes, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx, s_val, X, "    \
                                "W_n2l, W_conv, W_h1, W_h2, msg, h_final, pool, hidden, logits, probs, pred, status")                    \
     X(s2v_forward_batched_train_f32, "N, B, K, C, H, Q, L, max_graph_nodes, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx, s_val, " \
@@ -225,7 +247,7 @@ decltype(&gnnhip_adam_batch_f32) p_adam_batch = nullptr;
 #define GNNHIP_FUNCTION(name, names)                                                                        \
     PyObject* f_##name(PyObject*, PyObject* const* args, Py_ssize_t n)                                      \
     {                                                                                                       \
-        return Entry<decltype(&gnnhip_##name)>::checked(p_##name, #name, names, args, n);                   \
+        return Entry<decltype(&gnnhip_##name), host_argument(names)>::checked(p_##name, #name, names, args, n);                   \
     }
 GNNHIP_ENTRIES(GNNHIP_FUNCTION)
 

@@ -66,6 +66,29 @@ def test_argument_validation_needs_no_gpu():
     assert lib.gnnhip_memset0(None, 0, None) == 0
 
 
+def test_bindings_take_no_integer_for_a_device_tensor():
+    """every float* / int* parameter of the compiled bindings refuses an address (sizes are zero: nothing could be launched);
+    the host pointers, marked @ in the argument lists, are the only ones that take one"""
+    b = binding.load_bindings()
+    text = re.sub(r"/\*.*?\*/", "", open(HEADER).read(), flags=re.S)
+    tried = 0
+    for name, params in re.findall(r"\bint gnnhip_([a-z0-9_]+)\s*\(([^)]*)\)", text):
+        fn = getattr(b, name, None)
+        if fn is None or not fn.__doc__:
+            continue
+        kinds = [p.strip() for p in params.split(",")][:-1]        # the stream is not passed
+        names = [a.strip() for a in fn.__doc__.split(",")]
+        assert len(kinds) == len(names), name
+        args = [None if "*" in k else 0.0 if k.startswith("float") else 0 for k in kinds]
+        for i, (kind, arg) in enumerate(zip(kinds, names)):
+            if not re.match(r"(const )?(float|int)\*", kind) or arg.startswith("@"):
+                continue
+            with pytest.raises(ValueError, match="^%s must be" % arg):
+                fn(*args[:i], 4096, *args[i + 1:])
+            tried += 1
+    assert tried > 200
+
+
 def test_plan_entries_reject_what_is_not_a_plan():
     lib = binding.load_library()
     x = np.zeros(8, np.float32)
