@@ -303,28 +303,39 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_split_kernel(
             // the one after it arrive during this block, so its first batch is asked for after the block)
 
             const unsigned short* src = cur + (q & 1) * kHalf + (rt * 16 + t) * LDT + (q >> 1) * 8;
-            // A piece of the tile operand is read for the next step as soon as this step's products with it are issued:
-            // the pieces are used in the order 3, 2, 1, so that each read has six or more matrix instructions to arrive in.
+            // Two rounds over the contraction steps: first the five products that are corrections, whose sum is about 2^-8 of
+            // the result, then the products of the first pieces.  The result itself is then rounded once per step (KS times)
+            // and not six times: rms error against float64, relative to the sum of the terms' magnitudes, 1e-8 where all six
+            // in one round leave 2.2e-8 to 3.1e-8 and the FP32 matrix cores 2.4e-8 to 2.8e-8 (one sign: 6e-8 against 1.7e-7),
+            // for 5 us more per level (the first pieces of the tile are read twice).  The first round takes the negated
+            // steps first, so the sum changes its sign three times.
+            auto turn = [&]() {
+#pragma unroll
+                for (int jb = 0; jb < NB; ++jb) acc_m[jb] = -acc_m[jb];
+            };
+            auto first_round = [&](int i) { return i < KS / 2 ? i + KS / 4 : i < 3 * KS / 4 ? i - KS / 2 : i; };
+            auto piece = [&](int j, int step) { return *reinterpret_cast<const bf16_words4*>(src + j * kPiece + 16 * step); };
+            // A piece of the tile operand is read for the next step as soon as this step's products with it are issued, so
+            // that each read has six or more matrix instructions to arrive in; the first pieces of the second round's first
+            // three steps take the same registers.
             bool again = false;
             bf16_words4 b[3];
 #pragma unroll
-            for (int j = 2; j >= 0; --j) b[j] = *reinterpret_cast<const bf16_words4*>(src + j * kPiece);
+            for (int j = 2; j >= 0; --j) b[j] = piece(j, first_round(0));
 #pragma unroll
             for (int s = 0; s < KS; ++s) {
-                if (s > 0 && negated(s) != negated(s - 1)) {
-#pragma unroll
-                    for (int jb = 0; jb < NB; ++jb) acc_m[jb] = -acc_m[jb];
-                }
+                const int f = first_round(s);
+                if (s == KS / 2) turn();
                 bf16_words4 w3;
-                if (s < NF) w3 = w_lds[s * kWave];
+                if (f < NF) w3 = w_lds[f * kWave];
 #pragma unroll
                 for (int j = 2; j >= 0; --j) {
 #pragma unroll
-                    for (int i = 2 - j; i >= 0; --i)
+                    for (int i = 2 - j; i >= (j == 0 ? 1 : 0); --i)
 #pragma unroll
                         for (int jb = 0; jb < NB; ++jb)
-                            acc_m[jb] = mfma_bf16(i == 2 && jb == 0 && s < NF ? w3 : wreg[jb][s][i], b[j], acc_m[jb]);
-                    if (s + 1 < KS) b[j] = *reinterpret_cast<const bf16_words4*>(src + j * kPiece + 16 * (s + 1));
+                            acc_m[jb] = mfma_bf16(i == 2 && jb == 0 && f < NF ? w3 : wreg[jb][f][i], b[j], acc_m[jb]);
+                    b[j] = s + 1 < KS ? piece(j, first_round(s + 1)) : piece(0, 2 - j);
                     __builtin_amdgcn_sched_barrier(0);            // keeps the read-ahead where it is written
                 }
                 // the follower's columns are asked for here, behind the first wait for LDS of this block: a
@@ -351,6 +362,15 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_split_kernel(
                     again = ns < nend;
                 }
                 if (s == KS / 2 && again) cShift = load_batch(col_idx, ns, cC);
+            }
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+                if (s > 0 && negated(s) != negated(s - 1)) turn();
+                bf16_words4& a = b[2 - s % 3];
+#pragma unroll
+                for (int jb = 0; jb < NB; ++jb) acc_m[jb] = mfma_bf16(wreg[jb][s][0], a, acc_m[jb]);
+                if (s + 3 < KS) a = piece(0, s + 3);
+                __builtin_amdgcn_sched_barrier(0);
             }
             // One unconditional wait for everything this block asked for (gathered rows, msg).  The loads
             // and their uses sit under separate conditions; without this the compiler has to assume a

@@ -344,6 +344,49 @@ def test_training_iteration_composed_from_the_c_abi(gpu, oracle, config_id, C):
         assert np.allclose(_n(t), want_w, rtol=1e-6, atol=1e-8)
 
 
+def _relative_errors(got, want, terms):
+    """rms and mean of the errors, each against the sum of its terms' magnitudes (float64 tensors)"""
+    e = (got.double() - want) / terms
+    return float(e.square().mean().sqrt()), float(e.mean())
+
+
+@pytest.mark.parametrize("C", [128, 256])
+@pytest.mark.parametrize("N", [5003, 40_009])
+@pytest.mark.parametrize("kind", ["zero_mean", "relu", "one_sign"])
+def test_wide_products_in_pieces_are_no_less_exact_than_fp32_ones(gpu, C, N, kind):
+    """the contraction of the wide inference level and of the wide level backward (bf16 pieces) against float64, next to the FP32
+    matrix cores' (the level of a training forward, a GEMM) on the same operands: the rms of its errors is no larger"""
+    import torch
+    from graphnn_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(C + N)
+    normal = lambda *shape: torch.randn(*shape, generator=gen, device=gpu)
+    A = (torch.arange(N + 1, device=gpu).int(), torch.arange(N, device=gpu).int(), torch.ones(N, device=gpu))     # the identity
+    W = normal(C, C) * (0.8 / C ** 0.5)
+    x = normal(N, C)
+    if kind == "relu":
+        x = x.clamp(min=0)
+    if kind == "one_sign":
+        x, W = x.abs(), W.abs()
+    fp32 = _relative_errors(ops.gemm(x, W, transB=True), x.double() @ W.double().T.contiguous(), x.double().abs() @ W.double().abs().T.contiguous())
+    _, g = ops.s2v_level_backward(*A, x, W)
+    pieces = _relative_errors(g, x.double() @ W.double().T.contiguous(), x.double().abs() @ W.double().abs().T.contiguous())
+    print("backward: pieces rms %.2e mean %.1e, fp32 rms %.2e mean %.1e" % (pieces + fp32))
+    assert pieces[0] <= fp32[0] and abs(pieces[1]) < 0.1 * fp32[0]
+    # forward: msg = x W_n2l, h = ReLU(ReLU(msg) W + msg); the outputs that are not cut off
+    Wn = normal(64, C) * (0.1 if kind != "one_sign" else 0.0) + (0.1 if kind == "one_sign" else 0.0)
+    X = normal(N, 64)
+    S = (torch.tensor([0, N], device=gpu).int(), A[1], A[2])
+    bufs = ops.s2v_forward(A, S, X, Wn, W, normal(C, 4), normal(4, 2), 1)
+    h, msg = bufs.msg.clamp(min=0), bufs.msg
+    want = h.double() @ W.double() + msg.double()
+    terms = h.double() @ W.double().abs() + msg.double().abs()
+    on = want > 0
+    fp32 = _relative_errors(ops.s2v_level(*A, h, W, msg)[on], want[on], terms[on])
+    pieces = _relative_errors(bufs.h_final[on], want[on], terms[on])
+    print("forward: pieces rms %.2e mean %.1e, fp32 rms %.2e mean %.1e" % (pieces + fp32))
+    assert pieces[0] <= fp32[0] and abs(pieces[1]) < 0.1 * fp32[0]
+
+
 @pytest.mark.parametrize("m,n,k", [(256, 256, 8192), (256, 256, 20_011), (255, 33, 40_007), (129, 256, 9_001), (64, 256, 16_385),
                                    (1, 256, 1_048_577), (128, 128, 16_384), (100, 127, 23_456), (65, 64, 65_600), (64, 64, 65_543)])
 def test_weight_gradient_over_a_long_k(gpu, m, n, k):
