@@ -409,6 +409,28 @@ def test_weight_gradient_over_a_long_k(gpu, m, n, k):
     assert torch.equal(batched, got)
 
 
+@pytest.mark.parametrize("m,n,k", [(64, 64, 70_000), (64, 64, 400_003), (64, 128, 40_000), (128, 128, 20_000), (64, 256, 20_000), (128, 256, 20_011),
+                                   (256, 256, 8192), (256, 256, 300_007)])
+@pytest.mark.parametrize("kind", ["zero_mean", "relu", "one_sign"])
+def test_weight_gradient_in_pieces_is_no_less_exact_than_an_fp32_one(gpu, m, n, k, kind):
+    """A^T B over a long k from bf16 pieces against float64, next to the FP32 matrix cores' sum of the same terms (A stored
+    transposed takes the general kernel): the rms of its errors is no larger"""
+    import torch
+    from graphnn_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(m + n + k)
+    A, B = torch.randn(k, m, generator=gen, device=gpu), torch.randn(k, n, generator=gen, device=gpu)
+    if kind == "relu":
+        A = A.clamp(min=0)
+    if kind == "one_sign":
+        A, B = A.abs(), B.abs()
+    At = A.T.contiguous()
+    want, terms = At.double() @ B.double(), At.double().abs() @ B.double().abs()
+    pieces = _relative_errors(ops.gemm(A, B, transA=True), want, terms)
+    fp32 = _relative_errors(ops.gemm(At, B), want, terms)
+    print("%s %dx%d k %d: pieces rms %.2e mean %.1e, fp32 rms %.2e mean %.1e" % ((kind, m, n, k) + pieces + fp32))
+    assert pieces[0] <= fp32[0] and abs(pieces[1]) < 0.1 * fp32[0]
+
+
 def test_weight_gradient_carries_infinities_and_nan(gpu):
     """an infinite or NaN term reaches the outputs it is part of and no others, next to values whose bf16 rounding would overflow"""
     import torch
