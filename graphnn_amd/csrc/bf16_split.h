@@ -52,18 +52,6 @@ __device__ __forceinline__ mfma_f4 mfma_bf16(const bf16_words4& a, const bf16_wo
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-// hi + lo += a b over 32 terms: the largest of the six products in one accumulator, the corrections in the other, so
-// that the large sum is rounded once per instruction of the first kind only
-__device__ __forceinline__ void mfma_split(const bf16_words4 (&a)[3], const bf16_words4 (&b)[3], mfma_f4& hi, mfma_f4& lo)
-{
-    lo = mfma_bf16(a[2], b[0], lo);
-    hi = mfma_bf16(a[0], b[0], hi);
-    lo = mfma_bf16(a[0], b[2], lo);
-    lo = mfma_bf16(a[1], b[1], lo);
-    lo = mfma_bf16(a[1], b[0], lo);
-    lo = mfma_bf16(a[0], b[1], lo);
-}
-
 }  // namespace gnnhip
 
 #endif

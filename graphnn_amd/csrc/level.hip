@@ -47,9 +47,8 @@ int level_wide_dispatch(int N, int C, long long nnz, const int* row_ptr, const i
                         hipStream_t s);
 bool level_wide_covers(int N, int C);
 // level_wide_split.hip
-int level_split_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val,
-                         const float* h_in, const float* W, const float* msg, const float* bias, float* h_out, bool relu_in,
-                         hipStream_t s);
+int level_split_dispatch(int N, int C, const int* row_ptr, const int* col_idx, const float* val, const float* h_in, const float* W,
+                         const float* msg, float* h_out, bool relu_in, hipStream_t s);
 int level_split_backward_dispatch(int N, int C, const int* row_ptr, const int* col_idx, const float* val, const float* dz, const float* W,
                                  float* u, float* g_prev, const float* gate, float* acc, hipStream_t s);
 
@@ -556,7 +555,10 @@ int level_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* c
         }
     }
     if (!level_wide_covers(N, C)) return GNNHIP_EUNSUPPORTED;
-    const auto wide = inference ? level_split_dispatch : level_wide_dispatch;
+    auto wide = [&](long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* h_in, bool relu_in) {
+        return inference && !bias ? level_split_dispatch(N, C, row_ptr, col_idx, val, h_in, W, msg, h_out, relu_in, s)
+                                  : level_wide_dispatch(N, C, nnz, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, relu_in, s);
+    };
     // The wide kernel sums a row of any length inside one wavefront.  Large graphs with many entries per row
     // (in practice the skewed ones, see above) take two steps: the SpMM, which balances long rows, leaves A * h_in
     // in scratch, and the wide kernel reads those rows through the identity matrix (one entry per row: its
@@ -574,9 +576,9 @@ int level_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* c
         hipLaunchKernelGGL(identity_csr_kernel, dim3((unsigned)(((long long)N + kBlock) / kBlock)), dim3(kBlock), 0, s, N, id_row_ptr,
                            id_col, id_val);
         GNNHIP_LAUNCH_CHECK("identity_csr");
-        return wide(N, C, N, id_row_ptr, id_col, id_val, agg, W, msg, bias, h_out, false, s);
+        return wide(N, id_row_ptr, id_col, id_val, agg, false);
     }
-    return wide(N, C, nnz, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, relu_in, s);
+    return wide(nnz, row_ptr, col_idx, val, h_in, relu_in);
 }
 
 // u = A' dz and g_prev = u W^T in one pass (A' = the transposed adjacency in CSR form); GNNHIP_EUNSUPPORTED where

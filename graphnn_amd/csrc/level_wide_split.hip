@@ -1,5 +1,5 @@
 // The wide mean-field level (C = 128 or 256) with its contraction on the bf16 matrix cores:
-//     h_out = ReLU((A * h_in) * W + bias + msg)
+//     h_out = ReLU((A * h_in) * W + msg)
 // (examples/graph_classification/src/kernel_mean_field.cpp:35-42), every product formed from three bf16 pieces of
 // either operand (bf16_split.h: fp32 sums of exact products), and the backward pass of a level through the same
 // machinery.
@@ -48,11 +48,9 @@ template <int C, int WAVES, bool RELU_IN, int TR, bool BWD = false>
 __global__ __launch_bounds__(WAVES * kWave) void s2v_level_split_kernel(
     int N, int tiles_per_block, const int* __restrict__ row_ptr, const int* __restrict__ col_idx,
     const float* __restrict__ val, const float* __restrict__ h_in, const float* __restrict__ W,
-    const float* __restrict__ msg, const float* __restrict__ bias, float* __restrict__ h_out,
-    float* __restrict__ u_out, float* __restrict__ acc_io)
+    const float* __restrict__ msg, float* __restrict__ h_out, float* __restrict__ u_out, float* __restrict__ acc_io)
 {
     constexpr int KS = C / 32;                   // contraction steps
-    constexpr int kWideBlock = WAVES * kWave;
     constexpr int CW = C / WAVES;                // output columns per wavefront
     constexpr int NB = CW / 16;                  // 16-column blocks per wavefront
     constexpr int VEC = C / kWave;               // gathered floats per lane
@@ -76,9 +74,6 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_split_kernel(
     const int col0 = wave * CW;
     const int gather_off = (lane >> 5) * kHalf + (wave * RPW) * LDT + (lane & 31) * VEC;
     const int k_lane = (q & 1) * (C / 2) + (q >> 1) * 8;            // contraction step s of this lane: k = k_lane + 16 s .. + 7
-    float* bias_lds = reinterpret_cast<float*>(tiles + 2 * 3 * kPiece);      // [C], read in the epilogue without a trip to memory
-    if (bias)
-        for (int i = threadIdx.x; i < C; i += kWideBlock) bias_lds[i] = bias[i];
 
     // The matrix instruction rounds its sum towards minus infinity.  The middle half of the contraction steps is formed with
     // -W on the negated sum, so that the drift of one half of the steps cancels that of the other.
@@ -88,7 +83,7 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_split_kernel(
     // W[col0 + 16 jb + t][k_lane + 16 s + 0..7] (buffer loads: one lane offset, the steps as scalar offsets, so no 64-bit
     // address per element is formed)
     bf16_words4 wreg[NB][KS][3];
-    bf16_words4* w_lds = reinterpret_cast<bf16_words4*>(bias_lds + C) + (size_t)wave * NF * kWave + lane;
+    bf16_words4* w_lds = reinterpret_cast<bf16_words4*>(tiles + 2 * 3 * kPiece) + (size_t)wave * NF * kWave + lane;
     {
         const rsrc_t w_rsrc = make_rsrc(W, (unsigned)(C * C * 4));
         const int w_lane_off = BWD ? ((col0 + t) * C + k_lane) * 4 : (k_lane * C + col0 + t) * 4;
@@ -418,10 +413,6 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_split_kernel(
 #pragma unroll
                 for (int jb = 0; jb < NB; ++jb) {
                     float4 v = make_float4(acc_m[jb][0], acc_m[jb][1], acc_m[jb][2], acc_m[jb][3]);
-                    if (bias) {
-                        const float4 b4 = *reinterpret_cast<const float4*>(bias_lds + col0 + 16 * jb + 4 * q);
-                        v.x += b4.x; v.y += b4.y; v.z += b4.z; v.w += b4.w;
-                    }
                     outv[jb] = make_float4(relu_ref(v.x), relu_ref(v.y), relu_ref(v.z), relu_ref(v.w));
                 }
             }
@@ -447,8 +438,7 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_split_kernel(
 
 template <int C, int WAVES, bool RELU_IN, int TR, bool BWD = false>
 int launch_level_split_t(int N, const int* row_ptr, const int* col_idx, const float* val, const float* h_in,
-                      const float* W, const float* msg, const float* bias, float* h_out, hipStream_t s,
-                      float* u_out = nullptr, float* acc_io = nullptr)
+                      const float* W, const float* msg, float* h_out, hipStream_t s, float* u_out = nullptr, float* acc_io = nullptr)
 {
     if ((unsigned long long)N * C * 4ull >= (1ull << 32)) return GNNHIP_EUNSUPPORTED;   // 32-bit buffer offsets
     constexpr int kTileRows = TR;
@@ -458,12 +448,12 @@ int launch_level_split_t(int N, const int* row_ptr, const int* col_idx, const fl
     const long long slots = (long long)kNumCU * kPerCU;
     const long long per = (ntiles + slots - 1) / slots;              // contiguous run of tiles per workgroup
     const long long blocks = (ntiles + per - 1) / per;
-    const size_t smem = 2 * 3 * 2 * sizeof(unsigned short) * kTileRows * (C / 2 + 8) + sizeof(float) * C +
+    const size_t smem = 2 * 3 * 2 * sizeof(unsigned short) * kTileRows * (C / 2 + 8) +
                         sizeof(bf16_words4) * (size_t)wide_lds_fragments<C, BWD>() * WAVES * kWave;
     static LdsLimit lds_limit;                                       // one per kernel instantiation
     GNNHIP_HIP(lds_limit.raise(reinterpret_cast<const void*>(&s2v_level_split_kernel<C, WAVES, RELU_IN, TR, BWD>), smem));
     hipLaunchKernelGGL((s2v_level_split_kernel<C, WAVES, RELU_IN, TR, BWD>), dim3((unsigned)blocks), dim3(WAVES * kWave), smem, s,
-                       N, (int)per, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, u_out, acc_io);
+                       N, (int)per, row_ptr, col_idx, val, h_in, W, msg, h_out, u_out, acc_io);
     GNNHIP_LAUNCH_CHECK(BWD ? "s2v_level_split backward" : "s2v_level_split");
     return GNNHIP_OK;
 }
@@ -472,11 +462,11 @@ int launch_level_split_t(int N, const int* row_ptr, const int* col_idx, const fl
 // twice the workgroups.
 template <int C, int WAVES, bool RELU_IN>
 int launch_level_split(int N, const int* row_ptr, const int* col_idx, const float* val, const float* h_in,
-                      const float* W, const float* msg, const float* bias, float* h_out, hipStream_t s)
+                      const float* W, const float* msg, float* h_out, hipStream_t s)
 {
     constexpr int kSlots = kNumCU * ((C == 128) ? 2 : 1);
-    if (N >= 2 * kSlots * 32) return launch_level_split_t<C, WAVES, RELU_IN, 32>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, s);
-    return launch_level_split_t<C, WAVES, RELU_IN, 16>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, s);
+    if (N >= 2 * kSlots * 32) return launch_level_split_t<C, WAVES, RELU_IN, 32>(N, row_ptr, col_idx, val, h_in, W, msg, h_out, s);
+    return launch_level_split_t<C, WAVES, RELU_IN, 16>(N, row_ptr, col_idx, val, h_in, W, msg, h_out, s);
 }
 
 // The backward pass: same choice of rows per pass.
@@ -485,24 +475,22 @@ int launch_level_split_backward(int N, const int* row_ptr, const int* col_idx, c
                                float* u, float* g_prev, const float* gate, float* acc, hipStream_t s)
 {
     constexpr int kSlots = kNumCU * ((C == 128) ? 2 : 1);
-    if (N >= 2 * kSlots * 32) return launch_level_split_t<C, WAVES, false, 32, true>(N, row_ptr, col_idx, val, dz, W, gate, nullptr, g_prev, s, u, acc);
-    return launch_level_split_t<C, WAVES, false, 16, true>(N, row_ptr, col_idx, val, dz, W, gate, nullptr, g_prev, s, u, acc);
+    if (N >= 2 * kSlots * 32) return launch_level_split_t<C, WAVES, false, 32, true>(N, row_ptr, col_idx, val, dz, W, gate, g_prev, s, u, acc);
+    return launch_level_split_t<C, WAVES, false, 16, true>(N, row_ptr, col_idx, val, dz, W, gate, g_prev, s, u, acc);
 }
 
 }  // namespace
 
-int level_split_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val,
-                        const float* h_in, const float* W, const float* msg, const float* bias, float* h_out, bool relu_in,
-                        hipStream_t s)
+int level_split_dispatch(int N, int C, const int* row_ptr, const int* col_idx, const float* val,
+                        const float* h_in, const float* W, const float* msg, float* h_out, bool relu_in, hipStream_t s)
 {
-    (void)nnz;                                   // the kernel bounds its index reads with row_ptr[N]
     switch (C) {
     case 128:
-        return relu_in ? launch_level_split<128, 8, true>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, s)
-                       : launch_level_split<128, 8, false>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, s);
+        return relu_in ? launch_level_split<128, 8, true>(N, row_ptr, col_idx, val, h_in, W, msg, h_out, s)
+                       : launch_level_split<128, 8, false>(N, row_ptr, col_idx, val, h_in, W, msg, h_out, s);
     case 256:
-        return relu_in ? launch_level_split<256, 8, true>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, s)
-                       : launch_level_split<256, 8, false>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, s);
+        return relu_in ? launch_level_split<256, 8, true>(N, row_ptr, col_idx, val, h_in, W, msg, h_out, s)
+                       : launch_level_split<256, 8, false>(N, row_ptr, col_idx, val, h_in, W, msg, h_out, s);
     }
     return GNNHIP_EUNSUPPORTED;
 }

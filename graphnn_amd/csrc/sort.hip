@@ -196,7 +196,7 @@ int exclusive_scan_pair_i32(int* x, int* y, long long n, int* seg_scratch, hipSt
 
 namespace {
 
-// FIRST: the keys are the caller's and a pair's value is its index, or carried[index] where that is given
+// FIRST: the keys are the caller's and a pair's value is its index
 template <int BITS, bool FIRST>
 __global__ __launch_bounds__(kBlock) void radix_scatter_kernel(GroupJobs jobs, long long n, int rows, int shift, int ntiles)
 {
