@@ -7,9 +7,11 @@
 // of A and B is read from memory once per launch (64 x 64 tiles read them up to four times).  The products are formed on
 // the bf16 matrix cores from three pieces per operand (bf16_split.h).  An operand is split on its way into LDS: a thread
 // takes eight rows of one column, which is one lane's share of v_mfma_f32_32x32x16_bf16, and writes each piece as one
-// 128-bit word; words of neighbouring columns lie side by side, so neither the writes nor the reads conflict.  While a
-// stage is multiplied the next one is on its way from memory, and it goes to the other half of the LDS behind the
-// products (one barrier per stage).  The workgroups' raw sums go to scratch and are added in range order.
+// 128-bit word; words of neighbouring columns lie side by side, so neither the writes nor the reads conflict.  A stage's
+// pieces go to the other half of the LDS while the one before is multiplied, and the loads of the one after it are issued
+// as soon as that has freed their registers, ahead of the barrier (one per stage).  The workgroups' raw sums go to scratch and
+// are added in range order.  Bound by those loads: 300,000 rows, 64 x 64 outputs 36 us (4.2 TB/s), 128 x 128 80 (3.8),
+// 256 x 256 245 (2.5: 32 KB on their way per compute unit, which has no registers for more).
 #include "bf16_split.h"
 #include "buffer_addr.h"
 
@@ -41,9 +43,6 @@ template <int MT_, int NT_, int WR_, int WC_, int KW_, int KB_> struct TnShape {
     static constexpr int PIECE = 2 * KB * COLS;                          // 128-bit words of one piece of a stage
     static constexpr size_t LDS = 2 * 3 * (size_t)PIECE * 16;
     static constexpr int PER_CU = LDS <= 80 * 1024 ? 2 : 1;              // workgroups that share a compute unit
-    // four tiles in the 128 registers of two workgroups: one sum of 16 rows at a time, its operand read again from LDS
-    static constexpr bool KEEP_A = !(PER_CU == 2 && TR * TC >= 4);
-    static constexpr int SUMS = KEEP_A ? TR : 1;
     static_assert(WR * WC * KW == kTnWaves && KB % KW == 0 && TR >= 1 && TC >= 1, "shape");
 };
 
@@ -62,12 +61,9 @@ __global__ __launch_bounds__(kTnBlock, S::PER_CU * kTnWaves / 4) void sgemm_tn_s
     const rsrc_t b_rsrc = make_rsrc(B + (size_t)k_lo * ldb, (unsigned)(((size_t)(rows - 1) * ldb + n) * 4));
 
     mfma_f16 acc[S::TR][S::TC];
-#pragma unroll
-    for (int i = 0; i < S::TR; ++i)
-#pragma unroll
-        for (int j = 0; j < S::TC; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    // lane l ends with column l % 32 of a tile (of its transpose) and rows 8 (r / 4) + 4 (l / 32) + r % 4
+    auto tile_x = [&]() { return lane & 31; };
+    auto tile_y = [&](int r) { return 8 * (r / 4) + 4 * (lane >> 5) + r % 4; };
 
     // A wavefront's share of a stage: UNITS times 64 columns x 8 rows, a column per lane
     float f[S::UNITS][8];
@@ -86,17 +82,27 @@ __global__ __launch_bounds__(kTnBlock, S::PER_CU * kTnWaves / 4) void sgemm_tn_s
             for (int i = 0; i < 8; ++i) f[u][i] = buf_load_f(rsrc, voff, (r0 + 8 * group + i) * ld * 4);
         }
     };
-    auto park = [&](int buf, unsigned sign) {
+    // The scale of the pieces (bf16_split.h) is a column's, for all rows of the workgroup: up at first, and if a large element
+    // turned up in some column, everything once more with those columns scaled down.
+    __shared__ unsigned char large_in[S::COLS];           // per column
+    float largest[S::UNITS];                              // of what this lane has parked
+    bool down[S::UNITS];                                  // whether its column is scaled down the second time
+    auto park = [&](int buf, unsigned sign, auto again) __attribute__((always_inline)) {
+        constexpr bool kAgain = decltype(again)::value;
 #pragma unroll
         for (int u = 0; u < S::UNITS; ++u) {
             const int chunk = wave + u * kTnWaves;
             if (S::CHUNKS % kTnWaves && chunk >= S::CHUNKS) break;
             const unsigned flip = chunk % (S::COLS / kWave) < S::MT / kWave ? sign : 0u;
+            const bool scaled_down = kAgain && down[u];
+            const float scale = scaled_down ? kSplitDown : kSplitUp;
             bf16_words4 w[3];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
+                const float x = f[u][2 * i], y = f[u][2 * i + 1];
                 unsigned p[3];
-                bf16_split2(f[u][2 * i], f[u][2 * i + 1], p);
+                if (!kAgain) largest[u] = split_max(largest[u], x, y);
+                bf16_split2(x * scale, y * scale, scaled_down, p);
                 w[0][i] = p[0] ^ flip; w[1][i] = p[1] ^ flip; w[2][i] = p[2] ^ flip;
             }
 #pragma unroll
@@ -110,67 +116,115 @@ __global__ __launch_bounds__(kTnBlock, S::PER_CU * kTnWaves / 4) void sgemm_tn_s
     // every other workgroup: the pieces of A are negated there, and the sum is subtracted.
     // rms error against float64, relative to the sum of the terms' magnitudes, 128 x 128 over 20,000 rows, A past a ReLU: all
     // products into the running sum 3.3e-9, so 0.9e-9 (general kernel on the FP32 matrix cores 2.6e-9).
-    unsigned sign = blockIdx.x & 1 ? 0x80008000u : 0u;    // of the stage being multiplied
-    fetch(0);
-    park(0, sign);
-    __syncthreads();
-    int buf = 0;
-    for (int r0 = 0; r0 < rows; r0 += 16 * S::KB) {
-        const bool more = r0 + 16 * S::KB < rows;
-        if (more) fetch(r0 + 16 * S::KB);
-        const float factor = sign ? -1.f : 1.f;
+    auto run = [&](auto again) __attribute__((always_inline)) {
+        constexpr bool kAgain = decltype(again)::value;
+        // From four tiles on the pieces of the next stage are formed between the products of the last three tiles; with fewer
+        // there is not enough to hide them behind, and the loads would have less time (256 x 256 over 1.5M rows: 1,179 us
+        // with the pieces behind the products, 1,130 so).
+        constexpr bool kEarly = S::TR * S::TC >= 4;
 #pragma unroll
-        for (int kb = 0; kb < S::KB / S::KW; ++kb) {
-            const bf16_words4* src = words + buf * 3 * S::PIECE + (2 * (kb * S::KW + kw) + (lane >> 5)) * S::COLS + (lane & 31);
-            auto load_a = [&](int i, bf16_words4 (&a)[3]) {
+        for (int i = 0; i < S::TR; ++i)
 #pragma unroll
-                for (int p = 0; p < 3; ++p) a[p] = src[p * S::PIECE + (wr * S::TR + i) * 32];
-            };
-            bf16_words4 a[S::KEEP_A ? S::TR : 1][3];
-            if (S::KEEP_A) {
+            for (int j = 0; j < S::TC; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+        unsigned sign = blockIdx.x & 1 ? 0x80008000u : 0u;    // of the stage being multiplied
+        fetch(0);
+        park(0, sign, again);
+        fetch(16 * S::KB);
+        __syncthreads();
+        int buf = 0;
+        for (int r0 = 0; r0 < rows; r0 += 16 * S::KB) {
+            const bool more = r0 + 16 * S::KB < rows;
+            const float factor = sign ? -kSplitUpBack * kSplitUpBack : kSplitUpBack * kSplitUpBack;
+#pragma unroll
+            for (int kb = 0; kb < S::KB / S::KW; ++kb) {
+                const bf16_words4* src = words + buf * 3 * S::PIECE + (2 * (kb * S::KW + kw) + (lane >> 5)) * S::COLS + (lane & 31);
+                auto load_a = [&](int i, bf16_words4 (&a)[3]) {
+#pragma unroll
+                    for (int p = 0; p < 3; ++p) a[p] = src[p * S::PIECE + (wr * S::TR + i) * 32];
+                };
+                bf16_words4 a[S::TR][3], b[3];
 #pragma unroll
                 for (int i = 0; i < S::TR; ++i) load_a(i, a[i]);
-            }
+                // Tile after tile, two sums in turn: one is added to the running sum while the products of the other are formed.
+                mfma_f16 sum[2];
 #pragma unroll
-            for (int j = 0; j < S::TC; ++j) {
-                bf16_words4 b[3];
+                for (int q = 0; q <= S::TR * S::TC; ++q) {
+                    if (kEarly && kb == S::KB / S::KW - 1 && q == S::TR * S::TC - 3) {
+                        park(buf ^ 1, sign ^ 0x80008000u, again);
+                        fetch(r0 + 2 * 16 * S::KB);
+                    }
+                    if (q < S::TR * S::TC) {
+                        const int i = q % S::TR, j = q / S::TR;
+                        if (i == 0) {
 #pragma unroll
-                for (int p = 0; p < 3; ++p) b[p] = src[p * S::PIECE + S::MT + (wc * S::TC + j) * 32];
+                            for (int p = 0; p < 3; ++p) b[p] = src[p * S::PIECE + S::MT + (wc * S::TC + j) * 32];
+                        }
 #pragma unroll
-                for (int i0 = 0; i0 < S::TR; i0 += S::SUMS) {
-                    mfma_f16 sum[S::SUMS];
+                        for (int r = 0; r < 16; ++r) sum[q & 1][r] = 0.f;
 #pragma unroll
-                    for (int i = 0; i < S::SUMS; ++i)
+                        for (int p = 2; p >= 0; --p)
 #pragma unroll
-                        for (int r = 0; r < 16; ++r) sum[i][r] = 0.f;
-                    if (!S::KEEP_A) load_a(i0, a[0]);
+                            for (int o = 2 - p; o >= 0; --o)
+                                sum[q & 1] = TRANSPOSED ? mfma_32(b[p], a[i][o], sum[q & 1]) : mfma_32(a[i][o], b[p], sum[q & 1]);
+                    }
+                    if (q > 0) {
+                        const int i = (q - 1) % S::TR, j = (q - 1) / S::TR;
 #pragma unroll
-                    for (int p = 2; p >= 0; --p)
-#pragma unroll
-                        for (int o = 2 - p; o >= 0; --o)
-#pragma unroll
-                            for (int i = 0; i < S::SUMS; ++i) {
-                                const bf16_words4& x = a[S::KEEP_A ? i0 + i : 0][o];
-                                sum[i] = TRANSPOSED ? mfma_32(b[p], x, sum[i]) : mfma_32(x, b[p], sum[i]);
+                        for (int r = 0; r < 16; ++r) {
+                            float back = factor;
+                            if (kAgain) {
+                                const int a_col = (wr * S::TR + i) * 32 + (TRANSPOSED ? tile_x() : tile_y(r));
+                                const int b_col = (wc * S::TC + j) * 32 + (TRANSPOSED ? tile_y(r) : tile_x());
+                                back = (sign ? -1.f : 1.f) * (large_in[a_col] ? kSplitDownBack : kSplitUpBack) *
+                                       (large_in[S::MT + b_col] ? kSplitDownBack : kSplitUpBack);
                             }
+                            acc[i][j][r] = fmaf(sum[(q - 1) & 1][r], back, acc[i][j][r]);
+                        }
+                        // here, and not, as the compiler would have it, those of all tiles behind the last product: that many
+                        // sums do not fit the registers
+                        asm volatile("" : "+v"(acc[i][j]));
+                    }
+                    if (!kAgain && q > 0 && q < S::TR * S::TC) {
+                        // a product, three additions; towards the end the pieces of the next stage as well
+                        if (kEarly && kb == S::KB / S::KW - 1 && q >= S::TR * S::TC - 3) {
 #pragma unroll
-                    for (int i = 0; i < S::SUMS; ++i)
+                            for (int x = 0; x < 6; ++x) { __builtin_amdgcn_sched_group_barrier(0x8, 1, 0); __builtin_amdgcn_sched_group_barrier(0x2, 12, 0); }
+                        } else {
 #pragma unroll
-                        for (int r = 0; r < 16; ++r) acc[i0 + i][j][r] = fmaf(sum[i][r], factor, acc[i0 + i][j][r]);
-                    // the sums are added here: the compiler would gather the additions of all tiles behind the last product, and
-                    // that many sums do not fit the registers
-#pragma unroll
-                    for (int i = 0; i < S::SUMS; ++i) asm volatile("" : "+v"(acc[i0 + i][j]));
+                            for (int x = 0; x < 6; ++x) { __builtin_amdgcn_sched_group_barrier(0x8, 1, 0); __builtin_amdgcn_sched_group_barrier(0x2, 3, 0); }
+                        }
+                    }
                 }
             }
+            sign ^= 0x80008000u;
+            if (!kEarly && more) {
+                park(buf ^ 1, sign, again);
+                fetch(r0 + 2 * 16 * S::KB);
+            }
+            __syncthreads();
+            buf ^= 1;
         }
-        sign ^= 0x80008000u;
-        if (more) park(buf ^ 1, sign);
+    };
+    bool any_large = false;
+#pragma unroll
+    for (int u = 0; u < S::UNITS; ++u) largest[u] = 0.f;
+    run(std::false_type());
+#pragma unroll
+    for (int u = 0; u < S::UNITS; ++u) any_large |= largest[u] >= kSplitLarge;
+    if (__syncthreads_or(any_large)) {                    // the same for all wavefronts
+        auto column = [&](int u) { return (wave + u * kTnWaves) % (S::COLS / kWave) * kWave + lane; };
+        for (int i = threadIdx.x; i < S::COLS; i += kTnBlock) large_in[i] = 0;
         __syncthreads();
-        buf ^= 1;
+#pragma unroll
+        for (int u = 0; u < S::UNITS; ++u) if (largest[u] >= kSplitLarge) large_in[column(u)] = 1;
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < S::UNITS; ++u) down[u] = large_in[column(u)] != 0;
+        run(std::true_type());
     }
 
-    // lane l ends with column l % 32 of a tile (of its transpose) and rows 8 (r / 4) + 4 (l / 32) + r % 4
     float* part = partial + ((size_t)blockIdx.x * S::KW + kw) * m * n;
 #pragma unroll
     for (int i = 0; i < S::TR; ++i)
@@ -178,8 +232,7 @@ __global__ __launch_bounds__(kTnBlock, S::PER_CU * kTnWaves / 4) void sgemm_tn_s
         for (int j = 0; j < S::TC; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const int x = lane & 31, y = 8 * (r / 4) + 4 * (lane >> 5) + r % 4;
-                const int row = (wr * S::TR + i) * 32 + (TRANSPOSED ? x : y), col = (wc * S::TC + j) * 32 + (TRANSPOSED ? y : x);
+                const int row = (wr * S::TR + i) * 32 + (TRANSPOSED ? tile_x() : tile_y(r)), col = (wc * S::TC + j) * 32 + (TRANSPOSED ? tile_y(r) : tile_x());
                 if (row < m && col < n) part[TRANSPOSED ? (size_t)col * m + row : (size_t)row * n + col] = acc[i][j][r];
             }
 }
@@ -228,7 +281,8 @@ int choose_tn_split(int m, int n, int k, float alpha, const float* A, int lda, c
         GNNHIP_TN(128, 128, 2, 4, 1, 1);
     }
     if (m <= 64) GNNHIP_TN(64, 256, 1, 8, 1, 1);
-    if (m <= 128) GNNHIP_TN(128, 256, 2, 4, 1, 1);
+    // one workgroup per compute unit: in the 128 registers that two would leave a lane, the sums in turn are spilled (1.5M rows: 792 us, 675 so)
+    if (m <= 128) GNNHIP_TN(128, 256, 2, 4, 1, 2);
     GNNHIP_TN(256, 256, 4, 2, 1, 1);
 #undef GNNHIP_TN
 }

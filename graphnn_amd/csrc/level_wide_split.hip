@@ -9,7 +9,8 @@
 // level_wide.hip: a persistent workgroup of eight wavefronts per compute unit, W in registers for the whole launch,
 // the rows of a pass summed into one LDS tile while the matrix cores read the other, one batch of six row loads per
 // 16-row block.  What is different:
-//   * A row is split into its pieces once, by the wavefront that summed it, and lies in LDS as three bf16 planes.
+//   * A row is split into its pieces once, by the wavefront that summed it, and lies in LDS as three bf16 planes, its scale
+//     (bf16_split.h) behind them; a column of W has a scale of its own.
 //   * W in pieces takes 192 of a lane's 256 registers at C = 256.  The few fragments that do not fit are read from LDS;
 //     spilled to scratch memory they were reloaded behind the gather's loads, in whose order they had to wait (350 us
 //     per level instead of 240).
@@ -31,7 +32,7 @@ namespace {
 // C = 256: W in pieces takes 192 of a lane's 256 registers, and what does not fit would be reloaded from scratch memory
 // right behind the gather's loads, in whose order it would have to wait.  The third piece of this many contraction steps
 // of the first column block is read from LDS instead (one 128-bit read per step).
-template <int C, bool BWD> constexpr int wide_lds_fragments() { return C == 256 ? (BWD ? 7 : 6) : 0; }
+template <int C, int TR, bool BWD> constexpr int wide_lds_fragments() { return C != 256 ? 0 : TR == 16 ? (BWD ? 8 : 11) : (BWD ? 7 : 6); }
 
 // Everything that steers the gather (row pointers, column indices, edge weights) is uniform
 // across the wavefront and is fetched with scalar loads: the values land in scalar registers, cost
@@ -54,7 +55,8 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_split_kernel(
     constexpr int CW = C / WAVES;                // output columns per wavefront
     constexpr int NB = CW / 16;                  // 16-column blocks per wavefront
     constexpr int VEC = C / kWave;               // gathered floats per lane
-    // A tile in LDS is [3 pieces][2 halves of the columns][kTileRows][LDT] of bf16.  A 128-bit LDS read serves sixteen lanes per
+    // A tile in LDS is [3 pieces][2 halves of the columns][kTileRows][LDT] of bf16, with room behind every half row (the first
+    // piece's first half keeps the row's scale there).  A 128-bit LDS read serves sixteen lanes per
     // cycle, lanes 0-3, 12-15 of one sixteen together with lanes 4-11 of its neighbour; rows that start in distinct
     // 16-byte bank groups and neighbours that read the two halves (a multiple of 256 bytes apart) make that free of conflicts.
     constexpr int LDT = C / 2 + 8;
@@ -63,7 +65,7 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_split_kernel(
     constexpr int kHalf = kTileRows * LDT;
     constexpr int kPiece = 2 * kHalf;            // one piece of every element of a tile
     static_assert(kHalf * 2 % 256 == 0, "halves start at the same bank");
-    constexpr int NF = wide_lds_fragments<C, BWD>();
+    constexpr int NF = wide_lds_fragments<C, TR, BWD>();
     using vec_t = typename VecT<VEC>::type;
 
     extern __shared__ unsigned short tiles[];    // two tiles [3 pieces][kTileRows][LDT] of bf16: one read by the matrix
@@ -83,37 +85,56 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_split_kernel(
     // W[col0 + 16 jb + t][k_lane + 16 s + 0..7] (buffer loads: one lane offset, the steps as scalar offsets, so no 64-bit
     // address per element is formed)
     bf16_words4 wreg[NB][KS][3];
-    bf16_words4* w_lds = reinterpret_cast<bf16_words4*>(tiles + 2 * 3 * kPiece) + (size_t)wave * NF * kWave + lane;
+    float* w_down = reinterpret_cast<float*>(tiles + 2 * 3 * kPiece);         // [C]: a column's scale up over its scale
+    bf16_words4* w_lds = reinterpret_cast<bf16_words4*>(w_down + C) + (size_t)wave * NF * kWave + lane;
+    bool any_down;                               // columns of this wavefront that are scaled down (bf16_split.h): uniform
     {
         const rsrc_t w_rsrc = make_rsrc(W, (unsigned)(C * C * 4));
         const int w_lane_off = BWD ? ((col0 + t) * C + k_lane) * 4 : (k_lane * C + col0 + t) * 4;
+        unsigned long long large[NB];            // lanes that hold a large weight
+        auto load_w = [&](auto again) {
+            constexpr bool kAgain = decltype(again)::value;
 #pragma unroll
-        for (int jb = 0; jb < NB; ++jb)
+            for (int jb = 0; jb < NB; ++jb) {
+                float largest = 0.f;
+                const bool scaled_down = kAgain && ((large[jb] >> t) & 0x0001000100010001ull);      // in any quarter of the column
+                const float scale = scaled_down ? kSplitDown : kSplitUp;
+                if (kAgain && q == 0) w_down[col0 + 16 * jb + t] = scaled_down ? kSplitUp / kSplitDown : 1.f;
 #pragma unroll
-            for (int s = 0; s < KS; ++s) {
-                float w[8];
-                if constexpr (BWD) {             // consecutive floats of one row of W
+                for (int s = 0; s < KS; ++s) {
+                    float w[8];
+                    if constexpr (BWD) {         // consecutive floats of one row of W
 #pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        const float4 v = buf_load4(w_rsrc, w_lane_off + 16 * C * 4 * jb, s * 64 + 16 * h);
-                        w[4 * h + 0] = v.x; w[4 * h + 1] = v.y; w[4 * h + 2] = v.z; w[4 * h + 3] = v.w;
+                        for (int h = 0; h < 2; ++h) {
+                            const float4 v = buf_load4(w_rsrc, w_lane_off + 16 * C * 4 * jb, s * 64 + 16 * h);
+                            w[4 * h + 0] = v.x; w[4 * h + 1] = v.y; w[4 * h + 2] = v.z; w[4 * h + 3] = v.w;
+                        }
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) w[i] = buf_load_f(w_rsrc, w_lane_off + 64 * jb, (16 * s + i) * (C * 4));
                     }
-                } else {
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) w[i] = buf_load_f(w_rsrc, w_lane_off + 64 * jb, (16 * s + i) * (C * 4));
-                }
+                    for (int i = 0; i < 4; ++i) {
+                        if (!kAgain) largest = split_max(largest, w[2 * i], w[2 * i + 1]);
+                        unsigned p[3];
+                        bf16_split2(w[2 * i] * scale, w[2 * i + 1] * scale, scaled_down, p);
+                        wreg[jb][s][0][i] = p[0]; wreg[jb][s][1][i] = p[1]; wreg[jb][s][2][i] = p[2];
+                    }
+                    if (negated(s)) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    unsigned p[3];
-                    bf16_split2(w[2 * i], w[2 * i + 1], p);
-                    wreg[jb][s][0][i] = p[0]; wreg[jb][s][1][i] = p[1]; wreg[jb][s][2][i] = p[2];
+                        for (int p = 0; p < 3; ++p) wreg[jb][s][p] ^= 0x80008000u;
+                    }
+                    if (jb * KS + s < NF) w_lds[(jb * KS + s) * kWave] = wreg[jb][s][2];
                 }
-                if (negated(s)) {
-#pragma unroll
-                    for (int p = 0; p < 3; ++p) wreg[jb][s][p] ^= 0x80008000u;
-                }
-                if (jb == 0 && s < NF) w_lds[s * kWave] = wreg[jb][s][2];
+                if (!kAgain) large[jb] = __ballot(largest >= kSplitLarge);
             }
+        };
+        load_w(std::false_type());
+        unsigned long long all = 0;
+#pragma unroll
+        for (int jb = 0; jb < NB; ++jb) all |= large[jb];
+        any_down = all != 0;
+        if (any_down) load_w(std::true_type());                  // again, with the columns of large weights scaled down
     }
 
     const int ntiles = (int)(((long long)N + kTileRows - 1) / kTileRows);
@@ -180,8 +201,19 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_split_kernel(
     };
     auto flush_row = [&]() {
         unsigned p[VEC / 2][3];
+        float largest = 0.f;
 #pragma unroll
-        for (int i = 0; i < VEC / 2; ++i) bf16_split2(acc[2 * i], acc[2 * i + 1], p[i]);
+        for (int i = 0; i < VEC; i += 2) largest = split_max(largest, acc[i], acc[i + 1]);
+        const bool scaled_down = __any(largest >= kSplitLarge);
+        if (scaled_down) {
+#pragma unroll
+            for (int i = 0; i < VEC / 2; ++i) bf16_split2(acc[2 * i] * kSplitDown, acc[2 * i + 1] * kSplitDown, true, p[i]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < VEC / 2; ++i) bf16_split2(acc[2 * i] * kSplitUp, acc[2 * i + 1] * kSplitUp, false, p[i]);
+        }
+        // behind the row's first half: what undoes its scale
+        if (lane == 31) *reinterpret_cast<float*>(dstp + VEC) = scaled_down ? kSplitDownBack : kSplitUpBack;
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
             if constexpr (VEC == 4) *reinterpret_cast<uint2*>(dstp + j * kPiece) = make_uint2(p[0][j], p[1][j]);
@@ -314,6 +346,7 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_split_kernel(
             // that each read has six or more matrix instructions to arrive in; the first pieces of the second round's first
             // three steps take the same registers.
             bool again = false;
+            const float back = *reinterpret_cast<const float*>(cur + (rt * 16 + t) * LDT + C / 2) * kSplitUpBack;
             bf16_words4 b[3];
 #pragma unroll
             for (int j = 2; j >= 0; --j) b[j] = piece(j, first_round(0));
@@ -321,15 +354,17 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_split_kernel(
             for (int s = 0; s < KS; ++s) {
                 const int f = first_round(s);
                 if (s == KS / 2) turn();
-                bf16_words4 w3;
-                if (f < NF) w3 = w_lds[f * kWave];
+                bf16_words4 w3[NB];
+#pragma unroll
+                for (int jb = 0; jb < NB; ++jb)
+                    if (jb * KS + f < NF) w3[jb] = w_lds[(jb * KS + f) * kWave];
 #pragma unroll
                 for (int j = 2; j >= 0; --j) {
 #pragma unroll
                     for (int i = 2 - j; i >= (j == 0 ? 1 : 0); --i)
 #pragma unroll
                         for (int jb = 0; jb < NB; ++jb)
-                            acc_m[jb] = mfma_bf16(i == 2 && jb == 0 && f < NF ? w3 : wreg[jb][f][i], b[j], acc_m[jb]);
+                            acc_m[jb] = mfma_bf16(i == 2 && jb * KS + f < NF ? w3[jb] : wreg[jb][f][i], b[j], acc_m[jb]);
                     b[j] = s + 1 < KS ? piece(j, first_round(s + 1)) : piece(0, 2 - j);
                     __builtin_amdgcn_sched_barrier(0);            // keeps the read-ahead where it is written
                 }
@@ -391,10 +426,15 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_split_kernel(
                     eeN = __builtin_amdgcn_readlane(rp_next, RPW);
                 }
             }
-            if constexpr (BWD) {
 #pragma unroll
-                for (int jb = 0; jb < NB; ++jb) {
-                    float4 v = make_float4(acc_m[jb][0], acc_m[jb][1], acc_m[jb][2], acc_m[jb][3]);
+            for (int jb = 0; jb < NB; ++jb) {
+                float4 f = make_float4(back, back, back, back);
+                if (any_down) {
+                    const float4 d = *reinterpret_cast<const float4*>(w_down + col0 + 16 * jb + 4 * q);
+                    f.x *= d.x; f.y *= d.y; f.z *= d.z; f.w *= d.w;
+                }
+                if constexpr (BWD) {
+                    float4 v = make_float4(acc_m[jb][0] * f.x, acc_m[jb][1] * f.y, acc_m[jb][2] * f.z, acc_m[jb][3] * f.w);
                     if (msg) {                   // past the ReLU whose output these rows are
                         v.x = mm[jb].x > 0.f ? v.x : 0.f; v.y = mm[jb].y > 0.f ? v.y : 0.f;
                         v.z = mm[jb].z > 0.f ? v.z : 0.f; v.w = mm[jb].w > 0.f ? v.w : 0.f;
@@ -404,15 +444,9 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_split_kernel(
                         buf_store4(acc_rsrc, lane_off + rt * (16 * C * 4) + 64 * jb, 0, a);
                     }
                     outv[jb] = v;
-                }
-            } else {
-#pragma unroll
-                for (int jb = 0; jb < NB; ++jb) {
-                    acc_m[jb][0] += mm[jb].x; acc_m[jb][1] += mm[jb].y; acc_m[jb][2] += mm[jb].z; acc_m[jb][3] += mm[jb].w;
-                }
-#pragma unroll
-                for (int jb = 0; jb < NB; ++jb) {
-                    float4 v = make_float4(acc_m[jb][0], acc_m[jb][1], acc_m[jb][2], acc_m[jb][3]);
+                } else {
+                    const float4 v = make_float4(fmaf(acc_m[jb][0], f.x, mm[jb].x), fmaf(acc_m[jb][1], f.y, mm[jb].y),
+                                                 fmaf(acc_m[jb][2], f.z, mm[jb].z), fmaf(acc_m[jb][3], f.w, mm[jb].w));
                     outv[jb] = make_float4(relu_ref(v.x), relu_ref(v.y), relu_ref(v.z), relu_ref(v.w));
                 }
             }
@@ -448,8 +482,8 @@ int launch_level_split_t(int N, const int* row_ptr, const int* col_idx, const fl
     const long long slots = (long long)kNumCU * kPerCU;
     const long long per = (ntiles + slots - 1) / slots;              // contiguous run of tiles per workgroup
     const long long blocks = (ntiles + per - 1) / per;
-    const size_t smem = 2 * 3 * 2 * sizeof(unsigned short) * kTileRows * (C / 2 + 8) +
-                        sizeof(bf16_words4) * (size_t)wide_lds_fragments<C, BWD>() * WAVES * kWave;
+    const size_t smem = 2 * 3 * 2 * sizeof(unsigned short) * kTileRows * (C / 2 + 8) + sizeof(float) * C +
+                        sizeof(bf16_words4) * (size_t)wide_lds_fragments<C, TR, BWD>() * WAVES * kWave;
     static LdsLimit lds_limit;                                       // one per kernel instantiation
     GNNHIP_HIP(lds_limit.raise(reinterpret_cast<const void*>(&s2v_level_split_kernel<C, WAVES, RELU_IN, TR, BWD>), smem));
     hipLaunchKernelGGL((s2v_level_split_kernel<C, WAVES, RELU_IN, TR, BWD>), dim3((unsigned)blocks), dim3(WAVES * kWave), smem, s,

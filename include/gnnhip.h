@@ -15,6 +15,17 @@
  *     staging buffers that the library keeps per stream belong to the call in
  *     progress.  Threads that work side by side use a stream each.
  *
+ * Precision
+ *   - operands, accumulators and results are fp32; sums may be taken in another order than the reference's.
+ *   - three products run on the bf16 matrix cores, every fp32 operand as three bf16 numbers whose sum it is: the levels of
+ *     gnnhip_s2v_forward_f32 / _planned_f32 and gnnhip_s2v_level_backward_f32 at hidden 128 and 256, and A^T B with an
+ *     output of up to 256 x 256 over 8,192 rows and more (m n k >= 2^28).  Their errors against exact sums are smaller than
+ *     those of the FP32 matrix cores, over the whole range of fp32 and with infinities and NaNs carried on, with one
+ *     limit: where a row of the left operand or a column of W (a column of A or B, over a run of rows) holds an element of
+ *     2^38 or more, its elements below 2^-47 lose their last bits.
+ *   - the level entries run on the FP32 matrix cores, so at hidden 128 and 256 a forward and the same levels called one
+ *     by one agree to rounding and not to the last bit.
+ *
  * Each declaration cites the reference interface it stands in for
  * (paths relative to the graphnn source tree).
  *

@@ -431,6 +431,73 @@ def test_weight_gradient_in_pieces_is_no_less_exact_than_an_fp32_one(gpu, m, n, 
     assert pieces[0] <= fp32[0] and abs(pieces[1]) < 0.1 * fp32[0]
 
 
+def _in_pieces(route, gpu, x, W):
+    """(x W from bf16 pieces, the same product on the FP32 matrix cores); the wide forward's with negatives cut off in both"""
+    import torch
+    from graphnn_amd import ops
+    N, C = x.shape
+    if route == "gradient":
+        return ops.gemm(x.T.contiguous(), W, transA=True), ops.gemm(x, W)
+    A = (torch.arange(N + 1, device=gpu).int(), torch.arange(N, device=gpu).int(), torch.ones(N, device=gpu))     # the identity
+    if route == "backward":
+        _, g = ops.s2v_level_backward(*A, x, W.T.contiguous())
+        return g, ops.gemm(x, W)
+    # msg = the first 64 rows of x in turn; h1 = ReLU(ReLU(msg) W + msg), and the same level by itself
+    S = (torch.tensor([0, N], device=gpu).int(), A[1], A[2])
+    bufs = ops.ForwardBuffers(N, 1, C, 4, 2, gpu)
+    labels = torch.eye(64, device=gpu)[torch.arange(N, device=gpu) % 64].contiguous()
+    ops.s2v_forward(A, S, labels, x[:64].contiguous(), W, torch.zeros(C, 4, device=gpu), torch.zeros(4, 2, device=gpu), 1, bufs=bufs)
+    return bufs.h_final, ops.s2v_level(*A, bufs.msg.clamp(min=0), W, bufs.msg)
+
+
+@pytest.mark.parametrize("C", [128, 256])
+@pytest.mark.parametrize("route", ["backward", "forward", "gradient"])
+@pytest.mark.parametrize("x_size,w_size", [(1e-33, 1.0), (1e-36, 1.0), (3e-38, 8.0), (1e-41, 1e3), (1e-36, 1e36), (1e36, 1e-36), (3e11, 1.0), (1.0, 3e11),
+                                           (1e30, 1e-4), (1e18, 1e18), (1e37, 1e-20), (1e-20, 1e37)])
+def test_products_in_pieces_over_the_whole_range(gpu, C, route, x_size, w_size):
+    """operands anywhere between the smallest floats and the largest: no further from float64 than the FP32 matrix cores"""
+    import torch
+    N = 20_000 if route == "gradient" else 640
+    gen = torch.Generator(device=gpu).manual_seed(C)
+    x = torch.randn(N if route != "gradient" else C, C if route != "gradient" else N, generator=gen, device=gpu) * x_size
+    W = torch.randn(x.shape[1], C, generator=gen, device=gpu) * w_size
+    got, fp32 = _in_pieces(route, gpu, x, W)
+    if route == "forward":
+        x = x[torch.arange(N, device=gpu) % 64]
+        h = x.clamp(min=0).double()
+        want, terms = h @ W.double() + x.double(), h @ W.double().abs() + x.double().abs()
+    else:
+        want, terms = x.double() @ W.double(), x.double().abs() @ W.double().abs()
+    on = want > 0 if route == "forward" else torch.ones_like(want, dtype=torch.bool)
+    # where the result itself lies at the lower end of the range its own spacing (2^-149) comes on top
+    ours, theirs = (float(((t.double() - want).abs() / (terms + 2.0 ** -125))[on].square().mean().sqrt()) for t in (got, fp32))
+    print("%s %d, %g * %g: pieces rms %.2e, fp32 rms %.2e" % (route, C, x_size, w_size, ours, theirs))
+    assert ours <= 1.05 * theirs
+
+
+@pytest.mark.parametrize("C", [128, 256])
+@pytest.mark.parametrize("route,side", [("backward", "x"), ("backward", "W"), ("forward", "W"), ("gradient", "x"), ("gradient", "W")])
+def test_products_in_pieces_carry_infinities_and_nan(gpu, C, route, side):
+    """an infinity, a NaN or a product past the largest float on either side, against factors of three pieces whose corrections
+    have either sign: the classes (finite, infinite, NaN) and signs of the FP32 matrix cores in every output"""
+    import torch
+    gen = torch.Generator(device=gpu).manual_seed(7)
+    shape = (64, C) if route != "gradient" else (C, 20_000)
+    x = 1 + torch.rand(*shape, generator=gen, device=gpu)
+    W = 1000 + 1000 * torch.rand(shape[1], C, generator=gen, device=gpu)
+    t, at = (x, lambda i: (5 + i, 17 + 3 * i)) if side == "x" else (W, lambda i: (17 + 3 * i, 5 + i))
+    for i, v in enumerate([float("inf"), float("-inf"), float("nan"), 3.4e38, -3.4e38, 0.0]):
+        t[at(i)] = v
+    if side == "x":
+        x[30, 4] = x[31, 9] = float("inf")
+        W[4, 40], W[9, 41], W[9, 42] = float("inf"), float("-inf"), 0.0        # inf inf, inf -inf, inf 0
+    got, fp32 = _in_pieces(route, gpu, x, W)
+    assert torch.equal(torch.isnan(got), torch.isnan(fp32))
+    assert torch.equal(got == float("inf"), fp32 == float("inf")) and torch.equal(got == float("-inf"), fp32 == float("-inf"))
+    finite = torch.isfinite(fp32)
+    assert bool(finite.any()) and bool(((got - fp32)[finite].abs() <= 1e-5 * fp32[finite].abs()).all())
+
+
 def test_weight_gradient_carries_infinities_and_nan(gpu):
     """an infinite or NaN term reaches the outputs it is part of and no others, next to values whose bf16 rounding would overflow"""
     import torch
