@@ -64,6 +64,9 @@ SIGNATURES = {
     "gnnhip_s2v_forward_batched_f32": [_I] * 8 + [_P] * 11 + [_P] * 7 + [_P, _P],
     "gnnhip_s2v_forward_batched_train_f32": [_I] * 8 + [_P] * 11 + [_P] * 7 + [_P, _P],
     "gnnhip_s2v_forward_batched_labels_f32": [_I] * 8 + [_P] * 11 + [_P] * 7 + [_P, _P],
+    "gnnhip_s2v_forward_batched_sized_f32": [_I] * 9 + [_P] * 11 + [_P] * 7 + [_P, _P],
+    "gnnhip_s2v_forward_batched_train_sized_f32": [_I] * 9 + [_P] * 11 + [_P] * 7 + [_P, _P],
+    "gnnhip_s2v_forward_batched_labels_sized_f32": [_I] * 9 + [_P] * 11 + [_P] * 7 + [_P, _P],
     "gnnhip_s2v_input_labels_f32": [_I, _I, _I, _P, _P, _P, _P, _P, _P],
     "gnnhip_unary_f32": [_I, _P, _Z, _F, _F, _P],
     "gnnhip_relu_f32": [_P, _P, _Z, _P],

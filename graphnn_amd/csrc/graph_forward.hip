@@ -27,6 +27,8 @@
 // pointers, columns, weights, pooling weights, X) is issued before the first of them is used; the
 // first neighbours of a lane's rows stay in registers for all levels; the readout has three steps
 // (pool partials | pooled row + hidden layer | logits + softmax in the registers of one wavefront).
+#include <algorithm>
+
 #include "gnnhip_internal.h"
 #include "buffer_addr.h"
 
@@ -72,12 +74,12 @@ struct GraphLds {
         if (labels) f += (label_floats(n16, C, K) + 3) / 4 * 4;
         return f;
     }
-    // Entries of the edge cache with which two workgroups fit a compute unit, where that leaves five per node; else -1.  (Eight
-    // wavefronts of up to 128 registers: the latency chain of one workgroup then runs under the other's.)
+    // Entries of the edge cache with which two workgroups fit a compute unit (eight wavefronts of up to 128 registers: the latency
+    // chain of one workgroup then runs under the other's); negative: none do
     static int half_edge_cap(int n16, int C, int K, int H, int Q, int block, bool labels)
     {
         const long long left = (long long)(kLdsLimit / 2 / sizeof(float)) - (long long)fixed_floats(n16, C, K, H, Q, block, labels);
-        return left >= 10 * n16 ? (int)(left / 2 / 4 * 4) : -1;
+        return left >= 0 ? (int)(left / 2 / 4 * 4) : -1;
     }
     // entries of the edge cache that still fit under the LDS limit
     static int edge_cap(int n16, int C, int K, int H, int Q, int block, bool labels = false)
@@ -287,6 +289,16 @@ __global__ __launch_bounds__(kBinBlock) void graph_bins_kernel(int B, int cap, c
     }
 }
 
+// Whether the registers let two workgroups share a compute unit: four wavefronts always, eight with up to 128 registers per lane.
+template <int C, int WAVES, bool KEEP> constexpr bool two_per_cu() { return WAVES == 4 || (WAVES == 8 && C <= 32 && !KEEP); }
+// The variants that take 129 unless they are told (more than 48 label columns at hidden 32; what was priced as two workgroups then
+// ran as one: 60 columns, 116,000 nodes, bins of 144 nodes 103 us, 71 as two).  The others, which do not, lose 2 to 3 % to
+// the bound.
+template <int C, int KSX, int WAVES, bool KEEP, bool PACK> constexpr int min_waves()
+{
+    return two_per_cu<C, WAVES, KEEP>() && WAVES == 8 && C == 32 && KSX >= (PACK ? 16 : 8) ? 4 : (WAVES + 3) / 4;
+}
+
 // WAVES wavefronts per workgroup (4, 8 or 16): chosen by the host so that the largest graph's
 // (column block x row tile) tasks spread over the wavefronts.
 // order: null (graphs in batch order), or the records graph_order_kernel left.
@@ -296,7 +308,7 @@ __global__ __launch_bounds__(kBinBlock) void graph_bins_kernel(int B, int cap, c
 // carries a bin through the input stage and the levels as one block-diagonal graph, and its wavefronts run the
 // readout of the bin's graphs, one graph each (H <= 64 and Q <= 64: a lane per hidden unit and per class).
 template <int C, int KSX, int WAVES, bool KEEP = false, bool PACK = false>
-__global__ __launch_bounds__(WAVES * kWave) void s2v_graph_forward_kernel(
+__global__ __launch_bounds__(WAVES * kWave, (min_waves<C, KSX, WAVES, KEEP, PACK>())) void s2v_graph_forward_kernel(
     int B, int K, unsigned k_magic, int H, int Q, int L, int n16max, int ecap,
     const int* __restrict__ a_row_ptr, const int* __restrict__ a_col_idx, const float* __restrict__ a_val,
     const int* __restrict__ s_row_ptr, const int* __restrict__ s_col_idx, const float* __restrict__ s_val,
@@ -873,16 +885,13 @@ int launch_graph_forward(int B, int K, int H, int Q, int L, int n16max,
                          const int* s_row_ptr, const int* s_col_idx, const float* s_val,
                          const float* X, const float* Wn2l, const float* Wc, const float* Wh1, const float* Wh2,
                          float* msg, float* h_final, float* pool, float* hidden, float* logits, float* probs,
-                         int* pred, int* status, float* h_levels, long long level_stride, int pack, hipStream_t s)
+                         int* pred, int* status, float* h_levels, long long level_stride, int pack, bool half, hipStream_t s)
 {
     constexpr int kBlock = WAVES * kWave;
     constexpr bool LABELS = (KSX == 0);
     int ecap = GraphLds::edge_cap(n16max, C, K, H, Q, kBlock, LABELS);
     if (ecap < 0) return GNNHIP_EUNSUPPORTED;
-    if (WAVES <= 8) {
-        const int half = GraphLds::half_edge_cap(n16max, C, K, H, Q, kBlock, LABELS);
-        if (half >= 0 && half < ecap) ecap = half;
-    }
+    if (half && (h_levels ? two_per_cu<C, WAVES, true>() : two_per_cu<C, WAVES, false>())) ecap = std::min(ecap, GraphLds::half_edge_cap(n16max, C, K, H, Q, kBlock, LABELS));
     const size_t smem = sizeof(float) * (GraphLds::fixed_floats(n16max, C, K, H, Q, kBlock, LABELS) + 2 * (size_t)ecap);
     constexpr bool kKeepBuilt = !LABELS;    // the variant that keeps all levels exists for the dense input only
     // the variant that packs graphs into bins exists for the workgroup shapes bins of 128 nodes and more select
@@ -938,10 +947,10 @@ int dispatch_ksx(bool labels, int B, int K, int H, int Q, int L, int n16max,
                  const int* s_row_ptr, const int* s_col_idx, const float* s_val,
                  const float* X, const float* Wn2l, const float* Wc, const float* Wh1, const float* Wh2,
                  float* msg, float* h_final, float* pool, float* hidden, float* logits, float* probs,
-                 int* pred, int* status, float* h_levels, long long level_stride, int pack, hipStream_t s)
+                 int* pred, int* status, float* h_levels, long long level_stride, int pack, bool half, hipStream_t s)
 {
 #define GNNHIP_GF_ARGS B, K, H, Q, L, n16max, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx, s_val, \
-                       X, Wn2l, Wc, Wh1, Wh2, msg, h_final, pool, hidden, logits, probs, pred, status, h_levels, level_stride, pack, s
+                       X, Wn2l, Wc, Wh1, Wh2, msg, h_final, pool, hidden, logits, probs, pred, status, h_levels, level_stride, pack, half, s
     if (labels) return launch_graph_forward<C, 0, WAVES>(GNNHIP_GF_ARGS);
     if (K <= 16) return launch_graph_forward<C, 4, WAVES>(GNNHIP_GF_ARGS);
     if (K <= 32) return launch_graph_forward<C, 8, WAVES>(GNNHIP_GF_ARGS);
@@ -957,10 +966,10 @@ int dispatch_waves(bool labels, int B, int K, int H, int Q, int L, int n16max,
                    const int* s_row_ptr, const int* s_col_idx, const float* s_val,
                    const float* X, const float* Wn2l, const float* Wc, const float* Wh1, const float* Wh2,
                    float* msg, float* h_final, float* pool, float* hidden, float* logits, float* probs,
-                   int* pred, int* status, float* h_levels, long long level_stride, int pack, hipStream_t s)
+                   int* pred, int* status, float* h_levels, long long level_stride, int pack, bool half, hipStream_t s)
 {
 #define GNNHIP_GF_ARGS B, K, H, Q, L, n16max, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx, s_val, \
-                       X, Wn2l, Wc, Wh1, Wh2, msg, h_final, pool, hidden, logits, probs, pred, status, h_levels, level_stride, pack, s
+                       X, Wn2l, Wc, Wh1, Wh2, msg, h_final, pool, hidden, logits, probs, pred, status, h_levels, level_stride, pack, half, s
     // hidden 128: eight wavefronts, one per 16-column block (64 registers of a lane hold W^T and the tile operand of
     // a contraction; sixteen wavefronts would leave a lane 128 registers in all)
     if constexpr (C == 128) {
@@ -981,7 +990,7 @@ using namespace gnnhip;
 
 namespace {
 
-int forward_batched_entry(bool labels, int N, int B, int K, int C, int H, int Q, int L, int max_graph_nodes,
+int forward_batched_entry(bool labels, long long a_nnz, int N, int B, int K, int C, int H, int Q, int L, int max_graph_nodes,
                           const int* a_row_ptr, const int* a_col_idx, const float* a_val,
                           const int* s_row_ptr, const int* s_col_idx, const float* s_val,
                           const void* X, const float* W_n2l, const float* W_conv,
@@ -1009,9 +1018,10 @@ int forward_batched_entry(bool labels, int N, int B, int K, int C, int H, int Q,
     const float* Xf = static_cast<const float*>(X);
     if (h_levels && !aligned16(h_levels)) return set_error(GNNHIP_EUNSUPPORTED, "h_levels must be 16-byte aligned");
     const long long level_stride = (long long)N * C;
-    auto run = [&](int n16v, int pack) {      // pack: 0 graph by graph, 1 bins, 2 bins for workgroups of eight wavefronts
+    // pack: 0 graph by graph, 1 bins, 2 bins for workgroups of eight wavefronts; half: two of those per compute unit
+    auto run = [&](int n16v, int pack, bool half) {
 #define GNNHIP_GF_ARGS labels, B, K, H, Q, L, n16v, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx, s_val, \
-                       Xf, W_n2l, W_conv, W_h1, W_h2, msg, h_final, pool, hidden, logits, probs, pred, status, h_levels, level_stride, pack, s
+                       Xf, W_n2l, W_conv, W_h1, W_h2, msg, h_final, pool, hidden, logits, probs, pred, status, h_levels, level_stride, pack, half, s
         switch (C) {
         case 16: return dispatch_waves<16>(GNNHIP_GF_ARGS);
         case 32: return dispatch_waves<32>(GNNHIP_GF_ARGS);
@@ -1020,6 +1030,9 @@ int forward_batched_entry(bool labels, int N, int B, int K, int C, int H, int Q,
         }
 #undef GNNHIP_GF_ARGS
     };
+    // whether an edge cache of `cap` entries holds those of a bin of `nodes` nodes, most of which are a few nodes short of that;
+    // the host knows the mean only (not known at all, it is taken to)
+    auto holds = [&](int cap, int nodes) { return 0.95 * (double)a_nnz * nodes <= (double)cap * (double)N; };
     int rc = GNNHIP_EUNSUPPORTED;
     // more graphs than compute units: runs of consecutive graphs share a workgroup (bins of at least kPackNodes nodes)
     if (B >= kPackMinGraphs && B <= kBinMaxGraphs && H <= kWave && Q <= kWave && !h_levels) {
@@ -1029,26 +1042,36 @@ int forward_batched_entry(bool labels, int N, int B, int K, int C, int H, int Q,
         // 53 -> 43 us in one round of bins of 208 nodes).  Times of a round in us, from sweeps of the bin size at 17,000 to
         // 120,000 nodes.  The host knows the totals only: a bin wastes about half a mean graph, and every 64 graphs about half
         // a bin.
+        // A bin with more entries than its cache reads them from L2 in every level: a round of two workgroups per compute unit then
+        // takes about 1.3 times as long (hidden 32, 12 entries per node: bins of 208 nodes 53 us, of 192, which fit, 40), one
+        // of single workgroups, which have nothing to run meanwhile, twice (2,000 graphs of 50 nodes with 30 entries each:
+        // 226 us, 109 with two).
         int best = 0, best_pack = 1;
+        bool best_two = false;
         double best_cost = 0.0;
         for (int pack = C == 16 ? 2 : 1; pack <= (C <= 32 ? 2 : 1); ++pack) {
             for (int cand = n16 > kPackNodes ? n16 : kPackNodes; cand <= kPackMaxNodes; cand += 16) {
                 const int block = pack == 2 ? 512 : 1024;
-                if (GraphLds::edge_cap(cand, C, K, H, Q, block, labels) < 256) break;
-                const bool two = pack == 2 && GraphLds::half_edge_cap(cand, C, K, H, Q, block, labels) >= 0;
-                if (pack == 2 && C == 32 && !two) break;
-                const int slots = two ? 2 * kNumCU : kNumCU;
-                const double fill = (double)cand - 0.5 * (double)N / (double)B;
-                const double nbins = (double)N / (fill > 16.0 ? fill : 16.0) + (double)B / 128.0;
-                const double rounds = (double)(long long)((nbins + slots - 1) / slots);
-                const double per = cand / 128.0;
-                const double cost = rounds * (C == 64 ? 6.0 + 20.0 * per : pack == 2 ? 11.0 + 14.0 * per : 12.0 + 8.0 * per);
-                if (!best || cost < best_cost) { best = cand; best_cost = cost; best_pack = pack; }
+                const int full = GraphLds::edge_cap(cand, C, K, H, Q, block, labels);
+                if (full < 256) break;
+                const int half = pack == 2 && a_nnz >= 0 ? std::min(full, GraphLds::half_edge_cap(cand, C, K, H, Q, block, labels)) : -1;
+                for (int two = half < 0 ? 0 : 1; two >= (C == 32 && pack == 2 ? 1 : 0); --two) {
+                    const int slots = two ? 2 * kNumCU : kNumCU;
+                    const double fill = (double)cand - 0.5 * (double)N / (double)B;
+                    const double nbins = (double)N / (fill > 16.0 ? fill : 16.0) + (double)B / 128.0;
+                    const double rounds = (double)(long long)((nbins + slots - 1) / slots);
+                    const double per = cand / 128.0;
+                    double cost = rounds * (C == 64 ? 6.0 + 20.0 * per : pack == 2 ? 11.0 + 14.0 * per : 12.0 + 8.0 * per);
+                    if (!holds(two ? half : full, cand)) cost *= two ? 1.3 : 2.0;
+                    if (!best || cost < best_cost) { best = cand; best_cost = cost; best_pack = pack; best_two = two; }
+                }
             }
         }
-        if (best) rc = run(best, best_pack);
+        if (best) rc = run(best, best_pack, best_two);
     }
-    if (rc == GNNHIP_EUNSUPPORTED) rc = run(n16, 0);
+    // (up to one graph per compute unit nobody shares one)
+    if (rc == GNNHIP_EUNSUPPORTED)
+        rc = run(n16, 0, B > kNumCU && a_nnz >= 0 && holds(GraphLds::half_edge_cap(n16, C, K, H, Q, 512, labels), n16));
     if (rc == GNNHIP_EUNSUPPORTED) return set_error(rc, "graph-resident forward could not be configured for this shape");
     return rc;
 }
@@ -1063,7 +1086,7 @@ extern "C" int gnnhip_s2v_forward_batched_f32(int N, int B, int K, int C, int H,
                                               float* msg, float* h_final, float* pool, float* hidden, float* logits,
                                               float* probs, int* pred, int* status, void* stream)
 {
-    return forward_batched_entry(false, N, B, K, C, H, Q, L, max_graph_nodes, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx,
+    return forward_batched_entry(false, -1, N, B, K, C, H, Q, L, max_graph_nodes, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx,
                                  s_val, X, W_n2l, W_conv, W_h1, W_h2, msg, h_final, pool, hidden, logits, probs, pred, status, nullptr, stream);
 }
 
@@ -1075,9 +1098,54 @@ extern "C" int gnnhip_s2v_forward_batched_labels_f32(int N, int B, int K, int C,
                                                      float* msg, float* h_final, float* pool, float* hidden, float* logits,
                                                      float* probs, int* pred, int* status, void* stream)
 {
-    return forward_batched_entry(true, N, B, K, C, H, Q, L, max_graph_nodes, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx,
+    return forward_batched_entry(true, -1, N, B, K, C, H, Q, L, max_graph_nodes, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx,
                                  s_val, node_label, W_n2l, W_conv, W_h1, W_h2, msg, h_final, pool, hidden, logits, probs, pred, status, nullptr, stream);
 }
+
+extern "C" int gnnhip_s2v_forward_batched_sized_f32(int N, int B, int K, int C, int H, int Q, int L, int max_graph_nodes, int a_nnz,
+                                                    const int* a_row_ptr, const int* a_col_idx, const float* a_val,
+                                                    const int* s_row_ptr, const int* s_col_idx, const float* s_val,
+                                                    const float* X, const float* W_n2l, const float* W_conv,
+                                                    const float* W_h1, const float* W_h2,
+                                                    float* msg, float* h_final, float* pool, float* hidden, float* logits,
+                                                    float* probs, int* pred, int* status, void* stream)
+{
+    GNNHIP_REQUIRE(a_nnz >= 0, "negative entry count in s2v_forward_batched_sized (a_nnz=%d)", a_nnz);
+    return forward_batched_entry(false, a_nnz, N, B, K, C, H, Q, L, max_graph_nodes, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx,
+                                 s_val, X, W_n2l, W_conv, W_h1, W_h2, msg, h_final, pool, hidden, logits, probs, pred, status, nullptr, stream);
+}
+
+extern "C" int gnnhip_s2v_forward_batched_labels_sized_f32(int N, int B, int K, int C, int H, int Q, int L, int max_graph_nodes, int a_nnz,
+                                                           const int* a_row_ptr, const int* a_col_idx, const float* a_val,
+                                                           const int* s_row_ptr, const int* s_col_idx, const float* s_val,
+                                                           const int* node_label, const float* W_n2l, const float* W_conv,
+                                                           const float* W_h1, const float* W_h2,
+                                                           float* msg, float* h_final, float* pool, float* hidden, float* logits,
+                                                           float* probs, int* pred, int* status, void* stream)
+{
+    GNNHIP_REQUIRE(a_nnz >= 0, "negative entry count in s2v_forward_batched_labels_sized (a_nnz=%d)", a_nnz);
+    return forward_batched_entry(true, a_nnz, N, B, K, C, H, Q, L, max_graph_nodes, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx,
+                                 s_val, node_label, W_n2l, W_conv, W_h1, W_h2, msg, h_final, pool, hidden, logits, probs, pred, status, nullptr, stream);
+}
+
+namespace {
+
+int forward_batched_train_entry(long long a_nnz, int N, int B, int K, int C, int H, int Q, int L, int max_graph_nodes,
+                                const int* a_row_ptr, const int* a_col_idx, const float* a_val,
+                                const int* s_row_ptr, const int* s_col_idx, const float* s_val,
+                                const float* X, const float* W_n2l, const float* W_conv, const float* W_h1, const float* W_h2,
+                                float* msg, float* h_levels, float* pool, float* hidden, float* logits,
+                                float* probs, int* pred, int* status, void* stream)
+{
+    GNNHIP_REQUIRE(h_levels, "null h_levels in s2v_forward_batched_train");
+    // the last level doubles as the embedding output of the inference entry
+    float* h_last = h_levels + (size_t)(L > 0 ? L : 0) * (size_t)(N > 0 ? N : 0) * (size_t)(C > 0 ? C : 0);
+    return forward_batched_entry(false, a_nnz, N, B, K, C, H, Q, L, max_graph_nodes, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx,
+                                 s_val, X, W_n2l, W_conv, W_h1, W_h2, msg, h_last, pool, hidden, logits, probs, pred, status, h_levels,
+                                 stream);
+}
+
+}  // namespace
 
 extern "C" int gnnhip_s2v_forward_batched_train_f32(int N, int B, int K, int C, int H, int Q, int L, int max_graph_nodes,
                                                     const int* a_row_ptr, const int* a_col_idx, const float* a_val,
@@ -1087,10 +1155,19 @@ extern "C" int gnnhip_s2v_forward_batched_train_f32(int N, int B, int K, int C, 
                                                     float* msg, float* h_levels, float* pool, float* hidden, float* logits,
                                                     float* probs, int* pred, int* status, void* stream)
 {
-    GNNHIP_REQUIRE(h_levels, "null h_levels in s2v_forward_batched_train");
-    // the last level doubles as the embedding output of the inference entry
-    float* h_last = h_levels + (size_t)(L > 0 ? L : 0) * (size_t)(N > 0 ? N : 0) * (size_t)(C > 0 ? C : 0);
-    return forward_batched_entry(false, N, B, K, C, H, Q, L, max_graph_nodes, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx,
-                                 s_val, X, W_n2l, W_conv, W_h1, W_h2, msg, h_last, pool, hidden, logits, probs, pred, status, h_levels,
-                                 stream);
+    return forward_batched_train_entry(-1, N, B, K, C, H, Q, L, max_graph_nodes, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx, s_val, X,
+                                       W_n2l, W_conv, W_h1, W_h2, msg, h_levels, pool, hidden, logits, probs, pred, status, stream);
+}
+
+extern "C" int gnnhip_s2v_forward_batched_train_sized_f32(int N, int B, int K, int C, int H, int Q, int L, int max_graph_nodes, int a_nnz,
+                                                          const int* a_row_ptr, const int* a_col_idx, const float* a_val,
+                                                          const int* s_row_ptr, const int* s_col_idx, const float* s_val,
+                                                          const float* X, const float* W_n2l, const float* W_conv,
+                                                          const float* W_h1, const float* W_h2,
+                                                          float* msg, float* h_levels, float* pool, float* hidden, float* logits,
+                                                          float* probs, int* pred, int* status, void* stream)
+{
+    GNNHIP_REQUIRE(a_nnz >= 0, "negative entry count in s2v_forward_batched_train_sized (a_nnz=%d)", a_nnz);
+    return forward_batched_train_entry(a_nnz, N, B, K, C, H, Q, L, max_graph_nodes, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx, s_val, X,
+                                       W_n2l, W_conv, W_h1, W_h2, msg, h_levels, pool, hidden, logits, probs, pred, status, stream);
 }

@@ -205,12 +205,14 @@ template <size_t HOST, class... P> struct Entry<int (*)(P...), HOST> {
                        "W_h2, msg, h_a, h_b, pool, hidden, logits, probs, pred, @which")                                                 \
     X(s2v_forward_planned_f32, "plan, B, K, C, H, Q, L, s_row_ptr, s_col_idx, s_val, X, W_n2l, W_conv, W_h1, W_h2, msg, h_a, h_b, "     \
                                "pool, hidden, logits, probs, pred, @which")                                                              \
-    X(s2v_forward_batched_f32, "N, B, K, C, H, Q, L, max_graph_nodes, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx, s_val, X, "    \
-                               "W_n2l, W_conv, W_h1, W_h2, msg, h_final, pool, hidden, logits, probs, pred, status")                    \
-    X(s2v_forward_batched_train_f32, "N, B, K, C, H, Q, L, max_graph_nodes, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx, s_val, " \
-                                     "X, W_n2l, W_conv, W_h1, W_h2, msg, h_levels, pool, hidden, logits, probs, pred, status")          \
-    X(s2v_forward_batched_labels_f32, "N, B, K, C, H, Q, L, max_graph_nodes, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx, s_val, " \
-                                      "label, W_n2l, W_conv, W_h1, W_h2, msg, h_final, pool, hidden, logits, probs, pred, status")      \
+    X(s2v_forward_batched_sized_f32, "N, B, K, C, H, Q, L, max_graph_nodes, a_nnz, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx, "    \
+                                     "s_val, X, W_n2l, W_conv, W_h1, W_h2, msg, h_final, pool, hidden, logits, probs, pred, status")    \
+    X(s2v_forward_batched_train_sized_f32, "N, B, K, C, H, Q, L, max_graph_nodes, a_nnz, a_row_ptr, a_col_idx, a_val, s_row_ptr, "      \
+                                           "s_col_idx, s_val, X, W_n2l, W_conv, W_h1, W_h2, msg, h_levels, pool, hidden, logits, "      \
+                                           "probs, pred, status")                                                                       \
+    X(s2v_forward_batched_labels_sized_f32, "N, B, K, C, H, Q, L, max_graph_nodes, a_nnz, a_row_ptr, a_col_idx, a_val, s_row_ptr, "     \
+                                            "s_col_idx, s_val, label, W_n2l, W_conv, W_h1, W_h2, msg, h_final, pool, hidden, logits, "  \
+                                            "probs, pred, status")                                                                      \
     X(unary_f32, "op, x, n, a0, a1")                                                                                                    \
     X(relu_f32, "x, out, n")                                                                                                            \
     X(axpy_f32, "n, a, x, y")                                                                                                           \

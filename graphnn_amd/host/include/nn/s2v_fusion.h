@@ -4,7 +4,7 @@
 //   MatMul(sparse A, h) -> MatMul(., W) -> ElewiseAdd(., msg) -> ReLU      => gnnhip_s2v_level_f32
 //   MatMul(dense X, W)  -> ReLU                                             => gnnhip_s2v_input_f32
 //   input -> levels -> MatMul(S, h) -> MatMul(., W1) -> ReLU -> MatMul(., W2), when the batch is laid
-//   out as GetBatch lays it out (contiguous graphs, no edge between graphs)  => gnnhip_s2v_forward_batched_f32
+//   out as GetBatch lays it out (contiguous graphs, no edge between graphs)  => gnnhip_s2v_forward_batched_sized_f32
 //
 // (the chains of examples/graph_classification/src/kernel_mean_field.cpp:31-47).  A chain
 // is folded only at Phase::TEST and only when its intermediate variables have no other
@@ -441,8 +441,8 @@ inline void FactorGraph::FoldWholeForward(Plan& plan)
                 float* hs = st->hstack.data->ptr;
                 // small block-diagonal batches: everything in one launch, the levels stored on the way
                 if (n2n->block_diagonal && sub->max_subgraph_nodes > 0 && N <= detail::kOneLaunchTrainMaxNodes) {
-                    const int rc = gnnhip_s2v_forward_batched_train_f32(
-                        (int)N, (int)B, (int)K, (int)C, (int)H, (int)Q, L, sub->max_subgraph_nodes,
+                    const int rc = gnnhip_s2v_forward_batched_train_sized_f32(
+                        (int)N, (int)B, (int)K, (int)C, (int)H, (int)Q, L, sub->max_subgraph_nodes, (int)A->value.data->nnz,
                         A->value.data->row_ptr, A->value.data->col_idx, A->value.data->val,
                         S->value.data->row_ptr, S->value.data->col_idx, S->value.data->val,
                         X->value.data->ptr, Wn->value.data->ptr, Wc->value.data->ptr, W1->value.data->ptr, W2->value.data->ptr,
@@ -541,8 +541,8 @@ inline void FactorGraph::FoldWholeForward(Plan& plan)
             // small and medium block-diagonal batches in one launch (256 graphs of configuration 2: 23 us against 40)
             if (n2n->block_diagonal && sub->contiguous_subgraphs && sub->max_subgraph_nodes > 0 &&
                 N <= detail::kOneLaunchMaxNodes) {
-                const int rc = gnnhip_s2v_forward_batched_f32(
-                    (int)N, (int)B, (int)K, (int)C, (int)H, (int)Q, L, sub->max_subgraph_nodes,
+                const int rc = gnnhip_s2v_forward_batched_sized_f32(
+                    (int)N, (int)B, (int)K, (int)C, (int)H, (int)Q, L, sub->max_subgraph_nodes, (int)A->value.data->nnz,
                     A->value.data->row_ptr, A->value.data->col_idx, A->value.data->val,
                     S->value.data->row_ptr, S->value.data->col_idx, S->value.data->val,
                     X->value.data->ptr, Wn->value.data->ptr, Wc->value.data->ptr, W1->value.data->ptr, W2->value.data->ptr,

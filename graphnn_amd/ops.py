@@ -339,7 +339,7 @@ class BatchedBuffers:
 
 
 def s2v_forward_batched(a_csr, s_csr, X, W_n2l, W_conv, W_h1, W_h2, L, max_graph_nodes, bufs=None):
-    """One-launch forward for block-diagonal batches (see gnnhip_s2v_forward_batched_f32)."""
+    """One-launch forward for block-diagonal batches (see gnnhip_s2v_forward_batched_sized_f32)."""
     N, K = X.shape
     C, H, Q = W_n2l.shape[1], W_h1.shape[1], W_h2.shape[1]
     B = s_csr[0].numel() - 1
@@ -351,8 +351,8 @@ def s2v_forward_batched(a_csr, s_csr, X, W_n2l, W_conv, W_h1, W_h2, L, max_graph
         raise ValueError("weight shapes do not chain")
     if bufs is None:
         bufs = BatchedBuffers(N, B, C, H, Q, X.device)
-    _bound().s2v_forward_batched_f32(
-        N, B, K, C, H, Q, L, int(max_graph_nodes),
+    _bound().s2v_forward_batched_sized_f32(
+        N, B, K, C, H, Q, L, int(max_graph_nodes), int(a_csr[1].numel()),
         a_csr[0], a_csr[1], a_csr[2],
         s_csr[0], s_csr[1], s_csr[2],
         X, W_n2l, W_conv, W_h1, W_h2,
@@ -377,8 +377,8 @@ def s2v_forward_batched_train(a_csr, s_csr, X, W_n2l, W_conv, W_h1, W_h2, L, max
     if bufs is None:
         bufs = BatchedBuffers(N, B, C, H, Q, X.device)
     h_levels = _empty(X, "f", L + 1, N, C)
-    _bound().s2v_forward_batched_train_f32(
-        N, B, K, C, H, Q, L, int(max_graph_nodes),
+    _bound().s2v_forward_batched_train_sized_f32(
+        N, B, K, C, H, Q, L, int(max_graph_nodes), int(a_csr[1].numel()),
         a_csr[0], a_csr[1], a_csr[2],
         s_csr[0], s_csr[1], s_csr[2],
         X, W_n2l, W_conv, W_h1, W_h2,
@@ -402,8 +402,8 @@ def bind_s2v_forward_batched(a_csr, s_csr, X, W_n2l, W_conv, W_h1, W_h2, L, max_
         raise ValueError("S must list every node exactly once")
     if W_n2l.shape[0] != K or tuple(W_conv.shape) != (C, C) or W_h1.shape[0] != C or W_h2.shape[0] != H:
         raise ValueError("weight shapes do not chain")
-    fn = _lib().gnnhip_s2v_forward_batched_f32
-    args = (N, B, K, C, H, Q, L, int(max_graph_nodes),
+    fn = _lib().gnnhip_s2v_forward_batched_sized_f32
+    args = (N, B, K, C, H, Q, L, int(max_graph_nodes), int(a_csr[1].numel()),
             _i32(a_csr[0], "a_row_ptr"), _i32(a_csr[1], "a_col_idx"), _f32(a_csr[2], "a_val"),
             _i32(s_csr[0], "s_row_ptr"), _i32(s_csr[1], "s_col_idx"), _f32(s_csr[2], "s_val"),
             _f32(X, "X"), _f32(W_n2l, "W_n2l"), _f32(W_conv, "W_conv"), _f32(W_h1, "W_h1"), _f32(W_h2, "W_h2"),
@@ -419,7 +419,7 @@ def bind_s2v_forward_batched(a_csr, s_csr, X, W_n2l, W_conv, W_h1, W_h2, L, max_
 
 
 def s2v_forward_batched_labels(a_csr, s_csr, label, W_n2l, W_conv, W_h1, W_h2, L, max_graph_nodes, bufs=None):
-    """One-launch forward from one int label per node (see gnnhip_s2v_forward_batched_labels_f32)."""
+    """One-launch forward from one int label per node (see gnnhip_s2v_forward_batched_labels_sized_f32)."""
     N = label.numel()
     K, C = W_n2l.shape
     H, Q = W_h1.shape[1], W_h2.shape[1]
@@ -432,8 +432,8 @@ def s2v_forward_batched_labels(a_csr, s_csr, label, W_n2l, W_conv, W_h1, W_h2, L
         raise ValueError("weight shapes do not chain")
     if bufs is None:
         bufs = BatchedBuffers(N, B, C, H, Q, W_n2l.device)
-    _bound().s2v_forward_batched_labels_f32(
-        N, B, K, C, H, Q, L, int(max_graph_nodes),
+    _bound().s2v_forward_batched_labels_sized_f32(
+        N, B, K, C, H, Q, L, int(max_graph_nodes), int(a_csr[1].numel()),
         a_csr[0], a_csr[1], a_csr[2],
         s_csr[0], s_csr[1], s_csr[2],
         label, W_n2l, W_conv, W_h1, W_h2,

@@ -319,6 +319,32 @@ int gnnhip_s2v_forward_batched_labels_f32(int N, int B, int K, int C, int H, int
                                           float* msg, float* h_final, float* pool, float* hidden, float* logits,
                                           float* probs, int* pred, int* status, void* stream);
 
+/* ---- the three one-launch forwards above for callers that know the number of entries of A, a_nnz (GetBatch's host has it as the
+ *      length of its edge lists, examples/graph_classification/include/nn_common.h:36-105).  It decides whether two
+ *      workgroups can share a compute unit's LDS, which batches of few entries per node gain from (3,001 graphs, hidden 32:
+ *      53 -> 44 us); any value from 0 up gives the same results. */
+int gnnhip_s2v_forward_batched_sized_f32(int N, int B, int K, int C, int H, int Q, int L, int max_graph_nodes, int a_nnz,
+                                         const int* a_row_ptr, const int* a_col_idx, const float* a_val,
+                                         const int* s_row_ptr, const int* s_col_idx, const float* s_val,
+                                         const float* X, const float* W_n2l, const float* W_conv,
+                                         const float* W_h1, const float* W_h2,
+                                         float* msg, float* h_final, float* pool, float* hidden, float* logits,
+                                         float* probs, int* pred, int* status, void* stream);
+int gnnhip_s2v_forward_batched_train_sized_f32(int N, int B, int K, int C, int H, int Q, int L, int max_graph_nodes, int a_nnz,
+                                               const int* a_row_ptr, const int* a_col_idx, const float* a_val,
+                                               const int* s_row_ptr, const int* s_col_idx, const float* s_val,
+                                               const float* X, const float* W_n2l, const float* W_conv,
+                                               const float* W_h1, const float* W_h2,
+                                               float* msg, float* h_levels, float* pool, float* hidden, float* logits,
+                                               float* probs, int* pred, int* status, void* stream);
+int gnnhip_s2v_forward_batched_labels_sized_f32(int N, int B, int K, int C, int H, int Q, int L, int max_graph_nodes, int a_nnz,
+                                                const int* a_row_ptr, const int* a_col_idx, const float* a_val,
+                                                const int* s_row_ptr, const int* s_col_idx, const float* s_val,
+                                                const int* node_label, const float* W_n2l, const float* W_conv,
+                                                const float* W_h1, const float* W_h2,
+                                                float* msg, float* h_final, float* pool, float* hidden, float* logits,
+                                                float* probs, int* pred, int* status, void* stream);
+
 /* ---- UnaryEngine<GPU>::Exec<Functor> (include/tensor/gpu_unary_functor.h:331-384):
  *      in-place x[i] = f(x[i]); a0/a1 are the functor's constructor arguments. */
 int gnnhip_unary_f32(int op, float* x, size_t n, float a0, float a1, void* stream);

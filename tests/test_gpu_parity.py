@@ -5,6 +5,7 @@ PARITY_TOL = 1e-4 under conftest.max_rel (floors measured per tensor kind) for f
 fp32 summation orders legitimately differ by more, a float64 model of the same computation decides
 (conftest.assert_parity).
 """
+import ctypes
 import json
 import os
 
@@ -1240,6 +1241,53 @@ def test_batched_forward_of_more_graphs_than_compute_units(gpu, oracle, B, C, hi
         assert max_rel(_n(fresh.logits)[fits], got["logits"][fits]) < PARITY_TOL
         assert max_rel(_n(fresh.pool)[fits], got["pool"][fits]) < PARITY_TOL
         assert np.all(_n(fresh.logits)[~fits] == -7.0)
+
+
+@pytest.mark.parametrize("C,K,B", [(16, 60, 700), (32, 7, 900), (32, 60, 700), (32, 200, 700), (64, 7, 600), (16, 7, 300), (32, 40, 400)])
+@pytest.mark.parametrize("degree", [2, 9, 30])
+def test_batched_forward_whatever_the_entry_count_is_said_to_be(gpu, oracle, C, K, B, degree):
+    """the host's entry count decides how many workgroups share a compute unit's LDS, and with it how many entries fit the edge
+    cache: batches whose bins fit it, half fit it and never fit it, with the count said to be right, none, enormous and
+    (the entries without it) unknown: the same bits every time, and the oracle's values.  K = 200: labels"""
+    import torch
+    from graphnn_amd import ops
+    rng = np.random.default_rng(1000 * C + 10 * K + degree)
+    H, Q, L = 16, 3, 2
+    sizes = rng.integers(30, 61, B)
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    N = int(off[-1])
+    per_row = rng.integers(0, 2 * degree + 1, N)
+    a_rp = np.concatenate([[0], np.cumsum(per_row)]).astype(np.int32)
+    graph = np.repeat(np.repeat(np.arange(B), sizes), per_row)
+    a = (a_rp, (off[graph] + (rng.random(graph.size) * sizes[graph]).astype(np.int64)).astype(np.int32),
+         (rng.random(graph.size) / degree).astype(np.float32))
+    s = (off, np.arange(N, dtype=np.int32), np.ones(N, np.float32))
+    w = synth.make_weights(synth.Stream(C + K), K, C, H, Q)
+    label = rng.integers(0, K, N).astype(np.int32)
+    labels = K > 64
+    X = np.eye(K, dtype=np.float32)[label]
+    a_d, s_d = _csr_t(a, gpu), _csr_t(s, gpu)
+    wts = [_t(m, gpu) for m in (w.W_n2l, w.W_conv, w.W_h1, w.W_h2)]
+    x = _t(label if labels else X, gpu)
+    run = (ops.s2v_forward_batched_labels if labels else ops.s2v_forward_batched)
+    keys = ("msg", "h_final", "pool", "hidden", "logits", "probs", "pred")
+    bufs = run(a_d, s_d, x, *wts, L, 60)
+    got = {k: _n(getattr(bufs, k)) for k in keys}
+    assert int(_n(bufs.status)[0]) == 0
+    sized = getattr(ops._bound(), "s2v_forward_batched_labels_sized_f32" if labels else "s2v_forward_batched_sized_f32")
+    plain = getattr(ops._lib(), "gnnhip_s2v_forward_batched_labels_f32" if labels else "gnnhip_s2v_forward_batched_f32")
+    for count in (0, 2 ** 31 - 1, None):
+        o = ops.BatchedBuffers(N, B, C, H, Q, gpu)
+        args = [*a_d, *s_d, x, *wts, o.msg, o.h_final, o.pool, o.hidden, o.logits, o.probs, o.pred, o.status]
+        if count is not None:
+            sized(N, B, K, C, H, Q, L, 60, count, *args)
+        else:
+            assert plain(N, B, K, C, H, Q, L, 60, *[ctypes.c_void_p(t.data_ptr()) for t in args], ops._stream()) == 0
+        torch.cuda.synchronize()
+        for k in keys:
+            assert np.array_equal(_n(getattr(o, k)), got[k]), (count, k)
+    want = _forward_want(oracle, a, s, X, w, L)
+    _assert_forward_parity({k: got[k] for k in keys[:-1]}, want, L)
 
 
 def test_packed_batch_refuses_a_graph_larger_than_a_bin(gpu, oracle):
