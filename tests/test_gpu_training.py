@@ -168,6 +168,57 @@ def test_level_of_any_hidden_size_both_directions(gpu, oracle, C, N):
     assert np.array_equal(_n(h0), np.maximum(_n(m), 0))
 
 
+@pytest.mark.parametrize("C", [66, 100, 129, 150, 255])
+def test_level_of_wide_odd_hidden_sizes_with_long_rows(gpu, C):
+    """hidden sizes without a kernel of their own past 64 columns, from the row count on at which the balanced pass sums the rows
+    of more than 64 entries (one chunk, several chunks, the first and the last row of a tile and of the matrix): forward,
+    backward, with a plan, and reading its input through ReLU as a forward's first level does"""
+    import torch
+    from graphnn_amd import ops
+    rng = np.random.default_rng(C)
+    N = 32_768 + 37
+    lens = rng.integers(0, 6, N)
+    for r, n in ((0, 65), (63, 64), (64, 2048), (700, 2049), (701, 9000), (N // 2, 300), (N - 1, 4500)):
+        lens[r] = n
+    rp = np.zeros(N + 1, np.int32); np.cumsum(lens, out=rp[1:])
+    ci = rng.integers(0, N, rp[-1]).astype(np.int32)
+    v = (rng.random(rp[-1]) * 0.5).astype(np.float32)
+    gen = torch.Generator(device=gpu).manual_seed(C)
+    x = torch.rand(N, C, generator=gen, device=gpu) - 0.25
+    W = torch.randn(C, C, generator=gen, device=gpu) * 0.1
+    msg = torch.randn(N, C, generator=gen, device=gpu)
+    A = [_t(a, gpu) for a in (rp, ci, v)]
+    A64 = torch.sparse_csr_tensor(A[0].long(), A[1].long(), A[2].double(), (N, N))
+    # a chunk of 2,048 entries is summed in order and the chunks after it, then C products: an fp32 sum of t terms is within t 2^-24 of
+    # the sum of their magnitudes, and nothing near that far
+    bound = (2048 + 5 + C) * 2.0 ** -24
+
+    def close(got, left, right, extra=None, mask=None):
+        want, terms = left[0] @ right, left[1] @ right.abs()
+        if extra is not None:
+            want, terms = (want + extra).clamp(min=0), terms + extra.abs()
+        if mask is not None:
+            want = want * mask
+        assert bool(((got.double() - want).abs() <= bound * terms).all())
+
+    agg = (A64 @ x.double(), A64 @ x.double().abs())
+    got = ops.s2v_level(*A, x, W, msg)
+    close(got, agg, W.double(), msg.double())
+    with ops.CsrPlan(*A, N, N) as plan:
+        assert torch.equal(plan.level(x, W, msg), got)
+    acc = msg.clone()
+    u, g = ops.s2v_level_backward(*A, x, W, gate_h=msg, acc=acc)
+    assert bool(((u.double() - agg[0]).abs() <= bound * agg[1]).all())
+    close(g, agg, W.double().T.contiguous(), mask=(msg > 0).double())
+    assert torch.equal(acc, msg + g)
+    Wn = torch.randn(5, C, generator=gen, device=gpu)
+    X = torch.rand(N, 5, generator=gen, device=gpu)
+    S = (torch.tensor([0, N], device=gpu).int(), torch.arange(N, device=gpu).int(), torch.ones(N, device=gpu))
+    bufs = ops.s2v_forward(A, S, X, Wn, W, torch.zeros(C, 4, device=gpu), torch.zeros(4, 2, device=gpu), 1)
+    h0 = A64 @ bufs.msg.clamp(min=0).double()
+    close(bufs.h_final, (h0, h0), W.double(), bufs.msg.double())
+
+
 @pytest.mark.parametrize("C", [128, 256])
 @pytest.mark.parametrize("nnz", [0, 3, 6])
 def test_level_backward_wide_with_hardly_any_entries(gpu, oracle, C, nnz):
