@@ -572,7 +572,9 @@ int launch_level_stream_pieces(int N, const float* W, const float* msg, const fl
     constexpr int kMinW = 4;
     // 1,009 workgroups, a prime: on R-MAT matrices the rows of many pieces are those whose index has few bits
     // set, and a power-of-two stride between a wavefront's tiles would give all of them to the
-    // same wavefronts (4M rows, C = 64: 1,024 workgroups 828 us, 1,023 669, 1,009 605).
+    // same wavefronts (4M rows, C = 64: 1,024 workgroups 828 us, 1,023 669, 1,009 605).  Without such a pattern the count does not
+    // matter: the same graphs with their nodes renumbered at random, a forward of three levels, 1,009 workgroups against 1,024:
+    // 300,001 rows 478 us / 477, 1M 1,934 / 1,925, 4M 8,049 / 8,028.
     const long long resident = (long long)kNumCU * kMinW - 15;
     if (blocks > resident) blocks = resident;
     hipLaunchKernelGGL((s2v_level_stream_kernel<C, true, C == 64, kMinW, false, false, false, true>), dim3((unsigned)blocks), dim3(kBlock), 0, s,
