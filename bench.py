@@ -175,7 +175,7 @@ def time_gather_ceiling(dev, m=1_000_000, per=10, d=128):
     t = _event_median_ms(lambda: ops.spmm(rp, ci, v, X, m, out=Y), 20, 3)
     assert float(Y[12345, 7]) == float(per), "gather-ceiling product is wrong"
     nbytes = 4 * (m + 1) + 8 * k + 4 * k * d + 4 * m * d
-    return {"kernel": "spmm_rowgroup_kernel<4,1>", "workload": "%d rows x %d entries, %d distinct columns, width %d" % (m, per, k, d),
+    return {"kernel": "spmm_rowgroup_kernel<ColsWide,1>", "workload": "%d rows x %d entries, %d distinct columns, width %d" % (m, per, k, d),
             "bytes": nbytes, "median_ms": t["median_ms"], "GBps": nbytes / (t["median_ms"] * 1e-3) / 1e9}
 
 
@@ -197,7 +197,7 @@ def time_cached_gather_ceiling(dev, m=1_000_000, per=10, d=128, k=393_216):
     t = _event_median_ms(lambda: ops.spmm(rp, ci, v, X, m, out=Y), 20, 3)
     assert float(Y[12345, 7]) == float(per), "cached-gather product is wrong"
     nbytes = 4 * (m + 1) + 8 * m * per + 4 * m * per * d + 4 * m * d
-    return {"kernel": "spmm_rowgroup_kernel<4,1>", "workload": "%d rows x %d entries, uniform random over %d columns (operand %.0f MB), width %d"
+    return {"kernel": "spmm_rowgroup_kernel<ColsWide,1>", "workload": "%d rows x %d entries, uniform random over %d columns (operand %.0f MB), width %d"
                                                                % (m, per, k, k * d * 4 / 1e6, d),
             "bytes_gathered_and_written": nbytes, "median_ms": t["median_ms"], "GBps": nbytes / (t["median_ms"] * 1e-3) / 1e9}
 
@@ -241,7 +241,8 @@ def _event_ms(fn, reps, warmup=2):
 
 
 def time_level_cfg4(dev):
-    """One fused level at configuration 4 (10,000 graphs, hidden 256): the FP32 matrix-core kernel."""
+    """One fused level at configuration 4 (10,000 graphs, hidden 256): as the inference forward runs it (bf16 pieces on the matrix
+    cores; from forwards of all levels and of one) and as a training forward does (the level entry, FP32 matrix cores)."""
     import torch
     from graphnn_amd import batching, ops, synth
     batch, w, cfg = synth.make_config(4)
@@ -262,6 +263,7 @@ def time_level_cfg4(dev):
     bufs = ops.ForwardBuffers(N, B, C, H, Q, dev)
     ms_ro = _event_ms(lambda: ops.s2v_readout(*s_d, out, W1, W2, B), 20)
     ms_fw = _event_ms(lambda: ops.s2v_forward(a_d, s_d, X, Wn, Wc, W1, W2, L, bufs=bufs), 20)
+    ms_inf = (ms_fw - _event_ms(lambda: ops.s2v_forward(a_d, s_d, X, Wn, Wc, W1, W2, 1, bufs=bufs), 20)) / (L - 1)
     # the other reading of the configuration's text ("~660k undirected edges" on ~300k nodes = 1.32M entries, mean degree 4.4;
     # the generator rule shared with configurations 1 and 2 gives 1.1 n undirected edges = mean degree 2.2)
     batch2, _, _ = synth.make_config(4, edge_factor=2.2)
@@ -278,7 +280,9 @@ def time_level_cfg4(dev):
              "frac": flops2 / (ms2 * 1e-3) / 1e12 / FP32_MFMA_PEAK_TFLOPS, "forward_ms": ms_fw2}
     return {"workload": "configuration 4: one level, %d nodes, %d entries, hidden %d" % (N, E, C),
             "variant_660k_undirected_edges": dense,
-            "kernel": "s2v_level_wide_kernel<256,8,false,64,false>", "avg_ms": ms, "flops": flops,
+            "inference_level": {"kernel": "s2v_level_split_kernel<256,8,false,32,false>", "avg_ms": ms_inf, "flops": flops,
+                                "bytes": level_algorithmic_bytes(N, E, C)},
+            "kernel": "s2v_level_wide_kernel<256,8,false,64>", "avg_ms": ms, "flops": flops,
             "readout": {"avg_ms": ms_ro, "kernel": "s2v_readout_tile_kernel<256>", "graphs": B,
                         "algorithmic_GBps": (4.0 * N * C + 8.0 * N + 4.0 * B * (C + H + 2 * Q) + 4.0 * (C * H + H * Q)) / (ms_ro * 1e-3) / 1e9},
             "forward": {"avg_ms": ms_fw, "levels": L, "graphs_per_s": B / (ms_fw * 1e-3)},
@@ -312,7 +316,7 @@ def time_large_batch(dev, B=30000):
     gb = lambda nbytes, ms: nbytes / (ms * 1e-3) / 1e9
     return {"workload": "%d graphs of the configuration-2 distribution: %d nodes, %d entries, hidden %d, %d levels" % (B, N, E, C, L),
             "input": {"avg_ms": ms_in, "algorithmic_GBps": gb(4.0 * N * (K + 2 * C) + 4.0 * K * C, ms_in)},
-            "level": {"avg_ms": ms_lv, "kernel": "s2v_level_stream_kernel<64,false,true,3>",
+            "level": {"avg_ms": ms_lv, "kernel": "s2v_level_stream_kernel<64,false,true,3,...>",
                       "algorithmic_GBps": gb(level_algorithmic_bytes(N, E, C), ms_lv)},
             "readout": {"avg_ms": ms_ro, "kernel": "s2v_readout_wave_kernel<64>",
                         "algorithmic_GBps": gb(4.0 * N * C + 8.0 * N + 4.0 * B * (C + H + 2 * Q), ms_ro)},
@@ -521,8 +525,8 @@ CFG5_TRAFFIC_SOURCE = ("constant: FETCH_SIZE x 2.000 + WRITE_SIZE x 1.000 summed
 
 def kernel_rooflines(dev, forwards=None):
     """The other kernels of the path at the sizes they are built for, each against the roofline that bounds
-    it: the hidden-256 level of configuration 4 against the FP32 matrix peak, the configuration-5 kernels
-    (R-MAT, 4.2M rows) against HBM.  achieved = algorithmic bytes (or flops) per launch / HIP-event time."""
+    it: the hidden-256 level of configuration 4 as the inference forward runs it against HBM and as a training forward
+    does against the FP32 matrix peak, the configuration-5 kernels (R-MAT, 4.2M rows) against HBM.  achieved = algorithmic bytes (or flops) per launch / HIP-event time."""
     def hbm(kernel, workload, nbytes, ms, **more):
         gbs = nbytes / (ms * 1e-3) / 1e9
         d = {"kernel": kernel, "workload": workload, "bound": "hbm", "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
@@ -530,7 +534,8 @@ def kernel_rooflines(dev, forwards=None):
         d.update(more)
         return d
     c4 = time_level_cfg4(dev)
-    r4 = dict(c4["roofline"], kernel=c4["kernel"], workload=c4["workload"], avg_ms=c4["avg_ms"], flops=c4["flops"],
+    i4 = c4["inference_level"]
+    r4 = dict(c4["roofline"], kernel=c4["kernel"], workload=c4["workload"] + " (training forward)", avg_ms=c4["avg_ms"], flops=c4["flops"],
               algorithmic_GBps=c4["algorithmic_GBps"], traffic=None, variant_660k_undirected_edges=c4["variant_660k_undirected_edges"])
     c5 = time_cfg5(dev)
     N, E, C, B = c5["shape"]
@@ -541,26 +546,27 @@ def kernel_rooflines(dev, forwards=None):
         forwards["one_launch_by_graphs"] = time_one_launch_by_graphs(dev)
         forwards["hidden_128"] = time_forward_hidden128(dev)
     return [
+        hbm(i4["kernel"], c4["workload"] + " (inference forward)", i4["bytes"], i4["avg_ms"], flops=i4["flops"]),
         r4,
-        hbm("plan of the column-ordered pieces + piece_sum_kernel<4,1> + piece_combine_kernel<4,1> (sums of a row's pieces) + "
-            "s2v_level_stream_kernel<64,true,...> (contraction over the summed rows)", w5 + ": one level, plan included",
+        hbm("plan of the column-ordered pieces + piece_sum_kernel<ColsWide,1> + s2v_level_stream_kernel<64,true,...,PIECES> (puts the "
+            "rows of several pieces together and contracts)", w5 + ": one level, plan included",
             level_algorithmic_bytes(N, E, C), c5["level"]["avg_ms"], gather_GBps=c5["level"]["gather_GBps"],
             traffic=CFG5_TRAFFIC["level"], traffic_source=CFG5_TRAFFIC_SOURCE),
-        hbm("plan of the column-ordered pieces + piece_sum_kernel<4,1> + piece_combine_kernel<4,1>", w5 + ": SpMM A*h, plan included",
+        hbm("plan of the column-ordered pieces + piece_sum_kernel<ColsWide,1> + piece_combine_kernel<ColsWide,1>", w5 + ": SpMM A*h, plan included",
             spmm_algorithmic_bytes(N, N, E, C), c5["spmm"]["avg_ms"], gather_GBps=c5["spmm"]["gather_GBps"],
             traffic=CFG5_TRAFFIC["spmm"], traffic_source=CFG5_TRAFFIC_SOURCE),
-        hbm("piece_sum_kernel<4,1> + hub_partial_kernel<4,1> + piece_combine_kernel<4,1> + s2v_level_stream_kernel<64,true,...>",
+        hbm("piece_sum_kernel<ColsWide,1> + hub_partial_kernel<ColsWide,1> + s2v_level_stream_kernel<64,true,...,PIECES>",
             w5 + ": one level with the caller's plan (gnnhip_s2v_level_planned_f32)",
             level_algorithmic_bytes(N, E, C), c5["level_planned"]["avg_ms"], traffic=CFG5_TRAFFIC["level_planned"],
             traffic_source=CFG5_TRAFFIC_SOURCE),
-        hbm("piece_sum_kernel<4,1> + hub_partial_kernel<4,1> + piece_combine_kernel<4,1>",
+        hbm("piece_sum_kernel<ColsWide,1> + hub_partial_kernel<ColsWide,1> + piece_combine_kernel<ColsWide,1>",
             w5 + ": SpMM A*h with the caller's plan (gnnhip_spmm_csr_planned_f32)",
             spmm_algorithmic_bytes(N, N, E, C), c5["spmm_planned"]["avg_ms"], traffic=CFG5_TRAFFIC["spmm_planned"],
             traffic_source=CFG5_TRAFFIC_SOURCE),
         hbm("sgemm_skinny_rows_kernel<1>", w5 + ": node scores h*w", 4 * N * (C + 1), c5["score"]["avg_ms"]),
         hbm("jagged_softmax_fused_kernel", w5 + ": jagged softmax over %d segments of 1024" % B,
             8 * N + 4 * B, c5["jagged_softmax"]["avg_ms"]),
-        hbm("spmm_rowgroup_kernel<4,1>", w5 + ": sum-pool S*h", 4 * N * C + 8 * N + 4 * (B + 1) + 4 * B * C, c5["sum_pool"]["avg_ms"]),
+        hbm("spmm_rowgroup_kernel<ColsWide,1>", w5 + ": sum-pool S*h", 4 * N * C + 8 * N + 4 * (B + 1) + 4 * B * C, c5["sum_pool"]["avg_ms"]),
     ]
 
 
@@ -840,10 +846,10 @@ def main():
                                   "; graph sizes right-skewed with mean ~30 (10 + min(100, floor(-20 ln(1-u))))"),
                    "graphs": batch.num_graphs, "nodes": batch.num_nodes, "edges": batch.num_edges},
         "nodes_per_s": batch.num_nodes / sec,
-        "route": "graph-resident forward, one launch (gnnhip_s2v_forward_batched_f32)",
+        "route": "graph-resident forward, one launch (gnnhip_s2v_forward_batched_sized_f32)",
         "label_input_route": {"graphs_per_s": batch.num_graphs / sec_labels, "ms_per_step": sec_labels * 1e3,
                               "device_ms_per_step": dev_ms["graph_resident_labels"]["median_ms"],
-                              "what": "gnnhip_s2v_forward_batched_labels_f32: the same launch fed one int label per node "
+                              "what": "gnnhip_s2v_forward_batched_labels_sized_f32: the same launch fed one int label per node "
                                       "instead of the one-hot matrix X (bit-identical outputs); `value` keeps the "
                                       "reference's dense X"},
         "four_batches_in_flight": {"graphs_per_s": batch.num_graphs / sec_pipe, "ms_per_step": sec_pipe * 1e3, "streams": 4,
@@ -871,11 +877,11 @@ def main():
         out["roofline"] = {
             "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-            "traffic_source": "constant: FETCH_SIZE x 2.000 + WRITE_SIZE x 1.000 of spmm_rowgroup_kernel<4,1> from the rocprofv3 "
+            "traffic_source": "constant: FETCH_SIZE x 2.000 + WRITE_SIZE x 1.000 of spmm_rowgroup_kernel<ColsWide,1> from the rocprofv3 "
                               "--pmc runs summarised in profiles/spmm_cfg3_fetch_write_and_hbm_ceilings.md (not re-measured in this run). "
                               "These counters count what the L2 asks of the fabric; the 256 MB memory-side cache sits behind that "
                               "point and no counter this profiler exposes tells its hits from HBM reads",
-            "kernel": "spmm_rowgroup_kernel<4,1>",
+            "kernel": "spmm_rowgroup_kernel<ColsWide,1>",
             "workload": "configuration 3: CSR SpMM, %d rows, %d entries%s, width %d"
                         % (n, nnz, " (exactly 10 per row, --regular)" if args.regular else "", d),
             "algorithmic_bytes": bytes_alg, "avg_ms": med_ms, "median_ms": med_ms, "min_ms": ev["min_ms"], "mean_ms": ev["mean_ms"],
