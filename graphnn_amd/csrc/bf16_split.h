@@ -13,7 +13,7 @@
 //
 // The ends of the range.  The last bits of a number below 2^-110 lie under the smallest bf16, and near the top a correction
 // can overflow to the infinity of the other sign.  So operands are scaled before they are split: by 2^16 where everything
-// that shares the scale (a row, a group of columns of W, a stage of rows) is below 2^38, which every float down to
+// that shares the scale (a row, a column of W, a column over the rows of one workgroup) is below 2^38, which every float down to
 // 2^-149 survives whole, and by 2^-63 where something is larger, so that a sum of 256 products of operands scaled either
 // way stays finite.  (There, what is below 2^-47 loses its last bits, next to a number of 2^38 or more.  Products of two
 // such operands scale back to infinity where they overflow fp32.)  The result is scaled back exactly.  An infinite x is

@@ -5,20 +5,25 @@
 // machinery.
 //
 // On FP32 matrix cores the contraction takes 8,192 cycles of a SIMD per 16 rows at C = 256, twice what the level's HBM
-// traffic takes; six bf16 products take 3,072, which leaves the kernel bound by memory.  The structure is that of
+// traffic takes; six bf16 products take 3,072.  The structure is that of
 // level_wide.hip: a persistent workgroup of eight wavefronts per compute unit, W in registers for the whole launch,
 // the rows of a pass summed into one LDS tile while the matrix cores read the other, one batch of six row loads per
 // 16-row block.  What is different:
 //   * A row is split into its pieces once, by the wavefront that summed it, and lies in LDS as three bf16 planes, its scale
 //     (bf16_split.h) behind them; a column of W has a scale of its own.
 //   * W in pieces takes 192 of a lane's 256 registers at C = 256.  The few fragments that do not fit are read from LDS;
-//     spilled to scratch memory they were reloaded behind the gather's loads, in whose order they had to wait (350 us
-//     per level instead of 240).
+//     spilled to scratch memory they were reloaded behind the gather's loads, in whose order they had to wait (1.45 times the
+//     launch).
 //   * A wavefront whose rows hold more entries than the tops of the remaining blocks can take starts a second batch in
 //     the middle of a block; gathering behind the pass would hold up the other seven.
 //
-// 299,536 nodes, 659,010 entries, C = 256: 370 -> 240 us per level (0.92 GB of activations at 3.8 TB/s), backward
-// 474 -> 425 us (1.84 GB at 4.3 TB/s).
+// 299,536 nodes, 659,010 entries, C = 256, first level apart: 380 (FP32 matrix cores) -> 277 us per level (0.93 GB of
+// activations at 3.4 TB/s), backward 474 -> 428 us (1.85 GB at 4.3 TB/s).  Counted there: 0.64 GB fetched and 0.31 GB written, matrix
+// pipes busy 40 % of the cycles, 3.8 other instructions per matrix instruction of 16 cycles (1.9 of them vector ones, which
+// split the rows, 1.5 scalar ones, which steer the gather), no bank conflicts: neither memory nor the matrix pipes, but two
+// wavefronts per SIMD, too few to issue past each other's waits, that meet at the barrier of every pass.  Summing the
+// corrections apart from the large products costs 5 % of the launch (265 -> 277) and takes the rms error from 2.2 .. 3.1e-8 of
+// the terms' sum to 1e-8 (FP32 matrix cores: 2.4 .. 2.8e-8).
 //
 // Used by the inference forward and by the backward pass.  The levels of a training forward stay on level_wide.hip:
 // the sign of its outputs decides which gradients pass, so two roundings of the same sum give gradients that differ
@@ -477,7 +482,7 @@ int launch_level_split_t(int N, const int* row_ptr, const int* col_idx, const fl
     if ((unsigned long long)N * C * 4ull >= (1ull << 32)) return GNNHIP_EUNSUPPORTED;   // 32-bit buffer offsets
     constexpr int kTileRows = TR;
     const long long ntiles = ((long long)N + kTileRows - 1) / kTileRows;
-    // workgroups that fit one compute unit together: two at C = 128 (82 registers per lane, 68 KB of LDS each)
+    // workgroups that fit one compute unit together: two at C = 128 (107 registers per lane, 55 KB of LDS each)
     constexpr int kPerCU = (C == 128) ? 2 : 1;
     const long long slots = (long long)kNumCU * kPerCU;
     const long long per = (ntiles + slots - 1) / slots;              // contiguous run of tiles per workgroup

@@ -194,9 +194,9 @@ int gnnhip_gemm_f32(int transA, int transB, int m, int n, int k, float alpha, co
  *      (src/nn/matmul.cpp:35-76, x^T * dy through DTensor<GPU>::MM, src/tensor/gpu_dense_tensor.cu:192-224).
  *      m, n, k, lda, ldb, ldc and the pointer tables A, B, C are HOST arrays of count entries; the matrices are
  *      device memory.  Every product gives the bits gnnhip_gemm_f32(1, 0, ...) gives for it alone when that
- *      call splits k (few output tiles, k >= 256).  A product with a 128 x 128 or 256 x 256 output and k >= 8192 (the
- *      level weight gradient at hidden 128 / 256) is taken out of the batch and gets the two launches of its own that
- *      the single call gives it (the whole output in one workgroup's registers over a range of k). */
+ *      call splits k (few output tiles, k >= 256).  A product with an output of up to 256 x 256, k >= 8192 and
+ *      m n k >= 2^28 (the weight gradients of large batches) is taken out of the batch and gets the two launches of its own
+ *      that the single call gives it (the whole output in one workgroup's registers over a range of k). */
 int gnnhip_gemm_tn_batch_f32(int count, const int* m, const int* n, const int* k, const float* const* A, const int* lda,
                              const float* const* B, const int* ldb, float alpha, float beta, float* const* C, const int* ldc,
                              void* stream);
@@ -285,7 +285,7 @@ int gnnhip_s2v_forward_planned_f32(void* a_plan, int B, int K, int C, int H, int
  *      is then the bin size where that is larger than max_graph_nodes.  Node outputs keep their
  *      bits, graph outputs agree with the unpacked ones to rounding.
  *      Returns GNNHIP_EUNSUPPORTED (nothing launched) for shapes it does not cover
- *      (hidden not in {16,32,64}, more than 64 label types, graph too large for LDS). */
+ *      (hidden not in {16,32,64,128}, more than 64 feature columns, graph too large for LDS). */
 int gnnhip_s2v_forward_batched_f32(int N, int B, int K, int C, int H, int Q, int L, int max_graph_nodes,
                                    const int* a_row_ptr, const int* a_col_idx, const float* a_val,
                                    const int* s_row_ptr, const int* s_col_idx, const float* s_val,
@@ -486,8 +486,10 @@ int gnnhip_s2v_grad_gate_f32(size_t n, const float* h, const float* g, float* dz
  *      past that gate (g_prev where h_prev > 0, else 0: ReLUDeriv, src/nn/relu.cu:18-37), ready to be the dz of the
  *      level below.  acc (may be NULL): acc += g_prev as stored (the gradient ElewiseAdd::Backward hands to msg,
  *      src/nn/elewise_add.cpp:35-52, summed over the levels).
- *      One launch at C = 16, 32, 64 and at C = 128, 256 (N * C * 4 < 4 GiB); other widths, and matrices of 32,768 rows
- *      and more with 12 entries per row and more, run SpMM, GEMM and gate one after the other. */
+ *      One launch at C = 16, 32, 64, 128 and 256 (N * C * 4 < 4 GiB, tensors 16-byte aligned) and at any other
+ *      4 <= C <= 256.  SpMM, GEMM and gate run one after the other at C < 4 and C > 256, and on matrices that the SpMM
+ *      cuts by entries: from 32,768 rows and 12 entries per row on at C >= 128 and at the other widths without a kernel of their
+ *      own, below 32,768 rows from 256 entries per row on at those other widths. */
 int gnnhip_s2v_level_backward_f32(int N, int C, int nnz, const int* t_row_ptr, const int* t_col_idx, const float* t_val,
                                   const float* dz, const float* W, float* u, float* g_prev, const float* gate_h, float* acc,
                                   void* stream);
