@@ -514,9 +514,9 @@ def time_cfg5(dev, scale=22):
 
 # Bytes the L2 exchanges with the fabric per call on configuration 5 (FETCH_SIZE x 2.000 + WRITE_SIZE x 1.000 summed over the
 # launches of one call; rocprofv3 --pmc runs summarised in profiles/spmm_pieces_cfg5_fetch_write.md):
-#   sums 8.48 + 0.94, balanced pass over rows of many pieces 0.36 + 0.01, combining pass 0.24 + 0.63 (SpMM: zeros for the
-#   empty rows) or 0.24 + 0.07 (level: empty rows skipped), contraction 1.62 + 1.07, plan 2.60 + 1.34
-CFG5_TRAFFIC = {"spmm_planned": 10_658_000_000, "level_planned": 12_793_000_000, "plan": 3_940_000_000}
+#   sums 8.47 + 0.94, balanced pass over rows of many pieces 0.31 + 0.01, then for the SpMM the combining pass 0.23 + 0.63
+#   (zeros for the empty rows), for the level the contraction 1.80 + 1.08 (empty rows skipped); plan 2.62 + 1.30
+CFG5_TRAFFIC = {"spmm_planned": 10_592_000_000, "level_planned": 12_614_000_000, "plan": 3_922_000_000}
 CFG5_TRAFFIC["spmm"] = CFG5_TRAFFIC["spmm_planned"] + CFG5_TRAFFIC["plan"]
 CFG5_TRAFFIC["level"] = CFG5_TRAFFIC["level_planned"] + CFG5_TRAFFIC["plan"]
 CFG5_TRAFFIC_SOURCE = ("constant: FETCH_SIZE x 2.000 + WRITE_SIZE x 1.000 summed over the launches of one call, from the rocprofv3 "
