@@ -14,6 +14,9 @@
 // so such products are split along k from k = 256:
 // every workgroup takes a range of k, writes its partial tile to scratch, and a second kernel adds the
 // partial tiles in range order (deterministic) and applies alpha and beta.
+#include <algorithm>
+#include <limits.h>
+
 #include "columns.h"
 
 namespace gnnhip {
@@ -23,8 +26,7 @@ constexpr int BM = 64, BN = 64, BK = 16, kBlock = 256;
 
 // One 64 x 64 output tile (tile_x, tile_y) over k in [k_lo, k_hi).  part != nullptr: the raw sums go to
 // part[m][n]; otherwise the tile finishes C itself.
-// AHEAD: steps whose elements are under way (8 registers each).
-template <bool TA, bool TB, int AHEAD>
+template <bool TA, bool TB>
 __device__ __forceinline__ void sgemm_tile_body(
     int m, int n, float alpha, const float* __restrict__ A, int lda,
     const float* __restrict__ B, int ldb, float beta, float* C, int ldc, int k_lo, int k_hi, float* __restrict__ part,
@@ -48,10 +50,10 @@ __device__ __forceinline__ void sgemm_tile_body(
 #pragma unroll
     for (int jb = 0; jb < BN / 16; ++jb) acc[jb] = mfma_f4{0.f, 0.f, 0.f, 0.f};
 
-    // each lane moves 4 elements of each tile; the elements of AHEAD steps on are requested before the
-    // products of a step are formed, so a step costs the longer of the two instead of their sum
-    float ra[AHEAD][4], rb[AHEAD][4];
-    auto fetch = [&](int k0, float (&ra)[4], float (&rb)[4]) {
+    // each lane moves 4 elements of each tile; the elements of the next step are requested before the products of this one are
+    // formed, so a step costs the longer of the two instead of their sum
+    float ra[4], rb[4];
+    auto fetch = [&](int k0) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int idx = tid + e * kBlock;        // 0 .. 1023
@@ -78,33 +80,27 @@ __device__ __forceinline__ void sgemm_tile_body(
             }
         }
     };
+    fetch(k_lo);
+    for (int k0 = k_lo; k0 < k_hi; k0 += BK) {
 #pragma unroll
-    for (int d = 0; d < AHEAD; ++d) if (d == 0 || k_lo + d * BK < k_hi) fetch(k_lo + d * BK, ra[d], rb[d]);
-    for (int kb = k_lo; kb < k_hi; kb += AHEAD * BK) {
-#pragma unroll
-        for (int d = 0; d < AHEAD; ++d) {
-            const int k0 = kb + d * BK;
-            if (AHEAD > 1 && k0 >= k_hi) break;                // uniform
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int idx = tid + e * kBlock;
-                if (TA) As[idx & (BM - 1)][idx >> 6] = ra[d][e]; else As[idx >> 4][idx & (BK - 1)] = ra[d][e];
-                if (TB) Bs[idx >> 4][idx & (BK - 1)] = rb[d][e]; else Bs[idx & (BN - 1)][idx >> 6] = rb[d][e];
-            }
-            __syncthreads();
-            if (k0 + AHEAD * BK < k_hi) fetch(k0 + AHEAD * BK, ra[d], rb[d]);
-            // lane (q, t): k = 4 q + s at instruction s of the step
-            const float4 a = *reinterpret_cast<const float4*>(&As[wave * 16 + t][4 * q]);
-#pragma unroll
-            for (int jb = 0; jb < BN / 16; ++jb) {
-                const float4 b = *reinterpret_cast<const float4*>(&Bs[jb * 16 + t][4 * q]);
-                acc[jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.x, a.x, acc[jb], 0, 0, 0);
-                acc[jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.y, a.y, acc[jb], 0, 0, 0);
-                acc[jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.z, a.z, acc[jb], 0, 0, 0);
-                acc[jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.w, a.w, acc[jb], 0, 0, 0);
-            }
-            __syncthreads();
+        for (int e = 0; e < 4; ++e) {
+            const int idx = tid + e * kBlock;
+            if (TA) As[idx & (BM - 1)][idx >> 6] = ra[e]; else As[idx >> 4][idx & (BK - 1)] = ra[e];
+            if (TB) Bs[idx >> 4][idx & (BK - 1)] = rb[e]; else Bs[idx & (BN - 1)][idx >> 6] = rb[e];
         }
+        __syncthreads();
+        if (k0 + BK < k_hi) fetch(k0 + BK);
+        // lane (q, t): k = 4 q + s at instruction s of the step
+        const float4 a = *reinterpret_cast<const float4*>(&As[wave * 16 + t][4 * q]);
+#pragma unroll
+        for (int jb = 0; jb < BN / 16; ++jb) {
+            const float4 b = *reinterpret_cast<const float4*>(&Bs[jb * 16 + t][4 * q]);
+            acc[jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.x, a.x, acc[jb], 0, 0, 0);
+            acc[jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.y, a.y, acc[jb], 0, 0, 0);
+            acc[jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.z, a.z, acc[jb], 0, 0, 0);
+            acc[jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.w, a.w, acc[jb], 0, 0, 0);
+        }
+        __syncthreads();
     }
 
     // lane (q, t) holds out[row0 + 16 wave + t][col0 + 16 jb + 4 q + i], i = 0..3
@@ -137,76 +133,230 @@ __global__ __launch_bounds__(kBlock) void sgemm_tile_kernel(
 {
     const int k_lo = partial ? (int)blockIdx.z * k_chunk : 0;
     const int k_hi = partial ? min(k, k_lo + k_chunk) : k;
-    sgemm_tile_body<TA, TB, 1>(m, n, alpha, A, lda, B, ldb, beta, C, ldc, k_lo, k_hi,
+    sgemm_tile_body<TA, TB>(m, n, alpha, A, lda, B, ldb, beta, C, ldc, k_lo, k_hi,
                             partial ? partial + (size_t)blockIdx.z * m * n : nullptr, (int)blockIdx.x, (int)blockIdx.y);
 }
 
-// Several products C_p = alpha A_p^T B_p + beta C_p in one launch: the weight gradients at the end of a backward
-// pass, each a small output over a long k, none of which fills the GPU alone.  Product p owns the z range
-// [z0[p], z0[p+1]) of the grid, one range of k per z; tiles outside a product's own tile grid leave at once.
+// ---- A^T B: op(A) = A^T with A stored [k][m], B stored [k][n] (weight gradients, alone or several at the end of a backward pass)
+//
+// Four rows of k of either operand are what v_mfma_f32_16x16x4_f32 takes, and both lie in memory as it wants them: lane
+// (q = lane/16, t = lane%16) loads columns 4 t .. 4 t + 3 of row q in one 128-bit word, and word j of all lanes is the
+// operand of the block of columns {4 t + j}.  So a step of four rows is two loads and sixteen matrix instructions for a
+// 64 x 64 tile, without LDS and without a barrier; the four wavefronts of a workgroup take four rows of sixteen each and add
+// up their tiles in wavefront order at the end.  An output tile ends with a lane holding four consecutive columns.
+// What bounds it at the sizes of a training batch is one or two trips to memory, the sum over the wavefronts and the launch: with the
+// sums of the ranges 7,450 nodes x 4 levels at hidden 64 (four products) take 13.5 us, 1,625 x 3 10.0 (LDS tiles and a
+// barrier per sixteen rows: 20.5 and 12.5); 1,000 x 500 over 3,000 rows 57 (128), 2,048^3 178 = 96 TFLOP/s (210).
+// Six steps under way: four take 0.3 to 1 us more where a range is short, eight spill.
+constexpr int kTnWaves = kBlock / kWave;
+constexpr int kTnStep = 4 * kTnWaves;        // rows of k per step of the workgroup
+constexpr int kTnAhead = 6;                  // steps under way
+
+// Output tile (tile_x, tile_y), rows [k_lo, k_hi).  part != nullptr: the sums go to part[m][n]; otherwise the tile finishes C.
+// A tile narrower than 64 moves its last unit of four columns back to end with it (the columns that repeat have the same
+// sums twice, and one owner where C is updated); NA, NB: fewer than four columns of A, of B, read one by one.
+template <bool NA, bool NB>
+__device__ __forceinline__ void tn_tile_body(int m, int n, float alpha, const float* __restrict__ A, int lda, const float* __restrict__ B,
+                                             int ldb, float beta, float* C, int ldc, int k_lo, int k_hi, float* __restrict__ part,
+                                             int tile_x, int tile_y, float4 (&sums)[kTnWaves - 1][4][4][kWave])
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int q = lane >> 4, t = lane & 15;
+    const int wa = min(m - tile_x * BM, BM), wb = min(n - tile_y * BN, BN);          // columns of the operands in this tile
+    auto unit_a = [&](int u) { return NA ? 0 : min(4 * u, wa - 4); };
+    auto unit_b = [&](int u) { return NB ? 0 : min(4 * u, wb - 4); };
+    const float* a_col = A + (size_t)tile_x * BM + unit_a(t);
+    const float* b_col = B + (size_t)tile_y * BN + unit_b(t);
+    auto few = [](const float* p, int w) { return make_float4(p[0], w > 1 ? p[1] : 0.f, w > 2 ? p[2] : 0.f, 0.f); };
+    auto row_a = [&](size_t k) { const float* p = a_col + k * lda; if constexpr (NA) return few(p, wa); else return ColsLoose::load(p); };
+    auto row_b = [&](size_t k) { const float* p = b_col + k * ldb; if constexpr (NB) return few(p, wb); else return ColsLoose::load(p); };
+
+    mfma_f4 acc[4][4];                          // [block of A][block of B]
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = mfma_f4{0.f, 0.f, 0.f, 0.f};
+    auto products = [&](const float4& a4, const float4& b4) {
+        const float a[4] = {a4.x, a4.y, a4.z, a4.w}, b[4] = {b4.x, b4.y, b4.z, b4.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[j], acc[i][j], 0, 0, 0);
+    };
+
+    const int steps = (k_hi - k_lo) / kTnStep;
+    const size_t k0 = (size_t)k_lo + 4 * wave + q;
+    float4 a[kTnAhead], b[kTnAhead];
+#pragma unroll
+    for (int d = 0; d < kTnAhead; ++d)
+        if (d < steps) { a[d] = row_a(k0 + d * kTnStep); b[d] = row_b(k0 + d * kTnStep); }
+    // the rows short of a step: a row past the end is read as zeros (of both operands: 0 times an infinity is none)
+    const int rest = k_lo + steps * kTnStep + 4 * wave;         // this wavefront's first of them
+    float4 al = f4_zero(), bl = f4_zero();
+    if (rest + q < k_hi) { al = row_a((size_t)rest + q); bl = row_b((size_t)rest + q); }
+    int s = 0;
+    for (; s + kTnAhead <= steps; s += kTnAhead) {
+#pragma unroll
+        for (int d = 0; d < kTnAhead; ++d) {
+            products(a[d], b[d]);
+            const int ahead = s + d + kTnAhead;
+            if (ahead < steps) { a[d] = row_a(k0 + (size_t)ahead * kTnStep); b[d] = row_b(k0 + (size_t)ahead * kTnStep); }
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < kTnAhead - 1; ++d)
+        if (s + d < steps) products(a[d], b[d]);
+    if (rest < k_hi) products(al, bl);
+
+    // wavefront w adds up block w of A over the four wavefronts
+    mfma_f4 own[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (i == wave) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) own[j] = acc[i][j];
+        } else {
+            const int slot = wave < i ? wave : wave - 1;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) sums[slot][i][j][lane] = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
+        }
+    }
+    __syncthreads();
+    float out[4][4];                            // [row][column] of this lane
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        float4 v[kTnWaves - 1];
+#pragma unroll
+        for (int w = 0; w < kTnWaves - 1; ++w) v[w] = sums[w][wave][j][lane];
+        mfma_f4 total = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < kTnWaves; ++w) {
+            if (w == wave) total += own[j];
+            else {
+                const float4 x = v[w < wave ? (w < kTnWaves - 1 ? w : 0) : (w > 0 ? w - 1 : 0)];
+                total += mfma_f4{x.x, x.y, x.z, x.w};
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) out[i][j] = total[i];
+    }
+    // out[i][j]: row unit_a(4 q + i) + wave, column unit_b(t) + j of the tile
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int u = 4 * q + i, r = unit_a(u) + wave;
+        if (NA ? u > 0 || wave >= wa : r < 4 * u) continue;                  // a unit past the tile, or a row that an earlier unit has
+        const size_t gi = (size_t)tile_x * BM + r;
+        const int c = unit_b(t), gj = tile_y * BN + c;
+        if (NB ? t > 0 : 4 * t >= wb) continue;
+        if (!NB && part) {
+            ColsLoose::store(part + gi * n + gj, make_float4(out[i][0], out[i][1], out[i][2], out[i][3]));
+            continue;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (NB ? j >= wb : c + j < 4 * t) continue;
+            if (part) { part[gi * n + gj + j] = out[i][j]; continue; }
+            float* dst = C + gi * ldc + gj + j;
+            const float v = alpha * out[i][j];
+            *dst = (beta == 0.f) ? v : v + beta * (*dst);
+        }
+    }
+}
+
+// Several products C_p = alpha A_p^T B_p + beta C_p in one launch.  Product p owns the z range [z0[p], z0[p+1]) of the
+// grid, one range of k per z; tiles outside a product's own tile grid leave at once.
 constexpr int kGemmBatch = 8;
+struct GemmJob {                                // a cache line of the kernel's arguments each
+    const float* A;
+    const float* B;
+    float* C;
+    float* partial;                             // null: one range, finished by the product launch
+    int m, n, k, lda, ldb, ldc, k_chunk, splits;
+};
 struct GemmBatch {
-    const float* A[kGemmBatch];
-    const float* B[kGemmBatch];
-    float* C[kGemmBatch];
-    float* partial[kGemmBatch];
-    int m[kGemmBatch], n[kGemmBatch], k[kGemmBatch], lda[kGemmBatch], ldb[kGemmBatch], ldc[kGemmBatch];
-    int k_chunk[kGemmBatch], z0[kGemmBatch + 1];
+    int z0[kGemmBatch];                         // INT_MAX from `count` on
+    GemmJob job[kGemmBatch];
     int count;
 };
 
-__global__ __launch_bounds__(kBlock) void sgemm_tn_batch_kernel(GemmBatch b)
+__global__ __launch_bounds__(kBlock, 3) void sgemm_tn_batch_kernel(GemmBatch b, float alpha, float beta)
 {
+    __shared__ float4 sums[kTnWaves - 1][4][4][kWave];        // [wavefront other than a block's owner][block of A][block of B][lane]
     int p = 0;
-    while (p + 1 < b.count && (int)blockIdx.z >= b.z0[p + 1]) ++p;
-    const int m = b.m[p], n = b.n[p];
+#pragma unroll
+    for (int i = 1; i < kGemmBatch; ++i) p += (int)blockIdx.z >= b.z0[i];
+    const GemmJob j = b.job[p];
+    const int m = j.m, n = j.n;
     if ((long long)blockIdx.x * BM >= m || (int)blockIdx.y * BN >= n) return;
     const int z = (int)blockIdx.z - b.z0[p];
-    const int k_lo = z * b.k_chunk[p], k_hi = min(b.k[p], k_lo + b.k_chunk[p]);
-    sgemm_tile_body<true, false, 4>(m, n, 1.0f, b.A[p], b.lda[p], b.B[p], b.ldb[p], 0.0f, b.C[p], b.ldc[p], k_lo, k_hi,
-                                 b.partial[p] + (size_t)z * m * n, (int)blockIdx.x, (int)blockIdx.y);
+    const int k_lo = z * j.k_chunk, k_hi = min(j.k, k_lo + j.k_chunk);
+    float* part = j.partial ? j.partial + (size_t)z * m * n : nullptr;
+    const bool na = m - (int)blockIdx.x * BM < 4, nb = n - (int)blockIdx.y * BN < 4;
+#define GNNHIP_TN_BODY(NA, NB) \
+    tn_tile_body<NA, NB>(m, n, alpha, j.A, j.lda, j.B, j.ldb, beta, j.C, j.ldc, k_lo, k_hi, part, (int)blockIdx.x, (int)blockIdx.y, sums)
+    if (!na && !nb) GNNHIP_TN_BODY(false, false);
+    else if (!na) GNNHIP_TN_BODY(false, true);
+    else if (!nb) GNNHIP_TN_BODY(true, false);
+    else GNNHIP_TN_BODY(true, true);
+#undef GNNHIP_TN_BODY
 }
 
-// C = alpha * (sum over z of partial[z]) + beta * C.  A workgroup takes 64 consecutive elements; wavefront w
-// adds the ranges z = w, w + 4, ... (up to sixteen loads in flight per lane) and the four sums are added in
-// wavefront order, so the result is the same on every run.  The additions are in double: with up to 1,024 ranges an fp32
+// C = alpha * (sum over z of partial[z]) + beta * C.  A workgroup takes 64 consecutive elements, four to a lane: group g of
+// sixteen lanes adds the ranges z = g, g + 16, ... (up to eight 128-bit loads in flight per lane) and the sixteen sums are added in group order, so
+// the result is the same on every run.  The additions are in double: with up to 1,024 ranges an fp32
 // sum of theirs had a larger error than the ranges themselves (64 x 64 over 70,000 rows, terms of one sign: rms 9.5e-8 of the
 // sum, 2.5e-8 in double).  The kernel reads memory meanwhile; it takes the same time.
 __device__ __forceinline__ void sgemm_splitk_reduce_body(int m, int n, int splits, float alpha,
                                                          const float* __restrict__ partial, float beta,
                                                          float* C, int ldc)
 {
-    __shared__ double part[kBlock / kWave][kWave];
+    constexpr int kGroups = kBlock / 16, kBatch = 8;
+    __shared__ double part[kGroups][kWave];
     const size_t total = (size_t)m * n;
-    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    constexpr int kWaves = kBlock / kWave;
+    const int tid = threadIdx.x, group = tid >> 4, e = tid & 15;
     for (size_t base = (size_t)blockIdx.x * kWave; base < total; base += (size_t)gridDim.x * kWave) {
-        const size_t idx = base + lane;
-        double sum = 0.0;
-        float* dst = C + (idx / n) * (size_t)ldc + idx % n;
-        const float c_old = (wave == 0 && idx < total && beta != 0.f) ? *dst : 0.f;      // asked for before the sums, not after
-        if (idx < total) {
-            int z = wave;
-            for (; z + 15 * kWaves < splits; z += 16 * kWaves) {
-                float p[16];
-#pragma unroll
-                for (int u = 0; u < 16; ++u) p[u] = partial[(size_t)(z + u * kWaves) * total + idx];
-#pragma unroll
-                for (int u = 0; u < 16; ++u) sum += p[u];
-            }
-            for (; z + 3 * kWaves < splits; z += 4 * kWaves) {
-                const float p0 = partial[(size_t)z * total + idx], p1 = partial[(size_t)(z + kWaves) * total + idx];
-                const float p2 = partial[(size_t)(z + 2 * kWaves) * total + idx], p3 = partial[(size_t)(z + 3 * kWaves) * total + idx];
-                sum += p0; sum += p1; sum += p2; sum += p3;
-            }
-            for (; z < splits; z += kWaves) sum += partial[(size_t)z * total + idx];
+        const int width = (int)min(total - base, (size_t)kWave);
+        const size_t idx = base + tid;
+        float* dst = nullptr;
+        float c_old = 0.f;
+        if (tid < width) {
+            dst = C + (idx / n) * (size_t)ldc + idx % n;
+            if (beta != 0.f) c_old = *dst;                      // asked for before the sums, not after
         }
-        part[wave][lane] = sum;
-        __syncthreads();
-        if (wave == 0 && idx < total) {
-            double t = part[0][lane];
+        if (width >= 4) {
+            // (the last unit is moved back to end with the elements: those that repeat have the same sums twice)
+            const int at = min(4 * e, width - 4);
+            const float* src = partial + (size_t)group * total + base + at;
+            double s[4] = {0.0, 0.0, 0.0, 0.0};
+            auto add = [&](const float4& x) { s[0] += x.x; s[1] += x.y; s[2] += x.z; s[3] += x.w; };
+            const size_t step = (size_t)kGroups * total;
+            int z = group;
+            for (; z + (kBatch - 1) * kGroups < splits; z += kBatch * kGroups, src += kBatch * step) {
+                float4 x[kBatch];
 #pragma unroll
-            for (int w = 1; w < kWaves; ++w) t += part[w][lane];
+                for (int u = 0; u < kBatch; ++u) x[u] = ColsLoose::load(src + u * step);
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u) add(x[u]);
+            }
+            for (; z + kGroups < splits; z += 2 * kGroups, src += 2 * step) {
+                const float4 x0 = ColsLoose::load(src), x1 = ColsLoose::load(src + step);
+                add(x0);
+                add(x1);
+            }
+            if (z < splits) add(ColsLoose::load(src));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) part[group][at + i] = s[i];
+        } else if (e < width) {
+            double s = 0.0;
+            for (int z = group; z < splits; z += kGroups) s += partial[(size_t)z * total + base + e];
+            part[group][e] = s;
+        }
+        __syncthreads();
+        if (tid < width) {
+            double t = part[0][tid];
+#pragma unroll
+            for (int g = 1; g < kGroups; ++g) t += part[g][tid];
             const float r = alpha * (float)t;
             *dst = (beta == 0.f) ? r : r + beta * c_old;
         }
@@ -224,8 +374,8 @@ __global__ __launch_bounds__(kBlock) void sgemm_splitk_reduce_kernel(int m, int 
 // the sums of product blockIdx.y of a batch
 __global__ __launch_bounds__(kBlock) void sgemm_splitk_reduce_batch_kernel(GemmBatch b, float alpha, float beta)
 {
-    const int p = blockIdx.y;
-    sgemm_splitk_reduce_body(b.m[p], b.n[p], b.z0[p + 1] - b.z0[p], alpha, b.partial[p], beta, b.C[p], b.ldc[p]);
+    const GemmJob j = b.job[blockIdx.y];
+    if (j.partial) sgemm_splitk_reduce_body(j.m, j.n, j.splits, alpha, j.partial, beta, j.C, j.ldc);
 }
 
 }  // namespace
@@ -389,6 +539,15 @@ inline long long splitk_chunk(long long tiles, long long k)
     if (chunk < 4 * BK) chunk = 4 * BK;
     return (chunk + BK - 1) / BK * BK;
 }
+// The same for A^T B: a workgroup per CU, two steps of its four wavefronts at least.  (64 x 64 over 60,000 rows: 14.8 us with one,
+// 17.8 with two per CU, whose partial tiles are twice as many, 18.4 with one per two CUs; ranges of at least 128 rows cost
+// batches of up to 7,450 nodes 0.6 to 1.5 us.)
+inline long long tn_chunk(long long tiles, long long k)
+{
+    const long long want = kNumCU / tiles;                                 // tiles <= kNumCU / 4
+    const long long chunk = std::max((k + want - 1) / want, 2ll * kTnStep);
+    return (chunk + kTnStep - 1) / kTnStep * kTnStep;
+}
 
 // count <= kGemmBatch products C_p = alpha A_p^T B_p + beta C_p (A_p stored [k_p, m_p], B_p [k_p, n_p]) in two launches
 int gemm_tn_batch_dispatch(int count, const int* m, const int* n, const int* k, const float* const* A, const int* lda,
@@ -397,7 +556,8 @@ int gemm_tn_batch_dispatch(int count, const int* m, const int* n, const int* k, 
     GemmBatch b;
     b.count = 0;
     size_t floats = 0;
-    unsigned gx = 1, gy = 1, red = 1;
+    unsigned gx = 1, gy = 1, red = 0;
+    constexpr size_t kDirect = ~(size_t)0;
     size_t offset[kGemmBatch];
     int z = 0;
     for (int p = 0; p < count; ++p) {
@@ -409,31 +569,28 @@ int gemm_tn_batch_dispatch(int count, const int* m, const int* n, const int* k, 
             continue;
         }
         const int q = b.count++;
-        b.A[q] = A[p]; b.B[q] = B[p]; b.C[q] = C[p];
-        b.m[q] = m[p]; b.n[q] = n[p]; b.k[q] = k[p];
-        b.lda[q] = lda[p]; b.ldb[q] = ldb[p]; b.ldc[q] = ldc[p];
         const unsigned tx = ceil_div_u((size_t)m[p], BM), ty = ceil_div_u((size_t)n[p], BN);
         const long long tiles = (long long)tx * ty;
         // the rule of the single product, so that a batch gives the bits of its products done one by one
-        long long chunk = (tiles <= kNumCU / 4 && k[p] >= 256) ? splitk_chunk(tiles, k[p]) : (k[p] > 0 ? k[p] : 1);
+        long long chunk = tiles <= kNumCU / 4 && k[p] >= 256 ? tn_chunk(tiles, k[p]) : (k[p] > 0 ? k[p] : 1);
         const int splits = k[p] > 0 ? (int)(((long long)k[p] + chunk - 1) / chunk) : 1;
-        b.k_chunk[q] = (int)chunk;
+        b.job[q] = GemmJob{A[p], B[p], C[p], nullptr, m[p], n[p], k[p], lda[p], ldb[p], ldc[p], (int)chunk, splits};
         b.z0[q] = z;
         z += splits;
-        offset[q] = floats;
-        floats += (size_t)splits * m[p] * n[p];
+        offset[q] = splits > 1 ? floats : kDirect;
+        if (splits > 1) floats += (size_t)splits * m[p] * n[p];
         if (tx > gx) gx = tx;
         if (ty > gy) gy = ty;
-        const unsigned r = ceil_div_u((size_t)m[p] * n[p], kWave) < 2048u ? ceil_div_u((size_t)m[p] * n[p], kWave) : 2048u;
-        if (r > red) red = r;
+        if (splits > 1) red = std::max(red, std::min(ceil_div_u((size_t)m[p] * n[p], kWave), 2048u));
     }
     if (b.count == 0) return GNNHIP_OK;
-    b.z0[b.count] = z;
+    for (int p = b.count; p < kGemmBatch; ++p) b.z0[p] = INT_MAX;
     void* q = nullptr;
-    if (int rc = stream_scratch_slot(s, 2, sizeof(float) * floats, &q)) return rc;
-    for (int p = 0; p < b.count; ++p) b.partial[p] = static_cast<float*>(q) + offset[p];
-    hipLaunchKernelGGL(sgemm_tn_batch_kernel, dim3(gx, gy, (unsigned)z), dim3(kBlock), 0, s, b);
-    hipLaunchKernelGGL(sgemm_splitk_reduce_batch_kernel, dim3(red, (unsigned)b.count), dim3(kBlock), 0, s, b, alpha, beta);
+    if (floats)
+        if (int rc = stream_scratch_slot(s, 2, sizeof(float) * floats, &q)) return rc;
+    for (int p = 0; p < b.count; ++p) b.job[p].partial = offset[p] == kDirect ? nullptr : static_cast<float*>(q) + offset[p];
+    hipLaunchKernelGGL(sgemm_tn_batch_kernel, dim3(gx, gy, (unsigned)z), dim3(kBlock), 0, s, b, alpha, beta);
+    if (red) hipLaunchKernelGGL(sgemm_splitk_reduce_batch_kernel, dim3(red, (unsigned)b.count), dim3(kBlock), 0, s, b, alpha, beta);
     GNNHIP_LAUNCH_CHECK("sgemm_tn_batch");
     return GNNHIP_OK;
 }
@@ -452,9 +609,7 @@ int gemm_dispatch(int transA, int transB, int m, int n, int k, float alpha, cons
         GNNHIP_LAUNCH_CHECK("sgemm_skinny");
         return GNNHIP_OK;
     }
-    if (transA && !transB) {
-        if (int rc = gemm_tn_split_dispatch(m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, s); rc != GNNHIP_EUNSUPPORTED) return rc;
-    }
+    if (transA && !transB) return gemm_tn_batch_dispatch(1, &m, &n, &k, &A, &lda, &B, &ldb, alpha, beta, &C, &ldc, s);
     dim3 grid(ceil_div_u((size_t)m, BM), ceil_div_u((size_t)n, BN));
     dim3 block(kBlock);
     // few output tiles and a long k: split k so that about two workgroups per CU share the work
@@ -474,8 +629,6 @@ int gemm_dispatch(int transA, int transB, int m, int n, int k, float alpha, cons
     }
     if (!transA && !transB)
         hipLaunchKernelGGL((sgemm_tile_kernel<false, false>), grid, block, 0, s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, k_chunk, partial);
-    else if (transA && !transB)
-        hipLaunchKernelGGL((sgemm_tile_kernel<true, false>), grid, block, 0, s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, k_chunk, partial);
     else if (!transA && transB)
         hipLaunchKernelGGL((sgemm_tile_kernel<false, true>), grid, block, 0, s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, k_chunk, partial);
     else

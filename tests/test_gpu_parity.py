@@ -267,6 +267,38 @@ def test_gemm_batch_of_weight_gradient_products(gpu, oracle, alpha, beta):
             assert np.array_equal(_n(got), alone), (k, m, n)
 
 
+@pytest.mark.parametrize("m,n", [(1, 1), (2, 64), (3, 5), (4, 4), (5, 63), (38, 64), (64, 3), (63, 65), (67, 66), (66, 130), (577, 520)])
+@pytest.mark.parametrize("k", [1, 3, 15, 16, 17, 33, 63, 64, 255, 256, 257, 545, 4099])
+def test_transposed_product_at_the_edges_of_its_tiles(gpu, m, n, k):
+    """A^T B around the sizes where its kernel turns: fewer than four columns, units of four that are moved back, one and several
+    64 x 64 tiles, k short of a step of 16 rows, of a wavefront's four rows of it and of the four steps under way, one and
+    several ranges; the operands are the leading columns of wider rows that start at any float, with NaN behind the columns
+    and infinities behind the rows.  Every element within k + 8 roundings of the sum of its terms' magnitudes of float64
+    (one per product and sum, and those of alpha and beta), and the same bits from the batch call"""
+    import torch
+    from graphnn_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(1000 * m + n + k)
+    def operand(cols, pad):
+        rows = torch.full((k + 3, cols + pad), float("nan"), device=gpu)
+        rows[k:] = float("inf")
+        rows[:k, :cols] = torch.randn(k, cols, generator=gen, device=gpu)
+        return rows
+    for pad_a, pad_b, alpha, beta in ((0, 0, 1.0, 0.0), (3, 1, -0.75, 0.5)):
+        A, B = operand(m, pad_a), operand(n, pad_b)
+        if pad_a:                                       # rows that start at odd floats
+            A = torch.cat([torch.full((1,), float("nan"), device=gpu), A.reshape(-1)])[1:].view(k + 3, m + pad_a)
+        out0 = torch.randn(m, n, generator=gen, device=gpu)
+        a64, b64 = A[:k, :m].double(), B[:k, :n].double()
+        want = alpha * (a64.T.contiguous() @ b64) + beta * out0.double()
+        terms = abs(alpha) * (a64.abs().T.contiguous() @ b64.abs()) + abs(beta) * out0.double().abs()
+        got = ops.gemm(A[:k], B[:k], transA=True, alpha=alpha, beta=beta, out=out0.clone(), cols_a=m, cols_b=n)
+        assert bool(((got.double() - want).abs() <= (k + 8) * 2.0 ** -24 * terms).all())
+        if pad_a == 0:
+            batched = out0.clone()
+            ops.gemm_tn_batch([(A[:k], B[:k], batched), (A[:k], B[:k], torch.empty_like(out0))], alpha=alpha, beta=beta)
+            assert torch.equal(batched, got)
+
+
 def test_gemm_reference_test_shape(gpu, oracle):
     """10x20 . (30x20)^T with |delta ASum| <= 1e-4 (test/gpu_tensor_test.cpp:131-149)"""
     from graphnn_amd import ops
