@@ -20,6 +20,9 @@
 // At the sizes of training batches (10^5 to 10^6 pairs) a launch costs about what it does: 659,010 pairs on 299,536
 // rows, both ways, took 36 launches and 206 us with 8-bit digits, one grouping after the other; 9 launches and
 // 114 us now.
+#include <algorithm>
+#include <type_traits>
+
 #include "gnnhip_internal.h"
 
 namespace gnnhip {
@@ -307,7 +310,7 @@ __global__ __launch_bounds__(kBlock) void expand_rows_kernel(int m, const int* _
 
 // ---- small inputs: the whole grouping in one launch ----
 // A batch of a few hundred small graphs is latency, not bandwidth: the dozen launches of the radix passes
-// cost more than the host loop they replace.  One launch of up to 16 workgroups instead.  The rows are cut
+// cost more than the host loop they replace.  One launch of up to 64 workgroups instead.  The rows are cut
 // into as many runs; every workgroup reads ALL keys (they are a few L2 lines per lane) and keeps the pairs
 // of its own run of rows, so no workgroup ever waits for another: the number of keys below its first row,
 // which it counts on the way, is where its part of the result starts.  Between the first read of the keys
@@ -319,24 +322,28 @@ __global__ __launch_bounds__(kBlock) void expand_rows_kernel(int m, const int* _
 //              every row into input order again.  Ascending keys: the pairs of the run are consecutive
 //              and in order already, nothing to place or to order.
 //   order      rows of up to 8 entries: a thread sorts them in registers (a fixed network);
+//              up to 64: a lane of a wavefront holds an entry and counts the smaller ones;
 //              longer rows: a wavefront marks the row's pair indices in a bitmap of its own and reads
 //              the set bits back in ascending order, 64 words at a time (a prefix sum of the
 //              population counts gives every word its first slot)
 //   write      slot after slot, coalesced: payload (and value) of the pair the slot names
-// Global loads are issued sixteen to a thread before the first is used.  The order of the entries is a
+// Keys are read four to a load (where they are not strided), all of a thread's sixteen before the first is used.  What bounds it is
+// the chain of these steps: 16,380 pairs of 7,450 rows take 3 us to read and count, 0.9 to scan, 0.7 to place, 0.7 to order and
+// 1.5 to write, behind the 4 of any launch with much LDS (both ways at once 17.3 -> 11.5 us; 16 workgroups of 1,024 lanes with a
+// key per load before).  More, smaller workgroups shorten every step but the reading (6,175 pairs 11.5 -> 7.8, 60,000 41 -> 23 us);
+// rows of 9 to 64 entries cost 80 to 700 us per 65,000 pairs when each walked a bitmap.  The order of the entries is a
 // pure function of the input, as on the radix route.  Sizes: 4 bytes per row of a run, 2 per pair, one
 // bitmap of n bits (as many as fit, up to one per wavefront) in 160 KB of LDS; at most 65,536 pairs.
 constexpr int kSmallPairs = 1 << 16;
-constexpr int kSmallBlock = 1024;
-constexpr int kSmallWaves = kSmallBlock / kWave;
 constexpr int kSmallShort = 8;
 constexpr int kSmallBatch = 16;
 constexpr int kSmallLdsInts = 160 * 1024 / 4;
 constexpr int kSmallMisc = 48;
-constexpr int kSmallGroups = 16;           // workgroups at most
-constexpr int kSmallRunRows = 256;         // rows per workgroup at least
+constexpr int kSmallGroups = 64;           // workgroups at most, per grouping
+constexpr int kSmallRunRows = 64;          // rows per workgroup at least
 
 struct SmallLayout {
+    int block;                            // lanes per workgroup
     int groups, run;                      // workgroups, rows per workgroup (a multiple of 64)
     int slots, longs, misc, bitmaps;      // offsets in ints (the counters start at 0)
     int words, nbitmaps;                  // words per bitmap, number of bitmaps
@@ -359,7 +366,11 @@ inline bool small_layout(long long rows, long long n, SmallLayout* out)
     l.words = (int)((n + 31) / 32);
     const int room = kSmallLdsInts - l.bitmaps;
     if (room < l.words) return false;
-    l.nbitmaps = room / l.words < kSmallWaves ? room / l.words : kSmallWaves;
+    // the keys in one batch of loads where that can be, four rows of the run per lane at most
+    const long long per_lane = std::max((n + kSmallBatch - 1) / kSmallBatch, run / 4);
+    l.block = per_lane <= 256 ? 256 : per_lane <= 512 ? 512 : 1024;
+    const int waves = l.block / kWave;
+    l.nbitmaps = room / l.words < waves ? room / l.words : waves;
     *out = l;
     return true;
 }
@@ -396,8 +407,10 @@ struct SmallJob {
     int key_stride, payload_stride;
 };
 
-__global__ __launch_bounds__(kSmallBlock) void csr_group_small_kernel(int rows, int n, SmallLayout lay, SmallJob job0, SmallJob job1, int average)
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void csr_group_small_kernel(int rows, int n, SmallLayout lay, SmallJob job0, SmallJob job1, int average)
 {
+    constexpr int kWaves = BLOCK / kWave;
     const bool second = (int)blockIdx.x >= lay.groups;
     const int run_index = (int)blockIdx.x - (second ? lay.groups : 0);
     const int* __restrict__ key = second ? job1.key : job0.key;
@@ -418,39 +431,60 @@ __global__ __launch_bounds__(kSmallBlock) void csr_group_small_kernel(int rows, 
     const int top = rows - 1;
     const int lo = run_index * lay.run, mine = min(lay.run, rows - lo);            // this run: rows lo .. lo + mine - 1
 
-    for (int r = tid; r < mine; r += kSmallBlock) cnt[r] = 0;
+    for (int r = tid; r < mine; r += BLOCK) cnt[r] = 0;
     if (tid < kSmallMisc) misc[tid] = 0;
     __syncthreads();
 
-    // lengths.  Lanes hold consecutive pairs; a run of equal keys (a batch that arrives grouped is nothing
-    // else) is counted by its first lane alone.  The keys of the first batch stay in registers for `place`.
+    // lengths.  A lane takes four consecutive pairs at a time and counts equal neighbours among them together.  The keys of the
+    // first batch stay in registers for `place`.
     bool disorder = false;
     int below = 0;
     int first_keys[kSmallBatch];
-    for (int base0 = 0; base0 < n; base0 += kSmallBlock * kSmallBatch) {       // every lane walks every batch: the ballots need them
-        const int base = base0 + tid;
-        int k[kSmallBatch], before[kSmallBatch];
+    const bool words = key_stride == 1 && (reinterpret_cast<size_t>(key) & 15) == 0;
+    auto pair_of = [&](int base, int u) { return base + ((u / 4) * BLOCK + tid) * 4 + (u & 3); };
+    auto load_keys = [&](int base, int (&k)[kSmallBatch]) {       // clamped; -1 past the last pair
 #pragma unroll
-        for (int u = 0; u < kSmallBatch; ++u) {
-            const int e = base + u * kSmallBlock;
-            k[u] = e < n ? key[(long long)e * key_stride] : 0;
-            before[u] = (e < n && e > 0 && lane == 0) ? key[(long long)(e - 1) * key_stride] : 0;
+        for (int v = 0; v < kSmallBatch / 4; ++v) {
+            const int e = pair_of(base, 4 * v);
+            int4 x = make_int4(-1, -1, -1, -1);
+            if (words && e + 3 < n) {
+                x = *reinterpret_cast<const int4*>(key + e);
+            } else {
+                if (e + 0 < n) x.x = key[(long long)(e + 0) * key_stride];
+                if (e + 1 < n) x.y = key[(long long)(e + 1) * key_stride];
+                if (e + 2 < n) x.z = key[(long long)(e + 2) * key_stride];
+                if (e + 3 < n) x.w = key[(long long)(e + 3) * key_stride];
+            }
+            k[4 * v] = x.x; k[4 * v + 1] = x.y; k[4 * v + 2] = x.z; k[4 * v + 3] = x.w;
         }
 #pragma unroll
-        for (int u = 0; u < kSmallBatch; ++u) {
-            const int e = base + u * kSmallBlock;
-            const int kk = e < n ? min(max(k[u], 0), top) : -1;
-            if (base0 == 0) first_keys[u] = kk;
-            const int left = __shfl_up(kk, 1, kWave);
-            const int prev = lane == 0 ? (e > 0 && e < n ? min(max(before[u], 0), top) : -1) : left;
-            const bool head = lane == 0 || left != kk;
-            const unsigned long long heads = __ballot(head);
-            if (kk >= 0) {
-                disorder |= prev > kk;
-                below += kk < lo;
-                if (head && kk >= lo && kk - lo < mine) {
-                    const unsigned long long later = lane == kWave - 1 ? 0ull : heads >> (lane + 1);
-                    atomicAdd(&cnt[kk - lo], later ? __ffsll((long long)later) : kWave - lane);
+        for (int u = 0; u < kSmallBatch; ++u) k[u] = pair_of(base, u) < n ? min(max(k[u], 0), top) : -1;
+    };
+    for (int base = 0; base < n; base += BLOCK * kSmallBatch) {       // every lane walks every batch: the shuffles need them
+        int k[kSmallBatch], before[kSmallBatch / 4];
+#pragma unroll
+        for (int v = 0; v < kSmallBatch / 4; ++v) {
+            const int e = pair_of(base, 4 * v);
+            before[v] = lane == 0 && e > 0 && e < n ? key[(long long)(e - 1) * key_stride] : -1;
+        }
+        load_keys(base, k);
+#pragma unroll
+        for (int v = 0; v < kSmallBatch / 4; ++v) {
+            const int left = __shfl_up(k[4 * v + 3], 1, kWave);
+            int prev = lane == 0 ? (before[v] < 0 ? before[v] : min(before[v], top)) : left;
+            int run = 1;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int kk = k[4 * v + j];
+                if (base == 0) first_keys[4 * v + j] = kk;
+                disorder |= kk >= 0 && prev > kk;
+                below += kk >= 0 && kk < lo;
+                prev = kk;
+                if (j < 3 && k[4 * v + (j < 3 ? j + 1 : 3)] == kk) {
+                    ++run;
+                } else {
+                    if (kk >= 0 && (unsigned)(kk - lo) < (unsigned)mine) atomicAdd(&cnt[kk - lo], run);
+                    run = 1;
                 }
             }
         }
@@ -461,16 +495,16 @@ __global__ __launch_bounds__(kSmallBlock) void csr_group_small_kernel(int rows, 
     __syncthreads();
 
     // exclusive scan: a wavefront owns a stretch of the run and walks it 64 rows at a time
-    const int seg = ((mine + kSmallWaves - 1) / kSmallWaves + kWave - 1) & ~(kWave - 1);
+    const int seg = ((mine + kWaves - 1) / kWaves + kWave - 1) & ~(kWave - 1);
     const int s0 = min(uwave * seg, mine), s1 = min(s0 + seg, mine);
     int part = 0;
     for (int r = s0 + lane; r < s1; r += kWave) part += cnt[r];
     part = wave_sum_i(part);
     if (lane == 0) misc[2 + uwave] = part;
     __syncthreads();
-    const int upto = wave_inclusive_scan_i(lane < kSmallWaves ? misc[2 + lane] : 0);
-    const int first_slot = wave_sum_i(lane < kSmallWaves ? misc[18 + lane] : 0);      // pairs of the runs before this one
-    const int held = __builtin_amdgcn_readlane(upto, kSmallWaves - 1);                 // pairs of this run
+    const int upto = wave_inclusive_scan_i(lane < kWaves ? misc[2 + lane] : 0);
+    const int first_slot = wave_sum_i(lane < kWaves ? misc[18 + lane] : 0);      // pairs of the runs before this one
+    const int held = __builtin_amdgcn_readlane(upto, kWaves - 1);                 // pairs of this run
     int carry = uwave ? __builtin_amdgcn_readlane(upto, uwave - 1) : 0;
     for (int r = s0 + lane; r - lane < s1; r += kWave) {
         const int c = r < s1 ? cnt[r] : 0;
@@ -480,32 +514,27 @@ __global__ __launch_bounds__(kSmallBlock) void csr_group_small_kernel(int rows, 
     }
     const bool ascending = misc[1] == 0;
     __syncthreads();
-    for (int r = tid; r < mine; r += kSmallBlock) row_ptr[lo + r] = first_slot + cnt[r];
+    for (int r = tid; r < mine; r += BLOCK) row_ptr[lo + r] = first_slot + cnt[r];
     if (lo + mine == rows && tid == 0) row_ptr[rows] = n;
 
     if (!ascending) {
         __syncthreads();                  // the starts are on their way out; the counters turn into cursors
+        auto place = [&](int base, const int (&k)[kSmallBatch]) {
 #pragma unroll
-        for (int u = 0; u < kSmallBatch; ++u) {
-            const int e = tid + u * kSmallBlock, r = first_keys[u] - lo;
-            if (e < n && r >= 0 && r < mine) slots[atomicAdd(&cnt[r], 1)] = (unsigned short)e;
-        }
-        for (int base = tid + kSmallBlock * kSmallBatch; base < n; base += kSmallBlock * kSmallBatch) {
+            for (int u = 0; u < kSmallBatch; ++u) {
+                const int r = k[u] - lo;                  // -1: past the last pair, outside every run
+                if (k[u] >= 0 && (unsigned)r < (unsigned)mine) slots[atomicAdd(&cnt[r], 1)] = (unsigned short)pair_of(base, u);
+            }
+        };
+        place(0, first_keys);
+        for (int base = BLOCK * kSmallBatch; base < n; base += BLOCK * kSmallBatch) {
             int k[kSmallBatch];
-#pragma unroll
-            for (int u = 0; u < kSmallBatch; ++u) {
-                const int e = base + u * kSmallBlock;
-                k[u] = e < n ? key[(long long)e * key_stride] : 0;
-            }
-#pragma unroll
-            for (int u = 0; u < kSmallBatch; ++u) {
-                const int e = base + u * kSmallBlock, r = min(max(k[u], 0), top) - lo;
-                if (e < n && r >= 0 && r < mine) slots[atomicAdd(&cnt[r], 1)] = (unsigned short)e;
-            }
+            load_keys(base, k);
+            place(base, k);
         }
         __syncthreads();                  // cnt[r] is now the end of row r
 
-        for (int r0 = 0; r0 < mine; r0 += kSmallBlock) {
+        for (int r0 = 0; r0 < mine; r0 += BLOCK) {
             const int r = r0 + tid;
             int a = 0, len = 0;
             if (r < mine) {
@@ -550,12 +579,24 @@ __global__ __launch_bounds__(kSmallBlock) void csr_group_small_kernel(int rows, 
         __syncthreads();
 
         const int nlong = misc[0];
+        // up to 64 entries: a lane holds one and counts the smaller ones (the values are distinct)
+        for (int q = uwave; q < nlong; q += kWaves) {
+            const int r = longs[q];
+            const int a = r ? cnt[r - 1] : 0, len = cnt[r] - a;
+            if (len > kWave) continue;
+            const int v = lane < len ? (int)slots[a + lane] : 0;
+            const int ulen = __builtin_amdgcn_readfirstlane(len);
+            int rank = 0;
+            for (int j = 0; j < ulen; ++j) rank += __builtin_amdgcn_readlane(v, j) < v;
+            if (lane < len) slots[a + rank] = (unsigned short)v;
+        }
         if (nlong > 0 && wave < lay.nbitmaps) {
             unsigned* bits = reinterpret_cast<unsigned*>(small_lds + lay.bitmaps) + wave * lay.words;
             for (int i = lane; i < lay.words; i += kWave) bits[i] = 0u;
             for (int q = wave; q < nlong; q += lay.nbitmaps) {
                 const int r = longs[q];
                 const int a = r ? cnt[r - 1] : 0, b = cnt[r];
+                if (b - a <= kWave) continue;
                 int first = 0x7fffffff, last = -1;
                 for (int i = a + lane; i < b; i += kWave) {
                     const int e = slots[i];
@@ -596,24 +637,24 @@ __global__ __launch_bounds__(kSmallBlock) void csr_group_small_kernel(int rows, 
     }
 
     // slot i of this run holds pair e and is entry first_slot + i of the result: out it goes
-    for (int base = tid; base < held; base += kSmallBlock * kSmallBatch) {
+    for (int base = tid; base < held; base += BLOCK * kSmallBatch) {
         int e[kSmallBatch], pay[kSmallBatch], k[kSmallBatch];
         float w[kSmallBatch];
 #pragma unroll
         for (int u = 0; u < kSmallBatch; ++u) {
-            const int i = base + u * kSmallBlock;
+            const int i = base + u * BLOCK;
             e[u] = i < held ? (ascending ? first_slot + i : (int)slots[i]) : 0;
         }
 #pragma unroll
         for (int u = 0; u < kSmallBatch; ++u) {
-            const bool live = base + u * kSmallBlock < held;
+            const bool live = base + u * BLOCK < held;
             pay[u] = live ? payload[(long long)e[u] * payload_stride] : 0;
             w[u] = (live && val_in) ? val_in[e[u]] : 1.0f;
             k[u] = (live && average) ? key[(long long)e[u] * key_stride] : 0;
         }
 #pragma unroll
         for (int u = 0; u < kSmallBatch; ++u) {
-            const int i = base + u * kSmallBlock;
+            const int i = base + u * BLOCK;
             if (i >= held) continue;
             if (average) {
                 const int r = min(max(k[u], 0), top) - lo;
@@ -704,13 +745,20 @@ bool csr_group_small(int rows, long long n, const int* key, int key_stride, cons
 {
     SmallLayout lay;
     if (!small_layout(rows, n, &lay)) return false;
-    static LdsLimit limit;
-    if (limit.raise(reinterpret_cast<const void*>(csr_group_small_kernel), sizeof(int) * kSmallLdsInts) != hipSuccess) return false;
     const SmallJob job0 = {key, payload, val_in, row_ptr, col_idx, val, key_stride, payload_stride};
     const SmallJob job1 = {payload, key, nullptr, t_row_ptr, t_col_idx, t_val, payload_stride, key_stride};
-    hipLaunchKernelGGL(csr_group_small_kernel, dim3(lay.groups * (t_row_ptr ? 2 : 1)), dim3(kSmallBlock),
-                       sizeof(int) * (size_t)(lay.bitmaps + lay.words * lay.nbitmaps), s, rows, (int)n, lay, job0, job1, average);
-    return true;
+    const dim3 grid(lay.groups * (t_row_ptr ? 2 : 1));
+    const size_t lds = sizeof(int) * (size_t)(lay.bitmaps + lay.words * lay.nbitmaps);
+    auto launch = [&](auto block) {
+        constexpr int kSize = decltype(block)::value;
+        static LdsLimit limit;
+        if (limit.raise(reinterpret_cast<const void*>(csr_group_small_kernel<kSize>), sizeof(int) * kSmallLdsInts) != hipSuccess) return false;
+        hipLaunchKernelGGL(csr_group_small_kernel<kSize>, grid, dim3(kSize), lds, s, rows, (int)n, lay, job0, job1, average);
+        return true;
+    };
+    if (lay.block == 256) return launch(std::integral_constant<int, 256>());
+    if (lay.block == 512) return launch(std::integral_constant<int, 512>());
+    return launch(std::integral_constant<int, 1024>());
 }
 
 inline int last_launch_status(const char* what)

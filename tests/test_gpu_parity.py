@@ -2151,6 +2151,38 @@ def test_device_csr_group_of_a_small_batch_in_one_launch(gpu, case):
     assert np.array_equal(_n(rp), want[0]) and np.array_equal(_n(ci), want[1])
 
 
+@pytest.mark.parametrize("n", [3, 4, 255, 4095, 4096, 4097, 8191, 8193, 16_383, 16_385, 33_001, 65_535])
+@pytest.mark.parametrize("rows", [1, 63, 65, 4_097, 50_000, 300_000])
+def test_device_csr_group_at_the_edges_of_its_workgroups(gpu, n, rows):
+    """the one-launch grouping where its workgroups (256, 512 or 1,024 lanes, 64 rows or more each) and its batches of keys end:
+    keys that start at any int (read four at a time only where they are aligned), keys out of range (clamped to the first and
+    the last row), runs of equal keys across lanes and wavefronts, rows of 8, 9, 64 and 65 entries; the bits of the stable sort"""
+    from graphnn_amd import ops
+    rng = np.random.default_rng(n + rows)
+    key = rng.integers(0, rows, n)
+    key[n // 3:n // 3 + 300] = rng.integers(0, rows)
+    at = 0
+    for length in (8, 9, 64, 65):                             # rows of about these lengths, scattered
+        if n > 1000:
+            key[rng.permutation(n)[:length]] = rows * (at + 1) // 5
+        at += 1
+    for order in ("any", "ascending"):
+        if order == "ascending":
+            key = np.sort(key)
+        raw = key.copy()
+        raw[key == 0] -= rng.integers(0, 3, int((key == 0).sum()))
+        raw[key == rows - 1] += rng.integers(0, 3, int((key == rows - 1).sum()))
+        if rows == 1:
+            raw = key + rng.integers(-2, 3, n)
+        pay = rng.integers(0, 1 << 30, n).astype(np.int32)
+        want = _stable_group(rows, key, pay)
+        for shift in (0, 1):
+            key_d = _t(np.concatenate([np.zeros(shift, np.int32), raw.astype(np.int32)]), gpu)[shift:]
+            got = ops.csr_group(rows, key_d, _t(pay, gpu))
+            for g, w in zip(got, want):
+                assert np.array_equal(_n(g), w), (order, shift)
+
+
 @pytest.mark.parametrize("average", [False, True])
 def test_device_csr_of_consecutive_rows(gpu, oracle, average):
     """the pooling operand of a batch whose nodes were added subgraph after subgraph, from the subgraph offsets alone:
