@@ -34,6 +34,11 @@ int level_stream_dispatch(int N, int C, bool dense, const int* row_ptr, const in
                           const float* h_in, const float* W, const float* msg, const float* bias, float* h_out,
                           const HubPlan& hubs, bool relu_in, hipStream_t s);
 bool level_stream_covers(int N, int C);
+// level_tile.hip
+int level_tile_dispatch(int N, int C, const int* row_ptr, const int* col_idx, const float* val, const float* h_in, const float* W,
+                        const float* msg, const float* bias, float* h_out, bool relu_in, hipStream_t s);
+int level_tile_backward_dispatch(int N, int C, const int* row_ptr, const int* col_idx, const float* val, const float* x, const float* W,
+                                 float* agg_out, float* out, const float* gate, float* acc, hipStream_t s);
 int level_stream_backward_dispatch(int N, int C, const int* row_ptr, const int* col_idx, const float* val, const float* x,
                                    const float* W, float* agg_out, float* out, const float* gate, float* acc, const HubPlan& hubs,
                                    hipStream_t s);
@@ -540,6 +545,7 @@ int level_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* c
             default: return launch_level<64, true>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, none, s);
             }
         }
+        if (N <= kLevelTileMaxRows) return level_tile_dispatch(N, C, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, relu_in, s);
         HubPlan hubs{};
         if (int rc = hub_prepass(N, C, nnz, row_ptr, col_idx, val, h_in, C, s, &hubs, same_graph, relu_in, kHubThreshold, kHubChunk, -1,
                                  plan ? &plan->row_hub : nullptr))
@@ -599,6 +605,7 @@ int level_backward_dispatch(int N, int C, long long nnz, const int* row_ptr, con
     if (!(aligned16(dz) && aligned16(W) && aligned16(u) && aligned16(g_prev) && (!gate || aligned16(gate)) && (!acc || aligned16(acc))))
         return GNNHIP_EUNSUPPORTED;
     if (N >= kHubMinRows && nnz >= two_step_degree() * (long long)N) return GNNHIP_EUNSUPPORTED;     // dense and skewed: balanced SpMM
+    if (N <= kLevelTileMaxRows) return level_tile_backward_dispatch(N, C, row_ptr, col_idx, val, dz, W, u, g_prev, gate, acc, s);
     HubPlan hubs{};
     if (int rc = hub_prepass(N, C, nnz, row_ptr, col_idx, val, dz, C, s, &hubs, false, false)) return rc;
     return level_stream_backward_dispatch(N, C, row_ptr, col_idx, val, dz, W, u, g_prev, gate, acc, hubs, s);

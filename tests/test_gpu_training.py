@@ -401,6 +401,42 @@ def _relative_errors(got, want, terms):
     return float(e.square().mean().sqrt()), float(e.mean())
 
 
+@pytest.mark.parametrize("C", [16, 32, 64])
+@pytest.mark.parametrize("N", [1, 15, 16, 17, 31, 1000, 24_561, 24_576])
+def test_level_of_a_small_batch_has_the_bits_of_a_large_one(gpu, C, N):
+    """up to 24,576 rows a level runs a workgroup per 16-row tile, beyond that the streaming kernel: the same rows followed by
+    empty ones until the other kernel takes over give the same bits, forward and backward, with and without msg, bias, gate
+    and gradient sum; rows of 0, 4, 5, 8, 9, 16, 17, 48, 49 and 200 entries (taken at once, in a loop, by the whole wavefront)"""
+    import torch
+    from graphnn_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(C + N)
+    normal = lambda *shape: torch.randn(*shape, generator=gen, device=gpu)
+    lens = torch.tensor([0, 4, 5, 2, 8, 9, 1, 16, 17, 3, 48, 49, 0, 200, 2, 2, 1], device=gpu).repeat(N // 17 + 1)[:N]
+    if N > 2000:
+        lens = torch.where(torch.arange(N, device=gpu) % 1700 < 1600, lens.clamp(max=3), lens)
+    more = 24_577 + 13 - N                                  # empty rows behind them
+    grow = lambda x: torch.cat([x, normal(more, x.shape[1])])
+    rp = torch.zeros(N + 1, dtype=torch.int32, device=gpu)
+    rp[1:] = torch.cumsum(lens, 0)
+    nnz = int(rp[-1])
+    ci = torch.randint(0, N, (nnz,), generator=gen, device=gpu).int()
+    v = normal(nnz)
+    rp_more = torch.cat([rp, rp[-1:].expand(more)])
+    h, W, msg, bias, gate, acc0 = normal(N, C), normal(C, C) * 0.2, normal(N, C), normal(C), normal(N, C), normal(N, C)
+    h_more, msg_more, gate_more, acc_more0 = grow(h), grow(msg), grow(gate), grow(acc0)
+    for m, b in ((None, None), (msg, None), (msg, bias)):
+        got = ops.s2v_level(rp, ci, v, h, W, m, b)
+        want = ops.s2v_level(rp_more, ci, v, h_more, W, None if m is None else msg_more, b)
+        assert torch.equal(got, want[:N])
+    for g, a in ((None, None), (gate, None), (gate, acc0), (None, acc0)):
+        acc = None if a is None else acc0.clone()
+        acc_more = None if a is None else acc_more0.clone()
+        u, out = ops.s2v_level_backward(rp, ci, v, h, W, gate_h=g, acc=acc)
+        u_more, out_more = ops.s2v_level_backward(rp_more, ci, v, h_more, W, gate_h=None if g is None else gate_more, acc=acc_more)
+        assert torch.equal(u, u_more[:N]) and torch.equal(out, out_more[:N])
+        assert a is None or torch.equal(acc, acc_more[:N])
+
+
 @pytest.mark.parametrize("C", [128, 256])
 @pytest.mark.parametrize("N", [5003, 40_009])
 @pytest.mark.parametrize("kind", ["zero_mean", "relu", "one_sign"])
