@@ -697,11 +697,32 @@ __global__ __launch_bounds__(WAVES * kWave, (min_waves<C, KSX, WAVES, KEEP, PACK
             if (tid <= ng) l_gs[tid] = s_row_ptr[g + tid] - node0;
             __syncthreads();
             for (int k = wave; k < ng; k += kWavesPerBlock) {
-                const int r0 = l_gs[k], r1 = l_gs[k + 1];
+                const int r0 = __builtin_amdgcn_readfirstlane(l_gs[k]), r1 = __builtin_amdgcn_readfirstlane(l_gs[k + 1]);
                 const int gk = g + k;
+                // rows in order, eight asked for together: a row at a time is a trip through LDS each
                 float p = 0.f;
-                if (lane < C)
-                    for (int lr = r0; lr < r1; ++lr) p = fmaf(l_sv[lr], hbuf[(size_t)lr * LDT + lane], p);
+                if (lane < C) {
+                    float w[8], x[8];
+                    auto ask = [&](int lr, int last) {
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) {
+                            const int at = min(lr + u, last);
+                            w[u] = l_sv[at];
+                            x[u] = hbuf[(size_t)at * LDT + lane];
+                        }
+                    };
+                    int lr = r0;
+                    for (; lr + 8 <= r1; lr += 8) {
+                        ask(lr, r1 - 1);
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) p = fmaf(w[u], x[u], p);
+                    }
+                    if (lr < r1) {
+                        ask(lr, r1 - 1);
+#pragma unroll
+                        for (int u = 0; u < 7; ++u) if (lr + u < r1) p = fmaf(w[u], x[u], p);
+                    }
+                }
                 if (lane < C) pool[(size_t)gk * C + lane] = p;
                 const float* w1 = ro_staged ? w1s : Wh1;      // [C][H] either way
                 const float* w2 = ro_staged ? w2s : Wh2;      // [H][Q]
@@ -714,6 +735,7 @@ __global__ __launch_bounds__(WAVES * kWave, (min_waves<C, KSX, WAVES, KEEP, PACK
                 hv = relu_ref(hv);
                 if (lane < H) hidden[(size_t)gk * H + lane] = hv;
                 float sq = 0.f;
+#pragma unroll 8
                 for (int j = 0; j < H; ++j) {
                     const float hj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hv), j));
                     if (lane < Q) sq = fmaf(hj, w2[(size_t)j * Q + lane], sq);
@@ -723,11 +745,8 @@ __global__ __launch_bounds__(WAVES * kWave, (min_waves<C, KSX, WAVES, KEEP, PACK
                     const float first = row_value_f(sq, 0);
                     float mx = (lane < Q) ? max_keep(first, sq) : first;     // the reference scan starts at element 0
                     mx = wave_max(mx);
-                    float bv = -INFINITY;
-                    int bi = 0x7fffffff;
-                    if (lane < Q) { bv = (sq != sq) ? -INFINITY : sq; bi = lane; }   // a NaN that is not first never wins
-                    wave_argmax(bv, bi);
-                    if (first != first) bi = 0;                              // a NaN in column 0 is never displaced
+                    // the first class that has the maximum; a NaN in column 0 is never displaced, and any other never wins
+                    const int bi = first != first ? 0 : (int)__builtin_ctzll(__ballot(lane < Q && sq == mx));
                     if (pred && lane == 0) pred[gk] = bi;
                     if (probs) {
                         const float e = (lane < Q) ? expf(sq - mx) : 0.f;
@@ -751,9 +770,22 @@ __global__ __launch_bounds__(WAVES * kWave, (min_waves<C, KSX, WAVES, KEEP, PACK
             float acc[CPL];
 #pragma unroll
             for (int u = 0; u < CPL; ++u) acc[u] = 0.f;
-            for (int lr = wave * RS + pr; lr < n; lr += kWavesPerBlock * RS)
+            // (four rows asked for together; what lies past the graph is not added)
+            constexpr int kAsk = 4;
+            for (int lr = wave * RS + pr; lr < n; lr += kAsk * kWavesPerBlock * RS) {
+                float w[kAsk], x[kAsk][CPL];
 #pragma unroll
-                for (int u = 0; u < CPL; ++u) acc[u] = fmaf(l_sv[lr], hbuf[(size_t)lr * LDT + pc + u * kWave], acc[u]);
+                for (int i = 0; i < kAsk; ++i) {
+                    const int at = min(lr + i * kWavesPerBlock * RS, n - 1);
+                    w[i] = l_sv[at];
+#pragma unroll
+                    for (int u = 0; u < CPL; ++u) x[i][u] = hbuf[(size_t)at * LDT + pc + u * kWave];
+                }
+#pragma unroll
+                for (int i = 0; i < kAsk; ++i)
+#pragma unroll
+                    for (int u = 0; u < CPL; ++u) acc[u] = lr + i * kWavesPerBlock * RS < n ? fmaf(w[i], x[i][u], acc[u]) : acc[u];
+            }
             if constexpr (CPL == 1) {
 #pragma unroll
                 for (int off = GP; off < kWave; off <<= 1) acc[0] += __shfl_xor(acc[0], off, kWave);
@@ -805,33 +837,42 @@ __global__ __launch_bounds__(WAVES * kWave, (min_waves<C, KSX, WAVES, KEEP, PACK
         __syncthreads();
         GNNHIP_PHASE_MARK(14);
         if (Q <= 16) {
-            // few classes: lane q of the first wavefront adds up logit q, and softmax and arg-max follow in
-            // registers, with no further barrier or trip through LDS
+            // few classes: 16, 8 or 4 neighbouring lanes of the first wavefront add up a logit (units sub, sub + part, ... each, then
+            // their sums), lane q takes logit q, and softmax and arg-max follow in the registers of its sixteen lanes, with no
+            // further barrier.  The chain ends the kernel's: a lane per class that added up all units took 1.3 us
+            // (32 units, 2 classes; 2.8 with 64 and 6)
             if (wave == 0) {
+                const int log_part = Q <= 4 ? 4 : Q <= 8 ? 3 : 2, part_lanes = 1 << log_part;
+                const int qq = lane >> log_part, sub = lane & (part_lanes - 1);
+                const float* w2 = ro_staged ? w2s : Wh2;      // [H][Q] either way
                 float s = 0.f;
-                if (lane < Q) {
-                    if (ro_staged) {
-#pragma unroll 8
-                        for (int j = 0; j < H; ++j) s = fmaf(hid[j], w2s[j * Q + lane], s);
-                    } else {
-#pragma unroll 8
-                        for (int j = 0; j < H; ++j) s = fmaf(hid[j], Wh2[(size_t)j * Q + lane], s);
-                    }
-                    logits[(size_t)g * Q + lane] = s;
+                if (qq < Q) {
+#pragma unroll 4
+                    for (int j = sub; j < H; j += part_lanes) s = fmaf(hid[j], w2[j * Q + qq], s);
                 }
+                s += dpp_mov_f<kDppXor1>(s);
+                s += dpp_mov_f<kDppXor2>(s);
+                if (log_part >= 3) s += dpp_mov_f<kDppHalfMirror>(s);
+                if (log_part >= 4) s += dpp_mov_f<kDppMirror>(s);
+                s = __shfl(s, (lane << log_part) & (kWave - 1), kWave);
+                if (lane < Q) logits[(size_t)g * Q + lane] = s;
                 if (probs || pred) {
                     const float first = row_value_f(s, 0);
                     float mx = (lane < Q) ? max_keep(first, s) : first;     // the reference scan starts at element 0
-                    mx = wave_max(mx);
-                    float bv = -INFINITY;
-                    int bi = 0x7fffffff;
-                    if (lane < Q) { bv = (s != s) ? -INFINITY : s; bi = lane; }   // a NaN that is not first never wins
-                    wave_argmax(bv, bi);
-                    if (first != first) bi = 0;                             // a NaN in column 0 is never displaced
+                    mx = max_keep(mx, dpp_mov_f<kDppXor1>(mx));
+                    mx = max_keep(mx, dpp_mov_f<kDppXor2>(mx));
+                    mx = max_keep(mx, dpp_mov_f<kDppHalfMirror>(mx));
+                    mx = max_keep(mx, dpp_mov_f<kDppMirror>(mx));
+                    // the first class that has the maximum; a NaN in column 0 is never displaced, and any other never wins
+                    const int bi = first != first ? 0 : (int)__builtin_ctzll(__ballot(lane < Q && s == mx));
                     if (pred && lane == 0) pred[g] = bi;
                     if (probs) {
                         const float e = (lane < Q) ? expf(s - mx) : 0.f;
-                        const float sum = wave_sum(e);
+                        float sum = e;
+                        sum += dpp_mov_f<kDppXor1>(sum);
+                        sum += dpp_mov_f<kDppXor2>(sum);
+                        sum += dpp_mov_f<kDppHalfMirror>(sum);
+                        sum += dpp_mov_f<kDppMirror>(sum);
                         if (lane < Q) probs[(size_t)g * Q + lane] = e / sum;
                     }
                 }

@@ -2183,6 +2183,52 @@ def test_device_csr_group_at_the_edges_of_its_workgroups(gpu, n, rows):
                 assert np.array_equal(_n(g), w), (order, shift)
 
 
+@pytest.mark.parametrize("B", [40, 600])
+@pytest.mark.parametrize("H,Q", [(1, 1), (3, 2), (32, 4), (64, 5), (17, 8), (33, 9), (5, 16), (64, 17), (130, 3)])
+def test_one_launch_readout_of_any_number_of_classes(gpu, B, H, Q):
+    """the end of the one-launch forward, graph by graph (sixteen, eight or four lanes add up a logit up to 4, 8, 16 classes, a wavefront
+    beyond) and packed (a lane per class), graphs of 1 to 60 nodes so that the pooling ends inside its runs of rows: pooled row, hidden
+    layer and logits within the roundings of their sums of float64, from the operands the device itself formed; probabilities
+    likewise; classes that tie take the first, a NaN in class 0 is kept, one elsewhere never wins"""
+    import torch
+    from graphnn_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(B + 100 * H + Q)
+    C, K, L = 32, 5, 2
+    sizes = (torch.arange(B, device=gpu) * 7) % 60 + 1
+    off = torch.zeros(B + 1, dtype=torch.int32, device=gpu)
+    off[1:] = torch.cumsum(sizes, 0)
+    N = int(off[-1])
+    graph = torch.repeat_interleave(torch.arange(B, device=gpu), sizes)
+    ring = torch.arange(N, device=gpu) + 1
+    ring = torch.where(ring == off[1:][graph], off[:-1][graph].long(), ring).int()
+    A = (torch.arange(N + 1, device=gpu).int(), ring, torch.ones(N, device=gpu))
+    normal = lambda *shape: torch.randn(*shape, generator=gen, device=gpu)
+    S = (off, torch.arange(N, device=gpu).int(), torch.rand(N, generator=gen, device=gpu) + 0.5)
+    X, Wn, Wc, W1, W2 = normal(N, K), normal(K, C), normal(C, C) * 0.2, normal(C, H), normal(H, Q)
+    bufs = ops.s2v_forward_batched(A, S, X, Wn, Wc, W1, W2, L, int(sizes.max()))
+    h, w = bufs.h_final.double(), S[2].double()
+    zero = torch.zeros(B, C, dtype=torch.float64, device=gpu)
+    pool = zero.index_add(0, graph, h * w[:, None])
+    eps = 2.0 ** -24
+    def close(got, want, terms, roundings):
+        assert bool(((got.double() - want).abs() <= roundings * eps * terms).all())
+    close(bufs.pool, pool, zero.index_add(0, graph, (h * w[:, None]).abs()), 64)
+    hidden = (bufs.pool.double() @ W1.double()).clamp(min=0)
+    close(bufs.hidden, hidden, bufs.pool.double().abs() @ W1.double().abs(), C + 4)
+    close(bufs.logits, bufs.hidden.double() @ W2.double(), bufs.hidden.double().abs() @ W2.double().abs(), H + 4)
+    # e^x of a rounded x is off by the rounding of x, and what lies below the smallest normal float may be zero
+    want = torch.softmax(bufs.logits.double(), 1)
+    close(bufs.probs, want, want + 2.0 ** -126 / eps, 2 * Q + 16 + 4 * float(bufs.logits.abs().max()))
+    assert torch.equal(bufs.pred.long(), bufs.logits.argmax(1))
+    for bad in {0, Q - 1}:
+        W2_bad = torch.zeros(H, Q, device=gpu)
+        tied = ops.s2v_forward_batched(A, S, X, Wn, Wc, W1, W2_bad, L, int(sizes.max()))
+        assert not bool(tied.pred.any()) and bool((tied.probs == tied.probs[:, :1]).all())
+        W2_bad[:, bad] = float("nan")
+        got = ops.s2v_forward_batched(A, S, X, Wn, Wc, W1, W2_bad, L, int(sizes.max()))
+        assert bool(torch.isnan(got.logits[:, bad]).all()) and not bool(got.pred.any())
+
+
 @pytest.mark.parametrize("average", [False, True])
 def test_device_csr_of_consecutive_rows(gpu, oracle, average):
     """the pooling operand of a batch whose nodes were added subgraph after subgraph, from the subgraph offsets alone:
