@@ -28,6 +28,7 @@
 // first neighbours of a lane's rows stay in registers for all levels; the readout has three steps
 // (pool partials | pooled row + hidden layer | logits + softmax in the registers of one wavefront).
 #include <algorithm>
+#include <type_traits>
 
 #include "gnnhip_internal.h"
 #include "buffer_addr.h"
@@ -558,19 +559,23 @@ __global__ __launch_bounds__(WAVES * kWave, (min_waves<C, KSX, WAVES, KEEP, PACK
                     const float4 wv = *reinterpret_cast<const float4*>(wrow);
                     v = make_float4(0.f + wv.x, 0.f + wv.y, 0.f + wv.z, 0.f + wv.w);
                 } else {
+                    // (srt is KSX or KSX - 2: two straight runs instead of a branch per step)
                     const float* xrow = xs + min(lr, n - 1) * KP + srt * q;
-                    float xreg[KSXA];
+                    auto product = [&](auto steps) {
+                        constexpr int S = decltype(steps)::value;
+                        float2 x2[S / 2];
 #pragma unroll
-                    for (int s2 = 0; s2 < KSXA / 2; ++s2) {
-                        float2 v2 = make_float2(0.f, 0.f);
-                        if (2 * s2 < srt) v2 = *reinterpret_cast<const float2*>(xrow + 2 * s2);
-                        xreg[2 * s2] = v2.x; xreg[2 * s2 + 1] = v2.y;
-                    }
-                    mfma_f4 acc = {0.f, 0.f, 0.f, 0.f};
+                        for (int s2 = 0; s2 < S / 2; ++s2) x2[s2] = *reinterpret_cast<const float2*>(xrow + 2 * s2);
+                        mfma_f4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                    for (int s = 0; s < KSXA; ++s)
-                        if (s < srt) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wx[s], xreg[s], acc, 0, 0, 0);
-                    v = make_float4(acc[0], acc[1], acc[2], acc[3]);
+                        for (int s2 = 0; s2 < S / 2; ++s2) {
+                            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wx[2 * s2], x2[s2].x, acc, 0, 0, 0);
+                            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wx[2 * s2 + 1], x2[s2].y, acc, 0, 0, 0);
+                        }
+                        return make_float4(acc[0], acc[1], acc[2], acc[3]);
+                    };
+                    constexpr int kFewer = KSXA > 2 ? KSXA - 2 : KSXA;
+                    v = srt == KSXA ? product(std::integral_constant<int, KSXA>()) : product(std::integral_constant<int, kFewer>());
                 }
                 if (!valid) v = f4_zero();
                 if (valid) *reinterpret_cast<float4*>(msg + (size_t)(node0 + lr) * C + 16 * jb + 4 * q) = v;
