@@ -111,6 +111,19 @@ __device__ __forceinline__ int wave_sum_i(int v)
     return (row_value_i(v, 0) + row_value_i(v, 1)) + (row_value_i(v, 2) + row_value_i(v, 3));
 }
 
+// inclusive prefix sum over the wavefront: shifts inside the rows of 16 lanes (lanes without a source add 0),
+// then the totals of the rows below
+__device__ __forceinline__ int wave_inclusive_scan_i(int v)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true);      // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true);      // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true);      // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true);      // row_shr:8
+    const int t0 = __builtin_amdgcn_readlane(v, 15), t1 = __builtin_amdgcn_readlane(v, 31), t2 = __builtin_amdgcn_readlane(v, 47);
+    const int row = (threadIdx.x & (kWave - 1)) >> 4;
+    return v + (row >= 1 ? t0 : 0) + (row >= 2 ? t1 : 0) + (row >= 3 ? t2 : 0);
+}
+
 // max with "a < b ? b : a" so that a NaN in b never replaces a (the reference's
 // strict comparison never selects a NaN that is not first in the row).
 __device__ __forceinline__ float max_keep(float a, float b) { return a < b ? b : a; }

@@ -186,108 +186,56 @@ __global__ __launch_bounds__(kOrderBlock) void graph_order_kernel(int B, int n16
 // and the levels at the cost of one graph (the kernel's time is per workgroup: start-up, staging, a barrier
 // per stage, and matrix tiles that a 30-node graph leaves three quarters empty), and only the readout runs per
 // graph (a wavefront each).  1,024 graphs of the 10..110-node distribution: 59 -> 45 us.
-// The kernel below cuts the batch into such runs ("bins").  Every 64 consecutive graphs are packed on their
+// The kernel below cuts the batch into such runs ("bins").  Every 64 consecutive graphs (a segment) are packed on their
 // own by one wavefront (first fit in batch order; a bin never crosses such a boundary, which costs about one
-// partly filled bin per 64 graphs), so all of it is a few ballots per bin.  What bounds it is the chain of those
-// ballots and the trips to memory before and behind it; a segment is packed once, to a 64-bit mask of the graphs
-// that open a bin, and the lanes of those graphs write whole records from it (3,001 graphs: 14.3 -> 8.4 us).  A graph of more than cap nodes is a
-// bin of its own (the forward kernel refuses it).  Output: bins[0] = number of bins, then one record of
-// kOrderRec ints per bin from bins + kOrderRec on: first graph, first node, nodes, first entry, end of entries,
-// graphs.
+// partly filled bin per segment): a ballot per bin gives a 64-bit word in which the graphs that open one are set, and the lanes
+// of those graphs write the segment's records, from record 64 x segment on.  The forward kernel finds bin b by a prefix sum over the set
+// bits of the words, one of them per lane, so the segments need not know of each other: a wavefront each and three trips to
+// memory, 4.7 us for 3,001 graphs.  (One workgroup that packed the whole batch, to number the bins itself, took 8.5.  Without
+// this launch, a workgroup of the forward kernel either packs all segments, which costs it more than this launch from
+// some 500 bins on, or numbers bins by its own segment, which spreads them unevenly over the dies: 1,500 graphs at hidden 64 72
+// us where bins numbered through the batch take 45.)  A graph of more than cap nodes is a bin of its own (the forward kernel
+// refuses it).  Output: words[segment], then one record of kOrderRec ints per bin: first graph, first node, nodes, first entry, end of
+// entries, graphs.
 constexpr int kPackNodes = 128;                  // eight tiles: with four column blocks, two tasks for each of 16 wavefronts
 constexpr int kPackMaxNodes = 208;
 constexpr int kPackMinGraphs = 2 * kNumCU;       // below this the graphs taken one by one, largest first, are as fast
-constexpr int kBinBlock = 1024;
-constexpr int kBinMaxGraphs = 1 << 19;           // segment counts live in LDS (32 KB)
+constexpr int kPackMaxGraphs = 1 << 19;
+constexpr int kBinBlock = 128;
+// ints ahead of the records: the words of the segments, in whole records
+__host__ __device__ inline size_t bin_words_ints(int B) { return ((size_t)((B + kWave - 1) / kWave) * 2 + kOrderRec - 1) / kOrderRec * kOrderRec; }
+
 __global__ __launch_bounds__(kBinBlock) void graph_bins_kernel(int B, int cap, const int* __restrict__ a_row_ptr,
                                                                const int* __restrict__ s_row_ptr, int* __restrict__ bins)
 {
-    constexpr int kWaves = kBinBlock / kWave;
-    __shared__ int seg_bins[kBinMaxGraphs / kWave + 1];
-    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    const int nseg = (B + kWave - 1) / kWave;
-    // packs segment `seg` (start / end: first node and end of the lane's graph): bit g is set where graph g opens a bin
-    auto pack = [&](int seg, int start, int end) {
-        const bool live = seg * kWave + lane < B;
-        const int nlive = min(kWave, B - seg * kWave);
-        unsigned long long opens = 0;
-        int first = 0;
-        while (first < nlive) {
-            const int node0 = __builtin_amdgcn_readlane(start, first);
-            opens |= 1ull << first;
-            // lanes from `first` on whose graph still fits behind node0; the bin ends before the first that does not
-            const unsigned long long stop = __ballot(lane >= first && (!live || end - node0 > cap));
-            int next = stop ? (int)__builtin_ctzll(stop) : kWave;
-            if (next == first) next = first + 1;                     // larger than cap: alone
-            first = __builtin_amdgcn_readfirstlane(next);
-        }
-        return opens;
-    };
-    // the node ranges and bins of this wavefront's first kBinKeep segments stay in registers between the two passes
-    constexpr int kBinKeep = 4;
-    int st[kBinKeep], en[kBinKeep];
-    unsigned long long bits[kBinKeep];
-    auto ranges = [&](int seg, int& start, int& end) {
-        const int g = seg * kWave + lane;
-        start = end = 0;
-        if (g < B) { start = s_row_ptr[g]; end = s_row_ptr[g + 1]; }
-    };
-#pragma unroll
-    for (int j = 0; j < kBinKeep; ++j) ranges(wave + j * kWaves, st[j], en[j]);
-#pragma unroll
-    for (int j = 0; j < kBinKeep; ++j) {
-        const int seg = wave + j * kWaves;
-        bits[j] = 0;
-        if (seg < nseg) {
-            bits[j] = pack(seg, st[j], en[j]);
-            if (lane == 0) seg_bins[seg] = __popcll(bits[j]);
-        }
+    const int lane = threadIdx.x & (kWave - 1);
+    const int seg = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kBinBlock / kWave) + threadIdx.x / kWave));
+    const int nlive = min(kWave, B - seg * kWave);
+    if (nlive <= 0) return;
+    int start = 0, end = 0;                      // first node and end of the lane's graph
+    if (lane < nlive) { start = s_row_ptr[seg * kWave + lane]; end = s_row_ptr[seg * kWave + lane + 1]; }
+    unsigned long long opens = 0;
+    int first = 0;
+    while (first < nlive) {
+        const int node0 = __builtin_amdgcn_readlane(start, first);
+        opens |= 1ull << first;
+        // lanes from `first` on whose graph no longer fits behind node0: the bin ends before the first of them
+        const unsigned long long stop = __ballot(lane >= first && (lane >= nlive || end - node0 > cap));
+        int next = stop ? (int)__builtin_ctzll(stop) : kWave;
+        if (next == first) next = first + 1;                         // larger than cap: alone
+        first = __builtin_amdgcn_readfirstlane(next);
     }
-    for (int seg = wave + kBinKeep * kWaves; seg < nseg; seg += kWaves) {
-        int start, end;
-        ranges(seg, start, end);
-        const int c = __popcll(pack(seg, start, end));
-        if (lane == 0) seg_bins[seg] = c;
-    }
-    __syncthreads();
-    if (wave == 0) {                                                 // exclusive scan of the segment counts
-        int carry = 0;
-        for (int b0 = 0; b0 < nseg; b0 += kWave) {
-            const int i = b0 + lane;
-            const int v = i < nseg ? seg_bins[i] : 0;
-            int incl = v;
-#pragma unroll
-            for (int d = 1; d < kWave; d <<= 1) {
-                const int o = __shfl_up(incl, d, kWave);
-                if (lane >= d) incl += o;
-            }
-            if (i < nseg) seg_bins[i] = carry + incl - v;
-            carry += __shfl(incl, kWave - 1, kWave);
-        }
-        if (lane == 0) bins[0] = carry;
-    }
-    __syncthreads();
+    if (lane == 0) reinterpret_cast<unsigned long long*>(bins)[seg] = opens;
     // a lane whose graph opens a bin writes its record (a bin the forward kernel will refuse gets no entry range)
-    auto write = [&](int seg, unsigned long long opens, int start, int end) {
-        const int nlive = min(kWave, B - seg * kWave);
-        const unsigned long long behind = lane == kWave - 1 ? 0 : opens >> (lane + 1);
-        const int ng = (behind ? lane + 1 + (int)__builtin_ctzll(behind) : nlive) - lane;
-        const int n = __shfl(end, min(max(lane + ng - 1, 0), kWave - 1), kWave) - start;
-        if (!((opens >> lane) & 1ull)) return;
-        int e0 = 0, e1 = 0;
-        if (n >= 0 && n <= cap) { e0 = a_row_ptr[start]; e1 = a_row_ptr[start + n]; }
-        int* rec = bins + (size_t)(1 + seg_bins[seg] + __popcll(opens & ((1ull << lane) - 1ull))) * kOrderRec;
-        *reinterpret_cast<int4*>(rec) = make_int4(seg * kWave + lane, start, n, e0);
-        *reinterpret_cast<int2*>(rec + 4) = make_int2(e1, ng);
-    };
-#pragma unroll
-    for (int j = 0; j < kBinKeep; ++j)
-        if (wave + j * kWaves < nseg) write(wave + j * kWaves, bits[j], st[j], en[j]);
-    for (int seg = wave + kBinKeep * kWaves; seg < nseg; seg += kWaves) {
-        int start, end;
-        ranges(seg, start, end);
-        write(seg, pack(seg, start, end), start, end);
-    }
+    const unsigned long long behind = lane == kWave - 1 ? 0 : opens >> (lane + 1);
+    const int ng = (behind ? lane + 1 + (int)__builtin_ctzll(behind) : nlive) - lane;
+    const int n = __shfl(end, min(max(lane + ng - 1, 0), kWave - 1), kWave) - start;
+    if (!((opens >> lane) & 1ull)) return;
+    int e0 = 0, e1 = 0;
+    if (n >= 0 && n <= cap) { e0 = a_row_ptr[start]; e1 = a_row_ptr[start + n]; }
+    int* rec = bins + bin_words_ints(B) + (size_t)(seg * kWave + __popcll(opens & ((1ull << lane) - 1ull))) * kOrderRec;
+    *reinterpret_cast<int4*>(rec) = make_int4(seg * kWave + lane, start, n, e0);
+    *reinterpret_cast<int2*>(rec + 4) = make_int2(e1, ng);
 }
 
 // Whether the registers let two workgroups share a compute unit: four wavefronts always, eight with up to 128 registers per lane.
@@ -305,7 +253,7 @@ template <int C, int KSX, int WAVES, bool KEEP, bool PACK> constexpr int min_wav
 // order: null (graphs in batch order), or the records graph_order_kernel left.
 // KEEP: the embeddings of all levels are also stored for a backward pass, h_l at h_levels + l * level_stride
 // (a variant of its own: the extra stores cost the inference kernel 2 % when they are a run-time choice).
-// PACK: `order` holds the bins graph_bins_kernel made (order[0] bins, records from order + kOrderRec on); a workgroup
+// PACK: `order` holds the bins graph_bins_kernel made; a workgroup
 // carries a bin through the input stage and the levels as one block-diagonal graph, and its wavefronts run the
 // readout of the bin's graphs, one graph each (H <= 64 and Q <= 64: a lane per hidden unit and per class).
 template <int C, int KSX, int WAVES, bool KEEP = false, bool PACK = false>
@@ -366,27 +314,43 @@ __global__ __launch_bounds__(WAVES * kWave, (min_waves<C, KSX, WAVES, KEEP, PACK
     // The position of the first graph (node range, then entry range) is asked for ahead of the weight
     // loads, so the two dependent trips to memory run under them instead of after them.
     int next_g = blockIdx.x, next_node0 = 0, next_n = 0, next_e0 = 0, next_e1 = 0, next_ng = 1;
-    // PACK: the slots are the bins (their number is the first word of `order`, the records follow its first kOrderRec words)
-    const int* recs = PACK ? order + kOrderRec : order;
-    const int nslots = PACK ? order[0] : B;
-    if ((int)blockIdx.x < nslots) {
-        if (order) {
-            const int4 r0 = *reinterpret_cast<const int4*>(recs + (size_t)blockIdx.x * kOrderRec);
-            next_g = r0.x; next_node0 = r0.y; next_n = r0.z; next_e0 = r0.w;
-            const int2 r1 = *reinterpret_cast<const int2*>(recs + (size_t)blockIdx.x * kOrderRec + 4);
-            next_e1 = r1.x;
-            next_ng = r1.y;
-        } else {
-            next_node0 = s_row_ptr[blockIdx.x];
-            next_n = s_row_ptr[blockIdx.x + 1] - next_node0;
+    // PACK: the place of the record of a bin, or -1 past the last one
+    const int nseg = (B + kWave - 1) / kWave;
+    auto find_bin = [&](int bin) {
+        const unsigned long long* words = reinterpret_cast<const unsigned long long*>(order);
+        const int lane = tid0 & (kWave - 1);
+        int before = 0;
+        for (int s0 = 0; s0 < nseg; s0 += kWave) {
+            const int count = s0 + lane < nseg ? __popcll(words[s0 + lane]) : 0;
+            const int through = before + wave_inclusive_scan_i(count);
+            const unsigned long long behind = __ballot(bin < through);
+            if (behind) {
+                const int at = (int)__builtin_ctzll(behind);
+                return (s0 + at) * kWave + bin - __builtin_amdgcn_readlane(through - count, at);
+            }
+            before = __builtin_amdgcn_readlane(through, kWave - 1);
         }
+        return -1;
+    };
+    const int* recs = PACK ? order + bin_words_ints(B) : order;
+    if (order) {
+        const int at = PACK ? find_bin((int)blockIdx.x) : (int)blockIdx.x;
+        if (PACK && at < 0) return;
+        const int4 r0 = *reinterpret_cast<const int4*>(recs + (size_t)at * kOrderRec);
+        next_g = r0.x; next_node0 = r0.y; next_n = r0.z; next_e0 = r0.w;
+        const int2 r1 = *reinterpret_cast<const int2*>(recs + (size_t)at * kOrderRec + 4);
+        next_e1 = r1.x;
+        next_ng = r1.y;
+    } else {
+        next_node0 = s_row_ptr[blockIdx.x];
+        next_n = s_row_ptr[blockIdx.x + 1] - next_node0;
     }
     // this wavefront's 16 columns of W^T, level contraction: wreg[s] = Wc[KS q + s][16 jb + t]
     float wreg[KS];
 #pragma unroll
     for (int s = 0; s < KS; ++s)
         wreg[s] = Wc[(size_t)(KS * ((tid0 & (kWave - 1)) >> 4) + s) * C + 16 * ((tid0 / kWave) % NJB) + (tid0 & 15)];
-    if (!order && (int)blockIdx.x < nslots && next_n >= 0 && next_n <= n16max) {
+    if (!order && next_n >= 0 && next_n <= n16max) {
         next_e0 = a_row_ptr[next_node0];
         next_e1 = a_row_ptr[next_node0 + next_n];
     }
@@ -420,7 +384,7 @@ __global__ __launch_bounds__(WAVES * kWave, (min_waves<C, KSX, WAVES, KEEP, PACK
     // the staged rows of X have stride KP floats and zeros from column K on
     const int srt = GraphLds::input_steps(K);
     const int KP = 4 * srt;
-    for (int slot = blockIdx.x; slot < nslots; slot += gridDim.x) {
+    for (int slot = blockIdx.x; PACK || slot < B; slot += gridDim.x) {
         // The lane's coordinates are derived again for every graph from a value the compiler cannot see
         // through.  Otherwise every per-lane address of the loop body (a dozen 64-bit pointers) is computed
         // once ahead of the loop, does not fit the 128 registers of a 16-wavefront workgroup, and comes back
@@ -437,9 +401,11 @@ __global__ __launch_bounds__(WAVES * kWave, (min_waves<C, KSX, WAVES, KEEP, PACK
         if (first) {
             g = next_g; node0 = next_node0; n = next_n; ng = next_ng;
         } else if (order) {
-            const int4 r0 = *reinterpret_cast<const int4*>(recs + (size_t)slot * kOrderRec);
+            const int at = PACK ? find_bin(slot) : slot;
+            if (PACK && at < 0) return;
+            const int4 r0 = *reinterpret_cast<const int4*>(recs + (size_t)at * kOrderRec);
             g = r0.x; node0 = r0.y; n = r0.z; rec_e0 = r0.w;
-            const int2 r1 = *reinterpret_cast<const int2*>(recs + (size_t)slot * kOrderRec + 4);
+            const int2 r1 = *reinterpret_cast<const int2*>(recs + (size_t)at * kOrderRec + 4);
             rec_e1 = r1.x;
             ng = r1.y;
         } else {
@@ -963,9 +929,9 @@ int launch_graph_forward(int B, int K, int H, int Q, int L, int n16max,
         if (most > B) most = B;
         if (most < grid) grid = (int)most;
         void* p = nullptr;
-        if (int rc = stream_scratch(s, sizeof(int) * kOrderRec * ((size_t)B + 1), &p)) return rc;
+        if (int rc = stream_scratch(s, sizeof(int) * (bin_words_ints(B) + kOrderRec * (size_t)((B + kWave - 1) / kWave * kWave)), &p)) return rc;
         order = static_cast<int*>(p);
-        hipLaunchKernelGGL(graph_bins_kernel, dim3(1), dim3(kBinBlock), 0, s, B, n16max, a_row_ptr, s_row_ptr, order);
+        hipLaunchKernelGGL(graph_bins_kernel, dim3(ceil_div_u((size_t)B, kBinBlock)), dim3(kBinBlock), 0, s, B, n16max, a_row_ptr, s_row_ptr, order);
         GNNHIP_LAUNCH_CHECK("graph_bins");
     } else if (graphs_ordered(B) && n16max / 16 + 2 <= 64) {
         void* p = nullptr;
@@ -1081,7 +1047,7 @@ int forward_batched_entry(bool labels, long long a_nnz, int N, int B, int K, int
     auto holds = [&](int cap, int nodes) { return 0.95 * (double)a_nnz * nodes <= (double)cap * (double)N; };
     int rc = GNNHIP_EUNSUPPORTED;
     // more graphs than compute units: runs of consecutive graphs share a workgroup (bins of at least kPackNodes nodes)
-    if (B >= kPackMinGraphs && B <= kBinMaxGraphs && H <= kWave && Q <= kWave && !h_levels) {
+    if (B >= kPackMinGraphs && B <= kPackMaxGraphs && H <= kWave && Q <= kWave && !h_levels) {
         // Bin size: a workgroup's time grows with its bin and the bins run in rounds of one per compute unit, so the size that
         // just avoids another round wins.  Hidden 16 and 32 also have workgroups of eight wavefronts, two to a compute unit:
         // slower alone (1,000 graphs, hidden 32: 28 against 27 us), but a round of theirs takes twice the bins (3,001 graphs:

@@ -375,19 +375,6 @@ inline bool small_layout(long long rows, long long n, SmallLayout* out)
     return true;
 }
 
-// inclusive prefix sum over the wavefront: shifts inside the rows of 16 lanes (lanes without a source add 0),
-// then the totals of the rows below
-__device__ __forceinline__ int wave_inclusive_scan_i(int v)
-{
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true);      // row_shr:1
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true);      // row_shr:2
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true);      // row_shr:4
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true);      // row_shr:8
-    const int t0 = __builtin_amdgcn_readlane(v, 15), t1 = __builtin_amdgcn_readlane(v, 31), t2 = __builtin_amdgcn_readlane(v, 47);
-    const int row = (threadIdx.x & (kWave - 1)) >> 4;
-    return v + (row >= 1 ? t0 : 0) + (row >= 2 ? t1 : 0) + (row >= 3 ? t2 : 0);
-}
-
 __device__ __forceinline__ void order_pair(int& a, int& b)
 {
     const int lo = min(a, b), hi = max(a, b);

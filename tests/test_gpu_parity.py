@@ -2229,6 +2229,44 @@ def test_one_launch_readout_of_any_number_of_classes(gpu, B, H, Q):
         assert bool(torch.isnan(got.logits[:, bad]).all()) and not bool(got.pred.any())
 
 
+@pytest.mark.parametrize("B", [512, 513, 575, 577, 640, 4096, 4161, 70_001])
+@pytest.mark.parametrize("sizes", ["ones", "tiny", "full", "mixed"])
+def test_packed_batches_of_any_number_of_segments(gpu, B, sizes):
+    """the bins of a packed batch: segments of 64 graphs, the last one short; a whole segment in one bin (graphs of one node), bins of
+    one graph each (128 nodes), a bin per few graphs and graphs without nodes: node outputs with the bits of the forward that
+    takes graph by graph (it keeps all levels), graph outputs of the right graphs within the roundings of their sums of float64"""
+    import torch
+    from graphnn_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(B)
+    n = {"ones": torch.ones(B, device=gpu).long(), "tiny": torch.randint(1, 4, (B,), generator=gen, device=gpu),
+         "full": torch.full((B,), 128, device=gpu), "mixed": torch.randint(0, 12, (B,), generator=gen, device=gpu)}[sizes]
+    n[640:] = n[640:].clamp(max=12)
+    if sizes == "mixed":
+        n[::97] = 100
+    C, K, H, Q, L = 16, 4, 8, 3, 2
+    off = torch.zeros(B + 1, dtype=torch.int32, device=gpu)
+    off[1:] = torch.cumsum(n, 0)
+    N = int(off[-1])
+    graph = torch.repeat_interleave(torch.arange(B, device=gpu), n)
+    ring = torch.arange(N, device=gpu) + 1
+    ring = torch.where(ring == off[1:][graph], off[:-1][graph].long(), ring).int()
+    A = (torch.arange(N + 1, device=gpu).int(), ring, torch.ones(N, device=gpu))
+    S = (off, torch.arange(N, device=gpu).int(), torch.ones(N, device=gpu))
+    normal = lambda *shape: torch.randn(*shape, generator=gen, device=gpu)
+    X, Wn, Wc, W1, W2 = normal(N, K), normal(K, C), normal(C, C) * 0.3, normal(C, H), normal(H, Q)
+    got = ops.s2v_forward_batched(A, S, X, Wn, Wc, W1, W2, L, int(n.max()))
+    one_by_one, h = ops.s2v_forward_batched_train(A, S, X, Wn, Wc, W1, W2, L, int(n.max()))
+    assert torch.equal(got.msg, one_by_one.msg) and torch.equal(got.h_final, h[L])
+    zero = torch.zeros(B, C, dtype=torch.float64, device=gpu)
+    pool = zero.index_add(0, graph, h[L].double())               # embeddings are not negative: the sum is that of its terms' magnitudes
+    assert bool(((got.pool.double() - pool).abs() <= 130 * 2.0 ** -24 * pool).all())
+    want = (got.pool.double() @ W1.double()).clamp(min=0)
+    assert bool(((got.hidden.double() - want).abs() <= (C + 4) * 2.0 ** -24 * (got.pool.double() @ W1.double().abs())).all())
+    want = got.hidden.double() @ W2.double()
+    assert bool(((got.logits.double() - want).abs() <= (H + 4) * 2.0 ** -24 * (got.hidden.double() @ W2.double().abs())).all())
+    assert int(got.status.item()) == 0
+
+
 @pytest.mark.parametrize("average", [False, True])
 def test_device_csr_of_consecutive_rows(gpu, oracle, average):
     """the pooling operand of a batch whose nodes were added subgraph after subgraph, from the subgraph offsets alone:
