@@ -75,6 +75,15 @@ __global__ __launch_bounds__(kBlock, 3) void s2v_rows_kernel(RowsArgs a)
         for (int b = 0; b < NB; ++b) {
             if (b >= nb) continue;                             // uniform
             const int col = 16 * (wave + kWaves * b) + t;
+            if constexpr (WT) {
+                // a lane's four k lie next to each other: one load instead of four, which matters where the rows of W are far apart
+                // (backward at 48,750 nodes: hidden 120 47.8 -> 43.8 us, 160 109 -> 69, 199 105 -> 90)
+                if (k0 + 16 <= K) {                            // uniform
+                    const float4 w = V::load(a.W + (size_t)min(col, n - 1) * K + k0 + 4 * q);
+                    wf[b][0] = w.x; wf[b][1] = w.y; wf[b][2] = w.z; wf[b][3] = w.w;
+                    continue;
+                }
+            }
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
                 const int k = k0 + 4 * q + s;
