@@ -46,9 +46,9 @@ struct RowsArgs {
     HubPlan hubs;
 };
 
-// GATHER: the left operand is A * x.  WT: the product is with W^T.
-template <int RT, int NB, bool GATHER, bool WT>
-__global__ __launch_bounds__(kBlock, 3) void s2v_rows_kernel(RowsArgs a)
+// GATHER: the left operand is A * x.  WT: the product is with W^T.  MINW: wavefronts per SIMD the registers leave room for.
+template <int RT, int NB, int MINW, bool GATHER, bool WT>
+__global__ __launch_bounds__(kBlock, MINW) void s2v_rows_kernel(RowsArgs a)
 {
     using V = ColsLoose;
     constexpr int R = 16 * RT;
@@ -300,27 +300,40 @@ __global__ __launch_bounds__(kBlock, 3) void s2v_rows_kernel(RowsArgs a)
     }
 }
 
-template <int RT, int NB, bool GATHER, bool WT>
+template <int RT, int NB, int MINW, bool GATHER, bool WT>
 int launch_rows(const RowsArgs& a, hipStream_t s)
 {
     const int KP = (a.K + 15) & ~15;
     const int width = KP + 4 > a.n ? KP + 4 : a.n;
     const unsigned grid = (unsigned)(((long long)a.N + 16 * RT - 1) / (16 * RT));
-    hipLaunchKernelGGL((s2v_rows_kernel<RT, NB, GATHER, WT>), dim3(grid), dim3(kBlock), sizeof(float) * 16 * RT * width, s, a);
+    hipLaunchKernelGGL((s2v_rows_kernel<RT, NB, MINW, GATHER, WT>), dim3(grid), dim3(kBlock), sizeof(float) * 16 * RT * width, s, a);
     GNNHIP_LAUNCH_CHECK("s2v_rows");
     return GNNHIP_OK;
+}
+
+// Rows per tile for products of up to 128 columns.  Few rows: 16, so that there is a workgroup for every compute unit.  Many: 64, which
+// use every fetched word of W four times.  In between the tiles of 64 rows leave each compute unit one or two workgroups,
+// whose phases have nothing to hide behind, and 32 rows are the better ones (hidden 85, 22,000 nodes: 21.0 -> 15.4 us per
+// level, 24.7 -> 18.3 backward; 38,000: 29.7 -> 24.5), up to the 49,152 rows that six workgroups per compute unit hold at once
+// where the registers allow so many (from 40,960 on: 48,750 nodes, hidden 36 to 100 6 to 12 % less; below, the registers
+// that this takes away cost 3 %).  51,000 nodes take two rounds: 2 to 8 % slower than 64 rows.
+template <int NB, bool GATHER, bool WT>
+int rows_by_tile(const RowsArgs& a, hipStream_t s)
+{
+    if (a.N < 64 * kNumCU) return launch_rows<1, NB, 3, GATHER, WT>(a, s);
+    if (a.N < 160 * kNumCU) return launch_rows<2, NB, 3, GATHER, WT>(a, s);
+    if (a.N <= 6 * 32 * kNumCU) return launch_rows<2, NB, 6, GATHER, WT>(a, s);
+    return launch_rows<4, NB, 3, GATHER, WT>(a, s);
 }
 
 template <bool GATHER, bool WT>
 int rows_dispatch(RowsArgs a, hipStream_t s)
 {
     a.k_magic = a.K >= 2 ? (unsigned)(((1ull << 32) + a.K - 1) / a.K) : 0;
-    // Few rows: the smallest tiles, so that there is a workgroup for every compute unit; else 64 rows, which use every
-    // fetched word of W four times, or 32 where the tile would leave room for two workgroups per compute unit.
-    const bool few = a.N < 64 * kNumCU;
-    if (a.n <= 64) return few ? launch_rows<1, 1, GATHER, WT>(a, s) : launch_rows<4, 1, GATHER, WT>(a, s);
-    if (a.n <= 128) return few ? launch_rows<1, 2, GATHER, WT>(a, s) : launch_rows<4, 2, GATHER, WT>(a, s);
-    return few ? launch_rows<1, 4, GATHER, WT>(a, s) : launch_rows<2, 4, GATHER, WT>(a, s);
+    if (a.n <= 64) return rows_by_tile<1, GATHER, WT>(a, s);
+    if (a.n <= 128) return rows_by_tile<2, GATHER, WT>(a, s);
+    // wider: 32 rows, where the tile leaves room for two workgroups per compute unit
+    return a.N < 64 * kNumCU ? launch_rows<1, 4, 3, GATHER, WT>(a, s) : launch_rows<2, 4, 3, GATHER, WT>(a, s);
 }
 
 }  // namespace

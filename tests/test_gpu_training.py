@@ -437,6 +437,36 @@ def test_level_of_a_small_batch_has_the_bits_of_a_large_one(gpu, C, N):
         assert a is None or torch.equal(acc, acc_more[:N])
 
 
+@pytest.mark.parametrize("C", [5, 36, 100, 127])
+def test_level_of_any_hidden_size_has_the_same_bits_whatever_the_tile(gpu, C):
+    """levels of hidden sizes without a kernel of their own take 16, 32 or 64 rows per workgroup by the number of rows: the same rows
+    followed by empty ones, up to and past each of the turns, give the same bits forward, backward and in the input stage"""
+    import torch
+    from graphnn_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(C)
+    normal = lambda *shape: torch.randn(*shape, generator=gen, device=gpu)
+    most, N = 49_153, 1003
+    # (rows of more than 64 entries change their order with the balanced pass, from 32,768 rows on)
+    lens = torch.tensor([0, 4, 5, 2, 8, 9, 1, 16, 17, 3, 48, 49, 0, 64, 2, 2, 1], device=gpu).repeat(N // 17 + 1)[:N]
+    rp = torch.zeros(N + 1, dtype=torch.int32, device=gpu)
+    rp[1:] = torch.cumsum(lens, 0)
+    nnz = int(rp[-1])
+    ci, v = torch.randint(0, N, (nnz,), generator=gen, device=gpu).int(), normal(nnz)
+    h, W, msg, gate, acc0, X, Wn = normal(most, C), normal(C, C) * 0.2, normal(most, C), normal(most, C), normal(most, C), normal(most, 9), normal(9, C)
+    want = None
+    for n in (N, 16_383, 16_384, 20_001, 40_959, 40_960, 49_152, 49_153):
+        rows = torch.cat([rp, rp[-1:].expand(n - N)])
+        acc = acc0[:n].clone()
+        u, g = ops.s2v_level_backward(rows, ci, v, h[:n], W, gate_h=gate[:n], acc=acc)
+        got = [ops.s2v_level(rows, ci, v, h[:n], W, msg[:n]), u, g, acc, *ops.s2v_input(X[:n], Wn)]
+        # rows behind the matrix's own: no entries (ReLU(msg), nothing, zero, the old sum), and the last row of every size
+        assert torch.equal(got[0][N:], msg[N:n].clamp(min=0)) and not bool(u[N:].any()) and not bool(g[N:].any()) and torch.equal(acc[N:], acc0[N:n])
+        assert torch.equal(got[5], got[4].clamp(min=0))
+        if want is None:
+            want = got
+        assert all(torch.equal(x[:N], y[:N]) for x, y in zip(got, want)), n
+
+
 @pytest.mark.parametrize("C", [128, 256])
 @pytest.mark.parametrize("N", [5003, 40_009])
 @pytest.mark.parametrize("kind", ["zero_mean", "relu", "one_sign"])
