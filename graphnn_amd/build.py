@@ -61,7 +61,7 @@ def build_bindings(force=True):
            "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, "-w",
            "-I", os.path.join(ROOT, "include"), "-isystem", os.path.join(base, "include"), "-isystem", "/opt/rocm/include",
            "-isystem", sysconfig.get_paths()["include"], BINDINGS_SOURCE, "-o", BINDINGS,
-           "-L", os.path.join(base, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ldl"]
+           "-L", os.path.join(base, "lib"), "-ltorch_python", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", "-ldl"]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("g++ failed on %s:\n%s\n%s" % (BINDINGS_SOURCE, r.stdout, r.stderr))

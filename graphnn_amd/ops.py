@@ -48,7 +48,8 @@ def _bound():
 
 
 def _empty(where, kind, *sizes):
-    """uninitialised tensor of float32 ('f') or int32 ('i') on the device of a tensor, or on a torch.device"""
+    """uninitialised tensor of float32 ('f') or int32 ('i') on the device of a tensor, or on a torch.device; several letters: a
+    tuple of vectors ('f', 'i') and float32 matrices ('F'), each taking its sizes in turn"""
     return _bound().empty(where, kind, *sizes)
 
 
@@ -610,10 +611,7 @@ def csr_group(rows, key, payload, average=False, key_stride=1, payload_stride=1,
     """row i lists payload[e] of the pairs with key[e] == i in input order (device arrays, int32)"""
     if n is None:
         n = key.numel() // key_stride
-    dev = key.device
-    row_ptr = _empty(dev, "i", rows + 1)
-    col_idx = _empty(dev, "i", n)
-    val = _empty(dev, "f", n)
+    row_ptr, col_idx, val = _empty(key, "iif", rows + 1, n, n)
     _bound().csr_group_i32(rows, n, key, key_stride, payload, payload_stride,
                                       int(average), row_ptr, col_idx, val)
     return row_ptr, col_idx, val
@@ -623,15 +621,11 @@ def csr_group_both(rows, x, y, x_stride=1, y_stride=1, n=None):
     """the pairs (x, y) grouped by y (row i lists x) and by x (row i lists y): a matrix and its transpose, values 1"""
     if n is None:
         n = x.numel() // x_stride
-    dev = x.device
-    out = []
-    for _ in range(2):
-        out += [_empty(dev, "i", rows + 1), _empty(dev, "i", n),
-                _empty(dev, "f", n)]
+    out = _empty(x, "iifiif", rows + 1, n, n, rows + 1, n, n)
     _bound().csr_group_both_i32(rows, n, x, x_stride, y, y_stride,
                                            out[0], out[1], out[2],
                                            out[3], out[4], out[5])
-    return tuple(out[:3]), tuple(out[3:])
+    return out[:3], out[3:]
 
 
 def csr_consecutive_rows(row_ptr, average=False):
@@ -650,11 +644,8 @@ def csr_consecutive_rows_host(offsets, device, average=False):
     offsets = np.ascontiguousarray(offsets, np.int32)
     rows, n = offsets.size - 1, int(offsets[-1])
     device = torch.device(device)
-    row_ptr = _empty(device, "i", rows + 1)
-    col_idx = _empty(device, "i", n)
-    val = _empty(device, "f", n)
-    _bound().csr_consecutive_rows_host_f32(rows, offsets.__array_interface__["data"][0], int(average), row_ptr,
-                                                      col_idx if n else None, val if n else None)
+    row_ptr, col_idx, val = _empty(device, "iif", rows + 1, n, n)
+    _bound().csr_consecutive_rows_host_f32(rows, offsets, int(average), row_ptr, col_idx if n else None, val if n else None)
     return row_ptr, col_idx, val
 
 
@@ -673,12 +664,8 @@ def csr_transpose(row_ptr, col_idx, val, m, k):
 def loss_acc(logits, lrow_ptr, lcol, lval, want_rows=False):
     """mean cross-entropy (softmax inside) and mean top-1 accuracy of a batch in one pass over the logits"""
     B, Q = logits.shape
-    dev = logits.device
-    probs = _empty(logits, "f", B, Q)
-    loss = _empty(dev, "f", 1)
-    acc = _empty(dev, "f", 1)
-    loss_rows = _empty(dev, "f", B) if want_rows else None
-    hit = _empty(dev, "i", B) if want_rows else None
+    probs, loss, acc = _empty(logits, "Fff", B, Q, 1, 1)
+    loss_rows, hit = _empty(logits, "fi", B, B) if want_rows else (None, None)
     _bound().s2v_loss_acc_f32(B, Q, logits, lrow_ptr, lcol,
                                          lval, probs, loss_rows,
                                          hit, loss, acc)
@@ -688,10 +675,7 @@ def loss_acc(logits, lrow_ptr, lcol, lval, want_rows=False):
 def readout_backward(s_csr, probs, label_csr, scale, hidden, W_h1, W_h2, N):
     B, Q = probs.shape
     C, H = W_h1.shape
-    dev = probs.device
-    dlogits = _empty(dev, "f", B, Q)
-    du = _empty(dev, "f", B, H)
-    g_h = _empty(dev, "f", N, C)
+    dlogits, du, g_h = _empty(probs, "FFF", B, Q, B, H, N, C)
     _bound().s2v_readout_backward_f32(
         B, N, C, H, Q, s_csr[0], s_csr[1], s_csr[2],
         probs, label_csr[0], label_csr[1], label_csr[2],

@@ -128,3 +128,20 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(binding, "_LIB_PATH", str(tmp_path / "libgnnhip.so"))
     with pytest.raises(RuntimeError, match="no CPU fallback"):
         binding.load_library()
+
+
+def test_bindings_make_empty_tensors_of_every_kind():
+    """one letter: a tensor of the sizes given; several: a tuple, each taking its sizes in turn; too few or too many are refused"""
+    import torch
+    from graphnn_amd import _lib
+    empty = _lib.load_bindings().empty
+    cpu = torch.device("cpu")
+    one = empty(cpu, "f", 2, 3, 4)
+    assert one.shape == (2, 3, 4) and one.dtype == torch.float32 and one.is_contiguous()
+    a, b, c = empty(one, "iFf", 3, 4, 5, 0)
+    assert (a.shape, b.shape, c.shape) == ((3,), (4, 5), (0,)) and (a.dtype, b.dtype, c.dtype) == (torch.int32, torch.float32, torch.float32)
+    for bad in (("ff", 3), ("f", 1, 2, 3, 4), ("F" "f", 3, 4)):
+        with pytest.raises(TypeError):
+            empty(cpu, *bad)
+    with pytest.raises(RuntimeError):
+        empty(cpu, "f", -2)

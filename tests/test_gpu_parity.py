@@ -2414,3 +2414,24 @@ def test_sparse_upload_rebuilds_the_same_bits(gpu, shape, density):
     # int32 data takes the same route
     b = np.where(rng.random(50_000) < 0.02, rng.integers(-9, 9, 50_000), 0).astype(np.int32)
     assert np.array_equal(ops.upload_sparse32(b).cpu().numpy(), b)
+
+
+def test_bindings_make_tensors_as_torch_does(gpu):
+    """device, type and layout of torch.empty's tensors, in inference mode and under deterministic algorithms (which fill
+    them) too"""
+    import torch
+    from graphnn_amd import ops
+    def check(t, like):
+        assert t.device == like.device and t.dtype == like.dtype and t.shape == like.shape and t.stride() == like.stride()
+        assert t.requires_grad == like.requires_grad and t.is_inference() == like.is_inference()
+    where = torch.empty(1, device=gpu)
+    with torch.inference_mode():
+        check(ops._empty(where, "f", 3, 5), torch.empty(3, 5, device=gpu))
+    i, f = ops._empty(where, "iF", 7, 2, 3)
+    check(i, torch.empty(7, dtype=torch.int32, device=gpu))
+    check(f, torch.empty(2, 3, device=gpu))
+    torch.use_deterministic_algorithms(True)
+    try:
+        assert bool(torch.isnan(ops._empty(where, "f", 1000)).all())
+    finally:
+        torch.use_deterministic_algorithms(False)
