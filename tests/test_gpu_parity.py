@@ -1710,6 +1710,22 @@ def test_spmm_column_ordered_pieces_on_a_power_law_matrix(gpu, oracle, n):
         assert_parity("spmm", got_h, *_spmm_want(oracle, *csr, B, N, alpha=-0.5, beta=1.5, C=C0))
 
 
+@pytest.mark.parametrize("k", [1, 256, 257, 1 << 20, (1 << 20) + 1])
+def test_spmm_pieces_whatever_bits_their_order_takes(gpu, oracle, k):
+    """rows cut into pieces, as above, with as many columns as the eight bits their order takes up to 2^20 columns, one more,
+    and either side of that line; rows of at most 32 entries have the bits of the row-order sums whatever the order"""
+    from graphnn_amd import ops
+    rng = np.random.default_rng(k)
+    m, n = 32768, 32
+    deg = rng.integers(4, 33, m)
+    row_ptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    col = rng.integers(0, k, row_ptr[-1]).astype(np.int32)
+    val = np.ones(col.size, np.float32)               # products without rounding: the oracle's are not fused with its sums
+    B = rng.standard_normal((k, n)).astype(np.float32)
+    got = _n(ops.spmm(*_csr_t((row_ptr, col, val), gpu), _t(B, gpu), m))
+    assert np.array_equal(got, oracle.spmm(row_ptr, col, val, B, m))
+
+
 @pytest.mark.parametrize("n", [64, 128, 36, 9, 4, 300, 1100])
 def test_spmm_with_a_plan_has_the_bits_of_the_call_without(gpu, oracle, n):
     """gnnhip_csr_plan_create + gnnhip_spmm_csr_planned_f32 on the power-law matrix of the test above: the plan sizes its
