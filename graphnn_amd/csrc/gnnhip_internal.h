@@ -290,8 +290,10 @@ int spmm_dispatch(int m, int k, int n, long long nnz, float alpha, const int* ro
                   CsrPlan* plan = nullptr, bool relu_in = false);
 
 // sort.hip
-int exclusive_scan_i32(int* x, long long n, int* seg_scratch, hipStream_t s);
-int exclusive_scan_pair_i32(int* x, int* y, long long n, int* seg_scratch, hipStream_t s);
+constexpr int kScanSeg = 1024;          // elements whose sum a scan takes as one
+inline size_t scan_seg_ints(long long n) { return (size_t)((n + kScanSeg - 1) / kScanSeg); }
+int scan_from_sums_i32(int* x, long long n, int* seg, hipStream_t s);
+int scan_pair_from_sums_i32(int* x, int* y, long long n, int* seg, hipStream_t s);
 size_t radix_hist_ints(long long n);
 size_t radix_seg_ints(long long n);
 int radix_order(unsigned* keys, int bits, long long n, unsigned* keys_out, unsigned* spare, unsigned* order, int* hist, int* seg, hipStream_t s);

@@ -43,18 +43,44 @@ __device__ __forceinline__ int pieces_of(int deg) { return (deg + kPiece - 1) / 
 // is 0, so that the scans leave the totals there).  The host's entry count `cap` sizes every array of the plan; should
 // the matrix hold more entries than that, a row that reaches past entry `cap` (the last rows) is one piece whatever
 // its length: no entries are copied for it, and piece_tail forms the row's result from the CSR arrays.
-__global__ __launch_bounds__(kBlock) void piece_count_kernel(int m, const int* __restrict__ row_ptr, int cap, int* __restrict__ counts,
-                                                             int* __restrict__ pcounts)
+// A workgroup takes the kScanSeg elements of one segment of the scans that follow and leaves their sums (seg, and pseg).
+__device__ __forceinline__ int group_sum(int v)
 {
-    for (long long r = (long long)blockIdx.x * kBlock + threadIdx.x; r <= m; r += (long long)gridDim.x * kBlock) {
+    __shared__ int part[kBlock / kWave];
+    v = wave_sum_i(v);
+    __syncthreads();                                 // part may hold an earlier sum
+    if ((threadIdx.x & (kWave - 1)) == 0) part[threadIdx.x / kWave] = v;
+    __syncthreads();
+    v = 0;
+#pragma unroll
+    for (int w = 0; w < kBlock / kWave; ++w) v += part[w];
+    return v;
+}
+
+__global__ __launch_bounds__(kBlock) void piece_count_kernel(int m, const int* __restrict__ row_ptr, int cap, int* __restrict__ counts,
+                                                             int* __restrict__ pcounts, int* __restrict__ seg, int* __restrict__ pseg)
+{
+    static_assert(kScanSeg == kBlock * 4, "four rows per lane");
+    int sum = 0, psum = 0;
+    const long long base = (long long)blockIdx.x * kScanSeg + threadIdx.x;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const long long r = base + i * kBlock;
         int c = 0;
         if (r < m) {
             const int e0 = row_ptr[r], e1 = row_ptr[r + 1];
             c = e1 <= cap ? pieces_of(e1 - e0) : (e1 > e0 ? 1 : 0);
         }
+        if (r > m) continue;
+        const int pc = c > 1 ? c : 0;
         counts[r] = c;
-        pcounts[r] = c > 1 ? c : 0;
+        pcounts[r] = pc;
+        sum += c;
+        psum += pc;
     }
+    sum = group_sum(sum);
+    psum = group_sum(psum);
+    if (threadIdx.x == 0) { seg[blockIdx.x] = sum; pseg[blockIdx.x] = psum; }
 }
 
 // One lane per piece slot: the row that owns piece id is found by bisection in the scanned counts.
@@ -92,18 +118,27 @@ __global__ __launch_bounds__(kBlock) void piece_fill_kernel(int m, long long slo
 // lens[i] = entries of the i-th piece in order (lens[slots] = 0, so that the scan leaves the total there);
 // target[i]: where the sum of the i-th piece in order goes: the row r >= 0 when the piece is all of that row,
 // else -1 - (its place among the partial sums; a stand-in piece without entries and without place gets a place past the
-// end, which the sum kernel recognises).  order[i] = id of the i-th piece in order; ordered[i] = its record.
-__global__ __launch_bounds__(kBlock) void piece_place_kernel(long long slots, long long pslots, const unsigned* __restrict__ order,
+// end, which the sum kernel recognises).  order[i] = id of the i-th piece in order; ordered[i] = its record.  The sums of the lengths go to
+// seg as the counts' do.
+__global__ __launch_bounds__(kBlock) void piece_place_kernel(long long slots, const unsigned* __restrict__ order,
                                                              const PieceRec* __restrict__ rec, PieceRec* __restrict__ ordered,
-                                                             int* __restrict__ lens, int* __restrict__ target)
+                                                             int* __restrict__ lens, int* __restrict__ target, int* __restrict__ seg)
 {
-    for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i <= slots; i += (long long)gridDim.x * kBlock) {
-        if (i == slots) { lens[i] = 0; continue; }
+    int sum = 0;
+    const long long base = (long long)blockIdx.x * kScanSeg + threadIdx.x;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const long long i = base + u * kBlock;
+        if (i == slots) lens[i] = 0;
+        if (i >= slots) continue;
         const PieceRec r = rec[order[i]];
         ordered[i] = r;
         lens[i] = r.end - r.start;
         target[i] = r.row >= 0 ? r.row : (r.id >= 0 ? -1 - r.id : kNoPlace);
+        sum += r.end - r.start;
     }
+    sum = group_sum(sum);
+    if (threadIdx.x == 0) seg[blockIdx.x] = sum;
 }
 
 // Entries copied into piece order: half a wavefront per piece (kPiece = 32 entries, one per lane), four pieces
@@ -424,7 +459,7 @@ Layout layout_of(int m, long long nnz, long long slots, long long pslots)
     L.body_bytes = off;
     off = 0;
     const size_t longest = (size_t)(slots + 1 > (long long)m + 1 ? slots + 1 : (long long)m + 1);
-    L.o_seg = carve(sizeof(int) * (2 * (longest / 4096 + 2) + radix_seg_ints(slots)));
+    L.o_seg = carve(sizeof(int) * std::max(2 * scan_seg_ints((long long)longest), radix_seg_ints(slots)));
     L.o_rec = carve(sizeof(PieceRec) * (size_t)slots);
     L.o_ord = carve(sizeof(PieceRec) * (size_t)slots);
     L.o_keys = carve(sizeof(unsigned) * (size_t)slots);
@@ -441,8 +476,10 @@ constexpr unsigned kElemGrid = kNumCU * 16;
 // pieces per row and their scans: first, pfirst (the totals end up in entry m of each)
 int count_pieces(CsrPlan* p, int cap, int* seg, hipStream_t s)
 {
-    hipLaunchKernelGGL(piece_count_kernel, dim3(kElemGrid), dim3(kBlock), 0, s, p->m, p->row_ptr, cap, p->first, p->pfirst);
-    if (int rc = exclusive_scan_pair_i32(p->first, p->pfirst, (long long)p->m + 1, seg, s)) return rc;
+    const long long n = (long long)p->m + 1;
+    const size_t nseg = scan_seg_ints(n);
+    hipLaunchKernelGGL(piece_count_kernel, dim3((unsigned)nseg), dim3(kBlock), 0, s, p->m, p->row_ptr, cap, p->first, p->pfirst, seg, seg + nseg);
+    if (int rc = scan_pair_from_sums_i32(p->first, p->pfirst, n, seg, s)) return rc;
     GNNHIP_LAUNCH_CHECK("spmm_pieces count");
     return GNNHIP_OK;
 }
@@ -473,8 +510,9 @@ int order_pieces(CsrPlan* p, int cap, const Layout& L, char* temp, hipStream_t s
                        p->pfirst, shift, (1u << order_bits) - 1, rec, keys);
     // order[i] = id of the piece that comes i-th by the top order_bits bits of its first column, equal ones by id
     if (int rc = radix_order(keys, order_bits, p->slots, keys2, perm, order, hist, seg, s)) return rc;
-    hipLaunchKernelGGL(piece_place_kernel, dim3(kElemGrid), dim3(kBlock), 0, s, p->slots, p->pslots, order, rec, ordered, p->at, p->target);
-    if (int rc = exclusive_scan_i32(p->at, p->slots + 1, seg, s)) return rc;
+    hipLaunchKernelGGL(piece_place_kernel, dim3((unsigned)scan_seg_ints(p->slots + 1)), dim3(kBlock), 0, s, p->slots, order, rec, ordered, p->at,
+                       p->target, seg);
+    if (int rc = scan_from_sums_i32(p->at, p->slots + 1, seg, s)) return rc;
     hipLaunchKernelGGL(piece_gather_kernel, dim3(kElemGrid), dim3(kBlock), 0, s, p->first + p->m, ordered, p->at, p->col_idx, p->val,
                        p->col_ord, p->val_ord);
     GNNHIP_LAUNCH_CHECK("spmm_pieces plan");
@@ -683,7 +721,7 @@ extern "C" int gnnhip_csr_plan_create(int m, int k, const int* row_ptr, const in
         Layout L = layout_of(m, nnz, 1, 1);
         if (int rc = pool_acquire_exact(&p->head_block, L.head_bytes)) return fail(rc);
         void* segp = nullptr;
-        if (int rc = stream_scratch(s, sizeof(int) * ((size_t)m / 4096 + 4), &segp)) return fail(rc);
+        if (int rc = stream_scratch(s, sizeof(int) * 2 * scan_seg_ints((long long)m + 1), &segp)) return fail(rc);
         point_plan(p, L, static_cast<char*>(p->head_block), nullptr);
         if (int rc = count_pieces(p, nnz, static_cast<int*>(segp), s)) return fail(rc);
         int totals[2] = {0, 0};

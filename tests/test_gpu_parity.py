@@ -1726,6 +1726,28 @@ def test_spmm_pieces_whatever_bits_their_order_takes(gpu, oracle, k):
     assert np.array_equal(got, oracle.spmm(row_ptr, col, val, B, m))
 
 
+@pytest.mark.parametrize("m", [33_790, 33_791, 33_792, 34_000, 2_097_153])
+def test_spmm_pieces_at_the_edges_of_their_scans(gpu, m):
+    """rows whose counts fill segments of 1,024 to the last element, pass one by an element, and pass the 2,048 segments that a
+    workgroup adds up by itself; small whole numbers, whose sums are exact in any order, against the sums of 64-bit integers"""
+    from graphnn_amd import ops
+    import torch
+    n = 32
+    gen = torch.Generator(device=gpu).manual_seed(m)
+    deg = torch.randint(0, 29, (m,), device=gpu, generator=gen)
+    deg[m // 2] = 5_000
+    deg[-1] = 40
+    row_ptr = torch.cat([torch.zeros(1, dtype=torch.int64, device=gpu), deg.cumsum(0)])
+    col = torch.randint(0, m, (int(row_ptr[-1]),), device=gpu, generator=gen)
+    assert col.numel() >= 12 * m
+    B = torch.randint(-8, 9, (m, n), device=gpu, generator=gen)
+    got = ops.spmm(row_ptr.int(), col.int(), torch.ones(col.numel(), device=gpu), B.float(), m)
+    for at in range(0, n, 8):                                 # differences of running sums, a few columns at a time
+        run = torch.cat([torch.zeros(1, 8, dtype=torch.int64, device=gpu), B[:, at:at + 8][col].cumsum(0)])
+        assert torch.equal(got[:, at:at + 8].long(), run[row_ptr[1:]] - run[row_ptr[:-1]]), at
+        del run
+
+
 @pytest.mark.parametrize("n", [64, 128, 36, 9, 4, 300, 1100])
 def test_spmm_with_a_plan_has_the_bits_of_the_call_without(gpu, oracle, n):
     """gnnhip_csr_plan_create + gnnhip_spmm_csr_planned_f32 on the power-law matrix of the test above: the plan sizes its
@@ -2197,6 +2219,24 @@ def test_device_csr_group_at_the_edges_of_its_workgroups(gpu, n, rows):
             got = ops.csr_group(rows, key_d, _t(pay, gpu))
             for g, w in zip(got, want):
                 assert np.array_equal(_n(g), w), (order, shift)
+
+
+@pytest.mark.parametrize("n", [65_536, 67_584, 67_585, 8_192 * 2_048, 8_192 * 2_048 + 1])
+def test_device_csr_group_at_the_edges_of_its_scans(gpu, n):
+    """the sort's counters in whole segments of 1,024 and in a part of one more, and either side of the 2,048 segments that a
+    workgroup adds up by itself; the bits of the stable sort"""
+    from graphnn_amd import ops
+    import torch
+    rows = 50_000
+    gen = torch.Generator(device=gpu).manual_seed(n)
+    key = torch.randint(0, rows, (n,), dtype=torch.int32, device=gpu, generator=gen)
+    pay = torch.randint(0, 1 << 30, (n,), dtype=torch.int32, device=gpu, generator=gen)
+    row_ptr, col_idx, val = ops.csr_group(rows, key, pay)
+    kept, order = torch.sort(key, stable=True)
+    ends = torch.searchsorted(kept, torch.arange(rows + 1, dtype=torch.int32, device=gpu))
+    assert torch.equal(row_ptr.long(), ends)
+    assert torch.equal(col_idx, pay[order])
+    assert bool((val == 1).all())
 
 
 @pytest.mark.parametrize("B", [40, 600])
