@@ -89,6 +89,37 @@ def test_readout_backward(gpu, oracle, C, H, Q, B):
     assert_parity("g_h", _n(gh), w_gh, gh64)
 
 
+@pytest.mark.parametrize("C", [1, 4, 6, 100, 500, 1024, 1028])
+def test_readout_backward_rows_whatever_the_width(gpu, oracle, C):
+    """the node rows written as 128-bit words (a width that is a multiple of four, at most 1,024, into a buffer that starts on
+    one) and element by element, graphs of more rows than the lanes hold list entries of: the same bits, and the oracle's"""
+    import torch
+    from graphnn_amd import ops
+    rng = np.random.default_rng(C)
+    sizes = np.array([1, 7, 8, 9, 64, 65, 300, 2])
+    B, H, Q, N = sizes.size, 9, 3, int(sizes.sum())
+    s = (np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32), rng.permutation(N).astype(np.int32), rng.random(N).astype(np.float32))
+    lab = (np.arange(B + 1, dtype=np.int32), rng.integers(0, Q, B).astype(np.int32), np.ones(B, np.float32))
+    probs = oracle.row_softmax(rng.standard_normal((B, Q)).astype(np.float32))
+    hidden = np.maximum(rng.standard_normal((B, H)), 0).astype(np.float32)
+    W1 = (rng.standard_normal((C, H)) * 0.2).astype(np.float32)
+    W2 = (rng.standard_normal((H, Q)) * 0.2).astype(np.float32)
+    dev = [_t(a, gpu) for a in (*s, probs, *lab)]
+    hid, w1, w2 = _t(hidden, gpu), _t(W1, gpu), _t(W2, gpu)
+    got = []
+    for shift in (0, 1):
+        dl, du = torch.empty(B, Q, device=gpu), torch.empty(B, H, device=gpu)
+        gh = torch.zeros(N * C + shift, device=gpu)[shift:].view(N, C)
+        ops._bound().s2v_readout_backward_f32(B, N, C, H, Q, *dev, 0.25, hid, w1, w2, dl, du, gh)
+        got.append(_n(gh))
+    assert np.array_equal(got[0], got[1])
+    du64 = _n(du).astype(np.float64)
+    w_gh = oracle.spmm_T(*s, oracle.gemm(_n(du), W1, transB=True), B, N)
+    gh64 = np.zeros((N, C))
+    gh64[s[1]] = np.repeat(du64 @ W1.astype(np.float64).T, sizes, axis=0) * s[2][:, None]
+    assert_parity("g_h", got[0], w_gh, gh64)
+
+
 @pytest.mark.parametrize("N,C", [(N, C) for C in (16, 32, 64, 128, 256) for N in (77, 7450, 40_000)] + [(70_001, 128), (70_001, 256), (16_400, 256)])
 def test_level_backward(gpu, oracle, C, N):
     """u = A^T dz and g_prev = u W^T in one pass (hidden 16/32/64: the streaming kernel; hidden 128/256: the wide kernel's
