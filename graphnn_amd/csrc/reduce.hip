@@ -126,6 +126,7 @@ __global__ __launch_bounds__(kBlock) void jagged_softmax_kernel(float* x, const 
 // segments itself (a few KB from L2) instead of waiting for a scan launch (4,096 segments of 1,024: 14 -> 9 us).
 // A workgroup takes the kWavesPerBlock consecutive segments starting at blockIdx.x * kWavesPerBlock.
 constexpr int kFusedJaggedMaxSegments = 8192;
+constexpr int kBlockJaggedMaxSegments = 1024;
 __global__ __launch_bounds__(kBlock) void jagged_softmax_fused_kernel(float* x, const int* __restrict__ lens, int nseg)
 {
     __shared__ long long wave_part[kWavesPerBlock];
@@ -148,6 +149,83 @@ __global__ __launch_bounds__(kBlock) void jagged_softmax_fused_kernel(float* x, 
     if (seg >= nseg) return;
     for (int w = 0; w < wave; ++w) base += lens[first + w];
     wave_softmax_inplace(x + base, lens[seg], lane);
+}
+
+// Softmax of one contiguous run by a workgroup.  A lane holds HOLD elements, the loads of all of them in flight together: runs of
+// up to kBlock * HOLD elements are read once, longer ones in steps of as many, three times.
+template <int HOLD>
+__device__ __forceinline__ void block_softmax_inplace(float* x, long long len, float (*part)[kWavesPerBlock])
+{
+    constexpr int kStep = kBlock * HOLD;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    const float first = x[0];                         // reference scan starts at element 0
+    float v[HOLD], mx = first;
+    auto load = [&](long long at) {
+#pragma unroll
+        for (int k = 0; k < HOLD; ++k) v[k] = at + tid + k * kBlock < len ? x[at + tid + k * kBlock] : first;   // the filler cannot change the maximum
+    };
+    auto store = [&](long long at) {
+#pragma unroll
+        for (int k = 0; k < HOLD; ++k) if (at + tid + k * kBlock < len) x[at + tid + k * kBlock] = v[k];
+    };
+    for (long long at = 0; at < len; at += kStep) {
+        load(at);
+#pragma unroll
+        for (int k = 0; k < HOLD; ++k) mx = max_keep(mx, v[k]);
+    }
+    mx = wave_max(mx);
+    if (lane == 0) part[0][wave] = mx;
+    __syncthreads();                                  // x[0] is rewritten from here on
+    mx = part[0][0];
+#pragma unroll
+    for (int w = 1; w < kWavesPerBlock; ++w) mx = max_keep(mx, part[0][w]);
+    float s = 0.f;
+    for (long long at = 0; at < len; at += kStep) {
+        if (len > kStep) load(at);
+#pragma unroll
+        for (int k = 0; k < HOLD; ++k) {
+            if (at + tid + k * kBlock < len) {
+                v[k] = expf(v[k] - mx);
+                s += v[k];
+            }
+        }
+        if (len > kStep) store(at);
+    }
+    s = wave_sum(s);
+    if (lane == 0) part[1][wave] = s;
+    __syncthreads();
+    s = part[1][0];
+#pragma unroll
+    for (int w = 1; w < kWavesPerBlock; ++w) s += part[1][w];
+    for (long long at = 0; at < len; at += kStep) {
+        if (len > kStep) load(at);
+#pragma unroll
+        for (int k = 0; k < HOLD; ++k) v[k] = v[k] / s;
+        store(at);
+    }
+}
+
+// Few segments: a workgroup each, which finds its offset as above.  A wavefront alone with a segment of more than a thousand
+// elements leaves the chip idle behind its three passes: 301 segments of 4,096 elements 32.8 -> 6.3 us, of 20,000 203 -> 27, one of
+// 20,000 119 -> 21; 301 of 1,000 4.2 -> 3.9, of 23 3.9 -> 3.6.  At 1,024 segments of up to 1,000 elements the two are alike
+// (4.1, 4.9), and from there on a wavefront each is what fills the chip (2,048 of 23: 4.7, a workgroup each 5.3).
+__global__ __launch_bounds__(kBlock) void jagged_softmax_block_kernel(float* x, const int* __restrict__ lens)
+{
+    __shared__ long long before[kWavesPerBlock];
+    __shared__ float part[2][kWavesPerBlock];
+    const int tid = threadIdx.x;
+    const long long len = lens[blockIdx.x];
+    long long local = 0;
+    for (int i = tid; i < (int)blockIdx.x; i += kBlock) local += lens[i];
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) local += __shfl_xor(local, d, kWave);
+    if ((tid & (kWave - 1)) == 0) before[tid / kWave] = local;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kWavesPerBlock; ++w) x += before[w];
+    if (len <= 0) return;
+    if (len <= kBlock * 4) block_softmax_inplace<4>(x, len, part);
+    else block_softmax_inplace<16>(x, len, part);
 }
 
 // ---- gradient of the jagged softmax: per segment z = <grad, out>, dst += (grad - z) * out
@@ -389,6 +467,11 @@ int gnnhip_jagged_softmax_f32(float* x, const int* lens, int nseg, void* stream)
     GNNHIP_REQUIRE(x && lens, "null tensor in jagged_softmax");
     if (int rc = require_ready()) return rc;
     hipStream_t s = as_stream(stream);
+    if (nseg <= kBlockJaggedMaxSegments) {
+        hipLaunchKernelGGL(jagged_softmax_block_kernel, dim3((unsigned)nseg), dim3(kBlock), 0, s, x, lens);
+        GNNHIP_LAUNCH_CHECK("jagged_softmax_block");
+        return GNNHIP_OK;
+    }
     if (nseg <= kFusedJaggedMaxSegments) {
         const unsigned grid = (unsigned)((nseg + kWavesPerBlock - 1) / kWavesPerBlock);
         hipLaunchKernelGGL(jagged_softmax_fused_kernel, dim3(grid), dim3(kBlock), 0, s, x, lens, nseg);

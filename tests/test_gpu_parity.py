@@ -456,6 +456,46 @@ def test_jagged_softmax(gpu, oracle):
         assert max_rel(got3, oracle.jagged_softmax(x3, lens3)) < PARITY_TOL, nseg
 
 
+@pytest.mark.parametrize("nseg", [1, 7, 1024, 1025])
+def test_jagged_softmax_of_segments_of_any_length(gpu, nseg):
+    """a workgroup per segment (up to 1,024 segments) and a wavefront per segment: lengths around what a lane holds, empty segments,
+    the lowest value everywhere, infinities and NaN (only one that comes first survives the scan for the maximum); against
+    float64, each probability within the 2^-24 roundings of the exponent's argument, exponential, sum and division"""
+    from graphnn_amd import ops
+    rng = np.random.default_rng(nseg)
+    edge = [0, 1, 63, 64, 65, 255, 256, 257, 1023, 1024, 1025, 4095, 4096, 4097, 8193, 20_000]
+    lens = np.array([edge[i % len(edge)] if i < 2 * len(edge) else i % 5 for i in range(nseg)], np.int32)
+    if nseg == 1:
+        lens[0] = 70_001
+    x = (rng.standard_normal(int(lens.sum())) * 4).astype(np.float32)
+    off = np.concatenate([[0], np.cumsum(lens)])
+    special = {}
+    if nseg > 1:
+        for i, kind in ((5, "lowest"), (4, "inf"), (6, "nan later"), (3, "nan first")):
+            seg = x[off[i]:off[i + 1]]
+            special[i] = kind
+            if kind == "lowest": seg[:] = np.finfo(np.float32).min
+            elif kind == "inf": seg[7] = np.inf
+            elif kind == "nan later": seg[9] = np.nan
+            else: seg[0] = np.nan
+    got = _n(ops.jagged_softmax(_t(x, gpu), _t(lens, gpu)))
+    for i in range(nseg):
+        seg, out = x[off[i]:off[i + 1]], got[off[i]:off[i + 1]]
+        if seg.size == 0: continue
+        kind = special.get(i)
+        if kind == "lowest":
+            assert np.allclose(out, 1.0 / seg.size, rtol=4 * 2.0 ** -24, atol=0), i
+        elif kind is not None:
+            # inf - inf and NaN make the sum, and with it every quotient but 0 / NaN, NaN
+            assert np.isnan(out).all(), (i, kind)
+        else:
+            e = np.exp(seg.astype(np.float64) - float(seg.max()))
+            # argument up to 2^5 in magnitude (half an ulp of it, 2^-20), exponential 2 ulp, the sum as a tree over lanes of runs of
+            # len / 64 terms of one sign at most, division
+            bound = 2.0 ** -20 + (2 + max(1, seg.size / 64) + 16 + 1) * 2.0 ** -24
+            assert np.all(np.abs(out - e / e.sum()) <= bound * (e / e.sum()) + 2.0 ** -126), (i, seg.size)
+
+
 def test_jagged_softmax_gradient(gpu, oracle):
     """dst += (grad - <grad, out>) * out per segment (src/nn/jagged_softmax.cpp:8-31), ragged segments"""
     from graphnn_amd import ops
