@@ -309,7 +309,7 @@ int launch_readout_tile(int B, int H, int Q, const int* s_row_ptr, const int* s_
 
 // Readout for any hidden size up to 256 and any number of graphs: TG graphs per workgroup of BLOCK lanes, a quarter of it (one
 // wavefront) or all of it per graph.
-//   1. sum-pool   groups of G lanes (a power of two, 4 G >= C) take the graph's rows in turn, eight in flight each; the sums of a
+//   1. sum-pool   groups of G lanes (a power of two, 4 G >= C) take the graph's rows in turn, FLIGHT in flight each; the sums of a
 //                 wavefront's groups are added by shuffles, those of the graph's wavefronts in order through LDS;
 //   2. hidden     each wavefront of the graph adds up its share of the columns of W_h1, a lane per unit;
 //   3. logits     a wavefront per class, lanes over the hidden units;
@@ -318,15 +318,15 @@ int launch_readout_tile(int B, int H, int Q, const int* s_row_ptr, const int* s_
 // in flight per group of a 256-lane workgroup, 12 with eight of a 512-lane one, 18 with
 // 1,024 lanes, which leave 45 of the workgroups to a second turn), by the chain of its four steps where they are
 // small.  Hidden sizes without another readout took six launches (1,500 graphs of 32 nodes, hidden 100: 35 us).
-template <int TG, int BLOCK>
-__global__ __launch_bounds__(BLOCK) void s2v_readout_rows_kernel(
+template <int TG, int BLOCK, int MINW, int FLIGHT>
+__global__ __launch_bounds__(BLOCK, MINW) void s2v_readout_rows_kernel(
     int B, int C, int H, int Q, const int* __restrict__ s_row_ptr, const int* __restrict__ s_col_idx, const float* __restrict__ s_val,
     const float* __restrict__ h, const float* __restrict__ Wh1, const float* __restrict__ Wh2, float* __restrict__ pool,
     float* __restrict__ hidden, float* __restrict__ logits, float* __restrict__ probs, int* __restrict__ pred)
 {
     using V = ColsLoose;
     constexpr int LG = BLOCK / TG, WG = LG / kWave;      // lanes and wavefronts per graph
-    constexpr int kFlight = 8;
+    constexpr int kFlight = FLIGHT;
     const int units = (C + 3) / 4, C4 = 4 * units;
     const int logG = units <= 1 ? 0 : 32 - __builtin_clz((unsigned)(units - 1));
     const int G = 1 << logG;
@@ -379,7 +379,7 @@ __global__ __launch_bounds__(BLOCK) void s2v_readout_rows_kernel(
         const int share = (C + WG - 1) / WG, c_lo = min(w * share, C), c_hi = min(c_lo + share, C);
         for (int j = lane; j < H; j += kWave) {
             float s = 0.f;
-#pragma unroll 16
+#pragma unroll (2 * FLIGHT)
             for (int c = c_lo; c < c_hi; ++c) s = fmaf(pl[c], Wh1[(size_t)c * H + j], s);
             ph[w * H + j] = s;
         }
@@ -434,7 +434,7 @@ __global__ __launch_bounds__(BLOCK) void s2v_readout_rows_kernel(
     }
 }
 
-template <int TG, int BLOCK>
+template <int TG, int BLOCK, int MINW, int FLIGHT>
 int launch_readout_rows(int B, int C, int H, int Q, const int* s_row_ptr, const int* s_col_idx, const float* s_val, const float* h,
                         const float* Wh1, const float* Wh2, float* pool, float* hidden, float* logits, float* probs, int* pred, hipStream_t s)
 {
@@ -442,7 +442,7 @@ int launch_readout_rows(int B, int C, int H, int Q, const int* s_row_ptr, const 
     const size_t smem = sizeof(float) * TG * ((size_t)(WG + 1) * ((C + 3) / 4 * 4) + (size_t)(WG + 1) * H + Q);
     if (smem > 64 * 1024) return GNNHIP_EUNSUPPORTED;
     const int tiles = (B + TG - 1) / TG, most = kNumCU * (2048 / BLOCK);
-    hipLaunchKernelGGL((s2v_readout_rows_kernel<TG, BLOCK>), dim3((unsigned)(tiles < most ? tiles : most)), dim3(BLOCK), smem, s, B, C, H, Q,
+    hipLaunchKernelGGL((s2v_readout_rows_kernel<TG, BLOCK, MINW, FLIGHT>), dim3((unsigned)(tiles < most ? tiles : most)), dim3(BLOCK), smem, s, B, C, H, Q,
                        s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2, pool, hidden, logits, probs, pred);
     GNNHIP_LAUNCH_CHECK("s2v_readout_rows");
     return GNNHIP_OK;
@@ -492,9 +492,19 @@ int readout_rows_dispatch(int B, int N, int C, int H, int Q, const int* s_row_pt
     // 16.6 against 15.6).  Graphs of hundreds of rows: 512 lanes each.
     const long long mean = (long long)N / B;
     int rc = GNNHIP_EUNSUPPORTED;
-    if (B >= 8 * kNumCU && mean <= 256) rc = launch_readout_rows<4, kBlock>(GNNHIP_RO_ARGS);
-    else if (mean > 256) rc = launch_readout_rows<1, 512>(GNNHIP_RO_ARGS);
-    if (rc == GNNHIP_EUNSUPPORTED) rc = launch_readout_rows<1, kBlock>(GNNHIP_RO_ARGS);
+    // 1,025 to 1,536 small graphs, a workgroup each: three rows in flight per group take 74 registers, which leaves six workgroups per
+    // compute unit where eight take 108 and leave four and a second wave of workgroups (24 nodes each, 1,500 graphs: hidden 48
+    // 11.4 -> 6.6 us, 100 11.6 -> 7.7, 200 14.6 -> 11.3; 250 nodes each: hidden 48 23.1 -> 18.2, 33 20.5 -> 16.5 and, at 1,025 graphs,
+    // 14.6 -> 14.9).  Past 1,536 there are two waves either way, and hidden 200 loses 8 %; below 1,025 there is one, and which is
+    // faster changes with the width (hidden 48, 600 graphs of 60: 6.7 -> 5.9; 64: 6.1 -> 6.3; 200: 11.6 -> 15).
+    int lanes = 1;
+    while (4 * lanes < C) lanes *= 2;
+    const long long turn = mean * lanes;                 // lanes that the rows of a graph take together
+    const bool few = B > 4 * kNumCU && B <= 6 * kNumCU && turn <= 16 * kBlock;
+    if (B >= 8 * kNumCU && mean <= 256) rc = launch_readout_rows<4, kBlock, 5, 8>(GNNHIP_RO_ARGS);
+    else if (mean > 256) rc = launch_readout_rows<1, 512, 4, 8>(GNNHIP_RO_ARGS);
+    if (rc == GNNHIP_EUNSUPPORTED && few) rc = launch_readout_rows<1, kBlock, 6, 3>(GNNHIP_RO_ARGS);
+    if (rc == GNNHIP_EUNSUPPORTED) rc = launch_readout_rows<1, kBlock, 4, 8>(GNNHIP_RO_ARGS);
     return rc;
 #undef GNNHIP_RO_ARGS
 }

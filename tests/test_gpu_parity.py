@@ -2279,6 +2279,35 @@ def test_device_csr_group_at_the_edges_of_its_scans(gpu, n):
     assert bool((val == 1).all())
 
 
+@pytest.mark.parametrize("C,mean", [(5, 24), (48, 24), (100, 24), (100, 63), (100, 70), (128, 64), (200, 24), (200, 63), (256, 70)])
+def test_readout_has_the_same_bits_whatever_the_batch(gpu, C, mean):
+    """a workgroup per graph with three rows in flight and with eight: the first graphs of a batch past the line between them, as
+    batches on either side of it"""
+    from graphnn_amd import ops
+    import torch
+    rng = np.random.default_rng(C + mean)
+    most, H, Q = 1_700, 33, 3
+    sizes = rng.integers(0, 2 * mean + 1, most)
+    rp = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    col = np.concatenate([rp[i] + rng.permutation(n) for i, n in enumerate(sizes)]).astype(np.int32)
+    val = rng.random(col.size).astype(np.float32)
+    gen = torch.Generator(device=gpu).manual_seed(C)
+    h = torch.randn(col.size, C, device=gpu, generator=gen)
+    W1 = torch.randn(C, H, device=gpu, generator=gen)
+    W2 = torch.randn(H, Q, device=gpu, generator=gen)
+    want = ops.s2v_readout(_t(rp, gpu), _t(col, gpu), _t(val, gpu), h, W1, W2, most)
+    pool64 = np.add.reduceat(np.concatenate([h.cpu().numpy().astype(np.float64)[col] * val[:, None], np.zeros((1, C))]), rp[:-1])
+    pool64[sizes == 0] = 0
+    # a sum of n products: n + 1 roundings of terms whose magnitudes add up to no more than the absolute sum
+    mag = np.add.reduceat(np.concatenate([np.abs(h.cpu().numpy().astype(np.float64)[col]) * val[:, None], np.zeros((1, C))]), rp[:-1])
+    assert np.all(np.abs(_n(want[0]) - pool64) <= (sizes[:, None] + 1) * 2.0 ** -24 * mag + 2.0 ** -126)
+    for B in (1, 37, 1_024, 1_025, 1_536, 1_537):
+        e = int(rp[B])
+        got = ops.s2v_readout(_t(rp[:B + 1].copy(), gpu), _t(col[:e].copy(), gpu), _t(val[:e].copy(), gpu), h[:e], W1, W2, B)
+        for g, w in zip(got, want):
+            assert torch.equal(g, w[:B]), B
+
+
 @pytest.mark.parametrize("B", [40, 600])
 @pytest.mark.parametrize("H,Q", [(1, 1), (3, 2), (32, 4), (64, 5), (17, 8), (33, 9), (5, 16), (64, 17), (130, 3)])
 def test_one_launch_readout_of_any_number_of_classes(gpu, B, H, Q):
