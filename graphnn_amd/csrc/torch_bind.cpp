@@ -5,7 +5,7 @@
 // took longer than running them: 172 us per iteration against 96 us of kernels (50 graphs, hidden 64).  Here an
 // argument is checked and unpacked in C++: a float* or int* parameter takes a contiguous float32 / int32 device
 // tensor or None and nothing else, except for the few host pointers of the table below, which take an address as a
-// plain integer; the last parameter, the stream, is the current one.  The functions carry the names of the C entries
+// plain integer or an int32 array; the last parameter, the stream, is the current one.  The functions carry the names of the C entries
 // without `gnnhip_` and raise GnnHipError on a non-zero status.
 //
 // The entries are looked up in the library whose path bind() is given, so the module has no link to it.
@@ -55,15 +55,27 @@ bool tensor_pointer(PyObject* o, at::ScalarType type, const char* type_name, con
     return false;
 }
 
-// an address, or a contiguous object with the buffer protocol (a numpy array), which the caller keeps alive
-bool host_pointer(PyObject* o, void** p)
+// one of the struct module's codes for a 32-bit integer in the host's byte order (no code means bytes)
+bool is_int32(const Py_buffer& view)
+{
+    const char* f = view.format ? view.format : "B";
+    const bool standard = *f == '=' || *f == '<';
+    if (standard || *f == '@') ++f;
+    return view.itemsize == 4 && (*f == 'i' || (standard && *f == 'l')) && !f[1];
+}
+
+// an address, or a contiguous int32 array of one dimension with the buffer protocol (a numpy array), which the caller keeps
+// alive: of `need` elements at least, writable where the entry writes it
+bool host_pointer(PyObject* o, const char* name, long long need, bool written, void** p)
 {
     if (PyObject_CheckBuffer(o)) {
         Py_buffer view;
-        if (PyObject_GetBuffer(o, &view, PyBUF_SIMPLE)) return false;
+        if (PyObject_GetBuffer(o, &view, PyBUF_FORMAT | PyBUF_ND | (written ? PyBUF_WRITABLE : 0))) return false;
+        const bool ok = view.ndim == 1 && is_int32(view) && view.shape[0] >= need;
         *p = view.buf;
         PyBuffer_Release(&view);
-        return true;
+        if (!ok) PyErr_Format(PyExc_ValueError, "%s must be an address or an int32 array of %lld entries or more", name, need);
+        return ok;
     }
     *p = o == Py_None ? nullptr : PyLong_AsVoidPtr(o);
     return !PyErr_Occurred();
@@ -135,7 +147,7 @@ bool current_stream(void** s)
 
 // ---------------------------------------------------------------- one function per entry
 // An entry's parameter names as the C header spells them ("N, C, row_ptr, ..."), for error texts; '@' marks a pointer to
-// host memory.
+// host memory: a const one is read, one element more than the first parameter says; else one element is written.
 std::string nth_name(const char* names, size_t i)
 {
     for (; i > 0 && *names; ++names) i -= *names == ',';
@@ -159,6 +171,7 @@ constexpr size_t host_argument(const char* names)
 template <class Fn, size_t HOST> struct Entry;
 template <size_t HOST, class... P> struct Entry<int (*)(P...), HOST> {
     typedef int (*Fn)(P...);
+    typedef std::tuple_element_t<0, std::tuple<P...>> First;
     static constexpr size_t kArgs = sizeof...(P) - 1;       // the stream comes last and is not passed
 
     template <size_t... I>
@@ -167,8 +180,12 @@ template <size_t HOST, class... P> struct Entry<int (*)(P...), HOST> {
         std::tuple<Arg<P>...> a;
         size_t failed = kArgs;
         auto one = [&](auto& arg, size_t i, const char* name) {
-            if constexpr (std::is_pointer_v<decltype(arg.v)>)
-                if (i == HOST) return host_pointer(args[i], (void**)&arg.v);
+            if constexpr (HOST < kArgs && std::is_same_v<decltype(arg.v), int*>) {
+                constexpr bool kRead = std::is_same_v<std::decay_t<decltype(arg)>, Arg<const int*>>;
+                long long need = 1;
+                if constexpr (kRead && std::is_same_v<First, int>) need += std::get<0>(a).v;
+                if (i == HOST) return host_pointer(args[i], name, need, !kRead, (void**)&arg.v);
+            }
             return arg.take(args[i], name);
         };
         auto take = [&](auto& arg, size_t i) {

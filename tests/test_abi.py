@@ -145,3 +145,35 @@ def test_bindings_make_empty_tensors_of_every_kind():
             empty(cpu, *bad)
     with pytest.raises(RuntimeError):
         empty(cpu, "f", -2)
+
+
+@pytest.mark.parametrize("offsets", [
+    np.array([0, 2, 5], np.int64), np.array([0, 2, 5], np.float32), np.array([0, 2, 5], np.uint32), np.array([0, 2, 5], ">i4"), b"\0" * 12,
+    np.array([0, 2], np.int32), np.array([], np.int32), np.zeros((3, 1), np.int32), np.int32(5), np.int64(1 << 40),
+    np.array([0, 9, 2, 9, 5, 9], np.int32)[::2]])
+def test_bindings_refuse_host_arrays_of_another_kind(offsets):
+    """row offsets on the host are an int32 array with an element more than there are rows: other elements, a shorter array, another
+    number of dimensions, gaps, and a number in numpy's dress are refused before anything reads them"""
+    from graphnn_amd import _lib
+    with pytest.raises((ValueError, BufferError)):
+        _lib.load_bindings().csr_consecutive_rows_host_f32(2, offsets, 0, None, None, None)
+
+
+@pytest.mark.parametrize("offsets", [np.array([0, 2, 5], np.int32), np.array([0, 2, 5, 7], "<i4"), (ctypes.c_int * 3)(0, 2, 5),
+                                     memoryview(np.array([0, 2, 5], np.int32)).toreadonly(), 1 << 40])
+def test_bindings_take_host_arrays_of_int32_and_addresses(offsets):
+    """past the arguments: what refuses the call is the entry behind them (no row pointers to write), or no device to run it on.  The
+    address is never read: the null row pointers are found first"""
+    from graphnn_amd import _lib
+    with pytest.raises((RuntimeError, _lib.GnnHipError)):
+        _lib.load_bindings().csr_consecutive_rows_host_f32(2, offsets, 0, None, None, None)
+
+
+@pytest.mark.parametrize("which", [np.zeros(1, np.float32), np.zeros(1, np.int64), np.zeros(0, np.int32), b"\0\0\0\0",
+                                   memoryview(np.zeros(1, np.int32)).toreadonly(), np.int32(0)])
+def test_bindings_refuse_host_results_of_another_kind(which):
+    """the entry writes which buffer holds the last level: into one writable int32"""
+    from graphnn_amd import _lib
+    args = [0] * 8 + [None] * 19
+    with pytest.raises((ValueError, BufferError)):
+        _lib.load_bindings().s2v_forward_f32(*args, which)
