@@ -407,9 +407,9 @@ at::Tensor make_empty(at::Device device, at::ScalarType type, at::IntArrayRef si
     return at::empty(sizes, at::TensorOptions().device(device).dtype(type));
 }
 
-// empty(where, type, *sizes): an uninitialised tensor of up to three dimensions, type 'f' (float32) or 'i' (int32); several
-// letters: a tuple of tensors, 'f' and 'i' vectors, 'F' float32 matrices, each taking as many of the sizes.  where: a torch.device, or
-// a tensor on whose device they are made.
+// empty(where, types, *sizes): an uninitialised tensor, type 'f' (float32) or 'i' (int32) of one to three dimensions, or 'F' (a float32
+// matrix); several letters: a tuple of tensors, 'f' and 'i' vectors, 'F' matrices, each taking as many of the sizes.  where: a
+// torch.device, or a tensor on whose device they are made.
 PyObject* f_empty(PyObject*, PyObject* const* args, Py_ssize_t n)
 {
     if (n < 3 || !(THPVariable_Check(args[0]) || THPDevice_Check(args[0])) || !PyUnicode_Check(args[1]))
@@ -417,6 +417,14 @@ PyObject* f_empty(PyObject*, PyObject* const* args, Py_ssize_t n)
     Py_ssize_t count;
     const char* types = PyUnicode_AsUTF8AndSize(args[1], &count);
     if (!types) return nullptr;
+    auto dims_of = [&](Py_ssize_t k) { return types[k] == 'F' ? 2 : count == 1 ? n - 2 : 1; };
+    Py_ssize_t needed = 0;
+    for (Py_ssize_t k = 0; k < count; ++k) {
+        if (types[k] != 'f' && types[k] != 'i' && types[k] != 'F') return PyErr_Format(PyExc_TypeError, "empty(): types are 'f', 'i' and 'F'");
+        needed += dims_of(k);
+    }
+    if (count == 0 || needed != n - 2 || (count == 1 && needed > 3))
+        return PyErr_Format(PyExc_TypeError, "empty(): %zd sizes do not make the tensors of '%s'", n - 2, types);
     HANDLE_TH_ERRORS                          // an allocation that fails raises what torch.empty raises
     const at::Device device = THPVariable_Check(args[0]) ? THPVariable_Unpack(args[0]).device() : reinterpret_cast<THPDevice*>(args[0])->device;
     PyObject* all = count > 1 ? PyTuple_New(count) : nullptr;
@@ -424,11 +432,9 @@ PyObject* f_empty(PyObject*, PyObject* const* args, Py_ssize_t n)
     THPObjectPtr owner(all);
     Py_ssize_t next = 2;
     for (Py_ssize_t k = 0; k < count; ++k) {
-        const int dims = count == 1 ? (int)(n - 2) : types[k] == 'F' ? 2 : 1;
+        const int dims = (int)dims_of(k);
         int64_t sizes[3];
-        if (dims > 3) return PyErr_Format(PyExc_TypeError, "empty(): too many sizes");
         for (int d = 0; d < dims; ++d) {
-            if (next >= n) return PyErr_Format(PyExc_TypeError, "empty(): too few sizes");
             sizes[d] = PyLong_AsLongLong(args[next++]);
             if (sizes[d] == -1 && PyErr_Occurred()) return nullptr;
         }

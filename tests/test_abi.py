@@ -147,6 +147,16 @@ def test_bindings_make_empty_tensors_of_every_kind():
         empty(cpu, "f", -2)
 
 
+@pytest.mark.parametrize("args", [("", 3), ("ff", 3, 4, 5), ("iF", 3, 4, 5, 6), ("F", 3), ("F", 3, 4, 5), ("x", 3), ("fx", 3, 4), ("d", 3), ("I", 3),
+                                  ("\u00e9", 3), ("f\0", 3, 4), ("f",), ("i", 1, 2, 3, 4)])
+def test_bindings_make_no_tensors_of_a_list_that_does_not_add_up(args):
+    """no letters, letters that name no type, sizes left over or missing"""
+    import torch
+    from graphnn_amd import _lib
+    with pytest.raises(TypeError):
+        _lib.load_bindings().empty(torch.device("cpu"), *args)
+
+
 @pytest.mark.parametrize("offsets", [
     np.array([0, 2, 5], np.int64), np.array([0, 2, 5], np.float32), np.array([0, 2, 5], np.uint32), np.array([0, 2, 5], ">i4"), b"\0" * 12,
     np.array([0, 2], np.int32), np.array([], np.int32), np.zeros((3, 1), np.int32), np.int32(5), np.int64(1 << 40),

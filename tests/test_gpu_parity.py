@@ -2555,6 +2555,9 @@ def test_bindings_make_tensors_as_torch_does(gpu):
     i, f = ops._empty(where, "iF", 7, 2, 3)
     check(i, torch.empty(7, dtype=torch.int32, device=gpu))
     check(f, torch.empty(2, 3, device=gpu))
+    for sizes in ((-2,), (3, -1)):
+        with pytest.raises(RuntimeError):
+            ops._empty(where, "f", *sizes)
     torch.use_deterministic_algorithms(True)
     try:
         assert bool(torch.isnan(ops._empty(where, "f", 1000)).all())
