@@ -200,7 +200,12 @@ int static_offsets_ptr(int** out);
 // ---- high-degree rows (hub.hip)
 constexpr int kHubThreshold = 64;      // rows with more entries are summed by the pre-pass
 constexpr int kHubChunk = 2048;        // entries per partial sum of the pre-pass
-constexpr int kLevelTileMaxRows = 24576; // up to here a level at hidden 16/32/64 runs a workgroup per tile (level_tile.hip)
+constexpr int kLevelTileMaxRows = 24576; // up to here a level at hidden 16/32/64 runs a workgroup per tile (level_tile.hip),
+constexpr int kLevelTileDense = 20;      // at hidden 16 with more entries per row than this up to half as many rows
+inline bool level_by_tile(int N, int C, long long nnz)
+{
+    return N <= (C == 16 && nnz > kLevelTileDense * (long long)N ? kLevelTileMaxRows / 2 : kLevelTileMaxRows);
+}
 constexpr int kHubMinRows = 32768;     // smaller matrices skip the pre-pass: its launches would cost more than a long row
 struct HubPlan {
     const int* row_chunk = nullptr;    // [m], defined for rows longer than the pass's threshold only: first chunk, -1: not summed

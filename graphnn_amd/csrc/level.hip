@@ -545,7 +545,7 @@ int level_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* c
             default: return launch_level<64, true>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, none, s);
             }
         }
-        if (N <= kLevelTileMaxRows) return level_tile_dispatch(N, C, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, relu_in, s);
+        if (level_by_tile(N, C, nnz)) return level_tile_dispatch(N, C, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, relu_in, s);
         HubPlan hubs{};
         if (int rc = hub_prepass(N, C, nnz, row_ptr, col_idx, val, h_in, C, s, &hubs, same_graph, relu_in, kHubThreshold, kHubChunk, -1,
                                  plan ? &plan->row_hub : nullptr))
@@ -605,7 +605,7 @@ int level_backward_dispatch(int N, int C, long long nnz, const int* row_ptr, con
     if (!(aligned16(dz) && aligned16(W) && aligned16(u) && aligned16(g_prev) && (!gate || aligned16(gate)) && (!acc || aligned16(acc))))
         return GNNHIP_EUNSUPPORTED;
     if (N >= kHubMinRows && nnz >= two_step_degree() * (long long)N) return GNNHIP_EUNSUPPORTED;     // dense and skewed: balanced SpMM
-    if (N <= kLevelTileMaxRows) return level_tile_backward_dispatch(N, C, row_ptr, col_idx, val, dz, W, u, g_prev, gate, acc, s);
+    if (level_by_tile(N, C, nnz)) return level_tile_backward_dispatch(N, C, row_ptr, col_idx, val, dz, W, u, g_prev, gate, acc, s);
     HubPlan hubs{};
     if (int rc = hub_prepass(N, C, nnz, row_ptr, col_idx, val, dz, C, s, &hubs, false, false)) return rc;
     return level_stream_backward_dispatch(N, C, row_ptr, col_idx, val, dz, W, u, g_prev, gate, acc, hubs, s);

@@ -7,11 +7,17 @@
 // has C/16 wavefronts, each of which gathers 16/(C/16) of its rows, one per lane group and up to eight entries of it at
 // once, and contracts one 16-column block: a quarter of the gathers and of the matrix instructions in a row at
 // C = 64, and W straight into registers (16 values per lane) instead of through LDS.  msg, the gate and the gradient sum do not
-// hang on that chain and are asked for ahead of it.  Hidden 64, 2.2 entries per row, streaming kernel -> here: 1,625 rows 5.6 ->
-// 4.1 us forward and 6.5 -> 4.4 backward (4 is what a launch costs there), 7,450 rows 6.2 -> 4.2 and 7.1 -> 5.5, 24,000 rows
-// 8.8 -> 6.9 and 10.9 -> 10.5.  At 32,000 rows the backward pass is 12.2 -> 13.6: every workgroup reads W anew, and the
-// result leaves in 64-byte pieces of a row; so kLevelTileMaxRows.  The sums of a row and the products of an element have the order of the
-// streaming kernel, so the bits are the same.
+// hang on that chain and are asked for ahead of it.  Streaming kernel -> here, us forward and backward:
+//     hidden 64, 2.2 entries per row  1,600 rows 5.8 -> 2.9, 6.6 -> 3.8;  7,450 6.1 -> 3.8, 7.3 -> 5.3;  24,576 8.8 -> 7.2, 11.6 -> 11.1
+//                30                   1,600      18.6 -> 6.4, 19.6 -> 7.2;  24,576 23.0 -> 16.3, 27.5 -> 21.2
+//     hidden 32, 2.2                  1,600      3.6 -> 2.5, 3.9 -> 2.8;  24,576 5.1 -> 4.1, 6.8 -> 6.0;  30: 13.3 -> 9.6, 15.2 -> 12.3
+//     hidden 16, 2.2                  1,600      3.3 -> 2.6, 3.5 -> 2.8;  24,576 3.8 -> 3.2, 4.4 -> 4.0;  8: 4.9 -> 4.3, 5.5 -> 5.1
+// At 32,000 rows the backward pass at hidden 64 is 12.2 -> 13.6: every workgroup reads W anew, and the result leaves in 64-byte
+// pieces of a row; so kLevelTileMaxRows.  At hidden 16 a tile is one wavefront, with nobody to share its gathers: what is left of the
+// gain is that they start at once, which long rows outweigh.  With up to 20 entries per row it is as fast as the streaming kernel or faster
+// at every number of rows; with 24 to 100 it is, past 12,288 rows, anything from 8 % faster to 13 % slower (30 entries: 14,000 rows
+// 7.7 -> 7.9 and 8.1 -> 8.6, 18,000 rows 9.1 -> 8.6 and 9.5 -> 9.2; 100: 20,000 rows 23.9 -> 27.4 and 25.5 -> 29.1), up to there nowhere slower;
+// so level_by_tile.  The sums of a row and the products of an element have the order of the streaming kernel, so the bits are the same.
 #include "level_gather.h"
 
 namespace gnnhip {
@@ -205,7 +211,7 @@ int launch_level_tile_backward(int N, const int* row_ptr, const int* col_idx, co
 
 }  // namespace
 
-// N <= kLevelTileMaxRows; pointers as level_stream_dispatch takes them
+// N <= kLevelTileMaxRows (level_by_tile); pointers as level_stream_dispatch takes them
 int level_tile_dispatch(int N, int C, const int* row_ptr, const int* col_idx, const float* val, const float* h_in, const float* W,
                         const float* msg, const float* bias, float* h_out, bool relu_in, hipStream_t s)
 {

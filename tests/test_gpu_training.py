@@ -468,6 +468,32 @@ def test_level_of_a_small_batch_has_the_bits_of_a_large_one(gpu, C, N):
         assert a is None or torch.equal(acc, acc_more[:N])
 
 
+@pytest.mark.parametrize("N", [12_288, 12_289, 24_576])
+def test_level_of_long_rows_at_hidden_16_has_the_same_bits_either_way(gpu, N):
+    """from 12,289 rows on the entry count decides whether a level at hidden 16 runs a workgroup per tile or the streaming kernel: a
+    count of zero takes the former; rows of 0 to 60 entries, 24 on average, and a few of 200"""
+    import torch
+    from graphnn_amd import ops
+    C = 16
+    gen = torch.Generator(device=gpu).manual_seed(N)
+    normal = lambda *shape: torch.randn(*shape, generator=gen, device=gpu)
+    lens = torch.tensor([0, 60, 5, 24, 48, 49, 17, 16, 3, 15, 23, 31], device=gpu).repeat(N // 12 + 1)[:N]
+    lens[N // 3:N // 3 + 5] = 200
+    rp = torch.zeros(N + 1, dtype=torch.int32, device=gpu)
+    rp[1:] = torch.cumsum(lens, 0)
+    nnz = int(rp[-1])
+    assert 20 * N < nnz < 25 * N
+    ci, v = torch.randint(0, N, (nnz,), generator=gen, device=gpu).int(), normal(nnz)
+    h, W, msg, gate, acc0 = normal(N, C), normal(C, C) * 0.2, normal(N, C), normal(N, C), normal(N, C)
+    assert torch.equal(ops.s2v_level(rp, ci, v, h, W, msg), ops.s2v_level(rp, ci, v, h, W, msg, nnz_hint=0))
+    got = []
+    for count in (nnz, 0):
+        u, out, acc = torch.empty_like(h), torch.empty_like(h), acc0.clone()
+        ops._bound().s2v_level_backward_f32(N, C, count, rp, ci, v, h, W, u, out, gate, acc)
+        got.append((u, out, acc))
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
 @pytest.mark.parametrize("C", [5, 36, 100, 127])
 def test_level_of_any_hidden_size_has_the_same_bits_whatever_the_tile(gpu, C):
     """levels of hidden sizes without a kernel of their own take 16, 32 or 64 rows per workgroup by the number of rows: the same rows
