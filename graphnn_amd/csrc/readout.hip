@@ -318,6 +318,10 @@ int launch_readout_tile(int B, int H, int Q, const int* s_row_ptr, const int* s_
 // in flight per group of a 256-lane workgroup, 12 with eight of a 512-lane one, 18 with
 // 1,024 lanes, which leave 45 of the workgroups to a second turn), by the chain of its four steps where they are
 // small.  Hidden sizes without another readout took six launches (1,500 graphs of 32 nodes, hidden 100: 35 us).
+//
+// MINW: wavefronts per SIMD that the registers have to leave room for, 0: none asked for.  Only the variant with three rows in flight asks:
+// where it does not change their number, asking only makes the compiler wait for each load by itself (a wavefront per graph, five
+// asked for, which the kernel has anyway: 2,048 graphs of 24 nodes, hidden 160 16.1 -> 30.1 us, 256 21.6 -> 47.6).
 template <int TG, int BLOCK, int MINW, int FLIGHT>
 __global__ __launch_bounds__(BLOCK, MINW) void s2v_readout_rows_kernel(
     int B, int C, int H, int Q, const int* __restrict__ s_row_ptr, const int* __restrict__ s_col_idx, const float* __restrict__ s_val,
@@ -501,10 +505,10 @@ int readout_rows_dispatch(int B, int N, int C, int H, int Q, const int* s_row_pt
     while (4 * lanes < C) lanes *= 2;
     const long long turn = mean * lanes;                 // lanes that the rows of a graph take together
     const bool few = B > 4 * kNumCU && B <= 6 * kNumCU && turn <= 16 * kBlock;
-    if (B >= 8 * kNumCU && mean <= 256) rc = launch_readout_rows<4, kBlock, 5, 8>(GNNHIP_RO_ARGS);
-    else if (mean > 256) rc = launch_readout_rows<1, 512, 4, 8>(GNNHIP_RO_ARGS);
+    if (B >= 8 * kNumCU && mean <= 256) rc = launch_readout_rows<4, kBlock, 0, 8>(GNNHIP_RO_ARGS);
+    else if (mean > 256) rc = launch_readout_rows<1, 512, 0, 8>(GNNHIP_RO_ARGS);
     if (rc == GNNHIP_EUNSUPPORTED && few) rc = launch_readout_rows<1, kBlock, 6, 3>(GNNHIP_RO_ARGS);
-    if (rc == GNNHIP_EUNSUPPORTED) rc = launch_readout_rows<1, kBlock, 4, 8>(GNNHIP_RO_ARGS);
+    if (rc == GNNHIP_EUNSUPPORTED) rc = launch_readout_rows<1, kBlock, 0, 8>(GNNHIP_RO_ARGS);
     return rc;
 #undef GNNHIP_RO_ARGS
 }
