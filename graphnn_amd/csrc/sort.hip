@@ -338,8 +338,8 @@ __global__ __launch_bounds__(kBlock) void expand_rows_kernel(int m, const int* _
 //   write      slot after slot, coalesced: payload (and value) of the pair the slot names
 // Keys are read four to a load (where they are not strided), all of a thread's sixteen before the first is used.  What bounds it is
 // the chain of these steps: 16,380 pairs of 7,450 rows take 3 us to read and count, 0.9 to scan, 0.7 to place, 0.7 to order and
-// 1.5 to write, behind the 4 of any launch with much LDS (both ways at once 17.3 -> 11.5 us; 16 workgroups of 1,024 lanes with a
-// key per load before).  More, smaller workgroups shorten every step but the reading (6,175 pairs 11.5 -> 7.8, 60,000 41 -> 23 us);
+// 1.5 to write, behind the 4 of any launch with much LDS (both ways at once 16.5 -> 9.5 us; 16 workgroups of 1,024 lanes with a
+// key per load before).  More, smaller workgroups shorten every step but the reading (6,175 pairs 11.4 -> 7.6, 60,000 49 -> 24 us);
 // rows of 9 to 64 entries cost 80 to 700 us per 65,000 pairs when each walked a bitmap.  The order of the entries is a
 // pure function of the input, as on the radix route.  Sizes: 4 bytes per row of a run, 2 per pair, one
 // bitmap of n bits (as many as fit, up to one per wavefront) in 160 KB of LDS; at most 65,536 pairs.
@@ -403,7 +403,8 @@ struct SmallJob {
     int key_stride, payload_stride;
 };
 
-template <int BLOCK>
+// DENSE: keys follow each other in memory
+template <int BLOCK, bool DENSE>
 __global__ __launch_bounds__(BLOCK) void csr_group_small_kernel(int rows, int n, SmallLayout lay, SmallJob job0, SmallJob job1, int average)
 {
     constexpr int kWaves = BLOCK / kWave;
@@ -431,56 +432,79 @@ __global__ __launch_bounds__(BLOCK) void csr_group_small_kernel(int rows, int n,
     if (tid < kSmallMisc) misc[tid] = 0;
     __syncthreads();
 
-    // lengths.  A lane takes four consecutive pairs at a time and counts equal neighbours among them together.  The keys of the
-    // first batch stay in registers for `place`.
+    // lengths.  DENSE: a lane takes four consecutive pairs at a time and counts equal neighbours among them together.  Else the loads
+    // of four pairs a lane would each spread over four times as many lines (60,000 pairs of two ints: 58 us, 39 so): lanes hold consecutive
+    // pairs, and a run of equal keys is counted by its first lane alone.  The keys of the first batch stay in registers for `place`.
     bool disorder = false;
     int below = 0;
     int first_keys[kSmallBatch];
-    const bool words = key_stride == 1 && (reinterpret_cast<size_t>(key) & 15) == 0;
-    auto pair_of = [&](int base, int u) { return base + ((u / 4) * BLOCK + tid) * 4 + (u & 3); };
+    const bool words = DENSE && (reinterpret_cast<size_t>(key) & 15) == 0;
+    auto pair_of = [&](int base, int u) { return base + (DENSE ? ((u / 4) * BLOCK + tid) * 4 + (u & 3) : u * BLOCK + tid); };
     auto load_keys = [&](int base, int (&k)[kSmallBatch]) {       // clamped; -1 past the last pair
+        if constexpr (DENSE) {
 #pragma unroll
-        for (int v = 0; v < kSmallBatch / 4; ++v) {
-            const int e = pair_of(base, 4 * v);
-            int4 x = make_int4(-1, -1, -1, -1);
-            if (words && e + 3 < n) {
-                x = *reinterpret_cast<const int4*>(key + e);
-            } else {
-                if (e + 0 < n) x.x = key[(long long)(e + 0) * key_stride];
-                if (e + 1 < n) x.y = key[(long long)(e + 1) * key_stride];
-                if (e + 2 < n) x.z = key[(long long)(e + 2) * key_stride];
-                if (e + 3 < n) x.w = key[(long long)(e + 3) * key_stride];
+            for (int v = 0; v < kSmallBatch / 4; ++v) {
+                const int e = pair_of(base, 4 * v);
+                int4 x = make_int4(-1, -1, -1, -1);
+                if (words && e + 3 < n) {
+                    x = *reinterpret_cast<const int4*>(key + e);
+                } else {
+                    if (e + 0 < n) x.x = key[e + 0];
+                    if (e + 1 < n) x.y = key[e + 1];
+                    if (e + 2 < n) x.z = key[e + 2];
+                    if (e + 3 < n) x.w = key[e + 3];
+                }
+                k[4 * v] = x.x; k[4 * v + 1] = x.y; k[4 * v + 2] = x.z; k[4 * v + 3] = x.w;
             }
-            k[4 * v] = x.x; k[4 * v + 1] = x.y; k[4 * v + 2] = x.z; k[4 * v + 3] = x.w;
+        } else {
+#pragma unroll
+            for (int u = 0; u < kSmallBatch; ++u) {
+                const int e = pair_of(base, u);
+                k[u] = e < n ? key[(long long)e * key_stride] : -1;
+            }
         }
 #pragma unroll
         for (int u = 0; u < kSmallBatch; ++u) k[u] = pair_of(base, u) < n ? min(max(k[u], 0), top) : -1;
     };
     for (int base = 0; base < n; base += BLOCK * kSmallBatch) {       // every lane walks every batch: the shuffles need them
-        int k[kSmallBatch], before[kSmallBatch / 4];
+        constexpr int kEach = DENSE ? 4 : 1;                      // consecutive pairs of a lane
+        int k[kSmallBatch], before[kSmallBatch / kEach];
 #pragma unroll
-        for (int v = 0; v < kSmallBatch / 4; ++v) {
-            const int e = pair_of(base, 4 * v);
+        for (int v = 0; v < kSmallBatch / kEach; ++v) {
+            const int e = pair_of(base, kEach * v);
             before[v] = lane == 0 && e > 0 && e < n ? key[(long long)(e - 1) * key_stride] : -1;
         }
         load_keys(base, k);
 #pragma unroll
-        for (int v = 0; v < kSmallBatch / 4; ++v) {
-            const int left = __shfl_up(k[4 * v + 3], 1, kWave);
+        for (int v = 0; v < kSmallBatch / kEach; ++v) {
+            const int left = __shfl_up(k[kEach * v + kEach - 1], 1, kWave);
             int prev = lane == 0 ? (before[v] < 0 ? before[v] : min(before[v], top)) : left;
-            int run = 1;
+            if constexpr (DENSE) {
+                int run = 1;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int kk = k[4 * v + j];
-                if (base == 0) first_keys[4 * v + j] = kk;
+                for (int j = 0; j < 4; ++j) {
+                    const int kk = k[4 * v + j];
+                    if (base == 0) first_keys[4 * v + j] = kk;
+                    disorder |= kk >= 0 && prev > kk;
+                    below += kk >= 0 && kk < lo;
+                    prev = kk;
+                    if (j < 3 && k[4 * v + (j < 3 ? j + 1 : 3)] == kk) {
+                        ++run;
+                    } else {
+                        if (kk >= 0 && (unsigned)(kk - lo) < (unsigned)mine) atomicAdd(&cnt[kk - lo], run);
+                        run = 1;
+                    }
+                }
+            } else {
+                const int kk = k[v];
+                if (base == 0) first_keys[v] = kk;
                 disorder |= kk >= 0 && prev > kk;
                 below += kk >= 0 && kk < lo;
-                prev = kk;
-                if (j < 3 && k[4 * v + (j < 3 ? j + 1 : 3)] == kk) {
-                    ++run;
-                } else {
-                    if (kk >= 0 && (unsigned)(kk - lo) < (unsigned)mine) atomicAdd(&cnt[kk - lo], run);
-                    run = 1;
+                const bool head = lane == 0 || left != kk;
+                const unsigned long long heads = __ballot(head);
+                if (head && kk >= 0 && (unsigned)(kk - lo) < (unsigned)mine) {
+                    const unsigned long long later = lane == kWave - 1 ? 0ull : heads >> (lane + 1);
+                    atomicAdd(&cnt[kk - lo], later ? __ffsll((long long)later) : kWave - lane);
                 }
             }
         }
@@ -745,16 +769,21 @@ bool csr_group_small(int rows, long long n, const int* key, int key_stride, cons
     const SmallJob job1 = {payload, key, nullptr, t_row_ptr, t_col_idx, t_val, payload_stride, key_stride};
     const dim3 grid(lay.groups * (t_row_ptr ? 2 : 1));
     const size_t lds = sizeof(int) * (size_t)(lay.bitmaps + lay.words * lay.nbitmaps);
-    auto launch = [&](auto block) {
+    auto launch = [&](auto block, auto dense) {
         constexpr int kSize = decltype(block)::value;
+        constexpr bool kDense = decltype(dense)::value;
         static LdsLimit limit;
-        if (limit.raise(reinterpret_cast<const void*>(csr_group_small_kernel<kSize>), sizeof(int) * kSmallLdsInts) != hipSuccess) return false;
-        hipLaunchKernelGGL(csr_group_small_kernel<kSize>, grid, dim3(kSize), lds, s, rows, (int)n, lay, job0, job1, average);
+        if (limit.raise(reinterpret_cast<const void*>(csr_group_small_kernel<kSize, kDense>), sizeof(int) * kSmallLdsInts) != hipSuccess) return false;
+        hipLaunchKernelGGL((csr_group_small_kernel<kSize, kDense>), grid, dim3(kSize), lds, s, rows, (int)n, lay, job0, job1, average);
         return true;
     };
-    if (lay.block == 256) return launch(std::integral_constant<int, 256>());
-    if (lay.block == 512) return launch(std::integral_constant<int, 512>());
-    return launch(std::integral_constant<int, 1024>());
+    auto by_stride = [&](auto block) {
+        const bool dense = key_stride == 1 && (!t_row_ptr || payload_stride == 1);
+        return dense ? launch(block, std::true_type()) : launch(block, std::false_type());
+    };
+    if (lay.block == 256) return by_stride(std::integral_constant<int, 256>());
+    if (lay.block == 512) return by_stride(std::integral_constant<int, 512>());
+    return by_stride(std::integral_constant<int, 1024>());
 }
 
 inline int last_launch_status(const char* what)

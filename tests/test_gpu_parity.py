@@ -2261,6 +2261,38 @@ def test_device_csr_group_at_the_edges_of_its_workgroups(gpu, n, rows):
                 assert np.array_equal(_n(g), w), (order, shift)
 
 
+@pytest.mark.parametrize("n", [3, 63, 64, 65, 511, 513, 8191, 8193, 16_385, 65_535])
+@pytest.mark.parametrize("rows", [1, 65, 4_097, 50_000])
+def test_device_csr_group_of_strided_keys(gpu, n, rows):
+    """keys two and three ints apart, where a lane takes one pair at a time: runs of equal keys that end with a wavefront and inside
+    it, keys out of range, ascending ones; alone, and with the other member of the pair as the key of a second grouping, of the same
+    stride and of its own (one of the two strided); the bits of the stable sort"""
+    from graphnn_amd import ops
+    rng = np.random.default_rng(n + rows)
+    key, other = rng.integers(0, rows, n), rng.integers(0, rows, n)
+    key[n // 3:n // 3 + 300] = rng.integers(0, rows)
+    for order in ("any", "ascending"):
+        if order == "ascending":
+            key = np.sort(key)
+        raw = key.copy()
+        raw[key == 0] -= rng.integers(0, 3, int((key == 0).sum()))
+        raw[key == rows - 1] += rng.integers(0, 3, int((key == rows - 1).sum()))
+        want, turned = _stable_group(rows, key, raw), _stable_group(rows, key, other)
+        for stride in (2, 3):
+            held = np.full((n, stride), -7, np.int32)
+            held[:, stride - 1] = raw
+            held_d = _t(held.reshape(-1), gpu)[stride - 1:]
+            for g, w in zip(ops.csr_group(rows, held_d, held_d, False, stride, stride, n), want):
+                assert np.array_equal(_n(g), w), (order, stride)
+            back = _stable_group(rows, other, raw)
+            for x_stride in (1, stride):
+                x = np.full((n, x_stride), -7, np.int32)
+                x[:, 0] = other
+                got = ops.csr_group_both(rows, _t(x.reshape(-1), gpu), held_d, x_stride, stride, n)
+                for g, w in zip(got[0] + got[1], turned + back):
+                    assert np.array_equal(_n(g), w), (order, stride, x_stride)
+
+
 @pytest.mark.parametrize("n", [65_536, 67_584, 67_585, 8_192 * 2_048, 8_192 * 2_048 + 1])
 def test_device_csr_group_at_the_edges_of_its_scans(gpu, n):
     """the sort's counters in whole segments of 1,024 and in a part of one more, and either side of the 2,048 segments that a
