@@ -340,7 +340,9 @@ __global__ __launch_bounds__(kBlock) void expand_rows_kernel(int m, const int* _
 // the chain of these steps: 16,380 pairs of 7,450 rows take 3 us to read and count, 0.9 to scan, 0.7 to place, 0.7 to order and
 // 1.5 to write, behind the 4 of any launch with much LDS (both ways at once 16.5 -> 9.5 us; 16 workgroups of 1,024 lanes with a
 // key per load before).  More, smaller workgroups shorten every step but the reading (6,175 pairs 11.4 -> 7.6, 60,000 49 -> 24 us);
-// rows of 9 to 64 entries cost 80 to 700 us per 65,000 pairs when each walked a bitmap.  The order of the entries is a
+// rows of 9 to 64 entries cost 80 to 700 us per 65,000 pairs when each walked a bitmap.  By rank such a row takes a third of a
+// microsecond of a SIMD's instructions, so few rows are spread over many workgroups: runs of 8 rows, and 8 wavefronts at least (2,000 pairs of 66 rows:
+// runs of 64 rows and 4 wavefronts 27 us, of 16 rows 13, of 8 rows and 8 wavefronts 7.9).  The order of the entries is a
 // pure function of the input, as on the radix route.  Sizes: 4 bytes per row of a run, 2 per pair, one
 // bitmap of n bits (as many as fit, up to one per wavefront) in 160 KB of LDS; at most 65,536 pairs.
 constexpr int kSmallPairs = 1 << 16;
@@ -349,11 +351,11 @@ constexpr int kSmallBatch = 16;
 constexpr int kSmallLdsInts = 160 * 1024 / 4;
 constexpr int kSmallMisc = 48;
 constexpr int kSmallGroups = 64;           // workgroups at most, per grouping
-constexpr int kSmallRunRows = 64;          // rows per workgroup at least
+constexpr int kSmallRunRows = 8;           // rows per workgroup at least
 
 struct SmallLayout {
     int block;                            // lanes per workgroup
-    int groups, run;                      // workgroups, rows per workgroup (a multiple of 64)
+    int groups, run;                      // workgroups, rows per workgroup (a multiple of kSmallRunRows)
     int slots, longs, misc, bitmaps;      // offsets in ints (the counters start at 0)
     int words, nbitmaps;                  // words per bitmap, number of bitmaps
 };
@@ -364,7 +366,7 @@ inline bool small_layout(long long rows, long long n, SmallLayout* out)
     SmallLayout l;
     long long groups = (rows + kSmallRunRows - 1) / kSmallRunRows;
     if (groups > kSmallGroups) groups = kSmallGroups;
-    const long long run = ((rows + groups - 1) / groups + kWave - 1) / kWave * kWave;
+    const long long run = ((rows + groups - 1) / groups + kSmallRunRows - 1) / kSmallRunRows * kSmallRunRows;
     if (run > kSmallLdsInts) return false;
     l.run = (int)run;
     l.groups = (int)((rows + run - 1) / run);
@@ -377,7 +379,7 @@ inline bool small_layout(long long rows, long long n, SmallLayout* out)
     if (room < l.words) return false;
     // the keys in one batch of loads where that can be, four rows of the run per lane at most
     const long long per_lane = std::max((n + kSmallBatch - 1) / kSmallBatch, run / 4);
-    l.block = per_lane <= 256 ? 256 : per_lane <= 512 ? 512 : 1024;
+    l.block = per_lane <= 512 ? 512 : 1024;
     const int waves = l.block / kWave;
     l.nbitmaps = room / l.words < waves ? room / l.words : waves;
     *out = l;
@@ -604,10 +606,13 @@ __global__ __launch_bounds__(BLOCK) void csr_group_small_kernel(int rows, int n,
             const int r = longs[q];
             const int a = r ? cnt[r - 1] : 0, len = cnt[r] - a;
             if (len > kWave) continue;
-            const int v = lane < len ? (int)slots[a + lane] : 0;
+            const int v = lane < len ? (int)slots[a + lane] : kSmallPairs;
             const int ulen = __builtin_amdgcn_readfirstlane(len);
             int rank = 0;
-            for (int j = 0; j < ulen; ++j) rank += __builtin_amdgcn_readlane(v, j) < v;
+            for (int j0 = 0; j0 < ulen; j0 += 8) {        // (a lane past the row holds what is larger than any entry)
+#pragma unroll
+                for (int j = 0; j < 8; ++j) rank += __builtin_amdgcn_readlane(v, j0 + j) < v;
+            }
             if (lane < len) slots[a + rank] = (unsigned short)v;
         }
         if (nlong > 0 && wave < lay.nbitmaps) {
@@ -781,7 +786,6 @@ bool csr_group_small(int rows, long long n, const int* key, int key_stride, cons
         const bool dense = key_stride == 1 && (!t_row_ptr || payload_stride == 1);
         return dense ? launch(block, std::true_type()) : launch(block, std::false_type());
     };
-    if (lay.block == 256) return by_stride(std::integral_constant<int, 256>());
     if (lay.block == 512) return by_stride(std::integral_constant<int, 512>());
     return by_stride(std::integral_constant<int, 1024>());
 }

@@ -2182,7 +2182,7 @@ def _stable_group(rows, key, pay, average=False):
 @pytest.mark.parametrize("case", ["lengths_around_eight", "hub_in_a_window", "one_row_of_all", "largest", "past_the_largest", "many_rows", "ascending",
                                   "ascending_but_one", "long_rows_only", "two_pairs"])
 def test_device_csr_group_of_a_small_batch_in_one_launch(gpu, case):
-    """up to 65,536 pairs are grouped in one launch of up to 16 workgroups, each with a run of the rows (4 bytes per row of
+    """up to 65,536 pairs are grouped in one launch of up to 64 workgroups, each with a run of the rows (4 bytes per row of
     the run and 2.35 per pair have to fit 160 KB of LDS): rows of up to 8 entries ordered by a thread, longer rows by a
     wavefront with a bitmap (one bitmap only in the largest cases), keys that already ascend copied through;
     bit-identical to the stable sort"""
@@ -2232,7 +2232,7 @@ def test_device_csr_group_of_a_small_batch_in_one_launch(gpu, case):
 @pytest.mark.parametrize("n", [3, 4, 255, 4095, 4096, 4097, 8191, 8193, 16_383, 16_385, 33_001, 65_535])
 @pytest.mark.parametrize("rows", [1, 63, 65, 4_097, 50_000, 300_000])
 def test_device_csr_group_at_the_edges_of_its_workgroups(gpu, n, rows):
-    """the one-launch grouping where its workgroups (256, 512 or 1,024 lanes, 64 rows or more each) and its batches of keys end:
+    """the one-launch grouping where its workgroups (512 or 1,024 lanes, 8 rows or more each) and its batches of keys end:
     keys that start at any int (read four at a time only where they are aligned), keys out of range (clamped to the first and
     the last row), runs of equal keys across lanes and wavefronts, rows of 8, 9, 64 and 65 entries; the bits of the stable sort"""
     from graphnn_amd import ops
@@ -2291,6 +2291,21 @@ def test_device_csr_group_of_strided_keys(gpu, n, rows):
                 got = ops.csr_group_both(rows, _t(x.reshape(-1), gpu), held_d, x_stride, stride, n)
                 for g, w in zip(got[0] + got[1], turned + back):
                     assert np.array_equal(_n(g), w), (order, stride, x_stride)
+
+
+@pytest.mark.parametrize("rows", [1, 7, 8, 9, 16, 17, 511, 512, 513])
+@pytest.mark.parametrize("per", [3, 9, 30, 64, 100])
+def test_device_csr_group_of_few_rows(gpu, rows, per):
+    """runs of eight rows and more per workgroup: one run and several, the last one short, rows that a thread, a wavefront by rank and
+    a bitmap put in order, in one run; the bits of the stable sort"""
+    from graphnn_amd import ops
+    rng = np.random.default_rng(rows + per)
+    lens = rng.integers(0, 2 * per + 1, rows)
+    lens[rows // 2] = 64
+    key = rng.permutation(np.repeat(np.arange(rows), lens)).astype(np.int32)
+    pay = rng.integers(0, 1 << 30, key.size).astype(np.int32)
+    for g, w in zip(ops.csr_group(rows, _t(key, gpu), _t(pay, gpu)), _stable_group(rows, key, pay)):
+        assert np.array_equal(_n(g), w)
 
 
 @pytest.mark.parametrize("n", [65_536, 67_584, 67_585, 8_192 * 2_048, 8_192 * 2_048 + 1])
