@@ -525,13 +525,22 @@ __global__ __launch_bounds__(WAVES * kWave, (min_waves<C, KSX, WAVES, KEEP, PACK
                     const float4 wv = *reinterpret_cast<const float4*>(wrow);
                     v = make_float4(0.f + wv.x, 0.f + wv.y, 0.f + wv.z, 0.f + wv.w);
                 } else {
-                    // (srt is KSX or KSX - 2: two straight runs instead of a branch per step)
+                    // (srt is KSX or KSX - 2: two straight runs instead of a branch per step.  Rows of 32 and 64 floats start on the same
+                    // banks, and of such rows a load of two pairs takes longer than two loads: 256 graphs, 64 features, hidden 64
+                    // 23.2 us with them merged, 21.5 apart, hidden 128 50.9 and 47.9.  Volatile loads stay apart)
                     const float* xrow = xs + min(lr, n - 1) * KP + srt * q;
                     auto product = [&](auto steps) {
                         constexpr int S = decltype(steps)::value;
                         float2 x2[S / 2];
 #pragma unroll
-                        for (int s2 = 0; s2 < S / 2; ++s2) x2[s2] = *reinterpret_cast<const float2*>(xrow + 2 * s2);
+                        for (int s2 = 0; s2 < S / 2; ++s2) {
+                            if constexpr (S % 8 == 0) {
+                                const unsigned long long both = *reinterpret_cast<const volatile unsigned long long*>(xrow + 2 * s2);
+                                x2[s2] = make_float2(__uint_as_float((unsigned)both), __uint_as_float((unsigned)(both >> 32)));
+                            } else {
+                                x2[s2] = *reinterpret_cast<const float2*>(xrow + 2 * s2);
+                            }
+                        }
                         mfma_f4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                         for (int s2 = 0; s2 < S / 2; ++s2) {
