@@ -314,21 +314,23 @@ __global__ __launch_bounds__(WAVES * kWave, (min_waves<C, KSX, WAVES, KEEP, PACK
     // The position of the first graph (node range, then entry range) is asked for ahead of the weight
     // loads, so the two dependent trips to memory run under them instead of after them.
     int next_g = blockIdx.x, next_node0 = 0, next_n = 0, next_e0 = 0, next_e1 = 0, next_ng = 1;
-    // PACK: the place of the record of a bin, or -1 past the last one
+    // PACK: the place of the record of a bin, or -1 past the last one.  A workgroup asks for its bins in ascending order and goes on
+    // from the words that held the last one (from the first word for every bin: 500,000 graphs of 1 to 3 nodes, hidden 16 950 us, 709 so;
+    // 60,000 145, 141).
     const int nseg = (B + kWave - 1) / kWave;
+    int find_seg = 0, find_before = 0;           // 64 words from find_seg on, bins of the words before them
     auto find_bin = [&](int bin) {
         const unsigned long long* words = reinterpret_cast<const unsigned long long*>(order);
         const int lane = tid0 & (kWave - 1);
-        int before = 0;
-        for (int s0 = 0; s0 < nseg; s0 += kWave) {
-            const int count = s0 + lane < nseg ? __popcll(words[s0 + lane]) : 0;
-            const int through = before + wave_inclusive_scan_i(count);
+        for (; find_seg < nseg; find_seg += kWave) {
+            const int count = find_seg + lane < nseg ? __popcll(words[find_seg + lane]) : 0;
+            const int through = find_before + wave_inclusive_scan_i(count);
             const unsigned long long behind = __ballot(bin < through);
             if (behind) {
                 const int at = (int)__builtin_ctzll(behind);
-                return (s0 + at) * kWave + bin - __builtin_amdgcn_readlane(through - count, at);
+                return (find_seg + at) * kWave + bin - __builtin_amdgcn_readlane(through - count, at);
             }
-            before = __builtin_amdgcn_readlane(through, kWave - 1);
+            find_before = __builtin_amdgcn_readlane(through, kWave - 1);
         }
         return -1;
     };
