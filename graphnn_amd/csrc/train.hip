@@ -445,7 +445,9 @@ int gnnhip_s2v_readout_backward_f32(int B, int N, int C, int H, int Q,
         if (int rc = stream_scratch(s, sizeof(float) * (size_t)B * C, &dpool)) return rc;
     // (split: no rows are written, and the variant without the list entries' registers has more workgroups per compute unit: 22.5 us
     // at 10,000 graphs, hidden 256, against 29)
-    const bool vec = !split && C % 4 == 0 && C <= 4 * kBlock && aligned16(g_h);
+    // (few elements per graph: nothing to gain on the rows, and the entries' registers and the lanes' divisions come first: graphs of 3 nodes,
+    // hidden 32, 1,000 graphs 6.2 us against 6.8, 256 4.9 and 5.1; from two rounds of lanes per graph on the words are the faster ones)
+    const bool vec = !split && C % 4 == 0 && C <= 4 * kBlock && aligned16(g_h) && (long long)N * C >= 2ll * kBlock * B;
     hipLaunchKernelGGL(vec ? readout_backward_kernel<true> : readout_backward_kernel<false>, dim3((unsigned)blocks), dim3(kBlock), smem, s, B, C, H, Q,
                        s_row_ptr, s_col_idx, s_val, probs, lrow_ptr, lcol, lval, scale, hidden, W_h1, W_h2, dlogits, du, g_h, split ? 1 : 0);
     GNNHIP_LAUNCH_CHECK("readout_backward");

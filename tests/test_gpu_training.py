@@ -120,6 +120,30 @@ def test_readout_backward_rows_whatever_the_width(gpu, oracle, C):
     assert_parity("g_h", got[0], w_gh, gh64)
 
 
+@pytest.mark.parametrize("C,nodes", [(4, 3), (64, 7), (64, 8), (128, 3), (128, 4), (100, 5), (100, 6)])
+def test_readout_backward_of_small_graphs(gpu, C, nodes):
+    """from 512 elements per graph on the node rows are written as 128-bit words, below element by element: the same bits as in
+    a buffer that starts between two words, where they always are"""
+    import torch
+    from graphnn_amd import ops
+    B, H, Q = 37, 9, 3
+    N = B * nodes
+    gen = torch.Generator(device=gpu).manual_seed(C + nodes)
+    s = (torch.arange(B + 1, device=gpu).int() * nodes, torch.randperm(N, generator=gen, device=gpu).int(), torch.rand(N, generator=gen, device=gpu))
+    lab = (torch.arange(B + 1, device=gpu).int(), torch.randint(0, Q, (B,), generator=gen, device=gpu).int(), torch.ones(B, device=gpu))
+    probs, hidden = torch.rand(B, Q, generator=gen, device=gpu), torch.rand(B, H, generator=gen, device=gpu)
+    W1, W2 = torch.randn(C, H, generator=gen, device=gpu), torch.randn(H, Q, generator=gen, device=gpu)
+    dl, du, gh = ops.readout_backward(s, probs, lab, 0.25, hidden, W1, W2, N)
+    between = torch.zeros(N * C + 1, device=gpu)[1:].view(N, C)
+    ops._bound().s2v_readout_backward_f32(B, N, C, H, Q, *s, probs, *lab, 0.25, hidden, W1, W2, torch.empty_like(dl), torch.empty_like(du), between)
+    assert torch.equal(gh, between)
+    want = torch.zeros(N, C, dtype=torch.float64, device=gpu)
+    want[s[1].long()] = (du.double() @ W1.double().T).repeat_interleave(nodes, 0) * s[2].double()[:, None]
+    terms = torch.zeros_like(want)
+    terms[s[1].long()] = (du.double().abs() @ W1.double().abs().T).repeat_interleave(nodes, 0) * s[2].double()[:, None]
+    assert bool(((gh.double() - want).abs() <= (H + 2) * 2.0 ** -24 * terms).all())      # a rounding per product and sum, and the weight's
+
+
 @pytest.mark.parametrize("N,C", [(N, C) for C in (16, 32, 64, 128, 256) for N in (77, 7450, 40_000)] + [(70_001, 128), (70_001, 256), (16_400, 256)])
 def test_level_backward(gpu, oracle, C, N):
     """u = A^T dz and g_prev = u W^T in one pass (hidden 16/32/64: the streaming kernel; hidden 128/256: the wide kernel's
