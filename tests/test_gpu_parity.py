@@ -299,6 +299,37 @@ def test_transposed_product_at_the_edges_of_its_tiles(gpu, m, n, k):
             assert torch.equal(batched, got)
 
 
+@pytest.mark.parametrize("m,n", [(1, 1), (16, 16), (17, 33), (32, 32), (25, 41), (16, 65), (64, 2), (7, 256), (65, 64), (130, 66)])
+@pytest.mark.parametrize("k", [1, 2, 4, 5, 31, 32, 33, 47, 48, 49])
+def test_transposed_product_over_few_rows(gpu, m, n, k):
+    """A^T B over up to 32 rows, and up to 48 where the output has at most 1,024 elements, without sharing the rows between wavefronts:
+    NaN behind the columns and infinities behind the rows are not read into the result.  Every element within k + 8 roundings of
+    the sum of its terms' magnitudes of float64 (one per product and sum, and those of alpha and beta); the same bits from a batch
+    of products, short and long ones"""
+    import torch
+    from graphnn_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(1000 * m + n + k)
+    def operand(rows, cols, pad):
+        held = torch.full((rows + 3, cols + pad), float("nan"), device=gpu)
+        held[rows:] = float("inf")
+        held[:rows, :cols] = torch.randn(rows, cols, generator=gen, device=gpu)
+        return held
+    for pad, alpha, beta in ((0, 1.0, 0.0), (3, -0.75, 0.5)):
+        A, B = operand(k, m, pad), operand(k, n, pad)
+        out0 = torch.randn(m, n, generator=gen, device=gpu)
+        a64, b64 = A[:k, :m].double(), B[:k, :n].double()
+        want = alpha * (a64.T.contiguous() @ b64) + beta * out0.double()
+        terms = abs(alpha) * (a64.abs().T.contiguous() @ b64.abs()) + abs(beta) * out0.double().abs()
+        got = ops.gemm(A[:k], B[:k], transA=True, alpha=alpha, beta=beta, out=out0.clone(), cols_a=m, cols_b=n)
+        assert bool(((got.double() - want).abs() <= (k + 8) * 2.0 ** -24 * terms).all())
+        if pad == 0:
+            long_a, long_b = operand(400, 20, 0)[:400], operand(400, 30, 0)[:400]
+            batched = [out0.clone() for _ in range(2)]
+            ops.gemm_tn_batch([(A[:k], B[:k], batched[0]), (long_a, long_b, torch.zeros(20, 30, device=gpu)), (A[:k], B[:k], batched[1])],
+                              alpha=alpha, beta=beta)
+            assert torch.equal(batched[0], got) and torch.equal(batched[1], got)
+
+
 def test_gemm_reference_test_shape(gpu, oracle):
     """10x20 . (30x20)^T with |delta ASum| <= 1e-4 (test/gpu_tensor_test.cpp:131-149)"""
     from graphnn_amd import ops
