@@ -316,13 +316,15 @@ int launch_rows(const RowsArgs& a, hipStream_t s)
 // whose phases have nothing to hide behind, and 32 rows are the better ones (hidden 85, 22,000 nodes: 21.0 -> 15.4 us per
 // level, 24.7 -> 18.3 backward; 38,000: 29.7 -> 24.5), up to the 49,152 rows that six workgroups per compute unit hold at once
 // where the registers allow so many (from 40,960 on: 48,750 nodes, hidden 36 to 100 6 to 12 % less; below, the registers
-// that this takes away cost 3 %).  51,000 nodes take two rounds: 2 to 8 % slower than 64 rows.
+// that this takes away cost 3 %; up to 8 columns a tile is one short phase, and 64 rows are the faster ones there: hidden 4, 45,000
+// nodes 9.9 us, 10.4 with 32 rows; hidden 125 to 127 backward lose 1 to 4 % from 43,000 nodes on with 2.2 entries per row and gain 2 to 3 with 8).
+// 51,000 nodes take two rounds: 2 to 8 % slower than 64 rows.
 template <int NB, bool GATHER, bool WT>
 int rows_by_tile(const RowsArgs& a, hipStream_t s)
 {
     if (a.N < 64 * kNumCU) return launch_rows<1, NB, 3, GATHER, WT>(a, s);
     if (a.N < 160 * kNumCU) return launch_rows<2, NB, 3, GATHER, WT>(a, s);
-    if (a.N <= 6 * 32 * kNumCU) return launch_rows<2, NB, 6, GATHER, WT>(a, s);
+    if (a.N <= 6 * 32 * kNumCU && a.n > 8) return launch_rows<2, NB, 6, GATHER, WT>(a, s);
     return launch_rows<4, NB, 3, GATHER, WT>(a, s);
 }
 
