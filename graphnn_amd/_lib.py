@@ -50,6 +50,7 @@ SIGNATURES = {
     "gnnhip_s2v_level_planned_f32": [_P, _I, _P, _P, _P, _P, _P, _P],
     "gnnhip_release_scratch": [_P],
     "gnnhip_csr_group_i32": [_I, _I, _P, _I, _P, _I, _I, _P, _P, _P, _P],
+    "gnnhip_csr_group_one_launch": [_I, _I],
     "gnnhip_csr_group_both_i32": [_I, _I, _P, _I, _P, _I, _P, _P, _P, _P, _P, _P, _P],
     "gnnhip_csr_consecutive_rows_f32": [_I, _P, _I, _P, _P, _P],
     "gnnhip_csr_consecutive_rows_host_f32": [_I, _P, _I, _P, _P, _P, _P],

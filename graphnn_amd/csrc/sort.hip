@@ -881,6 +881,12 @@ int gnnhip_csr_group_i32(int rows, int n, const int* key, int key_stride, const 
     return csr_group(rows, n, key, key_stride, payload, payload_stride, nullptr, average, row_ptr, col_idx, val, as_stream(stream));
 }
 
+int gnnhip_csr_group_one_launch(int rows, int n)
+{
+    SmallLayout lay;
+    return small_layout(rows, n, &lay) ? 1 : 0;
+}
+
 int gnnhip_csr_consecutive_rows_f32(int rows, const int* row_ptr, int average, int* col_idx, float* val, void* stream)
 {
     GNNHIP_REQUIRE(rows >= 0, "negative row count in csr_consecutive_rows");

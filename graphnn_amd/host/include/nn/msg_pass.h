@@ -9,6 +9,7 @@
 #ifndef MSG_PASS_H
 #define MSG_PASS_H
 
+#include <climits>
 #include "nn/factor.h"
 #include "util/graph_struct.h"
 
@@ -147,14 +148,13 @@ inline void consecutive_rows_on_device(GraphStruct* graph, std::vector<int>& off
     GNN_HIP(gnnhip_csr_consecutive_rows_host_f32(B, offsets.data(), average ? 1 : 0, out.data->row_ptr, out.data->col_idx, out.data->val,
                                                  GpuHandle::Stream()));
 }
-// The device groups a batch in one launch (up to 16 workgroups, each a run of the rows) when a run's counters
-// (4 bytes per row) and the slots of all pairs (2.35 bytes each, with the lists and one bitmap) fit 160 KB of
-// LDS, and with a radix sort from 65,536 pairs.  What is left to the host loop is what neither covers (fewer
-// pairs than that over more than about 40,000 rows), where the dozen launches of the sort cost more than the loop.
+// The device groups a batch in one launch where the library says so (up to 65,535 pairs over as many rows as its LDS holds:
+// some 100,000 of them with 60,000 pairs, millions with few), and with a radix sort from 65,536 pairs.  What is left to the host loop is
+// what neither covers, where the dozen launches of the sort cost more than the loop.
 constexpr size_t kRadixGroupingPairs = 1u << 16;
 inline bool device_grouping_pays(size_t pairs, size_t rows)
 {
-    return pairs >= kRadixGroupingPairs || rows / 4 + 47 * pairs / 20 + 1024 <= 160 * 1024;
+    return pairs >= kRadixGroupingPairs || rows == 0 || (rows <= INT_MAX && gnnhip_csr_group_one_launch((int)rows, pairs ? (int)pairs : 1) != 0);
 }
 template<typename Dtype, typename SpT>
 inline bool group_edges_if_gpu(GraphStruct*, bool, bool, size_t, SpT&, DTensor<GPU, int>&, bool = false) { return false; }

@@ -150,11 +150,14 @@ int gnnhip_spmm_csr_planned_f32(void* plan, int n, float alpha, const float* B, 
  *      key[e * key_stride], payload[e * payload_stride] (strides in ints, so an array of (x, y) pairs
  *      can be passed as it is).  val = 1, or 1 / row length when average != 0.  Stable radix sort without
  *      atomics on global memory, or, for up to 65,536 pairs (2.35 bytes each, plus 4 bytes per row of a
- *      sixteenth of the rows, have to fit 160 KB of LDS), one launch that puts every row back into input order:
+ *      64th of the rows, have to fit 160 KB of LDS), one launch that puts every row back into input order:
  *      either way the result is a pure function of the input, bit-identical to the host construction.
  *      The outputs must not overlap key or payload. */
 int gnnhip_csr_group_i32(int rows, int n, const int* key, int key_stride, const int* payload, int payload_stride,
                          int average, int* row_ptr, int* col_idx, float* val, void* stream);
+/* 1 where gnnhip_csr_group_i32 groups n pairs over so many rows in one launch, 0 where it sorts them (a dozen launches; below
+ * 65,536 pairs a loop on the host is faster than those).  Needs no device. */
+int gnnhip_csr_group_one_launch(int rows, int n);
 
 /* ---- the entries of a CSR matrix whose row i lists the consecutive columns row_ptr[i] .. row_ptr[i+1]-1 with value 1
  *      (1 / row length when average != 0): the operand of SubgraphMsgPass (src/nn/msg_pass.cpp:156-177) for a batch

@@ -89,6 +89,15 @@ def test_bindings_take_no_integer_for_a_device_tensor():
     assert tried > 200
 
 
+@pytest.mark.parametrize("rows,n,fits", [(1, 1, 1), (7_450, 16_380, 1), (9_000, 60_000, 1), (100_000, 60_000, 1), (156_000, 65_536, 1),
+                                         (157_500, 65_536, 0), (300_000, 65_536, 0), (2_000_000, 1_000, 1), (2_700_000, 1_000, 0), (100, 65_537, 0),
+                                         (0, 5, 0), (5, 0, 0)])
+def test_grouping_in_one_launch_is_a_rule_of_its_own(rows, n, fits):
+    """which (rows, pairs) one launch groups: 2.35 bytes per pair and 4 per row of a 64th of the rows in 160 KB, at most 65,536 pairs.
+    The host layer asks this to choose between the device and its own loop"""
+    assert binding.load_library().gnnhip_csr_group_one_launch(rows, n) == fits
+
+
 def test_plan_entries_reject_what_is_not_a_plan():
     lib = binding.load_library()
     x = np.zeros(8, np.float32)

@@ -327,6 +327,43 @@ def test_host_api_large_batch_takes_the_separate_kernels(gpu, oracle, tmp_path):
     assert abs(loss_t - loss) <= 1e-5 * abs(loss) and acc_t == acc
 
 
+def test_host_api_many_nodes_with_few_edges(gpu, tmp_path):
+    """100,000 nodes with 60,000 edges in any order: more rows than the host layer once left to its own loop, few enough pairs for the
+    device's one launch; the tensor products and the levels over the operand that the message-pass factor builds, against float64"""
+    exe = os.path.join(BUILD, "host_big_graph_check")
+    assert os.path.exists(exe), "build the host layer first: make -C graphnn_amd/host"
+    N, E, K, C, L = 100_000, 60_000, 3, 16, 2
+    rng = np.random.default_rng(12)
+    x, y = rng.integers(0, N, E).astype(np.int32), rng.integers(0, N, E).astype(np.int32)
+    y[:300] = 77_777                                   # a long row among rows of one or two entries
+    val, val2 = (rng.random(E).astype(np.float32) - 0.3 for _ in range(2))
+    B = rng.standard_normal((N, C)).astype(np.float32)
+    X = rng.random((N, K)).astype(np.float32)
+    Wn, W = rng.standard_normal((K, C)).astype(np.float32), (rng.standard_normal((C, C)) * 0.2).astype(np.float32)
+    d = str(tmp_path)
+    np.stack([x, y], axis=1).astype(np.int32).tofile(d + "/edges.bin")
+    for name, arr in (("val", val), ("val2", val2), ("b", B), ("x", X), ("w_n2l", Wn), ("w", W)):
+        arr.tofile(d + "/%s.bin" % name)
+    r = subprocess.run([exe, d, str(N), str(K), str(C), str(L)], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
+    out = np.fromfile(d + "/out.bin", dtype=np.float32).reshape(5, N, C)
+    order = np.argsort(y, kind="stable")               # the values are listed row after row, a row's entries in edge order
+    rows, cols = y[order], x[order]
+    def product(v, dense, transposed=False):
+        got = np.zeros((N, C))
+        np.add.at(got, cols if transposed else rows, v[:, None] * dense[rows if transposed else cols])
+        return got
+    relu = lambda t: np.maximum(t, 0)
+    f8 = np.float64
+    h = relu(X.astype(f8) @ Wn)
+    msg = X.astype(f8) @ Wn
+    ones = np.ones(E)
+    for _ in range(L):
+        h = relu(product(ones, h) @ W.astype(f8) + msg)
+    for got, want in zip(out, (product(val, B.astype(f8)), product(val, B.astype(f8)), product(val, B.astype(f8), True), product(val2, B.astype(f8)), h)):
+        assert max_rel(got, want) < 1e-5
+
+
 def test_host_api_large_dense_graph_keeps_the_plan_of_its_operand(gpu, oracle, tmp_path):
     """one R-MAT graph of 65,536 nodes, 16 edges per node, through graphnn's tensor and FactorGraph API
     (host/tests/host_big_graph_check.cpp): the sparse operand takes the library's planned products, the plan is kept
