@@ -270,7 +270,7 @@ __device__ __forceinline__ void tn_tile_body(int m, int n, float alpha, const fl
 // take: 16 rows, 16 x 16 3.8 -> 2.2 us, 38 x 64 3.8 -> 3.3, 1,000 x 500 4.5 -> 3.9.  The line lies at 32 rows, and at 48 for outputs of
 // up to 1,024 elements (48 rows, 16 x 16: 4.6 -> 3.2; 38 x 64: 4.2 -> 4.7).
 constexpr int kTnShort = 32, kTnShortSmall = 48;
-__host__ __device__ inline bool tn_short(int m, int n, int k) { return k <= ((long long)m * n <= 1024 ? kTnShortSmall : kTnShort); }
+inline bool tn_short(int m, int n, int k) { return k <= ((long long)m * n <= 1024 ? kTnShortSmall : kTnShort); }
 template <int ROWS>
 __device__ __forceinline__ void tn_short_body(int m, int n, int k, float alpha, const float* __restrict__ A, int lda, const float* __restrict__ B,
                                               int ldb, float beta, float* C, int ldc, int tile_x, int tile_y)
@@ -318,7 +318,9 @@ struct GemmJob {                                // a cache line of the kernel's 
     const float* B;
     float* C;
     float* partial;                             // null: one range, finished by the product launch
-    int m, n, k, lda, ldb, ldc, k_chunk, splits;
+    int m, n, k, lda, ldb, ldc;
+    int k_chunk;                                // 0: tn_short
+    int splits;
 };
 struct GemmBatch {
     int z0[kGemmBatch];                         // INT_MAX from `count` on
@@ -332,6 +334,8 @@ __global__ __launch_bounds__(kBlock) void sgemm_tn_short_kernel(GemmJob j, float
     tn_short_body<ROWS>(j.m, j.n, j.k, alpha, j.A, j.lda, j.B, j.ldb, beta, j.C, j.ldc, (int)blockIdx.x, (int)blockIdx.y);
 }
 
+// SHORT: some of the products may be short ones
+template <bool SHORT>
 __global__ __launch_bounds__(kBlock, 3) void sgemm_tn_batch_kernel(GemmBatch b, float alpha, float beta)
 {
     __shared__ float4 sums[kTnWaves - 1][4][4][kWave];        // [wavefront other than a block's owner][block of A][block of B][lane]
@@ -341,7 +345,7 @@ __global__ __launch_bounds__(kBlock, 3) void sgemm_tn_batch_kernel(GemmBatch b, 
     const GemmJob j = b.job[p];
     const int m = j.m, n = j.n;
     if ((long long)blockIdx.x * BM >= m || (int)blockIdx.y * BN >= n) return;
-    if (tn_short(m, n, j.k)) {
+    if (SHORT && j.k_chunk == 0) {
         tn_short_body<kTnShortSmall>(m, n, j.k, alpha, j.A, j.lda, j.B, j.ldb, beta, j.C, j.ldc, (int)blockIdx.x, (int)blockIdx.y);
         return;
     }
@@ -630,7 +634,7 @@ int gemm_tn_batch_dispatch(int count, const int* m, const int* n, const int* k, 
         // the rule of the single product, so that a batch gives the bits of its products done one by one
         long long chunk = tiles <= kNumCU / 4 && k[p] >= 256 ? tn_chunk(tiles, k[p]) : (k[p] > 0 ? k[p] : 1);
         const int splits = k[p] > 0 ? (int)(((long long)k[p] + chunk - 1) / chunk) : 1;
-        b.job[q] = GemmJob{A[p], B[p], C[p], nullptr, m[p], n[p], k[p], lda[p], ldb[p], ldc[p], (int)chunk, splits};
+        b.job[q] = GemmJob{A[p], B[p], C[p], nullptr, m[p], n[p], k[p], lda[p], ldb[p], ldc[p], tn_short(m[p], n[p], k[p]) ? 0 : (int)chunk, splits};
         b.z0[q] = z;
         z += splits;
         offset[q] = splits > 1 ? floats : kDirect;
@@ -640,7 +644,7 @@ int gemm_tn_batch_dispatch(int count, const int* m, const int* n, const int* k, 
         if (splits > 1) red = std::max(red, std::min(ceil_div_u((size_t)m[p] * n[p], kWave), 2048u));
     }
     if (b.count == 0) return GNNHIP_OK;
-    if (b.count == 1 && tn_short(b.job[0].m, b.job[0].n, b.job[0].k)) {
+    if (b.count == 1 && b.job[0].k_chunk == 0) {
         hipLaunchKernelGGL(b.job[0].k <= kTnShort ? sgemm_tn_short_kernel<kTnShort> : sgemm_tn_short_kernel<kTnShortSmall>, dim3(gx, gy), dim3(kBlock), 0, s,
                            b.job[0], alpha, beta);
         GNNHIP_LAUNCH_CHECK("sgemm_tn_short");
@@ -651,7 +655,13 @@ int gemm_tn_batch_dispatch(int count, const int* m, const int* n, const int* k, 
     if (floats)
         if (int rc = stream_scratch_slot(s, 2, sizeof(float) * floats, &q)) return rc;
     for (int p = 0; p < b.count; ++p) b.job[p].partial = offset[p] == kDirect ? nullptr : static_cast<float*>(q) + offset[p];
-    hipLaunchKernelGGL(sgemm_tn_batch_kernel, dim3(gx, gy, (unsigned)z), dim3(kBlock), 0, s, b, alpha, beta);
+    // The two variants differ in what the compiler makes of the long products, too: the one without the short body starts sooner (64 x 64 over
+    // 200 rows 7.1 us, 7.3 with it; 7,450 nodes x 4 levels 13.5, 13.7), the other one is ahead where tiles follow each other on a
+    // compute unit (2,000^2 over 200 rows 35.0, 30.0; over 1,000 94.3, 92.9), from some two per compute unit on; 1,200^2 is even.
+    // Over 48 to 64 rows that one is 2 to 3 % behind at any size.
+    bool with_short = false;
+    for (int p = 0; p < b.count; ++p) with_short |= b.job[p].k_chunk == 0 || (b.job[p].k >= 128 && (long long)gx * gy > 2 * kNumCU);
+    hipLaunchKernelGGL(with_short ? sgemm_tn_batch_kernel<true> : sgemm_tn_batch_kernel<false>, dim3(gx, gy, (unsigned)z), dim3(kBlock), 0, s, b, alpha, beta);
     if (red) hipLaunchKernelGGL(sgemm_splitk_reduce_batch_kernel, dim3(red, (unsigned)b.count), dim3(kBlock), 0, s, b, alpha, beta);
     GNNHIP_LAUNCH_CHECK("sgemm_tn_batch");
     return GNNHIP_OK;
