@@ -523,14 +523,16 @@ int order_pieces(CsrPlan* p, int cap, const Layout& L, char* temp, hipStream_t s
     int* hist = reinterpret_cast<int*>(temp + L.o_hist);
     int bits = 1;
     while (bits < 31 && (1ll << bits) < (long long)p->k) ++bits;
-    // Up to 2^20 columns the top eight bits, one narrow pass: pieces that follow each other share 4,096 columns at most, whose
-    // rows of B an L2 holds, and a finer order gains nothing because a row's other entries lie elsewhere anyway.  A forward of
+    // Up to 2^20 columns the top eight bits, one narrow pass: pieces that follow each other share 4,096 columns at most, and a finer order
+    // gains nothing because a row's other entries lie elsewhere anyway.  A forward of
     // three levels over an R-MAT graph of 13 entries per row, no plan kept, eight bits against eleven: hidden 32, 100,000 rows
     // 201 us / 208, 300,001 344 / 354, 600,000 646 / 665, 1,000,000 1,072 / 1,102; hidden 64 266 / 270, 537 / 553, 1,077 / 1,100,
-    // 1,807 / 1,838; seven bits are within 1 % of eight, and with a plan that is kept the three are alike.  Past 2^20 sixteen
-    // bits in two passes: there a kept plan is what the order is for, and with eight bits it loses 0.5 % at 1,600,000 rows of
-    // 16 entries and 2.9 % at 4,194,304 (hidden 64: 7,808 us / 7,590; ten and eleven bits 0.8 % and 0.4 %).
-    const int order_bits = bits <= 20 ? 8 : 16;
+    // 1,807 / 1,838; one product of width 256 556 / 582 at 300,001 rows, 1,662 / 1,706 at 1,000,000.  With a plan that is kept the two are
+    // alike up to 2^19 columns (width 32 to 512: eight bits 0.4 % behind to 2.4 % ahead), and from there on rows of B are wide enough together
+    // to miss: 1,000,000 columns, width 256 1,470 / 1,451 us, of 30 entries per row 2,702 / 2,628, width 32 to 64 up to 0.7 % more; so
+    // those plans take eleven bits.  Past 2^20 sixteen bits in two passes: there a kept plan is what the order is for, and with eight bits it
+    // loses 0.5 % at 1,600,000 rows of 16 entries and 2.9 % at 4,194,304 (hidden 64: 7,808 us / 7,590; ten and eleven bits 0.8 % and 0.4 %).
+    const int order_bits = bits > 20 ? 16 : bits == 20 && p->owned ? 11 : 8;
     const int shift = bits > order_bits ? bits - order_bits : 0;
     hipLaunchKernelGGL(piece_fill_kernel, dim3(elem_grid(p->slots)), dim3(kBlock), 0, s, p->m, p->slots, p->row_ptr, cap, p->col_idx, p->first,
                        p->pfirst, shift, (1u << order_bits) - 1, rec, keys);

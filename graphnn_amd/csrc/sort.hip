@@ -717,10 +717,10 @@ inline size_t round_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 }  // namespace
 
-// order[i] = index of the key that comes i-th when n keys of `bits` bits (8: one pass of the radix sort, 16: two) are put in
+// order[i] = index of the key that comes i-th when n keys of `bits` bits (8 and 11: one pass of the radix sort, 16: two) are put in
 // order, equal keys in input order.  keys, keys_out and spare are overwritten.  hist needs radix_hist_ints(n) ints, seg
 // radix_seg_ints(n).
-size_t radix_hist_ints(long long n) { return ((size_t)1 << 8) * (size_t)((n + kTile - 1) / kTile > 0 ? (n + kTile - 1) / kTile : 1); }
+size_t radix_hist_ints(long long n) { return ((size_t)1 << 11) * (size_t)((n + kTile - 1) / kTile > 0 ? (n + kTile - 1) / kTile : 1); }
 size_t radix_seg_ints(long long n) { return scan_seg_ints((long long)radix_hist_ints(n)); }
 
 namespace {
@@ -752,9 +752,9 @@ int radix_order(unsigned* keys, int bits, long long n, unsigned* keys_out, unsig
     j.key_stride = 1;
     j.k1 = keys_out;
     j.hist = hist; j.seg = seg;
-    if (bits <= 8) {
+    if (bits <= 11) {
         j.v1 = order;
-        return radix_pass<8>(1, jobs, true, n, 1 << 8, 0, s);
+        return bits <= 8 ? radix_pass<8>(1, jobs, true, n, 1 << 8, 0, s) : radix_pass<11>(1, jobs, true, n, 1 << 11, 0, s);
     }
     j.v1 = spare;
     if (int rc = radix_pass<8>(1, jobs, true, n, 1 << 16, 0, s)) return rc;

@@ -1797,6 +1797,23 @@ def test_spmm_pieces_whatever_bits_their_order_takes(gpu, oracle, k):
     assert np.array_equal(got, oracle.spmm(row_ptr, col, val, B, m))
 
 
+@pytest.mark.parametrize("k", [257, 1 << 19, (1 << 19) + 1, 1 << 20, (1 << 20) + 1])
+def test_kept_plans_whatever_bits_their_order_takes(gpu, k):
+    """a plan that is kept orders its pieces by eight, eleven or sixteen bits of their first column, by the number of columns, a call
+    without one by eight up to 2^20: the same bits, whatever the order, with rows of one piece and of several"""
+    from graphnn_amd import ops
+    import torch
+    m, n = 32768, 33
+    gen = torch.Generator(device=gpu).manual_seed(k)
+    deg = torch.randint(4, 60, (m,), device=gpu, generator=gen)
+    row_ptr = torch.cat([torch.zeros(1, dtype=torch.int64, device=gpu), deg.cumsum(0)]).int()
+    col = torch.randint(0, k, (int(row_ptr[-1]),), device=gpu, generator=gen).int()
+    val, B = torch.randn(col.numel(), device=gpu, generator=gen), torch.randn(k, n, device=gpu, generator=gen)
+    want = ops.spmm(row_ptr, col, val, B, m)
+    with ops.CsrPlan(row_ptr, col, val, m, k) as plan:
+        assert torch.equal(plan.spmm(B), want)
+
+
 @pytest.mark.parametrize("m", [33_790, 33_791, 33_792, 34_000, 2_097_153])
 def test_spmm_pieces_at_the_edges_of_their_scans(gpu, m):
     """rows whose counts fill segments of 1,024 to the last element, pass one by an element, and pass the 2,048 segments that a
