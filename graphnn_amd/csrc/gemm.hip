@@ -145,8 +145,8 @@ __global__ __launch_bounds__(kBlock) void sgemm_tile_kernel(
 // 64 x 64 tile, without LDS and without a barrier; the four wavefronts of a workgroup take four rows of sixteen each and add
 // up their tiles in wavefront order at the end.  An output tile ends with a lane holding four consecutive columns.
 // What bounds it at the sizes of a training batch is one or two trips to memory, the sum over the wavefronts and the launch: with the
-// sums of the ranges 7,450 nodes x 4 levels at hidden 64 (four products) take 13.5 us, 1,625 x 3 10.0 (LDS tiles and a
-// barrier per sixteen rows: 20.5 and 12.5); 1,000 x 500 over 3,000 rows 57 (128), 2,048^3 178 = 96 TFLOP/s (210).
+// sums of the ranges 7,450 nodes x 4 levels at hidden 64 (four products) take 13.5 us, 1,625 x 3 8.4 (LDS tiles and a
+// barrier per sixteen rows: 20.4 and 11.4); 1,000 x 500 over 3,000 rows 57 (128), 2,048^3 178 = 96 TFLOP/s (210).
 // Six steps under way: four take 0.3 to 1 us more where a range is short, eight spill.
 constexpr int kTnWaves = kBlock / kWave;
 constexpr int kTnStep = 4 * kTnWaves;        // rows of k per step of the workgroup
