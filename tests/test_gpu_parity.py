@@ -300,7 +300,7 @@ def test_transposed_product_at_the_edges_of_its_tiles(gpu, m, n, k):
 
 
 @pytest.mark.parametrize("m,n", [(1, 1), (16, 16), (17, 33), (32, 32), (25, 41), (16, 65), (64, 2), (7, 256), (65, 64), (130, 66)])
-@pytest.mark.parametrize("k", [1, 2, 4, 5, 31, 32, 33, 47, 48, 49])
+@pytest.mark.parametrize("k", [0, 1, 2, 4, 5, 31, 32, 33, 47, 48, 49])
 def test_transposed_product_over_few_rows(gpu, m, n, k):
     """A^T B over up to 32 rows, and up to 48 where the output has at most 1,024 elements, without sharing the rows between wavefronts:
     NaN behind the columns and infinities behind the rows are not read into the result.  Every element within k + 8 roundings of
@@ -328,6 +328,21 @@ def test_transposed_product_over_few_rows(gpu, m, n, k):
             ops.gemm_tn_batch([(A[:k], B[:k], batched[0]), (long_a, long_b, torch.zeros(20, 30, device=gpu)), (A[:k], B[:k], batched[1])],
                               alpha=alpha, beta=beta)
             assert torch.equal(batched[0], got) and torch.equal(batched[1], got)
+
+
+@pytest.mark.parametrize("m,n,k", [(1409, 1473, 127), (1409, 1473, 128), (1409, 1473, 131), (33, 32_705, 141), (1409, 1472, 33)])
+def test_transposed_product_of_many_tiles(gpu, m, n, k):
+    """A^T B of more than 512 tiles over 128 rows and more, one row less, and few rows: every element within k + 8 roundings of the sum of its
+    terms' magnitudes of float64, and the bits that the same columns have as an output of a few tiles"""
+    import torch
+    from graphnn_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(m + k)
+    A, B = torch.randn(k, m, generator=gen, device=gpu), torch.randn(k, n, generator=gen, device=gpu)
+    got = ops.gemm(A, B, transA=True)
+    want, terms = A.double().T.contiguous() @ B.double(), A.double().abs().T.contiguous() @ B.double().abs()
+    assert bool(((got.double() - want).abs() <= (k + 8) * 2.0 ** -24 * terms).all())
+    few = ops.gemm(A, B, transA=True, cols_a=min(m, 128), cols_b=128)
+    assert torch.equal(few[:, :128], got[:few.shape[0], :128])
 
 
 def test_gemm_reference_test_shape(gpu, oracle):
