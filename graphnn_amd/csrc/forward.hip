@@ -9,13 +9,18 @@ namespace gnnhip {
 
 // defined in level.hip / spmm.hip / gemm.hip / reduce.hip
 bool fused_hidden_supported(int C);
-int input_dispatch(int N, int K, int C, const float* X, const float* Wn2l, float* msg, float* h0, hipStream_t s);
+int input_dispatch(int N, int K, int C, const float* X, const float* Wn2l, float* msg, float* h0, hipStream_t s, const int* gate);
 int level_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* h_in,
                    const float* W, const float* msg, const float* bias, float* h_out, hipStream_t s, bool same_graph = false,
-                   bool relu_in = false, CsrPlan* plan = nullptr, bool inference = false);
+                   bool relu_in = false, CsrPlan* plan = nullptr, bool inference = false, const int* gate = nullptr);
 bool level_accepts_relu_input(int N, int C);
 int level_backward_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* dz,
                             const float* W, float* u, float* g_prev, const float* gate, float* acc, hipStream_t s);
+// batch_forward.hip
+size_t batch_levels_work_ints(int B);
+int batch_levels_dispatch(int N, int B, int K, int C, int L, long long nnz, const int* a_row_ptr, const int* a_col_idx, const float* a_val,
+                          const int* s_row_ptr, const float* X, const float* Wn2l, const float* Wc, float* msg, float* h_out, int* work,
+                          const int** refused, hipStream_t s);
 // level_rows.hip
 int level_rows_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* h_in,
                         const float* W, const float* msg, const float* bias, float* h_out, bool same_graph, bool relu_in, CsrPlan* plan,
@@ -78,9 +83,9 @@ int product_any(int N, int K, int n, const float* x, const float* W, const float
     return GNNHIP_OK;
 }
 
-int input_any(int N, int K, int C, const float* X, const float* Wn2l, float* msg, float* h0, hipStream_t s)
+int input_any(int N, int K, int C, const float* X, const float* Wn2l, float* msg, float* h0, hipStream_t s, const int* gate = nullptr)
 {
-    int rc = input_dispatch(N, K, C, X, Wn2l, msg, h0, s);
+    int rc = input_dispatch(N, K, C, X, Wn2l, msg, h0, s, gate);
     if (rc != GNNHIP_EUNSUPPORTED) return rc;
     if (h0) return product_any(N, K, C, X, Wn2l, nullptr, nullptr, msg, h0, s);
     rc = level_rows_dense_dispatch(N, K, C, X, Wn2l, nullptr, nullptr, msg, false, nullptr, s);
@@ -90,9 +95,9 @@ int input_any(int N, int K, int C, const float* X, const float* Wn2l, float* msg
 
 int level_any(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* h_in,
               const float* W, const float* msg, const float* bias, float* h_out, hipStream_t s, bool same_graph = false,
-              bool relu_in = false, CsrPlan* plan = nullptr, bool inference = false)
+              bool relu_in = false, CsrPlan* plan = nullptr, bool inference = false, const int* gate = nullptr)
 {
-    int rc = level_dispatch(N, C, nnz, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, s, same_graph, relu_in, plan, inference);
+    int rc = level_dispatch(N, C, nnz, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, s, same_graph, relu_in, plan, inference, gate);
     if (rc != GNNHIP_EUNSUPPORTED) return rc;
     rc = level_rows_dispatch(N, C, nnz, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, same_graph, relu_in, plan, s);
     if (rc != GNNHIP_EUNSUPPORTED) return rc;
@@ -153,13 +158,21 @@ int forward_any(int N, int B, int K, int C, int H, int Q, int L, long long a_nnz
     // never stored: the first level gathers from msg.
     // (the routes of the other sizes can too)
     const bool lazy_h0 = L >= 1 && (level_accepts_relu_input(N, C) || !fused_hidden_supported(C)) && aligned16(msg) && aligned16(h_a) && aligned16(h_b) && aligned16(W_conv);
-    int rc = input_any(N, K, C, X, W_n2l, msg, lazy_h0 ? nullptr : h_a, s);
-    if (rc) return rc;
+    // Batches of small graphs: input stage and levels in one launch, which finds out on the device whether the batch is one; what it
+    // needs for that lies in pool, which is written last.  The level-by-level launches behind it do nothing if it is.
+    const int* gate = nullptr;
+    int rc;
+    if (lazy_h0 && aligned16(pool) && batch_levels_work_ints(B) <= (size_t)B * C) {
+        rc = batch_levels_dispatch(N, B, K, C, L, a_nnz, a_row_ptr, a_col_idx, a_val, s_row_ptr, X, W_n2l, W_conv, msg, (L & 1) ? h_a : h_b,
+                                   reinterpret_cast<int*>(pool), &gate, s);
+        if (rc && rc != GNNHIP_EUNSUPPORTED) return rc;
+    }
+    if ((rc = input_any(N, K, C, X, W_n2l, msg, lazy_h0 ? nullptr : h_a, s, gate))) return rc;
     float* cur = lazy_h0 ? msg : h_a;
     float* nxt = lazy_h0 ? h_a : h_b;
     for (int lv = 0; lv < L; ++lv) {
         if ((rc = level_any(N, C, a_nnz, a_row_ptr, a_col_idx, a_val, cur, W_conv, msg, nullptr, nxt, s, lv > 0,
-                            lazy_h0 && lv == 0, plan, true)))
+                            lazy_h0 && lv == 0, plan, true, gate)))
             return rc;
         float* t = (cur == msg) ? h_b : cur;     // msg stays what it is; the other buffer takes the next level
         cur = nxt;

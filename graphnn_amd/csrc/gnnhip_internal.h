@@ -158,6 +158,10 @@ __device__ __forceinline__ void wave_argmax(float& v, int& i)
     i = i0;
 }
 
+// A launch that is given a gate, a device word, does nothing where the word is 0: the level-by-level forward behind a launch that
+// has found out on the device whether it was needed (batch_forward.hip).  A wavefront that has nothing to do ends with its first load.
+__device__ __forceinline__ bool gated_off(const int* gate) { return gate && *gate == 0; }
+
 // ---------------------------------------------------------------- small vector helpers
 typedef float mfma_f4 __attribute__((ext_vector_type(4)));   // accumulator of v_mfma_f32_16x16x4_f32
 
@@ -250,7 +254,8 @@ struct HubStore {
 // AND same values (the column-ordered pieces keep a copy of the values), nothing rewritten in between.
 int hub_prepass(int m, int n, long long nnz, const int* row_ptr, const int* col_idx, const float* val,
                 const float* B, int ldb, hipStream_t s, HubPlan* plan, bool reuse_plan = false, bool relu_in = false,
-                int threshold = kHubThreshold, int chunk_len = kHubChunk, long long max_hubs = -1, HubStore* store = nullptr);
+                int threshold = kHubThreshold, int chunk_len = kHubChunk, long long max_hubs = -1, HubStore* store = nullptr,
+                const int* gate = nullptr);
 // scratch bytes of that call (0 when the pass does not apply)
 size_t hub_scratch_bytes(int m, int n, long long nnz, int threshold = kHubThreshold, int chunk_len = kHubChunk, long long max_hubs = -1);
 // runtime.hip: host bytes placed in the stream's pinned staging buffer for a kernel to read in place (null: not to be had)

@@ -32,6 +32,7 @@
 
 #include "gnnhip_internal.h"
 #include "buffer_addr.h"
+#include "graph_bins.h"
 
 // Phase markers for a timing build of this file; they expand to nothing in the library.
 #ifndef GNNHIP_PHASE_MARK
@@ -105,7 +106,6 @@ constexpr int kOrderMinGraphs = kNumCU;          // up to here every graph has a
 constexpr int kOrderBlock = 1024;
 constexpr int kOrderSlots = 4;                   // graphs a lane looks at
 constexpr int kOrderMaxGraphs = kOrderSlots * kOrderBlock;
-constexpr int kOrderRec = 8;                     // ints per record (five used; 32-byte records)
 inline bool graphs_ordered(int B) { return B > kOrderMinGraphs && B <= kOrderMaxGraphs; }
 
 __global__ __launch_bounds__(kOrderBlock) void graph_order_kernel(int B, int n16max, const int* __restrict__ a_row_ptr,
@@ -186,57 +186,11 @@ __global__ __launch_bounds__(kOrderBlock) void graph_order_kernel(int B, int n16
 // and the levels at the cost of one graph (the kernel's time is per workgroup: start-up, staging, a barrier
 // per stage, and matrix tiles that a 30-node graph leaves three quarters empty), and only the readout runs per
 // graph (a wavefront each).  1,024 graphs of the 10..110-node distribution: 59 -> 45 us.
-// The kernel below cuts the batch into such runs ("bins").  Every 64 consecutive graphs (a segment) are packed on their
-// own by one wavefront (first fit in batch order; a bin never crosses such a boundary, which costs about one
-// partly filled bin per segment): a ballot per bin gives a 64-bit word in which the graphs that open one are set, and the lanes
-// of those graphs write the segment's records, from record 64 x segment on.  The forward kernel finds bin b by a prefix sum over the set
-// bits of the words, one of them per lane, so the segments need not know of each other: a wavefront each and three trips to
-// memory, 4.7 us for 3,001 graphs.  (One workgroup that packed the whole batch, to number the bins itself, took 8.5.  Without
-// this launch, a workgroup of the forward kernel either packs all segments, which costs it more than this launch from
-// some 500 bins on, or numbers bins by its own segment, which spreads them unevenly over the dies: 1,500 graphs at hidden 64 72
-// us where bins numbered through the batch take 45.)  A graph of more than cap nodes is a bin of its own (the forward kernel
-// refuses it).  Output: words[segment], then one record of kOrderRec ints per bin: first graph, first node, nodes, first entry, end of
-// entries, graphs.
+// (graph_bins.h cuts the batch into such bins.)
 constexpr int kPackNodes = 128;                  // eight tiles: with four column blocks, two tasks for each of 16 wavefronts
 constexpr int kPackMaxNodes = 208;
 constexpr int kPackMinGraphs = 2 * kNumCU;       // below this the graphs taken one by one, largest first, are as fast
 constexpr int kPackMaxGraphs = 1 << 19;
-constexpr int kBinBlock = 128;
-// ints ahead of the records: the words of the segments, in whole records
-__host__ __device__ inline size_t bin_words_ints(int B) { return ((size_t)((B + kWave - 1) / kWave) * 2 + kOrderRec - 1) / kOrderRec * kOrderRec; }
-
-__global__ __launch_bounds__(kBinBlock) void graph_bins_kernel(int B, int cap, const int* __restrict__ a_row_ptr,
-                                                               const int* __restrict__ s_row_ptr, int* __restrict__ bins)
-{
-    const int lane = threadIdx.x & (kWave - 1);
-    const int seg = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kBinBlock / kWave) + threadIdx.x / kWave));
-    const int nlive = min(kWave, B - seg * kWave);
-    if (nlive <= 0) return;
-    int start = 0, end = 0;                      // first node and end of the lane's graph
-    if (lane < nlive) { start = s_row_ptr[seg * kWave + lane]; end = s_row_ptr[seg * kWave + lane + 1]; }
-    unsigned long long opens = 0;
-    int first = 0;
-    while (first < nlive) {
-        const int node0 = __builtin_amdgcn_readlane(start, first);
-        opens |= 1ull << first;
-        // lanes from `first` on whose graph no longer fits behind node0: the bin ends before the first of them
-        const unsigned long long stop = __ballot(lane >= first && (lane >= nlive || end - node0 > cap));
-        int next = stop ? (int)__builtin_ctzll(stop) : kWave;
-        if (next == first) next = first + 1;                         // larger than cap: alone
-        first = __builtin_amdgcn_readfirstlane(next);
-    }
-    if (lane == 0) reinterpret_cast<unsigned long long*>(bins)[seg] = opens;
-    // a lane whose graph opens a bin writes its record (a bin the forward kernel will refuse gets no entry range)
-    const unsigned long long behind = lane == kWave - 1 ? 0 : opens >> (lane + 1);
-    const int ng = (behind ? lane + 1 + (int)__builtin_ctzll(behind) : nlive) - lane;
-    const int n = __shfl(end, min(max(lane + ng - 1, 0), kWave - 1), kWave) - start;
-    if (!((opens >> lane) & 1ull)) return;
-    int e0 = 0, e1 = 0;
-    if (n >= 0 && n <= cap) { e0 = a_row_ptr[start]; e1 = a_row_ptr[start + n]; }
-    int* rec = bins + bin_words_ints(B) + (size_t)(seg * kWave + __popcll(opens & ((1ull << lane) - 1ull))) * kOrderRec;
-    *reinterpret_cast<int4*>(rec) = make_int4(seg * kWave + lane, start, n, e0);
-    *reinterpret_cast<int2*>(rec + 4) = make_int2(e1, ng);
-}
 
 // Whether the registers let two workgroups share a compute unit: four wavefronts always, eight with up to 128 registers per lane.
 template <int C, int WAVES, bool KEEP> constexpr bool two_per_cu() { return WAVES == 4 || (WAVES == 8 && C <= 32 && !KEEP); }
@@ -314,32 +268,14 @@ __global__ __launch_bounds__(WAVES * kWave, (min_waves<C, KSX, WAVES, KEEP, PACK
     // The position of the first graph (node range, then entry range) is asked for ahead of the weight
     // loads, so the two dependent trips to memory run under them instead of after them.
     int next_g = blockIdx.x, next_node0 = 0, next_n = 0, next_e0 = 0, next_e1 = 0, next_ng = 1;
-    // PACK: the place of the record of a bin, or -1 past the last one.  A workgroup asks for its bins in ascending order and goes on
-    // from the words that held the last one (from the first word for every bin: 500,000 graphs of 1 to 3 nodes, hidden 16 950 us, 709 so;
-    // 60,000 145, 141).
-    const int nseg = (B + kWave - 1) / kWave;
-    int find_seg = 0, find_before = 0;           // 64 words from find_seg on, bins of the words before them
-    auto find_bin = [&](int bin) {
-        const unsigned long long* words = reinterpret_cast<const unsigned long long*>(order);
-        const int lane = tid0 & (kWave - 1);
-        for (; find_seg < nseg; find_seg += kWave) {
-            const int count = find_seg + lane < nseg ? __popcll(words[find_seg + lane]) : 0;
-            const int through = find_before + wave_inclusive_scan_i(count);
-            const unsigned long long behind = __ballot(bin < through);
-            if (behind) {
-                const int at = (int)__builtin_ctzll(behind);
-                return (find_seg + at) * kWave + bin - __builtin_amdgcn_readlane(through - count, at);
-            }
-            find_before = __builtin_amdgcn_readlane(through, kWave - 1);
-        }
-        return -1;
-    };
+    // PACK: the places of the bins' records
+    BinFinder bins(B, order);
     const int* recs = PACK ? order + bin_words_ints(B) : order;
     // (the grid has no more workgroups than graphs: the test is for the compiler, which places the loads of the start better behind it,
     // 0.5 to 1 % of a forward over 50 to 400 graphs)
     if (PACK || (int)blockIdx.x < B) {
         if (order) {
-            const int at = PACK ? find_bin((int)blockIdx.x) : (int)blockIdx.x;
+            const int at = PACK ? bins.find((int)blockIdx.x) : (int)blockIdx.x;
             if (PACK && at < 0) return;
             const int4 r0 = *reinterpret_cast<const int4*>(recs + (size_t)at * kOrderRec);
             next_g = r0.x; next_node0 = r0.y; next_n = r0.z; next_e0 = r0.w;
@@ -407,7 +343,7 @@ __global__ __launch_bounds__(WAVES * kWave, (min_waves<C, KSX, WAVES, KEEP, PACK
         if (first) {
             g = next_g; node0 = next_node0; n = next_n; ng = next_ng;
         } else if (order) {
-            const int at = PACK ? find_bin(slot) : slot;
+            const int at = PACK ? bins.find(slot) : slot;
             if (PACK && at < 0) return;
             const int4 r0 = *reinterpret_cast<const int4*>(recs + (size_t)at * kOrderRec);
             g = r0.x; node0 = r0.y; n = r0.z; rec_e0 = r0.w;
@@ -944,9 +880,10 @@ int launch_graph_forward(int B, int K, int H, int Q, int L, int n16max,
         if (most > B) most = B;
         if (most < grid) grid = (int)most;
         void* p = nullptr;
-        if (int rc = stream_scratch(s, sizeof(int) * (bin_words_ints(B) + kOrderRec * (size_t)((B + kWave - 1) / kWave * kWave)), &p)) return rc;
+        if (int rc = stream_scratch(s, sizeof(int) * bin_ints(B), &p)) return rc;
         order = static_cast<int*>(p);
-        hipLaunchKernelGGL(graph_bins_kernel, dim3(ceil_div_u((size_t)B, kBinBlock)), dim3(kBinBlock), 0, s, B, n16max, a_row_ptr, s_row_ptr, order);
+        hipLaunchKernelGGL((graph_bins_kernel<false>), dim3(ceil_div_u((size_t)B, kBinBlock)), dim3(kBinBlock), 0, s, B, n16max, a_row_ptr, s_row_ptr, order, 0,
+                           (int*)nullptr);
         GNNHIP_LAUNCH_CHECK("graph_bins");
     } else if (graphs_ordered(B) && n16max / 16 + 2 <= 64) {
         void* p = nullptr;

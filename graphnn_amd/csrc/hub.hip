@@ -64,8 +64,10 @@ __device__ __forceinline__ int last_at_most(const int* v, int n, int x)
 // (list_chunk), both from the run's first row on, and the numbers of its hubs and of their chunks.
 __global__ __launch_bounds__(kBlock) void hub_count_kernel(int m, int rows, const int* __restrict__ row_ptr, int* __restrict__ run_hubs,
                                                            int* __restrict__ run_chunks, int* __restrict__ list_row,
-                                                           int* __restrict__ list_chunk, int threshold, int shift)
+                                                           int* __restrict__ list_chunk, int threshold, int shift,
+                                                           const int* __restrict__ gate)
 {
+    if (gated_off(gate)) return;
     __shared__ int sh[2][kWavesPerBlock];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const long long lo = (long long)blockIdx.x * rows, hi = min(lo + rows, (long long)m);
@@ -114,8 +116,9 @@ template <class V, int ITERS>
 __global__ __launch_bounds__(kBlock) void hub_partial_kernel(
     int run_rows, int runs, const int* __restrict__ run_hubs, const int* __restrict__ run_chunks, const int* __restrict__ list_row,
     const int* __restrict__ list_chunk, int chunk_cap, int n, const int* __restrict__ row_ptr, const int* __restrict__ col_idx, const float* __restrict__ val, const float* __restrict__ B, int ldb, int logG,
-    int* __restrict__ row_chunk, float* __restrict__ part, int ldp, int relu_in, int threshold, int shift)
+    int* __restrict__ row_chunk, float* __restrict__ part, int ldp, int relu_in, int threshold, int shift, const int* __restrict__ gate)
 {
+    if (gated_off(gate)) return;
     // relu_in: the rows of B are used as ReLU(B) (a first level that reads msg in place of h0)
     __shared__ float red[kWavesPerBlock][kWave * V::kVec * ITERS];
     __shared__ int before[kMaxRuns + 1];         // chunks ahead of a run
@@ -258,7 +261,7 @@ HubLayout hub_layout(int m, int n, long long nnz, int threshold, int chunk_len, 
 
 template <class V, int ITERS>
 void launch_partial(hipStream_t s, const HubLayout& L, char* base, int n, const int* row_ptr, const int* col_idx, const float* val,
-                    const float* B, int ldb, int logG, int relu_in, int threshold, int shift)
+                    const float* B, int ldb, int logG, int relu_in, int threshold, int shift, const int* gate)
 {
     // a wavefront per chunk the matrix can have, up to eight workgroups per compute unit
     long long grid = ((long long)L.chunk_cap + kWavesPerBlock - 1) / kWavesPerBlock;
@@ -266,7 +269,7 @@ void launch_partial(hipStream_t s, const HubLayout& L, char* base, int n, const 
     auto ints = [base](size_t o) { return reinterpret_cast<int*>(base + o); };
     hipLaunchKernelGGL((hub_partial_kernel<V, ITERS>), dim3((unsigned)grid), dim3(kBlock), 0, s, L.run_rows, L.runs, ints(L.o_hubs),
                        ints(L.o_chunks), ints(L.o_lrow), ints(L.o_lchunk), L.chunk_cap, n, row_ptr, col_idx, val, B, ldb, logG,
-                       ints(L.o_row), reinterpret_cast<float*>(base + L.o_part), L.ldp, relu_in, threshold, shift);
+                       ints(L.o_row), reinterpret_cast<float*>(base + L.o_part), L.ldp, relu_in, threshold, shift, gate);
 }
 
 inline bool hub_pass_applies(int m, int n, long long nnz, int threshold) { return !(m < kHubMinRows || nnz <= threshold || n > kWave * 16); }
@@ -290,7 +293,7 @@ size_t hub_scratch_bytes(int m, int n, long long nnz, int threshold, int chunk_l
 // this stream with the same arguments (the levels of one forward); the counting launch is then skipped.
 int hub_prepass(int m, int n, long long nnz, const int* row_ptr, const int* col_idx, const float* val,
                 const float* B, int ldb, hipStream_t s, HubPlan* plan, bool reuse_plan, bool relu_in, int threshold, int chunk_len,
-                long long max_hubs, HubStore* store)
+                long long max_hubs, HubStore* store, const int* gate)
 {
     *plan = HubPlan{};
     if (!hub_pass_applies(m, n, nnz, threshold)) return GNNHIP_OK;
@@ -340,19 +343,19 @@ int hub_prepass(int m, int n, long long nnz, const int* row_ptr, const int* col_
     if (!planned) {
         hipLaunchKernelGGL(hub_count_kernel, dim3((unsigned)L.runs), dim3(kBlock), 0, s, m, L.run_rows, row_ptr,
                            reinterpret_cast<int*>(b + L.o_hubs), reinterpret_cast<int*>(b + L.o_chunks), reinterpret_cast<int*>(b + L.o_lrow),
-                           reinterpret_cast<int*>(b + L.o_lchunk), threshold, shift);
+                           reinterpret_cast<int*>(b + L.o_lchunk), threshold, shift, store ? nullptr : gate);    // a kept plan is made either way
         if (store) store->planned = true;
     }
     if (n < 4) {
-        launch_partial<ColsOne, 1>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift);
+        launch_partial<ColsOne, 1>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift, gate);
     } else if (vec4) {
-        if (iters <= 1) launch_partial<ColsWide, 1>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift);
-        else if (iters == 2) launch_partial<ColsWide, 2>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift);
-        else launch_partial<ColsWide, 4>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift);
+        if (iters <= 1) launch_partial<ColsWide, 1>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift, gate);
+        else if (iters == 2) launch_partial<ColsWide, 2>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift, gate);
+        else launch_partial<ColsWide, 4>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift, gate);
     } else {
-        if (iters <= 1) launch_partial<ColsLoose, 1>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift);
-        else if (iters == 2) launch_partial<ColsLoose, 2>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift);
-        else launch_partial<ColsLoose, 4>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift);
+        if (iters <= 1) launch_partial<ColsLoose, 1>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift, gate);
+        else if (iters == 2) launch_partial<ColsLoose, 2>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift, gate);
+        else launch_partial<ColsLoose, 4>(s, L, b, n, row_ptr, col_idx, val, B, ldb, logG, relu_in ? 1 : 0, threshold, shift, gate);
     }
     GNNHIP_LAUNCH_CHECK("hub_prepass");
     *plan = HubPlan{reinterpret_cast<int*>(b + L.o_row), reinterpret_cast<float*>(b + L.o_part), L.ldp, shift};

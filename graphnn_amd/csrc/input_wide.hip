@@ -25,8 +25,9 @@ constexpr int kTileRows = 64;
 template <int C, int KS>
 __global__ __launch_bounds__(kBlock) void s2v_input_wide_kernel(
     int N, int K, unsigned k_magic, int x_vec, const float* __restrict__ X, const float* __restrict__ Wn2l,
-    float* __restrict__ msg, float* __restrict__ h0)
+    float* __restrict__ msg, float* __restrict__ h0, const int* __restrict__ gate)
 {
+    if (gated_off(gate)) return;
     constexpr int CW = C / kWaves;           // output columns per wavefront
     constexpr int NB = CW / 16;              // 16-column blocks per wavefront
     constexpr int LDT = 4 * KS + 4;          // LDS row stride
@@ -140,36 +141,36 @@ __global__ __launch_bounds__(kBlock) void s2v_input_wide_kernel(
 }
 
 template <int C, int KS>
-int launch_input_wide(int N, int K, const float* X, const float* Wn2l, float* msg, float* h0, hipStream_t s)
+int launch_input_wide(int N, int K, const float* X, const float* Wn2l, float* msg, float* h0, hipStream_t s, const int* gate)
 {
     const long long ntiles = ((long long)N + kTileRows - 1) / kTileRows;
     const long long cap = (long long)kNumCU * 4;
     const unsigned grid = (unsigned)(ntiles < cap ? ntiles : cap);
     const unsigned k_magic = K >= 2 ? (unsigned)((0x100000000ull + (unsigned)K - 1) / (unsigned)K) : 0u;   // ceil(2^32 / K)
     const int x_vec = aligned16(X) ? 1 : 0;
-    hipLaunchKernelGGL((s2v_input_wide_kernel<C, KS>), dim3(grid), dim3(kBlock), 0, s, N, K, k_magic, x_vec, X, Wn2l, msg, h0);
+    hipLaunchKernelGGL((s2v_input_wide_kernel<C, KS>), dim3(grid), dim3(kBlock), 0, s, N, K, k_magic, x_vec, X, Wn2l, msg, h0, gate);
     GNNHIP_LAUNCH_CHECK("s2v_input_wide");
     return GNNHIP_OK;
 }
 
 template <int C>
-int input_wide_c(int N, int K, const float* X, const float* Wn2l, float* msg, float* h0, hipStream_t s)
+int input_wide_c(int N, int K, const float* X, const float* Wn2l, float* msg, float* h0, hipStream_t s, const int* gate)
 {
-    if (K <= 16) return launch_input_wide<C, 4>(N, K, X, Wn2l, msg, h0, s);
-    if (K <= 32) return launch_input_wide<C, 8>(N, K, X, Wn2l, msg, h0, s);
-    if (K <= 48) return launch_input_wide<C, 12>(N, K, X, Wn2l, msg, h0, s);
-    return launch_input_wide<C, 16>(N, K, X, Wn2l, msg, h0, s);
+    if (K <= 16) return launch_input_wide<C, 4>(N, K, X, Wn2l, msg, h0, s, gate);
+    if (K <= 32) return launch_input_wide<C, 8>(N, K, X, Wn2l, msg, h0, s, gate);
+    if (K <= 48) return launch_input_wide<C, 12>(N, K, X, Wn2l, msg, h0, s, gate);
+    return launch_input_wide<C, 16>(N, K, X, Wn2l, msg, h0, s, gate);
 }
 
 }  // namespace
 
-int input_wide_dispatch(int N, int K, int C, const float* X, const float* Wn2l, float* msg, float* h0, hipStream_t s)
+int input_wide_dispatch(int N, int K, int C, const float* X, const float* Wn2l, float* msg, float* h0, hipStream_t s, const int* gate)
 {
     if (K > 64 || !(aligned16(msg) && aligned16(h0))) return GNNHIP_EUNSUPPORTED;
     switch (C) {
-    case 64: return input_wide_c<64>(N, K, X, Wn2l, msg, h0, s);
-    case 128: return input_wide_c<128>(N, K, X, Wn2l, msg, h0, s);
-    case 256: return input_wide_c<256>(N, K, X, Wn2l, msg, h0, s);
+    case 64: return input_wide_c<64>(N, K, X, Wn2l, msg, h0, s, gate);
+    case 128: return input_wide_c<128>(N, K, X, Wn2l, msg, h0, s, gate);
+    case 256: return input_wide_c<256>(N, K, X, Wn2l, msg, h0, s, gate);
     }
     return GNNHIP_EUNSUPPORTED;
 }

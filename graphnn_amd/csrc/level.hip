@@ -32,7 +32,7 @@ namespace gnnhip {
 // level_stream.hip
 int level_stream_dispatch(int N, int C, bool dense, const int* row_ptr, const int* col_idx, const float* val,
                           const float* h_in, const float* W, const float* msg, const float* bias, float* h_out,
-                          const HubPlan& hubs, bool relu_in, hipStream_t s);
+                          const HubPlan& hubs, bool relu_in, hipStream_t s, const int* gate = nullptr);
 bool level_stream_covers(int N, int C);
 // level_tile.hip
 int level_tile_dispatch(int N, int C, const int* row_ptr, const int* col_idx, const float* val, const float* h_in, const float* W,
@@ -45,7 +45,7 @@ int level_stream_backward_dispatch(int N, int C, const int* row_ptr, const int* 
 int level_stream_pieces_dispatch(int N, int C, const float* W, const float* msg, const float* bias, float* h_out, const PieceSums& sums,
                                  hipStream_t s);
 // input_wide.hip
-int input_wide_dispatch(int N, int K, int C, const float* X, const float* Wn2l, float* msg, float* h0, hipStream_t s);
+int input_wide_dispatch(int N, int K, int C, const float* X, const float* Wn2l, float* msg, float* h0, hipStream_t s, const int* gate);
 // level_wide.hip
 int level_wide_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val,
                         const float* h_in, const float* W, const float* msg, const float* bias, float* h_out, bool relu_in,
@@ -125,8 +125,9 @@ __device__ __forceinline__ void tile_times_w(const float* tile, int ldt, int kdi
 template <int C, int RT>
 __global__ __launch_bounds__(kBlock) void s2v_input_kernel(
     int N, int K, const float* __restrict__ X, const float* __restrict__ Wn2l,
-    float* __restrict__ msg, float* __restrict__ h0)
+    float* __restrict__ msg, float* __restrict__ h0, const int* __restrict__ gate)
 {
+    if (gated_off(gate)) return;
     constexpr int G = C / 4, P = kBlock / G, R = RT * P;
     extern __shared__ float smem[];
     const int ldt = ((K + 3) & ~3) + 4;              // padded row stride of the X tile, multiple of 4
@@ -434,7 +435,7 @@ __global__ __launch_bounds__(kBlock) void s2v_level_kernel(
 inline long long two_step_degree() { return (long long)kTwoStepMeanDegree; }
 
 template <int C, int RT>
-int launch_input(int N, int K, const float* X, const float* Wn2l, float* msg, float* h0, hipStream_t s)
+int launch_input(int N, int K, const float* X, const float* Wn2l, float* msg, float* h0, hipStream_t s, const int* gate)
 {
     constexpr int R = RT * (kBlock / (C / 4));
     const int ldt = ((K + 3) & ~3) + 4;
@@ -442,7 +443,7 @@ int launch_input(int N, int K, const float* X, const float* Wn2l, float* msg, fl
     if (smem > 64 * 1024) return GNNHIP_EUNSUPPORTED;
     const int ntiles = (N + R - 1) / R;
     const int grid = ntiles < kNumCU * 4 ? ntiles : kNumCU * 4;
-    hipLaunchKernelGGL((s2v_input_kernel<C, RT>), dim3(grid), dim3(kBlock), smem, s, N, K, X, Wn2l, msg, h0);
+    hipLaunchKernelGGL((s2v_input_kernel<C, RT>), dim3(grid), dim3(kBlock), smem, s, N, K, X, Wn2l, msg, h0, gate);
     GNNHIP_LAUNCH_CHECK("s2v_input");
     return GNNHIP_OK;
 }
@@ -469,21 +470,21 @@ inline bool small_batch(int N) { return N <= 32 * 1024; }
 // Return GNNHIP_EUNSUPPORTED (without setting an error text) when the shape has no fused kernel.
 bool fused_hidden_supported(int C) { return C == 16 || C == 32 || C == 64 || C == 128 || C == 256; }
 
-int input_dispatch(int N, int K, int C, const float* X, const float* Wn2l, float* msg, float* h0, hipStream_t s)
+int input_dispatch(int N, int K, int C, const float* X, const float* Wn2l, float* msg, float* h0, hipStream_t s, const int* gate)
 {
     if (!(aligned16(Wn2l) && aligned16(msg) && aligned16(h0))) return GNNHIP_EUNSUPPORTED;      // h0 may be null
     const bool small = small_batch(N);
     switch (C) {
-    case 16: return small ? launch_input<16, 1>(N, K, X, Wn2l, msg, h0, s) : launch_input<16, 4>(N, K, X, Wn2l, msg, h0, s);
-    case 32: return small ? launch_input<32, 1>(N, K, X, Wn2l, msg, h0, s) : launch_input<32, 4>(N, K, X, Wn2l, msg, h0, s);
+    case 16: return small ? launch_input<16, 1>(N, K, X, Wn2l, msg, h0, s, gate) : launch_input<16, 4>(N, K, X, Wn2l, msg, h0, s, gate);
+    case 32: return small ? launch_input<32, 1>(N, K, X, Wn2l, msg, h0, s, gate) : launch_input<32, 4>(N, K, X, Wn2l, msg, h0, s, gate);
     case 64:
         // msg alone (the forward that does not store h0): the matrix-core kernel of the wide sizes is faster
         // (880,690 nodes, 38 label types: 77 against 109 us); with h0 its 64-byte pieces per row and
         // wavefront cost more than they gain (158 against 144 us)
-        if (!h0 && K <= 64) return input_wide_dispatch(N, K, C, X, Wn2l, msg, h0, s);
-        return small ? launch_input<64, 1>(N, K, X, Wn2l, msg, h0, s) : launch_input<64, 4>(N, K, X, Wn2l, msg, h0, s);
+        if (!h0 && K <= 64) return input_wide_dispatch(N, K, C, X, Wn2l, msg, h0, s, gate);
+        return small ? launch_input<64, 1>(N, K, X, Wn2l, msg, h0, s, gate) : launch_input<64, 4>(N, K, X, Wn2l, msg, h0, s, gate);
     case 128:
-    case 256: return input_wide_dispatch(N, K, C, X, Wn2l, msg, h0, s);
+    case 256: return input_wide_dispatch(N, K, C, X, Wn2l, msg, h0, s, gate);
     }
     return GNNHIP_EUNSUPPORTED;
 }
@@ -507,12 +508,13 @@ __global__ __launch_bounds__(kBlock) void identity_csr_kernel(int n, int* __rest
 
 int level_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* h_in,
                    const float* W, const float* msg, const float* bias, float* h_out, hipStream_t s, bool same_graph,
-                   bool relu_in, CsrPlan* plan, bool inference)
+                   bool relu_in, CsrPlan* plan, bool inference, const int* gate)
 {
     // inference: no gradient passes through the result, so its contraction may be rounded differently from the
     // contraction whose signs a backward pass relies on (level_wide_split.hip)
     // plan: made by gnnhip_csr_plan_create for exactly these CSR arrays (then nnz is the matrix's own count), or null
     // relu_in: h_in is read as ReLU(h_in); only where level_accepts_relu_input says so
+    // gate: for the sizes that batch_levels_dispatch takes, else null
     // same_graph: the previous call on this stream had the same A (a later level of one forward), so the
     // plan of the long-row pass is still in place and only its sums are redone
     if (!(aligned16(h_in) && aligned16(W) && aligned16(h_out) && (!msg || aligned16(msg)) && (!bias || aligned16(bias))))
@@ -548,10 +550,10 @@ int level_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* c
         if (level_by_tile(N, C, nnz)) return level_tile_dispatch(N, C, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, relu_in, s);
         HubPlan hubs{};
         if (int rc = hub_prepass(N, C, nnz, row_ptr, col_idx, val, h_in, C, s, &hubs, same_graph, relu_in, kHubThreshold, kHubChunk, -1,
-                                 plan ? &plan->row_hub : nullptr))
+                                 plan ? &plan->row_hub : nullptr, gate))
             return rc;
         // activations of 4 GiB and more keep the kernel with 64-bit addressing below
-        if (int rc = level_stream_dispatch(N, C, false, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs, relu_in, s);
+        if (int rc = level_stream_dispatch(N, C, false, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs, relu_in, s, gate);
             rc != GNNHIP_EUNSUPPORTED)
             return rc;
         switch (C) {

@@ -62,8 +62,9 @@ __global__ __launch_bounds__(kBlock, MINW) void s2v_level_stream_kernel(
     const float* __restrict__ h_in, const float* __restrict__ W, const float* __restrict__ msg,
     const float* __restrict__ bias, float* __restrict__ h_out,
     HubPlan hubs, float* __restrict__ agg_out = nullptr,
-    float* __restrict__ acc_io = nullptr, PieceSums sums = PieceSums())
+    float* __restrict__ acc_io = nullptr, PieceSums sums = PieceSums(), const int* __restrict__ gate = nullptr)
 {
+    if (gated_off(gate)) return;
     constexpr int G = C / 4;             // lanes per gathered row
     constexpr int RPR = kWave / G;       // lane groups per wavefront
     constexpr int ROUNDS = 16 / RPR;     // rows per lane group
@@ -507,7 +508,7 @@ __global__ __launch_bounds__(kBlock, MINW) void s2v_level_stream_kernel(
 template <int C, bool DENSE, bool RELU_IN, bool PIPE>
 int launch_level_stream_p(int N, const int* row_ptr, const int* col_idx, const float* val, const float* h_in,
                           const float* W, const float* msg, const float* bias, float* h_out, const HubPlan& hubs,
-                          hipStream_t s)
+                          hipStream_t s, const int* gate)
 {
     const long long ntiles = ((long long)N + 15) / 16;
     long long blocks = (ntiles + kWavesPerBlock - 1) / kWavesPerBlock;
@@ -516,7 +517,7 @@ int launch_level_stream_p(int N, const int* row_ptr, const int* col_idx, const f
     const long long resident = (long long)kNumCU * kMinW;  // a workgroup puts one wavefront on each SIMD
     if (blocks > resident) blocks = resident;              // persistent beyond this
     hipLaunchKernelGGL((s2v_level_stream_kernel<C, DENSE, kWLds, kMinW, RELU_IN, PIPE>), dim3((unsigned)blocks), dim3(kBlock), 0, s,
-                       N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs);
+                       N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs, (float*)nullptr, (float*)nullptr, PieceSums(), gate);
     GNNHIP_LAUNCH_CHECK("s2v_level_stream");
     return GNNHIP_OK;
 }
@@ -545,26 +546,26 @@ int launch_level_stream_pieces(int N, const float* W, const float* msg, const fl
 template <int C, bool DENSE, bool RELU_IN>
 int launch_level_stream(int N, const int* row_ptr, const int* col_idx, const float* val, const float* h_in,
                         const float* W, const float* msg, const float* bias, float* h_out, const HubPlan& hubs,
-                        hipStream_t s)
+                        hipStream_t s, const int* gate)
 {
     // Gathers issued a tile ahead pay once every wavefront has several tiles (116,000 nodes: 35 -> 32 us,
     // uniform random graph of 1M rows, 2 entries per row: 223 -> 205 us); with one or two tiles per
     // wavefront the longer start of that variant costs more than it gains (7,450 nodes: +1 us per level).
     if constexpr (C == 64 && !DENSE) {
         if (N >= kPipeMinRows)
-            return launch_level_stream_p<C, DENSE, RELU_IN, true>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs, s);
+            return launch_level_stream_p<C, DENSE, RELU_IN, true>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs, s, gate);
     }
-    return launch_level_stream_p<C, DENSE, RELU_IN, false>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs, s);
+    return launch_level_stream_p<C, DENSE, RELU_IN, false>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs, s, gate);
 }
 
 template <int C>
 int launch_level_stream_c(int N, bool dense, bool relu_in, const int* row_ptr, const int* col_idx, const float* val,
                           const float* h_in, const float* W, const float* msg, const float* bias, float* h_out,
-                          const HubPlan& hubs, hipStream_t s)
+                          const HubPlan& hubs, hipStream_t s, const int* gate)
 {
-    if (dense) return launch_level_stream<C, true, false>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs, s);
-    if (relu_in) return launch_level_stream<C, false, true>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs, s);
-    return launch_level_stream<C, false, false>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs, s);
+    if (dense) return launch_level_stream<C, true, false>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs, s, gate);
+    if (relu_in) return launch_level_stream<C, false, true>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs, s, gate);
+    return launch_level_stream<C, false, false>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs, s, gate);
 }
 
 template <int C>
@@ -622,13 +623,13 @@ int level_stream_pieces_dispatch(int N, int C, const float* W, const float* msg,
 // relu_in (not with dense): h_in is read as ReLU(h_in); hub sums in `hubs` must have been formed the same way.
 int level_stream_dispatch(int N, int C, bool dense, const int* row_ptr, const int* col_idx, const float* val,
                           const float* h_in, const float* W, const float* msg, const float* bias, float* h_out,
-                          const HubPlan& hubs, bool relu_in, hipStream_t s)
+                          const HubPlan& hubs, bool relu_in, hipStream_t s, const int* gate)
 {
     if (!level_stream_covers(N, C) || (dense && relu_in)) return GNNHIP_EUNSUPPORTED;
     switch (C) {
-    case 16: return launch_level_stream_c<16>(N, dense, relu_in, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs, s);
-    case 32: return launch_level_stream_c<32>(N, dense, relu_in, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs, s);
-    default: return launch_level_stream_c<64>(N, dense, relu_in, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs, s);
+    case 16: return launch_level_stream_c<16>(N, dense, relu_in, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs, s, gate);
+    case 32: return launch_level_stream_c<32>(N, dense, relu_in, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs, s, gate);
+    default: return launch_level_stream_c<64>(N, dense, relu_in, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs, s, gate);
     }
 }
 

@@ -18,13 +18,14 @@
  * Precision
  *   - operands, accumulators and results are fp32; sums may be taken in another order than the reference's.
  *   - three products run on the bf16 matrix cores, every fp32 operand as three bf16 numbers whose sum it is: the levels of
- *     gnnhip_s2v_forward_f32 / _planned_f32 and gnnhip_s2v_level_backward_f32 at hidden 128 and 256, and A^T B with an
+ *     gnnhip_s2v_forward_f32 / _planned_f32 at hidden 128 and 256, and at hidden 64 over large batches of small graphs,
+ *     gnnhip_s2v_level_backward_f32 at hidden 128 and 256, and A^T B with an
  *     output of up to 256 x 256 over 8,192 rows and more (m n k >= 2^28).  Their errors against exact sums are smaller than
  *     those of the FP32 matrix cores, over the whole range of fp32 and with infinities and NaNs carried on, with one
  *     limit: where a row of the left operand or a column of W (a column of A or B, over a run of rows) holds an element of
  *     2^38 or more, its elements below 2^-47 lose their last bits.
- *   - the level entries run on the FP32 matrix cores, so at hidden 128 and 256 a forward and the same levels called one
- *     by one agree to rounding and not to the last bit.
+ *   - the level entries run on the FP32 matrix cores, so where its levels are formed in pieces a forward and the same
+ *     levels called one by one agree to rounding and not to the last bit.
  *
  * Each declaration cites the reference interface it stands in for
  * (paths relative to the graphnn source tree).
@@ -252,6 +253,8 @@ int gnnhip_s2v_readout_f32(int B, int N, int C, int H, int Q,
  *      receives 0 if the final embedding is in h_a, 1 if in h_b (which of the two holds which level is
  *      the library's choice: with L >= 1 the first level may read ReLU(msg) straight from msg, and
  *      h0 is then never stored).  a_nnz: entries of A.
+ *      A large batch whose rows of S are ascending ranges of nodes, of at most 128 each, that cover all nodes, with no entry of A between
+ *      two of them (found out on the device), runs its levels in one launch; the other of h_a and h_b is then not written.
  *      Op sequence of examples/graph_classification/src/kernel_mean_field.cpp:31-49 scheduled by
  *      FactorGraph::SequentialForward (src/nn/factor_graph.cpp:75-144). */
 int gnnhip_s2v_forward_f32(int N, int B, int K, int C, int H, int Q, int L, int a_nnz,

@@ -2673,3 +2673,130 @@ def test_bindings_make_tensors_as_torch_does(gpu):
         assert bool(torch.isnan(ops._empty(where, "f", 1000)).all())
     finally:
         torch.use_deterministic_algorithms(False)
+
+
+def _small_graphs(gpu, sizes, mean_entries, gen, unit=False):
+    """(A, S, N): graphs of the given sizes, entries drawn inside their graph, rows of 0 to 2 mean_entries entries"""
+    import torch
+    n = torch.as_tensor(sizes, device=gpu)
+    off = torch.zeros(n.numel() + 1, dtype=torch.long, device=gpu)
+    off[1:] = torch.cumsum(n, 0)
+    N = int(off[-1])
+    graph = torch.repeat_interleave(torch.arange(n.numel(), device=gpu), n)
+    deg = torch.randint(0, 2 * mean_entries + 1, (N,), generator=gen, device=gpu)
+    rp = torch.zeros(N + 1, dtype=torch.int32, device=gpu)
+    rp[1:] = torch.cumsum(deg, 0)
+    row = torch.repeat_interleave(torch.arange(N, device=gpu), deg)
+    ci = off[graph[row]] + (torch.rand(row.numel(), generator=gen, device=gpu) * n[graph[row]]).long().minimum(n[graph[row]] - 1)
+    val = torch.ones(row.numel(), device=gpu) if unit else torch.rand(row.numel(), generator=gen, device=gpu) / max(mean_entries, 1)
+    S = (off.int(), torch.arange(N, device=gpu).int(), torch.rand(N, generator=gen, device=gpu) + 0.5)
+    return (rp, ci.int(), val), S, N
+
+
+def _forward_one_by_one(A, S, X, Wn, Wc, W1, W2, L):
+    """the same forward from the stages' own entries (a level at a time)"""
+    from graphnn_amd import ops
+    msg, h = ops.s2v_input(X, Wn)
+    for _ in range(L):
+        h = ops.s2v_level(*A, h, Wc, msg)
+    return (msg, h) + tuple(ops.s2v_readout(*S, h, W1, W2, S[0].numel() - 1))
+
+
+def _check_forward(gpu, A, S, N, K, C, L, gen, exact):
+    import torch
+    from graphnn_amd import ops
+    H, Q = 8, 3
+    B = S[0].numel() - 1
+    normal = lambda *shape: torch.randn(*shape, generator=gen, device=gpu)
+    X = torch.zeros(N, K, device=gpu)
+    X[torch.arange(N, device=gpu), torch.randint(0, K, (N,), generator=gen, device=gpu)] = 1.0
+    w = (normal(K, C), normal(C, C) * (0.8 / C ** 0.5), normal(C, H), normal(H, Q))
+    bufs = ops.ForwardBuffers(N, B, C, H, Q, gpu)
+    for name in ("msg", "h_a", "h_b", "pool", "hidden", "logits", "probs"):
+        getattr(bufs, name).fill_(float("nan"))
+    ops.s2v_forward(A, S, X, *w, L, bufs=bufs)
+    got = (bufs.msg, bufs.h_final, bufs.pool, bufs.hidden, bufs.logits, bufs.probs, bufs.pred)
+    want = _forward_one_by_one(A, S, X, *w, L)
+    assert torch.equal(got[0], want[0])                      # one-hot features: rows of the weights
+    if exact:
+        for g, e in zip(got, want):
+            assert torch.equal(g, e)
+    # float64 and the sum of the terms' magnitudes, level by level: every level adds the rounding of its two sums
+    rp, ci, val = A
+    row = torch.repeat_interleave(torch.arange(N, device=gpu), (rp[1:] - rp[:-1]).long())
+    msg = X.double() @ w[0].double()
+    h, terms = msg.clamp(min=0), msg.abs()
+    for _ in range(L):
+        zero = torch.zeros(N, C, dtype=torch.float64, device=gpu)
+        h = (zero.index_add(0, row, h[ci.long()] * val.double()[:, None]) @ w[1].double() + msg).clamp(min=0)
+        terms = zero.index_add(0, row, terms[ci.long()] * val.double()[:, None].abs()) @ w[1].double().abs() + msg.abs()
+    longest = int((rp[1:] - rp[:-1]).max()) if row.numel() else 0
+    bound = L * (longest + C + 2) * 2.0 ** -24
+    assert bool(((got[1].double() - h).abs() <= bound * terms).all())
+    pool = torch.zeros(B, C, dtype=torch.float64, device=gpu)
+    graph = torch.repeat_interleave(torch.arange(B, device=gpu), (S[0][1:] - S[0][:-1]).long(), output_size=S[1].numel())
+    pool.index_add_(0, graph, got[1].double()[S[1].long()] * S[2].double()[:, None])
+    assert bool(((got[2].double() - pool).abs() <= 4200 * 2.0 ** -24 * pool.abs() + 1e-30).all())     # no negative terms
+    assert torch.equal(got[6].long(), got[4].argmax(1))
+
+
+def _enough(n, C, L):
+    """the sizes repeated until the batch is one that the forward tries to take in one launch"""
+    need = max(32768, (12e6 if C == 16 else 4e6) / ((L - 1) * C))
+    return np.tile(np.asarray(n, np.int64), int(np.ceil(need / np.sum(n))))
+
+
+@pytest.mark.parametrize("C", [16, 32, 64])
+@pytest.mark.parametrize("sizes", ["molecules", "ones", "full", "with_empty", "dense"])
+def test_forward_over_a_large_batch_of_small_graphs(gpu, C, sizes):
+    """batches whose levels run in one launch: bins of one graph of 128 nodes, of 64 graphs of one node, graphs without nodes, bins of
+    more entries than are kept in LDS, a last tile of one row; feature columns around the steps of the input stage.  Hidden 16 and
+    32 have the bits of the stages called one by one; hidden 64 (bf16 pieces) is held to the rounding of fp32 sums"""
+    import torch
+    gen = torch.Generator(device=gpu).manual_seed(C)
+    for K, L, seed in ((2, 2, 0), (3, 4, 1), (17, 3, 2), (33, 4, 3), (64, 2, 4)):
+        rng = np.random.default_rng(100 * C + seed)
+        n = {"molecules": rng.integers(10, 111, 1100), "ones": np.ones(33_001, np.int64), "full": np.full(300, 128),
+             "with_empty": np.where(rng.random(4000) < 0.3, 0, rng.integers(1, 40, 4000)), "dense": rng.integers(90, 129, 400)}[sizes]
+        n = _enough(n, C, L)
+        if sizes == "with_empty":
+            n[640:768] = 0                                       # two segments without nodes
+            n[-1] = 0
+        A, S, N = _small_graphs(gpu, n, 11 if sizes == "dense" else 2, gen)
+        _check_forward(gpu, A, S, N, K, C, L, gen, C != 64)
+
+
+@pytest.mark.parametrize("C", [16, 32, 64])
+@pytest.mark.parametrize("kind", ["crossing", "crossing_dense", "large_graph", "uncovered", "offset", "overlapping", "long_row"])
+def test_forward_over_a_batch_that_is_none(gpu, C, kind):
+    """what the one launch must refuse on the device: one entry that leaves its bin (kept in LDS, or read from memory), a graph of 129
+    nodes, rows of S that leave out nodes, begin past node 0 or name nodes twice: every output has the bits of the stages called one
+    by one"""
+    import torch
+    gen = torch.Generator(device=gpu).manual_seed(7)
+    rng = np.random.default_rng(C)
+    n = rng.integers(90, 129, 400) if kind == "crossing_dense" else rng.integers(10, 111, 1100)
+    n = _enough(rng.permutation(n), C, 3)
+    if kind == "large_graph":
+        n[700] = 129
+    A, S, N = _small_graphs(gpu, n, 11 if kind == "crossing_dense" else 2, gen)
+    rp, ci, val = A
+    if kind.startswith("crossing"):
+        first = int(torch.nonzero(rp[1:] > rp[:-1])[-1])         # the last row with entries points to node 0
+        ci[int(rp[first])] = 0
+    elif kind == "long_row":                                     # a row of 5,000 entries that stay inside: the one launch takes it
+        first = int(S[0][3])
+        width = int(S[0][4]) - first
+        at = int(rp[first])
+        extra = first + torch.arange(5000, device=gpu) % width
+        ci = torch.cat([ci[:at], extra.int(), ci[at:]])
+        val = torch.cat([val[:at], torch.rand(5000, generator=gen, device=gpu) / 5000, val[at:]])
+        rp = rp.clone(); rp[first + 1:] += 5000
+    elif kind == "uncovered":
+        S = (S[0][:-1].contiguous(), S[1], S[2])                 # the last graph's nodes belong to none
+        S = (S[0], S[1][:int(S[0][-1])].contiguous(), S[2][:int(S[0][-1])].contiguous())
+    elif kind == "offset":
+        S = (S[0][1:] - S[0][1], S[1][int(S[0][1]):].contiguous(), S[2][int(S[0][1]):].contiguous())
+    elif kind == "overlapping":                                  # the last row names all nodes of the batch again
+        S = (torch.cat([S[0], S[0][-1:] + N]), torch.cat([S[1], S[1]]), torch.cat([S[2], S[2]]))
+    _check_forward(gpu, (rp, ci, val), S, N, 9, C, 3, gen, kind != "long_row")
