@@ -25,6 +25,14 @@
 // 1.16e-11 of the terms' magnitudes after four levels, level by level 2.42e-11.  What bounds that kernel is the issue of vector
 // instructions, about 330 per 16 rows and level (64 sum the first four entries, 104 split the rows); two wavefronts per SIMD, 247
 // registers.  What a bin reads is asked for while the last level of the bin before it ends (428 us without).
+//
+// Hidden sizes from 17 to 112 without kernels of their own take the next multiple of 16, with zeros behind the last column, and msg from
+// memory (the general input stage).  Above 64 W lies in LDS in all three pieces (86 KB at 112) and a workgroup fills a compute unit:
+// its wavefronts wait for the same things at the same time, and a level of 16 rows reads all of W.  44,000 nodes, hidden 100, 3.8
+// entries per row: a level 28 -> 16 us, the forward of three 110 -> 97; 176,000 nodes, four levels 416 -> 285; error against float64
+// 6.7e-11, was 1.4e-10.  Above 112 columns W and the rows of 128 nodes do not fit the LDS together.  Tried there: the wavefronts share
+// the columns, as in level_wide_split.hip, and the rows are put into pieces in place between two barriers: 7.5 us for a bin of 112
+// nodes and a level at hidden 128, where the level-by-level route takes as long, and at hidden 256, where 64 nodes fit, 1.5 times that.
 #include <type_traits>
 
 #include "bf16_split.h"
@@ -46,39 +54,47 @@ __device__ __forceinline__ float4 relu_one(const float4& v)
                        __builtin_elementwise_maximum(v.w, 0.f));
 }
 
-template <int C> struct BatchShape;
-// TPW: tiles of 16 rows per wavefront.  MINW: wavefronts per SIMD.  PIECES: products from bf16 pieces
-template <> struct BatchShape<16> { static constexpr int TPW = 1, MINW = 6; static constexpr bool PIECES = false; };
-template <> struct BatchShape<32> { static constexpr int TPW = 1, MINW = 4; static constexpr bool PIECES = false; };
-template <> struct BatchShape<64> { static constexpr int TPW = 2, MINW = 2; static constexpr bool PIECES = true; };
-template <int C> constexpr int batch_waves() { return kRows / 16 / BatchShape<C>::TPW; }
-
-template <int C, int KSX>
-constexpr size_t batch_lds_bytes()
+// CP: hidden size, or the next multiple of 16 that has a kernel.  TPW: tiles of 16 rows per wavefront.  MINW: wavefronts per SIMD.
+// PIECES: products from bf16 pieces; WREG: the first two pieces of W in registers, else all three in LDS
+template <int CP> struct BatchShape { static constexpr int TPW = 1, MINW = 2; static constexpr bool PIECES = true, WREG = false; };
+template <> struct BatchShape<16> { static constexpr int TPW = 1, MINW = 6; static constexpr bool PIECES = false, WREG = true; };
+template <> struct BatchShape<32> { static constexpr int TPW = 1, MINW = 4; static constexpr bool PIECES = false, WREG = true; };
+template <> struct BatchShape<48> { static constexpr int TPW = 2, MINW = 2; static constexpr bool PIECES = true, WREG = true; };
+template <> struct BatchShape<64> { static constexpr int TPW = 2, MINW = 2; static constexpr bool PIECES = true, WREG = true; };
+template <int CP> constexpr int batch_waves() { return kRows / 16 / BatchShape<CP>::TPW; }
+template <int CP> constexpr int w_lds_words()    // 128-bit words of W in LDS
 {
-    return sizeof(float) * (size_t)(kRows + 1) * (C + 4) + (BatchShape<C>::PIECES ? sizeof(float) * C + sizeof(short) * C * C : 0) +
-           sizeof(float) * (size_t)(C / 16) * KSX * kWave + sizeof(int2) * kEdgeCap + sizeof(int) * (kRows + 4);
+    return !BatchShape<CP>::PIECES ? 0 : (CP / 4 + 7) / 8 * (CP / 16) * (BatchShape<CP>::WREG ? 1 : 3) * kWave;
 }
 
-// KSX: contraction steps of the input stage, K <= 4 KSX
-template <int C, int KSX>
-__global__ __launch_bounds__(batch_waves<C>() * kWave, BatchShape<C>::MINW) void s2v_batch_levels_kernel(
-    int N, int B, int K, int L, const int* __restrict__ a_row_ptr, const int* __restrict__ a_col_idx, const float* __restrict__ a_val,
+template <int CP, int KSX>
+constexpr size_t batch_lds_bytes()
+{
+    return sizeof(float) * (size_t)(kRows + 1) * (CP + 4) + sizeof(bf16_words4) * w_lds_words<CP>() + (BatchShape<CP>::PIECES ? sizeof(float) * CP : 0) +
+           sizeof(float) * (size_t)(CP / 16) * KSX * kWave + sizeof(int2) * kEdgeCap + sizeof(int) * (kRows + 4);
+}
+
+// KSX: contraction steps of the input stage, K <= 4 KSX, and the hidden size is CP; 0: msg is there, and the hidden size is C <= CP
+template <int CP, int KSX>
+__global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) void s2v_batch_levels_kernel(
+    int N, int B, int K, int hidden, int L, const int* __restrict__ a_row_ptr, const int* __restrict__ a_col_idx, const float* __restrict__ a_val,
     const float* __restrict__ X, const float* __restrict__ Wn2l, const float* __restrict__ Wc, float* __restrict__ msg,
     float* __restrict__ h_out, const int* __restrict__ bins, int* __restrict__ refused)
 {
-    constexpr int TPW = BatchShape<C>::TPW, kWaves = batch_waves<C>(), kBlock = kWaves * kWave;
-    constexpr bool PIECES = BatchShape<C>::PIECES;
-    constexpr int KS = C / 4;                    // columns of a lane, contraction steps of a level
-    constexpr int KS2 = C / 32;                  // contraction steps of a level in pieces
-    constexpr int NJB = C / 16;                  // output blocks of 16 columns
-    constexpr int LD = C + 4;
-    static_assert(!PIECES || KS2 == 2, "two sums of opposite signs");
+    using Shape = BatchShape<CP>;
+    constexpr int TPW = Shape::TPW, kWaves = batch_waves<CP>(), kBlock = kWaves * kWave;
+    constexpr bool PIECES = Shape::PIECES, WREG = Shape::WREG, INPUT = KSX > 0;
+    constexpr int KS = CP / 4;                   // columns of a lane, contraction steps of a level
+    constexpr int KS2 = (KS + 7) / 8;            // contraction steps of a level in pieces
+    constexpr int NJB = CP / 16;                 // output blocks of 16 columns
+    constexpr int LD = CP + 4;
+    const int C = INPUT ? CP : hidden;
+    static_assert(!PIECES || !WREG || KS2 == 2, "two sums of opposite signs");
     extern __shared__ float4 smem4[];
     float* hbuf = reinterpret_cast<float*>(smem4);                         // [kRows + 1][LD], the last row zeros
-    bf16_words4* w3 = reinterpret_cast<bf16_words4*>(hbuf + (kRows + 1) * LD);             // third pieces of W, [KS2][NJB][lane]
-    float* w_down = reinterpret_cast<float*>(w3 + (PIECES ? KS2 * NJB * kWave : 0));       // [C] a column's scale up over its scale
-    float2* wn = reinterpret_cast<float2*>(w_down + (PIECES ? C : 0));     // [NJB][KSX / 2][lane]
+    bf16_words4* w_lds = reinterpret_cast<bf16_words4*>(hbuf + (kRows + 1) * LD);          // W in pieces, [KS2][NJB][3][lane], or the third ones
+    float* w_down = reinterpret_cast<float*>(w_lds + w_lds_words<CP>());   // [CP] a column's scale up over its scale
+    float2* wn = reinterpret_cast<float2*>(w_down + (PIECES ? CP : 0));    // [NJB][KSX / 2][lane]
     int2* edges = reinterpret_cast<int2*>(wn + NJB * (KSX / 2) * kWave);   // [kEdgeCap] row offset, weight
     int* rp = reinterpret_cast<int*>(edges + kEdgeCap);                    // [kRows + 1], from the bin's first entry on
     __shared__ int stop;                         // another workgroup has come upon an entry that leaves its bin
@@ -93,17 +109,24 @@ __global__ __launch_bounds__(batch_waves<C>() * kWave, BatchShape<C>::MINW) void
     BinFinder finder(B, bins);
     int at = finder.find_checked((int)blockIdx.x);
 
-    // W as the operand of the matrix instructions.  fp32: wf[jb][s] = W[KS q + s][out_col + 4 jb]; in pieces: of W[KS q + 8 s + 0..7],
-    // the third ones in LDS, the second step's negated
+    // W as the operand of the matrix instructions, zeros past its last row and column.  fp32: wf[jb][s] = W[KS q + s][out_col + 4 jb]; in
+    // pieces: of W[KS q + 8 s + 0..7].  The matrix instructions on bf16 round towards minus infinity: in registers, the second step is
+    // negated and summed apart, so that the drifts cancel; in LDS, every other block of columns is negated, so that there is no drift
+    // from level to level.
     float wf[PIECES ? 1 : NJB][PIECES ? 1 : KS];
-    bf16_words4 wp[PIECES ? KS2 : 1][PIECES ? NJB : 1][2];
+    bf16_words4 wp[PIECES && WREG ? KS2 : 1][PIECES && WREG ? NJB : 1][2];
     bool any_down = false;                       // a column of W is scaled down (bf16_split.h): uniform
+    auto w_at = [&](int k, int jb) {             // k: of the lane's
+        const int row = KS * q + k, col = out_col + 4 * jb;
+        return INPUT || (row < C && col < C) ? Wc[(size_t)row * C + col] : 0.f;
+    };
     if constexpr (PIECES) {
 #pragma unroll
         for (int jb = 0; jb < NJB; ++jb) {
-            float w[KS], largest = 0.f;
+            if (!WREG && jb % kWaves != wave) continue;                    // uniform
+            float w[8 * KS2], largest = 0.f;
 #pragma unroll
-            for (int k = 0; k < KS; ++k) w[k] = Wc[(size_t)(KS * q + k) * C + out_col + 4 * jb];
+            for (int k = 0; k < 8 * KS2; ++k) w[k] = k < KS ? w_at(k, jb) : 0.f;
 #pragma unroll
             for (int k = 0; k < KS; k += 2) largest = split_max(largest, w[k], w[k + 1]);
             const unsigned long long large = __ballot(largest >= kSplitLarge);
@@ -113,31 +136,40 @@ __global__ __launch_bounds__(batch_waves<C>() * kWave, BatchShape<C>::MINW) void
             if (q == 0) w_down[out_col + 4 * jb] = down ? kSplitUp / kSplitDown : 1.f;
 #pragma unroll
             for (int s = 0; s < KS2; ++s) {
-                bf16_words4 third;
+                bf16_words4 w3[3];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     unsigned p[3];
                     bf16_split2(w[8 * s + 2 * i] * scale, w[8 * s + 2 * i + 1] * scale, down, p);
-                    const unsigned sign = s == 1 ? 0x80008000u : 0u;
-                    wp[s][jb][0][i] = p[0] ^ sign; wp[s][jb][1][i] = p[1] ^ sign; third[i] = p[2] ^ sign;
+                    const unsigned sign = (WREG ? s : jb) % 2 ? 0x80008000u : 0u;
+#pragma unroll
+                    for (int j = 0; j < 3; ++j) w3[j][i] = p[j] ^ sign;
                 }
-                if (wave == 0) w3[(s * NJB + jb) * kWave + lane] = third;
+                if constexpr (WREG) {
+                    wp[s][jb][0] = w3[0]; wp[s][jb][1] = w3[1];
+                    if (wave == 0) w_lds[(s * NJB + jb) * kWave + lane] = w3[2];
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 3; ++j) w_lds[((s * NJB + jb) * 3 + j) * kWave + lane] = w3[j];
+                }
             }
         }
     } else {
 #pragma unroll
         for (int jb = 0; jb < NJB; ++jb)
 #pragma unroll
-            for (int s = 0; s < KS; ++s) wf[jb][s] = Wc[(size_t)(KS * q + s) * C + out_col + 4 * jb];
+            for (int s = 0; s < KS; ++s) wf[jb][s] = w_at(s, jb);
     }
-    for (int i = wave; i < NJB * (KSX / 2); i += kWaves) {
-        const int jb = i / (KSX / 2), k = 8 * (i % (KSX / 2)) + 2 * q;
-        wn[i * kWave + lane] = make_float2(k < K ? Wn2l[(size_t)k * C + out_col + 4 * jb] : 0.f,
-                                           k + 1 < K ? Wn2l[(size_t)(k + 1) * C + out_col + 4 * jb] : 0.f);
+    if constexpr (INPUT) {
+        for (int i = wave; i < NJB * (KSX / 2); i += kWaves) {
+            const int jb = i / (KSX / 2), k = 8 * (i % (KSX / 2)) + 2 * q;
+            wn[i * kWave + lane] = make_float2(k < K ? Wn2l[(size_t)k * C + out_col + 4 * jb] : 0.f,
+                                               k + 1 < K ? Wn2l[(size_t)(k + 1) * C + out_col + 4 * jb] : 0.f);
+        }
     }
     if (tid < LD) hbuf[kRows * LD + tid] = 0.f;
     if (tid == 0) stop = 0;
-    __syncthreads();
+    any_down = __syncthreads_or(any_down);
 
     // ---- what a bin needs from memory, asked for together and a bin ahead
     struct Bin { int node0, n, e0, ne; };
@@ -147,13 +179,30 @@ __global__ __launch_bounds__(batch_waves<C>() * kWave, BatchShape<C>::MINW) void
         return at < 0 ? Bin{0, 0, 0, 0} : Bin{r.y, r.z, r.w, max(rec[4] - r.w, 0)};
     };
     constexpr int kEdgesEach = kEdgeCap / kBlock;
-    float x[TPW][KSX], e_val[kEdgesEach];
+    float x[TPW][INPUT ? KSX : 1], e_val[kEdgesEach];
+    float4 mx[TPW][INPUT ? 1 : NJB];             // rows of msg where they are there already
     int e_col[kEdgesEach], rp_v;
     auto ask = [&](const Bin& b) {
         // (every register is written whatever the bin is, or the old values would have to be kept through the levels)
 #pragma unroll
         for (int i = 0; i < TPW; ++i) {
-            const float* xr = X + (size_t)min(b.node0 + min(row0 + 16 * i, max(b.n - 1, 0)), N - 1) * K;
+            const size_t at_row = (size_t)min(b.node0 + min(row0 + 16 * i, max(b.n - 1, 0)), N - 1);
+            if constexpr (!INPUT) {
+                const float* mr = msg + at_row * C;
+#pragma unroll
+                for (int jb = 0; jb < NJB; ++jb) {
+                    const int col = KS * q + 4 * jb;
+                    mx[i][jb] = f4_zero();
+                    if (col + 4 <= C) {
+                        mx[i][jb] = ColsLoose::load(mr + col);
+                    } else {
+                        if (col < C) mx[i][jb].x = mr[col];
+                        if (col + 1 < C) mx[i][jb].y = mr[col + 1];
+                        if (col + 2 < C) mx[i][jb].z = mr[col + 2];
+                    }
+                }
+            }
+            const float* xr = X + at_row * K;
 #pragma unroll
             for (int s = 0; s < KSX; s += 2) {
                 if (s >= srt) { x[i][s] = x[i][s + 1] = 0.f; continue; }        // uniform
@@ -220,8 +269,10 @@ __global__ __launch_bounds__(batch_waves<C>() * kWave, BatchShape<C>::MINW) void
                 }
             }
 #pragma unroll
-            for (int jb = 0; jb < NJB; ++jb)
-                m[i][jb] = row0 + 16 * i < n ? make_float4(acc[jb][0], acc[jb][1], acc[jb][2], acc[jb][3]) : f4_zero();
+            for (int jb = 0; jb < NJB; ++jb) {
+                m[i][jb] = f4_zero();
+                if (row0 + 16 * i < n) m[i][jb] = INPUT ? make_float4(acc[jb][0], acc[jb][1], acc[jb][2], acc[jb][3]) : mx[i][INPUT ? 0 : jb];
+            }
         }
         __syncthreads();                         // the last bin's rows have left hbuf; rp and edges are there
         float* own = hbuf + row0 * LD + KS * q;
@@ -245,10 +296,28 @@ __global__ __launch_bounds__(batch_waves<C>() * kWave, BatchShape<C>::MINW) void
         __syncthreads();
         // the bin's rows as they lie in memory: whole lines
         auto copy_out = [&](float* dst) {
-            for (int i = tid; i < n * KS; i += kBlock)
-                *reinterpret_cast<float4*>(dst + (size_t)node0 * C + 4 * i) = *reinterpret_cast<const float4*>(hbuf + (i / KS) * LD + 4 * (i % KS));
+            if constexpr (INPUT) {
+                for (int i = tid; i < n * KS; i += kBlock)
+                    *reinterpret_cast<float4*>(dst + (size_t)node0 * C + 4 * i) = *reinterpret_cast<const float4*>(hbuf + (i / KS) * LD + 4 * (i % KS));
+            } else {
+                constexpr int G = KS <= 4 ? 4 : KS <= 8 ? 8 : KS <= 16 ? 16 : 32;      // lanes per row
+                const int col = 4 * (tid % G);
+                if (col < C) {
+                    for (int r = tid / G; r < n; r += kBlock / G) {
+                        const float4 v = *reinterpret_cast<const float4*>(hbuf + r * LD + col);
+                        float* d = dst + (size_t)(node0 + r) * C + col;
+                        if (col + 4 <= C) {
+                            ColsLoose::store(d, v);
+                        } else {
+                            d[0] = v.x;
+                            if (col + 1 < C) d[1] = v.y;
+                            if (col + 2 < C) d[2] = v.z;
+                        }
+                    }
+                }
+            }
         };
-        copy_out(msg);
+        if (INPUT) copy_out(msg);
         if (tid == 0) stop = __hip_atomic_load(refused, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
         auto level = [&](auto relu_in, auto last) {
@@ -271,9 +340,14 @@ __global__ __launch_bounds__(batch_waves<C>() * kWave, BatchShape<C>::MINW) void
                 if (staged) {
 #pragma unroll
                     for (int u = 0; u < kDirect; ++u) add(g_off[i][u], g_w[i][u]);
-                    for (int e = g_st[i] + kDirect; e < g_en[i]; ++e) {
-                        const int2 ed = edges[e];
-                        add(ed.x + KS * q, __int_as_float(ed.y));
+                    int e = g_st[i] + kDirect;
+                    if (e < g_en[i]) {
+                        int2 ed = edges[e];
+                        do {                     // the next entry is on its way while this one's row is added
+                            const int2 now = ed;
+                            ed = edges[min(++e, kEdgeCap - 1)];
+                            add(now.x + KS * q, __int_as_float(now.y));
+                        } while (e < g_en[i]);
                     }
                 } else {
                     for (int e = g_st[i]; e < g_en[i]; ++e) {
@@ -294,8 +368,8 @@ __global__ __launch_bounds__(batch_waves<C>() * kWave, BatchShape<C>::MINW) void
                         for (int s = 0; s < KS2; ++s)
 #pragma unroll
                             for (int u = 0; u < 4; ++u) {
-                                unsigned w[3];
-                                bf16_split2(agg[8 * s + 2 * u] * scale, agg[8 * s + 2 * u + 1] * scale, down, w);
+                                unsigned w[3] = {0, 0, 0};
+                                if (8 * s + 2 * u < KS) bf16_split2(agg[8 * s + 2 * u] * scale, agg[8 * s + 2 * u + 1] * scale, down, w);
                                 p[s][0][u] = w[0]; p[s][1][u] = w[1]; p[s][2][u] = w[2];
                             }
                     };
@@ -306,44 +380,45 @@ __global__ __launch_bounds__(batch_waves<C>() * kWave, BatchShape<C>::MINW) void
                     } else {
                         split(kSplitUp, false);
                     }
-                    // the corrections of either step first; the second step on a sum of the other sign, so that the drifts cancel
-                    mfma_f4 acc[KS2][NJB];
+                    // The corrections are summed apart from the products of the first pieces (level_wide_split.hip): in registers the second
+                    // step's sum has the other sign, and either step's corrections come first
+                    mfma_f4 acc[2][NJB];
 #pragma unroll
-                    for (int s = 0; s < KS2; ++s)
+                    for (int jb = 0; jb < NJB; ++jb) acc[0][jb] = acc[1][jb] = mfma_f4{0.f, 0.f, 0.f, 0.f};
+                    if constexpr (WREG) {
+                        auto products = [&](int w, int x) {
 #pragma unroll
-                        for (int jb = 0; jb < NJB; ++jb) acc[s][jb] = mfma_f4{0.f, 0.f, 0.f, 0.f};
+                            for (int s = 0; s < KS2; ++s)
 #pragma unroll
-                    for (int s = 0; s < KS2; ++s)
+                                for (int jb = 0; jb < NJB; ++jb)
+                                    acc[s][jb] = mfma_bf16(w == 2 ? w_lds[(s * NJB + jb) * kWave + lane] : wp[s][jb][w < 2 ? w : 0], p[s][x], acc[s][jb]);
+                        };
+                        products(2, 0); products(0, 2); products(1, 1); products(1, 0); products(0, 1); products(0, 0);
+                    } else {
 #pragma unroll
-                        for (int jb = 0; jb < NJB; ++jb) acc[s][jb] = mfma_bf16(w3[(s * NJB + jb) * kWave + lane], p[s][0], acc[s][jb]);
+                        for (int s = 0; s < KS2; ++s) {
 #pragma unroll
-                    for (int s = 0; s < KS2; ++s)
-#pragma unroll
-                        for (int jb = 0; jb < NJB; ++jb) acc[s][jb] = mfma_bf16(wp[s][jb][0], p[s][2], acc[s][jb]);
-#pragma unroll
-                    for (int s = 0; s < KS2; ++s)
-#pragma unroll
-                        for (int jb = 0; jb < NJB; ++jb) acc[s][jb] = mfma_bf16(wp[s][jb][1], p[s][1], acc[s][jb]);
-#pragma unroll
-                    for (int s = 0; s < KS2; ++s)
-#pragma unroll
-                        for (int jb = 0; jb < NJB; ++jb) acc[s][jb] = mfma_bf16(wp[s][jb][1], p[s][0], acc[s][jb]);
-#pragma unroll
-                    for (int s = 0; s < KS2; ++s)
-#pragma unroll
-                        for (int jb = 0; jb < NJB; ++jb) acc[s][jb] = mfma_bf16(wp[s][jb][0], p[s][1], acc[s][jb]);
-#pragma unroll
-                    for (int s = 0; s < KS2; ++s)
-#pragma unroll
-                        for (int jb = 0; jb < NJB; ++jb) acc[s][jb] = mfma_bf16(wp[s][jb][0], p[s][0], acc[s][jb]);
+                            for (int jb = 0; jb < NJB; ++jb) {
+                                const bf16_words4* w = w_lds + (s * NJB + jb) * 3 * kWave + lane;
+                                const bf16_words4 w0 = w[0], w1 = w[kWave], w2 = w[2 * kWave];
+                                acc[1][jb] = mfma_bf16(w2, p[s][0], acc[1][jb]);
+                                acc[0][jb] = mfma_bf16(w0, p[s][0], acc[0][jb]);
+                                acc[1][jb] = mfma_bf16(w0, p[s][2], acc[1][jb]);
+                                acc[1][jb] = mfma_bf16(w1, p[s][1], acc[1][jb]);
+                                acc[1][jb] = mfma_bf16(w1, p[s][0], acc[1][jb]);
+                                acc[1][jb] = mfma_bf16(w0, p[s][1], acc[1][jb]);
+                            }
+                        }
+                    }
 #pragma unroll
                     for (int jb = 0; jb < NJB; ++jb) {
-                        float4 f = make_float4(back, back, back, back);
+                        const float b = WREG || jb % 2 == 0 ? back : -back;
+                        float4 f = make_float4(b, b, b, b);
                         if (any_down) {
                             const float4 d = *reinterpret_cast<const float4*>(w_down + KS * q + 4 * jb);
                             f.x *= d.x; f.y *= d.y; f.z *= d.z; f.w *= d.w;
                         }
-                        const mfma_f4 r = acc[0][jb] - acc[1][jb];
+                        const mfma_f4 r = WREG ? acc[0][jb] - acc[1][jb] : acc[0][jb] + acc[1][jb];
                         v[i][jb] = relu_one(make_float4(fmaf(r[0], f.x, m[i][jb].x), fmaf(r[1], f.y, m[i][jb].y), fmaf(r[2], f.z, m[i][jb].z),
                                                          fmaf(r[3], f.w, m[i][jb].w)));
                     }
@@ -358,6 +433,21 @@ __global__ __launch_bounds__(batch_waves<C>() * kWave, BatchShape<C>::MINW) void
 #pragma unroll
                     for (int jb = 0; jb < NJB; ++jb)
                         v[i][jb] = relu_ref4(make_float4(acc[jb][0] + m[i][jb].x, acc[jb][1] + m[i][jb].y, acc[jb][2] + m[i][jb].z, acc[jb][3] + m[i][jb].w));
+                }
+            }
+            if constexpr (!INPUT) {              // columns past the last (in the last quarter, q = 3) stay zero whatever the others are
+                if (C < CP) {
+#pragma unroll
+                    for (int i = 0; i < TPW; ++i)
+#pragma unroll
+                        for (int jb = NJB > 4 ? NJB - 4 : 0; jb < NJB; ++jb) {
+                            const int col = KS * q + 4 * jb;
+                            if (i >= tiles) continue;
+                            v[i][jb].x = col < C ? v[i][jb].x : 0.f;
+                            v[i][jb].y = col + 1 < C ? v[i][jb].y : 0.f;
+                            v[i][jb].z = col + 2 < C ? v[i][jb].z : 0.f;
+                            v[i][jb].w = col + 3 < C ? v[i][jb].w : 0.f;
+                        }
                 }
             }
             if constexpr (decltype(last)::value) ask(next);      // ahead of this bin's stores
@@ -384,69 +474,81 @@ __global__ __launch_bounds__(batch_waves<C>() * kWave, BatchShape<C>::MINW) void
     if (finder.unpacked && tid == 0) *refused = 1;
 }
 
-template <int C, int KSX>
-int launch_batch_levels(int N, int B, int K, int L, const int* a_row_ptr, const int* a_col_idx, const float* a_val, const float* X,
-                        const float* Wn2l, const float* Wc, float* msg, float* h_out, const int* bins, int* refused, hipStream_t s)
+template <int CP, int KSX>
+int launch_batch_levels(int N, int B, int K, int C, int L, const int* a_row_ptr, const int* a_col_idx, const float* a_val, const float* X,
+                        const float* Wn2l, const float* Wc, float* msg, float* h_out, const int* bins, int* refused, int cap, hipStream_t s)
 {
-    constexpr size_t smem = batch_lds_bytes<C, KSX>();
+    constexpr size_t smem = batch_lds_bytes<CP, KSX>();
+    constexpr int kWaves = batch_waves<CP>();
+    static_assert(smem * (BatchShape<CP>::MINW * 4 / kWaves) <= 160 * 1024, "workgroups share the LDS of a compute unit");
     static LdsLimit lds_limit;
-    GNNHIP_HIP(lds_limit.raise(reinterpret_cast<const void*>(&s2v_batch_levels_kernel<C, KSX>), smem));
-    // two neighbouring bins hold more than kRows nodes together, and every 64 graphs may leave one bin short
-    long long most = 2ll * N / kRows + (B + kWave - 1) / kWave + 1;
+    GNNHIP_HIP(lds_limit.raise(reinterpret_cast<const void*>(&s2v_batch_levels_kernel<CP, KSX>), smem));
+    // two neighbouring bins hold more than cap nodes together, and every 64 graphs may leave one bin short
+    long long most = 2ll * N / cap + (B + kWave - 1) / kWave + 1;
     if (most > B) most = B;
-    constexpr int kWaves = batch_waves<C>();
-    const long long resident = (long long)kNumCU * (BatchShape<C>::MINW * 4 / kWaves);
+    const long long resident = (long long)kNumCU * (BatchShape<CP>::MINW * 4 / kWaves);
     const unsigned grid = (unsigned)(most < resident ? most : resident);
-    hipLaunchKernelGGL((s2v_batch_levels_kernel<C, KSX>), dim3(grid), dim3(kWaves * kWave), smem, s, N, B, K, L, a_row_ptr, a_col_idx, a_val, X, Wn2l,
-                       Wc, msg, h_out, bins, refused);
+    hipLaunchKernelGGL((s2v_batch_levels_kernel<CP, KSX>), dim3(grid), dim3(kWaves * kWave), smem, s, N, B, K, C, L, a_row_ptr, a_col_idx, a_val,
+                       X, Wn2l, Wc, msg, h_out, bins, refused);
     GNNHIP_LAUNCH_CHECK("s2v_batch_levels");
     return GNNHIP_OK;
-}
-
-template <int C>
-int batch_levels_c(int N, int B, int K, int L, const int* a_row_ptr, const int* a_col_idx, const float* a_val, const float* X,
-                   const float* Wn2l, const float* Wc, float* msg, float* h_out, const int* bins, int* refused, hipStream_t s)
-{
-#define GNNHIP_BL_ARGS N, B, K, L, a_row_ptr, a_col_idx, a_val, X, Wn2l, Wc, msg, h_out, bins, refused, s
-    if (K <= 16) return launch_batch_levels<C, 4>(GNNHIP_BL_ARGS);
-    if (K <= 32) return launch_batch_levels<C, 8>(GNNHIP_BL_ARGS);
-    if (K <= 48) return launch_batch_levels<C, 12>(GNNHIP_BL_ARGS);
-    return launch_batch_levels<C, 16>(GNNHIP_BL_ARGS);
-#undef GNNHIP_BL_ARGS
 }
 
 constexpr int kTwoStepMeanDegree = 12;           // denser matrices take the SpMM
 
 }  // namespace
 
-// msg and the last level's h of a batch of small graphs.  work: at least batch_levels_work_ints(B) ints, 16-byte aligned.  *refused: the
-// device word that says (1) that the batch is none and the outputs have to be formed by the level-by-level route.
-// GNNHIP_EUNSUPPORTED (nothing launched): sizes that this route does not take.
+// whether batch_levels_dispatch forms msg itself; else it is to be there
+bool batch_levels_with_input(int K, int C) { return K >= 2 && K <= 64 && (C == 16 || C == 32 || C == 64); }
+
 size_t batch_levels_work_ints(int B) { return kOrderRec + bin_ints(B); }
 
+// The last level's h (and msg) of a batch of small graphs.  work: at least batch_levels_work_ints(B) ints, 16-byte aligned.  *refused: the
+// device word that says (1) that the batch is none and the outputs have to be formed by the level-by-level route.
+// GNNHIP_EUNSUPPORTED (nothing launched): sizes that this route does not take.
 int batch_levels_dispatch(int N, int B, int K, int C, int L, long long nnz, const int* a_row_ptr, const int* a_col_idx, const float* a_val,
                           const int* s_row_ptr, const float* X, const float* Wn2l, const float* Wc, float* msg, float* h_out, int* work,
                           const int** refused, hipStream_t s)
 {
     // What the levels but the first save is reading h and msg and writing h.  Below these products the launches of both routes cost more
     // than that (hidden 64, 35,000 nodes: two levels 52 us against 48, three 59 against 62; hidden 32, 73,000 nodes: one level 35.6 against
-    // 35.2, two 42.9 against 45.6).
-    const bool enough = (long long)(L - 1) * N * C >= (C == 16 ? 12000000 : 4000000) && N >= 32768;
-    if (!enough || nnz >= kTwoStepMeanDegree * (long long)N || (long long)N > 96ll * B || K < 2 || K > 64 || !(C == 16 || C == 32 || C == 64))
-        return GNNHIP_EUNSUPPORTED;
+    // 35.2, two 42.9 against 45.6; hidden 50, 88,000 nodes: two levels 78 against 72, three 90 against 94; hidden 77: two levels 95 against
+    // 122, and with 44,000 nodes three 77 against 91; hidden 16, 235,000 nodes of 60 features: three levels 77 against 77).
+    const bool enough = (long long)(L - 1) * N * C >= (C == 16 ? 12000000 : C > 32 && C < 64 ? 6000000 : 4000000) && N >= 32768;
+    if (!enough || nnz >= kTwoStepMeanDegree * (long long)N || (long long)N > 96ll * B || C < 16 || C > 112) return GNNHIP_EUNSUPPORTED;
+    // Bins of fewer nodes where they fill the rounds of workgroups better: a round takes its tiles and about two more (start, barriers).
+    // The host knows the totals only: a bin wastes about half a mean graph, and every 64 graphs about half a bin.
+    const int slots = kNumCU * (C <= 16 ? 3 : C <= 64 ? 2 : 1);
+    int cap = kRows;
+    double best = 0.0;
+    for (int c = kRows; c >= 64; c -= 16) {
+        const double fill = (double)c - 0.5 * (double)N / (double)B;
+        const double nbins = (double)N / (fill > 16.0 ? fill : 16.0) + (double)B / 128.0;
+        const double cost = (double)((long long)(nbins / slots) + 1) * (2.0 + c / 16);
+        if (c == kRows || cost < best) { best = cost; cap = c; }
+    }
     int* word = work;
     int* bins = work + kOrderRec;
-    hipLaunchKernelGGL((graph_bins_kernel<true>), dim3(ceil_div_u((size_t)B, kBinBlock)), dim3(kBinBlock), 0, s, B, kRows, a_row_ptr, s_row_ptr,
-                       bins, N, word);
+    hipLaunchKernelGGL((graph_bins_kernel<true>), dim3(ceil_div_u((size_t)B, kBinBlock)), dim3(kBinBlock), 0, s, B, cap, a_row_ptr, s_row_ptr,
+                       bins, N, word, kRows);
     GNNHIP_LAUNCH_CHECK("graph_bins");
     *refused = word;
-#define GNNHIP_BL_ARGS N, B, K, L, a_row_ptr, a_col_idx, a_val, X, Wn2l, Wc, msg, h_out, bins, word, s
-    switch (C) {
-    case 16: return batch_levels_c<16>(GNNHIP_BL_ARGS);
-    case 32: return batch_levels_c<32>(GNNHIP_BL_ARGS);
-    default: return batch_levels_c<64>(GNNHIP_BL_ARGS);
+#define GNNHIP_BL(CP, KSX) launch_batch_levels<CP, KSX>(N, B, K, C, L, a_row_ptr, a_col_idx, a_val, X, Wn2l, Wc, msg, h_out, bins, word, cap, s)
+    if (batch_levels_with_input(K, C)) {
+#define GNNHIP_BL_K(CP) (K <= 16 ? GNNHIP_BL(CP, 4) : K <= 32 ? GNNHIP_BL(CP, 8) : K <= 48 ? GNNHIP_BL(CP, 12) : GNNHIP_BL(CP, 16))
+        return C == 16 ? GNNHIP_BL_K(16) : C == 32 ? GNNHIP_BL_K(32) : GNNHIP_BL_K(64);
+#undef GNNHIP_BL_K
     }
-#undef GNNHIP_BL_ARGS
+    switch ((C + 15) / 16) {
+    case 1: return GNNHIP_BL(16, 0);
+    case 2: return GNNHIP_BL(32, 0);
+    case 3: return GNNHIP_BL(48, 0);
+    case 4: return GNNHIP_BL(64, 0);
+    case 5: return GNNHIP_BL(80, 0);
+    case 6: return GNNHIP_BL(96, 0);
+    default: return GNNHIP_BL(112, 0);
+    }
+#undef GNNHIP_BL
 }
 
 }  // namespace gnnhip

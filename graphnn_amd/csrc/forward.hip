@@ -18,13 +18,14 @@ int level_backward_dispatch(int N, int C, long long nnz, const int* row_ptr, con
                             const float* W, float* u, float* g_prev, const float* gate, float* acc, hipStream_t s);
 // batch_forward.hip
 size_t batch_levels_work_ints(int B);
+bool batch_levels_with_input(int K, int C);
 int batch_levels_dispatch(int N, int B, int K, int C, int L, long long nnz, const int* a_row_ptr, const int* a_col_idx, const float* a_val,
                           const int* s_row_ptr, const float* X, const float* Wn2l, const float* Wc, float* msg, float* h_out, int* work,
                           const int** refused, hipStream_t s);
 // level_rows.hip
 int level_rows_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* h_in,
                         const float* W, const float* msg, const float* bias, float* h_out, bool same_graph, bool relu_in, CsrPlan* plan,
-                        hipStream_t s);
+                        hipStream_t s, const int* gate);
 int level_rows_backward_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* dz,
                                  const float* W, float* u, float* g_prev, const float* gate, float* acc, hipStream_t s);
 int level_rows_dense_dispatch(int N, int K, int n, const float* x, const float* W, const float* bias, const float* msg, float* out,
@@ -99,7 +100,7 @@ int level_any(int N, int C, long long nnz, const int* row_ptr, const int* col_id
 {
     int rc = level_dispatch(N, C, nnz, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, s, same_graph, relu_in, plan, inference, gate);
     if (rc != GNNHIP_EUNSUPPORTED) return rc;
-    rc = level_rows_dispatch(N, C, nnz, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, same_graph, relu_in, plan, s);
+    rc = level_rows_dispatch(N, C, nnz, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, same_graph, relu_in, plan, s, gate);
     if (rc != GNNHIP_EUNSUPPORTED) return rc;
     void* tmp = nullptr;
     if ((rc = stream_scratch(s, sizeof(float) * (size_t)N * C, &tmp))) return rc;
@@ -158,16 +159,22 @@ int forward_any(int N, int B, int K, int C, int H, int Q, int L, long long a_nnz
     // never stored: the first level gathers from msg.
     // (the routes of the other sizes can too)
     const bool lazy_h0 = L >= 1 && (level_accepts_relu_input(N, C) || !fused_hidden_supported(C)) && aligned16(msg) && aligned16(h_a) && aligned16(h_b) && aligned16(W_conv);
-    // Batches of small graphs: input stage and levels in one launch, which finds out on the device whether the batch is one; what it
-    // needs for that lies in pool, which is written last.  The level-by-level launches behind it do nothing if it is.
+    // Batches of small graphs: levels in one launch (the input stage too where the hidden size has such a kernel), which finds out on the
+    // device whether the batch is one; what it needs for that lies in pool, which is written last.  The level-by-level launches
+    // behind it do nothing if it is.
     const int* gate = nullptr;
+    const bool try_batch = lazy_h0 && aligned16(pool) && batch_levels_work_ints(B) <= (size_t)B * C;
+    const bool with_input = batch_levels_with_input(K, C);
+    auto batch_levels = [&]() {
+        const int rc = try_batch ? batch_levels_dispatch(N, B, K, C, L, a_nnz, a_row_ptr, a_col_idx, a_val, s_row_ptr, X, W_n2l, W_conv, msg,
+                                                         (L & 1) ? h_a : h_b, reinterpret_cast<int*>(pool), &gate, s)
+                                 : GNNHIP_OK;
+        return rc == GNNHIP_EUNSUPPORTED ? GNNHIP_OK : rc;
+    };
     int rc;
-    if (lazy_h0 && aligned16(pool) && batch_levels_work_ints(B) <= (size_t)B * C) {
-        rc = batch_levels_dispatch(N, B, K, C, L, a_nnz, a_row_ptr, a_col_idx, a_val, s_row_ptr, X, W_n2l, W_conv, msg, (L & 1) ? h_a : h_b,
-                                   reinterpret_cast<int*>(pool), &gate, s);
-        if (rc && rc != GNNHIP_EUNSUPPORTED) return rc;
-    }
+    if (with_input && (rc = batch_levels())) return rc;
     if ((rc = input_any(N, K, C, X, W_n2l, msg, lazy_h0 ? nullptr : h_a, s, gate))) return rc;
+    if (!with_input && (rc = batch_levels())) return rc;
     float* cur = lazy_h0 ? msg : h_a;
     float* nxt = lazy_h0 ? h_a : h_b;
     for (int lv = 0; lv < L; ++lv) {

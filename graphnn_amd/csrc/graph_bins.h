@@ -27,13 +27,13 @@ __host__ __device__ inline size_t bin_words_ints(int B) { return ((size_t)((B + 
 // and all of them
 __host__ __device__ inline size_t bin_ints(int B) { return bin_words_ints(B) + kOrderRec * (size_t)((B + kWave - 1) / kWave * kWave); }
 
-// CHECKED: nothing is known about s_row_ptr.  A segment whose graphs are no ascending ranges of nodes, of at most cap nodes each, that
+// CHECKED: nothing is known about s_row_ptr.  A segment whose graphs are no ascending ranges of nodes, of at most `limit` nodes each (at least cap), that
 // begin at node 0 and end at node N, gets the word 0 (a segment that is packed opens at least one bin), and *refused is set to 0 for the
 // forward kernel to set when it comes upon such a word.
 template <bool CHECKED>
 __global__ __launch_bounds__(kBinBlock) void graph_bins_kernel(int B, int cap, const int* __restrict__ a_row_ptr,
                                                                const int* __restrict__ s_row_ptr, int* __restrict__ bins, int N,
-                                                               int* __restrict__ refused)
+                                                               int* __restrict__ refused, int limit)
 {
     const int lane = threadIdx.x & (kWave - 1);
     const int seg = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kBinBlock / kWave) + threadIdx.x / kWave));
@@ -44,7 +44,7 @@ __global__ __launch_bounds__(kBinBlock) void graph_bins_kernel(int B, int cap, c
     if constexpr (CHECKED) {
         if (seg == 0 && lane == 0) *refused = 0;
         const int g = seg * kWave + lane;
-        const bool bad = start < 0 || end < start || end > N || end - start > cap || (g == 0 && start != 0) || (g == B - 1 && end != N);
+        const bool bad = start < 0 || end < start || end > N || end - start > limit || (g == 0 && start != 0) || (g == B - 1 && end != N);
         if (__any(lane < nlive && bad)) {
             if (lane == 0) reinterpret_cast<unsigned long long*>(bins)[seg] = 0;
             return;
@@ -68,7 +68,7 @@ __global__ __launch_bounds__(kBinBlock) void graph_bins_kernel(int B, int cap, c
     const int n = __shfl(end, min(max(lane + ng - 1, 0), kWave - 1), kWave) - start;
     if (!((opens >> lane) & 1ull)) return;
     int e0 = 0, e1 = 0;
-    if (n >= 0 && n <= cap) { e0 = a_row_ptr[start]; e1 = a_row_ptr[start + n]; }
+    if (n >= 0 && n <= (CHECKED ? limit : cap)) { e0 = a_row_ptr[start]; e1 = a_row_ptr[start + n]; }
     int* rec = bins + bin_words_ints(B) + (size_t)(seg * kWave + __popcll(opens & ((1ull << lane) - 1ull))) * kOrderRec;
     *reinterpret_cast<int4*>(rec) = make_int4(seg * kWave + lane, start, n, e0);
     *reinterpret_cast<int2*>(rec + 4) = make_int2(e1, ng);

@@ -44,12 +44,14 @@ struct RowsArgs {
     int relu, relu_in;
     unsigned k_magic;                     // ceil(2^32 / K)
     HubPlan hubs;
+    const int* launch_gate;               // see gated_off
 };
 
 // GATHER: the left operand is A * x.  WT: the product is with W^T.  MINW: wavefronts per SIMD the registers leave room for.
 template <int RT, int NB, int MINW, bool GATHER, bool WT>
 __global__ __launch_bounds__(kBlock, MINW) void s2v_rows_kernel(RowsArgs a)
 {
+    if (gated_off(a.launch_gate)) return;
     using V = ColsLoose;
     constexpr int R = 16 * RT;
     extern __shared__ float4 smem4[];
@@ -353,16 +355,16 @@ bool level_rows_covers(int N, int C, long long nnz)
 
 int level_rows_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* h_in,
                         const float* W, const float* msg, const float* bias, float* h_out, bool same_graph, bool relu_in, CsrPlan* plan,
-                        hipStream_t s)
+                        hipStream_t s, const int* gate)
 {
     if (!level_rows_covers(N, C, nnz)) return GNNHIP_EUNSUPPORTED;
     RowsArgs a{};
     if (int rc = hub_prepass(N, C, nnz, row_ptr, col_idx, val, h_in, C, s, &a.hubs, same_graph, relu_in, kHubThreshold, kHubChunk, -1,
-                             plan ? &plan->row_hub : nullptr))
+                             plan ? &plan->row_hub : nullptr, gate))
         return rc;
     a.N = N; a.K = C; a.n = C;
     a.row_ptr = row_ptr; a.col_idx = col_idx; a.val = val; a.x = h_in; a.W = W;
-    a.bias = bias; a.msg = msg; a.out = h_out; a.relu = 1; a.relu_in = relu_in;
+    a.bias = bias; a.msg = msg; a.out = h_out; a.relu = 1; a.relu_in = relu_in; a.launch_gate = gate;
     return rows_dispatch<true, false>(a, s);
 }
 

@@ -2742,16 +2742,16 @@ def _check_forward(gpu, A, S, N, K, C, L, gen, exact):
 
 def _enough(n, C, L):
     """the sizes repeated until the batch is one that the forward tries to take in one launch"""
-    need = max(32768, (12e6 if C == 16 else 4e6) / ((L - 1) * C))
+    need = max(32768, (12e6 if C == 16 else 6e6 if 32 < C < 64 else 4e6) / ((L - 1) * C))
     return np.tile(np.asarray(n, np.int64), int(np.ceil(need / np.sum(n))))
 
 
-@pytest.mark.parametrize("C", [16, 32, 64])
+@pytest.mark.parametrize("C", [16, 17, 31, 32, 33, 48, 50, 64, 65, 80, 95, 100, 112])
 @pytest.mark.parametrize("sizes", ["molecules", "ones", "full", "with_empty", "dense"])
 def test_forward_over_a_large_batch_of_small_graphs(gpu, C, sizes):
     """batches whose levels run in one launch: bins of one graph of 128 nodes, of 64 graphs of one node, graphs without nodes, bins of
-    more entries than are kept in LDS, a last tile of one row; feature columns around the steps of the input stage.  Hidden 16 and
-    32 have the bits of the stages called one by one; hidden 64 (bf16 pieces) is held to the rounding of fp32 sums"""
+    more entries than are kept in LDS, a last tile of one row; feature columns around the steps of the input stage, hidden sizes around
+    the padded ones.  Hidden 16 and 32 have the bits of the stages called one by one; the others are held to the rounding of fp32 sums"""
     import torch
     gen = torch.Generator(device=gpu).manual_seed(C)
     for K, L, seed in ((2, 2, 0), (3, 4, 1), (17, 3, 2), (33, 4, 3), (64, 2, 4)):
@@ -2763,10 +2763,10 @@ def test_forward_over_a_large_batch_of_small_graphs(gpu, C, sizes):
             n[640:768] = 0                                       # two segments without nodes
             n[-1] = 0
         A, S, N = _small_graphs(gpu, n, 11 if sizes == "dense" else 2, gen)
-        _check_forward(gpu, A, S, N, K, C, L, gen, C != 64)
+        _check_forward(gpu, A, S, N, K, C, L, gen, C in (16, 32))
 
 
-@pytest.mark.parametrize("C", [16, 32, 64])
+@pytest.mark.parametrize("C", [16, 30, 32, 46, 64, 77, 100])
 @pytest.mark.parametrize("kind", ["crossing", "crossing_dense", "large_graph", "uncovered", "offset", "overlapping", "long_row"])
 def test_forward_over_a_batch_that_is_none(gpu, C, kind):
     """what the one launch must refuse on the device: one entry that leaves its bin (kept in LDS, or read from memory), a graph of 129
@@ -2800,3 +2800,48 @@ def test_forward_over_a_batch_that_is_none(gpu, C, kind):
     elif kind == "overlapping":                                  # the last row names all nodes of the batch again
         S = (torch.cat([S[0], S[0][-1:] + N]), torch.cat([S[1], S[1]]), torch.cat([S[2], S[2]]))
     _check_forward(gpu, (rp, ci, val), S, N, 9, C, 3, gen, kind != "long_row")
+
+
+@pytest.mark.parametrize("C", [64, 100])
+def test_forward_over_small_graphs_with_large_and_tiny_values(gpu, C):
+    """products in bf16 pieces over a large batch of small graphs: rows of 2^38 and more and columns of W likewise (scaled down before they
+    are split) beside ordinary ones, values near the smallest floats, infinities and NaNs in a row, which stay in the columns and graphs
+    they belong to"""
+    import torch
+    from graphnn_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(5)
+    A, S, N = _small_graphs(gpu, _enough(np.full(700, 60), C, 2), 2, gen)
+    rp, ci, val = A
+    row = torch.repeat_interleave(torch.arange(N, device=gpu), (rp[1:] - rp[:-1]).long())
+    B, K = S[0].numel() - 1, 8
+    w1, w2 = torch.zeros(C, 4, device=gpu), torch.zeros(4, 2, device=gpu)
+    for scale in (1.0, 1e-36, 1e10):
+        X = torch.rand(N, K, generator=gen, device=gpu)
+        Wn = torch.rand(K, C, generator=gen, device=gpu) * scale
+        Wc = torch.randn(C, C, generator=gen, device=gpu) * 0.1
+        Wc[:, 5] *= 2.0 ** 40
+        Wc[5, 5] = 0.0                                           # or the second level overflows
+        X[1000:1100] *= 2.0 ** 40
+        bufs = ops.s2v_forward(A, S, X, Wn, Wc, w1, w2, 2)
+        h = bufs.msg.clamp(min=0)
+        h1 = ops.s2v_level(*A, h, Wc, bufs.msg)
+        want, zero = bufs.msg.double(), torch.zeros(N, C, dtype=torch.float64, device=gpu)
+        sums = zero.index_add(0, row, h1[ci.long()].double() * val.double()[:, None])
+        want = (sums @ Wc.double() + bufs.msg.double()).clamp(min=0)
+        terms = sums @ Wc.double().abs() + bufs.msg.double().abs()
+        # h1 comes from the FP32 matrix cores here: C + 2 roundings of its terms, which the second level multiplies
+        h1_terms = zero.index_add(0, row, h[ci.long()].double() * val.double()[:, None]) @ Wc.double().abs() + bufs.msg.double().abs()
+        terms = terms + zero.index_add(0, row, h1_terms[ci.long()] * val.double()[:, None]) @ Wc.double().abs()
+        bad = (bufs.h_final.double() - want).abs() > 2 * (C + 8) * 2.0 ** -24 * terms + 2.0 ** -140
+        assert bool(torch.isfinite(want).all()) and not bool(bad.any()), scale
+    # an infinity and a NaN in the features of one node each: nothing outside their graphs changes
+    X = torch.rand(N, K, generator=gen, device=gpu)
+    Wn, Wc = torch.rand(K, C, generator=gen, device=gpu), torch.randn(C, C, generator=gen, device=gpu) * 0.1
+    clean = ops.s2v_forward(A, S, X, Wn, Wc, w1, w2, 2).h_final.clone()
+    X[60 * 10 + 3, 2], X[60 * 20 + 4, 0] = float("inf"), float("nan")
+    got = ops.s2v_forward(A, S, X, Wn, Wc, w1, w2, 2).h_final
+    one_by_one = _forward_one_by_one(A, S, X, Wn, Wc, w1, w2, 2)[1]
+    touched = torch.zeros(N, dtype=torch.bool, device=gpu)
+    touched[600:660] = touched[1200:1260] = True
+    assert torch.equal(got[~touched], clean[~touched])
+    assert torch.equal(torch.isnan(got), torch.isnan(one_by_one)) and torch.equal(torch.isinf(got), torch.isinf(one_by_one))
