@@ -120,39 +120,44 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
         const int row = KS * q + k, col = out_col + 4 * jb;
         return INPUT || (row < C && col < C) ? Wc[(size_t)row * C + col] : 0.f;
     };
+    auto put_w = [&](int jb, const float (&w)[8 * KS2]) {
+        float largest = 0.f;
+#pragma unroll
+        for (int k = 0; k < KS; k += 2) largest = split_max(largest, w[k], w[k + 1]);
+        const unsigned long long large = __ballot(largest >= kSplitLarge);
+        const bool down = (large >> t) & 0x0001000100010001ull;            // in any quarter of the column
+        any_down |= large != 0;
+        const float scale = down ? kSplitDown : kSplitUp;
+        if (q == 0) w_down[out_col + 4 * jb] = down ? kSplitUp / kSplitDown : 1.f;
+#pragma unroll
+        for (int s = 0; s < KS2; ++s) {
+            bf16_words4 w3[3];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                unsigned p[3];
+                bf16_split2(w[8 * s + 2 * i] * scale, w[8 * s + 2 * i + 1] * scale, down, p);
+                const unsigned sign = (WREG ? s : jb) % 2 ? 0x80008000u : 0u;
+#pragma unroll
+                for (int j = 0; j < 3; ++j) w3[j][i] = p[j] ^ sign;
+            }
+            if constexpr (WREG) {
+                wp[s][jb][0] = w3[0]; wp[s][jb][1] = w3[1];
+                if (wave == 0) w_lds[(s * NJB + jb) * kWave + lane] = w3[2];
+            } else {
+#pragma unroll
+                for (int j = 0; j < 3; ++j) w_lds[((s * NJB + jb) * 3 + j) * kWave + lane] = w3[j];
+            }
+        }
+    };
     if constexpr (PIECES) {
 #pragma unroll
-        for (int jb = 0; jb < NJB; ++jb) {
-            if (!WREG && jb % kWaves != wave) continue;                    // uniform
-            float w[8 * KS2], largest = 0.f;
+        for (int j0 = 0; j0 < (WREG ? NJB : (NJB + kWaves - 1) / kWaves); ++j0) {
+            const int jb = WREG ? j0 : j0 * kWaves + wave;
+            if (jb >= NJB) continue;             // uniform
+            float w[8 * KS2];
 #pragma unroll
             for (int k = 0; k < 8 * KS2; ++k) w[k] = k < KS ? w_at(k, jb) : 0.f;
-#pragma unroll
-            for (int k = 0; k < KS; k += 2) largest = split_max(largest, w[k], w[k + 1]);
-            const unsigned long long large = __ballot(largest >= kSplitLarge);
-            const bool down = (large >> t) & 0x0001000100010001ull;        // in any quarter of the column
-            any_down |= large != 0;
-            const float scale = down ? kSplitDown : kSplitUp;
-            if (q == 0) w_down[out_col + 4 * jb] = down ? kSplitUp / kSplitDown : 1.f;
-#pragma unroll
-            for (int s = 0; s < KS2; ++s) {
-                bf16_words4 w3[3];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    unsigned p[3];
-                    bf16_split2(w[8 * s + 2 * i] * scale, w[8 * s + 2 * i + 1] * scale, down, p);
-                    const unsigned sign = (WREG ? s : jb) % 2 ? 0x80008000u : 0u;
-#pragma unroll
-                    for (int j = 0; j < 3; ++j) w3[j][i] = p[j] ^ sign;
-                }
-                if constexpr (WREG) {
-                    wp[s][jb][0] = w3[0]; wp[s][jb][1] = w3[1];
-                    if (wave == 0) w_lds[(s * NJB + jb) * kWave + lane] = w3[2];
-                } else {
-#pragma unroll
-                    for (int j = 0; j < 3; ++j) w_lds[((s * NJB + jb) * 3 + j) * kWave + lane] = w3[j];
-                }
-            }
+            put_w(jb, w);
         }
     } else {
 #pragma unroll
@@ -397,16 +402,22 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
                     } else {
 #pragma unroll
                         for (int s = 0; s < KS2; ++s) {
+                            // a few blocks at a time, so that no product waits for the sum of the one before it
+                            constexpr int kGroup = 4;
 #pragma unroll
-                            for (int jb = 0; jb < NJB; ++jb) {
-                                const bf16_words4* w = w_lds + (s * NJB + jb) * 3 * kWave + lane;
-                                const bf16_words4 w0 = w[0], w1 = w[kWave], w2 = w[2 * kWave];
-                                acc[1][jb] = mfma_bf16(w2, p[s][0], acc[1][jb]);
-                                acc[0][jb] = mfma_bf16(w0, p[s][0], acc[0][jb]);
-                                acc[1][jb] = mfma_bf16(w0, p[s][2], acc[1][jb]);
-                                acc[1][jb] = mfma_bf16(w1, p[s][1], acc[1][jb]);
-                                acc[1][jb] = mfma_bf16(w1, p[s][0], acc[1][jb]);
-                                acc[1][jb] = mfma_bf16(w0, p[s][1], acc[1][jb]);
+                            for (int j0 = 0; j0 < NJB; j0 += kGroup) {
+                                bf16_words4 w[kGroup][3];
+#pragma unroll
+                                for (int j = 0; j < kGroup; ++j)
+#pragma unroll
+                                    for (int i = 0; i < 3; ++i)
+                                        if (j0 + j < NJB) w[j][i] = w_lds[((s * NJB + j0 + j) * 3 + i) * kWave + lane];
+                                auto products = [&](int sum, int i, int x) {
+#pragma unroll
+                                    for (int j = 0; j < kGroup; ++j)
+                                        if (j0 + j < NJB) acc[sum][j0 + j] = mfma_bf16(w[j][i], p[s][x], acc[sum][j0 + j]);
+                                };
+                                products(1, 2, 0); products(0, 0, 0); products(1, 0, 2); products(1, 1, 1); products(1, 1, 0); products(1, 0, 1);
                             }
                         }
                     }

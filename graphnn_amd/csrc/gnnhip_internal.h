@@ -210,6 +210,7 @@ inline bool level_by_tile(int N, int C, long long nnz)
 {
     return N <= (C == 16 && nnz > kLevelTileDense * (long long)N ? kLevelTileMaxRows / 2 : kLevelTileMaxRows);
 }
+constexpr int kFewRows = 16 * kNumCU;  // up to here a level at the hidden sizes of level_rows.hip takes a workgroup per 16 rows and 64 columns
 constexpr int kHubMinRows = 32768;     // smaller matrices skip the pre-pass: its launches would cost more than a long row
 struct HubPlan {
     const int* row_chunk = nullptr;    // [m], defined for rows longer than the pass's threshold only: first chunk, -1: not summed

@@ -563,6 +563,9 @@ int level_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* c
         }
     }
     if (!level_wide_covers(N, C)) return GNNHIP_EUNSUPPORTED;
+    // FP32 levels of hidden 256 over few rows: the kernel of the other hidden sizes shares the columns of 16 rows out over workgroups, where
+    // the one of many rows starts by loading W into its registers (286 rows 11.0 -> 7.0 us, 1,760 11.2 -> 7.9; hidden 128 5.3, 5.7 so)
+    if (C == 256 && N <= kFewRows / 2 && !(inference && !bias)) return GNNHIP_EUNSUPPORTED;
     auto wide = [&](long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* h_in, bool relu_in) {
         return inference && !bias ? level_split_dispatch(N, C, row_ptr, col_idx, val, h_in, W, msg, h_out, relu_in, s)
                                   : level_wide_dispatch(N, C, nnz, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, relu_in, s);

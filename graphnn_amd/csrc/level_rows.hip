@@ -302,6 +302,247 @@ __global__ __launch_bounds__(kBlock, MINW) void s2v_rows_kernel(RowsArgs a)
     }
 }
 
+// The same for few rows, where a launch is one chain of waits and the matrix instructions of a workgroup are those of one compute unit: a
+// workgroup takes 16 rows and a share of the columns, a row is summed by a lane group of its own, a wavefront has one block of 16
+// columns of W, all of it in registers, and the product follows behind one barrier, straight to memory.  (W a step of 16 k ahead of the
+// product, as above, is a trip to L2 per step where nothing else runs.)  The workgroups that share a product sum its rows each; the
+// sums have the order of the kernel above.  286 rows, hidden 252: 19.3 -> 6.7 us per level; hidden 100 8.3 -> 5.7, 50 5.3 -> 4.6; 1,760
+// rows, hidden 200 16.7 -> 7.6, backward 16.3 -> 9.1.
+// BLOCKS: wavefronts, blocks of 16 columns that the left operand has at most.
+template <int BLOCKS, bool GATHER, bool WT>
+__global__ __launch_bounds__(BLOCKS * kWave) void s2v_rows_few_kernel(RowsArgs a, int blocks)
+{
+    using V = ColsLoose;
+    if (gated_off(a.launch_gate)) return;
+    constexpr int kThreads = BLOCKS * kWave;
+    constexpr int FL = BLOCKS == 16 ? 4 : kFlight;             // W takes 64 of 128 registers there
+    extern __shared__ float4 smem4[];
+    __shared__ float4 shared4[GATHER ? kBlock : 1];            // sums of a long row
+    __shared__ int long_row[GATHER ? 16 : 1];
+    __shared__ int long_count;
+    float* tile = reinterpret_cast<float*>(smem4);             // [16][LD]
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int q = lane >> 4, t = lane & 15;
+    const int K = a.K, n = a.n;
+    const int KP = (K + 15) & ~15, LD = KP + 4;
+    const long long row0 = (long long)blockIdx.x * 16;
+    const int rows = (int)min(16ll, (long long)a.N - row0);
+
+    const int units = (K + 3) / 4;
+    const int logG = units <= 1 ? 0 : 32 - __builtin_clz((unsigned)(units - 1));
+    const int G = 1 << logG, sub = tid & (G - 1), grp = tid >> logG;      // at least 16 groups
+    const bool live = sub < units;
+    const int col0 = V::at(sub, K);
+    // blocks: of the product, per workgroup; the workgroups of a row of the grid's y share the 16 rows' product
+    const int block = blockIdx.y * blocks + wave;
+    const bool wave_live = wave < blocks && 16 * block < n;    // uniform
+
+    float wf[BLOCKS][4];                                       // wf[k][s] = W[16 k + 4 q + s][16 block + t], zero from k = K on
+    auto ask_w = [&]() {
+        const rsrc_t w_rsrc = make_rsrc(a.W, (unsigned)((size_t)K * n * 4));
+        const int w_col = 16 * block + t;
+#pragma unroll
+        for (int k = 0; k < BLOCKS; ++k) {
+            if (16 * k >= KP || !wave_live) { wf[k][0] = wf[k][1] = wf[k][2] = wf[k][3] = 0.f; continue; }     // uniform
+            if constexpr (WT) {
+                if (16 * k + 16 <= K) {
+                    const float4 w = V::load(a.W + (size_t)min(w_col, n - 1) * K + 16 * k + 4 * q);
+                    wf[k][0] = w.x; wf[k][1] = w.y; wf[k][2] = w.z; wf[k][3] = w.w;
+                    continue;
+                }
+            }
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const int at = 16 * k + 4 * q + s;
+                wf[k][s] = buf_load_f(w_rsrc, at < K && w_col < n ? (WT ? w_col * K + at : at * n + w_col) * 4 : kBufPastEnd, 0);
+            }
+        }
+    };
+    // columns out_col .. + 3 of row t of the product are this lane's
+    const int out_col = 16 * block + 4 * q;
+    const size_t out_at = (size_t)(row0 + min(t, rows - 1)) * n + out_col;
+    auto ask = [&](const float* p) {
+        float4 v = f4_zero();
+        if (!p || t >= rows || !wave_live) return v;
+        if (out_col + 4 <= n) return V::load(p + out_at);
+        if (out_col < n) v.x = p[out_at];
+        if (out_col + 1 < n) v.y = p[out_at + 1];
+        if (out_col + 2 < n) v.z = p[out_at + 2];
+        return v;
+    };
+    float4 ex = f4_zero(), old = f4_zero();
+    auto ask_rest = [&]() {                                    // what the product is multiplied with and what is added to it
+        ask_w();
+        ex = ask(a.msg ? a.msg : a.gate);
+        if constexpr (WT) old = ask(a.acc);
+    };
+
+    // ---- the left operand's rows
+    if constexpr (GATHER) {
+        // Row pointers, entries, rows: three trips to memory, one after the other (buffer loads: what there is not is asked for past
+        // the end).  The rest is asked for behind the first rows and arrives with them.
+        int start = 0, end = 0;
+        {
+            const rsrc_t rp_rsrc = make_rsrc(a.row_ptr, (unsigned)(a.N + 1) * 4u);
+            start = buf_load_i(rp_rsrc, grp < rows ? (int)(row0 + grp) * 4 : kBufPastEnd, 0);
+            end = buf_load_i(rp_rsrc, grp < rows ? (int)(row0 + grp + 1) * 4 : kBufPastEnd, 0);
+        }
+        if (tid == 0) long_count = 0;
+        for (int i = tid; i < 16 * 16; i += kThreads) {        // the columns behind K
+            const int c = KP - 16 + (i & 15);
+            if (c >= K) tile[(i >> 4) * LD + c] = 0.f;
+        }
+        const rsrc_t col_rsrc = make_rsrc(a.col_idx, 0xFFFFFFFCu), val_rsrc = make_rsrc(a.val, 0xFFFFFFFCu);
+        const rsrc_t x_rsrc = make_rsrc(a.x, (unsigned)a.N * (unsigned)K * 4u);
+        const bool is_long = end - start > kLongRow;
+        const int stop = is_long ? start : end;
+        int c[FL];
+        float v[FL];
+        float4 x[FL];
+        auto ask_entries = [&](int base) {
+#pragma unroll
+            for (int u = 0; u < FL; ++u) {
+                const int off = base + u < stop ? (base + u) * 4 : kBufPastEnd;
+                c[u] = buf_load_i(col_rsrc, off, 0);
+                v[u] = buf_load_f(val_rsrc, off, 0);
+            }
+        };
+        auto ask_rows = [&](int base) {
+#pragma unroll
+            for (int u = 0; u < FL; ++u) x[u] = buf_load4(x_rsrc, base + u < stop && live ? (c[u] * K + col0) * 4 : kBufPastEnd, 0);
+        };
+        float4 sum = f4_zero();
+        auto add_rows = [&](int base, const float (&w)[FL]) {
+#pragma unroll
+            for (int u = 0; u < FL; ++u)
+                if (base + u < stop) f4_fma(sum, w[u], a.relu_in ? relu_ref4(x[u]) : x[u]);
+        };
+        ask_entries(start);
+        ask_rows(start);
+        ask_rest();
+        for (int base = start; base < stop; base += FL) {
+            float now[FL];
+#pragma unroll
+            for (int u = 0; u < FL; ++u) now[u] = v[u];
+            const bool more = base + FL < stop;
+            if (more) ask_entries(base + FL);
+            add_rows(base, now);
+            if (more) ask_rows(base + FL);
+        }
+        auto finish_row = [&](int r, const float4& total) {
+            if (!live) return;
+            V::store(tile + r * LD + col0, total);
+            if (a.agg_out && r < rows && blockIdx.y == 0) V::store(a.agg_out + (size_t)(row0 + r) * K + col0, total);
+        };
+        if (grp < 16 && !is_long) finish_row(grp, sum);
+        __syncthreads();
+        if (is_long && grp < 16 && sub == 0) long_row[atomicAdd(&long_count, 1)] = grp;
+        __syncthreads();
+        const int nlong = long_count;
+        const int lgroups = kBlock >> logG;                    // those of the kernel above: the same sums
+        for (int li = 0; li < nlong; ++li) {
+            const int r = long_row[li];
+            const int first = a.row_ptr[row0 + r], last = a.row_ptr[row0 + r + 1];
+            float4 total = f4_zero();
+            if (grp < lgroups) {
+                for (int e = first + grp; e < last; e += 4 * lgroups) {
+                    int lc[4];
+                    float lv[4];
+                    float4 lx[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const bool ok = e + u * lgroups < last;
+                        lc[u] = ok ? a.col_idx[e + u * lgroups] : 0;
+                        lv[u] = ok ? a.val[e + u * lgroups] : 0.f;
+                    }
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) lx[u] = e + u * lgroups < last && live ? V::load(a.x + (size_t)lc[u] * K + col0) : f4_zero();
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        if (e + u * lgroups < last) f4_fma(total, lv[u], a.relu_in ? relu_ref4(lx[u]) : lx[u]);
+                }
+                shared4[tid] = total;
+            }
+            __syncthreads();
+            if (grp == 0) {
+                float4 s = f4_zero();
+                for (int g = 0; g < lgroups; ++g) s = V::add(s, shared4[g * G + sub]);
+                finish_row(r, s);
+            }
+            __syncthreads();
+        }
+    } else {
+        ask_rest();
+        for (int i = tid; i < 16 * 16; i += kThreads) {
+            const int c = KP - 16 + (i & 15);
+            if (c >= K || (i >> 4) >= rows) tile[(i >> 4) * LD + c] = 0.f;
+        }
+        const float* src = a.x + (size_t)row0 * K;
+        const int total = rows * K;
+        for (int base = 0; base < total; base += 4 * kThreads) {
+            float v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) { const int i = base + tid + u * kThreads; v[u] = i < total ? src[i] : 0.f; }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int i = base + tid + u * kThreads;
+                const int r = K >= 2 ? (int)__umulhi((unsigned)i, a.k_magic) : i;
+                if (i < total) tile[r * LD + i - r * K] = v[u];
+            }
+        }
+        __syncthreads();
+    }
+    if (!wave_live) return;                                   // uniform; no barrier follows
+
+    // ---- the product, and what follows it, straight from the registers
+    mfma_f4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < BLOCKS; ++k) {
+        if (16 * k >= KP) continue;                            // uniform
+        const float4 x = *reinterpret_cast<const float4*>(tile + t * LD + 16 * k + 4 * q);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[k][0], x.x, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[k][1], x.y, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[k][2], x.z, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[k][3], x.w, acc, 0, 0, 0);
+    }
+    if (t >= rows) return;
+    float4 v = make_float4(acc[0], acc[1], acc[2], acc[3]);
+    if (a.bias) {
+        const int last = n - 1;
+        v.x += a.bias[min(out_col, last)]; v.y += a.bias[min(out_col + 1, last)]; v.z += a.bias[min(out_col + 2, last)]; v.w += a.bias[min(out_col + 3, last)];
+    }
+    if (a.msg) v = V::add(v, ex);
+    if constexpr (WT) {
+        if (a.gate) v = make_float4(ex.x > 0.f ? v.x : 0.f, ex.y > 0.f ? v.y : 0.f, ex.z > 0.f ? v.z : 0.f, ex.w > 0.f ? v.w : 0.f);
+    }
+    if (a.relu) v = relu_ref4(v);
+    auto put = [&](float* p, const float4& x) {
+        if (out_col + 4 <= n) { V::store(p + out_at, x); return; }
+        if (out_col < n) p[out_at] = x.x;
+        if (out_col + 1 < n) p[out_at + 1] = x.y;
+        if (out_col + 2 < n) p[out_at + 2] = x.z;
+    };
+    put(a.out, v);
+    if (a.relu_out) put(a.relu_out, relu_ref4(v));
+    if constexpr (WT) {
+        if (a.acc) put(a.acc, V::add(old, v));
+    }
+}
+
+template <int BLOCKS, bool GATHER, bool WT>
+int launch_rows_few(const RowsArgs& a, hipStream_t s)
+{
+    const int KP = (a.K + 15) & ~15;
+    const int tiles = (int)(((long long)a.N + 15) / 16), blocks = (a.n + 15) / 16;
+    // as long as there are compute units for it, four blocks to a workgroup: the matrix instructions of 16 x 256 x 256 on one of them take 4 us
+    int share = (blocks + 3) / 4;
+    while (share > 1 && share * tiles > kNumCU) --share;
+    const int per = (blocks + share - 1) / share;
+    hipLaunchKernelGGL((s2v_rows_few_kernel<BLOCKS, GATHER, WT>), dim3(tiles, share), dim3(BLOCKS * kWave), sizeof(float) * 16 * (KP + 4), s, a, per);
+    GNNHIP_LAUNCH_CHECK("s2v_rows_few");
+    return GNNHIP_OK;
+}
+
 template <int RT, int NB, int MINW, bool GATHER, bool WT>
 int launch_rows(const RowsArgs& a, hipStream_t s)
 {
@@ -334,6 +575,13 @@ template <bool GATHER, bool WT>
 int rows_dispatch(RowsArgs a, hipStream_t s)
 {
     a.k_magic = a.K >= 2 ? (unsigned)(((1ull << 32) + a.K - 1) / a.K) : 0;
+    // (a second workgroup per compute unit would wait for the first: 4,112 rows, hidden 200, backward 18.8 -> 20.5 us)
+    if (a.N <= kFewRows && a.K >= 4) {
+        const int widest = a.K > a.n ? a.K : a.n;
+        if (widest <= 64) return launch_rows_few<4, GATHER, WT>(a, s);
+        if (widest <= 128) return launch_rows_few<8, GATHER, WT>(a, s);
+        return launch_rows_few<16, GATHER, WT>(a, s);
+    }
     if (a.n <= 64) return rows_by_tile<1, GATHER, WT>(a, s);
     if (a.n <= 128) return rows_by_tile<2, GATHER, WT>(a, s);
     // wider: 32 rows, where the tile leaves room for two workgroups per compute unit

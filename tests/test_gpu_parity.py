@@ -2845,3 +2845,69 @@ def test_forward_over_small_graphs_with_large_and_tiny_values(gpu, C):
     touched[600:660] = touched[1200:1260] = True
     assert torch.equal(got[~touched], clean[~touched])
     assert torch.equal(torch.isnan(got), torch.isnan(one_by_one)) and torch.equal(torch.isinf(got), torch.isinf(one_by_one))
+
+
+@pytest.mark.parametrize("C", [4, 7, 16, 33, 64, 65, 100, 128, 129, 200, 252, 255, 256])
+def test_levels_over_few_rows_have_the_bits_of_many(gpu, C):
+    """a level, its backward and the input stage over up to 4,096 rows (a workgroup per 16 rows and share of the columns) against the same
+    rows inside a matrix of more (another kernel): 1 to 17 rows, the last rows where the columns are shared out and where they are not,
+    rows of 0, 1, 4, 5, 8, 9, 300 and 3,000 entries, a bias, a gate and a running sum"""
+    import torch
+    from graphnn_amd import ops
+    if C in (16, 64, 128, 256):                                # these sizes have kernels of their own: as widths of the input stage only
+        return _few_rows_input(gpu, C)
+    gen = torch.Generator(device=gpu).manual_seed(C)
+    rand = lambda *shape: torch.randn(*shape, generator=gen, device=gpu)
+    big = 4113
+    W, bias = rand(C, C) * 0.2, rand(C)
+    for N in (1, 16, 17, 272, 2048, 2049, 4096):
+        # columns of the first N rows lie below N, so both matrices mean the same for these rows
+        deg = torch.randint(0, 10, (big,), generator=gen, device=gpu)
+        deg[torch.randperm(min(N, 40), generator=gen, device=gpu)[:2]] = 300
+        deg[N // 2] = 3000
+        rp = torch.zeros(big + 1, dtype=torch.int32, device=gpu)
+        rp[1:] = torch.cumsum(deg, 0)
+        ci = torch.randint(0, N, (int(rp[-1]),), generator=gen, device=gpu).int()
+        val = rand(int(rp[-1]))
+        x, msg, gate, acc = rand(big, C), rand(big, C), rand(big, C), rand(big, C)
+        E = int(rp[N])
+        few = (rp[:N + 1].contiguous(), ci[:E].contiguous(), val[:E].contiguous())
+        part = lambda t: t[:N].contiguous()
+        for b in (None, bias):
+            assert torch.equal(ops.s2v_level(*few, part(x), W, part(msg), b), ops.s2v_level(rp, ci, val, x, W, msg, b)[:N]), (N, b is None)
+        a_few, a_big = part(acc), acc.clone()
+        u, g = ops.s2v_level_backward(*few, part(x), W, gate_h=part(gate), acc=a_few)
+        u2, g2 = ops.s2v_level_backward(rp, ci, val, x, W, gate_h=gate, acc=a_big)
+        assert torch.equal(u, u2[:N]) and torch.equal(g, g2[:N]) and torch.equal(a_few, a_big[:N]), N
+        u, g = ops.s2v_level_backward(*few, part(x), W)
+        assert torch.equal(g, ops.s2v_level_backward(rp, ci, val, x, W)[1][:N]), N
+    _few_rows_input(gpu, C)
+
+
+def _few_rows_input(gpu, C):
+    """the input stage of few rows, feature columns narrower and wider than its steps: within the rounding of its sums"""
+    import torch
+    from graphnn_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(C + 1)
+    for N, K in ((1, 4), (15, 5), (33, 17), (300, 64), (4096, 100)):
+        X, Wn = torch.randn(N, K, generator=gen, device=gpu), torch.randn(K, C, generator=gen, device=gpu)
+        msg, h = ops.s2v_input(X, Wn)
+        bound = (K + 2) * 2.0 ** -24 * (X.double().abs() @ Wn.double().abs())
+        assert bool(((msg.double() - X.double() @ Wn.double()).abs() <= bound).all()) and torch.equal(h, msg.clamp(min=0)), (N, K)
+
+
+@pytest.mark.parametrize("N", [1, 40, 2048])
+def test_level_of_hidden_256_over_few_rows(gpu, oracle, N):
+    """the FP32 level of hidden 256 takes the kernel of few rows: against the oracle, with a bias and without"""
+    from graphnn_amd import ops
+    rng = np.random.default_rng(N)
+    C = 256
+    csr = _random_csr(rng, N, N, 3 * N)
+    h_in = np.maximum(rng.standard_normal((N, C)), 0).astype(np.float32)
+    W = (rng.standard_normal((C, C)) * 0.1).astype(np.float32)
+    msg, bias = rng.standard_normal((N, C)).astype(np.float32), rng.standard_normal(C).astype(np.float32)
+    for b in (None, bias):
+        want, w64 = _level_want(oracle, *csr, h_in, W, msg, b)
+        got = _n(ops.s2v_level(*_csr_t(csr, gpu), _t(h_in, gpu), _t(W, gpu), _t(msg, gpu), None if b is None else _t(b, gpu)))
+        assert_parity("level", got, want, w64)
+        assert_condition("level", got, w64(), w64.cond())
