@@ -62,12 +62,13 @@ __device__ __forceinline__ int last_at_most(const int* v, int n, int x)
 
 // Per workgroup one run of `rows` rows: its hubs in row order (list_row) with the chunks of the run ahead of each
 // (list_chunk), both from the run's first row on, and the numbers of its hubs and of their chunks.
+template <bool GATED>
 __global__ __launch_bounds__(kBlock) void hub_count_kernel(int m, int rows, const int* __restrict__ row_ptr, int* __restrict__ run_hubs,
                                                            int* __restrict__ run_chunks, int* __restrict__ list_row,
                                                            int* __restrict__ list_chunk, int threshold, int shift,
                                                            const int* __restrict__ gate)
 {
-    if (gated_off(gate)) return;
+    if (gated_off<GATED>(gate)) return;
     __shared__ int sh[2][kWavesPerBlock];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const long long lo = (long long)blockIdx.x * rows, hi = min(lo + rows, (long long)m);
@@ -112,13 +113,13 @@ __global__ __launch_bounds__(kBlock) void hub_count_kernel(int m, int rows, cons
 // One wavefront per chunk.  The wavefront is split into 64 / G lane groups; group g takes the
 // chunk's entries g, g + ngroups, ... eight at a time, a lane owns the column slabs
 // (sub + it * G) * V::kVec.  The groups' sums are added through LDS in group order.
-template <class V, int ITERS>
+template <class V, int ITERS, bool GATED>
 __global__ __launch_bounds__(kBlock) void hub_partial_kernel(
     int run_rows, int runs, const int* __restrict__ run_hubs, const int* __restrict__ run_chunks, const int* __restrict__ list_row,
     const int* __restrict__ list_chunk, int chunk_cap, int n, const int* __restrict__ row_ptr, const int* __restrict__ col_idx, const float* __restrict__ val, const float* __restrict__ B, int ldb, int logG,
     int* __restrict__ row_chunk, float* __restrict__ part, int ldp, int relu_in, int threshold, int shift, const int* __restrict__ gate)
 {
-    if (gated_off(gate)) return;
+    if (gated_off<GATED>(gate)) return;
     // relu_in: the rows of B are used as ReLU(B) (a first level that reads msg in place of h0)
     __shared__ float red[kWavesPerBlock][kWave * V::kVec * ITERS];
     __shared__ int before[kMaxRuns + 1];         // chunks ahead of a run
@@ -267,7 +268,8 @@ void launch_partial(hipStream_t s, const HubLayout& L, char* base, int n, const 
     long long grid = ((long long)L.chunk_cap + kWavesPerBlock - 1) / kWavesPerBlock;
     if (grid > kNumCU * 8) grid = kNumCU * 8;
     auto ints = [base](size_t o) { return reinterpret_cast<int*>(base + o); };
-    hipLaunchKernelGGL((hub_partial_kernel<V, ITERS>), dim3((unsigned)grid), dim3(kBlock), 0, s, L.run_rows, L.runs, ints(L.o_hubs),
+    const auto kernel = gate ? &hub_partial_kernel<V, ITERS, true> : &hub_partial_kernel<V, ITERS, false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(kBlock), 0, s, L.run_rows, L.runs, ints(L.o_hubs),
                        ints(L.o_chunks), ints(L.o_lrow), ints(L.o_lchunk), L.chunk_cap, n, row_ptr, col_idx, val, B, ldb, logG,
                        ints(L.o_row), reinterpret_cast<float*>(base + L.o_part), L.ldp, relu_in, threshold, shift, gate);
 }
@@ -341,9 +343,11 @@ int hub_prepass(int m, int n, long long nnz, const int* row_ptr, const int* col_
         if (!planned) memos[s] = Memo{row_ptr, m, n, nnz, base, threshold, chunk_len, L.chunk_cap};
     }
     if (!planned) {
-        hipLaunchKernelGGL(hub_count_kernel, dim3((unsigned)L.runs), dim3(kBlock), 0, s, m, L.run_rows, row_ptr,
+        const int* off = store ? nullptr : gate;               // a kept plan is made either way
+        const auto kernel = off ? &hub_count_kernel<true> : &hub_count_kernel<false>;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)L.runs), dim3(kBlock), 0, s, m, L.run_rows, row_ptr,
                            reinterpret_cast<int*>(b + L.o_hubs), reinterpret_cast<int*>(b + L.o_chunks), reinterpret_cast<int*>(b + L.o_lrow),
-                           reinterpret_cast<int*>(b + L.o_lchunk), threshold, shift, store ? nullptr : gate);    // a kept plan is made either way
+                           reinterpret_cast<int*>(b + L.o_lchunk), threshold, shift, off);
         if (store) store->planned = true;
     }
     if (n < 4) {

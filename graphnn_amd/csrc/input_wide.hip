@@ -22,12 +22,12 @@ constexpr int kWaves = kBlock / kWave;       // 4
 constexpr int kTileRows = 64;
 
 // KS = contraction steps of four: K <= 4 KS.
-template <int C, int KS>
+template <int C, int KS, bool GATED>
 __global__ __launch_bounds__(kBlock) void s2v_input_wide_kernel(
     int N, int K, unsigned k_magic, int x_vec, const float* __restrict__ X, const float* __restrict__ Wn2l,
     float* __restrict__ msg, float* __restrict__ h0, const int* __restrict__ gate)
 {
-    if (gated_off(gate)) return;
+    if (gated_off<GATED>(gate)) return;
     constexpr int CW = C / kWaves;           // output columns per wavefront
     constexpr int NB = CW / 16;              // 16-column blocks per wavefront
     constexpr int LDT = 4 * KS + 4;          // LDS row stride
@@ -148,7 +148,9 @@ int launch_input_wide(int N, int K, const float* X, const float* Wn2l, float* ms
     const unsigned grid = (unsigned)(ntiles < cap ? ntiles : cap);
     const unsigned k_magic = K >= 2 ? (unsigned)((0x100000000ull + (unsigned)K - 1) / (unsigned)K) : 0u;   // ceil(2^32 / K)
     const int x_vec = aligned16(X) ? 1 : 0;
-    hipLaunchKernelGGL((s2v_input_wide_kernel<C, KS>), dim3(grid), dim3(kBlock), 0, s, N, K, k_magic, x_vec, X, Wn2l, msg, h0, gate);
+    constexpr bool kGated = C == 64;             // the size of batch_forward.hip among these
+    const auto kernel = kGated && gate ? &s2v_input_wide_kernel<C, KS, kGated> : &s2v_input_wide_kernel<C, KS, false>;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBlock), 0, s, N, K, k_magic, x_vec, X, Wn2l, msg, h0, gate);
     GNNHIP_LAUNCH_CHECK("s2v_input_wide");
     return GNNHIP_OK;
 }

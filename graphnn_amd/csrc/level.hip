@@ -122,12 +122,12 @@ __device__ __forceinline__ void tile_times_w(const float* tile, int ldt, int kdi
 }
 
 // ---------------------------------------------------------------- input: msg = X * W_n2l, h0 = ReLU(msg)
-template <int C, int RT>
+template <int C, int RT, bool GATED>
 __global__ __launch_bounds__(kBlock) void s2v_input_kernel(
     int N, int K, const float* __restrict__ X, const float* __restrict__ Wn2l,
     float* __restrict__ msg, float* __restrict__ h0, const int* __restrict__ gate)
 {
-    if (gated_off(gate)) return;
+    if (gated_off<GATED>(gate)) return;
     constexpr int G = C / 4, P = kBlock / G, R = RT * P;
     extern __shared__ float smem[];
     const int ldt = ((K + 3) & ~3) + 4;              // padded row stride of the X tile, multiple of 4
@@ -443,7 +443,8 @@ int launch_input(int N, int K, const float* X, const float* Wn2l, float* msg, fl
     if (smem > 64 * 1024) return GNNHIP_EUNSUPPORTED;
     const int ntiles = (N + R - 1) / R;
     const int grid = ntiles < kNumCU * 4 ? ntiles : kNumCU * 4;
-    hipLaunchKernelGGL((s2v_input_kernel<C, RT>), dim3(grid), dim3(kBlock), smem, s, N, K, X, Wn2l, msg, h0, gate);
+    const auto kernel = gate ? &s2v_input_kernel<C, RT, true> : &s2v_input_kernel<C, RT, false>;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBlock), smem, s, N, K, X, Wn2l, msg, h0, gate);
     GNNHIP_LAUNCH_CHECK("s2v_input");
     return GNNHIP_OK;
 }

@@ -48,10 +48,10 @@ struct RowsArgs {
 };
 
 // GATHER: the left operand is A * x.  WT: the product is with W^T.  MINW: wavefronts per SIMD the registers leave room for.
-template <int RT, int NB, int MINW, bool GATHER, bool WT>
+template <int RT, int NB, int MINW, bool GATHER, bool WT, bool GATED>
 __global__ __launch_bounds__(kBlock, MINW) void s2v_rows_kernel(RowsArgs a)
 {
-    if (gated_off(a.launch_gate)) return;
+    if (gated_off<GATED>(a.launch_gate)) return;
     using V = ColsLoose;
     constexpr int R = 16 * RT;
     extern __shared__ float4 smem4[];
@@ -313,7 +313,6 @@ template <int BLOCKS, bool GATHER, bool WT>
 __global__ __launch_bounds__(BLOCKS * kWave) void s2v_rows_few_kernel(RowsArgs a, int blocks)
 {
     using V = ColsLoose;
-    if (gated_off(a.launch_gate)) return;
     constexpr int kThreads = BLOCKS * kWave;
     constexpr int FL = BLOCKS == 16 ? 4 : kFlight;             // W takes 64 of 128 registers there
     extern __shared__ float4 smem4[];
@@ -549,7 +548,9 @@ int launch_rows(const RowsArgs& a, hipStream_t s)
     const int KP = (a.K + 15) & ~15;
     const int width = KP + 4 > a.n ? KP + 4 : a.n;
     const unsigned grid = (unsigned)(((long long)a.N + 16 * RT - 1) / (16 * RT));
-    hipLaunchKernelGGL((s2v_rows_kernel<RT, NB, MINW, GATHER, WT>), dim3(grid), dim3(kBlock), sizeof(float) * 16 * RT * width, s, a);
+    constexpr bool kGated = GATHER && !WT && RT > 1 && NB <= 2;            // the levels of batch_forward.hip's sizes
+    const auto kernel = kGated && a.launch_gate ? &s2v_rows_kernel<RT, NB, MINW, GATHER, WT, kGated> : &s2v_rows_kernel<RT, NB, MINW, GATHER, WT, false>;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBlock), sizeof(float) * 16 * RT * width, s, a);
     GNNHIP_LAUNCH_CHECK("s2v_rows");
     return GNNHIP_OK;
 }

@@ -56,7 +56,7 @@ constexpr int kPipeMinRows = 65536;   // from here on the kernel variant that as
 // CSR matrix: W is read transposed, the aggregated rows A' x are also stored (agg_out: they are the other
 // factor of the weight gradient).  No ReLU and no bias; `msg`, when given, is the embedding whose ReLU the
 // gradient passes next: out = out where msg > 0, else 0, and acc_io (when given) += out.
-template <int C, bool DENSE, bool WLDS, int MINW, bool RELU_IN, bool PIPE, bool BWD = false, bool PIECES = false>
+template <int C, bool DENSE, bool WLDS, int MINW, bool RELU_IN, bool PIPE, bool BWD = false, bool PIECES = false, bool GATED = false>
 __global__ __launch_bounds__(kBlock, MINW) void s2v_level_stream_kernel(
     int N, const int* __restrict__ row_ptr, const int* __restrict__ col_idx, const float* __restrict__ val,
     const float* __restrict__ h_in, const float* __restrict__ W, const float* __restrict__ msg,
@@ -64,7 +64,7 @@ __global__ __launch_bounds__(kBlock, MINW) void s2v_level_stream_kernel(
     HubPlan hubs, float* __restrict__ agg_out = nullptr,
     float* __restrict__ acc_io = nullptr, PieceSums sums = PieceSums(), const int* __restrict__ gate = nullptr)
 {
-    if (gated_off(gate)) return;
+    if (gated_off<GATED>(gate)) return;
     constexpr int G = C / 4;             // lanes per gathered row
     constexpr int RPR = kWave / G;       // lane groups per wavefront
     constexpr int ROUNDS = 16 / RPR;     // rows per lane group
@@ -516,7 +516,9 @@ int launch_level_stream_p(int N, const int* row_ptr, const int* col_idx, const f
     constexpr int kMinW = (C == 64 && !DENSE) ? 3 : 4;    // hidden 64 needs 128 registers and spills for four
     const long long resident = (long long)kNumCU * kMinW;  // a workgroup puts one wavefront on each SIMD
     if (blocks > resident) blocks = resident;              // persistent beyond this
-    hipLaunchKernelGGL((s2v_level_stream_kernel<C, DENSE, kWLds, kMinW, RELU_IN, PIPE>), dim3((unsigned)blocks), dim3(kBlock), 0, s,
+    const auto kernel = !DENSE && gate ? &s2v_level_stream_kernel<C, DENSE, kWLds, kMinW, RELU_IN, PIPE, false, false, !DENSE>
+                                       : &s2v_level_stream_kernel<C, DENSE, kWLds, kMinW, RELU_IN, PIPE>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kBlock), 0, s,
                        N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs, (float*)nullptr, (float*)nullptr, PieceSums(), gate);
     GNNHIP_LAUNCH_CHECK("s2v_level_stream");
     return GNNHIP_OK;
