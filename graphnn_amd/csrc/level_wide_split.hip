@@ -475,6 +475,212 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_split_kernel(
     }
 }
 
+// The same over few rows at C = 256, where the kernel above is its start: a wavefront there splits 32 columns of W (3,300 vector
+// instructions) ahead of the first row, and all of a tile's matrix instructions are one compute unit's.  Here a workgroup takes 16 rows, a
+// wavefront sums two of them, and the workgroups of the grid's y share the columns: `blocks` wavefronts have 16 of them each, split while
+// the entries are on their way.  Row sums, pieces and products have the order of the kernel above, so every bit is its.
+// 286 rows 11.5 -> 7.5 us per level of a forward, backward 14.7 -> 8.3; 1,760 rows 12.0 -> 10.0 and 15.4 -> 11.2.  Over more than 2,048 rows a second
+// workgroup per compute unit would follow the first.  (Sixteen wavefronts, a row each, leave a lane 128 registers, of which W takes
+// 96: spilled, 13 to 32 us.)
+constexpr int kFewWaves = 8, kFewEach = 16 / kFewWaves;         // wavefronts, rows that each sums
+template <int C, bool RELU_IN, bool BWD>
+__global__ __launch_bounds__(kFewWaves * kWave) void s2v_level_split_few_kernel(
+    int N, int blocks, const int* __restrict__ row_ptr, const int* __restrict__ col_idx, const float* __restrict__ val,
+    const float* __restrict__ h_in, const float* __restrict__ W, const float* __restrict__ msg, float* __restrict__ h_out,
+    float* __restrict__ u_out, float* __restrict__ acc_io)
+{
+    constexpr int KS = C / 32, VEC = C / kWave, LDT = C / 2 + 8, kHalf = 16 * LDT, kPiece = 2 * kHalf, kFlight = 8;
+    static_assert(VEC == 4, "a wavefront holds a row as one 128-bit word per lane");
+    __shared__ __align__(16) unsigned short tile[3 * kPiece];    // [3 pieces][2 halves of the columns][16][LDT], as above
+    __shared__ float w_down[C];
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int q = lane >> 4, t = lane & 15;
+    const int row0 = blockIdx.x * 16, rows = min(16, N - row0);
+    const int col0 = 16 * (blockIdx.y * blocks + wave);
+    const bool live = wave < blocks && col0 < C;                 // uniform: this wavefront multiplies
+    const int k_lane = (q & 1) * (C / 2) + (q >> 1) * 8;         // contraction step s: k = k_lane + 16 s .. + 7
+    auto negated = [](int s) { return s >= KS / 4 && s < KS - KS / 4; };
+
+    // ---- what is asked for first: W, then this wavefront's row pointers and entries
+    float w[KS][8];
+    if (live) {
+        const rsrc_t w_rsrc = make_rsrc(W, (unsigned)(C * C * 4));
+        const int w_lane_off = BWD ? ((col0 + t) * C + k_lane) * 4 : (k_lane * C + col0 + t) * 4;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            if constexpr (BWD) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const float4 v = buf_load4(w_rsrc, w_lane_off, s * 64 + 16 * h);
+                    w[s][4 * h + 0] = v.x; w[s][4 * h + 1] = v.y; w[s][4 * h + 2] = v.z; w[s][4 * h + 3] = v.w;
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) w[s][i] = buf_load_f(w_rsrc, w_lane_off, (16 * s + i) * (C * 4));
+            }
+        }
+    }
+    // row 8 r + wave for r = 0, 1: an entry per lane
+    int start[kFewEach], end[kFewEach], c_lane[kFewEach];
+    float v_lane[kFewEach];
+    const rsrc_t h_rsrc = make_rsrc(h_in, (unsigned)N * (C * 4));
+#pragma unroll
+    for (int r = 0; r < kFewEach; ++r) {
+        const int row = min(r * kFewWaves + wave, rows);         // past the last row: no entries
+        start[r] = row_ptr[row0 + row];
+        end[r] = row_ptr[min(row0 + row + 1, row0 + rows)];
+    }
+    auto ask_entries = [&](int r, int base) {
+        const bool ok = base + lane < end[r];
+        c_lane[r] = ok ? col_idx[base + lane] : 0;
+        v_lane[r] = ok ? val[base + lane] : 0.f;
+    };
+#pragma unroll
+    for (int r = 0; r < kFewEach; ++r) ask_entries(r, start[r]);
+
+    // ---- W in pieces
+    bf16_words4 wreg[KS][3];
+    bool any_down = false;
+    if (live) {
+        float largest = 0.f;
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+#pragma unroll
+            for (int i = 0; i < 8; i += 2) largest = split_max(largest, w[s][i], w[s][i + 1]);
+        const unsigned long long large = __ballot(largest >= kSplitLarge);
+        const bool down = (large >> t) & 0x0001000100010001ull;  // in any quarter of the column
+        any_down = large != 0;
+        const float scale = down ? kSplitDown : kSplitUp;
+        if (q == 0) w_down[col0 + t] = down ? kSplitUp / kSplitDown : 1.f;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                unsigned p[3];
+                bf16_split2(w[s][2 * i] * scale, w[s][2 * i + 1] * scale, down, p);
+                const unsigned sign = negated(s) ? 0x80008000u : 0u;
+                wreg[s][0][i] = p[0] ^ sign; wreg[s][1][i] = p[1] ^ sign; wreg[s][2][i] = p[2] ^ sign;
+            }
+        }
+    }
+
+    // ---- the rows: the first entries of both, then the rest of each
+    float4 x[kFewEach][kFlight];
+    auto ask_rows = [&](int r, int e, int count) {
+#pragma unroll
+        for (int u = 0; u < kFlight; ++u) {
+            const int c = __builtin_amdgcn_readlane(c_lane[r], min(e + u, kWave - 1));
+            x[r][u] = buf_load4(h_rsrc, e + u < count ? lane * 16 : kBufPastEnd, c * (C * 4));
+        }
+    };
+#pragma unroll
+    for (int r = 0; r < kFewEach; ++r) ask_rows(r, 0, min(end[r] - start[r], kWave));
+#pragma unroll
+    for (int r = 0; r < kFewEach; ++r) {
+        float acc[VEC] = {0.f, 0.f, 0.f, 0.f};
+        for (int base = start[r]; base < end[r]; base += kWave) {            // uniform
+            const int count = min(end[r] - base, kWave);
+            if (base > start[r]) { ask_entries(r, base); ask_rows(r, 0, count); }
+            for (int e = 0; e < count; e += kFlight) {
+                if (e > 0) ask_rows(r, e, count);
+#pragma unroll
+                for (int u = 0; u < kFlight; ++u) {
+                    const float a = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v_lane[r]), min(e + u, kWave - 1)));
+                    if (e + u < count) vec_fma<VEC, RELU_IN>(acc, a, x[r][u]);
+                }
+            }
+        }
+        float largest = 0.f;
+#pragma unroll
+        for (int i = 0; i < VEC; i += 2) largest = split_max(largest, acc[i], acc[i + 1]);
+        const bool down = __any(largest >= kSplitLarge);
+        unsigned p[2][3];
+        const float scale = down ? kSplitDown : kSplitUp;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            if (down) bf16_split2(acc[2 * i] * scale, acc[2 * i + 1] * scale, true, p[i]);
+            else bf16_split2(acc[2 * i] * scale, acc[2 * i + 1] * scale, false, p[i]);
+        }
+        const int row = r * kFewWaves + wave;
+        unsigned short* dst = tile + (lane >> 5) * kHalf + row * LDT + (lane & 31) * VEC;
+        if (lane == 31) *reinterpret_cast<float*>(dst + VEC) = down ? kSplitDownBack : kSplitUpBack;     // behind the row's first half
+#pragma unroll
+        for (int j = 0; j < 3; ++j) *reinterpret_cast<uint2*>(dst + j * kPiece) = make_uint2(p[0][j], p[1][j]);
+        if constexpr (BWD) {
+            if (row < rows && blockIdx.y == 0)
+                *reinterpret_cast<float4*>(u_out + (size_t)(row0 + row) * C + lane * 4) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+        }
+    }
+    // what the epilogue reads: columns col0 + 4 q .. + 3 of row t (rows past N lie outside the descriptors)
+    const int off = ((row0 + t) * C + col0 + 4 * q) * 4;
+    const rsrc_t msg_rsrc = make_rsrc(msg, msg ? (unsigned)N * (C * 4) : 0u);
+    const rsrc_t acc_rsrc = make_rsrc(acc_io, BWD && acc_io ? (unsigned)N * (C * 4) : 0u);
+    float4 mm = f4_zero(), aa = f4_zero();
+    if (live) {
+        mm = buf_load4(msg_rsrc, off, 0);
+        if constexpr (BWD) aa = buf_load4(acc_rsrc, off, 0);
+    }
+    __syncthreads();
+    if (!live) return;                           // no barrier follows
+
+    // ---- products: the corrections first, negated steps ahead of the others, then those of the first pieces
+    const unsigned short* src = tile + (q & 1) * kHalf + t * LDT + (q >> 1) * 8;
+    auto piece = [&](int j, int step) { return *reinterpret_cast<const bf16_words4*>(src + j * kPiece + 16 * step); };
+    const float back = *reinterpret_cast<const float*>(tile + t * LDT + C / 2) * kSplitUpBack;
+    auto first_round = [&](int i) { return i < KS / 2 ? i + KS / 4 : i < 3 * KS / 4 ? i - KS / 2 : i; };
+    mfma_f4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < KS; ++i) {
+        const int s = first_round(i);
+        if (i == KS / 2) sum = -sum;
+#pragma unroll
+        for (int j = 2; j >= 0; --j) {
+            const bf16_words4 b = piece(j, s);
+#pragma unroll
+            for (int k = 2 - j; k >= (j == 0 ? 1 : 0); --k) sum = mfma_bf16(wreg[s][k], b, sum);
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+        if (s > 0 && negated(s) != negated(s - 1)) sum = -sum;
+        sum = mfma_bf16(wreg[s][0], piece(0, s), sum);
+    }
+    float4 f = make_float4(back, back, back, back);
+    if (any_down) {
+        const float4 d = *reinterpret_cast<const float4*>(w_down + col0 + 4 * q);
+        f.x *= d.x; f.y *= d.y; f.z *= d.z; f.w *= d.w;
+    }
+    if (t >= rows) return;
+    float* out = h_out + (size_t)(row0 + t) * C + col0 + 4 * q;
+    if constexpr (BWD) {
+        float4 v = make_float4(sum[0] * f.x, sum[1] * f.y, sum[2] * f.z, sum[3] * f.w);
+        if (msg) {
+            v.x = mm.x > 0.f ? v.x : 0.f; v.y = mm.y > 0.f ? v.y : 0.f;
+            v.z = mm.z > 0.f ? v.z : 0.f; v.w = mm.w > 0.f ? v.w : 0.f;
+        }
+        if (acc_io)
+            *reinterpret_cast<float4*>(acc_io + (size_t)(row0 + t) * C + col0 + 4 * q) = make_float4(aa.x + v.x, aa.y + v.y, aa.z + v.z, aa.w + v.w);
+        *reinterpret_cast<float4*>(out) = v;
+    } else {
+        const float4 v = make_float4(fmaf(sum[0], f.x, mm.x), fmaf(sum[1], f.y, mm.y), fmaf(sum[2], f.z, mm.z), fmaf(sum[3], f.w, mm.w));
+        *reinterpret_cast<float4*>(out) = make_float4(relu_ref(v.x), relu_ref(v.y), relu_ref(v.z), relu_ref(v.w));
+    }
+}
+
+template <int C, bool RELU_IN, bool BWD>
+int launch_level_split_few(int N, const int* row_ptr, const int* col_idx, const float* val, const float* h_in, const float* W,
+                           const float* msg, float* h_out, hipStream_t s, float* u_out = nullptr, float* acc_io = nullptr)
+{
+    const int tiles = (N + 15) / 16;
+    int share = C / 64;                          // four blocks of columns to a workgroup as long as there are compute units for it
+    while (share > 2 && share * tiles > kNumCU) share /= 2;              // a workgroup has eight wavefronts
+    hipLaunchKernelGGL((s2v_level_split_few_kernel<C, RELU_IN, BWD>), dim3(tiles, share), dim3(kFewWaves * kWave), 0, s, N, C / 16 / share, row_ptr, col_idx,
+                       val, h_in, W, msg, h_out, u_out, acc_io);
+    GNNHIP_LAUNCH_CHECK(BWD ? "s2v_level_split_few backward" : "s2v_level_split_few");
+    return GNNHIP_OK;
+}
+
 template <int C, int WAVES, bool RELU_IN, int TR, bool BWD = false>
 int launch_level_split_t(int N, const int* row_ptr, const int* col_idx, const float* val, const float* h_in,
                       const float* W, const float* msg, float* h_out, hipStream_t s, float* u_out = nullptr, float* acc_io = nullptr)
@@ -528,6 +734,9 @@ int level_split_dispatch(int N, int C, const int* row_ptr, const int* col_idx, c
         return relu_in ? launch_level_split<128, 8, true>(N, row_ptr, col_idx, val, h_in, W, msg, h_out, s)
                        : launch_level_split<128, 8, false>(N, row_ptr, col_idx, val, h_in, W, msg, h_out, s);
     case 256:
+        if (N <= kFewRows / 2)
+            return relu_in ? launch_level_split_few<256, true, false>(N, row_ptr, col_idx, val, h_in, W, msg, h_out, s)
+                           : launch_level_split_few<256, false, false>(N, row_ptr, col_idx, val, h_in, W, msg, h_out, s);
         return relu_in ? launch_level_split<256, 8, true>(N, row_ptr, col_idx, val, h_in, W, msg, h_out, s)
                        : launch_level_split<256, 8, false>(N, row_ptr, col_idx, val, h_in, W, msg, h_out, s);
     }
@@ -541,7 +750,9 @@ int level_split_backward_dispatch(int N, int C, const int* row_ptr, const int* c
 {
     switch (C) {
     case 128: return launch_level_split_backward<128, 8>(N, row_ptr, col_idx, val, dz, W, u, g_prev, gate, acc, s);
-    case 256: return launch_level_split_backward<256, 8>(N, row_ptr, col_idx, val, dz, W, u, g_prev, gate, acc, s);
+    case 256:
+        if (N <= kFewRows / 2) return launch_level_split_few<256, false, true>(N, row_ptr, col_idx, val, dz, W, gate, g_prev, s, u, acc);
+        return launch_level_split_backward<256, 8>(N, row_ptr, col_idx, val, dz, W, u, g_prev, gate, acc, s);
     }
     return GNNHIP_EUNSUPPORTED;
 }

@@ -2911,3 +2911,45 @@ def test_level_of_hidden_256_over_few_rows(gpu, oracle, N):
         got = _n(ops.s2v_level(*_csr_t(csr, gpu), _t(h_in, gpu), _t(W, gpu), _t(msg, gpu), None if b is None else _t(b, gpu)))
         assert_parity("level", got, want, w64)
         assert_condition("level", got, w64(), w64.cond())
+
+
+@pytest.mark.parametrize("N", [1, 15, 16, 33, 1024, 1025, 2048])
+def test_wide_levels_in_pieces_over_few_rows_have_the_bits_of_many(gpu, N):
+    """hidden 256, up to 2,048 rows (workgroups share the columns of 16 rows) against the same rows inside a matrix of more (another
+    kernel): a level of a forward and a backward level, rows of 0 to 300 entries, rows and columns of W that are scaled down before they
+    are split"""
+    import torch
+    from graphnn_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(N)
+    rand = lambda *shape: torch.randn(*shape, generator=gen, device=gpu)
+    C, K, big = 256, 8, 2100
+    deg = torch.randint(0, 10, (big,), generator=gen, device=gpu)
+    deg[torch.arange(0, N, 97)] = torch.tensor([64, 65, 8, 300], device=gpu).repeat(6)[:len(range(0, N, 97))]
+    rp = torch.zeros(big + 1, dtype=torch.int32, device=gpu)
+    rp[1:] = torch.cumsum(deg, 0)
+    ci = torch.randint(0, N, (int(rp[-1]),), generator=gen, device=gpu).int()
+    val = rand(int(rp[-1]))
+    E = int(rp[N])
+    few = (rp[:N + 1].contiguous(), ci[:E].contiguous(), val[:E].contiguous())
+    part = lambda t: t[:N].contiguous()
+    W = rand(C, C) * 0.1
+    for large in (False, True):
+        X = torch.zeros(big, K, device=gpu)
+        X[torch.arange(big, device=gpu), torch.randint(0, K, (big,), generator=gen, device=gpu)] = 1.0
+        dz, gate, acc = rand(big, C), rand(big, C), rand(big, C)
+        if large:
+            W[:, 17] *= 2.0 ** 40
+            W[3, :] *= 2.0 ** 39
+            X[N // 3] *= 2.0 ** 39
+            dz[N // 2] *= 2.0 ** 41
+        a_few, a_big = part(acc), acc.clone()
+        u, g = ops.s2v_level_backward(*few, part(dz), W, gate_h=part(gate), acc=a_few)
+        u2, g2 = ops.s2v_level_backward(rp, ci, val, dz, W, gate_h=gate, acc=a_big)
+        assert torch.equal(u, u2[:N]) and torch.equal(g, g2[:N]) and torch.equal(a_few, a_big[:N])
+        assert torch.equal(ops.s2v_level_backward(*few, part(dz), W)[1], ops.s2v_level_backward(rp, ci, val, dz, W)[1][:N])
+        Wn, w1, w2 = rand(K, C), torch.zeros(C, 4, device=gpu), torch.zeros(4, 2, device=gpu)
+        whole = lambda n: (torch.tensor([0, n], device=gpu).int(), torch.arange(n, device=gpu).int(), torch.ones(n, device=gpu))
+        for L in (1, 2):                                       # the first level reads ReLU(msg)
+            got = ops.s2v_forward(few, whole(N), part(X), Wn, W, w1, w2, L)
+            want = ops.s2v_forward((rp, ci, val), whole(big), X, Wn, W, w1, w2, L)
+            assert torch.equal(got.h_final, want.h_final[:N]), (L, large)
