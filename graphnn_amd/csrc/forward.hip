@@ -12,7 +12,7 @@ bool fused_hidden_supported(int C);
 int input_dispatch(int N, int K, int C, const float* X, const float* Wn2l, float* msg, float* h0, hipStream_t s, const int* gate);
 int level_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* h_in,
                    const float* W, const float* msg, const float* bias, float* h_out, hipStream_t s, bool same_graph = false,
-                   bool relu_in = false, CsrPlan* plan = nullptr, bool inference = false, const int* gate = nullptr);
+                   bool relu_in = false, CsrPlan* plan = nullptr, bool inference = false, const int* gate = nullptr, const MsgFactors& factors = MsgFactors());
 bool level_accepts_relu_input(int N, int C);
 int level_backward_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* dz,
                             const float* W, float* u, float* g_prev, const float* gate, float* acc, hipStream_t s);
@@ -96,9 +96,9 @@ int input_any(int N, int K, int C, const float* X, const float* Wn2l, float* msg
 
 int level_any(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* h_in,
               const float* W, const float* msg, const float* bias, float* h_out, hipStream_t s, bool same_graph = false,
-              bool relu_in = false, CsrPlan* plan = nullptr, bool inference = false, const int* gate = nullptr)
+              bool relu_in = false, CsrPlan* plan = nullptr, bool inference = false, const int* gate = nullptr, const MsgFactors& factors = MsgFactors())
 {
-    int rc = level_dispatch(N, C, nnz, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, s, same_graph, relu_in, plan, inference, gate);
+    int rc = level_dispatch(N, C, nnz, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, s, same_graph, relu_in, plan, inference, gate, factors);
     if (rc != GNNHIP_EUNSUPPORTED) return rc;
     rc = level_rows_dispatch(N, C, nnz, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, same_graph, relu_in, plan, s, gate);
     if (rc != GNNHIP_EUNSUPPORTED) return rc;
@@ -179,7 +179,7 @@ int forward_any(int N, int B, int K, int C, int H, int Q, int L, long long a_nnz
     float* nxt = lazy_h0 ? h_a : h_b;
     for (int lv = 0; lv < L; ++lv) {
         if ((rc = level_any(N, C, a_nnz, a_row_ptr, a_col_idx, a_val, cur, W_conv, msg, nullptr, nxt, s, lv > 0,
-                            lazy_h0 && lv == 0, plan, true, gate)))
+                            lazy_h0 && lv == 0, plan, true, gate, MsgFactors{X, W_n2l, K})))
             return rc;
         float* t = (cur == msg) ? h_b : cur;     // msg stays what it is; the other buffer takes the next level
         cur = nxt;

@@ -328,6 +328,12 @@ struct PieceSums {
     unsigned bytes = 0;                // of part; less than 4 GiB
     HubPlan hubs;                      // of the rows of more than kCombineLong pieces (a row's entries are its pieces)
 };
+// The factors of msg = X W_n2l, for a level that forms msg again instead of reading it (level_stream.hip)
+struct MsgFactors {
+    const float* X = nullptr;          // [N, K]; null: msg is read
+    const float* W = nullptr;          // [K, C]
+    int K = 0;
+};
 constexpr int kCombineLong = 8;        // pieces; the balanced pass sums the pieces of such rows
 int spmm_pieces_dispatch(int m, int k, int n, long long nnz, float alpha, const int* row_ptr, const int* col_idx, const float* val,
                          const float* B, int ldb, float beta, float* C, int ldc, hipStream_t s, bool reuse_plan,

@@ -43,7 +43,7 @@ int level_stream_backward_dispatch(int N, int C, const int* row_ptr, const int* 
                                    const float* W, float* agg_out, float* out, const float* gate, float* acc, const HubPlan& hubs,
                                    hipStream_t s);
 int level_stream_pieces_dispatch(int N, int C, const float* W, const float* msg, const float* bias, float* h_out, const PieceSums& sums,
-                                 hipStream_t s);
+                                 const MsgFactors& factors, hipStream_t s);
 // input_wide.hip
 int input_wide_dispatch(int N, int K, int C, const float* X, const float* Wn2l, float* msg, float* h0, hipStream_t s, const int* gate);
 // level_wide.hip
@@ -509,8 +509,9 @@ __global__ __launch_bounds__(kBlock) void identity_csr_kernel(int n, int* __rest
 
 int level_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* h_in,
                    const float* W, const float* msg, const float* bias, float* h_out, hipStream_t s, bool same_graph,
-                   bool relu_in, CsrPlan* plan, bool inference, const int* gate)
+                   bool relu_in, CsrPlan* plan, bool inference, const int* gate, const MsgFactors& factors)
 {
+    // factors: of msg, where the caller has them
     // inference: no gradient passes through the result, so its contraction may be rounded differently from the
     // contraction whose signs a backward pass relies on (level_wide_split.hip)
     // plan: made by gnnhip_csr_plan_create for exactly these CSR arrays (then nnz is the matrix's own count), or null
@@ -534,7 +535,7 @@ int level_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* c
             if (level_stream_covers(N, C)) {
                 PieceSums sums;
                 const int rc = spmm_pieces_dispatch(N, N, C, nnz, 1.f, row_ptr, col_idx, val, h_in, C, 0.f, h_out, C, s, same_graph, plan, relu_in, &sums);
-                if (rc == GNNHIP_OK) return level_stream_pieces_dispatch(N, C, W, msg, bias, h_out, sums, s);
+                if (rc == GNNHIP_OK) return level_stream_pieces_dispatch(N, C, W, msg, bias, h_out, sums, factors, s);
                 if (rc != GNNHIP_EUNSUPPORTED && rc != GNNHIP_ENOMEM) return rc;
             }
             if (int rc = spmm_dispatch(N, N, C, nnz, 1.f, row_ptr, col_idx, val, h_in, C, 0.f, h_out, C, s, same_graph, plan, relu_in)) return rc;

@@ -33,6 +33,10 @@
 // read.  Putting the rows together in a launch of its own cost 155 us per level on R-MAT with
 // 4M rows; here it adds 60 to the 545 us of the level.
 //
+// REMAKE (with PIECES): msg is not read but formed again from up to 16 feature columns, a quarter of the bytes at C = 64 and four matrix
+// instructions per block of columns, in the order of the input stage of C = 64 (input_wide.hip), whose bits it has.  4M rows, 16 columns: 610 ->
+// 482 us of a level of 2.4 ms.
+//
 // Algorithmic bytes: 4(N+1) + 8E + 12NC + 4C^2.
 #include "level_gather.h"
 
@@ -56,13 +60,14 @@ constexpr int kPipeMinRows = 65536;   // from here on the kernel variant that as
 // CSR matrix: W is read transposed, the aggregated rows A' x are also stored (agg_out: they are the other
 // factor of the weight gradient).  No ReLU and no bias; `msg`, when given, is the embedding whose ReLU the
 // gradient passes next: out = out where msg > 0, else 0, and acc_io (when given) += out.
-template <int C, bool DENSE, bool WLDS, int MINW, bool RELU_IN, bool PIPE, bool BWD = false, bool PIECES = false, bool GATED = false>
+template <int C, bool DENSE, bool WLDS, int MINW, bool RELU_IN, bool PIPE, bool BWD = false, bool PIECES = false, bool GATED = false,
+          bool REMAKE = false>
 __global__ __launch_bounds__(kBlock, MINW) void s2v_level_stream_kernel(
     int N, const int* __restrict__ row_ptr, const int* __restrict__ col_idx, const float* __restrict__ val,
     const float* __restrict__ h_in, const float* __restrict__ W, const float* __restrict__ msg,
     const float* __restrict__ bias, float* __restrict__ h_out,
     HubPlan hubs, float* __restrict__ agg_out = nullptr,
-    float* __restrict__ acc_io = nullptr, PieceSums sums = PieceSums(), const int* __restrict__ gate = nullptr)
+    float* __restrict__ acc_io = nullptr, PieceSums sums = PieceSums(), const int* __restrict__ gate = nullptr, MsgFactors factors = MsgFactors())
 {
     if (gated_off<GATED>(gate)) return;
     constexpr int G = C / 4;             // lanes per gathered row
@@ -77,7 +82,7 @@ __global__ __launch_bounds__(kBlock, MINW) void s2v_level_stream_kernel(
     constexpr int kBufEntries = (1 << 30) - 1;                                // entries of col_idx / val a buffer covers
     constexpr int kDirect = G >= 8 ? 8 : 4;                                   // entries per row taken without a loop
 
-    __shared__ float lds[kWavesPerBlock][16 * LDT + RPR * C];
+    __shared__ float lds[kWavesPerBlock][16 * LDT + (DENSE ? 0 : RPR * C)];
     __shared__ float4 wl[WLDS ? NJB * (KS / 4) * kWave : 1];
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
@@ -136,6 +141,19 @@ __global__ __launch_bounds__(kBlock, MINW) void s2v_level_stream_kernel(
     const rsrc_t h_rsrc = make_rsrc(h_in, act_bytes);
     const rsrc_t msg_rsrc = make_rsrc(msg, msg ? act_bytes : 0u);      // no msg: every load reads 0
     const rsrc_t out_rsrc = make_rsrc(h_out, act_bytes);
+
+    // REMAKE: the operand of W_n2l, wn[jb][s] = W_n2l[4 q + s][KS (t / 4) + 4 jb + t % 4], zeros from k = K on
+    __shared__ float4 wnl[REMAKE ? NJB * kWave : 1];
+    const rsrc_t x_rsrc = make_rsrc(factors.X, REMAKE ? (unsigned)N * (unsigned)factors.K * 4u : 0u);
+    if constexpr (REMAKE) {
+        const rsrc_t wn_rsrc = make_rsrc(factors.W, (unsigned)(factors.K * kRowBytes));
+        for (int jb = wave; jb < NJB; jb += kWavesPerBlock) {
+            const int off = (4 * q * C + KS * (t >> 2) + 4 * jb + (t & 3)) * 4;      // rows from K on lie past the end
+            wnl[jb * kWave + lane] = make_float4(buf_load_f(wn_rsrc, off, 0), buf_load_f(wn_rsrc, off + kRowBytes, 0),
+                                                 buf_load_f(wn_rsrc, off + 2 * kRowBytes, 0), buf_load_f(wn_rsrc, off + 3 * kRowBytes, 0));
+        }
+        __syncthreads();
+    }
 
     float4 bias4 = f4_zero();                // columns 4 tx .. 4 tx + 3
     if (bias) bias4 = *reinterpret_cast<const float4*>(bias + tx * 4);
@@ -429,9 +447,22 @@ __global__ __launch_bounds__(kBlock, MINW) void s2v_level_stream_kernel(
                 buf_store4(agg_rsrc, out_off + rd * kRowBytes, 0, *reinterpret_cast<const float4*>(tile + (grp * ROUNDS + rd) * LDT + tx * 4));
         }
         // msg is asked for once the gathered rows have left their registers; the contraction covers its trip
-        float4 mrow[ROUNDS];
+        float4 mrow[REMAKE ? 1 : ROUNDS];
+        if constexpr (REMAKE) {
+            // row t of X, columns 4 q .. + 3 (rows past N lie past the end)
+            const int K = factors.K, k = 4 * q, at = ((row0 + t) * K + k) * 4;
+            if (K % 4 == 0) {                    // uniform
+                mrow[0] = buf_load4(x_rsrc, k < K ? at : kBufPastEnd, 0);
+            } else {
+                mrow[0].x = buf_load_f(x_rsrc, k < K ? at : kBufPastEnd, 0);
+                mrow[0].y = buf_load_f(x_rsrc, k + 1 < K ? at + 4 : kBufPastEnd, 0);
+                mrow[0].z = buf_load_f(x_rsrc, k + 2 < K ? at + 8 : kBufPastEnd, 0);
+                mrow[0].w = buf_load_f(x_rsrc, k + 3 < K ? at + 12 : kBufPastEnd, 0);
+            }
+        } else {
 #pragma unroll
-        for (int rd = 0; rd < ROUNDS; ++rd) mrow[rd] = buf_load4(msg_rsrc, out_off + rd * kRowBytes, 0);
+            for (int rd = 0; rd < ROUNDS; ++rd) mrow[rd] = buf_load4(msg_rsrc, out_off + rd * kRowBytes, 0);
+        }
 
         // ---- contraction: lane (q, t) supplies tile[t][KS q + s] at step s
         float areg[KS];
@@ -460,6 +491,19 @@ __global__ __launch_bounds__(kBlock, MINW) void s2v_level_stream_kernel(
             }
         }
 
+        if constexpr (REMAKE) {
+#pragma unroll
+            for (int jb = 0; jb < NJB; ++jb) {
+                const float4 w4 = wnl[jb * kWave + lane];
+                mfma_f4 m = {0.f, 0.f, 0.f, 0.f};
+                m = __builtin_amdgcn_mfma_f32_16x16x4f32(w4.x, mrow[0].x, m, 0, 0, 0);
+                m = __builtin_amdgcn_mfma_f32_16x16x4f32(w4.y, mrow[0].y, m, 0, 0, 0);
+                m = __builtin_amdgcn_mfma_f32_16x16x4f32(w4.z, mrow[0].z, m, 0, 0, 0);
+                m = __builtin_amdgcn_mfma_f32_16x16x4f32(w4.w, mrow[0].w, m, 0, 0, 0);
+                acc[jb] += m;
+            }
+        }
+
         GNNHIP_PHASE_ACC(4);
         // ---- epilogue: the lane owns row t, columns KS q + 4 jb + {0..3}; the tile goes back through LDS so
         // that the lane group of a row holds it contiguously (256-byte requests instead of 16-byte pieces)
@@ -485,7 +529,7 @@ __global__ __launch_bounds__(kBlock, MINW) void s2v_level_stream_kernel(
                 buf_store4(out_rsrc, out_off + rd * kRowBytes, 0, v);
             } else {
                 if (bias) { v.x += bias4.x; v.y += bias4.y; v.z += bias4.z; v.w += bias4.w; }
-                v.x += mrow[rd].x; v.y += mrow[rd].y; v.z += mrow[rd].z; v.w += mrow[rd].w;
+                if constexpr (!REMAKE) { v.x += mrow[rd].x; v.y += mrow[rd].y; v.z += mrow[rd].z; v.w += mrow[rd].w; }
                 buf_store4(out_rsrc, out_off + rd * kRowBytes, 0, relu_ref4(v));
             }
         }
@@ -519,14 +563,15 @@ int launch_level_stream_p(int N, const int* row_ptr, const int* col_idx, const f
     const auto kernel = !DENSE && gate ? &s2v_level_stream_kernel<C, DENSE, kWLds, kMinW, RELU_IN, PIPE, false, false, !DENSE>
                                        : &s2v_level_stream_kernel<C, DENSE, kWLds, kMinW, RELU_IN, PIPE>;
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kBlock), 0, s,
-                       N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs, (float*)nullptr, (float*)nullptr, PieceSums(), gate);
+                       N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, hubs, (float*)nullptr, (float*)nullptr, PieceSums(), gate, MsgFactors());
     GNNHIP_LAUNCH_CHECK("s2v_level_stream");
     return GNNHIP_OK;
 }
 
 // The level over sums of pieces: h_out holds the rows of one piece.
 template <int C>
-int launch_level_stream_pieces(int N, const float* W, const float* msg, const float* bias, float* h_out, const PieceSums& sums, hipStream_t s)
+int launch_level_stream_pieces(int N, const float* W, const float* msg, const float* bias, float* h_out, const PieceSums& sums,
+                               const MsgFactors& factors, hipStream_t s)
 {
     const long long ntiles = ((long long)N + 15) / 16;
     long long blocks = (ntiles + kWavesPerBlock - 1) / kWavesPerBlock;
@@ -538,9 +583,13 @@ int launch_level_stream_pieces(int N, const float* W, const float* msg, const fl
     // 300,001 rows 478 us / 477, 1M 1,934 / 1,925, 4M 8,049 / 8,028.
     const long long resident = (long long)kNumCU * kMinW - 15;
     if (blocks > resident) blocks = resident;
-    hipLaunchKernelGGL((s2v_level_stream_kernel<C, true, C == 64, kMinW, false, false, false, true>), dim3((unsigned)blocks), dim3(kBlock), 0, s,
+    // msg from its factors where a row of X is at most half as long as one of msg
+    const bool remake = factors.X && !bias && factors.K >= 1 && factors.K <= 16 && 2 * factors.K <= C;
+    const auto kernel = remake ? &s2v_level_stream_kernel<C, true, C == 64, kMinW, false, false, false, true, false, true>
+                               : &s2v_level_stream_kernel<C, true, C == 64, kMinW, false, false, false, true>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kBlock), 0, s,
                        N, sums.first, (const int*)nullptr, (const float*)nullptr, (const float*)nullptr, W, msg, bias, h_out, HubPlan(),
-                       (float*)nullptr, (float*)nullptr, sums);
+                       (float*)nullptr, (float*)nullptr, sums, (const int*)nullptr, factors);
     GNNHIP_LAUNCH_CHECK("s2v_level_stream (pieces)");
     return GNNHIP_OK;
 }
@@ -582,7 +631,7 @@ int launch_level_stream_backward(int N, const int* row_ptr, const int* col_idx, 
     const long long resident = (long long)kNumCU * kMinW;
     if (blocks > resident) blocks = resident;
     hipLaunchKernelGGL((s2v_level_stream_kernel<C, false, kWLds, kMinW, false, false, true>), dim3((unsigned)blocks), dim3(kBlock), 0, s,
-                       N, row_ptr, col_idx, val, x, W, gate, (const float*)nullptr, out, hubs, agg_out, acc);
+                       N, row_ptr, col_idx, val, x, W, gate, (const float*)nullptr, out, hubs, agg_out, acc, PieceSums(), (const int*)nullptr, MsgFactors());
     GNNHIP_LAUNCH_CHECK("s2v_level_stream (backward)");
     return GNNHIP_OK;
 }
@@ -612,12 +661,12 @@ int level_stream_backward_dispatch(int N, int C, const int* row_ptr, const int* 
 
 // The level whose product left sums of pieces (spmm_pieces_dispatch with `sums`, into h_out); sums.ld must be C.
 int level_stream_pieces_dispatch(int N, int C, const float* W, const float* msg, const float* bias, float* h_out, const PieceSums& sums,
-                                 hipStream_t s)
+                                 const MsgFactors& factors, hipStream_t s)
 {
     switch (C) {
-    case 16: return launch_level_stream_pieces<16>(N, W, msg, bias, h_out, sums, s);
-    case 32: return launch_level_stream_pieces<32>(N, W, msg, bias, h_out, sums, s);
-    default: return launch_level_stream_pieces<64>(N, W, msg, bias, h_out, sums, s);
+    case 16: return launch_level_stream_pieces<16>(N, W, msg, bias, h_out, sums, factors, s);
+    case 32: return launch_level_stream_pieces<32>(N, W, msg, bias, h_out, sums, factors, s);
+    default: return launch_level_stream_pieces<64>(N, W, msg, bias, h_out, sums, factors, s);
     }
 }
 

@@ -2953,3 +2953,43 @@ def test_wide_levels_in_pieces_over_few_rows_have_the_bits_of_many(gpu, N):
             got = ops.s2v_forward(few, whole(N), part(X), Wn, W, w1, w2, L)
             want = ops.s2v_forward((rp, ci, val), whole(big), X, Wn, W, w1, w2, L)
             assert torch.equal(got.h_final, want.h_final[:N]), (L, large)
+
+
+@pytest.mark.parametrize("C,K", [(64, 16), (64, 13), (64, 4), (64, 1), (64, 17), (32, 16), (32, 7), (16, 8), (16, 9)])
+def test_forward_of_a_power_law_graph_forms_msg_again(gpu, C, K):
+    """levels of a graph of more than twelve entries per row whose contraction forms msg from up to sixteen feature columns instead of reading
+    it (17 columns, or 9 at hidden 16, are the other side of that): features that are no one-hot rows, against the levels called one by one
+    on the msg that the forward gives; rows without entries, of one piece and of many, a last tile of one row"""
+    import torch
+    from graphnn_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(C + K)
+    N, L = 32785, 3
+    deg = torch.randint(0, 45, (N,), generator=gen, device=gpu)
+    deg[::3] = 0
+    deg[torch.arange(5, N, 1000)] = 900
+    rp = torch.zeros(N + 1, dtype=torch.int32, device=gpu)
+    rp[1:] = torch.cumsum(deg, 0)
+    E = int(rp[-1])
+    assert E >= 12 * N
+    ci = torch.randint(0, N, (E,), generator=gen, device=gpu).int()
+    row = torch.repeat_interleave(torch.arange(N, device=gpu), deg)
+    val = (torch.rand(E, generator=gen, device=gpu) / deg[row]).contiguous()
+    normal = lambda *shape: torch.randn(*shape, generator=gen, device=gpu)
+    X, Wn, Wc, w1, w2 = normal(N, K), normal(K, C), normal(C, C) * (0.8 / C ** 0.5), torch.zeros(C, 4, device=gpu), torch.zeros(4, 2, device=gpu)
+    S = (torch.tensor([0, N], device=gpu).int(), torch.arange(N, device=gpu).int(), torch.ones(N, device=gpu))
+    got = ops.s2v_forward((rp, ci, val), S, X, Wn, Wc, w1, w2, L)
+    with ops.CsrPlan(rp, ci, val, N, N) as plan:
+        planned = ops.s2v_forward_planned(plan, S, X, Wn, Wc, w1, w2, L)
+    assert torch.equal(planned.h_final, got.h_final) and torch.equal(planned.msg, got.msg)
+    h = got.msg.clamp(min=0)
+    terms = X.double().abs() @ Wn.double().abs()
+    err = (K + 1) * 2.0 ** -24 * terms                         # the two sums that make msg
+    zero = torch.zeros(N, C, dtype=torch.float64, device=gpu)
+    agg = lambda t: zero.index_add(0, row, t[ci.long()] * val.double()[:, None])
+    for _ in range(L):
+        h = ops.s2v_level(rp, ci, val, h, Wc, got.msg)
+        terms, err = agg(terms) @ Wc.double().abs() + X.double().abs() @ Wn.double().abs(), agg(err) @ Wc.double().abs() + (K + 1) * 2.0 ** -24 * (X.double().abs() @ Wn.double().abs())
+    if C == 64:
+        assert torch.equal(got.h_final, h)                     # the input stage adds in the same order
+    else:                                                      # and every level rounds its own sums from there on
+        assert bool(((got.h_final.double() - h.double()).abs() <= err + L * (C + 900) * 2.0 ** -24 * terms).all())
