@@ -10,8 +10,9 @@
 //
 // Level by level such a batch is bound by memory: every level reads h and msg and writes h, 3.3 GB for 880,690 nodes at hidden 64.
 // Here the rows of a bin stay in LDS and msg in registers: X and the entries are read once, msg and the last h written once
-// (0.6 GB).  880,690 nodes, four levels, the whole forward: hidden 64 768 -> 443 us, hidden 32 419 -> 230; a level more 158 -> 55 and
-// 87 -> 30.
+// (0.6 GB), and the pooled rows S h are added up from LDS as well, where enough is read less for the launch that this takes (the
+// readout's own pass over h: 71 us of 444).  880,690 nodes, four levels, the whole forward: hidden 64 768 -> 403 us, hidden 32
+// 419 -> 226; a level more 158 -> 55 and 87 -> 30.
 //
 // A wavefront owns 16 or 32 rows and all their columns.  Lane (q = lane / 16, t = lane % 16) holds columns KS q .. KS q + KS - 1 of
 // row t, in every role: it sums that part of the row's neighbours straight into the operand registers of the matrix
@@ -29,7 +30,7 @@
 // Hidden sizes from 17 to 112 without kernels of their own take the next multiple of 16, with zeros behind the last column, and msg from
 // memory (the general input stage).  Above 64 W lies in LDS in all three pieces (86 KB at 112) and a workgroup fills a compute unit:
 // its wavefronts wait for the same things at the same time, and a level of 16 rows reads all of W.  44,000 nodes, hidden 100, 3.8
-// entries per row: a level 28 -> 16 us, the forward of three 110 -> 97; 176,000 nodes, four levels 416 -> 285; error against float64
+// entries per row: a level 28 -> 15 us, the forward of three 111 -> 92; 176,000 nodes, four levels 416 -> 250; error against float64
 // 6.7e-11, was 1.4e-10.  Above 112 columns W and the rows of 128 nodes do not fit the LDS together.  Tried there: the wavefronts share
 // the columns, as in level_wide_split.hip, and the rows are put into pieces in place between two barriers: 7.5 us for a bin of 112
 // nodes and a level at hidden 128, where the level-by-level route takes as long, and at hidden 256, where 64 nodes fit, 1.5 times that.
@@ -71,15 +72,16 @@ template <int CP, int KSX>
 constexpr size_t batch_lds_bytes()
 {
     return sizeof(float) * (size_t)(kRows + 1) * (CP + 4) + sizeof(bf16_words4) * w_lds_words<CP>() + (BatchShape<CP>::PIECES ? sizeof(float) * CP : 0) +
-           sizeof(float) * (size_t)(CP / 16) * KSX * kWave + sizeof(int2) * kEdgeCap + sizeof(int) * (kRows + 4);
+           sizeof(float) * (size_t)(CP / 16) * KSX * kWave + sizeof(int2) * (kEdgeCap + kRows) + sizeof(int) * (kRows + 4 + kWave + 4);
 }
 
 // KSX: contraction steps of the input stage, K <= 4 KSX, and the hidden size is CP; 0: msg is there, and the hidden size is C <= CP
 template <int CP, int KSX>
 __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) void s2v_batch_levels_kernel(
     int N, int B, int K, int hidden, int L, const int* __restrict__ a_row_ptr, const int* __restrict__ a_col_idx, const float* __restrict__ a_val,
-    const float* __restrict__ X, const float* __restrict__ Wn2l, const float* __restrict__ Wc, float* __restrict__ msg,
-    float* __restrict__ h_out, const int* __restrict__ bins, int* __restrict__ refused)
+    const int* __restrict__ s_row_ptr, const int* __restrict__ s_col_idx, const float* __restrict__ s_val, const float* __restrict__ X,
+    const float* __restrict__ Wn2l, const float* __restrict__ Wc, float* __restrict__ msg, float* __restrict__ h_out,
+    float* __restrict__ pool, const int* __restrict__ bins, int* __restrict__ refused)
 {
     using Shape = BatchShape<CP>;
     constexpr int TPW = Shape::TPW, kWaves = batch_waves<CP>(), kBlock = kWaves * kWave;
@@ -89,6 +91,7 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
     constexpr int NJB = CP / 16;                 // output blocks of 16 columns
     constexpr int LD = CP + 4;
     const int C = INPUT ? CP : hidden;
+    const bool pooled = CP > 16 && pool;
     static_assert(!PIECES || !WREG || KS2 == 2, "two sums of opposite signs");
     extern __shared__ float4 smem4[];
     float* hbuf = reinterpret_cast<float*>(smem4);                         // [kRows + 1][LD], the last row zeros
@@ -96,7 +99,9 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
     float* w_down = reinterpret_cast<float*>(w_lds + w_lds_words<CP>());   // [CP] a column's scale up over its scale
     float2* wn = reinterpret_cast<float2*>(w_down + (PIECES ? CP : 0));    // [NJB][KSX / 2][lane]
     int2* edges = reinterpret_cast<int2*>(wn + NJB * (KSX / 2) * kWave);   // [kEdgeCap] row offset, weight
-    int* rp = reinterpret_cast<int*>(edges + kEdgeCap);                    // [kRows + 1], from the bin's first entry on
+    int2* members = edges + kEdgeCap;                                      // [kRows] row offset, weight: entries of S
+    int* rp = reinterpret_cast<int*>(members + kRows);                     // [kRows + 1], from the bin's first entry on
+    int* sp = rp + kRows + 4;                                              // [kWave + 1] the same of S
     __shared__ int stop;                         // another workgroup has come upon an entry that leaves its bin
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int q = lane >> 4, t = lane & 15;
@@ -177,16 +182,18 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
     any_down = __syncthreads_or(any_down);
 
     // ---- what a bin needs from memory, asked for together and a bin ahead
-    struct Bin { int node0, n, e0, ne; };
+    struct Bin { int node0, n, e0, ne, g0, ng; };
     auto record = [&](int at) {
         const int* rec = bins + bin_words_ints(B) + (size_t)max(at, 0) * kOrderRec;
         const int4 r = *reinterpret_cast<const int4*>(rec);
-        return at < 0 ? Bin{0, 0, 0, 0} : Bin{r.y, r.z, r.w, max(rec[4] - r.w, 0)};
+        const int2 r2 = *reinterpret_cast<const int2*>(rec + 4);
+        return at < 0 ? Bin{0, 0, 0, 0, 0, 0} : Bin{r.y, r.z, r.w, max(r2.x - r.w, 0), r.x, r2.y};
     };
     constexpr int kEdgesEach = kEdgeCap / kBlock;
     float x[TPW][INPUT ? KSX : 1], e_val[kEdgesEach];
     float4 mx[TPW][INPUT ? 1 : NJB];             // rows of msg where they are there already
-    int e_col[kEdgesEach], rp_v;
+    int e_col[kEdgesEach], rp_v, sp_v, s_col;
+    float s_w;
     auto ask = [&](const Bin& b) {
         // (every register is written whatever the bin is, or the old values would have to be kept through the levels)
 #pragma unroll
@@ -218,6 +225,9 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
             }
         }
         rp_v = a_row_ptr[b.node0 + min(tid, b.n)];
+        sp_v = pooled ? s_row_ptr[b.g0 + min(tid, b.ng)] : 0;
+        s_col = pooled && tid < b.n ? s_col_idx[b.node0 + tid] : b.node0;    // (graph g's entries of S are numbered as its nodes are)
+        s_w = pooled && tid < b.n ? s_val[b.node0 + tid] : 0.f;
         const int in_lds = b.ne <= kEdgeCap ? b.ne : 0;
 #pragma unroll
         for (int u = 0; u < kEdgesEach; ++u) {
@@ -232,7 +242,7 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
 
     for (int bin = blockIdx.x; more && !stop; bin += gridDim.x) {
         // (the same in all wavefronts: stop is written between two barriers that this test does not lie between)
-        const int node0 = cur.node0, n = cur.n, e0 = cur.e0, ne = cur.ne;
+        const int node0 = cur.node0, n = cur.n, e0 = cur.e0, ne = cur.ne, g0 = cur.g0, ng = cur.ng;
         const bool staged = ne <= kEdgeCap;
         const int tiles = min(max((n + 15) / 16 - TPW * wave, 0), TPW);    // of this wavefront: uniform
         if (tid <= n) rp[tid] = rp_v - e0;
@@ -280,6 +290,12 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
             }
         }
         __syncthreads();                         // the last bin's rows have left hbuf; rp and edges are there
+        if (pooled && tid < n) {
+            const int c = s_col - node0;
+            if (c < 0 || c >= n) *refused = 1;
+            members[tid] = make_int2(min(max(c, 0), n - 1) * LD, __float_as_int(s_w));
+        }
+        if (pooled && tid <= ng) sp[tid] = sp_v - node0;
         float* own = hbuf + row0 * LD + KS * q;
         int g_st[TPW], g_en[TPW], g_off[TPW][kDirect];
         float g_w[TPW][kDirect];
@@ -299,8 +315,12 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
             }
         }
         __syncthreads();
+        // (what follows from these is not kept through the levels)
+        auto lane_now = [&]() { int l = lane; asm("" : "+v"(l)); return l; };
+        auto tid_now = [&]() { int l = tid; asm("" : "+v"(l)); return l; };
         // the bin's rows as they lie in memory: whole lines
         auto copy_out = [&](float* dst) {
+            const int tid = tid_now();
             if constexpr (INPUT) {
                 for (int i = tid; i < n * KS; i += kBlock)
                     *reinterpret_cast<float4*>(dst + (size_t)node0 * C + 4 * i) = *reinterpret_cast<const float4*>(hbuf + (i / KS) * LD + 4 * (i % KS));
@@ -479,6 +499,43 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
             level(std::false_type(), std::true_type());
         }
         copy_out(h_out);
+        // pool = S h: a wavefront per graph, kLanes lanes per row
+        if (pooled) {
+            constexpr int kLanes = KS <= 4 ? 4 : KS <= 8 ? 8 : KS <= 16 ? 16 : 32, kApart = kWave / kLanes;
+            const int l = lane_now();
+            const int col = 4 * (l % kLanes);
+            for (int g = wave; g < ng; g += kWaves) {
+                const int end = min(sp[g + 1], n);
+                float4 sum = f4_zero();
+                for (int r = sp[g] + l / kLanes; r < end; r += 4 * kApart) {
+                    int2 of[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        of[u] = members[min(r + u * kApart, kRows - 1)];
+                        if (r + u * kApart >= end) of[u] = make_int2(kRows * LD, 0);
+                    }
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        if (kLanes == KS || col < CP) f4_fma(sum, __int_as_float(of[u].y), *reinterpret_cast<const float4*>(hbuf + of[u].x + col));
+                }
+#pragma unroll
+                for (int d = kLanes; d < kWave; d <<= 1)
+                    sum = ColsWide::add(sum, make_float4(__shfl_xor(sum.x, d, kWave), __shfl_xor(sum.y, d, kWave), __shfl_xor(sum.z, d, kWave),
+                                                         __shfl_xor(sum.w, d, kWave)));
+                float* to = pool + (size_t)(g0 + g) * C + col;
+                if (l < kLanes && col < C) {
+                    if (INPUT) {
+                        *reinterpret_cast<float4*>(to) = sum;
+                    } else if (col + 4 <= C) {
+                        ColsLoose::store(to, sum);
+                    } else {
+                        to[0] = sum.x;
+                        if (col + 1 < C) to[1] = sum.y;
+                        if (col + 2 < C) to[2] = sum.z;
+                    }
+                }
+            }
+        }
         cur = next;
     }
     // a segment that was not packed: every workgroup comes by all words
@@ -486,8 +543,9 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
 }
 
 template <int CP, int KSX>
-int launch_batch_levels(int N, int B, int K, int C, int L, const int* a_row_ptr, const int* a_col_idx, const float* a_val, const float* X,
-                        const float* Wn2l, const float* Wc, float* msg, float* h_out, const int* bins, int* refused, int cap, hipStream_t s)
+int launch_batch_levels(int N, int B, int K, int C, int L, const int* a_row_ptr, const int* a_col_idx, const float* a_val, const int* s_row_ptr,
+                        const int* s_col_idx, const float* s_val, const float* X, const float* Wn2l, const float* Wc, float* msg, float* h_out,
+                        float* pool, const int* bins, int* refused, int cap, hipStream_t s)
 {
     constexpr size_t smem = batch_lds_bytes<CP, KSX>();
     constexpr int kWaves = batch_waves<CP>();
@@ -500,7 +558,7 @@ int launch_batch_levels(int N, int B, int K, int C, int L, const int* a_row_ptr,
     const long long resident = (long long)kNumCU * (BatchShape<CP>::MINW * 4 / kWaves);
     const unsigned grid = (unsigned)(most < resident ? most : resident);
     hipLaunchKernelGGL((s2v_batch_levels_kernel<CP, KSX>), dim3(grid), dim3(kWaves * kWave), smem, s, N, B, K, C, L, a_row_ptr, a_col_idx, a_val,
-                       X, Wn2l, Wc, msg, h_out, bins, refused);
+                       s_row_ptr, s_col_idx, s_val, X, Wn2l, Wc, msg, h_out, pool, bins, refused);
     GNNHIP_LAUNCH_CHECK("s2v_batch_levels");
     return GNNHIP_OK;
 }
@@ -512,14 +570,20 @@ constexpr int kTwoStepMeanDegree = 12;           // denser matrices take the SpM
 // whether batch_levels_dispatch forms msg itself; else it is to be there
 bool batch_levels_with_input(int K, int C) { return K >= 2 && K <= 64 && (C == 16 || C == 32 || C == 64); }
 
-size_t batch_levels_work_ints(int B) { return kOrderRec + bin_ints(B); }
+size_t batch_levels_work_ints(int B) { return bin_ints(B); }
 
-// The last level's h (and msg) of a batch of small graphs.  work: at least batch_levels_work_ints(B) ints, 16-byte aligned.  *refused: the
-// device word that says (1) that the batch is none and the outputs have to be formed by the level-by-level route.
+// whether batch_levels_dispatch forms the pooled rows too: the readout reads h otherwise, but needs a launch less (hidden 100, 44,000
+// nodes 93 us, 96 with them, 88,000 135 and 138, 176,000 218 and 212, 352,000 405 and 390; hidden 64 of 9 features, 73,000 nodes 73 and 70; hidden
+// 50, 88,000 nodes 87 and 85; hidden 32, 73,000 nodes 51 and 50, 294,000 82 and 78; hidden 16 587,000 nodes 92 and 92, of 60 features 142 and 146)
+bool batch_levels_with_pool(int N, int C) { return C > 16 && (long long)N * C >= (C > 64 ? 12000000 : 4000000); }
+
+// The last level's h and, unless pool is null, the pooled rows (and msg) of a batch of small graphs.  work: at least batch_levels_work_ints(B) ints, 16-byte
+// aligned, free once the launches are done.  *refused: the device word that says (1) that the batch is none and the outputs have to be
+// formed by the level-by-level route.
 // GNNHIP_EUNSUPPORTED (nothing launched): sizes that this route does not take.
 int batch_levels_dispatch(int N, int B, int K, int C, int L, long long nnz, const int* a_row_ptr, const int* a_col_idx, const float* a_val,
-                          const int* s_row_ptr, const float* X, const float* Wn2l, const float* Wc, float* msg, float* h_out, int* work,
-                          const int** refused, hipStream_t s)
+                          const int* s_row_ptr, const int* s_col_idx, const float* s_val, const float* X, const float* Wn2l, const float* Wc,
+                          float* msg, float* h_out, float* pool, int* work, int* refused, hipStream_t s)
 {
     // What the levels but the first save is reading h and msg and writing h.  Below these products the launches of both routes cost more
     // than that (hidden 64, 35,000 nodes: two levels 52 us against 48, three 59 against 62; hidden 32, 73,000 nodes: one level 35.6 against
@@ -538,13 +602,12 @@ int batch_levels_dispatch(int N, int B, int K, int C, int L, long long nnz, cons
         const double cost = (double)((long long)(nbins / slots) + 1) * (2.0 + c / 16);
         if (c == kRows || cost < best) { best = cost; cap = c; }
     }
-    int* word = work;
-    int* bins = work + kOrderRec;
+    int* bins = work;
     hipLaunchKernelGGL((graph_bins_kernel<true>), dim3(ceil_div_u((size_t)B, kBinBlock)), dim3(kBinBlock), 0, s, B, cap, a_row_ptr, s_row_ptr,
-                       bins, N, word, kRows);
+                       bins, N, refused, kRows);
     GNNHIP_LAUNCH_CHECK("graph_bins");
-    *refused = word;
-#define GNNHIP_BL(CP, KSX) launch_batch_levels<CP, KSX>(N, B, K, C, L, a_row_ptr, a_col_idx, a_val, X, Wn2l, Wc, msg, h_out, bins, word, cap, s)
+#define GNNHIP_BL(CP, KSX) launch_batch_levels<CP, KSX>(N, B, K, C, L, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx, s_val, X, Wn2l, Wc, msg, h_out, \
+                                                pool, bins, refused, cap, s)
     if (batch_levels_with_input(K, C)) {
 #define GNNHIP_BL_K(CP) (K <= 16 ? GNNHIP_BL(CP, 4) : K <= 32 ? GNNHIP_BL(CP, 8) : K <= 48 ? GNNHIP_BL(CP, 12) : GNNHIP_BL(CP, 16))
         return C == 16 ? GNNHIP_BL_K(16) : C == 32 ? GNNHIP_BL_K(32) : GNNHIP_BL_K(64);

@@ -19,9 +19,10 @@ int level_backward_dispatch(int N, int C, long long nnz, const int* row_ptr, con
 // batch_forward.hip
 size_t batch_levels_work_ints(int B);
 bool batch_levels_with_input(int K, int C);
+bool batch_levels_with_pool(int N, int C);
 int batch_levels_dispatch(int N, int B, int K, int C, int L, long long nnz, const int* a_row_ptr, const int* a_col_idx, const float* a_val,
-                          const int* s_row_ptr, const float* X, const float* Wn2l, const float* Wc, float* msg, float* h_out, int* work,
-                          const int** refused, hipStream_t s);
+                          const int* s_row_ptr, const int* s_col_idx, const float* s_val, const float* X, const float* Wn2l, const float* Wc,
+                          float* msg, float* h_out, float* pool, int* work, int* refused, hipStream_t s);
 // level_rows.hip
 int level_rows_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* h_in,
                         const float* W, const float* msg, const float* bias, float* h_out, bool same_graph, bool relu_in, CsrPlan* plan,
@@ -32,6 +33,10 @@ int level_rows_dense_dispatch(int N, int K, int n, const float* x, const float* 
                               bool relu, float* relu_out, hipStream_t s);
 int readout_rows_dispatch(int B, int N, int C, int H, int Q, const int* s_row_ptr, const int* s_col_idx, const float* s_val, const float* h,
                           const float* Wh1, const float* Wh2, float* pool, float* hidden, float* logits, float* probs, int* pred, hipStream_t s);
+bool readout_gated_accepts(int C, int H, int Q);
+int readout_gated_dispatch(int B, int C, int H, int Q, bool wave, const int* s_row_ptr, const int* s_col_idx, const float* s_val, const float* h,
+                           const float* Wh1, const float* Wh2, float* pool, float* hidden, float* logits, float* probs, int* pred,
+                           hipStream_t s, const int* gate);
 int readout_wave_dispatch(int B, int C, int H, int Q, const int* s_row_ptr, const int* s_col_idx, const float* s_val,
                           const float* h, const float* Wh1, const float* Wh2, float* pool, float* hidden,
                           float* logits, float* probs, int* pred, hipStream_t s);
@@ -121,13 +126,15 @@ constexpr int kTileReadoutMinGraphs = 4096;        // hidden 128/256
 
 int readout_any(int B, int N, int C, int H, int Q, const int* s_row_ptr, const int* s_col_idx, const float* s_val,
                 const float* h, const float* Wh1, const float* Wh2, float* pool, float* hidden,
-                float* logits, float* probs, int* pred, hipStream_t s)
+                float* logits, float* probs, int* pred, hipStream_t s, const int* gate = nullptr)
 {
     // Many graphs of moderate size: one wavefront per graph (30,000 graphs of 29 nodes, hidden 64: 78 us with
     // a workgroup per graph).  Few graphs, and graphs of thousands of nodes: a workgroup per graph reaches more
     // of the chip.
     int rc = GNNHIP_EUNSUPPORTED;
-    if (B >= kWaveReadoutMinGraphs && (long long)N <= (long long)B * kWaveReadoutMaxMeanNodes)
+    const bool wave = B >= kWaveReadoutMinGraphs && (long long)N <= (long long)B * kWaveReadoutMaxMeanNodes;
+    if (gate) return readout_gated_dispatch(B, C, H, Q, wave, s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2, pool, hidden, logits, probs, pred, s, gate);
+    if (wave)
         rc = readout_wave_dispatch(B, C, H, Q, s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2, pool, hidden, logits, probs, pred, s);
     if (rc != GNNHIP_EUNSUPPORTED) return rc;
     // hidden 128/256: a workgroup per graph up to a few thousand graphs, then a tile of graphs per workgroup
@@ -160,15 +167,19 @@ int forward_any(int N, int B, int K, int C, int H, int Q, int L, long long a_nnz
     // (the routes of the other sizes can too)
     const bool lazy_h0 = L >= 1 && (level_accepts_relu_input(N, C) || !fused_hidden_supported(C)) && aligned16(msg) && aligned16(h_a) && aligned16(h_b) && aligned16(W_conv);
     // Batches of small graphs: levels in one launch (the input stage too where the hidden size has such a kernel), which finds out on the
-    // device whether the batch is one; what it needs for that lies in pool, which is written last.  The level-by-level launches
-    // behind it do nothing if it is.
+    // device whether the batch is one, and may add up the pooled rows.  The level-by-level launches behind it do nothing if it is.  What it
+    // needs for that lies in the other embedding, which nothing else writes then, and, as the later launches ask for it, the word that
+    // they go by in hidden, which is written by the last one.
     const int* gate = nullptr;
-    const bool try_batch = lazy_h0 && aligned16(pool) && batch_levels_work_ints(B) <= (size_t)B * C;
-    const bool with_input = batch_levels_with_input(K, C);
+    const bool try_batch = lazy_h0 && aligned16(pool) && batch_levels_work_ints(B) <= (size_t)N * C;
+    const bool with_input = batch_levels_with_input(K, C), with_pool = batch_levels_with_pool(N, C) && readout_gated_accepts(C, H, Q);
     auto batch_levels = [&]() {
-        const int rc = try_batch ? batch_levels_dispatch(N, B, K, C, L, a_nnz, a_row_ptr, a_col_idx, a_val, s_row_ptr, X, W_n2l, W_conv, msg,
-                                                         (L & 1) ? h_a : h_b, reinterpret_cast<int*>(pool), &gate, s)
-                                 : GNNHIP_OK;
+        int rc = GNNHIP_EUNSUPPORTED;
+        int* refused = reinterpret_cast<int*>(hidden);
+        if (try_batch)
+            rc = batch_levels_dispatch(N, B, K, C, L, a_nnz, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx, s_val, X, W_n2l, W_conv, msg,
+                                       (L & 1) ? h_a : h_b, with_pool ? pool : nullptr, reinterpret_cast<int*>((L & 1) ? h_b : h_a), refused, s);
+        if (rc == GNNHIP_OK) gate = refused;
         return rc == GNNHIP_EUNSUPPORTED ? GNNHIP_OK : rc;
     };
     int rc;
@@ -186,7 +197,7 @@ int forward_any(int N, int B, int K, int C, int H, int Q, int L, long long a_nnz
         nxt = t;
     }
     if (which_h) *which_h = (cur == h_a) ? 0 : 1;
-    return readout_any(B, N, C, H, Q, s_row_ptr, s_col_idx, s_val, cur, W_h1, W_h2, pool, hidden, logits, probs, pred, s);
+    return readout_any(B, N, C, H, Q, s_row_ptr, s_col_idx, s_val, cur, W_h1, W_h2, pool, hidden, logits, probs, pred, s, with_pool ? gate : nullptr);
 }
 
 }  // namespace

@@ -25,13 +25,15 @@ constexpr int kBlock = 256;
 constexpr int kWavesPerBlock = kBlock / kWave;
 constexpr int kMaxLds = 150 * 1024;
 
-template <int C>
+// POOL: the pooled rows alone, of a gated launch
+template <int C, bool POOL>
 __global__ __launch_bounds__(kBlock) void s2v_readout_wave_kernel(
     int B, int H, int Q, const int* __restrict__ s_row_ptr, const int* __restrict__ s_col_idx,
     const float* __restrict__ s_val, const float* __restrict__ h, const float* __restrict__ Wh1,
     const float* __restrict__ Wh2, float* __restrict__ pool, float* __restrict__ hidden,
-    float* __restrict__ logits, float* __restrict__ probs, int* __restrict__ pred)
+    float* __restrict__ logits, float* __restrict__ probs, int* __restrict__ pred, const int* __restrict__ gate)
 {
+    if (gated_off<POOL>(gate)) return;
     constexpr int G = C / 4;             // lanes per row of h
     constexpr int RPR = kWave / G;       // rows in flight per step of the wavefront
     extern __shared__ float smem[];
@@ -78,6 +80,7 @@ __global__ __launch_bounds__(kBlock) void s2v_readout_wave_kernel(
             pool[(size_t)g * C + cc] = s;
         }
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        if constexpr (POOL) continue;
         // ---- hidden = ReLU(pool * W_h1)
         for (int j = lane; j < H; j += kWave) {
             float s = 0.f;
@@ -128,15 +131,15 @@ __global__ __launch_bounds__(kBlock) void s2v_readout_wave_kernel(
     }
 }
 
-template <int C>
+template <int C, bool POOL = false>
 int launch_readout_wave(int B, int H, int Q, const int* s_row_ptr, const int* s_col_idx, const float* s_val,
                         const float* h, const float* Wh1, const float* Wh2, float* pool, float* hidden,
-                        float* logits, float* probs, int* pred, hipStream_t s)
+                        float* logits, float* probs, int* pred, hipStream_t s, const int* gate = nullptr)
 {
     constexpr int RPR = kWave / (C / 4);
     const size_t smem = sizeof(float) * ((size_t)C * H + (size_t)H * Q + (size_t)kWavesPerBlock * (RPR * C + C + H + Q));
     if (smem > (size_t)kMaxLds) return GNNHIP_EUNSUPPORTED;
-    auto kernel = s2v_readout_wave_kernel<C>;
+    auto kernel = s2v_readout_wave_kernel<C, POOL>;
     static LdsLimit lds_limit;               // one per kernel instantiation
     GNNHIP_HIP(lds_limit.raise(reinterpret_cast<const void*>(kernel), smem > 64 * 1024 ? (size_t)kMaxLds : smem));
     const long long blocks_needed = ((long long)B + kWavesPerBlock - 1) / kWavesPerBlock;
@@ -144,7 +147,7 @@ int launch_readout_wave(int B, int H, int Q, const int* s_row_ptr, const int* s_
     long long cap = (long long)kNumCU * (per_cu < 1 ? 1 : (per_cu > 8 ? 8 : per_cu));
     const unsigned grid = (unsigned)(blocks_needed < cap ? blocks_needed : cap);
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBlock), smem, s, B, H, Q, s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2,
-                       pool, hidden, logits, probs, pred);
+                       pool, hidden, logits, probs, pred, gate);
     GNNHIP_LAUNCH_CHECK("s2v_readout_wave");
     return GNNHIP_OK;
 }
@@ -322,12 +325,13 @@ int launch_readout_tile(int B, int H, int Q, const int* s_row_ptr, const int* s_
 // MINW: wavefronts per SIMD that the registers have to leave room for, 0: none asked for.  Only the variant with three rows in flight asks:
 // where it does not change their number, asking only makes the compiler wait for each load by itself (a wavefront per graph, five
 // asked for, which the kernel has anyway: 2,048 graphs of 24 nodes, hidden 160 16.1 -> 30.1 us, 256 21.6 -> 47.6).
-template <int TG, int BLOCK, int MINW, int FLIGHT>
+template <int TG, int BLOCK, int MINW, int FLIGHT, bool POOL>
 __global__ __launch_bounds__(BLOCK, MINW) void s2v_readout_rows_kernel(
     int B, int C, int H, int Q, const int* __restrict__ s_row_ptr, const int* __restrict__ s_col_idx, const float* __restrict__ s_val,
     const float* __restrict__ h, const float* __restrict__ Wh1, const float* __restrict__ Wh2, float* __restrict__ pool,
-    float* __restrict__ hidden, float* __restrict__ logits, float* __restrict__ probs, int* __restrict__ pred)
+    float* __restrict__ hidden, float* __restrict__ logits, float* __restrict__ probs, int* __restrict__ pred, const int* __restrict__ gate)
 {
+    if (gated_off<POOL>(gate)) return;
     using V = ColsLoose;
     constexpr int LG = BLOCK / TG, WG = LG / kWave;      // lanes and wavefronts per graph
     constexpr int kFlight = FLIGHT;
@@ -379,6 +383,7 @@ __global__ __launch_bounds__(BLOCK, MINW) void s2v_readout_rows_kernel(
             if (own) V::store(pool + (size_t)g * C + V::at(lane, C), s);
         }
         __syncthreads();
+        if constexpr (POOL) continue;
         // ---- hidden = ReLU(pool * W_h1)
         const int share = (C + WG - 1) / WG, c_lo = min(w * share, C), c_hi = min(c_lo + share, C);
         for (int j = lane; j < H; j += kWave) {
@@ -438,18 +443,142 @@ __global__ __launch_bounds__(BLOCK, MINW) void s2v_readout_rows_kernel(
     }
 }
 
-template <int TG, int BLOCK, int MINW, int FLIGHT>
+template <int TG, int BLOCK, int MINW, int FLIGHT, bool POOL = false>
 int launch_readout_rows(int B, int C, int H, int Q, const int* s_row_ptr, const int* s_col_idx, const float* s_val, const float* h,
-                        const float* Wh1, const float* Wh2, float* pool, float* hidden, float* logits, float* probs, int* pred, hipStream_t s)
+                        const float* Wh1, const float* Wh2, float* pool, float* hidden, float* logits, float* probs, int* pred, hipStream_t s,
+                        const int* gate = nullptr)
 {
     constexpr int WG = BLOCK / TG / kWave;
     const size_t smem = sizeof(float) * TG * ((size_t)(WG + 1) * ((C + 3) / 4 * 4) + (size_t)(WG + 1) * H + Q);
     if (smem > 64 * 1024) return GNNHIP_EUNSUPPORTED;
     const int tiles = (B + TG - 1) / TG, most = kNumCU * (2048 / BLOCK);
-    hipLaunchKernelGGL((s2v_readout_rows_kernel<TG, BLOCK, MINW, FLIGHT>), dim3((unsigned)(tiles < most ? tiles : most)), dim3(BLOCK), smem, s, B, C, H, Q,
-                       s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2, pool, hidden, logits, probs, pred);
+    hipLaunchKernelGGL((s2v_readout_rows_kernel<TG, BLOCK, MINW, FLIGHT, POOL>), dim3((unsigned)(tiles < most ? tiles : most)), dim3(BLOCK), smem, s, B, C, H, Q,
+                       s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2, pool, hidden, logits, probs, pred, gate);
     GNNHIP_LAUNCH_CHECK("s2v_readout_rows");
     return GNNHIP_OK;
+}
+
+// over 16 lanes
+__device__ __forceinline__ float row_sum(float v)
+{
+    v += dpp_mov_f<kDppXor1>(v);
+    v += dpp_mov_f<kDppXor2>(v);
+    v += dpp_mov_f<kDppHalfMirror>(v);
+    return v + dpp_mov_f<kDppMirror>(v);
+}
+
+__device__ __forceinline__ float row_max(float v)
+{
+    v = max_keep(v, dpp_mov_f<kDppXor1>(v));
+    v = max_keep(v, dpp_mov_f<kDppXor2>(v));
+    v = max_keep(v, dpp_mov_f<kDppHalfMirror>(v));
+    return max_keep(v, dpp_mov_f<kDppMirror>(v));
+}
+
+__device__ __forceinline__ void row_argmax(float& v, int& i)
+{
+    argmax_combine(v, i, dpp_mov_f<kDppXor1>(v), dpp_mov_i<kDppXor1>(i));
+    argmax_combine(v, i, dpp_mov_f<kDppXor2>(v), dpp_mov_i<kDppXor2>(i));
+    argmax_combine(v, i, dpp_mov_f<kDppHalfMirror>(v), dpp_mov_i<kDppHalfMirror>(i));
+    argmax_combine(v, i, dpp_mov_f<kDppMirror>(v), dpp_mov_i<kDppMirror>(i));
+}
+
+// The readout behind pooled rows that are there, a workgroup per 16 graphs: a wavefront forms the hidden layer in blocks of 16 units on the FP32 matrix
+// cores, both operands straight from memory, up to 64 columns in one trip; then 16 lanes per graph add up its logits, a unit in 16 each, and
+// do softmax and arg-max.  Bound by the chain of its steps.  30,000 graphs, hidden 64, 32 units:
+// 13 us in a trace; the wavefront-per-graph kernel from its second step on 33, a lane per unit and four graphs with LDS operands 17.
+constexpr int kPooledGraphs = 16;
+constexpr int kPooledWaves = 4;
+
+__global__ __launch_bounds__(kPooledWaves * kWave) void s2v_readout_pooled_kernel(int B, int C, int H, int Q, const float* __restrict__ pool,
+                                                                                  const float* __restrict__ Wh1, const float* __restrict__ Wh2,
+                                                                                  float* __restrict__ hidden, float* __restrict__ logits,
+                                                                                  float* __restrict__ probs, int* __restrict__ pred)
+{
+    constexpr int kSteps = 16;                       // contraction steps of a trip, four columns each
+    extern __shared__ float smem[];
+    const int ldh = H | 1;
+    float* hid = smem;                               // [kPooledGraphs][ldh]
+    float* lg = hid + (size_t)kPooledGraphs * ldh;   // [kPooledGraphs][Q]
+    float* w2 = lg + (size_t)kPooledGraphs * Q;      // [H][Q]
+    constexpr int kThreads = kPooledWaves * kWave;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), q = lane >> 4, t = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int g0 = (int)blockIdx.x * kPooledGraphs, ng = min(kPooledGraphs, B - g0);
+    const float w2_first = Wh2[min(tid, H * Q - 1)];
+
+    // ---- hidden = ReLU(pool * W_h1), transposed: lane (q, t) ends up with units 4 q .. of graph t
+    const float* row = pool + (size_t)(g0 + min(t, ng - 1)) * C;
+    for (int j0 = 16 * wave; j0 < H; j0 += 16 * kPooledWaves) {
+        const float* col = Wh1 + min(j0 + t, H - 1);
+        mfma_f4 acc = {0.f, 0.f, 0.f, 0.f};
+        for (int c0 = 0; c0 < C; c0 += 4 * kSteps) {
+            float x[kSteps], w[kSteps];
+#pragma unroll
+            for (int s = 0; s < kSteps; ++s) {
+                const int c = min(c0 + 4 * s + q, C - 1);
+                x[s] = row[c];
+                w[s] = col[c * H];
+            }
+            __builtin_amdgcn_sched_barrier(0);       // all of them in flight
+#pragma unroll
+            for (int s = 0; s < kSteps; ++s) {
+                const bool in = c0 + 4 * s + q < C;  // both are zero past the last column
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? w[s] : 0.f, in ? x[s] : 0.f, acc, 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int j = j0 + 4 * q + i;
+            const float v = relu_ref(acc[i]);
+            if (j < H) {
+                hid[t * ldh + j] = v;
+                if (t < ng) hidden[(size_t)(g0 + t) * H + j] = v;
+            }
+        }
+    }
+    if (tid < H * Q) w2[tid] = w2_first;
+    for (int i = tid + kThreads; i < H * Q; i += kThreads) w2[i] = Wh2[i];
+    __syncthreads();
+
+    // ---- logits = hidden * W_h2, softmax + argmax over Q
+    static_assert(kThreads == 16 * kPooledGraphs, "16 lanes per graph");
+    const int g = tid / 16, sub = t;
+    float* logit = lg + (size_t)g * Q;
+    for (int c = 0; c < Q; ++c) {
+        float s = 0.f;
+        for (int j = sub; j < H; j += 16) s = fmaf(hid[g * ldh + j], w2[j * Q + c], s);
+        s = row_sum(s);
+        if (sub == 0) logit[c] = s;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    const float first = logit[0];
+    float mx = first;                                // the reference scan starts at element 0
+    float bv = -INFINITY;
+    int bi = 0x7fffffff;
+    for (int c = sub; c < Q; c += 16) {
+        const float v = logit[c];
+        if (g < ng) logits[(size_t)(g0 + g) * Q + c] = v;
+        mx = max_keep(mx, v);
+        argmax_combine(bv, bi, (v != v) ? -INFINITY : v, c);          // a NaN that is not first never wins
+    }
+    if (pred) {
+        row_argmax(bv, bi);
+        if (first != first) bi = 0;                  // a NaN in column 0 is never displaced
+        if (sub == 0 && g < ng) pred[g0 + g] = bi;
+    }
+    if (probs) {
+        mx = row_max(mx);
+        float s = 0.f;
+        for (int c = sub; c < Q; c += 16) {
+            const float e = expf(logit[c] - mx);
+            logit[c] = e;
+            s += e;
+        }
+        s = row_sum(s);
+        if (g < ng)
+            for (int c = sub; c < Q; c += 16) probs[(size_t)(g0 + g) * Q + c] = logit[c] / s;
+    }
 }
 
 }  // namespace
@@ -511,6 +640,36 @@ int readout_rows_dispatch(int B, int N, int C, int H, int Q, const int* s_row_pt
     if (rc == GNNHIP_EUNSUPPORTED) rc = launch_readout_rows<1, kBlock, 0, 8>(GNNHIP_RO_ARGS);
     return rc;
 #undef GNNHIP_RO_ARGS
+}
+
+size_t pooled_lds_bytes(int H, int Q) { return sizeof(float) * ((size_t)kPooledGraphs * ((H | 1) + Q) + (size_t)H * Q); }
+
+// whether readout_gated_dispatch takes these sizes; that its first launch does follows (four of its wavefronts take 5 C and 5 H words)
+bool readout_gated_accepts(int C, int H, int Q) { return C >= 4 && C <= 256 && pooled_lds_bytes(H, Q) <= 64 * 1024; }
+
+// The readout behind the one launch of a batch's levels, which has added up the pooled rows: those again if the gate says so, by the kernel
+// that the whole readout would take, and what follows them.
+int readout_gated_dispatch(int B, int C, int H, int Q, bool wave, const int* s_row_ptr, const int* s_col_idx, const float* s_val, const float* h,
+                           const float* Wh1, const float* Wh2, float* pool, float* hidden, float* logits, float* probs, int* pred,
+                           hipStream_t s, const int* gate)
+{
+#define GNNHIP_RO_ARGS H, Q, s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2, pool, hidden, logits, probs, pred, s, gate
+    int rc = GNNHIP_EUNSUPPORTED;
+    if (wave && aligned16(h)) {
+        switch (C) {
+        case 16: rc = launch_readout_wave<16, true>(B, GNNHIP_RO_ARGS); break;
+        case 32: rc = launch_readout_wave<32, true>(B, GNNHIP_RO_ARGS); break;
+        case 64: rc = launch_readout_wave<64, true>(B, GNNHIP_RO_ARGS); break;
+        }
+    }
+    if (rc == GNNHIP_EUNSUPPORTED && B >= 8 * kNumCU) rc = launch_readout_rows<4, kBlock, 0, 8, true>(B, C, GNNHIP_RO_ARGS);
+    if (rc == GNNHIP_EUNSUPPORTED) rc = launch_readout_rows<1, kBlock, 0, 8, true>(B, C, GNNHIP_RO_ARGS);
+#undef GNNHIP_RO_ARGS
+    if (rc) return rc;
+    hipLaunchKernelGGL(s2v_readout_pooled_kernel, dim3(ceil_div_u((size_t)B, kPooledGraphs)), dim3(kPooledWaves * kWave), pooled_lds_bytes(H, Q), s, B, C, H, Q, pool, Wh1, Wh2,
+                       hidden, logits, probs, pred);
+    GNNHIP_LAUNCH_CHECK("s2v_readout_pooled");
+    return GNNHIP_OK;
 }
 
 }  // namespace gnnhip

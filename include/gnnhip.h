@@ -254,7 +254,7 @@ int gnnhip_s2v_readout_f32(int B, int N, int C, int H, int Q,
  *      the library's choice: with L >= 1 the first level may read ReLU(msg) straight from msg, and
  *      h0 is then never stored).  a_nnz: entries of A.
  *      A large batch whose rows of S are ascending ranges of nodes, of at most 128 each, that cover all nodes, with no entry of A between
- *      two of them (found out on the device), runs its levels in one launch; the other of h_a and h_b is then not written.
+ *      two of them (found out on the device), runs its levels in one launch; the other of h_a and h_b is then scratch.
  *      Op sequence of examples/graph_classification/src/kernel_mean_field.cpp:31-49 scheduled by
  *      FactorGraph::SequentialForward (src/nn/factor_graph.cpp:75-144). */
 int gnnhip_s2v_forward_f32(int N, int B, int K, int C, int H, int Q, int L, int a_nnz,

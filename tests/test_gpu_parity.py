@@ -2718,9 +2718,8 @@ def _check_forward(gpu, A, S, N, K, C, L, gen, exact):
     got = (bufs.msg, bufs.h_final, bufs.pool, bufs.hidden, bufs.logits, bufs.probs, bufs.pred)
     want = _forward_one_by_one(A, S, X, *w, L)
     assert torch.equal(got[0], want[0])                      # one-hot features: rows of the weights
-    if exact:
-        for g, e in zip(got, want):
-            assert torch.equal(g, e)
+    for g, e in list(zip(got, want))[:exact]:
+        assert torch.equal(g, e)
     # float64 and the sum of the terms' magnitudes, level by level: every level adds the rounding of its two sums
     rp, ci, val = A
     row = torch.repeat_interleave(torch.arange(N, device=gpu), (rp[1:] - rp[:-1]).long())
@@ -2737,12 +2736,18 @@ def _check_forward(gpu, A, S, N, K, C, L, gen, exact):
     graph = torch.repeat_interleave(torch.arange(B, device=gpu), (S[0][1:] - S[0][:-1]).long(), output_size=S[1].numel())
     pool.index_add_(0, graph, got[1].double()[S[1].long()] * S[2].double()[:, None])
     assert bool(((got[2].double() - pool).abs() <= 4200 * 2.0 ** -24 * pool.abs() + 1e-30).all())     # no negative terms
+    # the readout from its own pooled rows: a rounding per term, and expf's two units in the last place, the sum and the quotient
+    hidden, hidden_terms = got[2].double() @ w[2].double(), got[2].double().abs() @ w[2].double().abs()
+    assert bool(((got[3].double() - hidden.clamp(min=0)).abs() <= (C + 1) * 2.0 ** -24 * hidden_terms).all())
+    logits, logit_terms = got[3].double() @ w[3].double(), got[3].double().abs() @ w[3].double().abs()
+    assert bool(((got[4].double() - logits).abs() <= (H + 1) * 2.0 ** -24 * logit_terms).all())
+    assert bool(((got[5].double() - torch.softmax(got[4].double(), 1)).abs() <= 16 * 2.0 ** -24).all())
     assert torch.equal(got[6].long(), got[4].argmax(1))
 
 
-def _enough(n, C, L):
-    """the sizes repeated until the batch is one that the forward tries to take in one launch"""
-    need = max(32768, (12e6 if C == 16 else 6e6 if 32 < C < 64 else 4e6) / ((L - 1) * C))
+def _enough(n, C, L, pooled=False):
+    """the sizes repeated until the batch is one that the forward tries to take in one launch, with pooled: that adds up the pooled rows too"""
+    need = max(32768, (12e6 if C == 16 else 6e6 if 32 < C < 64 else 4e6) / ((L - 1) * C), (12e6 if C > 64 else 4e6) / C if pooled else 0)
     return np.tile(np.asarray(n, np.int64), int(np.ceil(need / np.sum(n))))
 
 
@@ -2751,32 +2756,34 @@ def _enough(n, C, L):
 def test_forward_over_a_large_batch_of_small_graphs(gpu, C, sizes):
     """batches whose levels run in one launch: bins of one graph of 128 nodes, of 64 graphs of one node, graphs without nodes, bins of
     more entries than are kept in LDS, a last tile of one row; feature columns around the steps of the input stage, hidden sizes around
-    the padded ones.  Hidden 16 and 32 have the bits of the stages called one by one; the others are held to the rounding of fp32 sums"""
+    the padded ones.  The embeddings of hidden 16 and 32 have the bits of the stages called one by one; all else is held to the rounding of
+    fp32 sums"""
     import torch
     gen = torch.Generator(device=gpu).manual_seed(C)
     for K, L, seed in ((2, 2, 0), (3, 4, 1), (17, 3, 2), (33, 4, 3), (64, 2, 4)):
         rng = np.random.default_rng(100 * C + seed)
         n = {"molecules": rng.integers(10, 111, 1100), "ones": np.ones(33_001, np.int64), "full": np.full(300, 128),
              "with_empty": np.where(rng.random(4000) < 0.3, 0, rng.integers(1, 40, 4000)), "dense": rng.integers(90, 129, 400)}[sizes]
-        n = _enough(n, C, L)
+        n = _enough(n, C, L, pooled=seed % 2 == 0)
         if sizes == "with_empty":
             n[640:768] = 0                                       # two segments without nodes
             n[-1] = 0
         A, S, N = _small_graphs(gpu, n, 11 if sizes == "dense" else 2, gen)
-        _check_forward(gpu, A, S, N, K, C, L, gen, C in (16, 32))
+        _check_forward(gpu, A, S, N, K, C, L, gen, 2 if C in (16, 32) else 0)
 
 
 @pytest.mark.parametrize("C", [16, 30, 32, 46, 64, 77, 100])
-@pytest.mark.parametrize("kind", ["crossing", "crossing_dense", "large_graph", "uncovered", "offset", "overlapping", "long_row"])
+@pytest.mark.parametrize("kind", ["crossing", "crossing_dense", "large_graph", "uncovered", "offset", "overlapping", "long_row", "foreign_member",
+                                  "permuted_members"])
 def test_forward_over_a_batch_that_is_none(gpu, C, kind):
     """what the one launch must refuse on the device: one entry that leaves its bin (kept in LDS, or read from memory), a graph of 129
-    nodes, rows of S that leave out nodes, begin past node 0 or name nodes twice: every output has the bits of the stages called one
-    by one"""
+    nodes, rows of S that leave out nodes, begin past node 0, name nodes twice or those of other graphs: embeddings and pooled rows
+    have the bits of the stages called one by one"""
     import torch
     gen = torch.Generator(device=gpu).manual_seed(7)
     rng = np.random.default_rng(C)
     n = rng.integers(90, 129, 400) if kind == "crossing_dense" else rng.integers(10, 111, 1100)
-    n = _enough(rng.permutation(n), C, 3)
+    n = _enough(rng.permutation(n), C, 3, pooled=kind in ("foreign_member", "permuted_members", "large_graph"))
     if kind == "large_graph":
         n[700] = 129
     A, S, N = _small_graphs(gpu, n, 11 if kind == "crossing_dense" else 2, gen)
@@ -2799,7 +2806,13 @@ def test_forward_over_a_batch_that_is_none(gpu, C, kind):
         S = (S[0][1:] - S[0][1], S[1][int(S[0][1]):].contiguous(), S[2][int(S[0][1]):].contiguous())
     elif kind == "overlapping":                                  # the last row names all nodes of the batch again
         S = (torch.cat([S[0], S[0][-1:] + N]), torch.cat([S[1], S[1]]), torch.cat([S[2], S[2]]))
-    _check_forward(gpu, (rp, ci, val), S, N, 9, C, 3, gen, kind != "long_row")
+    elif kind == "foreign_member":                               # the last graph's row names a node of the first in its own one's place
+        S[1][-1] = 0
+    elif kind == "permuted_members":                             # the nodes of a row in another order, one of them twice: the one launch takes it
+        first, last = int(S[0][5]), int(S[0][6])
+        S[1][first:last] = S[1][first:last].flip(0)
+        S[1][first] = first + 1
+    _check_forward(gpu, (rp, ci, val), S, N, 9, C, 3, gen, 0 if kind in ("long_row", "permuted_members") else 3)
 
 
 @pytest.mark.parametrize("C", [64, 100])
