@@ -154,11 +154,11 @@ int launch_readout_wave(int B, int H, int Q, const int* s_row_ptr, const int* s_
 
 // Readout for wide hidden sizes (C = 128 or 256) on batches of thousands of graphs: one workgroup per tile of
 // kTileGraphs graphs.  W_h1 (128 KB at 256 x 128) does not fit LDS next to anything else, so it stays in memory
-// and every tile streams it once through L2, each element feeding kTileGraphs / 2 graphs:
+// and every tile streams it once through L2:
 //   1. sum-pool   a wavefront per graph, the whole wavefront across the C columns of a row, rows in order
 //                 (the order of the reference path), eight loads in flight; pooled rows go to LDS [graphs][C];
-//   2. hidden     a lane owns one hidden unit j for half of the tile's graphs: W_h1[c][j] read by consecutive
-//                 lanes, pool[g][c..c+3] broadcast from LDS, the sum over c in order;
+//   2. hidden     on the FP32 matrix cores, a wavefront per 16 units (10,000 graphs of 30 nodes, hidden 256, 128 units: 92 -> 83 us; a lane per
+//                 unit and eight graphs, with the pooled rows broadcast from LDS, was a tenth of the launch);
 //   3. logits     a lane per (graph, class), the sum over the hidden units in order;
 //   4. softmax and arg-max inside a wavefront per graph, as in the kernel above.
 // Algorithmic bytes as above; W_h1 traffic from L2 is 4 C H per tile.
@@ -172,11 +172,12 @@ __global__ __launch_bounds__(kBlock) void s2v_readout_tile_kernel(
     float* __restrict__ logits, float* __restrict__ probs, int* __restrict__ pred)
 {
     constexpr int VEC = C / kWave;       // floats of a row per lane (2 or 4)
-    constexpr int HALF = kTileGraphs / 2;
+    constexpr int kAhead = 16;
+    constexpr int LD = C + 4;
     using vec_t = typename std::conditional<VEC == 4, float4, float2>::type;
     extern __shared__ float smem[];
-    float* pl = smem;                                // [kTileGraphs][C]
-    float* hid = pl + kTileGraphs * C;               // [kTileGraphs][H]
+    float* pl = smem;                                // [kTileGraphs][LD]
+    float* hid = pl + kTileGraphs * LD;              // [kTileGraphs][H]
     float* lg = hid + (size_t)kTileGraphs * H;       // [kTileGraphs][Q]
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int g0 = (int)blockIdx.x * kTileGraphs;
@@ -218,36 +219,45 @@ __global__ __launch_bounds__(kBlock) void s2v_readout_tile_kernel(
             }
             *reinterpret_cast<vec_t*>(pool + (size_t)(g0 + gi) * C + lane * VEC) = *reinterpret_cast<vec_t*>(acc);
         }
-        *reinterpret_cast<vec_t*>(pl + gi * C + lane * VEC) = *reinterpret_cast<vec_t*>(acc);   // zeros past the last graph
+        *reinterpret_cast<vec_t*>(pl + gi * LD + lane * VEC) = *reinterpret_cast<vec_t*>(acc);   // zeros past the last graph
     }
     __syncthreads();
 
-    // ---- hidden = ReLU(pool * W_h1)
-    for (int it = threadIdx.x; it < 2 * H; it += kBlock) {
-        const int j = it % H, gh = it / H;
-        const float* p = pl + gh * HALF * C;
-        float a[HALF];
+    // ---- hidden = ReLU(pool * W_h1): a wavefront per 16 units, whose operand comes straight from memory, 16 contraction steps ahead; lane
+    //      (q, t) takes columns KS q .. KS q + KS - 1 of graph t and ends up with units 4 q .. of it
+    constexpr int KS = C / 4;
+    const int q4 = lane >> 4, t = lane & 15;
+    for (int j0 = 16 * wave; j0 < H; j0 += 16 * kWavesPerBlock) {
+        const float* w1 = Wh1 + (size_t)(KS * q4) * H + min(j0 + t, H - 1);
+        const float* x = pl + t * LD + KS * q4;
+        float w[2][kAhead];
 #pragma unroll
-        for (int g = 0; g < HALF; ++g) a[g] = 0.f;
-        for (int c = 0; c < C; c += 4) {
-            float w[4];
+        for (int s = 0; s < kAhead; ++s) w[0][s] = w1[(size_t)s * H];
+        mfma_f4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int u = 0; u < 4; ++u) w[u] = Wh1[(size_t)(c + u) * H + j];
+        for (int s0 = 0; s0 < KS; s0 += kAhead) {
+            const int cur = s0 / kAhead % 2;
+            if (s0 + kAhead < KS) {
 #pragma unroll
-            for (int g = 0; g < HALF; ++g) {
-                const float4 x = *reinterpret_cast<const float4*>(p + g * C + c);
-                a[g] = fmaf(x.x, w[0], a[g]);
-                a[g] = fmaf(x.y, w[1], a[g]);
-                a[g] = fmaf(x.z, w[2], a[g]);
-                a[g] = fmaf(x.w, w[3], a[g]);
+                for (int s = 0; s < kAhead; ++s) w[cur ^ 1][s] = w1[(size_t)(s0 + kAhead + s) * H];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int s = 0; s < kAhead; s += 4) {
+                const float4 v = *reinterpret_cast<const float4*>(x + s0 + s);
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[cur][s], v.x, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[cur][s + 1], v.y, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[cur][s + 2], v.z, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[cur][s + 3], v.w, acc, 0, 0, 0);
             }
         }
 #pragma unroll
-        for (int g = 0; g < HALF; ++g) {
-            const float v = relu_ref(a[g]);
-            const int gi = gh * HALF + g;
-            hid[(size_t)gi * H + j] = v;
-            if (gi < ng) hidden[(size_t)(g0 + gi) * H + j] = v;
+        for (int i = 0; i < 4; ++i) {
+            const int j = j0 + 4 * q4 + i;
+            if (j >= H) continue;
+            const float v = relu_ref(acc[i]);
+            hid[(size_t)t * H + j] = v;
+            if (t < ng) hidden[(size_t)(g0 + t) * H + j] = v;
         }
     }
     __syncthreads();
@@ -301,7 +311,7 @@ int launch_readout_tile(int B, int H, int Q, const int* s_row_ptr, const int* s_
                         const float* h, const float* Wh1, const float* Wh2, float* pool, float* hidden,
                         float* logits, float* probs, int* pred, hipStream_t s)
 {
-    const size_t smem = sizeof(float) * (size_t)kTileGraphs * ((size_t)C + H + Q);
+    const size_t smem = sizeof(float) * (size_t)kTileGraphs * ((size_t)C + 4 + H + Q);
     if (smem > 64 * 1024) return GNNHIP_EUNSUPPORTED;
     const unsigned grid = (unsigned)(((long long)B + kTileGraphs - 1) / kTileGraphs);
     hipLaunchKernelGGL(s2v_readout_tile_kernel<C>, dim3(grid), dim3(kBlock), smem, s, B, H, Q, s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2,
