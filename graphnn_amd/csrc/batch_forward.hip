@@ -47,14 +47,6 @@ constexpr int kRows = 128;                       // nodes of a bin
 constexpr int kEdgeCap = 1024;                   // entries of a bin kept in LDS; those of a bin with more are read from memory in every level
 constexpr int kDirect = 4;                       // entries per row whose place and weight stay in registers
 
-// ReLU as one instruction: NaN passes, as in relu_ref4, but -0 becomes 0 (two instructions cost 3 % of a level in pieces, where nothing
-// else is the same to the bit either)
-__device__ __forceinline__ float4 relu_one(const float4& v)
-{
-    return make_float4(__builtin_elementwise_maximum(v.x, 0.f), __builtin_elementwise_maximum(v.y, 0.f), __builtin_elementwise_maximum(v.z, 0.f),
-                       __builtin_elementwise_maximum(v.w, 0.f));
-}
-
 // CP: hidden size, or the next multiple of 16 that has a kernel.  TPW: tiles of 16 rows per wavefront.  MINW: wavefronts per SIMD.
 // PIECES: products from bf16 pieces; WREG: the first two pieces of W in registers, else all three in LDS
 template <int CP> struct BatchShape { static constexpr int TPW = 1, MINW = 2; static constexpr bool PIECES = true, WREG = false; };
@@ -358,7 +350,7 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
 #pragma unroll
                     for (int k = 0; k < KS; k += 4) {
                         float4 r = *reinterpret_cast<const float4*>(hbuf + off + k);
-                        if (kRelu) r = PIECES ? relu_one(r) : relu_ref4(r);
+                        if (kRelu) r = PIECES ? relu_max4(r) : relu_ref4(r);
                         agg[k] += w * r.x; agg[k + 1] += w * r.y; agg[k + 2] += w * r.z; agg[k + 3] += w * r.w;
                     }
                 };
@@ -450,7 +442,7 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
                             f.x *= d.x; f.y *= d.y; f.z *= d.z; f.w *= d.w;
                         }
                         const mfma_f4 r = WREG ? acc[0][jb] - acc[1][jb] : acc[0][jb] + acc[1][jb];
-                        v[i][jb] = relu_one(make_float4(fmaf(r[0], f.x, m[i][jb].x), fmaf(r[1], f.y, m[i][jb].y), fmaf(r[2], f.z, m[i][jb].z),
+                        v[i][jb] = relu_max4(make_float4(fmaf(r[0], f.x, m[i][jb].x), fmaf(r[1], f.y, m[i][jb].y), fmaf(r[2], f.z, m[i][jb].z),
                                                          fmaf(r[3], f.w, m[i][jb].w)));
                     }
                 } else {

@@ -181,6 +181,13 @@ __device__ __forceinline__ float4 relu_ref4(const float4& v)
 {
     return make_float4(relu_ref(v.x), relu_ref(v.y), relu_ref(v.z), relu_ref(v.w));
 }
+// The same as one instruction: NaN passes, but -0 becomes 0.  For kernels whose bits no other route has: two instructions cost 3 % of a level in
+// pieces that stays on chip (batch_forward.hip) and 1.6 % of the wide one (level_wide_split.hip).
+__device__ __forceinline__ float4 relu_max4(const float4& v)
+{
+    return make_float4(__builtin_elementwise_maximum(v.x, 0.f), __builtin_elementwise_maximum(v.y, 0.f), __builtin_elementwise_maximum(v.z, 0.f),
+                       __builtin_elementwise_maximum(v.w, 0.f));
+}
 
 // Device memory from the library's pool (released with pool_release).
 int pool_acquire(void** p, size_t bytes);

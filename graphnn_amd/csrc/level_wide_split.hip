@@ -17,7 +17,7 @@
 //   * A wavefront whose rows hold more entries than the tops of the remaining blocks can take starts a second batch in
 //     the middle of a block; gathering behind the pass would hold up the other seven.
 //
-// 299,536 nodes, 659,010 entries, C = 256, first level apart: 380 (FP32 matrix cores) -> 277 us per level (0.93 GB of
+// 299,536 nodes, 659,010 entries, C = 256, first level apart: 380 (FP32 matrix cores) -> 273 us per level (0.93 GB of
 // activations at 3.4 TB/s), backward 474 -> 428 us (1.85 GB at 4.3 TB/s).  Counted there: 0.64 GB fetched and 0.31 GB written, matrix
 // pipes busy 40 % of the cycles, 3.8 other instructions per matrix instruction of 16 cycles (1.9 of them vector ones, which
 // split the rows, 1.5 scalar ones, which steer the gather), no bank conflicts: neither memory nor the matrix pipes, but two
@@ -452,7 +452,7 @@ __global__ __launch_bounds__(WAVES * kWave) void s2v_level_split_kernel(
                 } else {
                     const float4 v = make_float4(fmaf(acc_m[jb][0], f.x, mm[jb].x), fmaf(acc_m[jb][1], f.y, mm[jb].y),
                                                  fmaf(acc_m[jb][2], f.z, mm[jb].z), fmaf(acc_m[jb][3], f.w, mm[jb].w));
-                    outv[jb] = make_float4(relu_ref(v.x), relu_ref(v.y), relu_ref(v.z), relu_ref(v.w));
+                    outv[jb] = relu_max4(v);
                 }
             }
             out_rt = rt;
@@ -664,7 +664,7 @@ __global__ __launch_bounds__(kFewWaves * kWave) void s2v_level_split_few_kernel(
         *reinterpret_cast<float4*>(out) = v;
     } else {
         const float4 v = make_float4(fmaf(sum[0], f.x, mm.x), fmaf(sum[1], f.y, mm.y), fmaf(sum[2], f.z, mm.z), fmaf(sum[3], f.w, mm.w));
-        *reinterpret_cast<float4*>(out) = make_float4(relu_ref(v.x), relu_ref(v.y), relu_ref(v.z), relu_ref(v.w));
+        *reinterpret_cast<float4*>(out) = relu_max4(v);
     }
 }
 

@@ -3006,3 +3006,54 @@ def test_forward_of_a_power_law_graph_forms_msg_again(gpu, C, K):
         assert torch.equal(got.h_final, h)                     # the input stage adds in the same order
     else:                                                      # and every level rounds its own sums from there on
         assert bool(((got.h_final.double() - h.double()).abs() <= err + L * (C + 900) * 2.0 ** -24 * terms).all())
+
+
+@pytest.mark.parametrize("C,N,Ks", [(256, 1, (49, 64)), (256, 15, (64,)), (256, 65, (53, 64)), (256, 3001, (49, 50, 61, 64)), (256, 270_001, (17, 40, 64)),
+                                    (64, 1_048_577, (1, 5, 16, 19, 32, 33)), (128, 530_049, (1, 3, 16, 20, 64))])
+@pytest.mark.parametrize("with_h0", [False, True])
+def test_input_stage_of_wide_and_large_calls(gpu, C, N, Ks, with_h0):
+    """msg alone in bf16 pieces (hidden 256, more than 48 feature columns), whole rows per store and fewer workgroups (more than 256 MB of
+    outputs): sizes around a tile of 64 rows, the last rows of the last tile, and nothing written behind them"""
+    import torch
+    from graphnn_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(C + N)
+    for K in Ks:
+        X, W = torch.randn(N, K, generator=gen, device=gpu), torch.randn(K, C, generator=gen, device=gpu)
+        out = [torch.full((N + 1, C), float("nan"), device=gpu) for _ in range(1 + with_h0)]
+        ops._bound().s2v_input_f32(N, K, C, X, W, out[0], out[1] if with_h0 else None)
+        at = torch.cat([torch.arange(0, min(N, 300)), torch.randint(0, N, (300,)), torch.arange(max(N - 300, 0), N)]).to(gpu)
+        want, terms = X[at].double() @ W.double(), X[at].double().abs() @ W.double().abs()
+        # a rounding per term and two of the split operands' own sums
+        assert bool(((out[0][at].double() - want).abs() <= (K + 4) * 2.0 ** -24 * terms).all()), K
+        assert bool(torch.isfinite(out[0][:N]).all()) and all(bool(torch.isnan(o[N]).all()) for o in out)
+        if with_h0:
+            assert torch.equal(out[1][:N], out[0][:N].clamp(min=0))
+
+
+def test_input_stage_in_pieces_with_large_and_tiny_values(gpu):
+    """rows and columns of 2^38 and more (scaled down) beside ordinary and tiny ones, one-hot rows to the bit, infinities and NaN in
+    their rows only"""
+    import torch
+    from graphnn_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(3)
+    N, K, C = 1000, 64, 256
+    msg = torch.empty(N, C, device=gpu)
+    run = lambda X, W: (ops._bound().s2v_input_f32(N, K, C, X, W, msg, None), msg.clone())[1]
+    X, W = torch.randn(N, K, generator=gen, device=gpu), torch.randn(K, C, generator=gen, device=gpu)
+    for scale in (1.0, 1e-36, 1e8):
+        Xs, Ws = X.clone(), W * scale
+        Xs[100:200] *= 2.0 ** 40
+        Ws[:, 7] *= 2.0 ** 45
+        want, terms = Xs.double() @ Ws.double(), Xs.double().abs() @ Ws.double().abs()
+        assert bool(torch.isfinite(want).all()) and bool(((run(Xs, Ws).double() - want).abs() <= (K + 4) * 2.0 ** -24 * terms + 2.0 ** -148).all()), scale
+    one_hot = torch.zeros(N, K, device=gpu)
+    label = torch.randint(0, K, (N,), generator=gen, device=gpu)
+    one_hot[torch.arange(N, device=gpu), label] = 1.0
+    assert torch.equal(run(one_hot, W), W[label])
+    clean = run(X, W)
+    X[5, 3], X[17, 60] = float("inf"), float("nan")
+    got = run(X, W)
+    rest = torch.ones(N, dtype=torch.bool, device=gpu)
+    rest[5] = rest[17] = False
+    assert torch.equal(got[rest], clean[rest])
+    assert torch.equal(got[5], torch.sign(W[3]) * float("inf")) and bool(torch.isnan(got[17]).all())
