@@ -27,10 +27,11 @@
 // instructions, about 330 per 16 rows and level (64 sum the first four entries, 104 split the rows); two wavefronts per SIMD, 247
 // registers.  What a bin reads is asked for while the last level of the bin before it ends (428 us without).
 //
-// Hidden sizes from 17 to 112 without kernels of their own take the next multiple of 16, with zeros behind the last column, and msg from
-// memory (the general input stage).  Above 64 W lies in LDS in all three pieces (86 KB at 112) and a workgroup fills a compute unit:
+// Hidden sizes from 17 to 112 without kernels of their own take the next multiple of 16, with zeros behind the last column.  msg comes from
+// memory (the general input stage: 12 us of 91 at 44,000 nodes, hidden 100, and the launch) only where W_n2l does not fit or K is 1 or
+// more than 64.  Above 64 W lies in LDS in all three pieces (86 KB at 112) and a workgroup fills a compute unit:
 // its wavefronts wait for the same things at the same time, and a level of 16 rows reads all of W.  44,000 nodes, hidden 100, 3.8
-// entries per row: a level 28 -> 15 us, the forward of three 111 -> 92; 176,000 nodes, four levels 416 -> 250; error against float64
+// entries per row: a level 28 -> 15 us, the forward of three 111 -> 82; 176,000 nodes, four levels 416 -> 245; error against float64
 // 6.7e-11, was 1.4e-10.  Above 112 columns W and the rows of 128 nodes do not fit the LDS together.  Tried there: the wavefronts share
 // the columns, as in level_wide_split.hip, and the rows are put into pieces in place between two barriers: 7.5 us for a bin of 112
 // nodes and a level at hidden 128, where the level-by-level route takes as long, and at hidden 256, where 64 nodes fit, 1.5 times that.
@@ -67,8 +68,8 @@ constexpr size_t batch_lds_bytes()
            sizeof(float) * (size_t)(CP / 16) * KSX * kWave + sizeof(int2) * (kEdgeCap + kRows) + sizeof(int) * (kRows + 4 + kWave + 4);
 }
 
-// KSX: contraction steps of the input stage, K <= 4 KSX, and the hidden size is CP; 0: msg is there, and the hidden size is C <= CP
-template <int CP, int KSX>
+// KSX: contraction steps of the input stage, K <= 4 KSX; 0: msg is there.  ODD: the hidden size is C <= CP, else CP
+template <int CP, int KSX, bool ODD>
 __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) void s2v_batch_levels_kernel(
     int N, int B, int K, int hidden, int L, const int* __restrict__ a_row_ptr, const int* __restrict__ a_col_idx, const float* __restrict__ a_val,
     const int* __restrict__ s_row_ptr, const int* __restrict__ s_col_idx, const float* __restrict__ s_val, const float* __restrict__ X,
@@ -82,7 +83,7 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
     constexpr int KS2 = (KS + 7) / 8;            // contraction steps of a level in pieces
     constexpr int NJB = CP / 16;                 // output blocks of 16 columns
     constexpr int LD = CP + 4;
-    const int C = INPUT ? CP : hidden;
+    const int C = ODD ? hidden : CP;
     const bool pooled = CP > 16 && pool;
     static_assert(!PIECES || !WREG || KS2 == 2, "two sums of opposite signs");
     extern __shared__ float4 smem4[];
@@ -115,7 +116,7 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
     bool any_down = false;                       // a column of W is scaled down (bf16_split.h): uniform
     auto w_at = [&](int k, int jb) {             // k: of the lane's
         const int row = KS * q + k, col = out_col + 4 * jb;
-        return INPUT || (row < C && col < C) ? Wc[(size_t)row * C + col] : 0.f;
+        return !ODD || (row < C && col < C) ? Wc[(size_t)row * C + col] : 0.f;
     };
     auto put_w = [&](int jb, const float (&w)[8 * KS2]) {
         float largest = 0.f;
@@ -165,8 +166,9 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
     if constexpr (INPUT) {
         for (int i = wave; i < NJB * (KSX / 2); i += kWaves) {
             const int jb = i / (KSX / 2), k = 8 * (i % (KSX / 2)) + 2 * q;
-            wn[i * kWave + lane] = make_float2(k < K ? Wn2l[(size_t)k * C + out_col + 4 * jb] : 0.f,
-                                               k + 1 < K ? Wn2l[(size_t)(k + 1) * C + out_col + 4 * jb] : 0.f);
+            const bool in = !ODD || out_col + 4 * jb < C;
+            wn[i * kWave + lane] = make_float2(in && k < K ? Wn2l[(size_t)k * C + out_col + 4 * jb] : 0.f,
+                                               in && k + 1 < K ? Wn2l[(size_t)(k + 1) * C + out_col + 4 * jb] : 0.f);
         }
     }
     if (tid < LD) hbuf[kRows * LD + tid] = 0.f;
@@ -228,6 +230,17 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
             e_val[u] = e < in_lds ? a_val[b.e0 + e] : 0.f;
         }
     };
+    auto mask = [&](float4 (&v)[NJB]) {          // ODD: zeros past the last column (in the last quarter, q = 3)
+        if (C == CP) return;
+#pragma unroll
+        for (int jb = NJB > 4 ? NJB - 4 : 0; jb < NJB; ++jb) {
+            const int col = KS * q + 4 * jb;
+            v[jb].x = col < C ? v[jb].x : 0.f;
+            v[jb].y = col + 1 < C ? v[jb].y : 0.f;
+            v[jb].z = col + 2 < C ? v[jb].z : 0.f;
+            v[jb].w = col + 3 < C ? v[jb].w : 0.f;
+        }
+    };
     Bin cur = record(at), next;
     bool more = at >= 0;                         // there is a bin `cur`
     ask(cur);
@@ -280,6 +293,7 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
                 m[i][jb] = f4_zero();
                 if (row0 + 16 * i < n) m[i][jb] = INPUT ? make_float4(acc[jb][0], acc[jb][1], acc[jb][2], acc[jb][3]) : mx[i][INPUT ? 0 : jb];
             }
+            if constexpr (ODD && INPUT) mask(m[i]);
         }
         __syncthreads();                         // the last bin's rows have left hbuf; rp and edges are there
         if (pooled && tid < n) {
@@ -313,7 +327,7 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
         // the bin's rows as they lie in memory: whole lines
         auto copy_out = [&](float* dst) {
             const int tid = tid_now();
-            if constexpr (INPUT) {
+            if constexpr (!ODD) {
                 for (int i = tid; i < n * KS; i += kBlock)
                     *reinterpret_cast<float4*>(dst + (size_t)node0 * C + 4 * i) = *reinterpret_cast<const float4*>(hbuf + (i / KS) * LD + 4 * (i % KS));
             } else {
@@ -458,20 +472,10 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
                         v[i][jb] = relu_ref4(make_float4(acc[jb][0] + m[i][jb].x, acc[jb][1] + m[i][jb].y, acc[jb][2] + m[i][jb].z, acc[jb][3] + m[i][jb].w));
                 }
             }
-            if constexpr (!INPUT) {              // columns past the last (in the last quarter, q = 3) stay zero whatever the others are
-                if (C < CP) {
+            if constexpr (ODD) {                 // columns past the last stay zero whatever the others are
 #pragma unroll
-                    for (int i = 0; i < TPW; ++i)
-#pragma unroll
-                        for (int jb = NJB > 4 ? NJB - 4 : 0; jb < NJB; ++jb) {
-                            const int col = KS * q + 4 * jb;
-                            if (i >= tiles) continue;
-                            v[i][jb].x = col < C ? v[i][jb].x : 0.f;
-                            v[i][jb].y = col + 1 < C ? v[i][jb].y : 0.f;
-                            v[i][jb].z = col + 2 < C ? v[i][jb].z : 0.f;
-                            v[i][jb].w = col + 3 < C ? v[i][jb].w : 0.f;
-                        }
-                }
+                for (int i = 0; i < TPW; ++i)
+                    if (i < tiles) mask(v[i]);
             }
             if constexpr (decltype(last)::value) ask(next);      // ahead of this bin's stores
             __syncthreads();                     // every row of the old embedding has been read
@@ -516,7 +520,7 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
                                                          __shfl_xor(sum.w, d, kWave)));
                 float* to = pool + (size_t)(g0 + g) * C + col;
                 if (l < kLanes && col < C) {
-                    if (INPUT) {
+                    if (!ODD) {
                         *reinterpret_cast<float4*>(to) = sum;
                     } else if (col + 4 <= C) {
                         ColsLoose::store(to, sum);
@@ -534,7 +538,7 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
     if (finder.unpacked && tid == 0) *refused = 1;
 }
 
-template <int CP, int KSX>
+template <int CP, int KSX, bool ODD>
 int launch_batch_levels(int N, int B, int K, int C, int L, const int* a_row_ptr, const int* a_col_idx, const float* a_val, const int* s_row_ptr,
                         const int* s_col_idx, const float* s_val, const float* X, const float* Wn2l, const float* Wc, float* msg, float* h_out,
                         float* pool, const int* bins, int* refused, int cap, hipStream_t s)
@@ -543,13 +547,13 @@ int launch_batch_levels(int N, int B, int K, int C, int L, const int* a_row_ptr,
     constexpr int kWaves = batch_waves<CP>();
     static_assert(smem * (BatchShape<CP>::MINW * 4 / kWaves) <= 160 * 1024, "workgroups share the LDS of a compute unit");
     static LdsLimit lds_limit;
-    GNNHIP_HIP(lds_limit.raise(reinterpret_cast<const void*>(&s2v_batch_levels_kernel<CP, KSX>), smem));
+    GNNHIP_HIP(lds_limit.raise(reinterpret_cast<const void*>(&s2v_batch_levels_kernel<CP, KSX, ODD>), smem));
     // two neighbouring bins hold more than cap nodes together, and every 64 graphs may leave one bin short
     long long most = 2ll * N / cap + (B + kWave - 1) / kWave + 1;
     if (most > B) most = B;
     const long long resident = (long long)kNumCU * (BatchShape<CP>::MINW * 4 / kWaves);
     const unsigned grid = (unsigned)(most < resident ? most : resident);
-    hipLaunchKernelGGL((s2v_batch_levels_kernel<CP, KSX>), dim3(grid), dim3(kWaves * kWave), smem, s, N, B, K, C, L, a_row_ptr, a_col_idx, a_val,
+    hipLaunchKernelGGL((s2v_batch_levels_kernel<CP, KSX, ODD>), dim3(grid), dim3(kWaves * kWave), smem, s, N, B, K, C, L, a_row_ptr, a_col_idx, a_val,
                        s_row_ptr, s_col_idx, s_val, X, Wn2l, Wc, msg, h_out, pool, bins, refused);
     GNNHIP_LAUNCH_CHECK("s2v_batch_levels");
     return GNNHIP_OK;
@@ -559,8 +563,8 @@ constexpr int kTwoStepMeanDegree = 12;           // denser matrices take the SpM
 
 }  // namespace
 
-// whether batch_levels_dispatch forms msg itself; else it is to be there
-bool batch_levels_with_input(int K, int C) { return K >= 2 && K <= 64 && (C == 16 || C == 32 || C == 64); }
+// whether batch_levels_dispatch forms msg itself; else it is to be there (past 96 columns there is no more LDS for W_n2l of many rows)
+bool batch_levels_with_input(int K, int C) { return K >= 2 && C >= 16 && (K <= 16 ? C <= 112 : K <= 64 && C <= 96); }
 
 size_t batch_levels_work_ints(int B) { return bin_ints(B); }
 
@@ -598,22 +602,25 @@ int batch_levels_dispatch(int N, int B, int K, int C, int L, long long nnz, cons
     hipLaunchKernelGGL((graph_bins_kernel<true>), dim3(ceil_div_u((size_t)B, kBinBlock)), dim3(kBinBlock), 0, s, B, cap, a_row_ptr, s_row_ptr,
                        bins, N, refused, kRows);
     GNNHIP_LAUNCH_CHECK("graph_bins");
-#define GNNHIP_BL(CP, KSX) launch_batch_levels<CP, KSX>(N, B, K, C, L, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx, s_val, X, Wn2l, Wc, msg, h_out, \
+#define GNNHIP_BL(CP, KSX, ODD) launch_batch_levels<CP, KSX, ODD>(N, B, K, C, L, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx, s_val, X, Wn2l, Wc, msg, h_out, \
                                                 pool, bins, refused, cap, s)
-    if (batch_levels_with_input(K, C)) {
-#define GNNHIP_BL_K(CP) (K <= 16 ? GNNHIP_BL(CP, 4) : K <= 32 ? GNNHIP_BL(CP, 8) : K <= 48 ? GNNHIP_BL(CP, 12) : GNNHIP_BL(CP, 16))
+    const bool input = batch_levels_with_input(K, C);
+    if (input && (C == 16 || C == 32 || C == 64)) {
+#define GNNHIP_BL_K(CP) (K <= 16 ? GNNHIP_BL(CP, 4, false) : K <= 32 ? GNNHIP_BL(CP, 8, false) : K <= 48 ? GNNHIP_BL(CP, 12, false) : GNNHIP_BL(CP, 16, false))
         return C == 16 ? GNNHIP_BL_K(16) : C == 32 ? GNNHIP_BL_K(32) : GNNHIP_BL_K(64);
 #undef GNNHIP_BL_K
     }
+#define GNNHIP_BL_K(CP) (!input ? GNNHIP_BL(CP, 0, true) : K <= 16 ? GNNHIP_BL(CP, 4, true) : GNNHIP_BL(CP, 16, true))
     switch ((C + 15) / 16) {
-    case 1: return GNNHIP_BL(16, 0);
-    case 2: return GNNHIP_BL(32, 0);
-    case 3: return GNNHIP_BL(48, 0);
-    case 4: return GNNHIP_BL(64, 0);
-    case 5: return GNNHIP_BL(80, 0);
-    case 6: return GNNHIP_BL(96, 0);
-    default: return GNNHIP_BL(112, 0);
+    case 1: return GNNHIP_BL(16, 0, true);
+    case 2: return GNNHIP_BL_K(32);
+    case 3: return GNNHIP_BL_K(48);
+    case 4: return GNNHIP_BL_K(64);
+    case 5: return GNNHIP_BL_K(80);
+    case 6: return GNNHIP_BL_K(96);
+    default: return input ? GNNHIP_BL(112, 4, true) : GNNHIP_BL(112, 0, true);
     }
+#undef GNNHIP_BL_K
 #undef GNNHIP_BL
 }
 

@@ -30,7 +30,7 @@ int level_rows_dispatch(int N, int C, long long nnz, const int* row_ptr, const i
 int level_rows_backward_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* dz,
                                  const float* W, float* u, float* g_prev, const float* gate, float* acc, hipStream_t s);
 int level_rows_dense_dispatch(int N, int K, int n, const float* x, const float* W, const float* bias, const float* msg, float* out,
-                              bool relu, float* relu_out, hipStream_t s);
+                              bool relu, float* relu_out, hipStream_t s, const int* gate = nullptr);
 int readout_rows_dispatch(int B, int N, int C, int H, int Q, const int* s_row_ptr, const int* s_col_idx, const float* s_val, const float* h,
                           const float* Wh1, const float* Wh2, float* pool, float* hidden, float* logits, float* probs, int* pred, hipStream_t s);
 bool readout_gated_accepts(int C, int H, int Q);
@@ -94,7 +94,7 @@ int input_any(int N, int K, int C, const float* X, const float* Wn2l, float* msg
     int rc = input_dispatch(N, K, C, X, Wn2l, msg, h0, s, gate);
     if (rc != GNNHIP_EUNSUPPORTED) return rc;
     if (h0) return product_any(N, K, C, X, Wn2l, nullptr, nullptr, msg, h0, s);
-    rc = level_rows_dense_dispatch(N, K, C, X, Wn2l, nullptr, nullptr, msg, false, nullptr, s);
+    rc = level_rows_dense_dispatch(N, K, C, X, Wn2l, nullptr, nullptr, msg, false, nullptr, s, gate);
     if (rc != GNNHIP_EUNSUPPORTED) return rc;
     return gemm_dispatch(0, 0, N, C, K, 1.f, X, K, Wn2l, C, 0.f, msg, C, s);
 }

@@ -548,7 +548,7 @@ int launch_rows(const RowsArgs& a, hipStream_t s)
     const int KP = (a.K + 15) & ~15;
     const int width = KP + 4 > a.n ? KP + 4 : a.n;
     const unsigned grid = (unsigned)(((long long)a.N + 16 * RT - 1) / (16 * RT));
-    constexpr bool kGated = GATHER && !WT && RT > 1 && NB <= 2;            // the levels of batch_forward.hip's sizes
+    constexpr bool kGated = !WT && RT > 1 && NB <= 2;      // input and levels of batch_forward.hip's sizes
     const auto kernel = kGated && a.launch_gate ? &s2v_rows_kernel<RT, NB, MINW, GATHER, WT, kGated> : &s2v_rows_kernel<RT, NB, MINW, GATHER, WT, false>;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBlock), sizeof(float) * 16 * RT * width, s, a);
     GNNHIP_LAUNCH_CHECK("s2v_rows");
@@ -631,13 +631,13 @@ int level_rows_backward_dispatch(int N, int C, long long nnz, const int* row_ptr
 
 // out = x * W (+ bias + msg); relu: out = ReLU of that; relu_out (or null) = ReLU(out).  x [N, K], W [K, n].
 int level_rows_dense_dispatch(int N, int K, int n, const float* x, const float* W, const float* bias, const float* msg, float* out,
-                              bool relu, float* relu_out, hipStream_t s)
+                              bool relu, float* relu_out, hipStream_t s, const int* gate)
 {
     // (64 rows of more than 252 columns would not fit 64 KB of LDS)
     if (K < 1 || K > (n <= 128 ? 128 : kMaxWidth) || n > kMaxWidth) return GNNHIP_EUNSUPPORTED;
     RowsArgs a{};
     a.N = N; a.K = K; a.n = n;
-    a.x = x; a.W = W; a.bias = bias; a.msg = msg; a.out = out; a.relu = relu; a.relu_out = relu_out;
+    a.x = x; a.W = W; a.bias = bias; a.msg = msg; a.out = out; a.relu = relu; a.relu_out = relu_out; a.launch_gate = gate;
     return rows_dispatch<false, false>(a, s);
 }
 
