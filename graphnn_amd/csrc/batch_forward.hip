@@ -581,11 +581,18 @@ int batch_levels_dispatch(int N, int B, int K, int C, int L, long long nnz, cons
                           const int* s_row_ptr, const int* s_col_idx, const float* s_val, const float* X, const float* Wn2l, const float* Wc,
                           float* msg, float* h_out, float* pool, int* work, int* refused, hipStream_t s)
 {
-    // What the levels but the first save is reading h and msg and writing h.  Below these products the launches of both routes cost more
-    // than that (hidden 64, 35,000 nodes: two levels 52 us against 48, three 59 against 62; hidden 32, 73,000 nodes: one level 35.6 against
-    // 35.2, two 42.9 against 45.6; hidden 50, 88,000 nodes: two levels 78 against 72, three 90 against 94; hidden 77: two levels 95 against
-    // 122, and with 44,000 nodes three 77 against 91; hidden 16, 235,000 nodes of 60 features: three levels 77 against 77).
-    const bool enough = (long long)(L - 1) * N * C >= (C == 16 ? 12000000 : C > 32 && C < 64 ? 6000000 : 4000000) && N >= 32768;
+    // What the levels but the first save is reading h and msg and writing h, and, where the level-by-level kernels are those of any size, most
+    // of a level.  Below these products the launches of both routes cost more than that.  Forwards, level by level and so:
+    //     hidden 66     6,755 nodes, three levels (0.9 M) 39 us and 39, four 47 and 43; 14,102, two (0.9 M) 36 and 35, five 67 and 49
+    //            96     20,564, two (2 M) 49 and 37, four 81 and 48;  100 of 38 features, where the input is a launch: 20,564, two (2.1 M) 52 and 52
+    //            56     14,102, five (3.2 M) 52 and 54; 20,564, four (3.5 M) 51 and 50;  50: 26,440, four (4 M) 56 and 50; 52,870, three 80 and 63
+    //            20     26,440, three (1.1 M) 32 and 33, four 38 and 36; 52,870, three (2.1 M) 54 and 46
+    //            64     26,440, three (3.4 M) 41 and 42, four 50 and 48;  32: 52,870, three (3.4 M) 48 and 44
+    //            16     73,432, four (3.5 M) 53 and 51 or, of 38 features, 58 and 50; 52,870, five (3.4 M) 57 and 64
+    // Up to 24,576 nodes hidden 16, 32 and 64 have level_tile.hip, up to 4,096 the others the kernel of few rows: neither has a gated variant.
+    const bool own = C == 16 || C == 32 || C == 64, input = batch_levels_with_input(K, C);
+    const long long least = C == 16 ? 5000000 : C < 32 ? 1500000 : C == 32 ? 3000000 : C < 64 ? 3600000 : C == 64 || !input ? 4000000 : C <= 96 ? 1500000 : 1800000;
+    const bool enough = (long long)(L - 1) * N * C >= least && N > (own ? 24576 : C > 32 && C < 64 ? 16384 : kFewRows);
     if (!enough || nnz >= kTwoStepMeanDegree * (long long)N || (long long)N > 96ll * B || C < 16 || C > 112) return GNNHIP_EUNSUPPORTED;
     // Bins of fewer nodes where they fill the rounds of workgroups better: a round takes its tiles and about two more (start, barriers).
     // The host knows the totals only: a bin wastes about half a mean graph, and every 64 graphs about half a bin.
@@ -604,7 +611,6 @@ int batch_levels_dispatch(int N, int B, int K, int C, int L, long long nnz, cons
     GNNHIP_LAUNCH_CHECK("graph_bins");
 #define GNNHIP_BL(CP, KSX, ODD) launch_batch_levels<CP, KSX, ODD>(N, B, K, C, L, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx, s_val, X, Wn2l, Wc, msg, h_out, \
                                                 pool, bins, refused, cap, s)
-    const bool input = batch_levels_with_input(K, C);
     if (input && (C == 16 || C == 32 || C == 64)) {
 #define GNNHIP_BL_K(CP) (K <= 16 ? GNNHIP_BL(CP, 4, false) : K <= 32 ? GNNHIP_BL(CP, 8, false) : K <= 48 ? GNNHIP_BL(CP, 12, false) : GNNHIP_BL(CP, 16, false))
         return C == 16 ? GNNHIP_BL_K(16) : C == 32 ? GNNHIP_BL_K(32) : GNNHIP_BL_K(64);

@@ -548,7 +548,7 @@ int launch_rows(const RowsArgs& a, hipStream_t s)
     const int KP = (a.K + 15) & ~15;
     const int width = KP + 4 > a.n ? KP + 4 : a.n;
     const unsigned grid = (unsigned)(((long long)a.N + 16 * RT - 1) / (16 * RT));
-    constexpr bool kGated = !WT && RT > 1 && NB <= 2;      // input and levels of batch_forward.hip's sizes
+    constexpr bool kGated = !WT && NB <= 2;                // input and levels of batch_forward.hip's sizes
     const auto kernel = kGated && a.launch_gate ? &s2v_rows_kernel<RT, NB, MINW, GATHER, WT, kGated> : &s2v_rows_kernel<RT, NB, MINW, GATHER, WT, false>;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBlock), sizeof(float) * 16 * RT * width, s, a);
     GNNHIP_LAUNCH_CHECK("s2v_rows");

@@ -2815,6 +2815,23 @@ def test_forward_over_a_batch_that_is_none(gpu, C, kind):
     _check_forward(gpu, (rp, ci, val), S, N, 9, C, 3, gen, 0 if kind in ("long_row", "permuted_members") else 3)
 
 
+@pytest.mark.parametrize("C,K,N", [(20, 3, 20_000), (31, 40, 13_000), (40, 7, 24_000), (63, 64, 17_000), (65, 2, 8_000), (66, 64, 4_100), (96, 16, 4_097),
+                                   (96, 17, 16_400), (97, 16, 6_000), (100, 17, 12_000), (112, 5, 16_384), (112, 1, 16_385)])
+@pytest.mark.parametrize("crossing", [False, True])
+def test_forward_over_a_few_small_graphs_of_odd_hidden_sizes(gpu, C, K, N, crossing):
+    """some thousand nodes, which the levels' one launch takes where it is their input stage too, and its refusal, behind which the
+    level-by-level launches have tiles of 16 or 32 rows"""
+    import torch
+    gen = torch.Generator(device=gpu).manual_seed(N)
+    n = np.random.default_rng(C).integers(1, 60, N)
+    n = n[:int(np.searchsorted(np.cumsum(n), N))]
+    n = np.append(n, N - int(n.sum()))
+    A, S, N = _small_graphs(gpu, n, 2, gen)
+    if crossing:
+        A[1][int(A[0][int(torch.nonzero(A[0][1:] > A[0][:-1])[-1])])] = 0
+    _check_forward(gpu, A, S, N, K, C, 5, gen, 3 if crossing else 0)
+
+
 @pytest.mark.parametrize("C", [64, 100])
 def test_forward_over_small_graphs_with_large_and_tiny_values(gpu, C):
     """products in bf16 pieces over a large batch of small graphs: rows of 2^38 and more and columns of W likewise (scaled down before they
