@@ -104,8 +104,12 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
     // a pair of columns by all lanes covers 32 consecutive bytes of 16 rows
     const int srt = 2 * ((K + 7) / 8);
 
+    // a segment that was not packed (graph_bins.h): nothing is formed.  Every workgroup looks at all words, 64 graphs each, so that a batch that is
+    // none costs no more than the start (10 to 15 us: 600 graphs, hidden 100 96 -> 107, 30,000, hidden 64 805 -> 829, 971 where only those that came upon such a word left)
+    bool unpacked = false;
+    for (int i = tid; i < (B + kWave - 1) / kWave; i += kBlock) unpacked |= reinterpret_cast<const unsigned long long*>(bins)[i] == 0;
     BinFinder finder(B, bins);
-    int at = finder.find_checked((int)blockIdx.x);
+    int at = finder.find((int)blockIdx.x);
 
     // W as the operand of the matrix instructions, zeros past its last row and column.  fp32: wf[jb][s] = W[KS q + s][out_col + 4 jb]; in
     // pieces: of W[KS q + 8 s + 0..7].  The matrix instructions on bf16 round towards minus infinity: in registers, the second step is
@@ -174,6 +178,10 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
     if (tid < LD) hbuf[kRows * LD + tid] = 0.f;
     if (tid == 0) stop = 0;
     any_down = __syncthreads_or(any_down);
+    if (__syncthreads_or(unpacked)) {
+        if (tid == 0) *refused = 1;
+        return;
+    }
 
     // ---- what a bin needs from memory, asked for together and a bin ahead
     struct Bin { int node0, n, e0, ne, g0, ng; };
@@ -262,7 +270,7 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
                 }
             }
         }
-        at = finder.find_checked(bin + (int)gridDim.x);
+        at = finder.find(bin + (int)gridDim.x);
         more = at >= 0;
         next = record(at);
 
@@ -534,8 +542,6 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
         }
         cur = next;
     }
-    // a segment that was not packed: every workgroup comes by all words
-    if (finder.unpacked && tid == 0) *refused = 1;
 }
 
 template <int CP, int KSX, bool ODD>

@@ -79,7 +79,6 @@ __global__ __launch_bounds__(kBinBlock) void graph_bins_kernel(int B, int cap, c
 // 60,000 145, 141).
 struct BinFinder {
     int nseg, seg = 0, before = 0;               // 64 words from seg on, bins of the words before them
-    bool unpacked = false;                       // a word of a segment that was not packed came by
     const unsigned long long* words;
     __device__ BinFinder(int B, const int* bins) : nseg((B + kWave - 1) / kWave), words(reinterpret_cast<const unsigned long long*>(bins)) {}
     // the place of the record of a bin, or -1 past the last one
@@ -88,25 +87,6 @@ struct BinFinder {
         const int lane = threadIdx.x & (kWave - 1);
         for (; seg < nseg; seg += kWave) {
             const int count = seg + lane < nseg ? __popcll(words[seg + lane]) : 0;
-            const int through = before + wave_inclusive_scan_i(count);
-            const unsigned long long behind = __ballot(bin < through);
-            if (behind) {
-                const int at = (int)__builtin_ctzll(behind);
-                return (seg + at) * kWave + bin - __builtin_amdgcn_readlane(through - count, at);
-            }
-            before = __builtin_amdgcn_readlane(through, kWave - 1);
-        }
-        return -1;
-    }
-    // the same of checked bins: `unpacked` is set when a segment without bins is passed over, which every wavefront that
-    // asks until it gets -1 does
-    __device__ __forceinline__ int find_checked(int bin)
-    {
-        const int lane = threadIdx.x & (kWave - 1);
-        for (; seg < nseg; seg += kWave) {
-            const unsigned long long word = seg + lane < nseg ? words[seg + lane] : 1;
-            const int count = seg + lane < nseg ? __popcll(word) : 0;
-            unpacked |= __any(word == 0);
             const int through = before + wave_inclusive_scan_i(count);
             const unsigned long long behind = __ballot(bin < through);
             if (behind) {
