@@ -2815,6 +2815,41 @@ def test_forward_over_a_batch_that_is_none(gpu, C, kind):
     _check_forward(gpu, (rp, ci, val), S, N, 9, C, 3, gen, 0 if kind in ("long_row", "permuted_members") else 3)
 
 
+@pytest.mark.parametrize("C", [32, 64, 100])
+def test_large_batch_forward_replays_from_a_captured_graph(gpu, C):
+    """captured over a batch that the levels' one launch takes, then replayed over matrices changed in place: whether it takes them is
+    found out by every replay, and each has the bits of the same eager call"""
+    import torch
+    from graphnn_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(C)
+    A, S, N = _small_graphs(gpu, _enough(np.random.default_rng(C).integers(10, 111, 1100), C, 3, pooled=True), 2, gen)
+    B, K, H, Q = S[0].numel() - 1, 9, 8, 3
+    normal = lambda *shape: torch.randn(*shape, generator=gen, device=gpu)
+    X, w = normal(N, K), (normal(K, C), normal(C, C) * (0.8 / C ** 0.5), normal(C, H), normal(H, Q))
+    bufs, eager = ops.ForwardBuffers(N, B, C, H, Q, gpu), ops.ForwardBuffers(N, B, C, H, Q, gpu)
+    last = int(A[0][int(torch.nonzero(A[0][1:] > A[0][:-1])[-1])])          # an entry of the last graph
+    inside = int(A[1][last])
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        ops.s2v_forward(A, S, X, *w, 3, bufs=bufs)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        ops.s2v_forward(A, S, X, *w, 3, bufs=bufs)
+    torch.cuda.synchronize()
+    outputs = lambda b: [getattr(b, n) for n in ("msg", "h_final", "pool", "hidden", "logits", "probs", "pred")]
+    for column in (inside, 0, 0, inside, inside):
+        A[1][last] = column
+        for t in outputs(bufs):
+            t.fill_(-1)
+        ops.s2v_forward(A, S, X, *w, 3, bufs=eager)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for got, want in zip(outputs(bufs), outputs(eager)):
+            assert torch.equal(got, want), column
+
+
 @pytest.mark.parametrize("C,K,N", [(20, 3, 20_000), (31, 40, 13_000), (40, 7, 24_000), (63, 64, 17_000), (65, 2, 8_000), (66, 64, 4_100), (96, 16, 4_097),
                                    (96, 17, 16_400), (97, 16, 6_000), (100, 17, 12_000), (112, 5, 16_384), (112, 1, 16_385)])
 @pytest.mark.parametrize("crossing", [False, True])
