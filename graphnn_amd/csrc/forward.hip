@@ -122,7 +122,9 @@ __global__ __launch_bounds__(kBlock) void copy_kernel(const float* __restrict__ 
 
 constexpr int kWaveReadoutMinGraphs = 1024;        // below this a workgroup per graph
 constexpr int kWaveReadoutMaxMeanNodes = 2048;     // mean nodes per graph
-constexpr int kTileReadoutMinGraphs = 4096;        // hidden 128/256
+constexpr int kTileReadoutMinGraphs = 2048;        // hidden 128/256
+constexpr int kTileReadoutAnyNodes = 4096;         // more graphs than this: up to the mean above, else up to
+constexpr int kTileReadoutMaxMeanNodes = 128;
 
 int readout_any(int B, int N, int C, int H, int Q, const int* s_row_ptr, const int* s_col_idx, const float* s_val,
                 const float* h, const float* Wh1, const float* Wh2, float* pool, float* hidden,
@@ -137,8 +139,11 @@ int readout_any(int B, int N, int C, int H, int Q, const int* s_row_ptr, const i
     if (wave)
         rc = readout_wave_dispatch(B, C, H, Q, s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2, pool, hidden, logits, probs, pred, s);
     if (rc != GNNHIP_EUNSUPPORTED) return rc;
-    // hidden 128/256: a workgroup per graph up to a few thousand graphs, then a tile of graphs per workgroup
-    if (C > 64 && B > kTileReadoutMinGraphs && (long long)N <= (long long)B * kWaveReadoutMaxMeanNodes)
+    // hidden 128/256: a workgroup per graph up to two thousand graphs, then a tile of graphs per workgroup, a wavefront each, except where few graphs
+    // are large (hidden 256, a wavefront per graph without tiles and so: 2,048 graphs of 30 nodes 31.5 us and 20.0, of 100 55.9 and 42.2, of 400 165
+    // and 183; 4,096 48.1 and 28.5, 108 and 91, 315 and 307; a workgroup per graph: 1,500 of 30 20.2 and 18.1, 1,100 16.8 and 16.7, of 100 33.8 and 32.9,
+    // hidden 128 9.8 and 13.4)
+    if (C > 64 && B >= kTileReadoutMinGraphs && (long long)N <= (long long)B * (B > kTileReadoutAnyNodes ? kWaveReadoutMaxMeanNodes : kTileReadoutMaxMeanNodes))
         rc = readout_tile_dispatch(B, C, H, Q, s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2, pool, hidden, logits, probs, pred, s);
     if (rc != GNNHIP_EUNSUPPORTED) return rc;
     rc = readout_rows_dispatch(B, N, C, H, Q, s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2, pool, hidden, logits, probs, pred, s);

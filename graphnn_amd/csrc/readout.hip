@@ -156,7 +156,9 @@ int launch_readout_wave(int B, int H, int Q, const int* s_row_ptr, const int* s_
 // kTileGraphs graphs.  W_h1 (128 KB at 256 x 128) does not fit LDS next to anything else, so it stays in memory
 // and every tile streams it once through L2:
 //   1. sum-pool   a wavefront per graph, the whole wavefront across the C columns of a row, rows in order
-//                 (the order of the reference path), eight loads in flight; pooled rows go to LDS [graphs][C];
+//                 (the order of the reference path), eight loads in flight; pooled rows go to LDS [graphs][C].  A graph is a
+//                 chain of trips, so what bounds this is how many are summed at once: four wavefronts per tile, four graphs each in turn,
+//                 were 76 us at 10,000 graphs of 30 nodes, hidden 256, sixteen are 71, where a copy of the rows' bytes takes 59;
 //   2. hidden     on the FP32 matrix cores, a wavefront per 16 units (10,000 graphs of 30 nodes, hidden 256, 128 units: 92 -> 83 us; a lane per
 //                 unit and eight graphs, with the pooled rows broadcast from LDS, was a tenth of the launch);
 //   3. logits     a lane per (graph, class), the sum over the hidden units in order;
@@ -164,8 +166,8 @@ int launch_readout_wave(int B, int H, int Q, const int* s_row_ptr, const int* s_
 // Algorithmic bytes as above; W_h1 traffic from L2 is 4 C H per tile.
 constexpr int kTileGraphs = 16;
 
-template <int C>
-__global__ __launch_bounds__(kBlock) void s2v_readout_tile_kernel(
+template <int C, int WAVES>
+__global__ __launch_bounds__(WAVES * kWave) void s2v_readout_tile_kernel(
     int B, int H, int Q, const int* __restrict__ s_row_ptr, const int* __restrict__ s_col_idx,
     const float* __restrict__ s_val, const float* __restrict__ h, const float* __restrict__ Wh1,
     const float* __restrict__ Wh2, float* __restrict__ pool, float* __restrict__ hidden,
@@ -179,46 +181,53 @@ __global__ __launch_bounds__(kBlock) void s2v_readout_tile_kernel(
     float* pl = smem;                                // [kTileGraphs][LD]
     float* hid = pl + kTileGraphs * LD;              // [kTileGraphs][H]
     float* lg = hid + (size_t)kTileGraphs * H;       // [kTileGraphs][Q]
-    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
     const int g0 = (int)blockIdx.x * kTileGraphs;
     const int ng = min(kTileGraphs, B - g0);
 
-    // ---- sum-pool
-    for (int gi = wave; gi < kTileGraphs; gi += kWavesPerBlock) {
+    // ---- sum-pool: the offsets of all graphs in one trip, the first 64 node indices and weights of a graph on their way while the one
+    //      before it is summed, handed round lane by lane; eight rows in flight, added in row order
+    const int offsets = s_row_ptr[g0 + min(lane, ng)];
+    auto offset = [&](int gi) { return __builtin_amdgcn_readlane(offsets, min(gi, ng)); };
+    int next_c = 0;
+    float next_v = 0.f;
+    auto ask = [&](int gi) {
+        const int e = offset(gi) + lane;
+        if (e < offset(gi + 1)) { next_c = s_col_idx[e]; next_v = s_val[e]; }
+    };
+    ask(wave);
+    for (int gi = wave; gi < kTileGraphs; gi += WAVES) {
         float acc[VEC];
 #pragma unroll
         for (int i = 0; i < VEC; ++i) acc[i] = 0.f;
-        if (gi < ng) {
-            const int start = s_row_ptr[g0 + gi], end = s_row_ptr[g0 + gi + 1];
-            // the wavefront reads 64 node indices and weights at once and hands them round lane by lane;
-            // eight rows in flight, added in row order
-            for (int base = start; base < end; base += kWave) {
-                const int cnt = min(kWave, end - base);
-                int my_c = 0;
-                float my_v = 0.f;
-                if (lane < cnt) { my_c = s_col_idx[base + lane]; my_v = s_val[base + lane]; }
-                for (int j = 0; j < cnt; j += 8) {
-                    vec_t x[8];
-                    float v[8];
+        const int start = offset(gi), end = offset(gi + 1);      // the same past the last graph
+        int my_c = next_c;
+        float my_v = next_v;
+        if (gi + WAVES < kTileGraphs) ask(gi + WAVES);
+        for (int base = start; base < end; base += kWave) {
+            const int cnt = min(kWave, end - base);
+            if (base > start && lane < cnt) { my_c = s_col_idx[base + lane]; my_v = s_val[base + lane]; }
+            for (int j = 0; j < cnt; j += 8) {
+                vec_t x[8];
+                float v[8];
 #pragma unroll
-                    for (int u = 0; u < 8; ++u) {
-                        const int src = min(j + u, cnt - 1);                     // uniform
-                        const int c = __builtin_amdgcn_readlane(my_c, src);
-                        v[u] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_v), src));
-                        x[u] = *reinterpret_cast<const vec_t*>(h + (size_t)c * C + lane * VEC);
-                    }
+                for (int u = 0; u < 8; ++u) {
+                    const int src = min(j + u, cnt - 1);                     // uniform
+                    const int c = __builtin_amdgcn_readlane(my_c, src);
+                    v[u] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_v), src));
+                    x[u] = *reinterpret_cast<const vec_t*>(h + (size_t)c * C + lane * VEC);
+                }
 #pragma unroll
-                    for (int u = 0; u < 8; ++u) {
-                        if (j + u < cnt) {
-                            const float* xp = reinterpret_cast<const float*>(&x[u]);
+                for (int u = 0; u < 8; ++u) {
+                    if (j + u < cnt) {
+                        const float* xp = reinterpret_cast<const float*>(&x[u]);
 #pragma unroll
-                            for (int i = 0; i < VEC; ++i) acc[i] = fmaf(v[u], xp[i], acc[i]);
-                        }
+                        for (int i = 0; i < VEC; ++i) acc[i] = fmaf(v[u], xp[i], acc[i]);
                     }
                 }
             }
-            *reinterpret_cast<vec_t*>(pool + (size_t)(g0 + gi) * C + lane * VEC) = *reinterpret_cast<vec_t*>(acc);
         }
+        if (gi < ng) *reinterpret_cast<vec_t*>(pool + (size_t)(g0 + gi) * C + lane * VEC) = *reinterpret_cast<vec_t*>(acc);
         *reinterpret_cast<vec_t*>(pl + gi * LD + lane * VEC) = *reinterpret_cast<vec_t*>(acc);   // zeros past the last graph
     }
     __syncthreads();
@@ -227,7 +236,7 @@ __global__ __launch_bounds__(kBlock) void s2v_readout_tile_kernel(
     //      (q, t) takes columns KS q .. KS q + KS - 1 of graph t and ends up with units 4 q .. of it
     constexpr int KS = C / 4;
     const int q4 = lane >> 4, t = lane & 15;
-    for (int j0 = 16 * wave; j0 < H; j0 += 16 * kWavesPerBlock) {
+    for (int j0 = 16 * wave; j0 < H; j0 += 16 * WAVES) {
         const float* w1 = Wh1 + (size_t)(KS * q4) * H + min(j0 + t, H - 1);
         const float* x = pl + t * LD + KS * q4;
         float w[2][kAhead];
@@ -263,7 +272,7 @@ __global__ __launch_bounds__(kBlock) void s2v_readout_tile_kernel(
     __syncthreads();
 
     // ---- logits = hidden * W_h2
-    for (int it = threadIdx.x; it < kTileGraphs * Q; it += kBlock) {
+    for (int it = threadIdx.x; it < kTileGraphs * Q; it += WAVES * kWave) {
         const int gi = it / Q, q = it % Q;
         float sum = 0.f;
 #pragma unroll 8
@@ -275,7 +284,7 @@ __global__ __launch_bounds__(kBlock) void s2v_readout_tile_kernel(
 
     // ---- softmax + argmax over Q, a wavefront per graph
     if (probs || pred) {
-        for (int gi = wave; gi < ng; gi += kWavesPerBlock) {
+        for (int gi = wave; gi < ng; gi += WAVES) {
             float* row = lg + (size_t)gi * Q;
             const int g = g0 + gi;
             const float first = row[0];
@@ -314,7 +323,12 @@ int launch_readout_tile(int B, int H, int Q, const int* s_row_ptr, const int* s_
     const size_t smem = sizeof(float) * (size_t)kTileGraphs * ((size_t)C + 4 + H + Q);
     if (smem > 64 * 1024) return GNNHIP_EUNSUPPORTED;
     const unsigned grid = (unsigned)(((long long)B + kTileGraphs - 1) / kTileGraphs);
-    hipLaunchKernelGGL(s2v_readout_tile_kernel<C>, dim3(grid), dim3(kBlock), smem, s, B, H, Q, s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2,
+    // Sixteen wavefronts, a graph each, where the tiles are about one round of the two workgroups that a compute unit holds then, eight beyond
+    // (hidden 256, 128 units, 30 nodes: 10,000 graphs 76.4 us with four, 71.8 with eight, 71.1 with sixteen, 4,097 33.7, 29.8 and 29.3; 12,288 of 25, 64
+    // units 71.1, 67.4 and 72.4; hidden 128: 9,999 36.8, 34.4 and 32.9, 20,000 81.6, 79.7 and 85.9, 25,000 of 2 nodes 29.5, 29.0 and 33.4)
+    const int waves = 2 * grid <= 5 * kNumCU ? 16 : 8;
+    const auto kernel = waves == 16 ? &s2v_readout_tile_kernel<C, 16> : &s2v_readout_tile_kernel<C, 8>;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(waves * kWave), smem, s, B, H, Q, s_row_ptr, s_col_idx, s_val, h, Wh1, Wh2,
                        pool, hidden, logits, probs, pred);
     GNNHIP_LAUNCH_CHECK("s2v_readout_tile");
     return GNNHIP_OK;

@@ -3109,3 +3109,36 @@ def test_input_stage_in_pieces_with_large_and_tiny_values(gpu):
     rest[5] = rest[17] = False
     assert torch.equal(got[rest], clean[rest])
     assert torch.equal(got[5], torch.sign(W[3]) * float("inf")) and bool(torch.isnan(got[17]).all())
+
+
+@pytest.mark.parametrize("C", [128, 256])
+@pytest.mark.parametrize("B,nodes", [(2047, 20), (2048, 20), (2063, 128), (2064, 129), (4096, 3), (4097, 300), (10_240, 9), (10_241, 9), (16_385, 5)])
+def test_readout_of_wide_hidden_sizes_by_tiles_of_graphs(gpu, C, B, nodes):
+    """batches around the sizes from which a workgroup takes 16 graphs, and from which it has eight wavefronts for them instead of sixteen: a last
+    tile of one graph and of all, graphs of 0, 1, 8, 9, 64, 65 and 200 nodes among the others, nodes in another order than the rows"""
+    import torch
+    from graphnn_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(B + C)
+    rng = np.random.default_rng(B)
+    n = np.full(B, nodes, np.int64)
+    n[rng.permutation(B)[:70]] = np.tile([0, 1, 8, 9, 64, 65, 200], 10)
+    n[-1] = max(n[-1], 1)
+    off = np.zeros(B + 1, np.int32)
+    np.cumsum(n, out=off[1:])
+    N, H, Q = int(off[-1]), 33, 3
+    S = (torch.from_numpy(off).to(gpu), torch.randperm(N, generator=gen, device=gpu).int(), torch.rand(N, generator=gen, device=gpu) + 0.5)
+    normal = lambda *shape: torch.randn(*shape, generator=gen, device=gpu)
+    h, W1, W2 = normal(N, C), normal(C, H), normal(H, Q)
+    pool, hidden, logits, probs, pred = ops.s2v_readout(*S, h, W1, W2, B)
+    rows = h[S[1].long()].double() * S[2].double()[:, None]
+    graph = torch.repeat_interleave(torch.arange(B, device=gpu), torch.from_numpy(n).to(gpu), output_size=N)
+    zero = torch.zeros(B, C, dtype=torch.float64, device=gpu)
+    want, terms = zero.index_add(0, graph, rows), zero.index_add(0, graph, rows.abs())
+    assert bool(((pool.double() - want).abs() <= (max(nodes, 200) + 1) * 2.0 ** -24 * terms).all())          # a rounding per term
+    # each layer from the one before it as the call gave it
+    want, terms = (pool.double() @ W1.double()).clamp(min=0), pool.double().abs() @ W1.double().abs()
+    assert bool(((hidden.double() - want).abs() <= (C + 1) * 2.0 ** -24 * terms).all())
+    want, terms = hidden.double() @ W2.double(), hidden.double().abs() @ W2.double().abs()
+    assert bool(((logits.double() - want).abs() <= (H + 1) * 2.0 ** -24 * terms).all())
+    assert bool(((probs.double() - torch.softmax(logits.double(), 1)).abs() <= 16 * 2.0 ** -24).all())
+    assert torch.equal(pred.long(), logits.argmax(1))
