@@ -161,6 +161,13 @@ int readout_any(int B, int N, int C, int H, int Q, const int* s_row_ptr, const i
     return GNNHIP_OK;
 }
 
+// whether two arrays of floats have no byte in common
+inline bool apart(const float* a, size_t na, const float* b, size_t nb)
+{
+    const auto x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return x + na * sizeof(float) <= y || y + nb * sizeof(float) <= x;
+}
+
 // input, L levels, readout on one stream; plan: of A, or null
 int forward_any(int N, int B, int K, int C, int H, int Q, int L, long long a_nnz, const int* a_row_ptr, const int* a_col_idx,
                 const float* a_val, const int* s_row_ptr, const int* s_col_idx, const float* s_val, const float* X, const float* W_n2l,
@@ -175,8 +182,17 @@ int forward_any(int N, int B, int K, int C, int H, int Q, int L, long long a_nnz
     // device whether the batch is one, and may add up the pooled rows.  The level-by-level launches behind it do nothing if it is.  What it
     // needs for that lies in the other embedding, which nothing else writes then, and, as the later launches ask for it, the word that
     // they go by in hidden, which is written by the last one.
+    // A caller may have the features, and weights that are done with early, in an output that is written late (the embeddings of the forward
+    // before, fed back in): the input stage is all that reads X and W_n2l then.
+    const size_t NC = (size_t)N * C;
+    const bool features_stay = apart(X, (size_t)N * K, h_a, NC) && apart(X, (size_t)N * K, h_b, NC) && apart(W_n2l, (size_t)K * C, h_a, NC) &&
+                               apart(W_n2l, (size_t)K * C, h_b, NC);
+    const bool inputs_stay = features_stay && apart(X, (size_t)N * K, pool, (size_t)B * C) && apart(W_n2l, (size_t)K * C, pool, (size_t)B * C) &&
+                             apart(W_conv, (size_t)C * C, pool, (size_t)B * C) && apart(X, (size_t)N * K, hidden, (size_t)B * H) &&
+                             apart(W_n2l, (size_t)K * C, hidden, (size_t)B * H) && apart(W_conv, (size_t)C * C, hidden, (size_t)B * H);
+    const MsgFactors factors = features_stay ? MsgFactors{X, W_n2l, K} : MsgFactors();
     const int* gate = nullptr;
-    const bool try_batch = lazy_h0 && aligned16(pool) && batch_levels_work_ints(B) <= (size_t)N * C;
+    const bool try_batch = lazy_h0 && inputs_stay && aligned16(pool) && batch_levels_work_ints(B) <= NC;
     const bool with_input = batch_levels_with_input(K, C), with_pool = batch_levels_with_pool(N, C) && readout_gated_accepts(C, H, Q);
     auto batch_levels = [&]() {
         int rc = GNNHIP_EUNSUPPORTED;
@@ -195,7 +211,7 @@ int forward_any(int N, int B, int K, int C, int H, int Q, int L, long long a_nnz
     float* nxt = lazy_h0 ? h_a : h_b;
     for (int lv = 0; lv < L; ++lv) {
         if ((rc = level_any(N, C, a_nnz, a_row_ptr, a_col_idx, a_val, cur, W_conv, msg, nullptr, nxt, s, lv > 0,
-                            lazy_h0 && lv == 0, plan, true, gate, MsgFactors{X, W_n2l, K})))
+                            lazy_h0 && lv == 0, plan, true, gate, factors)))
             return rc;
         float* t = (cur == msg) ? h_b : cur;     // msg stays what it is; the other buffer takes the next level
         cur = nxt;

@@ -3142,3 +3142,40 @@ def test_readout_of_wide_hidden_sizes_by_tiles_of_graphs(gpu, C, B, nodes):
     assert bool(((logits.double() - want).abs() <= (H + 1) * 2.0 ** -24 * terms).all())
     assert bool(((probs.double() - torch.softmax(logits.double(), 1)).abs() <= 16 * 2.0 ** -24).all())
     assert torch.equal(pred.long(), logits.argmax(1))
+
+
+@pytest.mark.parametrize("where", ["h_a", "h_b", "hidden", "pool"])
+@pytest.mark.parametrize("kind,C,K", [("batch", 64, 64), ("batch", 32, 32), ("batch", 100, 16), ("graph", 64, 16), ("graph", 32, 8)])
+def test_forward_over_features_that_lie_in_an_output(gpu, kind, C, K, where):
+    """features in a buffer that the forward writes after it has formed msg (the embeddings of the call before, fed back in): the same outputs
+    as with features of their own, over a batch of small graphs and over a power-law graph"""
+    import torch
+    from graphnn_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(C + K)
+    if kind == "batch":
+        A, S, N = _small_graphs(gpu, _enough(np.random.default_rng(C).integers(10, 111, 1100), C, 3, pooled=True), 2, gen)
+    else:
+        N = 200_003
+        deg = torch.randint(0, 30, (N,), generator=gen, device=gpu)
+        rp = torch.zeros(N + 1, dtype=torch.int32, device=gpu)
+        rp[1:] = torch.cumsum(deg, 0)
+        E = int(rp[-1])
+        A = (rp, torch.randint(0, N, (E,), generator=gen, device=gpu).int(), torch.rand(E, generator=gen, device=gpu) / 15)
+        S = (torch.tensor([0, N // 3, N], device=gpu).int(), torch.arange(N, device=gpu).int(), torch.ones(N, device=gpu))
+    B, H, Q = S[0].numel() - 1, 8, 3
+    normal = lambda *shape: torch.randn(*shape, generator=gen, device=gpu)
+    X, w = normal(N, K), (normal(K, C), normal(C, C) * (0.8 / C ** 0.5), normal(C, H), normal(H, Q))
+    names = ("msg", "h_final", "pool", "hidden", "logits", "probs", "pred")
+    apart, bufs = ops.ForwardBuffers(N, B, C, H, Q, gpu), ops.ForwardBuffers(N, B, C, H, Q, gpu)
+    ops.s2v_forward(A, S, X, *w, 3, bufs=apart)
+    room = torch.empty(max(N * K, N * C), device=gpu)            # the features, with the output at their start
+    room[:N * K] = X.reshape(-1)
+    rows, width = {"h_a": (N, C), "h_b": (N, C), "hidden": (B, H), "pool": (B, C)}[where]
+    setattr(bufs, where, room[:rows * width].view(rows, width))
+    ops.s2v_forward(A, S, room[:N * K].view(N, K), *w, 3, bufs=bufs)
+    for name in names:
+        got, want = getattr(bufs, name), getattr(apart, name)
+        if got.dtype == torch.float32:                           # another route may form them, in another order of the sums
+            assert float((got - want).norm()) <= 1e-5 * float(want.norm()), name
+        else:
+            assert float((got != want).float().mean()) <= 1e-3, name
