@@ -572,13 +572,19 @@ int rows_by_tile(const RowsArgs& a, hipStream_t s)
     return launch_rows<4, NB, 3, GATHER, WT>(a, s);
 }
 
+// nnz: entries of A (GATHER)
 template <bool GATHER, bool WT>
-int rows_dispatch(RowsArgs a, hipStream_t s)
+int rows_dispatch(RowsArgs a, long long nnz, hipStream_t s)
 {
     a.k_magic = a.K >= 2 ? (unsigned)(((1ull << 32) + a.K - 1) / a.K) : 0;
-    // (a second workgroup per compute unit would wait for the first: 4,112 rows, hidden 200, backward 18.8 -> 20.5 us)
-    if (a.N <= kFewRows && a.K >= 4) {
-        const int widest = a.K > a.n ? a.K : a.n;
+    // A workgroup per 16 rows: a second one per compute unit would wait for the first (4,112 rows, hidden 200, backward 18.8 -> 20.5 us).  Up to 64
+    // columns nothing is shared out, and all that is gained is W's way into registers beside the first rows: rows of many entries, and of more
+    // than columns, are summed faster in the kernel of many rows (2,048 rows, level and backward, there and here: hidden 20, 5 entries per row 4.3 us and 4.0,
+    // 4.7 and 4.4; 16 5.0 and 4.9, 5.5 and 5.3; 30 6.4 and 6.6, 6.8 and 7.0; 60 9.2 and 10.4, 9.7 and 10.7; hidden 50, 16 5.6 and 5.2, 60 9.8 and
+    // 11.1; hidden 8, 5 4.2 and 4.0; 12 4.9 and 4.8, 5.2 and 5.3; 30 6.6 and 6.9, 6.9 and 7.5; 180 24.5 and 27.4, 24.7 and 28.3)
+    const int widest = a.K > a.n ? a.K : a.n;
+    const bool many_entries = GATHER && widest <= 64 && nnz > (a.K < 16 ? a.K : 16) * (long long)a.N;
+    if (a.N <= kFewRows && a.K >= 4 && !many_entries) {
         if (widest <= 64) return launch_rows_few<4, GATHER, WT>(a, s);
         if (widest <= 128) return launch_rows_few<8, GATHER, WT>(a, s);
         return launch_rows_few<16, GATHER, WT>(a, s);
@@ -614,7 +620,7 @@ int level_rows_dispatch(int N, int C, long long nnz, const int* row_ptr, const i
     a.N = N; a.K = C; a.n = C;
     a.row_ptr = row_ptr; a.col_idx = col_idx; a.val = val; a.x = h_in; a.W = W;
     a.bias = bias; a.msg = msg; a.out = h_out; a.relu = 1; a.relu_in = relu_in; a.launch_gate = gate;
-    return rows_dispatch<true, false>(a, s);
+    return rows_dispatch<true, false>(a, nnz, s);
 }
 
 int level_rows_backward_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* dz,
@@ -626,7 +632,7 @@ int level_rows_backward_dispatch(int N, int C, long long nnz, const int* row_ptr
     a.N = N; a.K = C; a.n = C;
     a.row_ptr = row_ptr; a.col_idx = col_idx; a.val = val; a.x = dz; a.W = W;
     a.gate = gate; a.agg_out = u; a.out = g_prev; a.acc = acc;
-    return rows_dispatch<true, true>(a, s);
+    return rows_dispatch<true, true>(a, nnz, s);
 }
 
 // out = x * W (+ bias + msg); relu: out = ReLU of that; relu_out (or null) = ReLU(out).  x [N, K], W [K, n].
@@ -638,7 +644,7 @@ int level_rows_dense_dispatch(int N, int K, int n, const float* x, const float* 
     RowsArgs a{};
     a.N = N; a.K = K; a.n = n;
     a.x = x; a.W = W; a.bias = bias; a.msg = msg; a.out = out; a.relu = relu; a.relu_out = relu_out; a.launch_gate = gate;
-    return rows_dispatch<false, false>(a, s);
+    return rows_dispatch<false, false>(a, 0, s);
 }
 
 }  // namespace gnnhip

@@ -2949,6 +2949,34 @@ def test_levels_over_few_rows_have_the_bits_of_many(gpu, C):
     _few_rows_input(gpu, C)
 
 
+@pytest.mark.parametrize("C", [4, 7, 20, 33, 63])
+@pytest.mark.parametrize("N", [1, 16, 17, 272, 2049])
+def test_narrow_levels_over_few_rows_with_many_entries(gpu, C, N):
+    """up to 64 columns, few rows of more entries on average than columns, or than sixteen, take the kernel of many rows: the last average on one side
+    and the first on the other, against the same rows inside a matrix of more, a row of half of all entries among them"""
+    import torch
+    from graphnn_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(C)
+    rand = lambda *shape: torch.randn(*shape, generator=gen, device=gpu)
+    big, line = 4113, min(C, 16)
+    W = rand(C, C) * 0.2
+    for E in (line * N, line * N + 1, 40 * N):
+        deg = torch.bincount(torch.randint(0, N, (E - E // 2,), generator=gen, device=gpu), minlength=N)
+        deg[N // 2] += E // 2
+        rp = torch.zeros(big + 1, dtype=torch.int32, device=gpu)
+        rp[1:N + 1] = torch.cumsum(deg, 0)
+        rp[N + 1:] = E + torch.cumsum(torch.randint(0, 10, (big - N,), generator=gen, device=gpu), 0)
+        ci = torch.randint(0, N, (int(rp[-1]),), generator=gen, device=gpu).int()
+        val, x, msg, acc = rand(int(rp[-1])), rand(big, C), rand(big, C), rand(big, C)
+        few = (rp[:N + 1].contiguous(), ci[:E].contiguous(), val[:E].contiguous())
+        part = lambda t: t[:N].contiguous()
+        assert torch.equal(ops.s2v_level(*few, part(x), W, part(msg)), ops.s2v_level(rp, ci, val, x, W, msg)[:N]), E
+        a_few, a_big = part(acc), acc.clone()
+        u, g = ops.s2v_level_backward(*few, part(x), W, gate_h=part(msg), acc=a_few)
+        u2, g2 = ops.s2v_level_backward(rp, ci, val, x, W, gate_h=msg, acc=a_big)
+        assert torch.equal(u, u2[:N]) and torch.equal(g, g2[:N]) and torch.equal(a_few, a_big[:N]), E
+
+
 def _few_rows_input(gpu, C):
     """the input stage of few rows, feature columns narrower and wider than its steps: within the rounding of its sums"""
     import torch
