@@ -246,9 +246,10 @@ int launch_input_wide(int N, int K, const float* X, const float* Wn2l, float* ms
     // where W's operand for all columns is small (hidden 64 without h0, K = 16: 2,500,000 rows 176 -> 148, 60,000 6.2 -> 6.6; 128, K = 16: 700,000
     // 98 -> 76).  At hidden 256 and K > 32 two workgroups leave room for their registers at any size (K = 48, 88,000 rows 28.7 -> 26.4).
     // K > 48, hidden 256, msg alone: the FP32 matrix instructions, and all that waits for a slot between them, are longer
-    // than the outputs (300,000 rows 109 us, K = 4 63); in pieces 85.  Hidden 128, and with h0, gain nothing from that.
+    // than the outputs (300,000 rows 109 us, K = 4 63); in pieces 85.  Hidden 128, and with h0, gain nothing from that, nor do up to two tiles per compute
+    // unit, which wait for W to be split (2,000 rows 8.7 us and 10.7 in pieces, 16,000 10.2 and 12.3, 30,000 14.7 and 15.5, 33,000 22.2 and 18.4).
     const bool big = (h0 ? 2ull : 1ull) * (unsigned long long)N * C * 4ull > (256ull << 20);
-    const bool pieces = C == 256 && KS == 16 && !h0, rows = big && !h0 && (C == 64 ? KS <= 8 : C == 128 && KS == 4);
+    const bool pieces = C == 256 && KS == 16 && !h0 && ntiles > 2 * kNumCU, rows = big && !h0 && (C == 64 ? KS <= 8 : C == 128 && KS == 4);
     const bool two = C == 256 && KS > 8 ? KS == 12 || pieces : C >= 128 && big && (h0 || KS < 16) && !rows;
     const long long cap = (long long)kNumCU * (two ? 2 : 4);
     const unsigned grid = (unsigned)(ntiles < cap ? ntiles : cap);

@@ -19,8 +19,8 @@
  *   - operands, accumulators and results are fp32; sums may be taken in another order than the reference's.
  *   - four products run on the bf16 matrix cores, every fp32 operand as three bf16 numbers whose sum it is: the levels of
  *     gnnhip_s2v_forward_f32 / _planned_f32 at hidden 128 and 256, and at 33 to 112 over large batches of small graphs,
- *     gnnhip_s2v_level_backward_f32 at hidden 128 and 256, the input stage at hidden 256 from 49 feature columns on where h0 is
- *     not asked for, and A^T B with an output of up to 256 x 256 over 8,192 rows and more (m n k >= 2^28).  Their errors against exact sums are smaller than
+ *     gnnhip_s2v_level_backward_f32 at hidden 128 and 256, the input stage at hidden 256 from 49 feature columns and
+ *     32,769 rows on where h0 is not asked for, and A^T B with an output of up to 256 x 256 over 8,192 rows and more (m n k >= 2^28).  Their errors against exact sums are smaller than
  *     those of the FP32 matrix cores, over the whole range of fp32 and with infinities and NaNs carried on, with one
  *     limit: where a row of the left operand or a column of W (a column of A or B, over a run of rows) holds an element of
  *     2^38 or more, its elements below 2^-47 lose their last bits.

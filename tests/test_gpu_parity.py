@@ -3088,11 +3088,12 @@ def test_forward_of_a_power_law_graph_forms_msg_again(gpu, C, K):
         assert bool(((got.h_final.double() - h.double()).abs() <= err + L * (C + 900) * 2.0 ** -24 * terms).all())
 
 
-@pytest.mark.parametrize("C,N,Ks", [(256, 1, (49, 64)), (256, 15, (64,)), (256, 65, (53, 64)), (256, 3001, (49, 50, 61, 64)), (256, 270_001, (17, 40, 64)),
+@pytest.mark.parametrize("C,N,Ks", [(256, 1, (49, 64)), (256, 15, (64,)), (256, 65, (53, 64)), (256, 3001, (49, 50, 61, 64)), (256, 32_768, (49, 64)),
+                                    (256, 32_769, (49, 50, 61, 64)), (256, 33_085, (53, 64)), (256, 270_001, (17, 40, 64)),
                                     (64, 1_048_577, (1, 5, 16, 19, 32, 33)), (128, 530_049, (1, 3, 16, 20, 64))])
 @pytest.mark.parametrize("with_h0", [False, True])
 def test_input_stage_of_wide_and_large_calls(gpu, C, N, Ks, with_h0):
-    """msg alone in bf16 pieces (hidden 256, more than 48 feature columns), whole rows per store and fewer workgroups (more than 256 MB of
+    """msg alone in bf16 pieces (hidden 256, more than 48 feature columns, more than 32,768 rows), whole rows per store and fewer workgroups (more than 256 MB of
     outputs): sizes around a tile of 64 rows, the last rows of the last tile, and nothing written behind them"""
     import torch
     from graphnn_amd import ops
@@ -3116,7 +3117,7 @@ def test_input_stage_in_pieces_with_large_and_tiny_values(gpu):
     import torch
     from graphnn_amd import ops
     gen = torch.Generator(device=gpu).manual_seed(3)
-    N, K, C = 1000, 64, 256
+    N, K, C = 33_000, 64, 256
     msg = torch.empty(N, C, device=gpu)
     run = lambda X, W: (ops._bound().s2v_input_f32(N, K, C, X, W, msg, None), msg.clone())[1]
     X, W = torch.randn(N, K, generator=gen, device=gpu), torch.randn(K, C, generator=gen, device=gpu)
