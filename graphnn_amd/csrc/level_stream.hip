@@ -35,7 +35,7 @@
 //
 // REMAKE (with PIECES): msg is not read but formed again from up to 16 feature columns, a quarter of the bytes at C = 64 and four matrix
 // instructions per block of columns, in the order of the input stage of C = 64 (input_wide.hip), whose bits it has.  4M rows, 16 columns: 610 ->
-// 482 us of a level of 2.4 ms.
+// 482 us of a level of 2.4 ms.  W_n2l's way into LDS is 2 us of a level, and short graphs have msg in a cache: see kRemakeMinRows.
 //
 // Algorithmic bytes: 4(N+1) + 8E + 12NC + 4C^2.
 #include "level_gather.h"
@@ -52,6 +52,10 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kWavesPerBlock = kBlock / kWave;
+// From here on the level over sums of pieces forms msg again (hidden 32 and 64; at 16 it gains nothing at any size).  A kept plan, 14 entries per row, three levels, hidden 64
+// of 16 features: 33,000 rows 124.7 us and 131.0 so, 100,000 230.6 and 236.7, 150,000 322 and 325.5, 200,000 412 and 412, 330,000 687 and 670, 1M 1,990 and 1,918;
+// hidden 32: 33,000 86.6 and 88.2, 150,000 182.9 and 183.3, 200,000 233.2 and 232.4, 330,000 364.9 and 360.9; hidden 16 of 8 500,000 632 and 632.
+constexpr int kRemakeMinRows = 196608;
 constexpr int kPipeMinRows = 65536;   // from here on the kernel variant that asks for a tile's gathers one tile early
 
 
@@ -583,10 +587,12 @@ int launch_level_stream_pieces(int N, const float* W, const float* msg, const fl
     // 300,001 rows 478 us / 477, 1M 1,934 / 1,925, 4M 8,049 / 8,028.
     const long long resident = (long long)kNumCU * kMinW - 15;
     if (blocks > resident) blocks = resident;
-    // msg from its factors where a row of X is at most half as long as one of msg
-    const bool remake = factors.X && !bias && factors.K >= 1 && factors.K <= 16 && 2 * factors.K <= C;
-    const auto kernel = remake ? &s2v_level_stream_kernel<C, true, C == 64, kMinW, false, false, false, true, false, true>
-                               : &s2v_level_stream_kernel<C, true, C == 64, kMinW, false, false, false, true>;
+    // msg from its factors where the kernel's four matrix instructions take a whole row of X, which then is at most half as long as one of msg
+    auto kernel = &s2v_level_stream_kernel<C, true, C == 64, kMinW, false, false, false, true>;
+    if constexpr (C >= 32) {
+        if (factors.X && !bias && factors.K >= 1 && factors.K <= 16 && N >= kRemakeMinRows)
+            kernel = &s2v_level_stream_kernel<C, true, C == 64, kMinW, false, false, false, true, false, true>;
+    }
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kBlock), 0, s,
                        N, sums.first, (const int*)nullptr, (const float*)nullptr, (const float*)nullptr, W, msg, bias, h_out, HubPlan(),
                        (float*)nullptr, (float*)nullptr, sums, (const int*)nullptr, factors);

@@ -3049,14 +3049,15 @@ def test_wide_levels_in_pieces_over_few_rows_have_the_bits_of_many(gpu, N):
 
 
 @pytest.mark.parametrize("C,K", [(64, 16), (64, 13), (64, 4), (64, 1), (64, 17), (32, 16), (32, 7), (16, 8), (16, 9)])
-def test_forward_of_a_power_law_graph_forms_msg_again(gpu, C, K):
-    """levels of a graph of more than twelve entries per row whose contraction forms msg from up to sixteen feature columns instead of reading
-    it (17 columns, or 9 at hidden 16, are the other side of that): features that are no one-hot rows, against the levels called one by one
-    on the msg that the forward gives; rows without entries, of one piece and of many, a last tile of one row"""
+@pytest.mark.parametrize("N", [32785, 196607, 196609])
+def test_forward_of_a_power_law_graph_forms_msg_again(gpu, C, K, N):
+    """levels of a graph of more than twelve entries per row and 196,608 rows or more whose contraction forms msg from up to sixteen feature columns
+    instead of reading it (fewer rows, 17 columns and hidden 16 are the other side of that): features that are no one-hot rows, against the
+    levels called one by one on the msg that the forward gives; rows without entries, of one piece and of many, a last tile of one row"""
     import torch
     from graphnn_amd import ops
     gen = torch.Generator(device=gpu).manual_seed(C + K)
-    N, L = 32785, 3
+    L = 3
     deg = torch.randint(0, 45, (N,), generator=gen, device=gpu)
     deg[::3] = 0
     deg[torch.arange(5, N, 1000)] = 900
