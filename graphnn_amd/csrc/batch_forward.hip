@@ -595,22 +595,30 @@ int batch_levels_dispatch(int N, int B, int K, int C, int L, long long nnz, cons
     //            20     26,440, three (1.1 M) 32 and 33, four 38 and 36; 52,870, three (2.1 M) 54 and 46
     //            64     26,440, three (3.4 M) 41 and 42, four 50 and 48;  32: 52,870, three (3.4 M) 48 and 44
     //            16     73,432, four (3.5 M) 53 and 51 or, of 38 features, 58 and 50; 52,870, five (3.4 M) 57 and 64
-    // Up to 24,576 nodes hidden 16, 32 and 64 have level_tile.hip, up to 4,096 the others the kernel of few rows: neither has a gated variant.
+    // Up to kLevelTileMaxRows nodes hidden 16, 32 and 64 have level_tile.hip, up to kFewRows the others the kernel of few rows: neither has a gated variant.
     const bool own = C == 16 || C == 32 || C == 64, input = batch_levels_with_input(K, C);
-    const long long least = C == 16 ? 5000000 : C < 32 ? 1500000 : C == 32 ? 3000000 : C < 64 ? 3600000 : C == 64 || !input ? 4000000 : C <= 96 ? 1500000 : 1800000;
-    const bool enough = (long long)(L - 1) * N * C >= least && N > (own ? 24576 : C > 32 && C < 64 ? 16384 : kFewRows);
-    if (!enough || nnz >= kTwoStepMeanDegree * (long long)N || (long long)N > 96ll * B || C < 16 || C > 112) return GNNHIP_EUNSUPPORTED;
+    // Up to 32 columns a bin whose entries do not fit the LDS costs more than it saves (hidden 16, three levels: 300,573 nodes, 9 entries per row 95 us and 94, 10
+    // 97 and 107, 11.5 105 and 122; hidden 32, graphs of 128 and of 20 nodes in turn, 8.4 141 and 177)
+    const long long dense = C <= 32 ? kEdgeCap / kRows : kTwoStepMeanDegree;
+    if (nnz >= dense * N || (long long)N > 96ll * B || C < 16 || C > 112) return GNNHIP_EUNSUPPORTED;
     // Bins of fewer nodes where they fill the rounds of workgroups better: a round takes its tiles and about two more (start, barriers).
     // The host knows the totals only: a bin wastes about half a mean graph, and every 64 graphs about half a bin.
     const int slots = kNumCU * (C <= 16 ? 3 : C <= 64 ? 2 : 1);
     int cap = kRows;
+    long long rounds = 1;
     double best = 0.0;
     for (int c = kRows; c >= 64; c -= 16) {
         const double fill = (double)c - 0.5 * (double)N / (double)B;
         const double nbins = (double)N / (fill > 16.0 ? fill : 16.0) + (double)B / 128.0;
-        const double cost = (double)((long long)(nbins / slots) + 1) * (2.0 + c / 16);
-        if (c == kRows || cost < best) { best = cost; cap = c; }
+        const long long r = (long long)(nbins / slots) + 1;
+        const double cost = (double)r * (2.0 + c / 16);
+        if (c == kRows || cost < best) { best = cost; cap = c; rounds = r; }
     }
+    // (hidden 64: below 65,536 nodes the level-by-level kernels have not yet slowed down as a second round does: 60,222 nodes, three levels 63 us and 70, four
+    // 75 and 75, five 88 and 85; 70,000 78 and 70)
+    const long long least = C == 16 ? 5000000 : C < 32 ? 1500000 : C == 32 ? 3000000 : C < 64 ? 3600000 : C == 64 && N < 65536 && rounds > 1 ? 8000000 :
+                            C == 64 || !input ? 4000000 : C <= 96 ? 1500000 : 1800000;
+    if ((long long)(L - 1) * N * C < least || N <= (own ? kLevelTileMaxRows : C > 32 && C < 64 ? 64 * kNumCU : kFewRows)) return GNNHIP_EUNSUPPORTED;
     int* bins = work;
     hipLaunchKernelGGL((graph_bins_kernel<true>), dim3(ceil_div_u((size_t)B, kBinBlock)), dim3(kBinBlock), 0, s, B, cap, a_row_ptr, s_row_ptr,
                        bins, N, refused, kRows);
