@@ -42,6 +42,10 @@
 #include "graph_bins.h"
 
 namespace gnnhip {
+
+// hub.hip
+int hub_count_with_bins(int m, int n, long long nnz, const int* row_ptr, const BinsArgs& bins, hipStream_t s, bool* counted);
+
 namespace {
 
 constexpr int kRows = 128;                       // nodes of a bin
@@ -104,10 +108,14 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
     // a pair of columns by all lanes covers 32 consecutive bytes of 16 rows
     const int srt = 2 * ((K + 7) / 8);
 
-    // a segment that was not packed (graph_bins.h): nothing is formed.  Every workgroup looks at all words, 64 graphs each, so that a batch that is
-    // none costs no more than the start (10 to 15 us: 600 graphs, hidden 100 96 -> 107, 30,000, hidden 64 805 -> 829, 971 where only those that came upon such a word left)
+    // a segment that was not packed (graph_bins.h): nothing is formed.  Every workgroup looks at all words, 64 graphs each, and does so ahead of
+    // all else, so that a batch that is none costs little more than the launch
     bool unpacked = false;
     for (int i = tid; i < (B + kWave - 1) / kWave; i += kBlock) unpacked |= reinterpret_cast<const unsigned long long*>(bins)[i] == 0;
+    if (__syncthreads_or(unpacked)) {
+        if (tid == 0) *refused = 1;
+        return;
+    }
     BinFinder finder(B, bins);
     int at = finder.find((int)blockIdx.x);
 
@@ -178,10 +186,6 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
     if (tid < LD) hbuf[kRows * LD + tid] = 0.f;
     if (tid == 0) stop = 0;
     any_down = __syncthreads_or(any_down);
-    if (__syncthreads_or(unpacked)) {
-        if (tid == 0) *refused = 1;
-        return;
-    }
 
     // ---- what a bin needs from memory, asked for together and a bin ahead
     struct Bin { int node0, n, e0, ne, g0, ng; };
@@ -569,24 +573,19 @@ constexpr int kTwoStepMeanDegree = 12;           // denser matrices take the SpM
 
 }  // namespace
 
-// whether batch_levels_dispatch forms msg itself; else it is to be there (past 96 columns there is no more LDS for W_n2l of many rows)
-bool batch_levels_with_input(int K, int C) { return K >= 2 && C >= 16 && (K <= 16 ? C <= 112 : K <= 64 && C <= 96); }
-
 size_t batch_levels_work_ints(int B) { return bin_ints(B); }
 
-// whether batch_levels_dispatch forms the pooled rows too: the readout reads h otherwise, but needs a launch less (hidden 100, 44,000
+// whether the levels' launch forms the pooled rows too: the readout reads h otherwise, but needs a launch less (hidden 100, 44,000
 // nodes 93 us, 96 with them, 88,000 135 and 138, 176,000 218 and 212, 352,000 405 and 390; hidden 64 of 9 features, 73,000 nodes 73 and 70; hidden
 // 50, 88,000 nodes 87 and 85; hidden 32, 73,000 nodes 51 and 50, 294,000 82 and 78; hidden 16 587,000 nodes 92 and 92, of 60 features 142 and 146)
 bool batch_levels_with_pool(int N, int C) { return C > 16 && (long long)N * C >= (C > 64 ? 12000000 : 4000000); }
 
-// The last level's h and, unless pool is null, the pooled rows (and msg) of a batch of small graphs.  work: at least batch_levels_work_ints(B) ints, 16-byte
-// aligned, free once the launches are done.  *refused: the device word that says (1) that the batch is none and the outputs have to be
-// formed by the level-by-level route.
-// GNNHIP_EUNSUPPORTED (nothing launched): sizes that this route does not take.
-int batch_levels_dispatch(int N, int B, int K, int C, int L, long long nnz, const int* a_row_ptr, const int* a_col_idx, const float* a_val,
-                          const int* s_row_ptr, const int* s_col_idx, const float* s_val, const float* X, const float* Wn2l, const float* Wc,
-                          float* msg, float* h_out, float* pool, int* work, int* refused, hipStream_t s)
+// Whether a forward tries the one launch, and how.
+BatchRoute batch_levels_route(int N, int B, int K, int C, int L, long long nnz)
 {
+    BatchRoute route;
+    // (past 96 columns there is no more LDS for W_n2l of many rows)
+    const bool input = K >= 2 && C >= 16 && (K <= 16 ? C <= 112 : K <= 64 && C <= 96);
     // What the levels but the first save is reading h and msg and writing h, and, where the level-by-level kernels are those of any size, most
     // of a level.  Below these products the launches of both routes cost more than that.  Forwards, level by level and so:
     //     hidden 66     6,755 nodes, three levels (0.9 M) 39 us and 39, four 47 and 43; 14,102, two (0.9 M) 36 and 35, five 67 and 49
@@ -596,15 +595,14 @@ int batch_levels_dispatch(int N, int B, int K, int C, int L, long long nnz, cons
     //            64     26,440, three (3.4 M) 41 and 42, four 50 and 48;  32: 52,870, three (3.4 M) 48 and 44
     //            16     73,432, four (3.5 M) 53 and 51 or, of 38 features, 58 and 50; 52,870, five (3.4 M) 57 and 64
     // Up to kLevelTileMaxRows nodes hidden 16, 32 and 64 have level_tile.hip, up to kFewRows the others the kernel of few rows: neither has a gated variant.
-    const bool own = C == 16 || C == 32 || C == 64, input = batch_levels_with_input(K, C);
-    // Up to 32 columns a bin whose entries do not fit the LDS costs more than it saves (hidden 16, three levels: 300,573 nodes, 9 entries per row 95 us and 94, 10
-    // 97 and 107, 11.5 105 and 122; hidden 32, graphs of 128 and of 20 nodes in turn, 8.4 141 and 177)
-    const long long dense = C <= 32 ? kEdgeCap / kRows : kTwoStepMeanDegree;
-    if (nnz >= dense * N || (long long)N > 96ll * B || C < 16 || C > 112) return GNNHIP_EUNSUPPORTED;
+    const bool own = C == 16 || C == 32 || C == 64;
+    // At hidden 16 a bin whose entries do not fit the LDS costs more than it saves (three levels, 300,573 nodes: 9 entries per row 95 us and 94, 10 97 and 107,
+    // 11.5 105 and 122; 587,454 in graphs of 10 to 110, 8.4 133 and 118, 10 155 and 179)
+    const long long dense = C == 16 ? 9 : kTwoStepMeanDegree;
+    if (nnz >= dense * N || (long long)N > 96ll * B || C < 16 || C > 112) return route;
     // Bins of fewer nodes where they fill the rounds of workgroups better: a round takes its tiles and about two more (start, barriers).
     // The host knows the totals only: a bin wastes about half a mean graph, and every 64 graphs about half a bin.
     const int slots = kNumCU * (C <= 16 ? 3 : C <= 64 ? 2 : 1);
-    int cap = kRows;
     long long rounds = 1;
     double best = 0.0;
     for (int c = kRows; c >= 64; c -= 16) {
@@ -612,17 +610,39 @@ int batch_levels_dispatch(int N, int B, int K, int C, int L, long long nnz, cons
         const double nbins = (double)N / (fill > 16.0 ? fill : 16.0) + (double)B / 128.0;
         const long long r = (long long)(nbins / slots) + 1;
         const double cost = (double)r * (2.0 + c / 16);
-        if (c == kRows || cost < best) { best = cost; cap = c; rounds = r; }
+        if (c == kRows || cost < best) { best = cost; route.cap = c; rounds = r; }
     }
     // (hidden 64: below 65,536 nodes the level-by-level kernels have not yet slowed down as a second round does: 60,222 nodes, three levels 63 us and 70, four
     // 75 and 75, five 88 and 85; 70,000 78 and 70)
     const long long least = C == 16 ? 5000000 : C < 32 ? 1500000 : C == 32 ? 3000000 : C < 64 ? 3600000 : C == 64 && N < 65536 && rounds > 1 ? 8000000 :
                             C == 64 || !input ? 4000000 : C <= 96 ? 1500000 : 1800000;
-    if ((long long)(L - 1) * N * C < least || N <= (own ? kLevelTileMaxRows : C > 32 && C < 64 ? 64 * kNumCU : kFewRows)) return GNNHIP_EUNSUPPORTED;
-    int* bins = work;
-    hipLaunchKernelGGL((graph_bins_kernel<true>), dim3(ceil_div_u((size_t)B, kBinBlock)), dim3(kBinBlock), 0, s, B, cap, a_row_ptr, s_row_ptr,
-                       bins, N, refused, kRows);
+    if ((long long)(L - 1) * N * C < least || N <= (own ? kLevelTileMaxRows : C > 32 && C < 64 ? 64 * kNumCU : kFewRows)) return route;
+    route.take = true;
+    route.input = input;
+    return route;
+}
+
+// The launch ahead of the levels' one: the bins.  work: at least batch_levels_work_ints(B) ints, 16-byte aligned, free once the levels'
+// launch is done.  planned: A has a kept plan, which counts the long rows of A once and for all; else *counted: the levels' first hub_prepass may
+// reuse the plan of them that the call has left in the stream's scratch.
+int batch_levels_bins(const BatchRoute& route, int N, int B, int C, long long nnz, const int* a_row_ptr, const int* s_row_ptr, int* work, int* refused,
+                      bool planned, bool* counted, hipStream_t s)
+{
+    const BinsArgs bins{B, route.cap, a_row_ptr, s_row_ptr, work, N, kRows, refused};
+    if (!planned) return hub_count_with_bins(N, C, nnz, a_row_ptr, bins, s, counted);
+    hipLaunchKernelGGL((graph_bins_kernel<true>), dim3(ceil_div_u((size_t)B, kBinBlock)), dim3(kBinBlock), 0, s, bins);
     GNNHIP_LAUNCH_CHECK("graph_bins");
+    return GNNHIP_OK;
+}
+
+// The last level's h and, unless pool is null, the pooled rows (and msg) of a batch of small graphs.  bins: as batch_levels_bins left them.  *refused: the device
+// word that says (1) that the batch is none and the outputs have to be formed by the level-by-level route.  L >= 2 (batch_levels_route).
+int batch_levels_dispatch(const BatchRoute& route, int N, int B, int K, int C, int L, const int* a_row_ptr, const int* a_col_idx, const float* a_val,
+                          const int* s_row_ptr, const int* s_col_idx, const float* s_val, const float* X, const float* Wn2l, const float* Wc,
+                          float* msg, float* h_out, float* pool, const int* bins, int* refused, hipStream_t s)
+{
+    const bool input = route.input;
+    const int cap = route.cap;
 #define GNNHIP_BL(CP, KSX, ODD) launch_batch_levels<CP, KSX, ODD>(N, B, K, C, L, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx, s_val, X, Wn2l, Wc, msg, h_out, \
                                                 pool, bins, refused, cap, s)
     if (input && (C == 16 || C == 32 || C == 64)) {

@@ -18,11 +18,13 @@ int level_backward_dispatch(int N, int C, long long nnz, const int* row_ptr, con
                             const float* W, float* u, float* g_prev, const float* gate, float* acc, hipStream_t s);
 // batch_forward.hip
 size_t batch_levels_work_ints(int B);
-bool batch_levels_with_input(int K, int C);
 bool batch_levels_with_pool(int N, int C);
-int batch_levels_dispatch(int N, int B, int K, int C, int L, long long nnz, const int* a_row_ptr, const int* a_col_idx, const float* a_val,
+BatchRoute batch_levels_route(int N, int B, int K, int C, int L, long long nnz);
+int batch_levels_bins(const BatchRoute& route, int N, int B, int C, long long nnz, const int* a_row_ptr, const int* s_row_ptr, int* work, int* refused,
+                      bool planned, bool* counted, hipStream_t s);
+int batch_levels_dispatch(const BatchRoute& route, int N, int B, int K, int C, int L, const int* a_row_ptr, const int* a_col_idx, const float* a_val,
                           const int* s_row_ptr, const int* s_col_idx, const float* s_val, const float* X, const float* Wn2l, const float* Wc,
-                          float* msg, float* h_out, float* pool, int* work, int* refused, hipStream_t s);
+                          float* msg, float* h_out, float* pool, const int* bins, int* refused, hipStream_t s);
 // level_rows.hip
 int level_rows_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* col_idx, const float* val, const float* h_in,
                         const float* W, const float* msg, const float* bias, float* h_out, bool same_graph, bool relu_in, CsrPlan* plan,
@@ -191,26 +193,26 @@ int forward_any(int N, int B, int K, int C, int H, int Q, int L, long long a_nnz
                              apart(W_conv, (size_t)C * C, pool, (size_t)B * C) && apart(X, (size_t)N * K, hidden, (size_t)B * H) &&
                              apart(W_n2l, (size_t)K * C, hidden, (size_t)B * H) && apart(W_conv, (size_t)C * C, hidden, (size_t)B * H);
     const MsgFactors factors = features_stay ? MsgFactors{X, W_n2l, K} : MsgFactors();
-    const int* gate = nullptr;
-    const bool try_batch = lazy_h0 && inputs_stay && aligned16(pool) && batch_levels_work_ints(B) <= NC;
-    const bool with_input = batch_levels_with_input(K, C), with_pool = batch_levels_with_pool(N, C) && readout_gated_accepts(C, H, Q);
-    auto batch_levels = [&]() {
-        int rc = GNNHIP_EUNSUPPORTED;
-        int* refused = reinterpret_cast<int*>(hidden);
-        if (try_batch)
-            rc = batch_levels_dispatch(N, B, K, C, L, a_nnz, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx, s_val, X, W_n2l, W_conv, msg,
-                                       (L & 1) ? h_a : h_b, with_pool ? pool : nullptr, reinterpret_cast<int*>((L & 1) ? h_b : h_a), refused, s);
-        if (rc == GNNHIP_OK) gate = refused;
-        return rc == GNNHIP_EUNSUPPORTED ? GNNHIP_OK : rc;
-    };
+    BatchRoute route;
+    if (lazy_h0 && inputs_stay && aligned16(pool) && batch_levels_work_ints(B) <= NC) route = batch_levels_route(N, B, K, C, L, a_nnz);
+    const bool with_pool = route.take && batch_levels_with_pool(N, C) && readout_gated_accepts(C, H, Q);
+    int* refused = reinterpret_cast<int*>(hidden);
+    const int* gate = route.take ? refused : nullptr;
+    bool counted = false;                        // the long rows of A, beside the bins
     int rc;
-    if (with_input && (rc = batch_levels())) return rc;
-    if ((rc = input_any(N, K, C, X, W_n2l, msg, lazy_h0 ? nullptr : h_a, s, gate))) return rc;
-    if (!with_input && (rc = batch_levels())) return rc;
+    if (!route.input && (rc = input_any(N, K, C, X, W_n2l, msg, lazy_h0 ? nullptr : h_a, s))) return rc;
+    if (route.take) {
+        int* bins = reinterpret_cast<int*>((L & 1) ? h_b : h_a);
+        if ((rc = batch_levels_bins(route, N, B, C, a_nnz, a_row_ptr, s_row_ptr, bins, refused, plan != nullptr, &counted, s))) return rc;
+        if ((rc = batch_levels_dispatch(route, N, B, K, C, L, a_row_ptr, a_col_idx, a_val, s_row_ptr, s_col_idx, s_val, X, W_n2l, W_conv, msg,
+                                        (L & 1) ? h_a : h_b, with_pool ? pool : nullptr, bins, refused, s)))
+            return rc;
+        if (route.input && (rc = input_any(N, K, C, X, W_n2l, msg, nullptr, s, gate))) return rc;
+    }
     float* cur = lazy_h0 ? msg : h_a;
     float* nxt = lazy_h0 ? h_a : h_b;
     for (int lv = 0; lv < L; ++lv) {
-        if ((rc = level_any(N, C, a_nnz, a_row_ptr, a_col_idx, a_val, cur, W_conv, msg, nullptr, nxt, s, lv > 0,
+        if ((rc = level_any(N, C, a_nnz, a_row_ptr, a_col_idx, a_val, cur, W_conv, msg, nullptr, nxt, s, lv > 0 || counted,
                             lazy_h0 && lv == 0, plan, true, gate, factors)))
             return rc;
         float* t = (cur == msg) ? h_b : cur;     // msg stays what it is; the other buffer takes the next level

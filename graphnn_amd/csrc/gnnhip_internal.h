@@ -341,6 +341,12 @@ struct MsgFactors {
     const float* W = nullptr;          // [K, C]
     int K = 0;
 };
+// How a forward over what may be a batch of small graphs runs its levels in one launch (batch_forward.hip)
+struct BatchRoute {
+    bool take = false;                 // else level by level
+    int cap = 0;                       // nodes of a bin
+    bool input = false;                // the levels' launch forms msg too; else it is to be there
+};
 constexpr int kCombineLong = 8;        // pieces; the balanced pass sums the pieces of such rows
 int spmm_pieces_dispatch(int m, int k, int n, long long nnz, float alpha, const int* row_ptr, const int* col_idx, const float* val,
                          const float* B, int ldb, float beta, float* C, int ldc, hipStream_t s, bool reuse_plan,

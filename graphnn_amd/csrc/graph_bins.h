@@ -18,6 +18,18 @@
 #include "gnnhip_internal.h"
 
 namespace gnnhip {
+
+// CHECKED: nothing is known about s_row_ptr.  A segment whose graphs are no ascending ranges of nodes, of at most `limit` nodes each (at least cap), that
+// begin at node 0 and end at node N, gets the word 0 (a segment that is packed opens at least one bin), and *refused is set to 0 for the forward
+// kernel to set when it comes upon such a word.
+struct BinsArgs {
+    int B, cap;
+    const int *a_row_ptr, *s_row_ptr;
+    int* bins;
+    int N, limit;
+    int* refused;
+};
+
 namespace {
 
 constexpr int kOrderRec = 8;                     // ints per record (32-byte records)
@@ -27,22 +39,21 @@ __host__ __device__ inline size_t bin_words_ints(int B) { return ((size_t)((B + 
 // and all of them
 __host__ __device__ inline size_t bin_ints(int B) { return bin_words_ints(B) + kOrderRec * (size_t)((B + kWave - 1) / kWave * kWave); }
 
-// CHECKED: nothing is known about s_row_ptr.  A segment whose graphs are no ascending ranges of nodes, of at most `limit` nodes each (at least cap), that
-// begin at node 0 and end at node N, gets the word 0 (a segment that is packed opens at least one bin), and *refused is set to 0 for the
-// forward kernel to set when it comes upon such a word.
+// one segment, by one wavefront
 template <bool CHECKED>
-__global__ __launch_bounds__(kBinBlock) void graph_bins_kernel(int B, int cap, const int* __restrict__ a_row_ptr,
-                                                               const int* __restrict__ s_row_ptr, int* __restrict__ bins, int N,
-                                                               int* __restrict__ refused, int limit)
+__device__ __forceinline__ void pack_segment(int seg, const BinsArgs& a)
 {
+    const int B = a.B, cap = a.cap, N = a.N, limit = a.limit;
+    const int* __restrict__ a_row_ptr = a.a_row_ptr;
+    const int* __restrict__ s_row_ptr = a.s_row_ptr;
+    int* __restrict__ bins = a.bins;
     const int lane = threadIdx.x & (kWave - 1);
-    const int seg = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kBinBlock / kWave) + threadIdx.x / kWave));
     const int nlive = min(kWave, B - seg * kWave);
     if (nlive <= 0) return;
     int start = 0, end = 0;                      // first node and end of the lane's graph
     if (lane < nlive) { start = s_row_ptr[seg * kWave + lane]; end = s_row_ptr[seg * kWave + lane + 1]; }
     if constexpr (CHECKED) {
-        if (seg == 0 && lane == 0) *refused = 0;
+        if (seg == 0 && lane == 0) *a.refused = 0;
         const int g = seg * kWave + lane;
         const bool bad = start < 0 || end < start || end > N || end - start > limit || (g == 0 && start != 0) || (g == B - 1 && end != N);
         if (__any(lane < nlive && bad)) {
@@ -72,6 +83,12 @@ __global__ __launch_bounds__(kBinBlock) void graph_bins_kernel(int B, int cap, c
     int* rec = bins + bin_words_ints(B) + (size_t)(seg * kWave + __popcll(opens & ((1ull << lane) - 1ull))) * kOrderRec;
     *reinterpret_cast<int4*>(rec) = make_int4(seg * kWave + lane, start, n, e0);
     *reinterpret_cast<int2*>(rec + 4) = make_int2(e1, ng);
+}
+
+template <bool CHECKED>
+__global__ __launch_bounds__(kBinBlock) void graph_bins_kernel(BinsArgs a)
+{
+    pack_segment<CHECKED>(__builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kBinBlock / kWave) + threadIdx.x / kWave)), a);
 }
 
 // Where the record of a bin is.  A wavefront asks for its bins in ascending order and goes on

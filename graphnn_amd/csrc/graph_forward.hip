@@ -882,8 +882,8 @@ int launch_graph_forward(int B, int K, int H, int Q, int L, int n16max,
         void* p = nullptr;
         if (int rc = stream_scratch(s, sizeof(int) * bin_ints(B), &p)) return rc;
         order = static_cast<int*>(p);
-        hipLaunchKernelGGL((graph_bins_kernel<false>), dim3(ceil_div_u((size_t)B, kBinBlock)), dim3(kBinBlock), 0, s, B, n16max, a_row_ptr, s_row_ptr, order, 0,
-                           (int*)nullptr, 0);
+        hipLaunchKernelGGL((graph_bins_kernel<false>), dim3(ceil_div_u((size_t)B, kBinBlock)), dim3(kBinBlock), 0, s,
+                           BinsArgs{B, n16max, a_row_ptr, s_row_ptr, order, 0, 0, nullptr});
         GNNHIP_LAUNCH_CHECK("graph_bins");
     } else if (graphs_ordered(B) && n16max / 16 + 2 <= 64) {
         void* p = nullptr;

@@ -47,9 +47,11 @@ __global__ __launch_bounds__(kBlock) void s2v_readout_wave_kernel(
     float* lg = hid + H;                 // [Q]
     const int grp = lane / G, tx = lane % G;
 
-    for (int i = threadIdx.x; i < C * H; i += kBlock) w1[i] = Wh1[i];
-    for (int i = threadIdx.x; i < H * Q; i += kBlock) w2[i] = Wh2[i];
-    __syncthreads();
+    if constexpr (!POOL) {
+        for (int i = threadIdx.x; i < C * H; i += kBlock) w1[i] = Wh1[i];
+        for (int i = threadIdx.x; i < H * Q; i += kBlock) w2[i] = Wh2[i];
+        __syncthreads();
+    }
 
     const int nwaves = (int)gridDim.x * kWavesPerBlock;
     for (int g = (int)blockIdx.x * kWavesPerBlock + wave; g < B; g += nwaves) {

@@ -2815,6 +2815,48 @@ def test_forward_over_a_batch_that_is_none(gpu, C, kind):
     _check_forward(gpu, (rp, ci, val), S, N, 9, C, 3, gen, 0 if kind in ("long_row", "permuted_members") else 3)
 
 
+@pytest.mark.parametrize("C", [16, 31, 64, 90])
+@pytest.mark.parametrize("planned", [False, True])
+def test_forward_over_a_batch_that_is_none_with_long_rows(gpu, C, planned):
+    """refused on the device (its last graph has 129 nodes) with rows of 64, 65, 2,048, 2,049 and 9,000 entries, which the launch of the bins counts for
+    all levels, or a kept plan: embeddings and pooled rows have the bits of the stages called one by one, twice over, and after a batch of
+    as many entries without long rows on the same arrays"""
+    import torch
+    from graphnn_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(C)
+    n = _enough(np.random.default_rng(C).integers(10, 111, 1100), C, 4, pooled=True)
+    n[-1] = 129
+    (rp, ci, val), S, N = _small_graphs(gpu, n, 3, gen)
+    deg = (rp[1:] - rp[:-1]).long()
+    long = [64, 65, 2048, 2049, 9000]
+    rows = torch.arange(5, device=gpu) * (N // 5) + 7
+    deg[rows] = torch.tensor(long, device=gpu)
+    rp2 = torch.zeros_like(rp)
+    rp2[1:] = torch.cumsum(deg, 0)
+    E = int(rp2[-1])
+    graph = torch.repeat_interleave(torch.arange(n.size, device=gpu), torch.from_numpy(n).to(gpu))
+    row = torch.repeat_interleave(torch.arange(N, device=gpu), deg)
+    off, size = S[0].long()[graph[row]], torch.from_numpy(n).to(gpu)[graph[row]]
+    ci = (off + (torch.rand(E, generator=gen, device=gpu) * size).long().minimum(size - 1)).int()
+    val = torch.rand(E, generator=gen, device=gpu) / deg[row]
+    H, Q, K, B = 8, 3, 9, n.size
+    normal = lambda *shape: torch.randn(*shape, generator=gen, device=gpu)
+    X = torch.zeros(N, K, device=gpu)
+    X[torch.arange(N, device=gpu), torch.randint(0, K, (N,), generator=gen, device=gpu)] = 1.0
+    w = (normal(K, C), normal(C, C) * (0.8 / C ** 0.5), normal(C, H), normal(H, Q))
+    even = torch.linspace(0, E, N + 1, device=gpu).round().int()               # the same entries in rows of as many each
+    for shape in (rp2, rp2, even, rp2):
+        A = (shape, ci, val)
+        want = _forward_one_by_one(A, S, X, *w, 4)
+        if planned:
+            with ops.CsrPlan(*A, N, N) as plan:
+                bufs = ops.s2v_forward_planned(plan, S, X, *w, 4)
+        else:
+            bufs = ops.s2v_forward(A, S, X, *w, 4)
+        for got, e in zip((bufs.msg, bufs.h_final, bufs.pool), want):
+            assert torch.equal(got, e)
+
+
 @pytest.mark.parametrize("C", [32, 64, 100])
 def test_large_batch_forward_replays_from_a_captured_graph(gpu, C):
     """captured over a batch that the levels' one launch takes, then replayed over matrices changed in place: whether it takes them is
