@@ -516,7 +516,7 @@ int level_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* c
     // contraction whose signs a backward pass relies on (level_wide_split.hip)
     // plan: made by gnnhip_csr_plan_create for exactly these CSR arrays (then nnz is the matrix's own count), or null
     // relu_in: h_in is read as ReLU(h_in); only where level_accepts_relu_input says so
-    // gate: for the sizes that batch_levels_dispatch takes, else null
+    // gate: only to kernels that go by it, or the sums of long rows that are left out with it would be read all the same
     // same_graph: the previous call on this stream had the same A (a later level of one forward), so the
     // plan of the long-row pass is still in place and only its sums are redone
     if (!(aligned16(h_in) && aligned16(W) && aligned16(h_out) && (!msg || aligned16(msg)) && (!bias || aligned16(bias))))
@@ -549,7 +549,8 @@ int level_dispatch(int N, int C, long long nnz, const int* row_ptr, const int* c
             default: return launch_level<64, true>(N, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, none, s);
             }
         }
-        if (level_by_tile(N, C, nnz)) return level_tile_dispatch(N, C, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, relu_in, s);
+        if (!gate && level_by_tile(N, C, nnz)) return level_tile_dispatch(N, C, row_ptr, col_idx, val, h_in, W, msg, bias, h_out, relu_in, s);
+        if (gate && !level_stream_covers(N, C)) return GNNHIP_EUNSUPPORTED;          // the kernel with 64-bit addressing below has no gate
         HubPlan hubs{};
         if (int rc = hub_prepass(N, C, nnz, row_ptr, col_idx, val, h_in, C, s, &hubs, same_graph, relu_in, kHubThreshold, kHubChunk, -1,
                                  plan ? &plan->row_hub : nullptr, gate))

@@ -549,6 +549,7 @@ int launch_rows(const RowsArgs& a, hipStream_t s)
     const int width = KP + 4 > a.n ? KP + 4 : a.n;
     const unsigned grid = (unsigned)(((long long)a.N + 16 * RT - 1) / (16 * RT));
     constexpr bool kGated = !WT && NB <= 2;                // input and levels of batch_forward.hip's sizes
+    if (!kGated && a.launch_gate) return GNNHIP_EUNSUPPORTED;
     const auto kernel = kGated && a.launch_gate ? &s2v_rows_kernel<RT, NB, MINW, GATHER, WT, kGated> : &s2v_rows_kernel<RT, NB, MINW, GATHER, WT, false>;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBlock), sizeof(float) * 16 * RT * width, s, a);
     GNNHIP_LAUNCH_CHECK("s2v_rows");
@@ -584,7 +585,7 @@ int rows_dispatch(RowsArgs a, long long nnz, hipStream_t s)
     // 11.1; hidden 8, 5 4.2 and 4.0; 12 4.9 and 4.8, 5.2 and 5.3; 30 6.6 and 6.9, 6.9 and 7.5; 180 24.5 and 27.4, 24.7 and 28.3)
     const int widest = a.K > a.n ? a.K : a.n;
     const bool many_entries = GATHER && widest <= 64 && nnz > (a.K < 16 ? a.K : 16) * (long long)a.N;
-    if (a.N <= kFewRows && a.K >= 4 && !many_entries) {
+    if (a.N <= kFewRows && a.K >= 4 && !many_entries && !a.launch_gate) {          // (these have no gated variants)
         if (widest <= 64) return launch_rows_few<4, GATHER, WT>(a, s);
         if (widest <= 128) return launch_rows_few<8, GATHER, WT>(a, s);
         return launch_rows_few<16, GATHER, WT>(a, s);
