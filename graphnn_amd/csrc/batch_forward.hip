@@ -499,13 +499,9 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
             }
             __syncthreads();
         };
-        if (L == 1) {
-            level(std::true_type(), std::true_type());
-        } else {
-            level(std::true_type(), std::false_type());
-            for (int lv = 2; lv < L; ++lv) level(std::false_type(), std::false_type());
-            level(std::false_type(), std::true_type());
-        }
+        level(std::true_type(), std::false_type());      // (L >= 2)
+        for (int lv = 2; lv < L; ++lv) level(std::false_type(), std::false_type());
+        level(std::false_type(), std::true_type());
         copy_out(h_out);
         // pool = S h: a wavefront per graph, kLanes lanes per row
         if (pooled) {
