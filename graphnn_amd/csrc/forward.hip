@@ -185,11 +185,11 @@ int forward_any(int N, int B, int K, int C, int H, int Q, int L, long long a_nnz
     // needs for that lies in the other embedding, which nothing else writes then, and, as the later launches ask for it, the word that
     // they go by in hidden, which is written by the last one.
     // A caller may have the features, and weights that are done with early, in an output that is written late (the embeddings of the forward
-    // before, fed back in): the input stage is all that reads X and W_n2l then.
+    // before, fed back in): the input stage is all that reads X and W_n2l then, and does so once, which lets X be msg's memory too.
     const size_t NC = (size_t)N * C;
     const bool features_stay = apart(X, (size_t)N * K, h_a, NC) && apart(X, (size_t)N * K, h_b, NC) && apart(W_n2l, (size_t)K * C, h_a, NC) &&
                                apart(W_n2l, (size_t)K * C, h_b, NC);
-    const bool inputs_stay = features_stay && apart(X, (size_t)N * K, pool, (size_t)B * C) && apart(W_n2l, (size_t)K * C, pool, (size_t)B * C) &&
+    const bool inputs_stay = features_stay && apart(X, (size_t)N * K, msg, NC) && apart(X, (size_t)N * K, pool, (size_t)B * C) && apart(W_n2l, (size_t)K * C, pool, (size_t)B * C) &&
                              apart(W_conv, (size_t)C * C, pool, (size_t)B * C) && apart(X, (size_t)N * K, hidden, (size_t)B * H) &&
                              apart(W_n2l, (size_t)K * C, hidden, (size_t)B * H) && apart(W_conv, (size_t)C * C, hidden, (size_t)B * H);
     const MsgFactors factors = features_stay ? MsgFactors{X, W_n2l, K} : MsgFactors();

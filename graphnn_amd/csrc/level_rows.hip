@@ -534,7 +534,8 @@ int launch_rows_few(const RowsArgs& a, hipStream_t s)
     const int KP = (a.K + 15) & ~15;
     const int tiles = (int)(((long long)a.N + 15) / 16), blocks = (a.n + 15) / 16;
     // as long as there are compute units for it, four blocks to a workgroup: the matrix instructions of 16 x 256 x 256 on one of them take 4 us
-    int share = (blocks + 3) / 4;
+    // (in place, rows are read by nobody else: the input stage with as many feature columns as hidden units)
+    int share = a.x == a.out || a.x == a.relu_out ? 1 : (blocks + 3) / 4;
     while (share > 1 && share * tiles > kNumCU) --share;
     const int per = (blocks + share - 1) / share;
     hipLaunchKernelGGL((s2v_rows_few_kernel<BLOCKS, GATHER, WT>), dim3(tiles, share), dim3(BLOCKS * kWave), sizeof(float) * 16 * (KP + 4), s, a, per);

@@ -3295,3 +3295,45 @@ def test_forward_over_features_that_lie_in_an_output(gpu, kind, C, K, where):
             assert float((got - want).norm()) <= 1e-5 * float(want.norm()), name
         else:
             assert float((got != want).float().mean()) <= 1e-3, name
+
+
+@pytest.mark.parametrize("C", [20, 64, 100, 130, 200, 252, 256])
+@pytest.mark.parametrize("N", [1, 33, 300, 4096, 5000])
+def test_input_stage_in_place(gpu, C, N):
+    """as many feature columns as hidden units, msg or h0 over the features: every row is read before it is written, whoever forms its columns"""
+    import torch
+    from graphnn_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(C + N)
+    X, W = torch.randn(N, C, generator=gen, device=gpu), torch.randn(C, C, generator=gen, device=gpu)
+    msg, h = ops.s2v_input(X, W)
+    run = ops._bound().s2v_input_f32
+    for in_msg in (True, False):
+        a, b = X.clone(), torch.empty_like(X)
+        run(N, C, C, a, W, a if in_msg else b, b if in_msg else a)
+        assert torch.equal(a if in_msg else b, msg) and torch.equal(b if in_msg else a, h), in_msg
+    a = X.clone()
+    run(N, C, C, a, W, a, None)
+    b = torch.empty_like(X)
+    run(N, C, C, X, W, b, None)                                  # (wide hidden sizes: another kernel where h0 is not asked for)
+    assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("C", [32, 64])
+@pytest.mark.parametrize("refused", [False, True])
+def test_forward_with_msg_over_the_features(gpu, C, refused):
+    """a forward whose msg is to lie where its features are, over a batch of small graphs that one launch takes, and over one that it refuses"""
+    import torch
+    from graphnn_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(C)
+    A, S, N = _small_graphs(gpu, _enough(np.random.default_rng(C).integers(10, 111, 1100), C, 3, pooled=True), 2, gen)
+    if refused:
+        A[1][int(A[0][int(torch.nonzero(A[0][1:] > A[0][:-1])[-1])])] = 0
+    B, H, Q = S[0].numel() - 1, 8, 3
+    normal = lambda *shape: torch.randn(*shape, generator=gen, device=gpu)
+    X, w = normal(N, C), (normal(C, C) / C ** 0.5, normal(C, C) * (0.8 / C ** 0.5), normal(C, H), normal(H, Q))
+    want, bufs = ops.s2v_forward(A, S, X, *w, 3), ops.ForwardBuffers(N, B, C, H, Q, gpu)
+    bufs.msg = X
+    ops.s2v_forward(A, S, X, *w, 3, bufs=bufs)
+    for name in ("msg", "h_final", "pool", "hidden", "logits", "probs"):
+        e = getattr(want, name)
+        assert float((getattr(bufs, name) - e).norm()) <= 1e-5 * float(e.norm()), name
