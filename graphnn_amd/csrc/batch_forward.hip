@@ -23,9 +23,10 @@
 // Hidden 16 and 32 run on the FP32 matrix cores; the order of the sums is that of level_stream.hip and graph_forward.hip, so
 // every bit of h is theirs.  At hidden 64 the FP32 matrix instructions were the longest part (480 us of a kernel that takes 380
 // now), so its products are formed from bf16 pieces (bf16_split.h), the first two pieces of W in registers: rms error against float64
-// 1.16e-11 of the terms' magnitudes after four levels, level by level 2.42e-11.  What bounds that kernel is the issue of vector
-// instructions, about 330 per 16 rows and level (64 sum the first four entries, 104 split the rows); two wavefronts per SIMD, 247
-// registers.  What a bin reads is asked for while the last level of the bin before it ends (428 us without).
+// 1.16e-11 of the terms' magnitudes after four levels, level by level 2.42e-11.  Counted there, vector instructions
+// take 40 % of the cycles (about 330 per 16 rows and level: 64 sum the first four entries, 104 split the rows), the matrix pipes 28 %, the LDS 27 %,
+// a quarter of that bank conflicts, and memory moves 1.6 TB/s: no unit bounds that kernel but that it has two wavefronts per SIMD (247 registers), which
+// meet at two barriers per level and wait 41 % of their time.  What a bin reads is asked for while the last level of the bin before it ends (428 us without).
 //
 // Hidden sizes from 17 to 112 without kernels of their own take the next multiple of 16, with zeros behind the last column.  msg comes from
 // memory (the general input stage: 12 us of 91 at 44,000 nodes, hidden 100, and the launch) only where W_n2l does not fit or K is 1 or
@@ -109,7 +110,11 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
     const int srt = 2 * ((K + 7) / 8);
 
     // a segment that was not packed (graph_bins.h): nothing is formed.  Every workgroup looks at all words, 64 graphs each, and does so ahead of
-    // all else, so that a batch that is none costs little more than the launch
+    // all else, so that a batch that is none costs little more than the launch (with W loaded and split first 8 to 10 us in a trace, so 3 to 4).
+    // A forward that tries this for nothing, one graph of 600 nodes among others, four levels, without the attempt and with it: 30,000 graphs,
+    // hidden 64 696 us and 706; 1,500, hidden 64 81 and 87; hidden 100 159 and 163; 600, hidden 100 97 and 104.  (Packing the segments of few graphs
+    // in every workgroup here, without the bins' launch: as long for a batch that is none, 1 to 16 % longer for one that is taken.  The input stage
+    // of a refused batch here: 15 us where its own kernel takes 8.)
     bool unpacked = false;
     for (int i = tid; i < (B + kWave - 1) / kWave; i += kBlock) unpacked |= reinterpret_cast<const unsigned long long*>(bins)[i] == 0;
     if (__syncthreads_or(unpacked)) {
@@ -423,8 +428,8 @@ __global__ __launch_bounds__(batch_waves<CP>() * kWave, BatchShape<CP>::MINW) vo
                     } else {
                         split(kSplitUp, false);
                     }
-                    // The corrections are summed apart from the products of the first pieces (level_wide_split.hip): in registers the second
-                    // step's sum has the other sign, and either step's corrections come first
+                    // The corrections come ahead of the products of the first pieces: with W in registers in the same sum, one per step, the second of
+                    // the other sign; with W in LDS in a sum of their own
                     mfma_f4 acc[2][NJB];
 #pragma unroll
                     for (int jb = 0; jb < NJB; ++jb) acc[0][jb] = acc[1][jb] = mfma_f4{0.f, 0.f, 0.f, 0.f};

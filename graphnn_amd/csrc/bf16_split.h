@@ -5,7 +5,7 @@
 // the sum of the three is x itself.  A product of two such sums has nine terms; the three smallest (x2 y3, x3 y2,
 // x3 y3) are together at most 2^-26 of |x y|, a quarter of what rounding the product once to fp32 costs, and are left
 // out.  The other six are exact products of bf16 numbers, which the matrix instruction adds up in fp32.  It rounds
-// towards minus infinity, so each kernel sums the corrections (all but x1 y1) first and apart from what is large; the
+// towards minus infinity, so each kernel sums the corrections (all but x1 y1) ahead of what is large, in the same sum or in one of their own; the
 // results are then two to three times closer to float64 than those of v_mfma_f32_16x16x4_f32.
 //
 // Six v_mfma_f32_16x16x32_bf16 cover what takes eight v_mfma_f32_16x16x4_f32: 96 cycles of the matrix pipe instead of

@@ -178,7 +178,7 @@ __global__ __launch_bounds__(kBlock) void s2v_input_wide_kernel(
                 } else {
                     split(kSplitUp, false);
                 }
-                // the corrections first, apart from what is large
+                // the corrections first, in the same sum
                 auto products = [&](int w, int n) {
 #pragma unroll
                     for (int s = 0; s < KS2; ++s)

@@ -17,7 +17,7 @@
 //   * A wavefront whose rows hold more entries than the tops of the remaining blocks can take starts a second batch in
 //     the middle of a block; gathering behind the pass would hold up the other seven.
 //
-// 299,536 nodes, 659,010 entries, C = 256, first level apart: 380 (FP32 matrix cores) -> 273 us per level (0.93 GB of
+// 299,536 nodes, 659,010 entries, C = 256, first level apart: 380 (FP32 matrix cores) -> 276 us per level (0.93 GB of
 // activations at 3.4 TB/s), backward 474 -> 428 us (1.85 GB at 4.3 TB/s).  Counted there: 0.64 GB fetched and 0.31 GB written, matrix
 // pipes busy 40 % of the cycles, 3.8 other instructions per matrix instruction of 16 cycles (1.9 of them vector ones, which
 // split the rows, 1.5 scalar ones, which steer the gather), no bank conflicts: neither memory nor the matrix pipes, but two

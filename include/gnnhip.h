@@ -25,7 +25,8 @@
  *     limit: where a row of the left operand or a column of W (a column of A or B, over a run of rows) holds an element of
  *     2^38 or more, its elements below 2^-47 lose their last bits.
  *   - the level entries run on the FP32 matrix cores, so where its levels are formed in pieces a forward and the same
- *     levels called one by one agree to rounding and not to the last bit.
+ *     levels called one by one agree to rounding and not to the last bit.  The ReLU of levels formed in pieces gives 0 for
+ *     -0; elsewhere -0 passes, as in the reference.
  *
  * Each declaration cites the reference interface it stands in for
  * (paths relative to the graphnn source tree).
