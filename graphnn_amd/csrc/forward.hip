@@ -163,11 +163,11 @@ int readout_any(int B, int N, int C, int H, int Q, const int* s_row_ptr, const i
     return GNNHIP_OK;
 }
 
-// whether two arrays of floats have no byte in common
-inline bool apart(const float* a, size_t na, const float* b, size_t nb)
+// whether two arrays of 32-bit words have no byte in common
+inline bool apart(const void* a, size_t na, const void* b, size_t nb)
 {
     const auto x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
-    return x + na * sizeof(float) <= y || y + nb * sizeof(float) <= x;
+    return x + na * 4 <= y || y + nb * 4 <= x;
 }
 
 // input, L levels, readout on one stream; plan: of A, or null
@@ -185,16 +185,19 @@ int forward_any(int N, int B, int K, int C, int H, int Q, int L, long long a_nnz
     // needs for that lies in the other embedding, which nothing else writes then, and, as the later launches ask for it, the word that
     // they go by in hidden, which is written by the last one.
     // A caller may have the features, and weights that are done with early, in an output that is written late (the embeddings of the forward
-    // before, fed back in): the input stage is all that reads X and W_n2l then, and does so once, which lets X be msg's memory too.
+    // before, fed back in): the input stage is all that reads X and W_n2l then, and does so once, which lets X be msg's memory too.  And the pooled rows
+    // and the hidden layer may lie in what is done with before the readout (A, msg, the other embedding).
     const size_t NC = (size_t)N * C;
     const bool features_stay = apart(X, (size_t)N * K, h_a, NC) && apart(X, (size_t)N * K, h_b, NC) && apart(W_n2l, (size_t)K * C, h_a, NC) &&
                                apart(W_n2l, (size_t)K * C, h_b, NC);
-    const bool inputs_stay = features_stay && apart(X, (size_t)N * K, msg, NC) && apart(X, (size_t)N * K, pool, (size_t)B * C) && apart(W_n2l, (size_t)K * C, pool, (size_t)B * C) &&
-                             apart(W_conv, (size_t)C * C, pool, (size_t)B * C) && apart(X, (size_t)N * K, hidden, (size_t)B * H) &&
-                             apart(W_n2l, (size_t)K * C, hidden, (size_t)B * H) && apart(W_conv, (size_t)C * C, hidden, (size_t)B * H);
+    const auto late_apart = [&](const void* p, size_t n) { return apart(p, n, pool, (size_t)B * C) && apart(p, n, hidden, (size_t)B * H); };
+    const bool all_apart = features_stay && apart(X, (size_t)N * K, msg, NC) && late_apart(X, (size_t)N * K) && late_apart(W_n2l, (size_t)K * C) &&
+                           late_apart(W_conv, (size_t)C * C) && late_apart(a_row_ptr, (size_t)N + 1) && late_apart(a_col_idx, (size_t)a_nnz) &&
+                           late_apart(a_val, (size_t)a_nnz) && late_apart(s_row_ptr, (size_t)B + 1) && late_apart(msg, NC) && late_apart(h_a, NC) &&
+                           late_apart(h_b, NC) && apart(pool, (size_t)B * C, hidden, (size_t)B * H);
     const MsgFactors factors = features_stay ? MsgFactors{X, W_n2l, K} : MsgFactors();
     BatchRoute route;
-    if (lazy_h0 && inputs_stay && aligned16(pool) && batch_levels_work_ints(B) <= NC) route = batch_levels_route(N, B, K, C, L, a_nnz);
+    if (lazy_h0 && all_apart && aligned16(pool) && batch_levels_work_ints(B) <= NC) route = batch_levels_route(N, B, K, C, L, a_nnz);
     const bool with_pool = route.take && batch_levels_with_pool(N, C) && readout_gated_accepts(C, H, Q);
     int* refused = reinterpret_cast<int*>(hidden);
     const int* gate = route.take ? refused : nullptr;

@@ -3337,3 +3337,30 @@ def test_forward_with_msg_over_the_features(gpu, C, refused):
     for name in ("msg", "h_final", "pool", "hidden", "logits", "probs"):
         e = getattr(want, name)
         assert float((getattr(bufs, name) - e).norm()) <= 1e-5 * float(e.norm()), name
+
+
+@pytest.mark.parametrize("C", [20, 64, 100])
+@pytest.mark.parametrize("late", ["pool", "hidden"])
+@pytest.mark.parametrize("where", ["msg", "h_b", "a_val"])
+def test_forward_whose_late_outputs_lie_in_what_is_done_with(gpu, C, late, where):
+    """pooled rows or hidden layer in an array that nothing reads any more when they are written: msg, the embedding that is not the last one, the entries
+    of A.  The same outputs as with arrays of their own, over a batch of small graphs that one launch would take otherwise"""
+    import torch
+    from graphnn_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(C)
+    n = _enough(np.random.default_rng(C).integers(10, 111, 1100), C, 3, pooled=True)
+    assert _tried(gpu, n, 2, 9, C, 3)
+    A, S, N = _small_graphs(gpu, n, 2, gen)
+    B, H, Q = S[0].numel() - 1, 8, 3
+    normal = lambda *shape: torch.randn(*shape, generator=gen, device=gpu)
+    X, w = normal(N, 9), (normal(9, C), normal(C, C) * (0.8 / C ** 0.5), normal(C, H), normal(H, Q))
+    want, bufs = ops.s2v_forward(A, S, X, *w, 3), ops.ForwardBuffers(N, B, C, H, Q, gpu)
+    rows, width = {"hidden": (B, H), "pool": (B, C)}[late]
+    room = A[2] if where == "a_val" else getattr(bufs, where).view(-1)
+    assert room.numel() >= rows * width
+    setattr(bufs, late, room[:rows * width].view(rows, width))
+    ops.s2v_forward(A, S, X, *w, 3, bufs=bufs)
+    for name in ("h_final", "pool", "hidden", "logits", "probs"):
+        e = getattr(want, name)
+        assert float((getattr(bufs, name) - e).norm()) <= 1e-5 * float(e.norm()), name
+    assert float((bufs.pred != want.pred).float().mean()) <= 1e-3
