@@ -602,21 +602,32 @@ BatchRoute batch_levels_route(int N, int B, int K, int C, int L, long long nnz)
     const long long dense = C == 16 ? 9 : kTwoStepMeanDegree;
     if (nnz >= dense * N || (long long)N > 96ll * B || C < 16 || C > 112) return route;
     // Bins of fewer nodes where they fill the rounds of workgroups better: a round takes its tiles and about two more (start, barriers).
-    // The host knows the totals only: a bin wastes about half a mean graph, and every 64 graphs about half a bin.
+    // The host knows the totals only: a bin wastes about 0.6 of a mean graph (half of the graph that no longer fits, and large ones are met more often), and every
+    // 64 graphs about half a bin.
     const int slots = kNumCU * (C <= 16 ? 3 : C <= 64 ? 2 : 1);
     long long rounds = 1;
     double best = 0.0;
     for (int c = kRows; c >= 64; c -= 16) {
-        const double fill = (double)c - 0.5 * (double)N / (double)B;
+        const double fill = (double)c - 0.6 * (double)N / (double)B;
         const double nbins = (double)N / (fill > 16.0 ? fill : 16.0) + (double)B / 128.0;
         const long long r = (long long)(nbins / slots) + 1;
         const double cost = (double)r * (2.0 + c / 16);
         if (c == kRows || cost < best) { best = cost; route.cap = c; rounds = r; }
     }
-    // (hidden 64: below 65,536 nodes the level-by-level kernels have not yet slowed down as a second round does: 60,222 nodes, three levels 63 us and 70, four
-    // 75 and 75, five 88 and 85; 70,000 78 and 70)
-    const long long least = C == 16 ? 5000000 : C < 32 ? 1500000 : C == 32 ? 3000000 : C < 64 ? 3600000 : C == 64 && N < 65536 && rounds > 1 ? 8000000 :
-                            C == 64 || !input ? 4000000 : C <= 96 ? 1500000 : 1800000;
+    // Up to 128 rows per compute unit the level-by-level kernels are at their best, and bins that need a second round of workgroups lose to them with few levels (28,000
+    // nodes of 38 features, hidden 72, two levels 44.8 us and 48.3; hidden 100 of 7, two 53.4 and 54.4; of 38, three 77.6 and 79.0); so does hidden 64 in one
+    // round (28,000, four levels 44.9 and 48.3, five 58 and 56), which meets a second one below 65,536 nodes, where they have not yet slowed down again
+    // (60,000, three 64.3 and 65.8, four 76.3 and 78.1, five 100 and 95)
+    const bool few = N <= 128 * kNumCU, again = rounds > 1;
+    long long least;
+    if (C <= 32) least = C == 16 ? 5000000 : C == 32 ? 3000000 : 1500000;
+    else if (C < 64) least = L == 2 || (L == 3 && few) ? 4100000 : 3600000;        // (hidden 56, 70,000 nodes, two levels 71.6 us and 74.9, 75,000 73 and 68)
+    else if (C == 64) least = few ? 6300000 : again && N < 65536 ? 12000000 : 4000000;
+    else if (!input) least = few && again ? 7500000 : 4000000;
+    else least = few && again ? 3700000 : C <= 96 ? 1500000 : 1800000;
+    // Graphs of more than half a bin leave much of it empty (all of 65 nodes, hidden 64 of 38 features: 52,000, five levels 86 us and 101, 150,000, two 86 and 100, three
+    // 114 and 119, 300,000, two 146 and 158; hidden 56, 90,000, two 69 and 81)
+    if (2ll * N > (long long)kRows * B) least *= L == 2 ? 6 : 3;
     if ((long long)(L - 1) * N * C < least || N <= (own ? kLevelTileMaxRows : C > 32 && C < 64 ? 64 * kNumCU : kFewRows)) return route;
     route.take = true;
     route.input = input;

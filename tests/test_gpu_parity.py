@@ -2776,7 +2776,8 @@ def _check_forward(gpu, A, S, N, K, C, L, gen, exact, taken):
 
 def _enough(n, C, L, pooled=False):
     """the sizes repeated until the batch is one that the forward tries to take in one launch, with pooled: that adds up the pooled rows too"""
-    need = max(32768, (12e6 if C == 16 else 8e6 if C == 64 else 6e6 if 32 < C < 64 else 4e6) / ((L - 1) * C), (12e6 if C > 64 else 4e6) / C if pooled else 0)
+    least = (12e6 if C in (16, 64) else 6e6 if 32 < C < 64 else 4e6) * (1 if np.sum(n) <= 64 * np.size(n) else 6 if L == 2 else 3)
+    need = max(32769, least / ((L - 1) * C), (12e6 if C > 64 else 4e6) / C if pooled else 0)
     return np.tile(np.asarray(n, np.int64), int(np.ceil(need / np.sum(n))))
 
 
@@ -3364,3 +3365,30 @@ def test_forward_whose_late_outputs_lie_in_what_is_done_with(gpu, C, late, where
         e = getattr(want, name)
         assert float((getattr(bufs, name) - e).norm()) <= 1e-5 * float(e.norm()), name
     assert float((bufs.pred != want.pred).float().mean()) <= 1e-3
+
+
+@pytest.mark.parametrize("C,K,L,nodes,mean,taken", [(64, 38, 4, 31_000, 29, False), (64, 38, 5, 32_000, 29, True), (64, 38, 4, 60_000, 39, False), (64, 38, 5, 60_000, 39, True),
+                                                    (64, 9, 3, 68_000, 39, True), (72, 38, 2, 31_000, 39, False), (72, 38, 3, 31_000, 39, True), (100, 38, 3, 31_000, 39, False),
+                                                    (100, 38, 4, 31_000, 39, True), (56, 38, 2, 70_000, 39, False), (56, 38, 3, 34_000, 39, True), (64, 38, 2, 150_000, 65, False),
+                                                    (64, 38, 4, 150_000, 65, True)])
+def test_which_batches_the_forward_tries_to_take_in_one_launch(gpu, C, K, L, nodes, mean, taken):
+    """both sides of the lines below which the level-by-level kernels are the faster ones: graphs of half to one and a half times the mean size, or, where
+    that is more than half a bin, all of one size"""
+    n = np.random.default_rng(nodes).integers(mean // 2, mean + mean // 2 + 1, nodes // mean) if mean < 64 else np.full(nodes // mean, mean)
+    assert _tried(gpu, n, 2, K, C, L) == taken
+
+
+def test_bins_of_a_batch_fill_one_round_of_workgroups(gpu):
+    """sizes of molecules, whose bins waste more than half a mean graph: where a round of 512 workgroups can take the batch, its bins are no more than that"""
+    import torch
+    from graphnn_amd import ops
+    n = np.clip((np.random.default_rng(33_000).gamma(2.0, 10.0, 1138) + 9).astype(int), 10, 110)
+    A, S, N = _small_graphs(gpu, n, 2, torch.Generator(device=gpu).manual_seed(1))
+    bufs = ops.ForwardBuffers(N, n.size, 64, 8, 3, gpu)
+    _fill(bufs)
+    zero = lambda *shape: torch.zeros(*shape, device=gpu)
+    ops.s2v_forward(A, S, zero(N, 9), zero(9, 64), zero(64, 64), zero(64, 8), zero(8, 3), 5, bufs=bufs)
+    assert _in_one_launch(bufs)
+    other = bufs.h_b if bufs.which.value == 0 else bufs.h_a
+    words = other.view(-1)[:2 * ((n.size + 63) // 64)].contiguous().view(torch.int32).cpu().numpy()
+    assert sum(bin(int(w) & 0xffffffff).count("1") for w in words) <= 512
