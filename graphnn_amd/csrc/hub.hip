@@ -136,7 +136,6 @@ __global__ __launch_bounds__(kBlock) void hub_partial_kernel(
     const int* __restrict__ list_chunk, int chunk_cap, int n, const int* __restrict__ row_ptr, const int* __restrict__ col_idx, const float* __restrict__ val, const float* __restrict__ B, int ldb, int logG,
     int* __restrict__ row_chunk, float* __restrict__ part, int ldp, int relu_in, int threshold, int shift, const int* __restrict__ gate)
 {
-    if (gated_off<GATED>(gate)) return;
     // relu_in: the rows of B are used as ReLU(B) (a first level that reads msg in place of h0)
     __shared__ float red[kWavesPerBlock][kWave * V::kVec * ITERS];
     __shared__ int before[kMaxRuns + 1];         // chunks ahead of a run
@@ -165,6 +164,8 @@ __global__ __launch_bounds__(kBlock) void hub_partial_kernel(
             nchunks += wave_total[w];
         }
         if (nchunks == 0) return;
+        // (here and not ahead of the counts: most matrices have no long rows, and the word would be a trip to memory of its own)
+        if (gated_off<GATED>(gate)) return;
 #pragma unroll
         for (int i = 0; i < kEach; ++i) {
             if (i < per && threadIdx.x * per + i < runs) before[threadIdx.x * per + i] = at;
