@@ -244,14 +244,18 @@ int launch_input_wide(int N, int K, const float* X, const float* Wn2l, float* ms
     // writing at once are faster (hidden 128 with h0, K = 7: 300,000 rows 67 us with four workgroups per compute unit, 63 with two,
     // 700,000 171 and 135; hidden 256 without, K = 32: 300,000 rows 88 and 79; six or eight are slower than four), and so are whole rows per store
     // where W's operand for all columns is small (hidden 64 without h0, K = 16: 2,500,000 rows 176 -> 148, 60,000 6.2 -> 6.6; 128, K = 16: 700,000
-    // 98 -> 76).  At hidden 256 and K > 32 two workgroups leave room for their registers at any size (K = 48, 88,000 rows 28.7 -> 26.4; K = 64
-    // with h0 40,000 26.3 -> 23.3, 90,000 46.5 -> 40.9, 300,000 150.6 -> 148.6), but for K > 48 with h0 over more rows than these (600,000 283.9 and 289.1).
+    // 98 -> 76); at hidden 256 with h0 fewer in the writing gain from 400 MB on (K = 32: 180,000 rows 89.7 and 93.3, 250,000 133.7 and 129.7).
+    // At hidden 256 and K > 32 two workgroups leave room for their registers (K = 48: 60,000 rows 22.8 -> 19.6, 90,000 28.4 -> 26.4; K = 64
+    // with h0 45,000 26.3 -> 23.4, 90,000 45.9 -> 41.8), but up to three tiles per compute unit at K <= 48 (45,000 15.9 and 16.5), and for K > 48 with h0 past
+    // what the cache holds (180,000 93.6 and 97.3, 300,000 150.6 and 153.6).
     // K > 48, hidden 256, msg alone: the FP32 matrix instructions, and all that waits for a slot between them, are longer
     // than the outputs (300,000 rows 109 us, K = 4 63); in pieces 85.  Hidden 128, and with h0, gain nothing from that, nor do up to two tiles per compute
     // unit, which wait for W to be split (2,000 rows 8.7 us and 10.7 in pieces, 16,000 10.2 and 12.3, 30,000 14.7 and 15.5, 33,000 22.2 and 18.4).
-    const bool big = (h0 ? 2ull : 1ull) * (unsigned long long)N * C * 4ull > (256ull << 20);
+    const unsigned long long out_bytes = (h0 ? 2ull : 1ull) * (unsigned long long)N * C * 4ull;
+    const bool big = out_bytes > (256ull << 20);
     const bool pieces = C == 256 && KS == 16 && !h0 && ntiles > 2 * kNumCU, rows = big && !h0 && (C == 64 ? KS <= 8 : C == 128 && KS == 4);
-    const bool two = C == 256 && KS > 8 ? KS == 12 || pieces || (h0 && N <= 400000) : C >= 128 && big && (h0 || KS < 16) && !rows;
+    const bool two = C == 256 && KS == 12 ? ntiles > 3 * kNumCU : C == 256 && KS == 16 ? (h0 ? !big : pieces) :
+                     C >= 128 && out_bytes > ((C == 256 && h0 ? 400ull : 256ull) << 20) && (h0 || KS < 16) && !rows;
     const long long cap = (long long)kNumCU * (two ? 2 : 4);
     const unsigned grid = (unsigned)(ntiles < cap ? ntiles : cap);
     const unsigned k_magic = K >= 2 ? (unsigned)((0x100000000ull + (unsigned)K - 1) / (unsigned)K) : 0u;   // ceil(2^32 / K)
